@@ -284,9 +284,21 @@ int kutacc_hip_triangle_multiplication(const kutacc_hip_triangle_multiplication_
     }
     const int64_t n = a->n_res, cz = a->c_z, ci = a->c_i, rows = n * n, buf = need / 4, plane = rows + TM_PLANE_PAD;
     char *ws = static_cast<char *>(a->workspace);
+    hipStream_t s = kutacc_api::stream_or_default(stream);
+    const bool ends = kutacc_launch::triangle_ends_support(*a);
+    if (ends && (kutacc_launch::gated_projection_mode() < 2 || n % 8 != 0)) {
+        // 128 channels: three launches on planes whose rows start on 16 bytes at every n.  Three such planes per channel fit
+        // what four dense ones take: 3 (n (n + 7) + 63 + pad) <= 4 (n^2 + pad) for every n.
+        const int64_t np = (n + 7) / 8 * 8, padded = (n * np + 63) / 64 * 64 + TM_PLANE_PAD;
+        void *left = ws, *right = ws + align256(ci * padded * 2), *centre = ws + 2 * align256(ci * padded * 2);
+        int rc = kutacc_launch::triangle_front(*a, left, right, np, padded, s);
+        if (rc == 0) {
+            rc = kutacc_launch::triangle_equation(left, right, centre, n, np, padded, ci, a->incoming != 0, s);
+        }
+        return rc != 0 ? rc : kutacc_launch::triangle_back(*a, centre, np, padded, s);
+    }
     void *act = ws, *left = ws + buf, *right = ws + 2 * buf, *center_cf = ws + 3 * buf;
     void *center = left, *gate = right, *out = center_cf; // each is free again by the time its second tenant arrives
-    hipStream_t s = kutacc_api::stream_or_default(stream);
 
     // 1. layer_norm_input
     int rc = kutacc_launch::layernorm_rows(a->pair_act, cz, a->ln_in_gamma, a->ln_in_beta, act, cz, rows, cz, a->ln_eps,
@@ -329,19 +341,17 @@ int kutacc_hip_triangle_multiplication(const kutacc_hip_triangle_multiplication_
         g.c = center_cf, g.c_stride_m = n;
         rc = kutacc_launch::pair_gemm(g, s);
     }
-    // The last kernel can form the gate itself (128 channels in and out: the gate tensor is then never written), and with
-    // positions in whole 16-byte runs it also reads the centre channel-first and normalises it on the way in
-    const bool gate_inside = kutacc_launch::row_projection_projected_gate_supports(
-        center, ci, a->output_w, a->output_b, act, cz, a->gating_w, a->gating_b, a->pair_act, cz, rows, cz, ci, cz);
-    const bool norm_inside = gate_inside && rows % 8 == 0 && kutacc_hip_aligned16(a->ln_center_gamma) &&
-                             kutacc_hip_aligned16(a->ln_center_beta);
+    // (128 channels, behind the tuning hook of the gated projections: the last steps in one kernel)
+    if (rc == 0 && ends) {
+        return kutacc_launch::triangle_back(*a, center_cf, n, plane, s);
+    }
     // 4. center_layer_norm, channel-first in, channel-last out
-    if (rc == 0 && !norm_inside) {
+    if (rc == 0) {
         rc = kutacc_launch::layernorm_channel_first(center_cf, plane, a->ln_center_gamma, a->ln_center_beta, center, ci, ci, rows,
                                                     a->ln_eps, KUTACC_DTYPE_BF16, s);
     }
     // 5. gate from the normalised input
-    if (rc == 0 && !gate_inside) {
+    if (rc == 0) {
         kutacc_hip_gemm_args_t g;
         std::memset(&g, 0, sizeof(g));
         g.dtype = KUTACC_DTYPE_BF16, g.path = KUTACC_HIP_PATH_AUTO, g.batches = 1;
@@ -354,14 +364,7 @@ int kutacc_hip_triangle_multiplication(const kutacc_hip_triangle_multiplication_
     }
     // 6. output projection of the normalised centre, times sigmoid(gate), added to the pair activation: one kernel
     //    when the shape allows, else projection, gating and residual as three passes
-    if (rc == 0 && norm_inside) {
-        rc = kutacc_launch::row_projection_projected_gate_residual(center_cf, plane, a->output_w, a->output_b, act, cz,
-                                                                   a->gating_w, a->gating_b, a->pair_act, cz, rows, s,
-                                                                   a->ln_center_gamma, a->ln_center_beta, a->ln_eps);
-    } else if (rc == 0 && gate_inside) {
-        rc = kutacc_launch::row_projection_projected_gate_residual(center, ci, a->output_w, a->output_b, act, cz, a->gating_w,
-                                                                   a->gating_b, a->pair_act, cz, rows, s);
-    } else if (rc == 0) {
+    if (rc == 0) {
         rc = kutacc_launch::row_projection_gated_residual(center, ci, a->output_w, a->output_b, gate, cz, a->pair_act, cz, rows,
                                                           cz, ci, s);
         if (rc == KUTACC_HIP_EUNSUPPORTED) {

@@ -2281,245 +2281,6 @@ __global__ __launch_bounds__(C == 128 ? 256 : 512, C == 128 ? 2 : 1) void output
     }
 }
 
-// out[t][:] += bf16( bf16(x[t] . Wo^T + bo) * sigmoid(bf16(y[t] . Wg^T + bg)) ) for rows of 128 features in and out: the last
-// three steps of the triangle multiplication with the gate projection folded in (reference
-// src/attention/triangle_multiplication.cpp:106-150: gate = Linear(normalised input), out = Linear(normalised centre),
-// out * sigmoid(gate), residual).  The gate tensor never exists in memory: against the separate gate projection this
-// saves its write, its read and a launch.  Same structure as output_projection_kernel: both weight slabs stay in LDS
-// (64 KB), every wave streams an equal range of rows 32 at a time, rows in and out as whole cache lines through its
-// panel, the next step's rows requested while the current one is multiplied.  The gate goes first: its accumulators,
-// rounded to bf16 as the reference stores them, wait as 32 packed registers for the projection of the same rows.
-//
-// X_CHANNEL_FIRST: x is the centre of the triangle multiplication as the equation leaves it, channel-first ([128, M],
-// channel stride x_ld) and not yet normalised.  The kernel then takes the place of the channel-first LayerNorm too: a
-// wave loads 64 channels x 32 positions (64 contiguous bytes per channel), stores them in its panel as they lie, gets
-// its MFMA fragments -- 8 consecutive channels of one position per lane -- with the LDS transposing read, and normalises
-// them in registers (a position's 128 channels sit in two lanes; the arithmetic is that of the LayerNorm kernels,
-// reference src/normalization/layernorm_kernel.h:21-53, the result rounded to bf16 as the tensor it replaces was).
-template <bool X_CHANNEL_FIRST>
-__global__ __launch_bounds__(256, 2) void projected_gate_residual_kernel(
-    const bf16_t *__restrict__ x, int64_t x_ld, const bf16_t *__restrict__ wo, const float *__restrict__ bo,
-    const bf16_t *__restrict__ y, int64_t y_ld, const bf16_t *__restrict__ wg, const float *__restrict__ bg,
-    bf16_t *__restrict__ out, int64_t out_ld, int64_t M, int rows_per_wave, const float *__restrict__ ln_gamma,
-    const float *__restrict__ ln_beta, float ln_eps)
-{
-    constexpr int C = 128, CK = C / 16;
-    extern __shared__ uint4 lds[]; // [Wo, Wg][4 feature blocks][CK][64 lanes], then 4 panels of 256
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6); // uniform
-    uint4 *panel = lds + 2 * 4 * CK * 64 + wave * 256;
-    // The workgroup owns 4 * rows_per_wave consecutive rows and its waves take the 32-row steps of that range in turn
-    // (wave w: steps w, w + 4, ...): neighbouring steps run at the same time, so the two 64-byte halves of a 128-byte
-    // line of the channel-first tensor (32 positions each) are asked for together instead of a whole step apart, by
-    // which time the line has left the L2.
-    // Rows are addressed relative to the workgroup's first one, by 32-bit byte offsets from uniform bases; positions of
-    // the channel-first tensor by 32-bit offsets from its first element (the launcher checks that both fit).
-    const int64_t start = (int64_t)blockIdx.x * 4 * rows_per_wave;
-    const int64_t stop = start + 4 * rows_per_wave < M ? start + 4 * rows_per_wave : M;
-    const int64_t first = start + 32 * wave; // this wave's first step
-    const int last_rel = (int)(stop - 1 - start);
-    const bf16_t *y_w = y + start * y_ld, *x_w = x + start * x_ld;
-    const uint32_t y_pitch = (uint32_t)y_ld, x_pitch = (uint32_t)x_ld, m32 = (uint32_t)M;
-    // the first 64 features of the next step's rows of y and x are requested a step ahead; the second 64 at the top of
-    // their own step, behind the first (four sets of registers held across a step do not fit)
-    // channel-first x: 64 channels (from c0) x 32 positions (from p0), lane -> channel c0 + 16 i + lane / 4, positions
-    // p0 + 8 (lane & 3) .. +7; a chunk past the end of the tensor repeats the last one (M is a multiple of 8)
-    auto load_cf = [&](int c0, int64_t p0, int ln) {
-        uint32_t pos = (uint32_t)p0 + 8u * (ln & 3);
-        pos = pos + 8u <= m32 ? pos : m32 - 8u;
-        PanelRegs t;
-        const char *src = reinterpret_cast<const char *>(x + (int64_t)c0 * x_ld);
-        const uint32_t off = 2u * (__umul24((uint32_t)(ln >> 2), x_pitch) + pos), step = 32u * x_pitch; // 16 channels on
-        t.r0 = *reinterpret_cast<const uint4 *>(src + off);
-        t.r1 = *reinterpret_cast<const uint4 *>(src + (off + step));
-        t.r2 = *reinterpret_cast<const uint4 *>(src + (off + 2u * step));
-        t.r3 = *reinterpret_cast<const uint4 *>(src + (off + 3u * step));
-        return t;
-    };
-    PanelRegs ya, xa;
-    if (first < stop) {
-        ya = panel_load_near(y_w, y_pitch, 32 * wave, last_rel, 0, lane);
-        if constexpr (X_CHANNEL_FIRST) {
-            xa = load_cf(0, first, lane);
-        } else {
-            xa = panel_load_near(x_w, x_pitch, 32 * wave, last_rel, 0, lane);
-        }
-    }
-    {
-        constexpr int PER = 2 * 4 * CK * 64 / 256;
-        uint4 wreg[PER];
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int idx = tid + i * 256;
-            const int mat = idx / (4 * CK * 64), nb_ = (idx / (CK * 64)) % 4, ks = (idx >> 6) % CK, ln = idx & 63;
-            const bf16_t *w = mat ? wg : wo;
-            wreg[i] = *reinterpret_cast<const uint4 *>(w + (int64_t)(nb_ * 32 + (ln & 31)) * C + ks * 16 + (ln >> 5) * 8);
-        }
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            lds[tid + i * 256] = wreg[i];
-        }
-    }
-    __syncthreads();
-    const uint4 *wo_s = lds, *wg_s = lds + 4 * CK * 64;
-    for (int64_t rbase = first; rbase < stop; rbase += 128) {
-        const int rel0 = (int)(rbase - start);
-        int lv = lane; // opaque: addresses and panel offsets are formed per step, not kept across the loop
-        asm volatile("" : "+v"(lv));
-        const int rv = lv & 31, gv = lv >> 5;
-        const int rnext = rbase + 128 < stop ? rel0 + 128 : rel0; // clamped: one harmless re-read at the end
-        // ---- gate: 128 features of the 32 rows, rounded to bf16, kept in accumulator order ----
-        bf16x8 gate[4][2];
-        {
-            bf16x8 yf[CK];
-            const PanelRegs yb = panel_load_near(y_w + 64, y_pitch, rel0, last_rel, 0, lv);
-            panel_store(panel, lv, ya);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                yf[k] = as_bf16x8(panel[panel_slot(rv, 2 * k + gv)]);
-            }
-            panel_store(panel, lv, yb);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                yf[4 + k] = as_bf16x8(panel[panel_slot(rv, 2 * k + gv)]);
-            }
-            ya = panel_load_near(y_w, y_pitch, rnext, last_rel, 0, lv);
-            const float *gbias = bg + 4 * gv;
-#pragma unroll
-            for (int nb_ = 0; nb_ < 4; ++nb_) {
-                f32x16 acc = zero16();
-#pragma unroll
-                for (int ks = 0; ks < CK; ++ks) {
-                    acc = mfma(as_bf16x8(wg_s[(nb_ * CK + ks) * 64 + lv]), yf[ks], acc);
-                }
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    const f32x4 bv = *reinterpret_cast<const f32x4 *>(gbias + nb_ * 32 + 8 * a);
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        gate[nb_][a >> 1][4 * (a & 1) + c] = (bf16_t)(acc[4 * a + c] + bv[c]);
-                    }
-                }
-            }
-        }
-        // ---- projection of the same rows, gating, residual ----
-        bf16x8 xf[CK];
-        if constexpr (X_CHANNEL_FIRST) {
-            const PanelRegs xb = load_cf(64, rbase, lv);
-            // the panel holds [64 channels][32 positions], 64 bytes per channel, lane ln's pieces at slots ln + 64 i
-            const lds_char *tile = (const lds_char *)panel;
-            const int tr_off = ((lv >> 5) * 8 + ((lv & 15) >> 2)) * 64 + (4 * ((lv >> 4) & 1) + (lv & 3)) * 8;
-            panel[lv] = xa.r0, panel[64 + lv] = xa.r1, panel[128 + lv] = xa.r2, panel[192 + lv] = xa.r3;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                xf[k] = lds_transposed_fragment(tile + tr_off + k * 1024, tile + tr_off + k * 1024 + 256);
-            }
-            panel[lv] = xb.r0, panel[64 + lv] = xb.r1, panel[128 + lv] = xb.r2, panel[192 + lv] = xb.r3;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                xf[4 + k] = lds_transposed_fragment(tile + tr_off + k * 1024, tile + tr_off + k * 1024 + 256);
-            }
-            xa = load_cf(0, rbase + 128 < stop ? rbase + 128 : rbase, lv);
-            // LayerNorm over the 128 channels of the lane's position: this lane holds channels 16 k + 8 g + 0..7
-            float x0 = to_f32(xf[0][0]);
-            x0 = __shfl(x0, lv & 31, 64); // channel 0 sits in the lane of the lower half
-            float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-            for (int k = 0; k < CK; ++k) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float d = to_f32(xf[k][e]) - x0;
-                    s1 += d;
-                    s2 = fmaf(d, d, s2);
-                }
-            }
-            s1 = half_swap_sum(s1), s2 = half_swap_sum(s2);
-            const float nch = (float)C;
-            const float mean = s1 / nch + x0;
-            const float var = fmaxf((s2 - s1 * s1 / nch) / nch, 0.f);
-            const float rstd = 1.0f / sqrtf(var + ln_eps);
-            const float shift = -rstd * mean;
-#pragma unroll
-            for (int k = 0; k < CK; ++k) {
-                const float *gm = ln_gamma + 16 * k + 8 * gv, *bt = ln_beta + 16 * k + 8 * gv;
-                const f32x4 g0 = *reinterpret_cast<const f32x4 *>(gm), g1 = *reinterpret_cast<const f32x4 *>(gm + 4);
-                const f32x4 b0 = *reinterpret_cast<const f32x4 *>(bt), b1 = *reinterpret_cast<const f32x4 *>(bt + 4);
-                bf16x8 o;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    o[e] = (bf16_t)fmaf(fmaf(to_f32(xf[k][e]), rstd, shift), g0[e], b0[e]);
-                    o[4 + e] = (bf16_t)fmaf(fmaf(to_f32(xf[k][4 + e]), rstd, shift), g1[e], b1[e]);
-                }
-                xf[k] = o;
-            }
-        } else {
-            const PanelRegs xb = panel_load_near(x_w + 64, x_pitch, rel0, last_rel, 0, lv);
-            panel_store(panel, lv, xa);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                xf[k] = as_bf16x8(panel[panel_slot(rv, 2 * k + gv)]);
-            }
-            panel_store(panel, lv, xb);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                xf[4 + k] = as_bf16x8(panel[panel_slot(rv, 2 * k + gv)]);
-            }
-            xa = panel_load_near(x_w, x_pitch, rnext, last_rel, 0, lv);
-        }
-        const float *bias = bo + 4 * gv;
-#pragma unroll
-        for (int half = 0; half < 2; ++half) { // 64 output features per panel
-            uint4 zq[4]; // the rows of `out` to add to, requested before the MFMAs
-            char *out_w = reinterpret_cast<char *>(out + start * out_ld + half * 64);
-            uint32_t out_off[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                int rel = rel0 + 8 * i + (lv >> 3);
-                rel = rel < last_rel ? rel : last_rel;
-                out_off[i] = __umul24((uint32_t)rel, 2u * (uint32_t)out_ld) + 16u * (lv & 7);
-                zq[i] = *reinterpret_cast<const uint4 *>(out_w + out_off[i]);
-            }
-            f32x16 acc[2];
-            acc[0] = zero16(), acc[1] = zero16();
-#pragma unroll
-            for (int ks = 0; ks < CK; ++ks) {
-#pragma unroll
-                for (int n = 0; n < 2; ++n) {
-                    acc[n] = mfma(as_bf16x8(wo_s[((2 * half + n) * CK + ks) * 64 + lv]), xf[ks], acc[n]);
-                }
-            }
-#pragma unroll
-            for (int n = 0; n < 2; ++n) {
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    const f32x4 bv = *reinterpret_cast<const f32x4 *>(bias + (2 * half + n) * 32 + 8 * a);
-                    bf16x4 ov;
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        // bf16(out) * sigmoid(bf16(gate)), rounded to bf16: the reference's rounding points
-                        const float o = to_f32((bf16_t)(acc[n][4 * a + c] + bv[c]));
-                        const float gt = to_f32(gate[2 * half + n][a >> 1][4 * (a & 1) + c]);
-                        ov[c] = (bf16_t)(o * sigmoid_fast(gt));
-                    }
-                    *(reinterpret_cast<bf16x4 *>(panel + panel_slot(rv, n * 4 + a)) + gv) = ov;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int prow_ = 8 * i + (lv >> 3);
-                const bf16x8 u = as_bf16x8(panel[panel_slot(prow_, lv & 7)]), z = as_bf16x8(zq[i]);
-                bf16x8 res;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    res[e] = (bf16_t)(to_f32(z[e]) + to_f32(u[e]));
-                }
-                if (rel0 + prow_ <= last_rel) {
-                    *reinterpret_cast<uint4 *>(out_w + out_off[i]) = as_uint4(res);
-                }
-            }
-        }
-    }
-}
-
 // Pair bias [H, S, S] -> fragment-major order: for head h, query block j and key tile t the two B
 // operands of the selector MFMAs, [h][j][t][2][64 lanes] x 16 bytes, so that a wave of the attention
 // kernels fetches the pair bias of a tile with two contiguous 1 KB loads straight into registers.
@@ -3072,55 +2833,6 @@ int row_projection_gated_residual(const void *a, int64_t a_ld, const void *w, co
     kutacc_prof::KernelTimer t("output_projection_kernel<gated residual>", 2.0 * (double)m * (double)n * (double)k, stream);
     return k == 128 ? launch_output_projection<128, EPILOGUE_GATED_RESIDUAL>(a, a_ld, w, bias, acc, acc_ld, m, n, stream, gate, gate_ld)
                     : launch_output_projection<256, EPILOGUE_GATED_RESIDUAL>(a, a_ld, w, bias, acc, acc_ld, m, n, stream, gate, gate_ld);
-}
-
-// acc[m, 128] += bf16(bf16(a . w^T + bias) * sigmoid(bf16(y . wg^T + bg))), a and y rows of 128 features: the gate
-// projection inside the kernel (no gate tensor)
-bool row_projection_projected_gate_supports(const void *a, int64_t a_ld, const void *w, const float *bias, const void *y,
-                                            int64_t y_ld, const void *wg, const float *bg, const void *acc, int64_t acc_ld,
-                                            int64_t m, int64_t n, int64_t k, int64_t ky)
-{
-    // the kernel addresses rows by 32-bit byte offsets: of a wave's rows from its first one, of a channel-first `a`
-    // (a_ld >= m) from its first element
-    const int64_t lim = (int64_t)1 << 31;
-    const bool near = m < (1 << 23) && a_ld > 0 && a_ld < (1 << 23) && y_ld > 0 && acc_ld > 0 && m * y_ld * 2 < lim &&
-                      m * acc_ld * 2 < lim && (a_ld >= m || m * a_ld * 2 < lim);
-    return k == 128 && ky == 128 && n == 128 && m > 0 && near && bias && bg && y && wg && a_ld % 8 == 0 &&
-           y_ld % 8 == 0 && acc_ld % 8 == 0 && aligned(a, 16) && aligned(w, 16) && aligned(bias, 16) && aligned(y, 16) &&
-           aligned(wg, 16) && aligned(bg, 16) && aligned(acc, 16);
-}
-
-// ln_gamma != nullptr: `a` is channel-first ([128, m], channel stride a_ld, m a multiple of 8) and not yet normalised;
-// the kernel applies LayerNorm(ln_gamma, ln_beta, ln_eps) over its 128 channels on the way in
-int row_projection_projected_gate_residual(const void *a, int64_t a_ld, const void *w, const float *bias, const void *y,
-                                           int64_t y_ld, const void *wg, const float *bg, void *acc, int64_t acc_ld, int64_t m,
-                                           hipStream_t stream, const float *ln_gamma, const float *ln_beta, float ln_eps)
-{
-    if (!row_projection_projected_gate_supports(a, a_ld, w, bias, y, y_ld, wg, bg, acc, acc_ld, m, 128, 128, 128)) {
-        return KUTACC_HIP_EUNSUPPORTED;
-    }
-    const bool cf = ln_gamma != nullptr;
-    if (cf && (!ln_beta || m % 8 != 0 || m < 8 || !aligned(ln_gamma, 16) || !aligned(ln_beta, 16))) {
-        return KUTACC_HIP_EUNSUPPORTED;
-    }
-    constexpr size_t lds_bytes = (size_t)2 * 4 * 8 * 64 * 16 + 4 * 4096;
-    static size_t configured[2][KUTACC_DEVICE_SLOTS] = {};
-    if (const int rc = cf ? opt_in_lds(projected_gate_residual_kernel<true>, lds_bytes, configured[1])
-                          : opt_in_lds(projected_gate_residual_kernel<false>, lds_bytes, configured[0])) {
-        return rc;
-    }
-    kutacc_prof::KernelTimer t(cf ? "projected_gate_residual_kernel<channel-first>" : "projected_gate_residual_kernel",
-                               4.0 * (double)m * 128.0 * 128.0, stream);
-    const int64_t tiles = (m + 31) / 32;
-    int64_t gx = (tiles + 3) / 4;
-    const int64_t cap = (int64_t)num_cus() * 2; // two workgroups per CU, each wave with an equal share of the rows
-    gx = gx > cap ? cap : gx;
-    const int64_t rpw = ((m + gx * 4 - 1) / (gx * 4) + 7) / 8 * 8; // a workgroup's range, 4 rpw rows, is whole 32-row steps
-    auto kern = cf ? projected_gate_residual_kernel<true> : projected_gate_residual_kernel<false>;
-    kern<<<dim3((unsigned)gx), 256, lds_bytes, stream>>>((const bf16_t *)a, a_ld, (const bf16_t *)w, bias, (const bf16_t *)y, y_ld,
-                                                         (const bf16_t *)wg, bg, (bf16_t *)acc, acc_ld, m, (int)rpw, ln_gamma,
-                                                         ln_beta, ln_eps);
-    return kutacc_hip_status(hipGetLastError());
 }
 
 } // namespace kutacc_launch

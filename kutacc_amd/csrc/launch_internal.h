@@ -132,16 +132,6 @@ int row_projection(const void *a, int64_t a_ld, const void *w, const float *bias
 int row_projection_gated_residual(const void *a, int64_t a_ld, const void *w, const float *bias, const void *gate,
                                   int64_t gate_ld, void *acc, int64_t acc_ld, int64_t m, int64_t n, int64_t k,
                                   hipStream_t stream);
-// the same with the gate projected inside the kernel from rows y of 128 features (no gate tensor); 128 features in and out
-bool row_projection_projected_gate_supports(const void *a, int64_t a_ld, const void *w, const float *bias, const void *y,
-                                            int64_t y_ld, const void *wg, const float *bg, const void *acc, int64_t acc_ld,
-                                            int64_t m, int64_t n, int64_t k, int64_t ky);
-// ln_gamma != nullptr: `a` is channel-first ([128, m], channel stride a_ld) and is normalised over its channels on the way in
-int row_projection_projected_gate_residual(const void *a, int64_t a_ld, const void *w, const float *bias, const void *y,
-                                           int64_t y_ld, const void *wg, const float *bg, void *acc, int64_t acc_ld, int64_t m,
-                                           hipStream_t stream, const float *ln_gamma = nullptr, const float *ln_beta = nullptr,
-                                           float ln_eps = 0.f);
-
 // global_attention.hip
 int global_attention(const kutacc_hip_global_attention_args_t &args, hipStream_t stream);
 
@@ -149,6 +139,9 @@ int global_attention(const kutacc_hip_global_attention_args_t &args, hipStream_t
 // `second`: a second gated projection of the same B and mask to run in the same launch (KUTACC_HIP_EUNSUPPORTED, with
 // nothing launched, when the two cannot share one: the caller then makes two calls)
 int pair_gemm(const kutacc_hip_gemm_args_t &args, hipStream_t stream, const kutacc_hip_gemm_args_t *second = nullptr);
+int gated_projection_mode(); // 0: the default rule (see pair_gemm_tuning)
+int triangle_equation(const void *left, const void *right, void *centre, int64_t n, int64_t np, int64_t plane, int64_t channels, bool incoming,
+                      hipStream_t stream);
 bool transition_fused_supports(int64_t rows, int64_t c_o, int64_t c_i, const void *x, const void *w1, const float *b1,
                                const void *w2, const float *b2, const void *out);
 int transition_fused(const void *x, const void *w1, const float *b1, const void *w2, const float *b2, void *out,
@@ -157,6 +150,12 @@ int transition_block_fused(void *act, const float *ln_gamma, const float *ln_bet
                            const void *w2, const float *b2, int64_t rows, int64_t c_o, int64_t c_i, hipStream_t stream);
 int sigmoid_gate_rows(void *out, int64_t out_s0, int64_t out_s1, const void *gate, int64_t gate_s0, int64_t gate_s1,
                       int64_t n0, int64_t n1, int64_t size, hipStream_t stream);
+
+// triangle_multiplication.hip: the block's LayerNorm + gated projections, and its centre LayerNorm + gated output projection +
+// residual, at 128 channels; planes of n rows of np positions, np = n rounded up to 8, `plane` elements apart
+bool triangle_ends_support(const kutacc_hip_triangle_multiplication_args_t &args);
+int triangle_front(const kutacc_hip_triangle_multiplication_args_t &args, void *left, void *right, int64_t np, int64_t plane, hipStream_t stream);
+int triangle_back(const kutacc_hip_triangle_multiplication_args_t &args, const void *centre, int64_t np, int64_t plane, hipStream_t stream);
 
 // glue_kernels.hip
 int mask_bias(const void *mask, void *bias, int64_t n0, int64_t n1, int transposed, int32_t dtype, hipStream_t stream);

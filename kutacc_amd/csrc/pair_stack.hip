@@ -53,6 +53,7 @@ struct GemmParams {
     const bf16_t *mask; // gated epilogue: multiplier per column of C
     int64_t mask_sb;
     int M, N, K, batches;
+    int a_rows, b_rows; // rows of A and B that may be loaded (M and N, or more where their padding may be read)
     int bias_axis; // 0 none, 1 per column n, 2 per row m
     int relu;
     int MT, NT; // tiles along m and n
@@ -192,18 +193,18 @@ __global__ __launch_bounds__(256, (A_MMAJOR && B_MMAJOR) ? 4 : 3) void pair_gemm
 
     auto fetch_a = [&](int k0) -> PanelRegs {
         if constexpr (A_MMAJOR) {
-            return load_mmajor(a, p.a_sk, m0 + 64 * (wave & 1), p.M, k0 + 32 * (wave >> 1), p.K, lane);
+            return load_mmajor(a, p.a_sk, m0 + 64 * (wave & 1), p.a_rows, k0 + 32 * (wave >> 1), p.K, lane);
         } else if constexpr (GATED) {
-            return load_kmajor(wave < 2 ? a : a_gate, p.a_sm, m0 + 32 * (wave & 1), p.M - 1, k0, p.K, lane);
+            return load_kmajor(wave < 2 ? a : a_gate, p.a_sm, m0 + 32 * (wave & 1), p.a_rows - 1, k0, p.K, lane);
         } else {
-            return load_kmajor(a, p.a_sm, m0 + 32 * wave, p.M - 1, k0, p.K, lane);
+            return load_kmajor(a, p.a_sm, m0 + 32 * wave, p.a_rows - 1, k0, p.K, lane);
         }
     };
     auto fetch_b = [&](int k0) -> PanelRegs {
         if constexpr (B_MMAJOR) {
-            return load_mmajor(b, p.b_sk, n0 + 64 * (wave & 1), p.N, k0 + 32 * (wave >> 1), p.K, lane);
+            return load_mmajor(b, p.b_sk, n0 + 64 * (wave & 1), p.b_rows, k0 + 32 * (wave >> 1), p.K, lane);
         } else {
-            return load_kmajor(b, p.b_sn, n0 + 32 * wave, p.N - 1, k0, p.K, lane);
+            return load_kmajor(b, p.b_sn, n0 + 32 * wave, p.b_rows - 1, k0, p.K, lane);
         }
     };
     auto park = [&](uint4 *stage, const PanelRegs &ra, const PanelRegs &rb) {
@@ -1352,20 +1353,17 @@ __global__ __launch_bounds__(256 * SIDES, 2 / SIDES) void gated_projection_kerne
 // requested RING - 1 steps ahead) and the mask (128 bytes, each wave's own copy), multiplies, gates and writes 32
 // channels x 128 bytes.  Eight equal shares of every step, an eighth of the LDS reads.  Same arithmetic in the same
 // order as the kernel above: the results are bit-identical.
-template <int SIDES>
-__global__ __launch_bounds__(256 * SIDES, 2 / SIDES) void gated_projection_blocks_kernel(const bf16_t *__restrict__ x, GatedSide s0, GatedSide s1,
-                                                                                        const bf16_t *__restrict__ mask, int64_t out_ld,
-                                                                                        int64_t n_pos, int steps_per_group)
+__global__ __launch_bounds__(256, 2) void gated_projection_blocks_kernel(const bf16_t *__restrict__ x, GatedSide sd, const bf16_t *__restrict__ mask,
+                                                                         int64_t out_ld, int64_t n_pos, int steps_per_group)
 {
     typedef __attribute__((address_space(3))) void *lds_ptr;
-    constexpr int C = 128, CK = C / 16, WAVES = 4 * SIDES, RING = SIDES == 2 ? 4 : 3, UNITS = 16 / WAVES;
+    constexpr int C = 128, CK = C / 16, WAVES = 4, RING = 3, UNITS = 16 / WAVES;
     constexpr int STAGE_SLOTS = 1024; // 64 positions x 256 bytes
     constexpr int WAVE_SLOTS = 256 + RING * 16; // a panel for the way out, and RING mask rows of 256 bytes
     extern __shared__ uint4 lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rv = lane & 31, gv = lane >> 5;
-    const GatedSide &sd = (SIDES == 2 && wave >= 4) ? s1 : s0;
-    const int cb = wave & 3; // this wave's 32 channels
+    const int cb = wave; // this wave's 32 channels
     uint4 *panel = lds + RING * STAGE_SLOTS + wave * WAVE_SLOTS;
     const uint4 *mask_rows = panel + 256;
 
@@ -1514,20 +1512,10 @@ __global__ __launch_bounds__(256 * SIDES, 2 / SIDES) void gated_projection_block
         // flight: the requests of the steps after it (UNITS + 1 each) and four stores per step gone by.  Behind the
         // barrier every wave's part of it has, and every wave has left this step's stage.
         const int64_t gone = step - first;
-        if constexpr (RING == 4) {
-            if (gone == 0) {
-                asm volatile("s_waitcnt vmcnt(10)\n\ts_barrier" ::: "memory");
-            } else if (gone == 1) {
-                asm volatile("s_waitcnt vmcnt(14)\n\ts_barrier" ::: "memory");
-            } else {
-                asm volatile("s_waitcnt vmcnt(18)\n\ts_barrier" ::: "memory");
-            }
+        if (gone == 0) {
+            asm volatile("s_waitcnt vmcnt(9)\n\ts_barrier" ::: "memory");
         } else {
-            if (gone == 0) {
-                asm volatile("s_waitcnt vmcnt(9)\n\ts_barrier" ::: "memory");
-            } else {
-                asm volatile("s_waitcnt vmcnt(13)\n\ts_barrier" ::: "memory");
-            }
+            asm volatile("s_waitcnt vmcnt(13)\n\ts_barrier" ::: "memory");
         }
         slot = ring(slot + 1);
     }
@@ -1721,29 +1709,24 @@ hipError_t launch_gated_projection(const kutacc_hip_gemm_args_t &g, const kutacc
     return hipGetLastError();
 }
 
-template <int SIDES>
-hipError_t launch_gated_projection_blocks(const kutacc_hip_gemm_args_t &g, const kutacc_hip_gemm_args_t *second, hipStream_t stream)
+hipError_t launch_gated_projection_blocks(const kutacc_hip_gemm_args_t &g, hipStream_t stream)
 {
-    constexpr int WAVES = 4 * SIDES, RING = SIDES == 2 ? 4 : 3;
+    constexpr int WAVES = 4, RING = 3;
     constexpr size_t lds_bytes = (size_t)(RING * 1024 + WAVES * (256 + RING * 16)) * 16;
     static size_t configured[KUTACC_DEVICE_SLOTS] = {};
     static int cu_table[KUTACC_DEVICE_SLOTS] = {};
-    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&gated_projection_blocks_kernel<SIDES>), lds_bytes, configured)) {
+    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&gated_projection_blocks_kernel), lds_bytes, configured)) {
         return e;
     }
     const int cus = kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, cu_table);
-    // eight resident waves per CU (two workgroups of four, or one of eight); every workgroup an equal run of steps
+    // two resident workgroups per CU; every workgroup an equal run of steps
     const int64_t steps = (g.n + 63) / 64;
-    const int64_t cap = (int64_t)cus * (2 / SIDES);
+    const int64_t cap = (int64_t)cus * 2;
     const int64_t groups = steps < cap ? steps : cap;
     const int64_t per_group = (steps + groups - 1) / groups;
-    const GatedSide s0 = {(const bf16_t *)g.a, (const bf16_t *)g.a_gate, g.bias, g.bias_gate, (bf16_t *)g.c};
-    GatedSide s1 = s0;
-    if (SIDES == 2) {
-        s1 = GatedSide{(const bf16_t *)second->a, (const bf16_t *)second->a_gate, second->bias, second->bias_gate, (bf16_t *)second->c};
-    }
-    gated_projection_blocks_kernel<SIDES><<<dim3((unsigned)((steps + per_group - 1) / per_group)), 64 * WAVES, lds_bytes, stream>>>(
-        (const bf16_t *)g.b, s0, s1, (const bf16_t *)g.mask, g.c_stride_m, g.n, (int)per_group);
+    const GatedSide side = {(const bf16_t *)g.a, (const bf16_t *)g.a_gate, g.bias, g.bias_gate, (bf16_t *)g.c};
+    gated_projection_blocks_kernel<<<dim3((unsigned)((steps + per_group - 1) / per_group)), 64 * WAVES, lds_bytes, stream>>>(
+        (const bf16_t *)g.b, side, (const bf16_t *)g.mask, g.c_stride_m, g.n, (int)per_group);
     return hipGetLastError();
 }
 
@@ -1831,6 +1814,47 @@ int pair_gemm_tuning(const char *name, const char *value)
     return KUTACC_HIP_EINVAL;
 }
 
+// A plain product with both operands in the orientation `mmajor` on the kernels with large tiles, where its sides are whole
+// ones and there are enough of them; KUTACC_HIP_EUNSUPPORTED, with nothing launched, where not.
+static int large_tiles(GemmParams &p, bool mmajor, double flops, hipStream_t stream)
+{
+    const int64_t lda = mmajor ? p.a_sk : p.a_sm, ldb = mmajor ? p.b_sk : p.b_sn;
+    const int64_t M = p.M, N = p.N;
+    // whole k-steps, and lane offsets within 32 bits: the kernels' addresses are a uniform pointer plus a lane constant
+    const int tile_mode = g_big_tile_mode.load();
+    if (p.K % KSTEP != 0 || lda >= (1 << 26) || ldb >= (1 << 26) || tile_mode == 2) {
+        return KUTACC_HIP_EUNSUPPORTED;
+    }
+    // (the direct kernel's lane offsets span the tile's 256 rows: pitches below 2^22 elements keep them in 32 bits)
+    if ((tile_mode == 4 || tile_mode == 0) && lda < (1 << 22) && ldb < (1 << 22) && M % BIG_TILE == 0 && N % BIG_TILE == 0 &&
+        p.K >= 3 * DIRECT_KSTEP && M / BIG_TILE * (N / BIG_TILE) * p.batches <= INT32_MAX &&
+        (tile_mode == 4 || M / BIG_TILE * (N / BIG_TILE) * p.batches >= BIG_TILE_MIN_WORKGROUPS / 2)) {
+        p.MT = (int)(M / BIG_TILE), p.NT = (int)(N / BIG_TILE);
+        const int64_t blocks = (int64_t)p.MT * p.NT * p.batches;
+        kutacc_prof::KernelTimer t(mmajor ? "pair_gemm_direct_kernel<m-major>" : "pair_gemm_direct_kernel", flops, stream);
+        return kutacc_hip_status(mmajor ? launch_direct_tiles<true>(p, blocks, stream) : launch_direct_tiles<false>(p, blocks, stream));
+    }
+    // 256 x 256 tiles where every CU gets at least four; else 192 x 192 where every CU gets at least two
+    for (const int side : {BIG_TILE, 192}) {
+        const bool forced = tile_mode == (side == BIG_TILE ? 1 : 3);
+        if (M % side != 0 || N % side != 0 || (!forced && tile_mode != 0)) {
+            continue;
+        }
+        p.MT = (int)(M / side), p.NT = (int)(N / side);
+        const int64_t blocks = (int64_t)p.MT * p.NT * p.batches;
+        const int64_t enough = side == BIG_TILE ? BIG_TILE_MIN_WORKGROUPS : BIG_TILE_MIN_WORKGROUPS / 2;
+        if (blocks <= INT32_MAX && (blocks >= enough || forced)) {
+            kutacc_prof::KernelTimer t(side == BIG_TILE ? (mmajor ? "pair_gemm_big_kernel<m-major>" : "pair_gemm_big_kernel")
+                                                        : (mmajor ? "pair_gemm_big_kernel<m-major, 192>" : "pair_gemm_big_kernel<192>"),
+                                       flops, stream);
+            const hipError_t e = side == BIG_TILE ? (mmajor ? launch_big_tiles<true, 4>(p, blocks, stream) : launch_big_tiles<false, 4>(p, blocks, stream))
+                                                  : (mmajor ? launch_big_tiles<true, 3>(p, blocks, stream) : launch_big_tiles<false, 3>(p, blocks, stream));
+            return kutacc_hip_status(e);
+        }
+    }
+    return KUTACC_HIP_EUNSUPPORTED;
+}
+
 int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_hip_gemm_args_t *second)
 {
     if (g.m <= 0 || g.n <= 0 || g.k <= 0 || g.batches <= 0 || !g.a || !g.b || !g.c || g.dtype != KUTACC_DTYPE_BF16) {
@@ -1851,6 +1875,7 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
     p.c_sm = g.c_stride_m, p.c_sb = g.c_stride_batch;
     p.bias = g.bias, p.bias_gate = g.bias_gate, p.mask = (const bf16_t *)g.mask, p.mask_sb = g.mask_stride_batch;
     p.M = (int)g.m, p.N = (int)g.n, p.K = (int)g.k, p.batches = (int)g.batches;
+    p.a_rows = p.M, p.b_rows = p.N;
     p.bias_axis = g.bias_axis, p.relu = g.relu ? 1 : 0;
     p.a_alt = p.a_gate_alt = nullptr, p.bias_alt = p.bias_gate_alt = nullptr, p.c_alt = nullptr;
 
@@ -1889,13 +1914,9 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
         if (!same || !gated || g.path == KUTACC_HIP_PATH_GENERIC) {
             return KUTACC_HIP_EUNSUPPORTED;
         }
-        if (dedicated) { // both sides in one pass over the activation
-            if (gated_mode == 2) {
-                kutacc_prof::KernelTimer t("gated_projection_kernel<2>", 8.0 * (double)g.m * (double)g.n * (double)g.k, stream);
-                return kutacc_hip_status(launch_gated_projection<2>(g, second, stream));
-            }
-            kutacc_prof::KernelTimer t("gated_projection_blocks_kernel<2>", 8.0 * (double)g.m * (double)g.n * (double)g.k, stream);
-            return kutacc_hip_status(launch_gated_projection_blocks<2>(g, second, stream));
+        if (dedicated && gated_mode == 2) { // both sides in one pass over the activation
+            kutacc_prof::KernelTimer t("gated_projection_kernel<2>", 8.0 * (double)g.m * (double)g.n * (double)g.k, stream);
+            return kutacc_hip_status(launch_gated_projection<2>(g, second, stream));
         }
         // (one that fits a dedicated kernel by itself: the caller runs the two separately)
         if (!mfma_ok || (gated_mode != 3 && gated_projection_fits(g))) {
@@ -1912,7 +1933,7 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
             return kutacc_hip_status(launch_gated_projection<1>(g, nullptr, stream));
         }
         kutacc_prof::KernelTimer t("gated_projection_blocks_kernel", 4.0 * (double)g.m * (double)g.n * (double)g.k, stream);
-        return kutacc_hip_status(launch_gated_projection_blocks<1>(g, nullptr, stream));
+        return kutacc_hip_status(launch_gated_projection_blocks(g, stream));
     }
     // rows of 128 or 256 features against a dense weight matrix: the attention's output-projection kernel keeps
     // the weight slab in LDS and streams the rows, which suits these HBM-bound shapes better than square tiles
@@ -1931,36 +1952,10 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
         pair_gemm_scalar_kernel<<<dim3((unsigned)blocks), 256, 0, stream>>>(p);
         return kutacc_hip_status(hipGetLastError());
     }
-    // (whole tiles and k-steps, and lane offsets within 32 bits: the kernel's addresses are a uniform pointer plus a lane constant)
-    const int tile_mode = g_big_tile_mode.load();
-    if (!gated && am == bm && g.bias_axis == 0 && !g.relu && g.k % KSTEP == 0 && (am ? g.a_stride_k : g.a_stride_m) < (1 << 26) &&
-        (bm ? g.b_stride_k : g.b_stride_n) < (1 << 26) && tile_mode != 2) {
-        // (the direct kernel's lane offsets span the tile's 256 rows: pitches below 2^22 elements keep them in 32 bits)
-        if ((tile_mode == 4 || tile_mode == 0) && (am ? g.a_stride_k : g.a_stride_m) < (1 << 22) && (bm ? g.b_stride_k : g.b_stride_n) < (1 << 22) &&
-            g.m % BIG_TILE == 0 && g.n % BIG_TILE == 0 && g.k >= 3 * DIRECT_KSTEP && g.m / BIG_TILE * (g.n / BIG_TILE) * p.batches <= INT32_MAX &&
-            (tile_mode == 4 || g.m / BIG_TILE * (g.n / BIG_TILE) * p.batches >= BIG_TILE_MIN_WORKGROUPS / 2)) {
-            p.MT = (int)(g.m / BIG_TILE), p.NT = (int)(g.n / BIG_TILE);
-            const int64_t big_blocks = (int64_t)p.MT * p.NT * p.batches;
-            kutacc_prof::KernelTimer t(am ? "pair_gemm_direct_kernel<m-major>" : "pair_gemm_direct_kernel", flops, stream);
-            return kutacc_hip_status(am ? launch_direct_tiles<true>(p, big_blocks, stream) : launch_direct_tiles<false>(p, big_blocks, stream));
-        }
-        // 256 x 256 tiles where every CU gets at least four; else 192 x 192 where every CU gets at least two
-        for (const int side : {BIG_TILE, 192}) {
-            const bool forced = tile_mode == (side == BIG_TILE ? 1 : 3);
-            if (g.m % side != 0 || g.n % side != 0 || (!forced && tile_mode != 0)) {
-                continue;
-            }
-            p.MT = (int)(g.m / side), p.NT = (int)(g.n / side);
-            const int64_t big_blocks = (int64_t)p.MT * p.NT * p.batches;
-            const int64_t enough = side == BIG_TILE ? BIG_TILE_MIN_WORKGROUPS : BIG_TILE_MIN_WORKGROUPS / 2;
-            if (big_blocks <= INT32_MAX && (big_blocks >= enough || forced)) {
-                kutacc_prof::KernelTimer t(side == BIG_TILE ? (am ? "pair_gemm_big_kernel<m-major>" : "pair_gemm_big_kernel")
-                                                            : (am ? "pair_gemm_big_kernel<m-major, 192>" : "pair_gemm_big_kernel<192>"),
-                                           flops, stream);
-                const hipError_t e = side == BIG_TILE ? (am ? launch_big_tiles<true, 4>(p, big_blocks, stream) : launch_big_tiles<false, 4>(p, big_blocks, stream))
-                                                      : (am ? launch_big_tiles<true, 3>(p, big_blocks, stream) : launch_big_tiles<false, 3>(p, big_blocks, stream));
-                return kutacc_hip_status(e);
-            }
+    if (!gated && am == bm && g.bias_axis == 0 && !g.relu) {
+        const int rc = large_tiles(p, am, flops, stream);
+        if (rc != KUTACC_HIP_EUNSUPPORTED) {
+            return rc;
         }
     }
     p.MT = (int)((g.m + (gated ? 64 : 128) - 1) / (gated ? 64 : 128));
@@ -1984,6 +1979,35 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
         e = launch_tiles<false, false, false>(p, blocks, stream);
     }
     return kutacc_hip_status(e);
+}
+
+int gated_projection_mode() { return g_gated_mode.load(); }
+
+// The equation of the triangle multiplication on planes whose rows of n positions lie np apart (np a multiple of 8, zeros
+// in the padding): centre[c] = left[c] right[c]^T (outgoing) or right[c]^T left[c] (incoming).  The columns past n of the
+// result's rows are written too, with whatever the padding gives.
+int triangle_equation(const void *left, const void *right, void *centre, int64_t n, int64_t np, int64_t plane, int64_t channels, bool incoming,
+                      hipStream_t stream)
+{
+    GemmParams p;
+    std::memset(&p, 0, sizeof(p));
+    p.a = (const bf16_t *)(incoming ? right : left), p.b = (const bf16_t *)(incoming ? left : right), p.c = (bf16_t *)centre;
+    p.a_sm = p.b_sn = incoming ? 1 : np, p.a_sk = p.b_sk = incoming ? np : 1;
+    p.a_sb = p.b_sb = p.c_sb = plane, p.c_sm = np;
+    p.M = (int)n, p.N = (int)np, p.K = (int)(incoming ? n : np), p.batches = (int)channels;
+    p.a_rows = p.b_rows = (int)(incoming ? np : n);
+    const double flops = 2.0 * (double)n * (double)n * (double)n * (double)channels;
+    const int rc = n == np ? large_tiles(p, incoming, flops, stream) : KUTACC_HIP_EUNSUPPORTED;
+    if (rc != KUTACC_HIP_EUNSUPPORTED) {
+        return rc;
+    }
+    p.MT = (p.M + 127) / 128, p.NT = (p.N + 127) / 128;
+    const int64_t blocks = (int64_t)p.MT * p.NT * p.batches;
+    if (blocks > INT32_MAX) {
+        return KUTACC_HIP_EUNSUPPORTED;
+    }
+    kutacc_prof::KernelTimer t(incoming ? "pair_gemm_kernel<m-major>" : "pair_gemm_kernel", flops, stream);
+    return kutacc_hip_status(incoming ? launch_tiles<true, true, false>(p, blocks, stream) : launch_tiles<false, false, false>(p, blocks, stream));
 }
 
 int sigmoid_gate_rows(void *out, int64_t out_s0, int64_t out_s1, const void *gate, int64_t gate_s0, int64_t gate_s1,

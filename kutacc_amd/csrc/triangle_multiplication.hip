@@ -1,0 +1,529 @@
+// The two ends of the triangle-multiplication block at 128 channels (reference
+// src/attention/triangle_multiplication.cpp:25-150 with the LayerNorms and the residual a caller adds around it).  Between
+// them lies the equation, one n x n product per channel (pair_stack.hip).
+//
+// Layout of the intermediates.  The projections and the centre are channel-first, one plane per channel, and a plane's
+// rows are n positions padded to a pitch of np = n rounded up to 8: every row then starts on 16 bytes, whatever n is, and
+// the products run on the matrix cores with vector loads at every length.  The projections write zeros into the padding
+// (their mask is zero there), so a contraction over np positions is one over n.  With dense rows an n that is no multiple
+// of 8 left the product to scalar loads: 217 ms for the block at 691 residues, 0.39 ms so.
+//
+// Both kernels take the padded positions p = i np + j in steps of 64.  Eight consecutive positions share the row i, because
+// np is a multiple of 8: a wave follows (i, j) of its eights with scalar additions.
+//
+// Both are bound by HBM (front: 256 bytes in, 512 out per position; back: 512 in, 256 out).  Neither reads a normalised copy of
+// the pair activation: the front kernel normalises the rows on their way into the LDS, the back kernel does it again for
+// its gate, from the same rows that its residual needs.  At 384 residues that saves a pass of 76 MB and a read of 38 MB.
+#include <hip/hip_runtime.h>
+
+#include "launch_internal.h"
+#include "mfma_tiles.h"
+#include "profiler.h"
+
+namespace {
+using namespace kutacc_dev;
+
+constexpr int C = 128, CK = C / 16;
+constexpr int STEP = 64;              // positions per step
+constexpr int ROW_SLOTS = C * 2 / 16; // 16-byte slots of a position's row
+
+// (i, j) of the first of eight consecutive padded positions
+struct Place {
+    int i, j;
+};
+
+__device__ __forceinline__ Place place_of(uint32_t p, uint32_t np) { return Place{(int)(p / np), (int)(p % np)}; }
+
+__device__ __forceinline__ void advance(Place &q, int np)
+{
+    q.j += STEP;
+    while (q.j >= np) {
+        q.j -= np, ++q.i;
+    }
+}
+
+// Rows of the pair activation in the LDS: [64 positions][16 slots], the slot index XOR-ed with position % 8 (a fragment
+// read, lane -> its own position, then hits eight different bank groups per eight lanes)
+__device__ __forceinline__ int row_slot(int pos, int chunk) { return pos * ROW_SLOTS + (chunk ^ (pos & 7)); }
+
+// LayerNorm of a row of 128 channels held by 16 consecutive lanes, 8 each: the arithmetic of layernorm_rows_bf16_kernel
+// (reference src/normalization/layernorm_kernel.h:21-53)
+__device__ __forceinline__ uint4 normalise_row(uint4 raw, int lane, const float (&gm)[8], const float (&bt)[8], float eps)
+{
+    const bf16x8 b = as_bf16x8(raw);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        v[e] = to_f32(b[e]);
+    }
+    const float x0 = __shfl(v[0], lane & ~15, 64);
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float d = v[e] - x0;
+        s1 += d;
+        s2 = fmaf(d, d, s2);
+    }
+    s1 = group_sum<16>(s1);
+    s2 = group_sum<16>(s2);
+    const float n = (float)C;
+    const float mean = s1 / n + x0;
+    const float var = fmaxf((s2 - s1 * s1 / n) / n, 0.f);
+    const float rstd = __builtin_amdgcn_rsqf(var + eps);
+    const float shift = -rstd * mean;
+    bf16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        o[e] = (bf16_t)fmaf(fmaf(v[e], rstd, shift), gm[e], bt[e]);
+    }
+    return as_uint4(o);
+}
+
+struct Side {
+    const bf16_t *wp, *wg;
+    const float *bp, *bg;
+    bf16_t *out;
+};
+
+// LayerNorm and both gated projections: out[c][p] = bf16(bf16(y . wp[c] + bp[c]) * mask * sigmoid(y . wg[c] + bg[c])), y the
+// normalised row of position p.  Eight waves, one workgroup per CU; a wave owns 32 channels of one side and keeps its two
+// 32 x 128 weight blocks in 64 registers.  Per step it normalises eight of the 64 rows, loaded two steps ahead, into the
+// shared stage, multiplies the whole stage and writes 32 channels x 128 bytes.  Same arithmetic in the same order as
+// LayerNorm followed by gated_projection_kernel: the results are bit-identical.
+constexpr int FRONT_WAVES = 8;
+constexpr int FRONT_STAGE = STEP * ROW_SLOTS;
+constexpr size_t FRONT_LDS = (size_t)(2 * FRONT_STAGE + FRONT_WAVES * 256) * 16 + 2 * STEP * 2;
+
+__global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(const bf16_t *__restrict__ x, const float *__restrict__ gamma,
+                                                                             const float *__restrict__ beta, float eps, Side s0, Side s1,
+                                                                             const bf16_t *__restrict__ mask, int64_t plane, int n, int np,
+                                                                             int steps_per_group)
+{
+    extern __shared__ uint4 lds[]; // two stages, a panel per wave, two mask rows
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rv = lane & 31, gv = lane >> 5;
+    const Side &sd = wave >= 4 ? s1 : s0;
+    const int cb = wave & 3; // this wave's 32 channels
+    uint4 *panel = lds + 2 * FRONT_STAGE + wave * 256;
+    uint16_t *mask_rows = reinterpret_cast<uint16_t *>(lds + 2 * FRONT_STAGE + FRONT_WAVES * 256);
+
+    const int positions = n * np, total_steps = (positions + STEP - 1) / STEP;
+    const int first = (int)blockIdx.x * steps_per_group;
+    const int stop = first + steps_per_group < total_steps ? first + steps_per_group : total_steps;
+    if (first >= stop) {
+        return;
+    }
+
+    // This wave's eight rows of a step: lane (l / 16, l % 16) holds chunk l % 16 of rows l / 16 and 4 + l / 16.  Padding
+    // repeats the row's last position, steps past the end repeat the last row: valid addresses, results masked or dropped.
+    struct Rows {
+        uint4 r[2];
+        uint16_t m; // mask of position lane % 8 of the eight
+    };
+    Place at = place_of((uint32_t)(first * STEP + 8 * wave), (uint32_t)np);
+    auto load = [&](Rows &t) {
+        const bool there = at.i < n;
+        const int i = there ? at.i : n - 1;
+        const char *row = reinterpret_cast<const char *>(x + (int64_t)i * n * C);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int j = min(at.j + 4 * u + (lane >> 4), n - 1);
+            t.r[u] = *reinterpret_cast<const uint4 *>(row + ((uint32_t)j * (2u * C) + 16u * (lane & 15)));
+        }
+        const int jm = at.j + (lane & 7);
+        const uint16_t m = reinterpret_cast<const uint16_t *>(mask)[(int64_t)i * n + min(jm, n - 1)];
+        t.m = there && jm < n ? m : (uint16_t)0;
+        advance(at, np);
+    };
+    float gm[8], bt[8];
+    auto stage_rows = [&](const Rows &t, int s) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            lds[s * FRONT_STAGE + row_slot(8 * wave + 4 * u + (lane >> 4), lane & 15)] = normalise_row(t.r[u], lane, gm, bt, eps);
+        }
+        if (lane < 8) {
+            mask_rows[s * STEP + 8 * wave + lane] = t.m;
+        }
+    };
+
+    Rows even, odd;
+    load(even);
+    load(odd);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        gm[e] = gamma[(lane & 15) * 8 + e], bt[e] = beta[(lane & 15) * 8 + e];
+    }
+    bf16x8 wp[CK], wg[CK];
+#pragma unroll
+    for (int ks = 0; ks < CK; ++ks) {
+        wp[ks] = *reinterpret_cast<const bf16x8 *>(sd.wp + (cb * 32 + rv) * C + ks * 16 + gv * 8);
+        wg[ks] = *reinterpret_cast<const bf16x8 *>(sd.wg + (cb * 32 + rv) * C + ks * 16 + gv * 8);
+    }
+    const float pbias = sd.bp[cb * 32 + rv], gneg = -LOG2E * sd.bg[cb * 32 + rv];
+    bf16_t *out = sd.out + (int64_t)cb * 32 * plane;
+    stage_rows(even, 0);
+    __syncthreads();
+
+    auto do_step = [&](int step, int s, Rows &next, Rows &after) {
+        if (step + 2 < stop) {
+            load(after);
+        }
+        if (step + 1 < stop) {
+            stage_rows(next, s ^ 1);
+        }
+        const uint4 *stage = lds + s * FRONT_STAGE;
+        const char *mrow = reinterpret_cast<const char *>(mask_rows + s * STEP);
+        bf16x8 af[2][CK];
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+#pragma unroll
+            for (int ks = 0; ks < CK; ++ks) {
+                af[rb][ks] = as_bf16x8(stage[row_slot(rb * 32 + rv, 2 * ks + gv)]);
+            }
+        }
+        // projection first, rounded to bf16 and parked as packed pairs, then the gate: half the accumulators live
+        bf16x8 pp[2][2];
+        {
+            f32x16 pa[2] = {zero16(), zero16()};
+#pragma unroll
+            for (int ks = 0; ks < CK; ++ks) {
+#pragma unroll
+                for (int rb = 0; rb < 2; ++rb) {
+                    pa[rb] = mfma(af[rb][ks], wp[ks], pa[rb]);
+                }
+            }
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    pa[rb][v] += pbias;
+                }
+                pp[rb][0] = pack8(pa[rb], 0), pp[rb][1] = pack8(pa[rb], 8);
+            }
+        }
+        f32x16 ga[2] = {zero16(), zero16()};
+#pragma unroll
+        for (int ks = 0; ks < CK; ++ks) {
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb) {
+                ga[rb] = mfma(af[rb][ks], wg[ks], ga[rb]);
+            }
+        }
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const bf16x4 mk = *reinterpret_cast<const bf16x4 *>(mrow + 2 * (rb * 32 + 8 * a + 4 * gv)); // the lane's four positions
+                bf16x4 ov;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float pv = to_f32(pp[rb][a >> 1][4 * (a & 1) + c]) * to_f32(mk[c]);
+                    // sigmoid(gate + bias) = 1 / (1 + 2^-(gate*log2e + bias*log2e)); the gate stays in fp32
+                    const float e = __builtin_amdgcn_exp2f(fmaf(ga[rb][4 * a + c], -LOG2E, gneg));
+                    ov[c] = (bf16_t)(pv * __builtin_amdgcn_rcpf(1.0f + e));
+                }
+                *(reinterpret_cast<bf16x4 *>(panel + panel_slot(rv, rb * 4 + a)) + gv) = ov;
+            }
+        }
+        // 32 channels x eight 16-byte pieces of 8 positions
+        const int piece = lane & 7;
+        if (step * STEP + 8 * piece < positions) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int ch = 8 * i + (lane >> 3);
+                *reinterpret_cast<uint4 *>(out + (int64_t)ch * plane + step * STEP + 8 * piece) = panel[panel_slot(ch, piece)];
+            }
+        }
+        __syncthreads(); // the other stage is complete, this one no longer read
+    };
+    int step = first;
+    while (true) {
+        do_step(step, 0, odd, even);
+        if (++step >= stop) {
+            break;
+        }
+        do_step(step, 1, even, odd);
+        if (++step >= stop) {
+            break;
+        }
+    }
+}
+
+// x[i, j] += bf16(bf16(centre' . wo^T + bo) * sigmoid(bf16(y . wg^T + bg))), centre' the normalised centre of (i, j), y its
+// normalised row of x.  Four waves, two workgroups per CU (the three barriers of a step of one are covered by the
+// other); a wave owns 32 output features, keeps both 32 x 128 weight blocks in 64 registers and moves 16 of the step's 64
+// positions: it normalises their rows of x, transposes and normalises their centre (a lane holds 8 positions of a
+// channel as it lies in memory; transpose8x8_lanes turns them into 8 channels of one position), and finishes them with the
+// residual, for which the rows of x have stayed in its registers.
+constexpr int BACK_STAGE = STEP * ROW_SLOTS; // slots of each of the four stages: centre as it lies, y, centre', result
+constexpr size_t BACK_LDS = (size_t)4 * BACK_STAGE * 16 + 6 * C * sizeof(float);
+
+__global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__restrict__ centre, int64_t plane, const float *__restrict__ c_gamma,
+                                                               const float *__restrict__ c_beta, const bf16_t *__restrict__ wo,
+                                                               const float *__restrict__ bo, const bf16_t *__restrict__ wg,
+                                                               const float *__restrict__ bg, bf16_t *__restrict__ x,
+                                                               const float *__restrict__ gamma, const float *__restrict__ beta, float eps,
+                                                               int n, int np, int steps_per_group)
+{
+    extern __shared__ uint4 lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rv = lane & 31, gv = lane >> 5;
+    uint4 *raw = lds, *ys = lds + BACK_STAGE, *cs = lds + 2 * BACK_STAGE, *res = lds + 3 * BACK_STAGE;
+    float *params = reinterpret_cast<float *>(lds + 4 * BACK_STAGE); // gamma, beta, centre's gamma and beta, bo, bg
+    const int positions = n * np, total_steps = (positions + STEP - 1) / STEP;
+    const int first = (int)blockIdx.x * steps_per_group;
+    const int stop = first + steps_per_group < total_steps ? first + steps_per_group : total_steps;
+    if (first >= stop) {
+        return;
+    }
+
+    // rows of x: this wave's 16 positions of a step, in two eights: 16 wave + 4 u + lane / 16
+    struct Eight {
+        uint4 r0, r1; // named members, so that they always live in registers
+        Place at;
+    };
+    Place at_lo = place_of((uint32_t)(first * STEP + 16 * wave), (uint32_t)np), at_hi = place_of((uint32_t)(first * STEP + 16 * wave + 8), (uint32_t)np);
+    auto load_eight = [&](Eight &t, Place &at) {
+        t.at = at;
+        const char *row = reinterpret_cast<const char *>(x + (int64_t)(at.i < n ? at.i : n - 1) * n * C);
+        const int j = at.j + (lane >> 4);
+        t.r0 = *reinterpret_cast<const uint4 *>(row + ((uint32_t)min(j, n - 1) * (2u * C) + 16u * (lane & 15)));
+        t.r1 = *reinterpret_cast<const uint4 *>(row + ((uint32_t)min(j + 4, n - 1) * (2u * C) + 16u * (lane & 15)));
+        advance(at, np);
+    };
+    // the centre: channels 32 wave + 8 i + lane / 8, positions 8 (lane % 8) .. + 7 of the step; past the end the last eight
+    const uint32_t lane_plane = (uint32_t)(lane >> 3) * (uint32_t)plane * 2u;
+    auto load_centre = [&](int step) {
+        PanelRegs t;
+        const uint32_t pos = (uint32_t)min(step * STEP + 8 * (lane & 7), positions - 8);
+        const char *src = reinterpret_cast<const char *>(centre + (int64_t)(32 * wave) * plane);
+        const int64_t eight = 16 * plane; // bytes of eight channels
+        const uint32_t off = lane_plane + 2u * pos;
+        t.r0 = *reinterpret_cast<const uint4 *>(src + off);
+        t.r1 = *reinterpret_cast<const uint4 *>(src + eight + off);
+        t.r2 = *reinterpret_cast<const uint4 *>(src + 2 * eight + off);
+        t.r3 = *reinterpret_cast<const uint4 *>(src + 3 * eight + off);
+        return t;
+    };
+
+    Eight lo, hi, next_lo, next_hi;
+    PanelRegs ct = load_centre(first);
+    load_eight(lo, at_lo);
+    load_eight(hi, at_hi);
+    next_lo = lo, next_hi = hi;
+    bf16x8 wof[CK], wgf[CK];
+#pragma unroll
+    for (int ks = 0; ks < CK; ++ks) {
+        wof[ks] = *reinterpret_cast<const bf16x8 *>(wo + (wave * 32 + rv) * C + ks * 16 + gv * 8);
+        wgf[ks] = *reinterpret_cast<const bf16x8 *>(wg + (wave * 32 + rv) * C + ks * 16 + gv * 8);
+    }
+    if (tid < C) {
+        params[tid] = gamma[tid], params[C + tid] = beta[tid];
+        params[2 * C + tid] = c_gamma[tid], params[3 * C + tid] = c_beta[tid];
+        params[4 * C + tid] = bo[tid], params[5 * C + tid] = bg[tid];
+    }
+    __syncthreads();
+    const uint32_t sel = transpose8x8_selector(lane);
+
+    for (int step = first; step < stop; ++step) {
+        int lv = lane; // opaque: LDS addresses are formed per step, not kept across the loop
+        asm volatile("" : "+v"(lv));
+        // the centre as it lies: [128 channels][8 slots], the slot XOR-ed with channel / 8 % 8, under which the reads below
+        // (eight lanes: channels 8 apart, one slot) and these writes are free of bank conflicts
+        {
+            uint4 *mine = raw + (32 * wave + (lv >> 3)) * 8;
+            const int f = 4 * (wave & 1); // channel / 8 % 8 of this wave's first eight channels
+            mine[(lv & 7) ^ f] = ct.r0;
+            mine[64 + ((lv & 7) ^ (f + 1))] = ct.r1;
+            mine[128 + ((lv & 7) ^ (f + 2))] = ct.r2;
+            mine[192 + ((lv & 7) ^ (f + 3))] = ct.r3;
+        }
+        if (step + 1 < stop) {
+            ct = load_centre(step + 1);
+        }
+        {
+            float gm[8], bt[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                gm[e] = params[(lv & 15) * 8 + e], bt[e] = params[C + (lv & 15) * 8 + e];
+            }
+            const int pos = 16 * wave + (lv >> 4);
+            ys[row_slot(pos, lv & 15)] = normalise_row(lo.r0, lv, gm, bt, eps);
+            ys[row_slot(pos + 4, lv & 15)] = normalise_row(lo.r1, lv, gm, bt, eps);
+            ys[row_slot(pos + 8, lv & 15)] = normalise_row(hi.r0, lv, gm, bt, eps);
+            ys[row_slot(pos + 12, lv & 15)] = normalise_row(hi.r1, lv, gm, bt, eps);
+        }
+        if (step + 1 < stop) {
+            load_eight(next_lo, at_lo);
+            load_eight(next_hi, at_hi);
+        }
+        __syncthreads();
+        // gate: this wave's 32 features of all 64 positions, rounded to bf16
+        bf16x8 gate[2][2];
+        {
+            f32x16 acc[2] = {zero16(), zero16()};
+#pragma unroll
+            for (int ks = 0; ks < CK; ++ks) {
+#pragma unroll
+                for (int pb = 0; pb < 2; ++pb) {
+                    acc[pb] = mfma(wgf[ks], as_bf16x8(ys[row_slot(32 * pb + (lv & 31), 2 * ks + (lv >> 5))]), acc[pb]);
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const f32x4 bv = *reinterpret_cast<const f32x4 *>(params + 5 * C + wave * 32 + 8 * a + 4 * (lv >> 5));
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+#pragma unroll
+                    for (int pb = 0; pb < 2; ++pb) {
+                        gate[pb][a >> 1][4 * (a & 1) + c] = (bf16_t)(acc[pb][4 * a + c] + bv[c]);
+                    }
+                }
+            }
+        }
+        // the centre of this wave's positions, eight at a time: lane (k, c) has channel 8 c + k (+ 64 t) of all eight, after
+        // the exchange channels 8 c .. + 7 (+ 64 t) of position k; a position's channels lie in eight consecutive lanes
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int k8 = lv >> 3, c8 = lv & 7;
+            bf16x8 v[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int ch = 64 * t + 8 * c8 + k8;
+                v[t] = as_bf16x8(transpose8x8_lanes(raw[ch * 8 + ((2 * wave + q) ^ c8)], sel));
+            }
+            const float x0 = __shfl(to_f32(v[0][0]), lv & ~7, 64);
+            float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float d = to_f32(v[t][e]) - x0;
+                    s1 += d;
+                    s2 = fmaf(d, d, s2);
+                }
+            }
+            s1 = group_sum<8>(s1), s2 = group_sum<8>(s2);
+            const float nch = (float)C;
+            const float mean = s1 / nch + x0;
+            const float var = fmaxf((s2 - s1 * s1 / nch) / nch, 0.f);
+            const float rstd = __builtin_amdgcn_rsqf(var + eps);
+            const float shift = -rstd * mean;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const float *gm = params + 2 * C + 64 * t + 8 * c8, *bt = gm + C;
+                bf16x8 o;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    o[e] = (bf16_t)fmaf(fmaf(to_f32(v[t][e]), rstd, shift), gm[e], bt[e]);
+                }
+                cs[row_slot(16 * wave + 8 * q + k8, 8 * t + c8)] = as_uint4(o);
+            }
+        }
+        __syncthreads();
+        {
+            f32x16 acc[2] = {zero16(), zero16()};
+#pragma unroll
+            for (int ks = 0; ks < CK; ++ks) {
+#pragma unroll
+                for (int pb = 0; pb < 2; ++pb) {
+                    acc[pb] = mfma(wof[ks], as_bf16x8(cs[row_slot(32 * pb + (lv & 31), 2 * ks + (lv >> 5))]), acc[pb]);
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const f32x4 bv = *reinterpret_cast<const f32x4 *>(params + 4 * C + wave * 32 + 8 * a + 4 * (lv >> 5));
+#pragma unroll
+                for (int pb = 0; pb < 2; ++pb) {
+                    bf16x4 ov;
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        // bf16(out) * sigmoid(bf16(gate)), rounded to bf16: the reference's rounding points
+                        const float o = to_f32((bf16_t)(acc[pb][4 * a + c] + bv[c]));
+                        ov[c] = (bf16_t)(o * sigmoid_fast(to_f32(gate[pb][a >> 1][4 * (a & 1) + c])));
+                    }
+                    *(reinterpret_cast<bf16x4 *>(res + row_slot(32 * pb + (lv & 31), 4 * wave + a)) + (lv >> 5)) = ov;
+                }
+            }
+        }
+        __syncthreads();
+        auto finish = [&](const Place &at, uint4 raw_row, int local) { // position `local` of the eight at `at`
+            const int j = at.j + (local & 7);
+            const bf16x8 d = as_bf16x8(res[row_slot(16 * wave + local, lv & 15)]), z = as_bf16x8(raw_row);
+            bf16x8 o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                o[e] = (bf16_t)(to_f32(z[e]) + to_f32(d[e]));
+            }
+            if (at.i < n && j < n) {
+                *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(x + (int64_t)at.i * n * C) + ((uint32_t)j * (2u * C) + 16u * (lv & 15))) = as_uint4(o);
+            }
+        };
+        finish(lo.at, lo.r0, lv >> 4);
+        finish(lo.at, lo.r1, 4 + (lv >> 4));
+        finish(hi.at, hi.r0, 8 + (lv >> 4));
+        finish(hi.at, hi.r1, 12 + (lv >> 4));
+        lo = next_lo, hi = next_hi;
+    }
+}
+
+int cu_count()
+{
+    static int table[KUTACC_DEVICE_SLOTS] = {};
+    return kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, table);
+}
+
+// equal runs of steps for at most `cap` workgroups
+struct Split {
+    unsigned groups;
+    int per_group;
+};
+Split split_steps(int64_t n, int64_t np, int64_t cap)
+{
+    const int64_t steps = (n * np + STEP - 1) / STEP;
+    const int64_t per = (steps + cap - 1) / cap;
+    return Split{(unsigned)((steps + per - 1) / per), (int)per};
+}
+} // namespace
+
+namespace kutacc_launch {
+
+bool triangle_ends_support(const kutacc_hip_triangle_multiplication_args_t &a)
+{
+    // 16-byte loads of the activation's rows and of the weights; positions and a plane's bytes times eight in 32 bits
+    return a.c_z == C && a.c_i == C && a.n_res <= 8192 && kutacc_hip_aligned16(a.pair_act) && kutacc_hip_aligned16(a.left_proj_w) &&
+           kutacc_hip_aligned16(a.left_gate_w) && kutacc_hip_aligned16(a.right_proj_w) && kutacc_hip_aligned16(a.right_gate_w) &&
+           kutacc_hip_aligned16(a.output_w) && kutacc_hip_aligned16(a.gating_w);
+}
+
+int triangle_front(const kutacc_hip_triangle_multiplication_args_t &a, void *left, void *right, int64_t np, int64_t plane, hipStream_t stream)
+{
+    static size_t configured[KUTACC_DEVICE_SLOTS] = {};
+    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&triangle_front_kernel), FRONT_LDS, configured)) {
+        return kutacc_hip_status(e);
+    }
+    kutacc_prof::KernelTimer t("gated_projection_blocks_kernel<2>", 8.0 * (double)(a.n_res * a.n_res) * C * C, stream);
+    const Split s = split_steps(a.n_res, np, cu_count());
+    const Side l = {(const bf16_t *)a.left_proj_w, (const bf16_t *)a.left_gate_w, a.left_proj_b, a.left_gate_b, (bf16_t *)left};
+    const Side r = {(const bf16_t *)a.right_proj_w, (const bf16_t *)a.right_gate_w, a.right_proj_b, a.right_gate_b, (bf16_t *)right};
+    triangle_front_kernel<<<dim3(s.groups), 64 * FRONT_WAVES, FRONT_LDS, stream>>>((const bf16_t *)a.pair_act, a.ln_in_gamma, a.ln_in_beta, a.ln_eps, l,
+                                                                                  r, (const bf16_t *)a.pair_mask, plane, (int)a.n_res, (int)np,
+                                                                                  s.per_group);
+    return kutacc_hip_status(hipGetLastError());
+}
+
+int triangle_back(const kutacc_hip_triangle_multiplication_args_t &a, const void *centre, int64_t np, int64_t plane, hipStream_t stream)
+{
+    static size_t configured[KUTACC_DEVICE_SLOTS] = {};
+    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&triangle_back_kernel), BACK_LDS, configured)) {
+        return kutacc_hip_status(e);
+    }
+    kutacc_prof::KernelTimer t("triangle_back_kernel", 4.0 * (double)(a.n_res * a.n_res) * C * C, stream);
+    const Split s = split_steps(a.n_res, np, 2 * (int64_t)cu_count());
+    triangle_back_kernel<<<dim3(s.groups), 256, BACK_LDS, stream>>>(
+        (const bf16_t *)centre, plane, a.ln_center_gamma, a.ln_center_beta, (const bf16_t *)a.output_w, a.output_b, (const bf16_t *)a.gating_w,
+        a.gating_b, (bf16_t *)a.pair_act, a.ln_in_gamma, a.ln_in_beta, a.ln_eps, (int)a.n_res, (int)np, s.per_group);
+    return kutacc_hip_status(hipGetLastError());
+}
+
+} // namespace kutacc_launch

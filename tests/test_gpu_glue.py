@@ -411,6 +411,28 @@ def test_triangle_multiplication_block_seeded_sweep(torch_cuda, index, n):
     helpers.check_close(helpers.to_numpy(pair), tm_block_oracle(c, incoming), "bf16", f"TM block sweep {index}: n={n} incoming={incoming}")
 
 
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 33, 63, 64, 65, 127, 129, 200])
+def test_triangle_multiplication_block_at_any_length(torch_cuda, n):
+    """128 channels, lengths around the padded pitch (8), the steps of the block's first and last kernel (64 positions) and the
+    tiles of the product (128), both orientations; a guard behind the activation shows a store past the last row."""
+    torch = torch_cuda
+    case = tm_block_case(3000 + n, n, 128, 128)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
+        device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
+    w = {k: dev(v) for k, v in case.items() if k not in ("z", "mask")}
+    for incoming in (False, True):
+        guarded = torch.full((n * n + 64, 128), 7.0, device="cuda", dtype=torch.bfloat16)
+        pair = guarded[:n * n].view(n, n, 128)
+        pair.copy_(dev(case["z"]))
+        print(f"n={n} incoming={incoming}", flush=True)
+        assert capi.TriangleMultiplicationBlock(pair, dev(case["mask"]), w, incoming).run() == 0
+        torch.cuda.synchronize()
+        want = tm_block_oracle(case, incoming)
+        # half as much again as the usual bar: six bf16 roundings in a chain, up to five million values per orientation
+        helpers.assert_within(helpers.to_numpy(pair), want, 3e-2 + 1.5e-2 * np.abs(want), f"TM block n={n} incoming={incoming}")
+        assert bool((guarded[n * n:] == 7.0).all())
+
+
 @pytest.mark.parametrize("n", [48, 72, 384])
 def test_triangle_multiplication_block_on_each_gated_projection_kernel(torch_cuda, n):
     """The block's two gated projections go out in one launch.  Its default kernel (weights in registers, both sides in
