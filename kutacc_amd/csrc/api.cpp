@@ -246,8 +246,7 @@ int kutacc_hip_linear(const void *act, int64_t ld_act, const void *weight, int64
     if (!act || !weight || !result || ld_act < k || ld_w < k) {
         return KUTACC_HIP_EINVAL;
     }
-    return kutacc_launch::gemm_nt(dtype, act, ld_act, weight, ld_w, bias, result, n, 1, m, n, k, beta,
-                                  pick_stream(stream));
+    return kutacc_launch::linear(dtype, act, ld_act, weight, ld_w, bias, result, m, n, k, beta, pick_stream(stream));
 }
 
 int kutacc_hip_pair_bias(const void *z, const float *gamma, const float *beta, const void *w, void *nb, void *z_norm,

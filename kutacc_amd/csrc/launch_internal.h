@@ -167,6 +167,8 @@ int layernorm_channel_first(const void *x, int64_t ld_x, const float *gamma, con
                             int64_t channels, int64_t positions, float eps, int32_t dtype, hipStream_t stream);
 
 // row_kernels.hip
+int linear(int32_t dtype, const void *act, int64_t ld_act, const void *w, int64_t ld_w, const float *bias, void *result, int64_t m,
+           int64_t n, int64_t k, float beta, hipStream_t stream);
 // swap_j != 0: rows are pairs (i, j) of an [rows / swap_j, swap_j] grid and output row (i, j) is computed from input
 // row (j, i) of the transposed grid
 int layernorm_rows(const void *x, int64_t ld_x, const float *gamma, const float *beta, void *out, int64_t ld_out,

@@ -718,6 +718,36 @@ def test_linear_matches_oracle(torch_cuda):
     helpers.assert_within(helpers.to_numpy(res), ref2, 2.0 ** -7 * np.abs(ref2) + 1e-6, "linear beta=1")
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 64), (31, 3, 128), (33, 4, 128), (129, 8, 128), (300, 20, 64), (64, 33, 256), (1000, 64, 64), (257, 72, 128),
+    (40000, 96, 128), (515, 250, 256), (70001, 256, 256),
+    (130, 264, 128), (65, 48, 40), (33, 5, 24),  # past the row kernel: MFMA tiles (264 outputs, 40 features), scalar
+])
+def test_linear_shapes(torch_cuda, m, n, k):
+    """kutacc_hip_linear in bf16 around the blocks of its row kernel (32 rows, 32 and 64 outputs; results written in pieces of 8,
+    4 and 1) against a float64 product, with bias and, on top of it, beta = 0.5; a padded pitch of the input rows."""
+    torch = torch_cuda
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    act = torch.randn(m, k + 8, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(n, k, device="cuda", generator=g) / k ** 0.5).bfloat16()
+    bias = torch.randn(n, device="cuda", generator=g)
+    guarded = torch.full((m * n + 64,), 7.0, device="cuda", dtype=torch.bfloat16)
+    print(f"linear m={m} n={n} k={k}", flush=True)
+    call = lambda b, beta: capi.lib().kutacc_hip_linear(act.data_ptr(), k + 8, w.data_ptr(), k, b, guarded.data_ptr(), m, n, k,  # noqa: E731
+                                                         beta, capi.K_BF16, None)
+    assert call(bias.data_ptr(), 0.0) == 0
+    torch.cuda.synchronize()
+    first = guarded[:m * n].double().cpu().numpy().reshape(m, n)
+    prod = act[:, :k].double().cpu().numpy() @ w.double().cpu().numpy().T
+    want = prod + bias.double().cpu().numpy()
+    helpers.assert_within(first, want, 2.0 ** -8 * np.abs(want) + 1e-5, "linear")
+    assert call(None, 0.5) == 0
+    torch.cuda.synchronize()
+    want = prod + 0.5 * first
+    helpers.assert_within(guarded[:m * n].double().cpu().numpy().reshape(m, n), want, 2.0 ** -8 * np.abs(want) + 1e-5, "linear beta=0.5")
+    assert bool((guarded[m * n:] == 7.0).all())
+
+
 def test_pair_bias_producer_at_1024_residues(torch_cuda):
     """z [1024, 1024, 128], four heads: the oracle's LayerNorm + Linear on a sample of rows i (all j), for the producer and
     for the form that reads z transposed."""
