@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "api_internal.h"
+#include "attention_util.h"
 #include "device_util.h"
 #include "launch_internal.h"
 #include "mfma_tiles.h"
@@ -177,13 +178,7 @@ __device__ __forceinline__ void stage_mask_words(const bf16_t *bias_row, uint32_
             mv *= scale;
         }
         if (k < NB * 32) {
-            const bf16_t hi = (bf16_t)mv;
-            const float hf = to_f32(hi);
-            const float rest = (hf == mv || !(fabsf(hf) < INFINITY)) ? 0.f : mv - hf; // a NaN stays one through hi
-            const bf16_t lo = (bf16_t)rest;
-            bf16x2 pair;
-            pair[0] = hi, pair[1] = lo;
-            words[k] = __builtin_bit_cast(uint32_t, pair);
+            words[k] = mask_word(mv);
         }
         const unsigned long long nz = __ballot(k < NB * 32 && mv != 0.f);
         const uint32_t bits = (((uint32_t)nz != 0u ? 1u : 0u) | ((uint32_t)(nz >> 32) != 0u ? 2u : 0u)) << (2 * wave);
@@ -191,11 +186,6 @@ __device__ __forceinline__ void stage_mask_words(const bf16_t *bias_row, uint32_
             atomicOr(flag_word, bits);
         }
     }
-}
-
-__device__ __forceinline__ float mask_word_value(uint32_t w)
-{
-    return __uint_as_float(w << 16) + __uint_as_float(w & 0xffff0000u);
 }
 
 // The value stage_mask_part would store for key k, in two steps for kernels that fetch the mask early and store it
@@ -489,32 +479,6 @@ __device__ __forceinline__ void timeslice_priority(uint32_t turn, int shift)
                  : "scc");
 }
 
-// A operand of the row-sum MFMA (16x16x32: lane -> row lane&15, k-chunk lane>>4).  The B operand is a
-// probability fragment of the 32x32x16 layout (lane -> query lane&31, 8 keys of half lane>>5), which the
-// 16x16x32 shape reads as column lane&15, k-chunk lane>>4: chunks 0 and 2 belong to query n, chunks 1 and
-// 3 to query n+16.  Row 0 of A therefore sums chunks 0 and 2, row 1 chunks 1 and 3; the sums of
-// queries n and n+16 end up in lane n, accumulator registers 0 and 1.
-__device__ __forceinline__ bf16x8 rowsum_selector(int lane)
-{
-    const int i = lane & 15, c = lane >> 4;
-    const float v = ((i == 0 && (c & 1) == 0) || (i == 1 && (c & 1) == 1)) ? 1.0f : 0.0f;
-    bf16x8 a;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        a[e] = (bf16_t)v;
-    }
-    return a;
-}
-
-__device__ __forceinline__ float rowsum_fetch(const f32x4 &lacc, int lane)
-{
-    const int q = lane & 31;
-    const int src = (q & 15) * 4;
-    const float a0 = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(lacc[0])));
-    const float a1 = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(lacc[1])));
-    return (q >> 4) ? a1 : a0;
-}
-
 template <bool HAS_NB, bool WITH_MASK, bool SHIFT>
 __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 *lds_v, const f32x4 *mask4,
                                                 const uint4 *nbf, bf16x8 q0, bf16x8 q1, f16x8 sel0, f16x8 sel1,
@@ -790,20 +754,6 @@ __device__ __forceinline__ void attend_block_direct(const uint4 *lds_k, const ui
     }
     o_out = o;
     l_out = half_swap_sum(lsum);
-}
-
-// avg[b, q, h, :] = O / l * gate for the 32 queries of one block; gate values in accumulator order
-__device__ __forceinline__ void store_gated(bf16_t *dst, const f32x16 &o, float inv, const f32x16 &gate)
-{
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        bf16x4 ov;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            ov[c] = (bf16_t)(o[4 * a + c] * inv * gate[4 * a + c]);
-        }
-        *reinterpret_cast<bf16x4 *>(dst + 8 * a) = ov;
-    }
 }
 
 // Copies head h's rows of `count` weight matrices (first, first + 1, ...) into LDS in MFMA fragment order.  One
@@ -2420,32 +2370,33 @@ bool make_plan(int64_t S, int C, Plan &pl)
             return true;
         }
     }
-    // fewest idle wave slots first, then fewest blocks per wave (more waves to overlap MFMA and VALU)
-    int best_idle = 1 << 30;
-    pl.BPW = 0;
+    // Most waves resident on a CU first -- a second workgroup where registers and LDS allow one, if need be with the weights
+    // staged in smaller groups --, then fewest idle block slots, then most matrices per group, then fewest blocks per wave.
+    // With the idle slots first, lengths with many divisors of their block count got few waves: 256 channels and 259
+    // positions (nine blocks) three a CU, 321 us at 400 rows against 244 with 2 x 3; 128 channels and 470 positions (15
+    // blocks) five, 239 us against 192 with eight.
+    int best_waves = 0, best_idle = 0, best_gw = 0;
     for (int bpw = 1; bpw <= 4; ++bpw) {
         const int nw = (int)((NB + bpw - 1) / bpw);
         if (nw > max_waves(C, bpw)) {
             continue;
         }
-        const int idle = nw * bpw - (int)NB;
-        if (idle < best_idle) {
-            best_idle = idle, pl.BPW = bpw, pl.NW = nw;
+        // The 128-channel kernels and the 256-channel one with four blocks per wave are compiled for one group of four.
+        const int gw_min = (C == 128 || bpw == 4) ? 4 : 1;
+        for (int gw = 4; gw >= gw_min; gw >>= 1) {
+            const size_t need = head_kernel_lds(C, (int)NB, gw, nw, bpw);
+            if (need > cap) {
+                continue;
+            }
+            const int by_lds = (int)(cap / need), by_waves = max_waves(C, bpw) / nw;
+            const int waves = nw * (by_lds < by_waves ? by_lds : by_waves), idle = nw * bpw - (int)NB;
+            if (waves > best_waves || (waves == best_waves && (idle < best_idle || (idle == best_idle && gw > best_gw)))) {
+                best_waves = waves, best_idle = idle, best_gw = gw;
+                pl.BPW = bpw, pl.NW = nw, pl.GW = gw, pl.lds_bytes = need;
+            }
         }
     }
-    if (pl.BPW == 0) {
-        return false;
-    }
-    // The 128-channel kernels and the 256-channel one with four blocks per wave are compiled for one group of four.
-    const int gw_min = (C == 128 || pl.BPW == 4) ? 4 : 1;
-    for (int gw = 4; gw >= gw_min; gw >>= 1) {
-        const size_t need = head_kernel_lds(C, pl.NB, gw, pl.NW, pl.BPW);
-        if (need <= cap) {
-            pl.GW = gw, pl.lds_bytes = need;
-            return true;
-        }
-    }
-    return false;
+    return best_waves > 0;
 }
 
 inline bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }

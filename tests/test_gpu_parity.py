@@ -267,6 +267,19 @@ def test_two_row_kernel_matches_the_oracle(torch_cuda, row_pairs_forced, config,
     helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, w.dtype, "out")
 
 
+@pytest.mark.parametrize("config,seq", [(2, 257), (4, 320), (2, 345), (4, 384), (2, 416), (4, 640), (5, 385), (3, 450), (5, 512), (5, 513), (5, 800)])
+def test_long_row_plans_at_their_edges(torch_cuda, config, seq):
+    """One length on either side of where the long-row kernel's plan changes -- blocks per wave, matrices per LDS group, one or two
+    workgroups per CU -- in a batch with more rows than fit one round of an XCD's workgroups."""
+    w = make_workload(config, batch=9, seq_len=seq)
+    print(f"plan edge config {config} S={seq}", flush=True)
+    ten, scratch = helpers.to_device(w)
+    assert helpers.run_hip(w, ten, scratch, capi.PATH_FUSED) == 0
+    ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
+    helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), ref_avg, w.dtype, "gated average")
+    helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, w.dtype, "out")
+
+
 def test_two_row_kernel_is_what_the_headline_shape_runs(torch_cuda, capfd):
     """Configuration 3 at a batch that gives every workgroup two rows takes the two-row kernel by itself, and a large
     pair-bias offset (overflow / underflow repeat with shifted rows) leaves its result where the oracle has it."""
