@@ -164,7 +164,7 @@ int kutacc_hip_set_tuning(const char *name, const char *value)
         g_block_layernorm.store(value && !std::strcmp(value, "fused") ? 1 : (value && !std::strcmp(value, "separate") ? 2 : 0));
         return 0;
     }
-    if (kutacc_launch::pair_gemm_tuning(name, value) == 0) {
+    if (kutacc_launch::pair_gemm_tuning(name, value) == 0 || kutacc_launch::streamed_attention_tuning(name, value) == 0) {
         return 0;
     }
     return kutacc_launch::fused_attention_tuning(name, value);

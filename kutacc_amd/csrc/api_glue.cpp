@@ -29,7 +29,8 @@ struct Workspace {
 // fused_ln: the head kernel normalises the rows of the pair tensor itself, so no normalised copy is kept.
 // tiled: rows beyond the fused head kernels (more than 1024 residues) -- the operator runs on the tiled MFMA route, which
 // forms k, v and gate in memory, and its result is added to the pair activation by a pass of its own.
-Workspace layout(int64_t n, int64_t heads, bool fused_ln, bool tiled = false)
+// streamed: the same for 128 and 256 channels -- the attention's own workspace lies at q, k, v and gate do not exist
+Workspace layout(int64_t n, int64_t heads, bool fused_ln, bool tiled = false, bool streamed = false)
 {
     const int64_t c = heads * HEAD, act = align256(n * n * c * 2);
     Workspace w;
@@ -39,7 +40,10 @@ Workspace layout(int64_t n, int64_t heads, bool fused_ln, bool tiled = false)
     w.q = w.bias + align256(n * n * 2);
     w.avg = w.q + act;
     w.k = w.v = w.gate = w.out = w.total = w.avg + act;
-    if (tiled) {
+    if (streamed) {
+        w.avg = w.q + align256(kutacc_launch::streamed_workspace_bytes(n, n, heads, true));
+        w.out = w.avg + act, w.total = w.out + act;
+    } else if (tiled) {
         w.v = w.k + act, w.gate = w.v + act, w.out = w.gate + act, w.total = w.out + act;
     }
     return w;
@@ -106,7 +110,12 @@ bool beyond_fused_kernels(int64_t seq_len, int64_t heads)
     const int64_t c = heads * HEAD;
     return (c != 128 && c != 256) || seq_len > 1024;
 }
-bool triangle_block_is_tiled(int64_t n, int64_t heads) { return beyond_fused_kernels(n, heads); }
+// ... and of those, the ones with 128 or 256 channels the streamed kernels (the tuning hook sends all lengths there)
+bool block_is_streamed(int64_t seq_len, int64_t heads)
+{
+    return (heads == 4 || heads == 8) && (seq_len > 1024 || kutacc_launch::streamed_attention_forced());
+}
+bool triangle_block_is_tiled(int64_t n, int64_t heads) { return beyond_fused_kernels(n, heads) || block_is_streamed(n, heads); }
 
 bool triangle_block_fuses_layernorm(int64_t n, int64_t heads)
 {
@@ -157,7 +166,9 @@ int64_t kutacc_hip_triangle_attention_workspace(int64_t n_res, int64_t nheads)
     if (n_res <= 0 || nheads <= 0 || n_res > 65536 || nheads > 64) {
         return -1;
     }
-    return layout(n_res, nheads, triangle_block_fuses_layernorm(n_res, nheads), triangle_block_is_tiled(n_res, nheads)).total;
+    return layout(n_res, nheads, triangle_block_fuses_layernorm(n_res, nheads), triangle_block_is_tiled(n_res, nheads),
+                  block_is_streamed(n_res, nheads))
+        .total;
 }
 
 int kutacc_hip_triangle_attention(const kutacc_hip_triangle_attention_args_t *a, void *stream)
@@ -174,7 +185,8 @@ int kutacc_hip_triangle_attention(const kutacc_hip_triangle_attention_args_t *a,
     // then the first link of the fused chain, and the workspace holds no normalised copy); elsewhere the producer below
     // writes one.
     const bool fused_ln = triangle_block_fuses_layernorm(n, heads), tiled = triangle_block_is_tiled(n, heads);
-    const Workspace w = layout(n, heads, fused_ln, tiled);
+    const bool streamed = block_is_streamed(n, heads);
+    const Workspace w = layout(n, heads, fused_ln, tiled, streamed);
     if (a->workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(a->workspace) & 255u) != 0) {
         return KUTACC_HIP_EINVAL;
     }
@@ -183,6 +195,26 @@ int kutacc_hip_triangle_attention(const kutacc_hip_triangle_attention_args_t *a,
     const int ending = a->ending_node != 0;
 
     const kutacc_hip_attention_args_t g = triangle_attention_call(a, ws, w, fused_ln);
+    if (streamed) {
+        // LayerNorm + pair bias, with the tiles the attention reads where the producer can write them; the operator, which
+        // forms the mask bias from the pair mask itself; residual sum (transposed back for the ending node).
+        kutacc_hip_attention_args_t t = g;
+        t.out = ws + w.out;
+        kutacc_launch::FusedAttentionOptions opt;
+        opt.bias_is_mask = true, opt.bias_stride_k = ending ? n : 1;
+        const int nb_blocks = (int)((n + 31) / 32);
+        opt.nb_tiles_ready = kutacc_launch::pair_bias_writes_fragments(a->pair_act, a->bias_w, ws + w.z_norm, n, n, c, heads, KUTACC_DTYPE_BF16);
+        int rc = kutacc_launch::pair_bias(a->pair_act, a->ln_gamma, a->ln_beta, a->bias_w, ws + w.nb, ws + w.z_norm, n, n, c, heads,
+                                          a->ln_eps, KUTACC_DTYPE_BF16, ending, s, opt.nb_tiles_ready ? ws + w.q : nullptr, nb_blocks,
+                                          (nb_blocks + 1) & ~1, 1);
+        if (rc == 0) {
+            rc = kutacc_launch::gating_attention_streamed(t, opt, ws + w.q, w.avg - w.q, s);
+        }
+        if (rc == 0) {
+            rc = kutacc_launch::residual_add(a->pair_act, ws + w.out, n, n, c, ending, KUTACC_DTYPE_BF16, s);
+        }
+        return rc;
+    }
     if (tiled) {
         // Rows beyond the fused head kernels: the same chain as separate passes -- LayerNorm + pair bias (read transposed
         // for the ending node), mask bias, the operator on the tiled MFMA route, residual sum (transposed back).
@@ -446,7 +478,7 @@ struct MsaWorkspace {
 
 // fused_ln: the head kernel normalises the msa rows itself, so no normalised copy is kept; tiled: as for the
 // triangle-attention block
-MsaWorkspace msa_layout(int64_t n_seq, int64_t n_res, int64_t heads, bool column, bool fused_ln, bool tiled = false)
+MsaWorkspace msa_layout(int64_t n_seq, int64_t n_res, int64_t heads, bool column, bool fused_ln, bool tiled = false, bool streamed = false)
 {
     const int64_t act = align256(n_seq * n_res * heads * HEAD * 2);
     MsaWorkspace w;
@@ -456,7 +488,10 @@ MsaWorkspace msa_layout(int64_t n_seq, int64_t n_res, int64_t heads, bool column
     w.q = w.bias + align256(n_seq * n_res * 2);
     w.avg = w.q + act;
     w.k = w.v = w.gate = w.out = w.total = w.avg + act;
-    if (tiled) {
+    if (streamed) {
+        w.avg = w.q + align256(kutacc_launch::streamed_workspace_bytes(column ? n_res : n_seq, column ? n_seq : n_res, heads, !column));
+        w.out = w.avg + act, w.total = w.out + act;
+    } else if (tiled) {
         w.v = w.k + act, w.gate = w.v + act, w.out = w.gate + act, w.total = w.out + act;
     }
     return w;
@@ -494,7 +529,7 @@ kutacc_hip_attention_args_t msa_attention_call(const kutacc_hip_msa_attention_ar
 
 bool msa_block_is_tiled(int64_t n_seq, int64_t n_res, int64_t heads, bool column)
 {
-    return beyond_fused_kernels(column ? n_seq : n_res, heads);
+    return beyond_fused_kernels(column ? n_seq : n_res, heads) || block_is_streamed(column ? n_seq : n_res, heads);
 }
 
 bool msa_block_fuses_layernorm(int64_t n_seq, int64_t n_res, int64_t heads, bool column)
@@ -521,7 +556,7 @@ int64_t kutacc_hip_msa_attention_workspace(int64_t n_seq, int64_t n_res, int64_t
         return -1;
     }
     return msa_layout(n_seq, n_res, nheads, column != 0, msa_block_fuses_layernorm(n_seq, n_res, nheads, column != 0),
-                      msa_block_is_tiled(n_seq, n_res, nheads, column != 0))
+                      msa_block_is_tiled(n_seq, n_res, nheads, column != 0), block_is_streamed(column ? n_seq : n_res, nheads))
         .total;
 }
 
@@ -541,13 +576,37 @@ int kutacc_hip_msa_attention(const kutacc_hip_msa_attention_args_t *a, void *str
     const int64_t n_seq = a->n_seq, n_res = a->n_res, heads = a->nheads, c = heads * HEAD;
     // where the persistent head kernel takes the call it normalises the msa rows itself: no normalised copy, no LayerNorm pass
     const bool fused_ln = msa_block_fuses_layernorm(n_seq, n_res, heads, column), tiled = msa_block_is_tiled(n_seq, n_res, heads, column);
-    const MsaWorkspace w = msa_layout(n_seq, n_res, heads, column, fused_ln, tiled);
+    const bool streamed = block_is_streamed(column ? n_seq : n_res, heads);
+    const MsaWorkspace w = msa_layout(n_seq, n_res, heads, column, fused_ln, tiled, streamed);
     if (a->workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(a->workspace) & 255u) != 0) {
         return KUTACC_HIP_EINVAL;
     }
     char *ws = static_cast<char *>(a->workspace);
     hipStream_t s = kutacc_api::stream_or_default(stream);
     const kutacc_hip_attention_args_t g = msa_attention_call(a, ws, w, fused_ln);
+    if (streamed) {
+        kutacc_hip_attention_args_t t = g;
+        t.out = ws + w.out;
+        kutacc_launch::FusedAttentionOptions opt;
+        opt.bias_is_mask = true, opt.bias_stride_k = column ? n_res : 1;
+        int rc = kutacc_launch::layernorm_rows(a->msa_act, c, a->ln_gamma, a->ln_beta, ws + w.m_norm, c, n_seq * n_res, c, a->ln_eps,
+                                               KUTACC_DTYPE_BF16, s, column ? n_seq : 0);
+        if (rc == 0 && !column) {
+            const int nb_blocks = (int)((n_res + 31) / 32);
+            opt.nb_tiles_ready =
+                kutacc_launch::pair_bias_writes_fragments(a->pair_act, a->bias_w, nullptr, n_res, n_res, a->c_z, heads, KUTACC_DTYPE_BF16);
+            rc = kutacc_launch::pair_bias(a->pair_act, a->pair_ln_gamma, a->pair_ln_beta, a->bias_w, ws + w.nb, nullptr, n_res, n_res,
+                                          a->c_z, heads, a->ln_eps, KUTACC_DTYPE_BF16, 0, s, opt.nb_tiles_ready ? ws + w.q : nullptr,
+                                          nb_blocks, (nb_blocks + 1) & ~1, 1);
+        }
+        if (rc == 0) {
+            rc = kutacc_launch::gating_attention_streamed(t, opt, ws + w.q, w.avg - w.q, s);
+        }
+        if (rc == 0) {
+            rc = kutacc_launch::residual_add(a->msa_act, ws + w.out, n_seq, n_res, c, column ? 1 : 0, KUTACC_DTYPE_BF16, s);
+        }
+        return rc;
+    }
     if (tiled) {
         // Rows beyond the fused head kernels (more than 1024 keys): LayerNorm (read transposed column-wise), pair bias
         // (row-wise), mask bias, the operator on the tiled MFMA route, residual sum (transposed back column-wise).

@@ -2633,6 +2633,16 @@ bool fused_attention_supports(const kutacc_hip_attention_args_t &a)
     return make_plan(a.seq_len, (int)C, pl);
 }
 
+int pair_bias_tiles(const kutacc_hip_attention_args_t &a, void *tiles, hipStream_t stream)
+{
+    const int NB = (int)((a.seq_len + 31) / 32), NT = (NB + 1) & ~1;
+    const int vec = aligned(a.nonbatched_bias, 16) && a.nb_stride_h % 8 == 0 && a.nb_stride_q % 8 == 0;
+    kutacc_prof::KernelTimer t("pair_bias_tiles_kernel", 0.0, stream);
+    pair_bias_tiles_kernel<<<dim3((unsigned)NB * NT, (unsigned)a.nheads), 64, 0, stream>>>(
+        (const bf16_t *)a.nonbatched_bias, a.nb_stride_h, a.nb_stride_q, (int)a.seq_len, NB, NT, vec, (f32x4 *)tiles);
+    return kutacc_hip_status(hipGetLastError());
+}
+
 int gating_attention_fused(const kutacc_hip_attention_args_t &a, hipStream_t stream, const FusedAttentionOptions &opt)
 {
     const int residual = opt.out_mode;
@@ -2685,10 +2695,7 @@ int gating_attention_fused(const kutacc_hip_attention_args_t &a, hipStream_t str
         if (p.nb != nullptr && opt.nb_tiles_ready) {
             p.nbf = (const uint4 *)tiles; // the producer of the pair bias wrote the tiles
         } else if (p.nb != nullptr) {
-            kutacc_prof::KernelTimer t("pair_bias_tiles_kernel", 0.0, stream);
-            pair_bias_tiles_kernel<<<dim3((unsigned)(pl.NB * p.NT), (unsigned)a.nheads), 64, 0, stream>>>(
-                p.nb, p.nb_sh, p.nb_sq, p.S, pl.NB, p.NT, p.nb_vec, (f32x4 *)tiles);
-            rc = kutacc_hip_status(hipGetLastError());
+            rc = kutacc_launch::pair_bias_tiles(a, tiles, stream);
             if (rc != 0) {
                 return rc;
             }

@@ -119,6 +119,19 @@ bool fused_attention_tile_layout(const kutacc_hip_attention_args_t &args, const 
 int gating_attention_fused(const kutacc_hip_attention_args_t &args, hipStream_t stream,
                            const FusedAttentionOptions &opt = FusedAttentionOptions());
 
+// pair bias -> fp32 tiles in log2 units, [nheads][ceil(S/32)][ceil(S/32) rounded up to even][4][64 lanes] x 16 bytes
+int pair_bias_tiles(const kutacc_hip_attention_args_t &args, void *tiles, hipStream_t stream);
+
+// streamed_attention.hip: rows of any length, 128 or 256 channels in heads of 32, on a workspace of streamed_workspace_bytes()
+// (256-byte aligned) that starts with the tiles of the pair bias; opt.nb_tiles_ready: they lie there already.  args.q, k, v
+// and gate are not used; the result is stored (opt.out_mode FUSED_OUT_STORE).
+bool streamed_attention_supports(const kutacc_hip_attention_args_t &args);
+int64_t streamed_workspace_bytes(int64_t batch, int64_t seq_len, int64_t nheads, bool pair_bias);
+int gating_attention_streamed(const kutacc_hip_attention_args_t &args, const FusedAttentionOptions &opt, void *workspace, int64_t bytes,
+                              hipStream_t stream);
+bool streamed_attention_forced(); // the "streamed" hook: blocks of every size on these kernels
+int streamed_attention_tuning(const char *name, const char *value);
+
 // "plan" / "fragments" / "debug" hooks of the attention launcher (kutacc_hip_set_tuning); KUTACC_HIP_EINVAL for other names
 int fused_attention_tuning(const char *name, const char *value);
 // "gemm_tile" hook of the matrix products of the pair stack; KUTACC_HIP_EINVAL for other names

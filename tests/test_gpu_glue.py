@@ -289,6 +289,25 @@ def test_triangle_attention_block_with_other_channel_counts(torch_cuda, n, heads
         helpers.check_close(helpers.to_numpy(got), block_oracle(c, ending), "bf16", f"block n={n} heads={heads} ending={ending}")
 
 
+@pytest.fixture
+def streamed_everywhere():
+    assert capi.set_tuning("streamed", "1") == 0
+    yield
+    capi.set_tuning("streamed", None)
+
+
+@pytest.mark.parametrize("n,heads", [(1, 4), (31, 4), (33, 8), (64, 4), (97, 8), (128, 4), (130, 4), (161, 8), (290, 4)])
+def test_triangle_attention_block_on_the_streamed_kernels(torch_cuda, streamed_everywhere, n, heads):
+    """The attention that keeps q, k, v and gate in memory, at lengths on either side of its key tiles (32), workgroups (four
+    query blocks) and placement groups (eight of those), odd numbers of rows, whole and ragged tiles (the producer writes
+    the tiles of the pair bias, or a pass of its own does); 128 and 256 channels, whole result against the oracle."""
+    for ending in (False, True):
+        c = block_case(9400 + n, n, heads)
+        print(f"streamed block n={n} heads={heads} ending={ending}", flush=True)
+        got = run_block(torch_cuda, c, ending)
+        helpers.check_close(helpers.to_numpy(got), block_oracle(c, ending), "bf16", f"streamed block n={n} heads={heads} ending={ending}")
+
+
 def test_fused_layernorm_drops_the_normalised_copy_from_the_workspace(torch_cuda):
     """With the LayerNorm inside the attention kernel the blocks keep no normalised activation: the workspace is one
     activation smaller wherever the persistent kernel runs (384 residues), and unchanged where it does not (1024)."""
@@ -729,6 +748,22 @@ def test_msa_attention_blocks_on_the_tiled_route(torch_cuda, column, n_seq, n_re
     torch.cuda.synchronize()
     assert res["rc"] == 0 and "attention_tiles_kernel" in names, (res, names)
     helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, column), "bf16", f"msa block {n_seq}x{n_res} heads={heads} column={column}")
+
+
+@pytest.mark.parametrize("column,n_seq,n_res,heads", [(True, 100, 7, 8), (False, 5, 70, 8), (False, 6, 64, 4), (True, 257, 3, 4), (True, 32, 1, 8)])
+def test_msa_attention_blocks_on_the_streamed_kernels(torch_cuda, streamed_everywhere, column, n_seq, n_res, heads):
+    torch = torch_cuda
+    c = msa_case(9500 + n_seq + n_res, n_seq, n_res, heads, 128)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
+        device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
+    msa = dev(c["m"])
+    w = {k: dev(c[k]) for k in ("ln_gamma", "ln_beta", "wq", "wk", "wv", "wg", "bg", "wo", "bo")}
+    pair = None if column else {"pair_act": dev(c["z"]), "pair_ln_gamma": dev(c["pair_ln_gamma"]),
+                                "pair_ln_beta": dev(c["pair_ln_beta"]), "bias_w": dev(c["bias_w"])}
+    print(f"streamed msa {n_seq}x{n_res} heads={heads} column={column}", flush=True)
+    assert capi.MsaAttentionBlock(msa, dev(c["mask"]), w, heads, pair).run() == 0
+    torch.cuda.synchronize()
+    helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, column), "bf16", f"streamed msa block {n_seq}x{n_res} heads={heads} column={column}")
 
 
 def test_msa_attention_blocks_full_size_sampled_rows(torch_cuda):
