@@ -119,6 +119,46 @@ __device__ __forceinline__ float half_swap_sum(float x)
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+__device__ __forceinline__ uint4 zero_u4() { return make_uint4(0u, 0u, 0u, 0u); }
+
+// Eight bf16 from a row of `length`, from element `at` on; elements past the end are zero (never read).  Rows start on any
+// even address: the hardware's unaligned 16-byte loads serve them, and the last piece of a row is the row's last eight
+// elements, shifted down.
+__device__ __forceinline__ uint4 load8_any(const bf16_t *row, int at)
+{
+    uint4 v;
+    __builtin_memcpy(&v, row + at, 16);
+    return v;
+}
+
+__device__ __forceinline__ uint4 load8_checked(const bf16_t *row, int at, int length)
+{
+    union {
+        uint4 u;
+        uint64_t q[2];
+        bf16_t e[8];
+    } c;
+    if (length < 8) {
+        c.u = zero_u4();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (at + i < length) {
+                c.e[i] = row[at + i];
+            }
+        }
+        return c.u;
+    }
+    const int from = min(at, length - 8), drop = min(at - from, 8);
+    c.u = load8_any(row, from);
+    const int bits = 16 * (drop & 3);
+    if (drop >= 4) {
+        c.q[0] = drop == 8 ? 0 : c.q[1] >> bits, c.q[1] = 0;
+    } else if (drop > 0) {
+        c.q[0] = c.q[0] >> bits | c.q[1] << (64 - bits), c.q[1] >>= bits;
+    }
+    return c.u;
+}
+
 // Wave-private staging panel in LDS: 32 rows x 128 bytes, in 16-byte slots.  A panel is filled with
 // four fully coalesced loads (each instruction reads 8 rows x 128 contiguous bytes = 8 whole cache
 // lines, lane l -> row 8i + l/8, slot l%8) and read back in MFMA fragment order (lane -> its own

@@ -20,8 +20,8 @@
 // points of the reference, which rounds both GEMM results to bf16 before its element-wise pass
 // (triangle_multiplication.cpp:37-66).
 //
-// Shapes the MFMA kernel does not take (k, n or a leading dimension not a multiple of 8, pointers not
-// 16-byte aligned) run on a scalar kernel with the same epilogues.
+// Shapes whose k, n or leading dimensions are no multiples of 8, or whose pointers are not 16-byte aligned, run on the same
+// tiles with unaligned loads and stores; operands that are contiguous along neither index on a scalar kernel.
 //
 // The batched product of the triangle equation, where its sides are whole large tiles and there are enough of them,
 // runs on persistent kernels with 256 x 256 (or 192 x 192) tiles per workgroup: pair_gemm_direct_kernel, whose
@@ -73,7 +73,10 @@ constexpr int CT_LD = 136;                      // bf16 elements per row of the 
 // the second stage did (triangle-multiplication products at 384 residues: 30.7 -> 26.6 us, gated projection 32 -> 27).
 constexpr size_t GEMM_LDS = TILE * CT_LD * 2 > STAGE_SLOTS * 16 ? TILE * CT_LD * 2 : STAGE_SLOTS * 16;
 
-// K-major operand: rows row0..row0+31 (clamped), 64 k from k0; chunks past K read as zero
+// K-major operand: rows row0..row0+31 (clamped), 64 k from k0; chunks past K read as zero.  ANY (here and below): extents,
+// pitches and pointers need not be multiples of 8 elements -- unaligned 16-byte loads, and the last piece of a row shifted
+// into place.
+template <bool ANY>
 __device__ __forceinline__ PanelRegs load_kmajor(const bf16_t *base, int64_t ld, int row0, int last_row, int k0, int K, int lane)
 {
     const int col = k0 + (lane & 7) * 8;
@@ -85,6 +88,10 @@ __device__ __forceinline__ PanelRegs load_kmajor(const bf16_t *base, int64_t ld,
     for (int i = 0; i < 4; ++i) {
         int row = row0 + 8 * i + (lane >> 3);
         row = row < last_row ? row : last_row;
+        if constexpr (ANY) {
+            *dst[i] = k0 + KSTEP <= K ? load8_any(base + (int64_t)row * ld, col) : load8_checked(base + (int64_t)row * ld, col, K);
+            continue;
+        }
         uint4 v = *reinterpret_cast<const uint4 *>(base + (int64_t)row * ld + colc);
         if (!ok) {
             v = make_uint4(0u, 0u, 0u, 0u);
@@ -107,16 +114,24 @@ __device__ __forceinline__ PanelRegs load_kmajor(const bf16_t *base, int64_t ld,
 // hold rows with different k & 3 (different bank halves after the swizzle).
 __device__ __forceinline__ int mm_row(int kk) { return (kk & 4) | ((kk & 1) << 1) | ((kk >> 1) & 1); }
 
+template <bool ANY = false>
 __device__ __forceinline__ PanelRegs load_mmajor(const bf16_t *base, int64_t ld, int m0, int rows, int k0, int K, int lane)
 {
     int m = m0 + (lane & 7) * 8;
-    m = m + 8 <= rows ? m : rows - 8; // rows past the end are never stored; any valid address will do
+    const bool whole = m + 8 <= rows;
+    m = ANY || whole ? m : rows - 8; // rows past the end are never stored; any valid address will do
     PanelRegs p;
     uint4 *dst[4] = {&p.r0, &p.r1, &p.r2, &p.r3};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int k = k0 + 8 * i + mm_row(lane >> 3);
         const bool ok = k < K;
+        if constexpr (ANY) {
+            const bf16_t *row = base + (int64_t)(ok ? k : 0) * ld;
+            const uint4 v = whole ? load8_any(row, m) : load8_checked(row, m, rows);
+            *dst[i] = ok ? v : zero_u4();
+            continue;
+        }
         uint4 v = *reinterpret_cast<const uint4 *>(base + (int64_t)(ok ? k : 0) * ld + m);
         if (!ok) {
             v = make_uint4(0u, 0u, 0u, 0u);
@@ -153,8 +168,8 @@ __device__ __forceinline__ bf16x8 mm_fragment(const lds_char *operand, int lane_
     return lds_transposed_fragment(operand + lane_off + s * 4096, operand + lane_off + s * 4096 + 1024);
 }
 
-template <bool A_MMAJOR, bool B_MMAJOR, bool GATED>
-__global__ __launch_bounds__(256, (A_MMAJOR && B_MMAJOR) ? 4 : 3) void pair_gemm_kernel(const GemmParams p)
+template <bool A_MMAJOR, bool B_MMAJOR, bool GATED, bool ANY>
+__global__ __launch_bounds__(256, ANY ? 2 : (A_MMAJOR && B_MMAJOR) ? 4 : 3) void pair_gemm_kernel(const GemmParams p)
 {
     extern __shared__ uint4 lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -193,18 +208,18 @@ __global__ __launch_bounds__(256, (A_MMAJOR && B_MMAJOR) ? 4 : 3) void pair_gemm
 
     auto fetch_a = [&](int k0) -> PanelRegs {
         if constexpr (A_MMAJOR) {
-            return load_mmajor(a, p.a_sk, m0 + 64 * (wave & 1), p.a_rows, k0 + 32 * (wave >> 1), p.K, lane);
+            return load_mmajor<ANY>(a, p.a_sk, m0 + 64 * (wave & 1), p.a_rows, k0 + 32 * (wave >> 1), p.K, lane);
         } else if constexpr (GATED) {
-            return load_kmajor(wave < 2 ? a : a_gate, p.a_sm, m0 + 32 * (wave & 1), p.a_rows - 1, k0, p.K, lane);
+            return load_kmajor<ANY>(wave < 2 ? a : a_gate, p.a_sm, m0 + 32 * (wave & 1), p.a_rows - 1, k0, p.K, lane);
         } else {
-            return load_kmajor(a, p.a_sm, m0 + 32 * wave, p.a_rows - 1, k0, p.K, lane);
+            return load_kmajor<ANY>(a, p.a_sm, m0 + 32 * wave, p.a_rows - 1, k0, p.K, lane);
         }
     };
     auto fetch_b = [&](int k0) -> PanelRegs {
         if constexpr (B_MMAJOR) {
-            return load_mmajor(b, p.b_sk, n0 + 64 * (wave & 1), p.b_rows, k0 + 32 * (wave >> 1), p.K, lane);
+            return load_mmajor<ANY>(b, p.b_sk, n0 + 64 * (wave & 1), p.b_rows, k0 + 32 * (wave >> 1), p.K, lane);
         } else {
-            return load_kmajor(b, p.b_sn, n0 + 32 * wave, p.b_rows - 1, k0, p.K, lane);
+            return load_kmajor<ANY>(b, p.b_sn, n0 + 32 * wave, p.b_rows - 1, k0, p.K, lane);
         }
     };
     auto park = [&](uint4 *stage, const PanelRegs &ra, const PanelRegs &rb) {
@@ -290,7 +305,12 @@ __global__ __launch_bounds__(256, (A_MMAJOR && B_MMAJOR) ? 4 : 3) void pair_gemm
             for (int q = 0; q < 4; ++q) {
                 const int tcol = 64 * wn + 32 * j + 8 * q + 4 * g;
                 f32x4 bv = {row_bias, row_bias, row_bias, row_bias};
-                if (p.bias_axis == 1 && n0 + tcol + 4 <= p.N) {
+                if (ANY && p.bias_axis == 1) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        bv[c] = bsrc[min(n0 + tcol + c, p.N - 1)];
+                    }
+                } else if (p.bias_axis == 1 && n0 + tcol + 4 <= p.N) {
                     bv = *reinterpret_cast<const f32x4 *>(bsrc + n0 + tcol);
                 }
                 bf16x4 ov;
@@ -309,6 +329,24 @@ __global__ __launch_bounds__(256, (A_MMAJOR && B_MMAJOR) ? 4 : 3) void pair_gemm
     __syncthreads();
 
     bf16_t *c = alt ? p.c_alt : p.c + (int64_t)batch * p.c_sb;
+    auto store = [&](int gm, int gn, uint4 v) {
+        bf16_t *to = c + (int64_t)gm * p.c_sm + gn;
+        if constexpr (ANY) {
+            if (gn + 8 <= p.N) {
+                __builtin_memcpy(to, &v, 16);
+            } else {
+                const bf16x8 e = as_bf16x8(v);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    if (gn + i < p.N) {
+                        to[i] = e[i];
+                    }
+                }
+            }
+        } else {
+            *reinterpret_cast<uint4 *>(to) = v;
+        }
+    };
     if constexpr (GATED) {
         const bf16_t *mask = p.mask + (int64_t)batch * p.mask_sb;
 #pragma unroll
@@ -319,13 +357,13 @@ __global__ __launch_bounds__(256, (A_MMAJOR && B_MMAJOR) ? 4 : 3) void pair_gemm
             if (gm < p.M && gn < p.N) {
                 const bf16x8 pv = *reinterpret_cast<const bf16x8 *>(ct + row * CT_LD + chunk * 8);
                 const bf16x8 gv = *reinterpret_cast<const bf16x8 *>(ct + (64 + row) * CT_LD + chunk * 8);
-                const bf16x8 mv = *reinterpret_cast<const bf16x8 *>(mask + gn);
+                const bf16x8 mv = as_bf16x8(ANY ? load8_checked(mask, gn, p.N) : *reinterpret_cast<const uint4 *>(mask + gn));
                 bf16x8 ov;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     ov[e] = (bf16_t)(to_f32(pv[e]) * to_f32(mv[e]) * sigmoid_fast(to_f32(gv[e])));
                 }
-                *reinterpret_cast<bf16x8 *>(c + (int64_t)gm * p.c_sm + gn) = ov;
+                store(gm, gn, as_uint4(ov));
             }
         }
     } else {
@@ -335,8 +373,7 @@ __global__ __launch_bounds__(256, (A_MMAJOR && B_MMAJOR) ? 4 : 3) void pair_gemm
             const int row = piece >> 4, chunk = piece & 15;
             const int gm = m0 + row, gn = n0 + chunk * 8;
             if (gm < p.M && gn < p.N) {
-                *reinterpret_cast<uint4 *>(c + (int64_t)gm * p.c_sm + gn) =
-                    *reinterpret_cast<const uint4 *>(ct + row * CT_LD + chunk * 8);
+                store(gm, gn, *reinterpret_cast<const uint4 *>(ct + row * CT_LD + chunk * 8));
             }
         }
     }
@@ -1608,14 +1645,14 @@ bool operand_ok(const void *ptr, int64_t s_row, int64_t s_k, int64_t s_batch, in
     return false;
 }
 
-template <bool AM, bool BM, bool G>
+template <bool AM, bool BM, bool G, bool ANY = false>
 hipError_t launch_tiles(const GemmParams &p, int64_t blocks, hipStream_t stream)
 {
     static size_t configured[KUTACC_DEVICE_SLOTS] = {}; // per instantiation and device: dynamic LDS is set through the opt-in
-    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&pair_gemm_kernel<AM, BM, G>), GEMM_LDS, configured)) {
+    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&pair_gemm_kernel<AM, BM, G, ANY>), GEMM_LDS, configured)) {
         return e;
     }
-    pair_gemm_kernel<AM, BM, G><<<dim3((unsigned)blocks), 256, GEMM_LDS, stream>>>(p);
+    pair_gemm_kernel<AM, BM, G, ANY><<<dim3((unsigned)blocks), 256, GEMM_LDS, stream>>>(p);
     return hipGetLastError();
 }
 
@@ -1888,10 +1925,17 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
         mfma_ok = mfma_ok && !am && !bm && kutacc_hip_aligned16(g.a_gate) && kutacc_hip_aligned16(g.mask) && g.mask_stride_batch % 8 == 0 &&
                   (g.bias_axis != 1 || kutacc_hip_aligned16(g.bias_gate));
     }
+    // The same tiles with unaligned loads and stores for every other shape whose operands are contiguous along one index: a
+    // product of 691 x 691 x 691 x 128 channels 77 ms on the scalar kernel.  (The forced MFMA path keeps to the aligned form.)
+    const bool any_ok = !mfma_ok && g.path == KUTACC_HIP_PATH_AUTO && second == nullptr && (g.a_stride_k == 1 || (g.a_stride_m == 1 && !gated)) &&
+                        (g.b_stride_k == 1 || (g.b_stride_n == 1 && !gated));
     if (g.path == KUTACC_HIP_PATH_GENERIC) {
         mfma_ok = false;
     } else if (g.path == KUTACC_HIP_PATH_FUSED && !mfma_ok) {
         return KUTACC_HIP_EUNSUPPORTED;
+    }
+    if (any_ok) {
+        am = g.a_stride_k != 1, bm = g.b_stride_k != 1;
     }
     // Gated projections of 128 channels on dense operands have kernels of their own (gated_projection_fits): by default
     // the one with the weights in registers, at every size (one side, us, against the tiled kernel up to 384 x 384
@@ -1942,7 +1986,7 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
         return kutacc_launch::row_projection(g.a, g.a_stride_m, g.b, g.bias, g.c, g.c_stride_m, g.m, g.n, g.k, stream);
     }
     const double flops = 2.0 * (double)g.m * (double)g.n * (double)g.k * (double)p.batches * (gated ? 2.0 : 1.0);
-    if (!mfma_ok) {
+    if (!mfma_ok && !any_ok) {
         const int64_t total = g.m * g.n * g.batches;
         const int64_t blocks = (total + 255) / 256;
         if (blocks > INT32_MAX) {
@@ -1952,7 +1996,7 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
         pair_gemm_scalar_kernel<<<dim3((unsigned)blocks), 256, 0, stream>>>(p);
         return kutacc_hip_status(hipGetLastError());
     }
-    if (!gated && am == bm && g.bias_axis == 0 && !g.relu) {
+    if (mfma_ok && !gated && am == bm && g.bias_axis == 0 && !g.relu) {
         const int rc = large_tiles(p, am, flops, stream);
         if (rc != KUTACC_HIP_EUNSUPPORTED) {
             return rc;
@@ -1967,7 +2011,13 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
     kutacc_prof::KernelTimer t(gated ? "pair_gemm_kernel<gated>" : (am || bm ? "pair_gemm_kernel<m-major>" : "pair_gemm_kernel"),
                                flops, stream);
     hipError_t e;
-    if (gated) {
+    if (any_ok) {
+        e = gated      ? launch_tiles<false, false, true, true>(p, blocks, stream)
+            : am && bm ? launch_tiles<true, true, false, true>(p, blocks, stream)
+            : am       ? launch_tiles<true, false, false, true>(p, blocks, stream)
+            : bm       ? launch_tiles<false, true, false, true>(p, blocks, stream)
+                       : launch_tiles<false, false, false, true>(p, blocks, stream);
+    } else if (gated) {
         e = launch_tiles<false, false, true>(p, blocks, stream);
     } else if (am && bm) {
         e = launch_tiles<true, true, false>(p, blocks, stream);

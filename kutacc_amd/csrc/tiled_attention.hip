@@ -37,7 +37,6 @@ struct TileParams {
     int64_t bias_sb, nb_sh, nb_sq;
     int B, S, H, hd;
     int groups, groups_q, query_blocks; // placement of workgroups, below
-    int v_vec, nb_vec;                  // rows of v / of the pair bias can be read 16 bytes at a time
     float scale;
 };
 
@@ -50,25 +49,6 @@ constexpr int GROUP_ROWS = 8, GROUP_QBLOCKS = 8;
 // registers.  Both hold if row i of the K fragment is key swap23(i) of the block (bits 2 and 3 of the index exchanged):
 // register 8 j + e of lane half g is then key 16 j + 8 g + e.
 __device__ __forceinline__ int swap23(int i) { return (i & ~12) | ((i & 4) << 1) | ((i & 8) >> 1); }
-
-__device__ __forceinline__ uint4 zero_u4() { return make_uint4(0u, 0u, 0u, 0u); }
-
-// eight bf16 at src[0 .. 7]; elements from `valid` on are zero (never read)
-__device__ __forceinline__ uint4 load8_checked(const bf16_t *src, int valid)
-{
-    union {
-        uint4 u;
-        bf16_t e[8];
-    } c;
-    c.u = zero_u4();
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        if (i < valid) {
-            c.e[i] = src[i];
-        }
-    }
-    return c.u;
-}
 
 // acc + the sum of eight bf16: four dot products of a pair with (1, 1)
 __device__ __forceinline__ float pair_sums(bf16x8 v, float acc)
@@ -139,7 +119,7 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const TileParam
     // What a thread stages of every chunk: PK 16-byte pieces of K (key kap, values 8 o .. 8 o + 7 of the head) and DB of
     // V^T (value d, keys 8 ko .. 8 ko + 7 of the chunk); pieces that lie in the padding are stored as zeros.
     int k_kap[PK], k_slot[PK], v_slot[DB];
-    int64_t k_off[PK], v_off[DB];
+    int64_t k_off[PK], v_row[DB], v_off[DB];
     bool k_real[PK], v_real[DB];
 #pragma unroll
     for (int i = 0; i < PK; ++i) {
@@ -155,17 +135,17 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const TileParam
         const int idx = tid + 256 * i;
         const int d = idx >> 3, ko = idx & 7;
         v_real[i] = d < hd;
-        v_off[i] = (int64_t)(v_real[i] ? d : 0) * p.v_se + 8 * ko;
+        v_row[i] = (int64_t)(v_real[i] ? d : 0) * p.v_se;
+        v_off[i] = v_row[i] + 8 * ko;
         v_slot[i] = K_SLOTS + ((d >> 5) * 4 + (ko >> 1)) * 64 + (d & 31) + 32 * (ko & 1);
     }
     auto keep = [](uint4 v, bool ok) { // a select, not a branch around the load
         const uint32_t m = ok ? 0xffffffffu : 0u;
         return make_uint4(v.x & m, v.y & m, v.z & m, v.w & m);
     };
-    // Two forms of the loads of a chunk.  PLAIN: every key of the chunk exists and every row can be read 16 bytes at a
-    // time -- no condition anywhere (a thread without a piece of its own repeats another thread's, to the same slot), so
+    // Two forms of the loads of a chunk.  PLAIN: every key of the chunk exists -- no condition anywhere (a thread without a piece of its own repeats another thread's, to the same slot), so
     // that the loop made of such chunks is one basic block per phase and the loads stay in flight across the compute
-    // phase.  Otherwise: the checked form (clamped rows, element-wise reads past alignment or the end).  Nothing touches
+    // phase.  Otherwise: the checked form (clamped rows and ends).  Nothing touches
     // what a load returns before park(): a use right behind the load makes the wave wait out the memory latency.
     uint4 kreg[PK], vreg[DB];
     bool k_keep[PK];
@@ -183,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const TileParam
         if constexpr (PLAIN) {
 #pragma unroll
             for (int i = 0; i < DB; ++i) {
-                vreg[i] = *reinterpret_cast<const uint4 *>(vbase + v_off[i] + kc0);
+                vreg[i] = load8_any(vbase + v_off[i], kc0);
             }
             bias_raw = bias_row[kc0 + (tid & (CHUNK - 1))];
             bias_keep = true;
@@ -193,8 +173,7 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const TileParam
                 const int key = kc0 + 8 * ((tid + 256 * i) & 7);
                 vreg[i] = zero_u4();
                 if (v_real[i] && key < S) {
-                    const bf16_t *src = vbase + v_off[i] + kc0;
-                    vreg[i] = (p.v_vec && key + 8 <= S) ? *reinterpret_cast<const uint4 *>(src) : load8_checked(src, S - key);
+                    vreg[i] = load8_checked(vbase + v_row[i], key, S);
                 }
             }
             const int key = kc0 + (tid & (CHUNK - 1));
@@ -231,10 +210,9 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const TileParam
                 if constexpr (HAS_NB) {
                     const int key = c * CHUNK + 32 * kb + 16 * j + 8 * g;
                     if constexpr (PLAIN) {
-                        f.v[kb][j] = *reinterpret_cast<const uint4 *>(nb_row + key);
+                        f.v[kb][j] = load8_any(nb_row, key);
                     } else if (key < S) {
-                        f.v[kb][j] = (p.nb_vec && key + 8 <= S) ? *reinterpret_cast<const uint4 *>(nb_row + key)
-                                                                : load8_checked(nb_row + key, S - key);
+                        f.v[kb][j] = load8_checked(nb_row, key, S);
                     }
                 }
             }
@@ -259,7 +237,7 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const TileParam
         m_run = -INFINITY, l_run = 0.f;
         NbRegs nb_cur, nb_next;
         // chunks [0, plain) take the PLAIN loads
-        const int plain = (p.v_vec && (!HAS_NB || p.nb_vec)) ? S / CHUNK : 0;
+        const int plain = S / CHUNK;
         if (plain > 0) {
             fetch(0, std::true_type{});
             nb_cur = fetch_nb(0, std::true_type{});
@@ -472,8 +450,6 @@ int gating_attention_tiled(const kutacc_hip_attention_args_t &a, hipStream_t str
     p.query_blocks = (int)((S + QUERIES - 1) / QUERIES);
     p.groups_q = (p.query_blocks + GROUP_QBLOCKS - 1) / GROUP_QBLOCKS;
     p.groups = (int)(H * ((B + GROUP_ROWS - 1) / GROUP_ROWS) * p.groups_q);
-    p.v_vec = (aligned16(a.v) && a.v_stride_e % 8 == 0 && a.v_stride_b % 8 == 0) ? 1 : 0;
-    p.nb_vec = (p.nb != nullptr && aligned16(p.nb) && a.nb_stride_h % 8 == 0 && a.nb_stride_q % 8 == 0) ? 1 : 0;
     // (float)(1 / sqrt(head_size)) as the reference forms it (gating_attention.cpp:68)
     p.scale = (float)(1.0 / sqrt((double)hd));
     const int64_t blocks = ((int64_t)p.groups + 7) / 8 * 8 * 64;

@@ -265,6 +265,49 @@ def test_gemm_seeded_sweep(torch_cuda, index, nb, M, N, K, am, bm, bias_axis, re
     helpers.assert_within(got, ref, GEMM_TOL(ref), f"gemm sweep {index}: {nb}x{M}x{N}x{K} am={am} bm={bm}")
 
 
+@pytest.mark.parametrize("nb,M,N,K", [(1, 5, 3, 2), (2, 33, 37, 29), (1, 129, 131, 65), (3, 127, 8, 71), (2, 64, 250, 128), (1, 300, 129, 201)])
+@pytest.mark.parametrize("a_mmajor,b_mmajor", [(False, False), (True, True), (True, False), (False, True)])
+def test_gemm_any_extent(torch_cuda, nb, M, N, K, a_mmajor, b_mmajor):
+    """Extents and pitches that are no multiples of 8 on the tiled kernel's unaligned form: last pieces of rows, rows shorter than
+    a piece, results whose rows start on odd elements, every orientation and bias axis; nothing written past n."""
+    for bias_axis in (0, 1, 2):
+        rng = np.random.Generator(np.random.PCG64(1200 + M + N))
+        A, B = draw(rng, nb, M, K), draw(rng, nb, N, K, scale=1 / math.sqrt(K))
+        bias = rng.standard_normal(N if bias_axis == 1 else M).astype(np.float32) if bias_axis else None
+        res = {}
+        name = first_profiled_kernel(torch_cuda, lambda: res.setdefault("c", run_gemm(torch_cuda, A, B, a_mmajor=a_mmajor, b_mmajor=b_mmajor,
+                                                                                     bias=bias, bias_axis=bias_axis, c_pad=3)))
+        assert name.startswith("pair_gemm_kernel"), name
+        ref = gemm_ref(A, B, bias, bias_axis)
+        helpers.assert_within(res["c"], ref, GEMM_TOL(ref), f"gemm {nb, M, N, K} axis {bias_axis}")
+
+
+@pytest.mark.parametrize("M,N,K", [(6, 49, 5), (65, 130, 67), (128, 259, 128)])
+def test_gemm_gated_form_any_extent(torch_cuda, M, N, K):
+    torch = torch_cuda
+    rng = np.random.Generator(np.random.PCG64(1300 + N))
+    A, G, B = draw(rng, 1, M, K), draw(rng, 1, M, K), draw(rng, 1, N, K, scale=1 / math.sqrt(K))
+    mask = (rng.random((1, N)) > 0.2).astype(np.float32)
+    bias, bias_gate = (rng.standard_normal(M).astype(np.float32) for _ in range(2))
+    t = [dev(torch, A), dev(torch, G), dev(torch, B), dev(torch, mask), dev(torch, bias, torch.float32), dev(torch, bias_gate, torch.float32)]
+    dC = torch.full((M * N + 64,), -7.0, dtype=torch.bfloat16, device="cuda")
+    g = capi.HipGemmArgs()
+    g.m, g.n, g.k, g.batches, g.dtype, g.path = M, N, K, 1, capi.K_BF16, capi.PATH_AUTO
+    g.a, g.a_gate, g.a_stride_m, g.a_stride_k = t[0].data_ptr(), t[1].data_ptr(), K, 1
+    g.b, g.b_stride_n, g.b_stride_k = t[2].data_ptr(), K, 1
+    g.c, g.c_stride_m, g.mask = dC.data_ptr(), N, t[3].data_ptr()
+    g.bias, g.bias_gate, g.bias_axis = t[4].data_ptr(), t[5].data_ptr(), 2
+    name = first_profiled_kernel(torch, lambda: capi.lib().kutacc_hip_gemm(ctypes.byref(g), None))
+    torch.cuda.synchronize()
+    assert name == "pair_gemm_kernel<gated>", name
+    proj, gate = gemm_ref(A, B, bias, 2), gemm_ref(G, B, bias_gate, 2)
+    proj, gate = round_to_bf16(proj.astype(np.float32)).astype(np.float64), round_to_bf16(gate.astype(np.float32)).astype(np.float64)
+    ref = (proj * mask[:, None, :] / (1.0 + np.exp(-gate)))[0]
+    got = helpers.to_numpy(dC)
+    helpers.assert_within(got[:M * N].reshape(M, N), ref, 2e-3 + 1.2e-2 * np.abs(ref), f"gated gemm {M, N, K}")
+    assert np.all(got[M * N:] == -7.0)
+
+
 def test_gemm_rejects_what_it_cannot_run(torch_cuda):
     torch = torch_cuda
     t = torch.zeros(64 * 64, dtype=torch.bfloat16, device="cuda")
