@@ -74,6 +74,10 @@ int gemm_nt(int32_t dtype, const void *a, int64_t lda, const void *w, int64_t ld
 bool tiled_attention_supports(const kutacc_hip_attention_args_t &args);
 int gating_attention_tiled(const kutacc_hip_attention_args_t &args, hipStream_t stream);
 
+// small_head_attention.hip: the attention step of that route for heads of 8, on the same tensors
+bool small_head_attention_supports(const kutacc_hip_attention_args_t &args);
+int small_head_attention(const kutacc_hip_attention_args_t &args, hipStream_t stream);
+
 // fp32_attention.hip: fp32 storage on the fp32 matrix core (head_size 32, up to 256 channels, up to 224 positions)
 bool fp32_attention_supports(const kutacc_hip_attention_args_t &args);
 int gating_attention_fp32(const kutacc_hip_attention_args_t &args, hipStream_t stream);

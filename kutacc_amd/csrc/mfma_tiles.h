@@ -124,7 +124,7 @@ __device__ __forceinline__ uint4 zero_u4() { return make_uint4(0u, 0u, 0u, 0u); 
 // Eight bf16 from a row of `length`, from element `at` on; elements past the end are zero (never read).  Rows start on any
 // even address: the hardware's unaligned 16-byte loads serve them, and the last piece of a row is the row's last eight
 // elements, shifted down.
-__device__ __forceinline__ uint4 load8_any(const bf16_t *row, int at)
+__device__ __forceinline__ uint4 load8_any(const bf16_t *row, uint32_t at)
 {
     uint4 v;
     __builtin_memcpy(&v, row + at, 16);

@@ -437,6 +437,11 @@ int gating_attention_tiled(const kutacc_hip_attention_args_t &a, hipStream_t str
         (rc = project(a.input, a.input_ld, M, a.gating_w, C, C, C, a.gate, a.gate_stride_s, a.gating_b, stream))) {
         return rc;
     }
+    if (small_head_attention_supports(a)) {
+        kutacc_prof::KernelTimer t("attention_tiles_kernel", 4.0 * (double)B * (double)S * (double)S * (double)C, stream);
+        rc = small_head_attention(a, stream);
+        return rc != 0 ? rc : project(a.avg, a.avg_stride_s, M, a.output_w, C, C, C, a.out, a.out_ld, a.output_b, stream);
+    }
     TileParams p;
     p.q = (const bf16_t *)a.q, p.k = (const bf16_t *)a.k, p.v = (const bf16_t *)a.v, p.gate = (const bf16_t *)a.gate;
     p.bias = (const bf16_t *)a.bias, p.nb = (const bf16_t *)a.nonbatched_bias, p.avg = (bf16_t *)a.avg;

@@ -144,6 +144,23 @@ def test_large_pair_bias_and_logit_offsets(torch_cuda):
     run_and_check(w)
 
 
+@pytest.mark.parametrize("B,S", [(1, 1), (2, 7), (4, 32), (5, 33), (3, 128), (9, 130), (4, 385), (1, 1120), (2, 1121)])
+@pytest.mark.parametrize("pair_bias", [True, False])
+def test_heads_of_eight_at_tile_edges(torch_cuda, B, S, pair_bias):
+    """One position, less than one piece of eight, whole blocks of 32 and one key past them, four to eight waves, sets of
+    four batch rows with one to four members, the longest row whose keys lie in the LDS and the first past it; keys masked
+    from a late tile on, a fully masked row, and queries whose logits leave the range of the unshifted softmax."""
+    w = draw_workload(60 + S, B, S, 8, 8, pair_bias=pair_bias, masked=0.0)
+    w.bias[B // 2, max(1, 2 * S // 3):] = MASK_BIAS
+    w.bias[B - 1, :] = MASK_BIAS if B > 1 else 0.0
+    if pair_bias:
+        w.nb[:, S // 2, :] += np.float32(150.0)
+        w.nb[:, S - 1, :] -= np.float32(150.0)
+        w.nb = round_to_bf16(w.nb)
+    w.bias = round_to_bf16(w.bias)
+    run_and_check(w)
+
+
 def test_pair_bias_entries_of_minus_infinity(torch_cuda):
     """Pairs excluded by a -inf pair bias get zero weight; a row keeps at least one finite key."""
     w = draw_workload(9, 2, 140, 4, 16)
