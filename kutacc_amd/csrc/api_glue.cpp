@@ -439,14 +439,17 @@ int kutacc_hip_transition_block(void *act, const float *ln_gamma, const float *l
         dtype != KUTACC_DTYPE_BF16) {
         return KUTACC_HIP_EINVAL;
     }
+    const int64_t norm_bytes = align256(rows * c_o * 2), need = kutacc_hip_transition_block_workspace(rows, c_o, c_i);
+    if (need != 0 && (need < 0 || !workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)) {
+        return KUTACC_HIP_EINVAL;
+    }
     hipStream_t s = kutacc_api::stream_or_default(stream);
     int rc = kutacc_launch::transition_block_fused(act, ln_gamma, ln_beta, ln_eps, w1, b1, w2, b2, rows, c_o, c_i, s);
     if (rc != KUTACC_HIP_EUNSUPPORTED) {
         return rc;
     }
     // three passes through the workspace: LayerNorm, the transition (its result takes the place of its input), residual
-    const int64_t norm_bytes = align256(rows * c_o * 2), need = norm_bytes + align256(rows * c_i * 2);
-    if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) {
+    if (!workspace || workspace_bytes < norm_bytes + align256(rows * c_i * 2) || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) {
         return KUTACC_HIP_EINVAL;
     }
     char *ws = static_cast<char *>(workspace);

@@ -62,6 +62,12 @@ static inline int kutacc_device_attribute(hipDeviceAttribute_t attr, int fallbac
     return v;
 }
 
+static inline int kutacc_cu_count()
+{
+    static int table[KUTACC_DEVICE_SLOTS] = {};
+    return kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, table);
+}
+
 namespace kutacc_launch {
 
 // generic_kernels.hip

@@ -26,7 +26,7 @@
 // The batched product of the triangle equation, where its sides are whole large tiles and there are enough of them,
 // runs on persistent kernels with 256 x 256 (or 192 x 192) tiles per workgroup: pair_gemm_direct_kernel, whose
 // operands go straight from global memory into the LDS, and pair_gemm_big_kernel, which stages them through
-// registers.  The transition keeps its hidden layer on chip (transition_fused_kernel); the gated projections of 128
+// registers.  The transition of 64, 128 and 256 channels is in transition.hip; the gated projections of 128
 // channels have kernels of their own that read the activation once (gated_projection_blocks_kernel, and
 // gated_projection_kernel behind a tuning switch).
 #include <hip/hip_runtime.h>
@@ -909,319 +909,6 @@ __global__ __launch_bounds__(256, 1) void pair_gemm_direct_kernel(const GemmPara
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the requests for a tile past the last one: let them land before the LDS is given back
 }
 
-// Transition with the hidden layer kept on chip: out = relu(x . W1^T + b1) . W2^T + b2 for row tiles of x
-// (reference src/attention/transition.cpp:31-38 runs two GEMMs through a [rows, c_i] intermediate; with
-// c_i = 4 c_o that intermediate is four fifths of the HBM traffic).  A wave owns RB blocks of 32 rows, whose
-// input fragments stay in registers; the workgroup streams the two weight matrices through LDS in slices
-// of 64 hidden units, double buffered, one barrier per slice.  Both products are formed transposed
-// (MFMA rows = hidden units, then output channels; columns = rows of x): the accumulators of the first,
-// after bias, ReLU and rounding to bf16 (the reference's rounding point: its intermediate is a bf16
-// tensor), are the B operand of the second without leaving the registers.  For that the lane that feeds
-// MFMA row i with a row of W1 takes hidden unit sigma(i) (bits 2 and 3 of i swapped), which makes the
-// eight values a lane holds per k-step consecutive hidden units.
-typedef __attribute__((ext_vector_type(2))) float f32x2;
-
-__device__ __forceinline__ int sigma_row(int r) { return (r & 0x13) | ((r & 4) << 1) | ((r & 8) >> 1); }
-
-//
-// BLOCK: the whole transition block of an Evoformer layer in place, out += transition(LayerNorm(out)) with x == out.
-// The rows are normalised between their coalesced load and the fragment staging (a row's 16-byte chunks sit in the 8
-// lanes that loaded them: sums by DPP adds, arithmetic of reference src/normalization/layernorm_kernel.h:21-53), and
-// the epilogue re-reads the rows in the order it writes them and adds.  One read and one write of the activation
-// for LayerNorm, both linears and the residual.
-template <int CO, int RB, bool BLOCK, int WAVES = 4>
-__global__ __launch_bounds__(64 * WAVES, 1) void transition_fused_kernel(const bf16_t *__restrict__ x,
-                                                                 const bf16_t *__restrict__ w1,
-                                                                 const float *__restrict__ b1,
-                                                                 const bf16_t *__restrict__ w2,
-                                                                 const float *__restrict__ b2, bf16_t *__restrict__ out,
-                                                                 int64_t rows, int c_i, const float *__restrict__ ln_gamma,
-                                                                 const float *__restrict__ ln_beta, float ln_eps)
-{
-    constexpr int KS = CO / 16; // k-steps of the first product
-    constexpr int CP = CO / 64; // 64-column panels across a row of x or W1
-    constexpr int CB = CO / 32; // 32-channel blocks of the output
-    constexpr int W1_PANELS = 2 * CP, STAGE_PANELS = W1_PANELS + CB, PPW = STAGE_PANELS / WAVES;
-    static_assert(STAGE_PANELS % WAVES == 0, "every wave stages the same number of weight panels");
-    extern __shared__ uint4 lds[]; // [2 stages][STAGE_PANELS][256 slots], one private panel per wave, b1 as fp32
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int r = lane & 31, g = lane >> 5, sr = sigma_row(r);
-    uint4 *xpanel = lds + 2 * STAGE_PANELS * 256 + wave * 256;
-    float *b1s = reinterpret_cast<float *>(lds + 2 * STAGE_PANELS * 256 + WAVES * 256);
-    for (int i = tid; i < c_i; i += 64 * WAVES) {
-        b1s[i] = b1[i]; // visible after the first barrier of the slice loop
-    }
-
-    int64_t row0 = ((int64_t)blockIdx.x * WAVES + wave) * (32 * RB);
-    const bool active = row0 < rows;
-    if (!active) {
-        row0 = rows - 1; // keeps every address valid; nothing is stored
-    }
-    const int last_local = (int)((rows - row0 < 32 * RB ? rows - row0 : 32 * RB) - 1);
-    const bf16_t *xb = x + row0 * CO;
-
-    auto fetch = [&](int jc, PanelRegs *wr) {
-        const int h0 = jc * 64;
-#pragma unroll
-        for (int i = 0; i < PPW; ++i) {
-            const int pnl = wave * PPW + i;
-            if (pnl < W1_PANELS) {
-                wr[i] = panel_load(w1 + (int64_t)(h0 + 32 * (pnl / CP)) * CO, CO, 0, 31, (pnl % CP) * 64, lane);
-            } else {
-                wr[i] = panel_load(w2 + (int64_t)((pnl - W1_PANELS) * 32) * c_i, c_i, 0, 31, h0, lane);
-            }
-        }
-    };
-    PanelRegs wr[PPW];
-    fetch(0, wr);
-
-    bf16x8 xf[RB][KS];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-        PanelRegs t[CP];
-#pragma unroll
-        for (int cp = 0; cp < CP; ++cp) {
-            t[cp] = panel_load(xb, CO, rb * 32, last_local, cp * 64, lane);
-        }
-        if constexpr (BLOCK) {
-            // lane (lane >> 3, lane & 7) holds chunk lane & 7 of every 64-channel panel of rows 8i + (lane >> 3)
-            float gm[CP][8], bt[CP][8];
-#pragma unroll
-            for (int cp = 0; cp < CP; ++cp) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    gm[cp][e] = ln_gamma[cp * 64 + (lane & 7) * 8 + e];
-                    bt[cp][e] = ln_beta[cp * 64 + (lane & 7) * 8 + e];
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                uint4 *regs[CP];
-#pragma unroll
-                for (int cp = 0; cp < CP; ++cp) {
-                    regs[cp] = i == 0 ? &t[cp].r0 : i == 1 ? &t[cp].r1 : i == 2 ? &t[cp].r2 : &t[cp].r3;
-                }
-                const float x0 = __shfl(to_f32(as_bf16x8(*regs[0])[0]), lane & ~7, 64); // first element of the row
-                float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-                for (int cp = 0; cp < CP; ++cp) {
-                    const bf16x8 b = as_bf16x8(*regs[cp]);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float d = to_f32(b[e]) - x0;
-                        s1 += d;
-                        s2 = fmaf(d, d, s2);
-                    }
-                }
-                s1 = group_sum<8>(s1);
-                s2 = group_sum<8>(s2);
-                const float n = (float)CO;
-                const float mean = s1 / n + x0;
-                const float var = fmaxf((s2 - s1 * s1 / n) / n, 0.f);
-                const float rstd = 1.0f / sqrtf(var + ln_eps);
-                const float shift = -rstd * mean;
-#pragma unroll
-                for (int cp = 0; cp < CP; ++cp) {
-                    const bf16x8 b = as_bf16x8(*regs[cp]);
-                    bf16x8 o;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        o[e] = (bf16_t)fmaf(fmaf(to_f32(b[e]), rstd, shift), gm[cp][e], bt[cp][e]);
-                    }
-                    *regs[cp] = as_uint4(o);
-                }
-            }
-        }
-#pragma unroll
-        for (int cp = 0; cp < CP; ++cp) {
-            panel_store(xpanel, lane, t[cp]);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                xf[rb][cp * 4 + k] = as_bf16x8(xpanel[panel_slot(r, 2 * k + g)]);
-            }
-        }
-    }
-
-    f32x16 oacc[RB][CB];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) {
-            oacc[rb][cb] = zero16();
-        }
-    }
-
-    // Blocks of 32 hidden units, t = 0 .. c_i/32 - 1; block t lives in slice t/2.  The loop is software-pipelined by
-    // hand: while the matrix core runs the first product of block t+1, the vector ALU turns the finished accumulators
-    // of block t into the bf16 operand of its second product (bias, ReLU, rounding), whose MFMAs follow.  Fences keep
-    // the compiler from pulling the two instruction streams apart again.
-    auto first_product = [&](const uint4 *stage, int hb, f32x16 (&hn)[RB]) {
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            hn[rb] = zero16();
-        }
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const bf16x8 a = as_bf16x8(stage[(hb * CP + ks / 4) * 256 + panel_slot(sr, 2 * (ks % 4) + g)]);
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) {
-                hn[rb] = mfma(a, xf[rb][ks], hn[rb]);
-            }
-        }
-    };
-    // element pair q of k-step s2 of block t: + b1, ReLU, round to bf16 (the pair form maps onto one conversion)
-    auto convert_pair = [&](const f32x16 (&hc)[RB], const float *bp, int s2, int q, bf16x2 (&w)[RB][2][4]) {
-        const f32x2 bias = *reinterpret_cast<const f32x2 *>(bp + 16 * s2 + 2 * q);
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            const f32x2 pr = {fmaxf(hc[rb][8 * s2 + 2 * q] + bias[0], 0.f), fmaxf(hc[rb][8 * s2 + 2 * q + 1] + bias[1], 0.f)};
-            w[rb][s2][q] = __builtin_convertvector(pr, bf16x2);
-        }
-    };
-    // first product of the next block (if any) interleaved with the conversion of the current one
-    auto overlap = [&](const uint4 *stage_next, int hb_next, bool have_next, f32x16 (&hn)[RB], const f32x16 (&hc)[RB], int t,
-                       bf16x8 (&hf)[RB][2]) {
-        const float *bp = b1s + t * 32 + 8 * g;
-        bf16x2 w[RB][2][4];
-        if (have_next) {
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) {
-                hn[rb] = zero16();
-            }
-            constexpr int PER = KS / 8; // k-steps per converted pair
-            // all weight fragments of the block are requested up front: with one wave per SIMD nothing else hides an
-            // LDS round trip, and the fences below would otherwise pin each read right in front of its MFMA
-            bf16x8 af[KS];
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                af[ks] = as_bf16x8(stage_next[(hb_next * CP + ks / 4) * 256 + panel_slot(sr, 2 * (ks % 4) + g)]);
-            }
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const bf16x8 a = af[ks];
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb) {
-                    hn[rb] = mfma(a, xf[rb][ks], hn[rb]);
-                }
-                if (ks % PER == 0) {
-                    convert_pair(hc, bp, (ks / PER) >> 2, (ks / PER) & 3, w);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                convert_pair(hc, bp, i >> 2, i & 3, w);
-            }
-        }
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-                const bf16x8 all = {w[rb][s2][0][0], w[rb][s2][0][1], w[rb][s2][1][0], w[rb][s2][1][1],
-                                    w[rb][s2][2][0], w[rb][s2][2][1], w[rb][s2][3][0], w[rb][s2][3][1]};
-                hf[rb][s2] = all;
-            }
-        }
-    };
-    auto second_fragments = [&](const uint4 *stage, int hb, bf16x8 (&a2)[CB][2]) {
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) {
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-                a2[cb][s2] = as_bf16x8(stage[(W1_PANELS + cb) * 256 + panel_slot(r, 2 * (2 * hb + s2) + g)]);
-            }
-        }
-    };
-    auto second_product = [&](const bf16x8 (&a2)[CB][2], const bf16x8 (&hf)[RB][2]) {
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) {
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb) {
-                    oacc[rb][cb] = mfma(a2[cb][s2], hf[rb][s2], oacc[rb][cb]);
-                }
-            }
-        }
-    };
-
-    const int NJ = c_i / 64;
-#pragma unroll
-    for (int i = 0; i < PPW; ++i) {
-        panel_store(lds + (wave * PPW + i) * 256, lane, wr[i]);
-    }
-    __syncthreads();
-    if (NJ > 1) {
-        fetch(1, wr);
-    }
-    f32x16 ha[RB], hb_[RB];
-    first_product(lds, 0, ha);
-    for (int jc = 0; jc < NJ; ++jc) {
-        const uint4 *stage = lds + (jc & 1) * STAGE_PANELS * 256;
-        uint4 *other = lds + ((jc + 1) & 1) * STAGE_PANELS * 256;
-        const bool more = jc + 1 < NJ;
-        // every wave is done with the other stage (its last readers were the second products of the previous slice)
-        __syncthreads();
-        if (more) {
-#pragma unroll
-            for (int i = 0; i < PPW; ++i) {
-                panel_store(other + (wave * PPW + i) * 256, lane, wr[i]);
-            }
-            if (jc + 2 < NJ) {
-                fetch(jc + 2, wr);
-            }
-        }
-        bf16x8 hf[RB][2], a2[CB][2];
-        second_fragments(stage, 0, a2); // on their way while the first product of the next block runs
-        overlap(stage, 1, true, hb_, ha, 2 * jc, hf);
-        second_product(a2, hf);
-        __syncthreads(); // the other stage is complete and visible before the first product of its block 0 reads it
-        second_fragments(stage, 1, a2);
-        overlap(other, 0, more, ha, hb_, 2 * jc + 1, hf);
-        second_product(a2, hf);
-    }
-
-    // accumulators (+ b2) -> bf16 through the private panel, 64 channels at a time, out as whole 128-byte runs
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-        for (int half = 0; half < CB / 2; ++half) {
-#pragma unroll
-            for (int n = 0; n < 2; ++n) {
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    const f32x4 bv = *reinterpret_cast<const f32x4 *>(b2 + (2 * half + n) * 32 + 8 * a + 4 * g);
-                    bf16x4 ov;
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        ov[c] = (bf16_t)(oacc[rb][2 * half + n][4 * a + c] + bv[c]);
-                    }
-                    *(reinterpret_cast<bf16x4 *>(xpanel + panel_slot(r, n * 4 + a)) + g) = ov;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int prow = 8 * i + (lane >> 3);
-                uint4 v = xpanel[panel_slot(prow, lane & 7)];
-                if (active && rb * 32 + prow <= last_local) {
-                    bf16_t *dst = out + (row0 + rb * 32 + prow) * CO + half * 64 + (lane & 7) * 8;
-                    if constexpr (BLOCK) { // residual: the row as it was before the LayerNorm
-                        const bf16x8 o = as_bf16x8(v), z = as_bf16x8(*reinterpret_cast<const uint4 *>(dst));
-                        bf16x8 res;
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            res[e] = (bf16_t)(to_f32(z[e]) + to_f32(o[e]));
-                        }
-                        v = as_uint4(res);
-                    }
-                    *reinterpret_cast<uint4 *>(dst) = v;
-                }
-            }
-        }
-    }
-}
-
 // Gated projection of the triangle multiplication for 128 pair channels and 128 projected channels
 // (reference src/attention/triangle_multiplication.cpp:37-66):
 //   out[c][p] = bf16( bf16(x[p] . wp[c] + bp[c]) * mask[p] * sigmoid(x[p] . wg[c] + bg[c]) )
@@ -1767,76 +1454,9 @@ hipError_t launch_gated_projection_blocks(const kutacc_hip_gemm_args_t &g, hipSt
     return hipGetLastError();
 }
 
-constexpr int MAX_HIDDEN = 2048; // hidden units whose bias fits next to the weight stages in LDS
-
-template <int CO, int RB, bool BLOCK, int WAVES = 4>
-hipError_t launch_transition(const void *x, const void *w1, const float *b1, const void *w2, const float *b2, void *out,
-                             int64_t rows, int c_i, const float *ln_gamma, const float *ln_beta, float ln_eps,
-                             hipStream_t stream)
-{
-    constexpr int STAGE_PANELS = 2 * (CO / 64) + CO / 32;
-    const size_t lds_bytes = (size_t)(2 * STAGE_PANELS + WAVES) * 4096 + (size_t)c_i * sizeof(float);
-    static size_t configured[KUTACC_DEVICE_SLOTS] = {};
-    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&transition_fused_kernel<CO, RB, BLOCK, WAVES>),
-                                               (size_t)(2 * STAGE_PANELS + WAVES) * 4096 + MAX_HIDDEN * sizeof(float), configured)) {
-        return e;
-    }
-    const int64_t per_group = 32 * RB * WAVES;
-    const int64_t blocks = (rows + per_group - 1) / per_group;
-    transition_fused_kernel<CO, RB, BLOCK, WAVES><<<dim3((unsigned)blocks), 64 * WAVES, lds_bytes, stream>>>(
-        (const bf16_t *)x, (const bf16_t *)w1, b1, (const bf16_t *)w2, b2, (bf16_t *)out, rows, c_i, ln_gamma, ln_beta, ln_eps);
-    return hipGetLastError();
-}
 } // namespace
 
 namespace kutacc_launch {
-
-bool transition_fused_supports(int64_t rows, int64_t c_o, int64_t c_i, const void *x, const void *w1, const float *b1,
-                               const void *w2, const float *b2, const void *out)
-{
-    return (c_o == 128 || c_o == 256) && c_i >= 64 && c_i % 64 == 0 && c_i <= MAX_HIDDEN && rows > 0 &&
-           rows <= ((int64_t)1 << 31) * 64 && kutacc_hip_aligned16(x) && kutacc_hip_aligned16(w1) && kutacc_hip_aligned16(b1) && kutacc_hip_aligned16(w2) &&
-           kutacc_hip_aligned16(b2) && kutacc_hip_aligned16(out);
-}
-
-// 128 channels: eight waves of 32 rows each per workgroup (one workgroup per CU, two waves per SIMD, which hide each
-// other's LDS round trips and barriers).  Measured against four waves of 64 rows, which reads every weight fragment from
-// LDS half as often but leaves a SIMD to one wave: 12 % faster for the transition at n = 384, 14 % for the block with
-// its LayerNorm and residual, 5 % and 17 % at n = 1024.  (With the four-wave kernel a separate, smaller-workgroup launch
-// for the rows of a last, partial round of workgroups paid off; with this one it no longer does.)
-template <bool BLOCK>
-static hipError_t launch_transition_128(const void *x, const void *w1, const float *b1, const void *w2, const float *b2, void *out,
-                                        int64_t rows, int c_i, const float *ln_gamma, const float *ln_beta, float ln_eps,
-                                        hipStream_t stream)
-{
-    return launch_transition<128, 1, BLOCK, 8>(x, w1, b1, w2, b2, out, rows, c_i, ln_gamma, ln_beta, ln_eps, stream);
-}
-
-int transition_fused(const void *x, const void *w1, const float *b1, const void *w2, const float *b2, void *out,
-                     int64_t rows, int64_t c_o, int64_t c_i, hipStream_t stream)
-{
-    if (!transition_fused_supports(rows, c_o, c_i, x, w1, b1, w2, b2, out)) {
-        return KUTACC_HIP_EUNSUPPORTED;
-    }
-    kutacc_prof::KernelTimer t("transition_fused_kernel", 4.0 * (double)rows * (double)c_o * (double)c_i, stream);
-    const hipError_t e = c_o == 128 ? launch_transition_128<false>(x, w1, b1, w2, b2, out, rows, (int)c_i, nullptr, nullptr, 0.f, stream)
-                                    : launch_transition<256, 1, false>(x, w1, b1, w2, b2, out, rows, (int)c_i, nullptr, nullptr, 0.f, stream);
-    return kutacc_hip_status(e);
-}
-
-// act += transition(LayerNorm(act)) in place, one kernel
-int transition_block_fused(void *act, const float *ln_gamma, const float *ln_beta, float ln_eps, const void *w1, const float *b1,
-                           const void *w2, const float *b2, int64_t rows, int64_t c_o, int64_t c_i, hipStream_t stream)
-{
-    if (!ln_gamma || !ln_beta || !transition_fused_supports(rows, c_o, c_i, act, w1, b1, w2, b2, act)) {
-        return KUTACC_HIP_EUNSUPPORTED;
-    }
-    kutacc_prof::KernelTimer t("transition_fused_kernel<block>", 4.0 * (double)rows * (double)c_o * (double)c_i, stream);
-    const hipError_t e =
-        c_o == 128 ? launch_transition_128<true>(act, w1, b1, w2, b2, act, rows, (int)c_i, ln_gamma, ln_beta, ln_eps, stream)
-                   : launch_transition<256, 1, true>(act, w1, b1, w2, b2, act, rows, (int)c_i, ln_gamma, ln_beta, ln_eps, stream);
-    return kutacc_hip_status(e);
-}
 
 int pair_gemm_tuning(const char *name, const char *value)
 {

@@ -247,12 +247,6 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
 
 size_t lds_bytes(int NB) { return (size_t)(2 * NB + 1) * TILE * 16 + (size_t)(TILE * NB + 1) * 4; }
 
-int cu_count()
-{
-    static int table[KUTACC_DEVICE_SLOTS] = {};
-    return kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, table);
-}
-
 template <bool HAS_NB>
 int launch(SmallHeadParams p, hipStream_t stream)
 {
@@ -265,7 +259,7 @@ int launch(SmallHeadParams p, hipStream_t stream)
     // multiple of four leaves SIMDs without their share: 1024 rows of 301 took 288 us at five waves, 240 at eight, 200 at four.
     const int waves = std::min(p.NB, 3 * lds <= (size_t)CU_LDS_BYTES ? 4 : 8);
     // a set's queries are dealt to several workgroups, each staging the keys again, only while the chip has room for them
-    const int turns = (p.NB + waves - 1) / waves, room = 2 * cu_count() / std::max(1, p.sets * p.H);
+    const int turns = (p.NB + waves - 1) / waves, room = 2 * kutacc_cu_count() / std::max(1, p.sets * p.H);
     p.splits = std::max(1, std::min(turns, room));
     const int64_t blocks = (int64_t)(p.sets + 7) / 8 * 8 * p.H * p.splits;
     small_head_attention_kernel<HAS_NB><<<dim3((unsigned)blocks), 64 * waves, lds, stream>>>(p);

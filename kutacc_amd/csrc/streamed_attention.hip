@@ -488,12 +488,6 @@ __global__ __launch_bounds__(768) void streamed_attention_kernel(const StreamedP
     }
 }
 
-int cu_count()
-{
-    static int table[KUTACC_DEVICE_SLOTS] = {};
-    return kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, table);
-}
-
 template <int C>
 int launch_projection(const StreamedParams &p, hipStream_t stream)
 {
@@ -502,7 +496,7 @@ int launch_projection(const StreamedParams &p, hipStream_t stream)
         return kutacc_hip_status(e);
     }
     const int halves = C / 128; // workgroups that share a step, one per 128 channels of outputs
-    const int64_t steps = ((int64_t)p.B * p.NB + 1) / 2, cap = std::max(1, cu_count() / halves);
+    const int64_t steps = ((int64_t)p.B * p.NB + 1) / 2, cap = std::max(1, kutacc_cu_count() / halves);
     const int64_t per = (steps + cap - 1) / cap;
     kutacc_prof::KernelTimer t("qkvg_projection_kernel", 8.0 * (double)p.B * p.S * C * C, stream);
     qkvg_projection_kernel<C><<<dim3((unsigned)((steps + per - 1) / per), halves), 512, projection_lds<C>(), stream>>>(p, (int)per);

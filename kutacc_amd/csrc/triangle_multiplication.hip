@@ -467,12 +467,6 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
     }
 }
 
-int cu_count()
-{
-    static int table[KUTACC_DEVICE_SLOTS] = {};
-    return kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, table);
-}
-
 // equal runs of steps for at most `cap` workgroups
 struct Split {
     unsigned groups;
@@ -503,7 +497,7 @@ int triangle_front(const kutacc_hip_triangle_multiplication_args_t &a, void *lef
         return kutacc_hip_status(e);
     }
     kutacc_prof::KernelTimer t("gated_projection_blocks_kernel<2>", 8.0 * (double)(a.n_res * a.n_res) * C * C, stream);
-    const Split s = split_steps(a.n_res, np, cu_count());
+    const Split s = split_steps(a.n_res, np, kutacc_cu_count());
     const Side l = {(const bf16_t *)a.left_proj_w, (const bf16_t *)a.left_gate_w, a.left_proj_b, a.left_gate_b, (bf16_t *)left};
     const Side r = {(const bf16_t *)a.right_proj_w, (const bf16_t *)a.right_gate_w, a.right_proj_b, a.right_gate_b, (bf16_t *)right};
     triangle_front_kernel<<<dim3(s.groups), 64 * FRONT_WAVES, FRONT_LDS, stream>>>((const bf16_t *)a.pair_act, a.ln_in_gamma, a.ln_in_beta, a.ln_eps, l,
@@ -519,7 +513,7 @@ int triangle_back(const kutacc_hip_triangle_multiplication_args_t &a, const void
         return kutacc_hip_status(e);
     }
     kutacc_prof::KernelTimer t("triangle_back_kernel", 4.0 * (double)(a.n_res * a.n_res) * C * C, stream);
-    const Split s = split_steps(a.n_res, np, 2 * (int64_t)cu_count());
+    const Split s = split_steps(a.n_res, np, 2 * (int64_t)kutacc_cu_count());
     triangle_back_kernel<<<dim3(s.groups), 256, BACK_LDS, stream>>>(
         (const bf16_t *)centre, plane, a.ln_center_gamma, a.ln_center_beta, (const bf16_t *)a.output_w, a.output_b, (const bf16_t *)a.gating_w,
         a.gating_b, (bf16_t *)a.pair_act, a.ln_in_gamma, a.ln_in_beta, a.ln_eps, (int)a.n_res, (int)np, s.per_group);

@@ -584,6 +584,32 @@ def test_transition_block(torch_cuda, rows, c_o, c_i):
                                              capi.K_BF16, None) == capi.EINVAL
 
 
+# one row; a row past a wave's 32; the last row count of the kernel for few rows (32 per CU) and the first past it; whole
+# rounds of workgroups and a remainder, for each width; the narrowest and the widest hidden layer
+@pytest.mark.parametrize("rows,c_o,c_i", [(1, 64, 64), (1, 256, 64), (33, 128, 2048), (33, 64, 2048), (31, 256, 2048), (8192, 128, 192),
+                                          (8193, 128, 192), (8192, 256, 64), (8193, 256, 64), (98304 + 4133, 128, 64),
+                                          (65536 + 33, 256, 64), (131072 + 33, 64, 128)])
+def test_transition_block_at_the_edges_of_its_kernels(torch_cuda, rows, c_o, c_i):
+    from oracle import oracle
+    torch = torch_cuda
+    print(rows, c_o, c_i, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(rows + c_i)
+    draw = lambda *s, scale=1.0, centre=0.0: torch.randn(*s, device="cuda", generator=g) * scale + centre  # noqa: E731
+    act = draw(rows, c_o, scale=1.5, centre=0.3).to(torch.bfloat16)
+    gamma, beta, b1, b2 = draw(c_o, scale=0.1, centre=1.0), draw(c_o, scale=0.2), draw(c_i, scale=0.3), draw(c_o, scale=0.3)
+    w1, w2 = draw(c_i, c_o, scale=c_o ** -0.5).to(torch.bfloat16), draw(c_o, c_i, scale=c_i ** -0.5).to(torch.bfloat16)
+    num = helpers.to_numpy
+    x = num(act)
+    want = x + oracle.transition_f32(oracle.layernorm_rows_f32(x, num(gamma), num(beta), 1e-5), num(w1), num(b1), num(w2), num(b2))
+    L = capi.lib()
+    nbytes = L.kutacc_hip_transition_block_workspace(rows, c_o, c_i)
+    ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device="cuda")
+    assert L.kutacc_hip_transition_block(act.data_ptr(), gamma.data_ptr(), beta.data_ptr(), 1e-5, w1.data_ptr(), b1.data_ptr(),
+                                         w2.data_ptr(), b2.data_ptr(), ws.data_ptr(), nbytes, rows, c_o, c_i, capi.K_BF16, None) == 0
+    torch.cuda.synchronize()
+    helpers.check_close(num(act), want, "bf16", f"transition block {rows}x{c_o}->{c_i}")
+
+
 # ---- MSA attention blocks ------------------------------------------------------------------------------------------
 def msa_case(seed, n_seq, n_res, heads, c_z):
     rng = np.random.Generator(np.random.PCG64(seed))
