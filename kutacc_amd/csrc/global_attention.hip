@@ -6,11 +6,11 @@
 //   q_avg = sum_s mask[s] x[s,:] / (sum_s mask[s] + 1e-10);  q = q_avg.Wq^T  viewed [H, d]
 //   logit[h,s] = q[h].(Wk x[s]) / sqrt(d) + (mask[s]*1e9 - 1e9);  p = softmax_s
 //   wavg[h,:] = sum_s p[h,s] (Wv x[s]);  out[s,:] = (sigmoid(x[s].Wg^T + bg) * wavg).Wo^T + bo
-// One workgroup (four waves) owns a batch row and walks it in 32-token tiles in three phases: (A) masked
-// mean, (B) logits, online softmax and weighted average, (C) gate, gating and output projection.  Tiles
-// arrive with whole-cache-line loads through the wave's LDS staging panel, the next one in flight while
-// the current one is processed; up to seq_len 1024 a wave keeps the fragments of its tiles in registers
-// after phase A, so the row is read from memory once.  Nothing but q_avg and out is written to memory.  All contractions are v_mfma_f32_32x32x16_bf16:
+// One workgroup owns a batch row and walks it in 32-token tiles in three phases: (A) masked mean, (B) logits, online
+// softmax and weighted average, (C) gate, gating and output projection.  A wave keeps the fragments of its first tiles in
+// registers after phase A -- all of them up to 1024 tokens, 64 tiles of a longer row's -- and what is left of a longer row
+// is read again in phases B and C, straight into the LDS.  Nothing but q_avg and out is written to memory.  All
+// contractions are v_mfma_f32_32x32x16_bf16:
 //   B: logits^T[s, h] = X[s, :] . QK^T with QK[h, :] = q[h].Wk / sqrt(d) folded per batch row (heads are the
 //      columns, 8 of 32 used for H = 8); V[s, e] = X . Wv^T; O^T[e, h] += V^T . P^T -- the accumulators
 //      of the first two products are directly the operands of the third, as in the gated attention
@@ -34,6 +34,7 @@ using namespace kutacc_dev;
 namespace {
 
 constexpr int GC = 64;        // channels
+constexpr int PANEL_SLOTS = 288; // of a wave: 32 rows of 128 bytes, or 64 lanes of MERGE_LD floats
 constexpr int MERGE_LD = 18;  // floats per lane in the cross-wave merge area: m, l, 16 accumulators
 
 struct GlobalParams {
@@ -52,17 +53,18 @@ __device__ __forceinline__ int gate_channel(int rb, int v, int g)
     return 16 * (idx >> 3) + 8 * g + (idx & 7);
 }
 
-// CACHED: the row has at most 32 tiles (seq_len <= 1024), so each wave keeps the fragments of its (at most 8) tiles
-// in registers after phase A and the row is read from memory once; otherwise every phase streams the row again.
-template <bool CACHED, int NW>
+// A wave keeps the fragments of its first KEEP tiles in registers from phase A on.  STREAM: the row may have more tiles than
+// NW * KEEP; the rest is read again in every phase, straight into the LDS, two tiles of a wave ahead.
+// What bounds it: in phase C the vector ALU (two transcendentals per gate element, 67 % busy on a row that has the chip to
+// itself), in phases A and B the memory.  Measured at 5120 tokens x 384 rows: phases 48 + 36 + 100 us; 220 us with every
+// phase streaming the whole row through registers, 184 with 64 of its 160 tiles kept.  1508 x 107: 32.4 -> 24.9 us.
+template <int NW, int KEEP, bool STREAM>
 __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalParams p)
 {
     constexpr int NTHR = 64 * NW;
-    constexpr int MAXI = CACHED ? 32 / NW : (1 << 24); // tiles per wave
-    constexpr int UNR = CACHED ? 32 / NW : 1;          // the cached tile array needs compile-time indices
-    bf16x8 xs[CACHED ? 32 / NW : 1][4];
+    bf16x8 xs[KEEP][4];
     extern __shared__ uint4 lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
     const int b = blockIdx.x;
     const int S = p.S, NT = p.NT, H = p.H, d = p.d;
@@ -73,14 +75,16 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     uint4 *wg_frag = wv_frag + 256;  // [2 row blocks][4][64]
     uint4 *wo_frag = wg_frag + 512;  // [2 row blocks][4][64]
     uint4 *wk_rows = wo_frag + 512;  // the key weights as they lie in memory, [d][64 channels] bf16 (d <= 32)
-    uint4 *panel = wk_rows + 256 + wave * 256;
-    float *maskb = reinterpret_cast<float *>(wk_rows + 256 + NW * 256); // mask bias per token, -inf past S
-    float *mask01 = maskb + spad;                                       // mask value per token, 0 past S
-    float *part = mask01 + spad;                                        // [NW waves][68]: channel sums, mask sum
-    float *qavg = part + NW * 68;                                        // [64]
-    float *qv = qavg + GC;                                              // [64] q, bf16-rounded
-    float *wavg = qv + GC;                                              // [64]
-    float *merge = wavg + GC;                                           // [NW waves][64 lanes][MERGE_LD]
+    uint4 *panels = wk_rows + 256;                  // [NW][PANEL_SLOTS]: a panel of phase A, the merge area of phase B
+    uint4 *panel = panels + wave * PANEL_SLOTS;
+    uint4 *ring = panels + NW * PANEL_SLOTS + wave * 512; // STREAM: two tiles per wave
+    bf16_t *mask16 = reinterpret_cast<bf16_t *>(panels + NW * (PANEL_SLOTS + (STREAM ? 512 : 0))); // per token, -inf past S
+    float *part = reinterpret_cast<float *>(mask16 + spad); // [NW waves][68]: channel sums, mask sum
+    float *qavg = part + NW * 68;                           // [64]
+    float *qv = qavg + GC;                                  // [64] q, bf16-rounded
+    float *wavg = qv + GC;                                  // [64]
+    float *bos = wavg + GC;                                 // [64] output bias
+    float *merge = reinterpret_cast<float *>(panels);       // [NW waves][64 lanes][MERGE_LD]
 
     const bf16_t *xb = p.x + (int64_t)b * p.x_sb;
     const uint32_t x_pitch = (uint32_t)p.x_ss; // tokens of a row by 32-bit byte offsets from xb (the launcher checks the range)
@@ -88,13 +92,46 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     // Requested before anything else, so that their latency passes under the staging of the weights: the first tiles of
     // the row (all of a wave's tiles when they are kept in registers and there are at most four) and this thread's slice
     // of the query weights (output o = tid / TPR, channels part * 64 / TPR ...).
-    constexpr int PRE = CACHED ? (MAXI < 4 ? MAXI : 4) : 1;
+    constexpr int PRE = KEEP < 4 ? KEEP : 4;
     PanelRegs ahead[PRE];
 #pragma unroll
     for (int i = 0; i < PRE; ++i) {
         const int t = wave + NW * i;
         ahead[i] = panel_load_near(xb, x_pitch, (t < NT ? t : NT - 1) * 32, S - 1, 0, lane);
     }
+    const int first = wave + NW * KEEP; // first of the wave's tiles that are not kept
+    const uint32_t ring_lds = (uint32_t)(uintptr_t)(const lds_char *)ring;
+    auto ask = [&](int slot, int t) { // tile t into a slot of the ring, in the panel's layout
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int rl = lane >> 3, row = min(t * 32 + 8 * i + rl, S - 1);
+            load_to_lds(ring_lds + slot * 4096u + i * 1024u, xb, __umul24((uint32_t)row, 2u * x_pitch) + 16u * (uint32_t)((lane & 7) ^ rl ^ (i >> 1)));
+        }
+    };
+    auto stream_start = [&]() {
+        if (STREAM && first < NT) {
+            ask(0, first);
+            if (first + NW < NT) {
+                ask(1, first + NW);
+            }
+        }
+    };
+    struct Tile {
+        bf16x8 f[4];
+    };
+    auto ring_tile = [&](int slot, int t) { // out of the ring, and the tile after the next one asked for in its place
+        Tile x;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            x.f[ks] = as_bf16x8(ring[slot * 256 + panel_slot(r, 2 * ks + g)]);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (t + 2 * NW < NT) {
+            ask(slot, t + 2 * NW);
+        }
+        return x;
+    };
+    stream_start();
     constexpr int TPR = NTHR / GC, WQV = GC / TPR / 8; // threads per output of q, 16-byte pieces per thread
     uint4 wq_part[WQV];
 #pragma unroll
@@ -122,13 +159,10 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         wo_frag[idx] = *reinterpret_cast<const uint4 *>(p.wo + o * GC + ks * 16 + gg * 8);
     }
     for (int s = tid; s < spad; s += NTHR) {
-        float m = 0.f, mb = -INFINITY;
-        if (s < S) {
-            m = to_f32(p.mask[(int64_t)b * p.mask_sb + s]);
-            mb = fmaf(m, 1e9f, -1e9f); // reference :120-121
-        }
-        mask01[s] = m;
-        maskb[s] = mb;
+        mask16[s] = s < S ? p.mask[(int64_t)b * p.mask_sb + s] : (bf16_t)-INFINITY;
+    }
+    if (tid < GC) {
+        bos[tid] = p.bo[tid];
     }
     __syncthreads();
 
@@ -143,27 +177,9 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
             }
         }
         float msum = 0.f;
-        // the loads of the next PRE tiles are in flight while this one is summed
-#pragma unroll(UNR)
-        for (int i = 0; i < MAXI; ++i) {
-            const int t = wave + NW * i;
-            if (t >= NT) {
-                break;
-            }
-            bf16x8 xf[4];
-            panel_store(panel, lane, ahead[i % PRE]);
-            if (!CACHED || i + PRE < MAXI) {
-                const int tn = t + NW * PRE;
-                ahead[i % PRE] = panel_load_near(xb, x_pitch, (tn < NT ? tn : NT - 1) * 32, S - 1, 0, lane);
-            }
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                xf[ks] = as_bf16x8(panel[panel_slot(r, 2 * ks + g)]);
-                if (CACHED) {
-                    xs[i][ks] = xf[ks];
-                }
-            }
-            const float m = mask01[t * 32 + r];
+        auto add_tile = [&](int t, const bf16x8 (&xf)[4]) {
+            float m = to_f32(mask16[t * 32 + r]);
+            m = m == -INFINITY ? 0.f : m;
             msum += g == 0 ? m : 0.f;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
@@ -172,17 +188,45 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
                     acc[ks][e] = fmaf(m, to_f32(xf[ks][e]), acc[ks][e]);
                 }
             }
-        }
-        // sum over the 32 lanes of each half (they hold different tokens of the same channels)
+        };
+        // the loads of the next PRE tiles are in flight while this one is summed
 #pragma unroll
-        for (int off = 16; off > 0; off >>= 1) {
-            msum += __shfl_xor(msum, off, 64);
+        for (int i = 0; i < KEEP; ++i) {
+            const int t = wave + NW * i;
+            if (t >= NT) {
+                break;
+            }
+            panel_store(panel, lane, ahead[i % PRE]);
+            if (i + PRE < KEEP) {
+                const int tn = t + NW * PRE;
+                ahead[i % PRE] = panel_load_near(xb, x_pitch, (tn < NT ? tn : NT - 1) * 32, S - 1, 0, lane);
+            }
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    acc[ks][e] += __shfl_xor(acc[ks][e], off, 64);
+                xs[i][ks] = as_bf16x8(panel[panel_slot(r, 2 * ks + g)]);
+            }
+            add_tile(t, xs[i]);
+        }
+        if constexpr (STREAM) {
+            int slot = 0;
+            for (int t = first; t < NT; t += NW, slot ^= 1) {
+                if (t + NW < NT) {
+                    wait_for_loads<4>(); // all but the next tile's
+                } else {
+                    wait_for_loads<0>();
                 }
+                const Tile x = ring_tile(slot, t);
+                add_tile(t, x.f);
+            }
+            stream_start();
+        }
+        // sum over the 32 lanes of each half (they hold different tokens of the same channels)
+        msum = group_sum<32>(msum);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                acc[ks][e] = group_sum<32>(acc[ks][e]);
             }
         }
         if (r == 0) {
@@ -260,38 +304,15 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     {
         f32x16 o = zero16();
         float m_run = -1e30f, lsum = 0.f;
-        PanelRegs nxt;
-        if (!CACHED) {
-            nxt = panel_load_near(xb, x_pitch, wave * 32, S - 1, 0, lane);
-        }
-#pragma unroll(UNR)
-        for (int i = 0; i < MAXI; ++i) {
-            const int t = wave + NW * i;
-            if (t >= NT) {
-                break;
-            }
-            bf16x8 xf[4];
-            if (CACHED) {
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    xf[ks] = xs[i][ks];
-                }
-            } else {
-                panel_store(panel, lane, nxt);
-                nxt = panel_load_near(xb, x_pitch, (t + NW < NT ? t + NW : t) * 32, S - 1, 0, lane);
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    xf[ks] = as_bf16x8(panel[panel_slot(r, 2 * ks + g)]);
-                }
-            }
+        auto attend = [&](int t, const bf16x8 (&xf)[4]) {
             f32x16 x1, vv = zero16();
-            const f32x4 *mb4 = reinterpret_cast<const f32x4 *>(maskb + t * 32 + 4 * g);
+            const bf16x4 *mb4 = reinterpret_cast<const bf16x4 *>(mask16 + t * 32 + 4 * g);
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
-                const f32x4 mv = mb4[2 * a];
+                const bf16x4 mv = mb4[2 * a];
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    x1[4 * a + c] = mv[c];
+                    x1[4 * a + c] = fmaf(to_f32(mv[c]), 1e9f, -1e9f); // reference :120-121
                 }
             }
 #pragma unroll
@@ -322,6 +343,26 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
             }
             o = mfma(pack8(vv, 0), p0, o);
             o = mfma(pack8(vv, 8), p1, o);
+        };
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i) {
+            if (wave + NW * i >= NT) {
+                break;
+            }
+            attend(wave + NW * i, xs[i]);
+        }
+        if constexpr (STREAM) {
+            int slot = 0;
+            for (int t = first; t < NT; t += NW, slot ^= 1) {
+                if (t + NW < NT) {
+                    wait_for_loads<4>();
+                } else {
+                    wait_for_loads<0>();
+                }
+                const Tile x = ring_tile(slot, t);
+                attend(t, x.f);
+            }
+            stream_start();
         }
         float *mine = merge + (wave * 64 + lane) * MERGE_LD;
         mine[0] = m_run;
@@ -373,42 +414,22 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
             bgv[i] = p.bg[ch];
             wv_[i] = wavg[ch];
         }
-        const float *bop = p.bo + 16 * g;
-        PanelRegs nxt;
-        if (!CACHED) {
-            nxt = panel_load_near(xb, x_pitch, wave * 32, S - 1, 0, lane);
-        }
-#pragma unroll(UNR)
-        for (int i = 0; i < MAXI; ++i) {
-            const int t = wave + NW * i;
-            if (t >= NT) {
-                break;
-            }
-            bf16x8 xf[4];
-            if (CACHED) {
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    xf[ks] = xs[i][ks];
-                }
-            } else {
-                panel_store(panel, lane, nxt);
-                nxt = panel_load_near(xb, x_pitch, (t + NW < NT ? t + NW : t) * 32, S - 1, 0, lane);
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    xf[ks] = as_bf16x8(panel[panel_slot(r, 2 * ks + g)]);
-                }
-            }
+        auto put_out = [&](int t, const bf16x8 (&xf)[4]) {
             bf16x8 gf[4];
 #pragma unroll
             for (int rb = 0; rb < 2; ++rb) {
-                f32x16 ga = zero16();
+                f32x16 ga;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    ga[v] = bgv[rb * 16 + v];
+                }
 #pragma unroll
                 for (int ks = 0; ks < 4; ++ks) {
                     ga = mfma(as_bf16x8(wg_frag[(rb * 4 + ks) * 64 + lane]), xf[ks], ga);
                 }
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
-                    ga[v] = wv_[rb * 16 + v] * sigmoid_fast(ga[v] + bgv[rb * 16 + v]);
+                    ga[v] = wv_[rb * 16 + v] * sigmoid_fast(ga[v]);
                 }
                 gf[2 * rb] = pack8(ga, 0);
                 gf[2 * rb + 1] = pack8(ga, 8);
@@ -416,18 +437,18 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
             const int s = t * 32 + r;
 #pragma unroll
             for (int ob = 0; ob < 2; ++ob) {
-                f32x16 oa = zero16();
+                f32x16 oa;
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    const f32x4 bv = *reinterpret_cast<const f32x4 *>(bos + 32 * ob + 16 * g + 4 * a);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        oa[4 * a + c] = bv[c];
+                    }
+                }
 #pragma unroll
                 for (int kk = 0; kk < 4; ++kk) {
                     oa = mfma(as_bf16x8(wo_frag[(ob * 4 + kk) * 64 + lane]), gf[kk], oa);
-                }
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    const f32x4 bv = *reinterpret_cast<const f32x4 *>(bop + 32 * ob + 4 * a);
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        oa[4 * a + c] += bv[c];
-                    }
                 }
                 if (s < S) {
                     char *row_out = reinterpret_cast<char *>(p.out + (int64_t)b * p.out_sb + 32 * ob); // uniform
@@ -436,20 +457,49 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
                     dst[1] = as_uint4(pack8(oa, 8));
                 }
             }
+        };
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i) {
+            if (wave + NW * i >= NT) {
+                break;
+            }
+            put_out(wave + NW * i, xs[i]);
+        }
+        if constexpr (STREAM) {
+            int slot = 0;
+            for (int t = first; t < NT; t += NW, slot ^= 1) {
+                // younger than the tile's loads are the stores of the two tiles before it, four each (of kept ones, for the
+                // first two tiles)
+                wait_for_loads<8>();
+                const Tile x = ring_tile(slot, t);
+                put_out(t, x.f);
+            }
         }
     }
 }
 
-// Dynamic LDS of global_attention_kernel<., NW> for NT key tiles: staged weights and the waves' panels (16-byte units),
-// then mask and logits rows, per-wave states and the merge area (floats).
+// Dynamic LDS of global_attention_kernel for NT tiles: staged weights, the waves' panels and rings (16-byte units), mask
+// (bf16), then per-wave sums and the vectors of the row (floats).
 constexpr size_t LDS_PER_WORKGROUP = 160 * 1024;
-constexpr size_t lds_bytes_for(int nw, int nt)
+constexpr size_t lds_bytes_for(int nw, bool stream, int nt)
 {
-    return (size_t)(256 + 256 + 512 + 512 + 256 + nw * 256) * 16 + (size_t)(2 * nt * 32 + nw * 68 + 3 * GC + nw * 64 * MERGE_LD) * 4;
+    return (size_t)(256 + 256 + 512 + 512 + 256 + nw * (PANEL_SLOTS + (stream ? 512 : 0))) * 16 + (size_t)nt * 64 + (size_t)(nw * 68 + 4 * GC) * 4;
 }
-constexpr int MAX_SEQ_LEN = 12288; // what the four-wave layout holds
-static_assert(lds_bytes_for(4, MAX_SEQ_LEN / 32) <= LDS_PER_WORKGROUP && lds_bytes_for(4, MAX_SEQ_LEN / 32 + 1) > LDS_PER_WORKGROUP,
-              "MAX_SEQ_LEN must be the longest row whose four-wave layout fits the LDS");
+constexpr int MAX_SEQ_LEN = 12288;
+static_assert(lds_bytes_for(8, true, MAX_SEQ_LEN / 32) <= LDS_PER_WORKGROUP);
+
+template <int NW, int KEEP, bool STREAM>
+hipError_t launch(const GlobalParams &p, hipStream_t stream)
+{
+    static size_t configured[KUTACC_DEVICE_SLOTS] = {};
+    const size_t lds_bytes = lds_bytes_for(NW, STREAM, p.NT);
+    const auto kernel = &global_attention_kernel<NW, KEEP, STREAM>;
+    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(kernel), lds_bytes, configured)) {
+        return e;
+    }
+    kernel<<<dim3((unsigned)p.B), 64 * NW, lds_bytes, stream>>>(p);
+    return hipGetLastError();
+}
 
 } // namespace
 
@@ -490,49 +540,14 @@ int global_attention(const kutacc_hip_global_attention_args_t &a, hipStream_t st
     p.scale = (float)(1.0 / sqrt((double)a.head_size)); // reference :98
     // A batch row is one workgroup and its three phases follow one another (load and mean, logits, gate and output), so what
     // overlaps them is other rows on the same CU.  With the row kept in registers (up to 1024 positions) four waves hold
-    // 128 + 113 registers and two rows share a CU; eight waves hold half the tiles each (174 registers) and one row has the
+    // 128 + 107 registers and two rows share a CU; eight waves hold half the tiles each (171 registers) and one row has the
     // CU to itself, which is faster only while there is no second row to put there -- batch <= CUs: 28.1 against 30.7 us at
-    // 256 x 1024, 48.3 against 39.3 us at 384 x 1024.  Rows streamed three times (longer sequences) always take eight
-    // waves: 220 against 282 us at 384 x 5120.
-    const bool cached = p.NT <= 32;
-    static int cu_table[KUTACC_DEVICE_SLOTS] = {};
-    const int ncu = kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, cu_table);
-    // ... as long as the eight-wave layout fits the LDS: its fixed part is 36 KB larger than the four-wave one's, and
-    // both grow by 256 bytes per key tile (7808 positions with eight waves, MAX_SEQ_LEN with four).
-    int nw = (p.NT >= 16 && (!cached || a.batch <= ncu)) ? 8 : 4;
-    if (nw == 8 && lds_bytes_for(8, p.NT) > LDS_PER_WORKGROUP) {
-        nw = 4;
-    }
-    const size_t lds_bytes = lds_bytes_for(nw, p.NT);
-    if (lds_bytes > LDS_PER_WORKGROUP) {
-        return KUTACC_HIP_EUNSUPPORTED; // not reached while MAX_SEQ_LEN is what four waves can hold
-    }
-    static size_t configured[4][KUTACC_DEVICE_SLOTS] = {};
-    const void *fn = nw == 8 ? (cached ? reinterpret_cast<const void *>(global_attention_kernel<true, 8>)
-                                       : reinterpret_cast<const void *>(global_attention_kernel<false, 8>))
-                             : (cached ? reinterpret_cast<const void *>(global_attention_kernel<true, 4>)
-                                       : reinterpret_cast<const void *>(global_attention_kernel<false, 4>));
-    {
-        const hipError_t e = kutacc_opt_in_lds(fn, lds_bytes, configured[(nw == 8 ? 2 : 0) + (cached ? 1 : 0)]);
-        if (e != hipSuccess) {
-            return (int)e;
-        }
-    }
+    // 256 x 1024, 48.3 against 39.3 us at 384 x 1024.  Longer rows take eight waves with 64 tiles kept.
     const double BS = (double)a.batch * (double)a.seq_len;
     kutacc_prof::KernelTimer t("global_attention_kernel", BS * (4.0 * GC * a.head_size + 4.0 * GC * GC + 4.0 * GC), stream);
-    const dim3 grid((unsigned)a.batch), block((unsigned)(64 * nw));
-    if (nw == 8) {
-        if (cached) {
-            global_attention_kernel<true, 8><<<grid, block, lds_bytes, stream>>>(p);
-        } else {
-            global_attention_kernel<false, 8><<<grid, block, lds_bytes, stream>>>(p);
-        }
-    } else if (cached) {
-        global_attention_kernel<true, 4><<<grid, block, lds_bytes, stream>>>(p);
-    } else {
-        global_attention_kernel<false, 4><<<grid, block, lds_bytes, stream>>>(p);
-    }
-    return kutacc_hip_status(hipGetLastError());
+    const hipError_t e = p.NT > 32 ? launch<8, 8, true>(p, stream)
+                         : p.NT >= 16 && a.batch <= kutacc_cu_count() ? launch<8, 4, false>(p, stream) : launch<4, 8, false>(p, stream);
+    return kutacc_hip_status(e);
 }
 
 } // namespace kutacc_launch

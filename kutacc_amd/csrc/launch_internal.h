@@ -165,6 +165,7 @@ int pair_gemm(const kutacc_hip_gemm_args_t &args, hipStream_t stream, const kuta
 int gated_projection_mode(); // 0: the default rule (see pair_gemm_tuning)
 int triangle_equation(const void *left, const void *right, void *centre, int64_t n, int64_t np, int64_t plane, int64_t channels, bool incoming,
                       hipStream_t stream);
+// transition.hip
 bool transition_fused_supports(int64_t rows, int64_t c_o, int64_t c_i, const void *x, const void *w1, const float *b1,
                                const void *w2, const float *b2, const void *out);
 int transition_fused(const void *x, const void *w1, const float *b1, const void *w2, const float *b2, void *out,

@@ -223,6 +223,20 @@ __device__ __forceinline__ void panel_store(uint4 *panel, int lane, const PanelR
     panel[(s0 ^ 1) + 192] = p.r3;
 }
 
+// A read of global memory that lands in the LDS: lane l's 16 bytes, `lane_bytes` past `from`, at `to` + 16 l.  Completion is
+// counted like that of any load; s_waitcnt vmcnt(N) says when.
+__device__ __forceinline__ void load_to_lds(uint32_t to, const void *from, uint32_t lane_bytes)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(lane_bytes), "s"(from) : "memory");
+}
+
+// until at most N of a wave's loads (and stores) are on their way
+template <int N>
+__device__ __forceinline__ void wait_for_loads()
+{
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
 // 8 x 8 transposition of 16-bit elements over the eight lanes that differ in lane bits 3, 4, 5 (same lane & 7).
 // Before: lane with index kk = lane >> 3 holds elements (kk, 0..7) as four dwords; after: elements (0..7, kk).
 // Three exchange steps in registers: halves of a dword against lane bit 3 (row rotation by 8 + byte permute;

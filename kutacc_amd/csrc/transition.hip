@@ -38,12 +38,6 @@ struct TransitionParams {
     int full_groups, tail_waves; // workgroups whose waves all have rows, and how many waves of the others have
 };
 
-// Reads of global memory that land in the LDS: lane l's 16 bytes at `to` + 16 l
-__device__ __forceinline__ void load_to_lds(uint32_t to, const void *from, uint32_t lane_bytes)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(lane_bytes), "s"(from) : "memory");
-}
-
 // 32 rows of x as they come from memory: lane (lane >> 3, lane & 7) holds chunk lane & 7 of every 64-channel panel of rows
 // 8 i + (lane >> 3), and as operands of the first product
 template <int CO>
@@ -202,12 +196,6 @@ template <int N>
 __device__ __forceinline__ void wait_and_barrier()
 {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_for_loads()
-{
-    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
 }
 
 // SLICE: hidden units per stage of the ring of STAGES; GROUPS: workgroups a CU is meant to hold.

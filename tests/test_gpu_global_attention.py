@@ -85,6 +85,19 @@ def test_global_attention_matches_oracle(torch_cuda, B, S, H, d, mask_mode):
     helpers.assert_within(helpers.to_numpy(scratch["avg"][rows]), ref_qavg, 2.0 ** -8 * np.abs(ref_qavg) + 1e-6, "masked mean q_avg")
 
 
+@pytest.mark.parametrize("B,S,H,d", [(2, 1025, 8, 8), (2, 2048, 8, 8), (2, 2049, 4, 16), (2, 2305, 8, 8), (2, 2590, 2, 32), (2, 3201, 16, 4)])
+def test_global_attention_rows_past_the_kept_tiles(torch_cuda, B, S, H, d):
+    """The first length past the rows that are kept whole; all tiles kept by eight waves; one wave with one tile that is read
+    again, one with two (the depth of its ring) and the others with one, all with two and a partial third, four to five."""
+    c = make_case(300 + S, B, S, H, d)
+    op, ten, scratch = device_op(torch_cuda, c)
+    op.run()
+    assert not capi.error_flag() and capi.last_path() == "global_mfma"
+    ref, ref_qavg = oracle_out(c)
+    helpers.check_close(helpers.to_numpy(ten["out"]), ref, "bf16", "global attention out")
+    helpers.assert_within(helpers.to_numpy(scratch["avg"]), ref_qavg, 2.0 ** -8 * np.abs(ref_qavg) + 1e-6, "masked mean q_avg")
+
+
 def test_global_attention_full_extra_msa_shape(torch_cuda):
     """An extra-MSA sized call (N_res = 256 batch rows of 1024 extra sequences): spot-check rows against the oracle."""
     c = make_case(7, 256, 1024, 8, 8, "random")
