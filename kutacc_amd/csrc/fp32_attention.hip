@@ -5,23 +5,31 @@
 // fp32 MFMA multiplies fp32 operands exactly and accumulates in fp32, at a sixteenth of the bf16 rate -- enough for the
 // small fp32 problems (the MSA-row benchmark shape is 0.74 GFLOP), which are bound by latency, not by arithmetic.
 //
-//   fp32_head_kernel     one workgroup of four waves per (batch row b, head h): the four projections of the head
-//       (K, V, Q, gate -- one matrix per wave, the input rows staged through LDS 32 positions at a time), then
-//       flash-style attention with a running maximum, one 32-query block per wave at a time, the sigmoid gate, and the
-//       gated average stored where the reference leaves it (src/attention/gating_attention.cpp:47-66, 73-150).
-//       q, k, v, gate, logits and probabilities never leave the chip.
-//   fp32_rows_gemm_kernel   out[m, n] = sum_k a[m, k] * w[n, k] + bias[n], one 32 x 32 tile per wave: the output
-//       projection (reference :152-157).
+//   fp32_head_kernel     one workgroup of eight waves per (batch row b, head h) and share of its queries: the four
+//       projections of the head (a wave holds 16 features of one matrix in registers; the positions are staged
+//       through the LDS, 32 at a time), then flash-style attention with a running maximum, 16 queries per wave at a time, the
+//       sigmoid gate, and the gated average stored where the reference leaves it
+//       (src/attention/gating_attention.cpp:47-66, 73-150).  q, k, v, gate, logits and probabilities never leave the chip.
+//   fp32_rows_gemm_kernel   out[m, n] = sum_k a[m, k] * w[n, k] + bias[n]: the output projection (reference :152-157).
 //
-// Operand and accumulator layouts of the 32x32x2 MFMA: A is 32 x 2, lane l holds A[l % 32][l / 32]; B is 2 x 32, lane l
-// holds B[l / 32][l % 32]; D[i][j] sits in lane j + 32 g, register v with i = 8 (v / 4) + 4 g + v % 4.  As in the bf16
-// kernels, products are formed transposed (rows = keys or head dims, columns = queries) so that an accumulator is the
-// next product's B operand as it stands: register v of the probabilities is the k-step of P.V whose two keys are the
-// ones that register holds in the two halves of the wave.
+// What bounds it: the fp32 matrix rate (64 multiply-adds per cycle and SIMD: 16 positions x 32 features x 256 channels
+// take 4096 cycles) once loads are out of the way.  The smaller 16x16x4 form has the rate of 32x32x2 and twice the
+// pieces to deal out: two waves per SIMD cover each other's LDS reads, and 64 queries occupy four SIMDs instead of two.
+// A wave's whole weight block is in flight before the first position arrives.
+// 16 rows x 64 positions x 256 channels, whole operator: 40.9 us with four waves of 32x32x2 and weights
+// loaded as they were used, 21.9 now; 64 x 200 x 256: 235 and 151.
+//
+// Operand and accumulator layouts of the 16x16x4 MFMA: A is 16 x 4, lane l holds A[l % 16][l / 16]; B is 4 x 16, lane l
+// holds B[l / 16][l % 16]; D[4 g + v][j] sits in lane j + 16 g, register v.  A lane reads four consecutive k with one
+// 16-byte load and uses them in four successive products (the order of k is the same for both operands).  Products are
+// formed so that an accumulator is the next product's B operand as it stands: register v of the transposed
+// probabilities holds keys 4 g + v, and the value operand reads the same four keys from a transposed V.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
+#include <type_traits>
 
 #include "device_util.h"
 #include "launch_internal.h"
@@ -31,227 +39,332 @@ using namespace kutacc_dev;
 
 namespace {
 
-typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef f32x4 f32x4_any __attribute__((aligned(4))); // global loads and stores of 16 bytes need 4-byte alignment only
 
 constexpr int HEAD = 32;
-constexpr int LDP = 33;            // row pitch of the [position][feature] arrays in LDS, in floats: odd, so a column read is conflict-free
+constexpr int LDP = 36;            // row pitch of the [position][feature] arrays in LDS, in floats: 16 rows' 16-byte pieces in 16 bank groups
 constexpr int MAX_SEQ = 224;       // what the LDS holds of K, V, Q and gate of one head in fp32
 constexpr int MAX_CHANNELS = 256;  // input rows are staged 32 positions x C channels at a time
 constexpr float LOG2E_F = 1.44269504088896340736f;
 
-__device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-__device__ __forceinline__ float swap_halves_max(float x)
+__device__ __forceinline__ f32x4 load4(const float *ptr) { return *reinterpret_cast<const f32x4 *>(ptr); }
+
+// the four lanes that hold one query's keys: l, l ^ 16, l ^ 32, l ^ 48
+__device__ __forceinline__ float quad_max(float x)
 {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    const float y = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+    return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
-__device__ __forceinline__ float swap_halves_sum(float x)
+__device__ __forceinline__ float quad_sum(float x)
 {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    const float y = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+    return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
 struct Fp32Params {
     const float *x, *wq, *wk, *wv, *wg, *bg, *bias, *nb;
     float *avg;
     int64_t x_ld, bias_sb, nb_sh, nb_sq, avg_sb, avg_ss, avg_sh;
-    int B, S, H, C;
-    int nb_vec; // pair-bias rows may be read with 16-byte loads
+    int S, H;
+    int parts; // workgroups that share a head's queries
     float scale;
 };
 
-__global__ __launch_bounds__(256) void fp32_head_kernel(Fp32Params p)
+// PIECES: C / 16, the 16-channel pieces of a row, of which a lane holds four channels each
+template <int PIECES>
+__global__ __launch_bounds__(512, 2) void fp32_head_kernel(Fp32Params p)
 {
     extern __shared__ float lds_f[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int r = lane & 31, g = lane >> 5;
-    const int S = p.S, C = p.C, NB = (S + 31) / 32, S32 = NB * 32;
-    const int b = blockIdx.x / p.H, h = blockIdx.x % p.H;
-    const int XP = C + 4; // staged input rows: 16 bytes of padding per row, so that 16 lanes reading 16 bytes of 16 rows hit 16 bank groups
+    const int r = lane & 15, g = lane >> 4;
+    constexpr int C = 16 * PIECES;
+    const int S = p.S, NB = (S + 31) / 32, S32 = NB * 32;
+    const int part = blockIdx.x % p.parts, bh = blockIdx.x / p.parts;
+    const int b = bh / p.H, h = bh % p.H;
+    const int t_lo = NB * part / p.parts, t_hi = NB * (part + 1) / p.parts; // query tiles of this workgroup
+    const int XP = C + 4, VP = S32 + 4; // odd multiples of 16 bytes, as LDP
 
     float *xs = lds_f;             // [32][XP]
     float *ks = xs + 32 * XP;      // [S32][LDP]
-    float *vs = ks + S32 * LDP;    // [S32][LDP]
-    float *qs = vs + S32 * LDP;    // [S32][LDP], scaled by 1/sqrt(d)
+    float *qs = ks + S32 * LDP;    // [S32][LDP], scaled by 1/sqrt(d)
     float *gs = qs + S32 * LDP;    // [S32][LDP], sigmoid applied
-    float *ms = gs + S32 * LDP;    // [S32] mask bias, -inf past S
+    float *vt = gs + S32 * LDP;    // [32][VP], transposed
+    float *ms = vt + HEAD * VP;    // [S32] mask bias, -inf past S
 
-    for (int k = tid; k < S32; k += 256) {
+    // ---- projections: waves w and w + 4 share a SIMD, so they take different matrices: where the queries are shared out,
+    // every SIMD has one of k, v (all positions) and one of q, gate (this workgroup's) ----
+    const int half = wave >> 2, mat = (wave + 2 * half) & 3; // 0 k, 1 v, 2 q, 3 gate
+    const float *wmat = mat == 0 ? p.wk : mat == 1 ? p.wv : mat == 2 ? p.wq : p.wg;
+    const float *wrow = wmat + (int64_t)(h * HEAD + 16 * half + r) * C + 4 * g;
+    // the next 32 positions wait in registers while the staged ones are used
+    const float *xb = p.x + (int64_t)b * S * p.x_ld;
+    constexpr int c4 = C / 4, pieces = 32 * c4, LOADS = (pieces + 511) / 512;
+    f32x4 xr[LOADS];
+    int xrow_i[LOADS], xcol[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int idx = tid + 512 * i < pieces ? tid + 512 * i : pieces - 1;
+        xrow_i[i] = idx / c4;
+        xcol[i] = 4 * (idx % c4);
+    }
+    const auto fetch = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int pos = t * 32 + xrow_i[i] < S ? t * 32 + xrow_i[i] : S - 1;
+            xr[i] = load4(xb + (int64_t)pos * p.x_ld + xcol[i]);
+        }
+    };
+    fetch(0);
+    f32x4 w[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        w[i] = load4(wrow + 16 * i);
+    }
+    f32x4 start = {0.f, 0.f, 0.f, 0.f};
+    if (mat == 3) {
+        start = *reinterpret_cast<const f32x4_any *>(p.bg + h * HEAD + 16 * half + 4 * g);
+    }
+    for (int k = tid; k < S32; k += 512) {
         ms[k] = k < S ? p.bias[(int64_t)b * p.bias_sb + k] : -INFINITY;
     }
-
-    // ---- projections: wave w forms matrix w of the head for 32 positions at a time ----
-    const float *xb = p.x + (int64_t)b * S * p.x_ld;
-    const float *wmat = wave == 0 ? p.wk : wave == 1 ? p.wv : wave == 2 ? p.wq : p.wg;
-    float *dst = wave == 0 ? ks : wave == 1 ? vs : wave == 2 ? qs : gs;
-    const float *wrow = wmat + (int64_t)(h * HEAD + r) * C + 4 * g; // this lane's weight row, its half of every 8 channels
-    const float gate_bias = p.bg[h * HEAD + r];
-    const int c4 = C / 4;
+    // four keys' pair bias of query q0 + r; a step's is requested one step ahead, the first one's before the projections
+    const auto pair_bias = [&](int q0, int key0) {
+        f32x4 nv = {0.f, 0.f, 0.f, 0.f};
+        if (p.nb != nullptr) {
+            const float *nbrow = p.nb + (int64_t)h * p.nb_sh + (int64_t)(q0 + r < S ? q0 + r : S - 1) * p.nb_sq;
+            if (key0 + 4 <= S) {
+                nv = *reinterpret_cast<const f32x4_any *>(nbrow + key0);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    nv[c] = key0 + c < S ? nbrow[key0 + c] : 0.f;
+                }
+            }
+        }
+        return nv;
+    };
+    const int q_first = 32 * t_lo + 16 * wave, q_end = 32 * t_hi < S ? 32 * t_hi : S;
+    f32x4 next0 = pair_bias(q_first, 4 * g), next1 = pair_bias(q_first, 16 + 4 * g);
     for (int t = 0; t < NB; ++t) {
         __syncthreads(); // the previous tile's readers are done with xs
-        for (int idx = tid; idx < 32 * c4; idx += 256) {
-            const int row = idx / c4, cc = idx % c4;
-            const int pos = t * 32 + row < S ? t * 32 + row : S - 1;
-            *reinterpret_cast<f32x4 *>(xs + row * XP + 4 * cc) = *reinterpret_cast<const f32x4 *>(xb + (int64_t)pos * p.x_ld + 4 * cc);
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            if (tid + 512 * i < pieces) {
+                *reinterpret_cast<f32x4 *>(xs + xrow_i[i] * XP + xcol[i]) = xr[i];
+            }
         }
         __syncthreads();
-        f32x16 acc;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            acc[v] = wave == 3 ? gate_bias : 0.f; // D[position][feature]: a lane's registers all belong to feature r
+        if (t + 1 < NB) {
+            fetch(t + 1);
         }
+        if (mat >= 2 && (t < t_lo || t >= t_hi)) {
+            continue;
+        }
+        f32x4 acc[2] = {start, start}; // positions 0-15 and 16-31 of the tile
         const float *xrow = xs + r * XP + 4 * g;
-#pragma unroll 4
-        for (int c0 = 0; c0 < C; c0 += 8) {
-            const f32x4 xa = *reinterpret_cast<const f32x4 *>(xrow + c0);
-            const f32x4 wb = *reinterpret_cast<const f32x4 *>(wrow + c0);
-            acc = mfma_f32(xa[0], wb[0], acc);
-            acc = mfma_f32(xa[1], wb[1], acc);
-            acc = mfma_f32(xa[2], wb[2], acc);
-            acc = mfma_f32(xa[3], wb[3], acc);
+        const auto project = [&](auto transposed, auto units) { // D[position][feature] for v, D[feature][position] for the others
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) {
+                f32x4 xa[2];
+#pragma unroll
+                for (int u = 0; u < units; ++u) {
+                    xa[u] = load4(xrow + 16 * u * XP + 16 * i);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                    for (int u = 0; u < units; ++u) {
+                        acc[u] = transposed ? mfma_f32(xa[u][j], w[i][j], acc[u]) : mfma_f32(w[i][j], xa[u][j], acc[u]);
+                    }
+                }
+            }
+        };
+        using One = std::integral_constant<int, 1>;
+        using Two = std::integral_constant<int, 2>;
+        const bool full = t * 32 + 16 < S; // else the second half's keys and values are zero, and their mask -inf
+        if (mat == 1) {
+            full ? project(std::true_type{}, Two{}) : project(std::true_type{}, One{});
+        } else {
+            full ? project(std::false_type{}, Two{}) : project(std::false_type{}, One{});
         }
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            float val = acc[v];
-            if (wave == 2) {
-                val *= p.scale;
-            } else if (wave == 3) {
-                val = 1.0f / (1.0f + __builtin_amdgcn_exp2f(-val * LOG2E_F));
+        for (int u = 0; u < 2; ++u) {
+            const int pos0 = t * 32 + 16 * u;
+            if (mat == 1) {
+                *reinterpret_cast<f32x4 *>(vt + (16 * half + r) * VP + pos0 + 4 * g) = acc[u];
+                continue;
             }
-            dst[(t * 32 + 8 * (v >> 2) + 4 * g + (v & 3)) * LDP + r] = val;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                acc[u][v] = mat == 2   ? acc[u][v] * p.scale
+                            : mat == 3 ? 1.0f / (1.0f + __builtin_amdgcn_exp2f(-acc[u][v] * LOG2E_F))
+                                       : acc[u][v];
+            }
+            *reinterpret_cast<f32x4 *>((mat == 0 ? ks : mat == 2 ? qs : gs) + (pos0 + r) * LDP + 16 * half + 4 * g) = acc[u];
         }
     }
     __syncthreads();
 
-    // ---- attention: one 32-query block per wave at a time ----
-    for (int qt = wave; qt < NB; qt += 4) {
-        float qop[16]; // Q^T operand: this lane's query, head dims 2 i + g
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            qop[i] = qs[(qt * 32 + r) * LDP + 2 * i + g];
-        }
-        const int qpos = qt * 32 + r;
-        const int qrow = qpos < S ? qpos : S - 1;
-        const float *nbrow = p.nb != nullptr ? p.nb + (int64_t)h * p.nb_sh + (int64_t)qrow * p.nb_sq + 4 * g : nullptr;
+    // ---- attention: 16 queries per wave at a time, 32 keys per step ----
+    for (int q0 = q_first; q0 < q_end; q0 += 128) {
+        const int qpos = q0 + r;
+        const f32x4 qop0 = load4(qs + qpos * LDP + 4 * g), qop1 = load4(qs + qpos * LDP + 16 + 4 * g);
         float m_run = -INFINITY, lsum = 0.f;
-        f32x16 o;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            o[v] = 0.f;
-        }
+        f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = o0;
         for (int kt = 0; kt < NB; ++kt) {
-            f32x16 x;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                x[v] = 0.f;
+            const f32x4 nv0 = next0, nv1 = next1;
+            if (kt + 1 < NB) {
+                next0 = pair_bias(q0, 32 * kt + 32 + 4 * g);
+                next1 = pair_bias(q0, 32 * kt + 48 + 4 * g);
+            } else if (q0 + 128 < q_end) {
+                next0 = pair_bias(q0 + 128, 4 * g);
+                next1 = pair_bias(q0 + 128, 16 + 4 * g);
             }
-            const float *krow = ks + (kt * 32 + r) * LDP + g;
+            // logits^T: rows = keys, columns = queries
+            const float *krow = ks + (32 * kt + r) * LDP + 4 * g;
+            const f32x4 k00 = load4(krow), k01 = load4(krow + 16), k10 = load4(krow + 16 * LDP), k11 = load4(krow + 16 * LDP + 16);
+            f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = x0;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                x = mfma_f32(krow[2 * i], qop[i], x); // logits^T: rows = keys, columns = queries
+            for (int j = 0; j < 4; ++j) {
+                x0 = mfma_f32(k00[j], qop0[j], x0);
+                x1 = mfma_f32(k10[j], qop0[j], x1);
             }
-            // (logit * scale + bias[b, k]) + nb[h, q, k], in that order (reference :109-118); register v holds key
-            // 32 kt + 8 (v / 4) + 4 g + v % 4
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const int key0 = kt * 32 + 8 * a + 4 * g;
-                const f32x4 mv = *reinterpret_cast<const f32x4 *>(ms + key0);
-                f32x4 nv = {0.f, 0.f, 0.f, 0.f};
-                if (nbrow != nullptr) {
-                    if (p.nb_vec && key0 + 4 <= S) {
-                        nv = *reinterpret_cast<const f32x4 *>(nbrow + kt * 32 + 8 * a);
-                    } else {
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) {
-                            nv[c] = key0 + c < S ? nbrow[kt * 32 + 8 * a + c] : 0.f;
-                        }
-                    }
-                }
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    x[4 * a + c] = (x[4 * a + c] + mv[c]) + nv[c];
-                }
+            for (int j = 0; j < 4; ++j) {
+                x0 = mfma_f32(k01[j], qop1[j], x0);
+                x1 = mfma_f32(k11[j], qop1[j], x1);
             }
-            float mx = x[0];
+            // (logit * scale + bias[b, k]) + nb[h, q, k], in that order (reference :109-118)
+            const f32x4 mv0 = load4(ms + 32 * kt + 4 * g), mv1 = load4(ms + 32 * kt + 16 + 4 * g);
+            float mx = -INFINITY;
 #pragma unroll
-            for (int v = 1; v < 16; ++v) {
-                mx = fmaxf(mx, x[v]);
+            for (int c = 0; c < 4; ++c) {
+                x0[c] = (x0[c] + mv0[c]) + nv0[c];
+                x1[c] = (x1[c] + mv1[c]) + nv1[c];
+                mx = fmaxf(mx, fmaxf(x0[c], x1[c]));
             }
-            mx = swap_halves_max(mx);
+            mx = quad_max(mx);
             const float m_new = fmaxf(m_run, mx); // finite: every tile has a key below S, whose bias is finite
             const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * LOG2E_F);
             m_run = m_new;
             float psum = 0.f;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                x[v] = __builtin_amdgcn_exp2f((x[v] - m_new) * LOG2E_F);
-                psum += x[v];
-                o[v] *= alpha;
+            for (int c = 0; c < 4; ++c) {
+                x0[c] = __builtin_amdgcn_exp2f((x0[c] - m_new) * LOG2E_F);
+                x1[c] = __builtin_amdgcn_exp2f((x1[c] - m_new) * LOG2E_F);
+                psum += x0[c] + x1[c];
+                o0[c] *= alpha;
+                o1[c] *= alpha;
             }
             lsum = lsum * alpha + psum;
-            // O^T += V^T . P^T: k-step v pairs the two keys register v holds in the two halves of the wave
+            // O^T += V^T . P^T: k-step j takes the keys 4 g + j that register j holds
+            const float *vrow = vt + r * VP + 32 * kt + 4 * g;
+            const f32x4 v00 = load4(vrow), v01 = load4(vrow + 16), v10 = load4(vrow + 16 * VP), v11 = load4(vrow + 16 * VP + 16);
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                o = mfma_f32(vs[(kt * 32 + 8 * (v >> 2) + 4 * g + (v & 3)) * LDP + r], x[v], o);
+            for (int j = 0; j < 4; ++j) {
+                o0 = mfma_f32(v00[j], x0[j], o0);
+                o1 = mfma_f32(v10[j], x0[j], o1);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                o0 = mfma_f32(v01[j], x1[j], o0);
+                o1 = mfma_f32(v11[j], x1[j], o1);
             }
         }
-        const float inv = 1.0f / swap_halves_sum(lsum);
-        if (qpos < S) {
+        const float inv = 1.0f / quad_sum(lsum);
+        if (qpos < S) { // register c of o0 is head dim 4 g + c, of o1 16 + 4 g + c
             float *out = p.avg + (int64_t)b * p.avg_sb + (int64_t)qpos * p.avg_ss + (int64_t)h * p.avg_sh + 4 * g;
-            const float *grow = gs + qpos * LDP + 4 * g;
+            const f32x4 g0 = load4(gs + qpos * LDP + 4 * g), g1 = load4(gs + qpos * LDP + 16 + 4 * g);
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                f32x4 ov;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    ov[c] = o[4 * a + c] * inv * grow[8 * a + c]; // register 4 a + c is head dim 8 a + 4 g + c
-                }
-                *reinterpret_cast<f32x4 *>(out + 8 * a) = ov;
+            for (int c = 0; c < 4; ++c) {
+                o0[c] = o0[c] * inv * g0[c];
+                o1[c] = o1[c] * inv * g1[c];
             }
+            *reinterpret_cast<f32x4 *>(out) = o0;
+            *reinterpret_cast<f32x4 *>(out + 16) = o1;
         }
     }
 }
 
-// out[m, n] = sum_k a[m, k] * w[n, k] + bias[n]; one 32 x 32 tile per wave, four tiles along n per workgroup.  k is a
-// multiple of 8; rows are 16-byte aligned.
-__global__ __launch_bounds__(256) void fp32_rows_gemm_kernel(const float *__restrict__ a, int64_t a_ld, const float *__restrict__ w,
-                                                             int64_t w_ld, const float *__restrict__ bias, float *__restrict__ out,
-                                                             int64_t out_ld, int64_t M, int N, int K)
+// out[m, n] = sum_k a[m, k] * w[n, k] + bias[n] over 16 PIECES k; 16 T x 16 T outputs per wave, four waves along n.  Rows
+// of a and w are 16-byte aligned.  P pieces of 16 k are fetched at a time, the next P while these are used.  T = 1 with a
+// whole row in flight is bound by one memory latency; T = 2 reads half as much per product.
+template <int PIECES, int T, int P>
+__global__ __launch_bounds__(256, 2) void fp32_rows_gemm_kernel(const float *__restrict__ a, int64_t a_ld, const float *__restrict__ w,
+                                                                const float *__restrict__ bias, float *__restrict__ out,
+                                                                int64_t out_ld, int64_t M, int N)
 {
+    static_assert(PIECES % P == 0, "whole steps");
+    constexpr int K = 16 * PIECES;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r = lane & 31, g = lane >> 5;
-    const int64_t m0 = (int64_t)blockIdx.x * 32;
-    const int n0 = (blockIdx.y * 4 + wave) * 32;
+    const int r = lane & 15, g = lane >> 4;
+    const int64_t m0 = (int64_t)blockIdx.x * 16 * T;
+    const int n0 = (blockIdx.y * 4 + wave) * 16 * T;
     if (n0 >= N) {
         return;
     }
-    const int64_t arow = m0 + r < M ? m0 + r : M - 1;
-    const int wrow_i = n0 + r < N ? n0 + r : N - 1;
-    const float *ap = a + arow * a_ld + 4 * g;
-    const float *wp = w + (int64_t)wrow_i * w_ld + 4 * g;
-    f32x16 acc;
+    const float *ap[T], *wp[T];
+    f32x4 acc[T][T]; // [n][m]: D[output feature][row]
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        acc[v] = 0.f;
-    }
-#pragma unroll 4
-    for (int k0 = 0; k0 < K; k0 += 8) {
-        const f32x4 av = *reinterpret_cast<const f32x4 *>(ap + k0);
-        const f32x4 wv = *reinterpret_cast<const f32x4 *>(wp + k0);
-        acc = mfma_f32(av[0], wv[0], acc);
-        acc = mfma_f32(av[1], wv[1], acc);
-        acc = mfma_f32(av[2], wv[2], acc);
-        acc = mfma_f32(av[3], wv[3], acc);
-    }
-    if (n0 + r < N) {
-        const float bv = bias != nullptr ? bias[n0 + r] : 0.f;
+    for (int i = 0; i < T; ++i) {
+        const int64_t arow = m0 + 16 * i + r < M ? m0 + 16 * i + r : M - 1;
+        ap[i] = a + arow * a_ld + 4 * g;
+        wp[i] = w + (int64_t)(n0 + 16 * i + r) * K + 4 * g; // n0 + 16 T <= N: N is a multiple of 32
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int64_t m = m0 + 8 * (v >> 2) + 4 * g + (v & 3);
+        for (int j = 0; j < T; ++j) {
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    f32x4 av[2][T][P], wv[2][T][P];
+    const auto fetch = [&](int step) {
+#pragma unroll
+        for (int s = 0; s < P; ++s) {
+#pragma unroll
+            for (int i = 0; i < T; ++i) {
+                wv[step & 1][i][s] = load4(wp[i] + 16 * (step * P + s));
+                av[step & 1][i][s] = load4(ap[i] + 16 * (step * P + s));
+            }
+        }
+    };
+    fetch(0);
+#pragma unroll
+    for (int step = 0; step < PIECES / P; ++step) {
+        if (step + 1 < PIECES / P) {
+            fetch(step + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0); // the loads stay ahead of the products
+#pragma unroll
+        for (int s = 0; s < P; ++s) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int i = 0; i < T; ++i) {
+#pragma unroll
+                    for (int j = 0; j < T; ++j) {
+                        acc[i][j] = mfma_f32(wv[step & 1][i][s][e], av[step & 1][j][s][e], acc[i][j]);
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+        f32x4 bv = {0.f, 0.f, 0.f, 0.f};
+        if (bias != nullptr) {
+            bv = *reinterpret_cast<const f32x4_any *>(bias + n0 + 16 * i + 4 * g);
+        }
+#pragma unroll
+        for (int j = 0; j < T; ++j) {
+            const int64_t m = m0 + 16 * j + r;
             if (m < M) {
-                out[m * out_ld + n0 + r] = acc[v] + bv;
+                *reinterpret_cast<f32x4_any *>(out + m * out_ld + n0 + 16 * i + 4 * g) = acc[i][j] + bv;
             }
         }
     }
@@ -262,7 +375,46 @@ inline bool aligned16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr
 size_t head_kernel_lds(int S, int C)
 {
     const int S32 = (S + 31) / 32 * 32;
-    return (size_t)(32 * (C + 4) + 4 * S32 * LDP + S32) * sizeof(float);
+    return (size_t)(32 * (C + 4) + 3 * S32 * LDP + HEAD * (S32 + 4) + S32) * sizeof(float);
+}
+
+template <int PIECES, int T, int P>
+void launch_rows_gemm(const kutacc_hip_attention_args_t &a, int64_t M, hipStream_t stream)
+{
+    constexpr int C = 16 * PIECES;
+    const dim3 grid((unsigned)((M + 16 * T - 1) / (16 * T)), (unsigned)((C / (16 * T) + 3) / 4));
+    fp32_rows_gemm_kernel<PIECES, T, P><<<grid, 256, 0, stream>>>((const float *)a.avg, a.avg_stride_s, (const float *)a.output_w,
+                                                                  a.output_b, (float *)a.out, a.out_ld, M, C);
+}
+
+template <int PIECES>
+int launch(const kutacc_hip_attention_args_t &a, const Fp32Params &p, hipStream_t stream)
+{
+    constexpr int C = 16 * PIECES;
+    const size_t lds_bytes = head_kernel_lds(p.S, C);
+    static size_t configured[KUTACC_DEVICE_SLOTS] = {};
+    const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(fp32_head_kernel<PIECES>), lds_bytes, configured);
+    if (e != hipSuccess) {
+        return (int)e;
+    }
+    const double BS = (double)a.batch * (double)a.seq_len;
+    {
+        kutacc_prof::KernelTimer t("fp32_head_kernel", 8.0 * BS * C * C + 4.0 * BS * (double)a.seq_len * C, stream);
+        fp32_head_kernel<PIECES><<<dim3((unsigned)(a.batch * a.nheads * p.parts)), 512, lds_bytes, stream>>>(p);
+        const int rc = kutacc_hip_status(hipGetLastError());
+        if (rc != 0) {
+            return rc;
+        }
+    }
+    const int64_t M = a.batch * a.seq_len;
+    kutacc_prof::KernelTimer t("fp32_rows_gemm_kernel", 2.0 * BS * C * C, stream);
+    // 32 x 32 outputs per wave where that gives every SIMD a wave
+    if ((M + 31) / 32 * (C / 32) >= 4 * (int64_t)kutacc_cu_count()) {
+        launch_rows_gemm<PIECES, 2, 2>(a, M, stream);
+    } else {
+        launch_rows_gemm<PIECES, 1, PIECES>(a, M, stream);
+    }
+    return kutacc_hip_status(hipGetLastError());
 }
 
 } // namespace
@@ -293,39 +445,29 @@ int gating_attention_fp32(const kutacc_hip_attention_args_t &a, hipStream_t stre
     if (!fp32_attention_supports(a)) {
         return KUTACC_HIP_EUNSUPPORTED;
     }
-    const int C = (int)(a.nheads * a.head_size);
     Fp32Params p;
     p.x = (const float *)a.input, p.wq = (const float *)a.query_w, p.wk = (const float *)a.key_w, p.wv = (const float *)a.value_w;
     p.wg = (const float *)a.gating_w, p.bg = a.gating_b, p.bias = (const float *)a.bias, p.nb = (const float *)a.nonbatched_bias;
     p.avg = (float *)a.avg;
     p.x_ld = a.input_ld, p.bias_sb = a.bias_stride_b, p.nb_sh = a.nb_stride_h, p.nb_sq = a.nb_stride_q;
     p.avg_sb = a.avg_stride_b, p.avg_ss = a.avg_stride_s, p.avg_sh = a.avg_stride_h;
-    p.B = (int)a.batch, p.S = (int)a.seq_len, p.H = (int)a.nheads, p.C = C;
-    p.nb_vec = (p.nb != nullptr && aligned16(p.nb) && a.nb_stride_h % 4 == 0 && a.nb_stride_q % 4 == 0) ? 1 : 0;
+    p.S = (int)a.seq_len, p.H = (int)a.nheads;
+    // With fewer heads than CUs a head's queries go to several workgroups, each of which forms all keys and values: the
+    // projections of a workgroup shrink towards half, on CUs that were idle (16 rows x 64
+    // positions x 8 heads 24.0 us unshared, 22.3 shared; 4 x 64 x 4 heads 15.6 and 14.5).
+    const int64_t heads = a.batch * a.nheads, tiles = (a.seq_len + 31) / 32;
+    p.parts = (int)std::max<int64_t>(1, std::min<int64_t>(tiles, kutacc_cu_count() / heads));
     p.scale = (float)(1.0 / sqrt((double)a.head_size)); // reference gating_attention.cpp:68
-    const size_t lds_bytes = head_kernel_lds(p.S, C);
-    static size_t configured[KUTACC_DEVICE_SLOTS] = {};
-    {
-        const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(fp32_head_kernel), lds_bytes, configured);
-        if (e != hipSuccess) {
-            return (int)e;
-        }
+    switch (a.nheads) {
+    case 1: return launch<2>(a, p, stream);
+    case 2: return launch<4>(a, p, stream);
+    case 3: return launch<6>(a, p, stream);
+    case 4: return launch<8>(a, p, stream);
+    case 5: return launch<10>(a, p, stream);
+    case 6: return launch<12>(a, p, stream);
+    case 7: return launch<14>(a, p, stream);
+    default: return launch<16>(a, p, stream);
     }
-    const double BS = (double)a.batch * (double)a.seq_len;
-    {
-        kutacc_prof::KernelTimer t("fp32_head_kernel", 8.0 * BS * C * C + 4.0 * BS * (double)a.seq_len * C, stream);
-        fp32_head_kernel<<<dim3((unsigned)(a.batch * a.nheads)), 256, lds_bytes, stream>>>(p);
-        const int rc = kutacc_hip_status(hipGetLastError());
-        if (rc != 0) {
-            return rc;
-        }
-    }
-    const int64_t M = a.batch * a.seq_len;
-    kutacc_prof::KernelTimer t("fp32_rows_gemm_kernel", 2.0 * BS * C * C, stream);
-    const dim3 grid((unsigned)((M + 31) / 32), (unsigned)((C / 32 + 3) / 4));
-    fp32_rows_gemm_kernel<<<grid, 256, 0, stream>>>((const float *)a.avg, a.avg_stride_s, (const float *)a.output_w, C, a.output_b,
-                                                    (float *)a.out, a.out_ld, M, C, C);
-    return kutacc_hip_status(hipGetLastError());
 }
 
 } // namespace kutacc_launch

@@ -147,6 +147,19 @@ def test_fp32_storage_on_the_fp32_matrix_core(torch_cuda, config, batch, seq):
         assert not bool(scratch[name].any()), f"{name} was written"
 
 
+@pytest.mark.parametrize("config,batch,seq", [(1, 1, 1), (1, 1, 16), (1, 2, 17), (2, 1, 49), (2, 1, 224), (3, 33, 80), (2, 40, 113), (3, 64, 160)])
+def test_fp32_storage_shared_queries_and_projection_tiles(torch_cuda, config, batch, seq):
+    """The splits of the fp32 route: a head's queries over one to seven workgroups, half-empty tiles of 32 positions, no split
+    where heads outnumber the CUs, and both tile sizes of the output projection."""
+    w = make_workload(config, batch=batch, seq_len=seq)
+    w.dtype = "fp32"
+    ten, scratch = helpers.to_device(w)
+    assert helpers.run_hip(w, ten, scratch, capi.PATH_FUSED) == 0 and capi.last_path() == "fp32_mfma"
+    ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
+    helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), ref_avg, "fp32", "gated average")
+    helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, "fp32", "out")
+
+
 def test_fp32_storage_beyond_the_matrix_core_path_takes_the_generic_kernels(torch_cuda):
     w = make_workload(1, batch=2, seq_len=225)
     ten, scratch = helpers.to_device(w)
