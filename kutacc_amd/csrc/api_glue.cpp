@@ -321,11 +321,17 @@ int kutacc_hip_triangle_multiplication(const kutacc_hip_triangle_multiplication_
     if (ends && (kutacc_launch::gated_projection_mode() < 2 || n % 8 != 0)) {
         // 128 channels: three launches on planes whose rows start on 16 bytes at every n.  Three such planes per channel fit
         // what four dense ones take: 3 (n (n + 7) + 63 + pad) <= 4 (n^2 + pad) for every n.
-        const int64_t np = (n + 7) / 8 * 8, padded = (n * np + 63) / 64 * 64 + TM_PLANE_PAD;
+        // The direct kernel of the equation takes whole steps of 32: zeros up to there, as columns, and for incoming edges
+        // as rows.  Its last tiles read on past a plane's edges, into what follows in the workspace, and drop the results.
+        const auto plane_of = [](int64_t r, int64_t p) { return (r * p + 63) / 64 * 64 + TM_PLANE_PAD; };
+        const int64_t n32 = (n + 31) / 32 * 32;
+        const bool whole_steps = kutacc_launch::triangle_equation_whole_steps(n, ci) && 3 * align256(ci * plane_of(n32, n32) * 2) <= need;
+        const int64_t np = whole_steps ? n32 : (n + 7) / 8 * 8, lines = whole_steps && a->incoming ? n32 : n;
+        const int64_t padded = plane_of(lines, np);
         void *left = ws, *right = ws + align256(ci * padded * 2), *centre = ws + 2 * align256(ci * padded * 2);
-        int rc = kutacc_launch::triangle_front(*a, left, right, np, padded, s);
+        int rc = kutacc_launch::triangle_front(*a, left, right, lines, np, padded, s);
         if (rc == 0) {
-            rc = kutacc_launch::triangle_equation(left, right, centre, n, np, padded, ci, a->incoming != 0, s);
+            rc = kutacc_launch::triangle_equation(left, right, centre, n, lines, np, padded, ci, a->incoming != 0, whole_steps, s);
         }
         return rc != 0 ? rc : kutacc_launch::triangle_back(*a, centre, np, padded, s);
     }

@@ -163,8 +163,11 @@ int global_attention(const kutacc_hip_global_attention_args_t &args, hipStream_t
 // nothing launched, when the two cannot share one: the caller then makes two calls)
 int pair_gemm(const kutacc_hip_gemm_args_t &args, hipStream_t stream, const kutacc_hip_gemm_args_t *second = nullptr);
 int gated_projection_mode(); // 0: the default rule (see pair_gemm_tuning)
-int triangle_equation(const void *left, const void *right, void *centre, int64_t n, int64_t np, int64_t plane, int64_t channels, bool incoming,
-                      hipStream_t stream);
+// whole_steps, where triangle_equation_whole_steps(n, channels) says so: np a multiple of 32 and, for incoming edges, rows as well, with
+// zeros past n; 255 rows (columns, incoming) past a plane's end are readable
+bool triangle_equation_whole_steps(int64_t n, int64_t channels);
+int triangle_equation(const void *left, const void *right, void *centre, int64_t n, int64_t rows, int64_t np, int64_t plane, int64_t channels,
+                      bool incoming, bool whole_steps, hipStream_t stream);
 // transition.hip
 bool transition_fused_supports(int64_t rows, int64_t c_o, int64_t c_i, const void *x, const void *w1, const float *b1,
                                const void *w2, const float *b2, const void *out);
@@ -176,9 +179,10 @@ int sigmoid_gate_rows(void *out, int64_t out_s0, int64_t out_s1, const void *gat
                       int64_t n0, int64_t n1, int64_t size, hipStream_t stream);
 
 // triangle_multiplication.hip: the block's LayerNorm + gated projections, and its centre LayerNorm + gated output projection +
-// residual, at 128 channels; planes of n rows of np positions, np = n rounded up to 8, `plane` elements apart
+// residual, at 128 channels; planes of `rows` >= n rows of np positions, np a multiple of 8, `plane` elements apart; zeros past n
 bool triangle_ends_support(const kutacc_hip_triangle_multiplication_args_t &args);
-int triangle_front(const kutacc_hip_triangle_multiplication_args_t &args, void *left, void *right, int64_t np, int64_t plane, hipStream_t stream);
+int triangle_front(const kutacc_hip_triangle_multiplication_args_t &args, void *left, void *right, int64_t rows, int64_t np, int64_t plane,
+                   hipStream_t stream);
 int triangle_back(const kutacc_hip_triangle_multiplication_args_t &args, const void *centre, int64_t np, int64_t plane, hipStream_t stream);
 
 // glue_kernels.hip

@@ -898,7 +898,9 @@ __global__ __launch_bounds__(256, 1) void pair_gemm_direct_kernel(const GemmPara
                     const int piece = lane + 64 * e;
                     const int row = piece >> 3, chunk = piece & 7;
                     const int64_t gm = cur.m0 + 128 * wm + 32 * i + row, gn = cur.n0 + 128 * wn + 64 * jh + chunk * 8;
-                    *reinterpret_cast<uint4 *>(c + gm * p.c_sm + gn) = *reinterpret_cast<const uint4 *>(ct + row * DIRECT_STRIP_LD + chunk * 8);
+                    if (gm < p.M && gn < p.N) {
+                        *reinterpret_cast<uint4 *>(c + gm * p.c_sm + gn) = *reinterpret_cast<const uint4 *>(ct + row * DIRECT_STRIP_LD + chunk * 8);
+                    }
                 }
                 __builtin_amdgcn_wave_barrier();
             }
@@ -1653,20 +1655,39 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
 
 int gated_projection_mode() { return g_gated_mode.load(); }
 
+// A length that is no multiple of 256 on the direct kernel, whose last tiles then run over the planes' edges.  Its tiles take
+// half the time of as much work on the 128 x 128 ones but pad more: by default three tiles a side and at most 14 % of
+// padding.  The whole block, us, 128 x 128 tiles against these, outgoing and incoming:
+//   691: 397 358, 384 361    760: 469 414, 453 410    900: 730 693, 716 638    1000: 873 764, 851 749    1250: 1480 1298, 1450 1228
+// and beyond the rule: 508: 173 177, 177 177    640: 300 323, 294 309    800: 534 563, 526 510    1100: 1088 1101, 1071 989
+bool triangle_equation_whole_steps(int64_t n, int64_t channels)
+{
+    const int mode = g_big_tile_mode.load();
+    const int64_t side = (n + BIG_TILE - 1) / BIG_TILE;
+    const bool pays = side >= 3 && 100 * side * BIG_TILE <= 114 * n;
+    return n % BIG_TILE != 0 && n > BIG_TILE && n < (1 << 22) && side * side * channels <= INT32_MAX && (mode == 4 || (mode == 0 && pays));
+}
+
 // The equation of the triangle multiplication on planes whose rows of n positions lie np apart (np a multiple of 8, zeros
 // in the padding): centre[c] = left[c] right[c]^T (outgoing) or right[c]^T left[c] (incoming).  The columns past n of the
 // result's rows are written too, with whatever the padding gives.
-int triangle_equation(const void *left, const void *right, void *centre, int64_t n, int64_t np, int64_t plane, int64_t channels, bool incoming,
-                      hipStream_t stream)
+int triangle_equation(const void *left, const void *right, void *centre, int64_t n, int64_t rows, int64_t np, int64_t plane, int64_t channels,
+                      bool incoming, bool whole_steps, hipStream_t stream)
 {
     GemmParams p;
     std::memset(&p, 0, sizeof(p));
     p.a = (const bf16_t *)(incoming ? right : left), p.b = (const bf16_t *)(incoming ? left : right), p.c = (bf16_t *)centre;
     p.a_sm = p.b_sn = incoming ? 1 : np, p.a_sk = p.b_sk = incoming ? np : 1;
     p.a_sb = p.b_sb = p.c_sb = plane, p.c_sm = np;
-    p.M = (int)n, p.N = (int)np, p.K = (int)(incoming ? n : np), p.batches = (int)channels;
+    p.M = (int)n, p.N = (int)np, p.K = (int)(incoming ? rows : np), p.batches = (int)channels;
     p.a_rows = p.b_rows = (int)(incoming ? np : n);
     const double flops = 2.0 * (double)n * (double)n * (double)n * (double)channels;
+    if (whole_steps) {
+        p.MT = p.NT = (int)((n + BIG_TILE - 1) / BIG_TILE);
+        const int64_t blocks = (int64_t)p.MT * p.NT * p.batches;
+        kutacc_prof::KernelTimer t(incoming ? "pair_gemm_direct_kernel<m-major>" : "pair_gemm_direct_kernel", flops, stream);
+        return kutacc_hip_status(incoming ? launch_direct_tiles<true>(p, blocks, stream) : launch_direct_tiles<false>(p, blocks, stream));
+    }
     const int rc = n == np ? large_tiles(p, incoming, flops, stream) : KUTACC_HIP_EUNSUPPORTED;
     if (rc != KUTACC_HIP_EUNSUPPORTED) {
         return rc;

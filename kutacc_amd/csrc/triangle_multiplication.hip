@@ -96,8 +96,8 @@ constexpr size_t FRONT_LDS = (size_t)(2 * FRONT_STAGE + FRONT_WAVES * 256) * 16 
 
 __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(const bf16_t *__restrict__ x, const float *__restrict__ gamma,
                                                                              const float *__restrict__ beta, float eps, Side s0, Side s1,
-                                                                             const bf16_t *__restrict__ mask, int64_t plane, int n, int np,
-                                                                             int steps_per_group)
+                                                                             const bf16_t *__restrict__ mask, int64_t plane, int n, int rows,
+                                                                             int np, int steps_per_group)
 {
     extern __shared__ uint4 lds[]; // two stages, a panel per wave, two mask rows
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
     uint4 *panel = lds + 2 * FRONT_STAGE + wave * 256;
     uint16_t *mask_rows = reinterpret_cast<uint16_t *>(lds + 2 * FRONT_STAGE + FRONT_WAVES * 256);
 
-    const int positions = n * np, total_steps = (positions + STEP - 1) / STEP;
+    const int positions = rows * np, total_steps = (positions + STEP - 1) / STEP;
     const int first = (int)blockIdx.x * steps_per_group;
     const int stop = first + steps_per_group < total_steps ? first + steps_per_group : total_steps;
     if (first >= stop) {
@@ -490,19 +490,19 @@ bool triangle_ends_support(const kutacc_hip_triangle_multiplication_args_t &a)
            kutacc_hip_aligned16(a.output_w) && kutacc_hip_aligned16(a.gating_w);
 }
 
-int triangle_front(const kutacc_hip_triangle_multiplication_args_t &a, void *left, void *right, int64_t np, int64_t plane, hipStream_t stream)
+int triangle_front(const kutacc_hip_triangle_multiplication_args_t &a, void *left, void *right, int64_t rows, int64_t np, int64_t plane, hipStream_t stream)
 {
     static size_t configured[KUTACC_DEVICE_SLOTS] = {};
     if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&triangle_front_kernel), FRONT_LDS, configured)) {
         return kutacc_hip_status(e);
     }
     kutacc_prof::KernelTimer t("gated_projection_blocks_kernel<2>", 8.0 * (double)(a.n_res * a.n_res) * C * C, stream);
-    const Split s = split_steps(a.n_res, np, kutacc_cu_count());
+    const Split s = split_steps(rows, np, kutacc_cu_count());
     const Side l = {(const bf16_t *)a.left_proj_w, (const bf16_t *)a.left_gate_w, a.left_proj_b, a.left_gate_b, (bf16_t *)left};
     const Side r = {(const bf16_t *)a.right_proj_w, (const bf16_t *)a.right_gate_w, a.right_proj_b, a.right_gate_b, (bf16_t *)right};
     triangle_front_kernel<<<dim3(s.groups), 64 * FRONT_WAVES, FRONT_LDS, stream>>>((const bf16_t *)a.pair_act, a.ln_in_gamma, a.ln_in_beta, a.ln_eps, l,
-                                                                                  r, (const bf16_t *)a.pair_mask, plane, (int)a.n_res, (int)np,
-                                                                                  s.per_group);
+                                                                                  r, (const bf16_t *)a.pair_mask, plane, (int)a.n_res, (int)rows,
+                                                                                  (int)np, s.per_group);
     return kutacc_hip_status(hipGetLastError());
 }
 

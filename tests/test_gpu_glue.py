@@ -452,6 +452,31 @@ def test_triangle_multiplication_block_at_any_length(torch_cuda, n):
         assert bool((guarded[n * n:] == 7.0).all())
 
 
+@pytest.mark.parametrize("n,mode", [(257, "direct"), (290, "direct"), (480, "direct"), (509, "direct"), (674, None), (765, None)])
+def test_triangle_multiplication_block_on_tiles_over_the_edge(torch_cuda, n, mode):
+    """Lengths that are no multiple of 256 on the 256 x 256 tiles, which read past the planes' edges: the same bits as on the
+    128 x 128 tiles, in a workspace that holds NaN beforehand."""
+    torch = torch_cuda
+    case = tm_block_case(3500 + n, n, 128, 128)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
+        device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
+    w = {k: dev(v) for k, v in case.items() if k not in ("z", "mask")}
+    for incoming in (False, True):
+        got = {}
+        for tile in ("128", mode):
+            assert capi.set_tuning("gemm_tile", tile) == 0
+            try:
+                pair = dev(case["z"])
+                blk = capi.TriangleMultiplicationBlock(pair, dev(case["mask"]), w, incoming)
+                blk.workspace.fill_(255)
+                assert blk.run() == 0
+                torch.cuda.synchronize()
+            finally:
+                capi.set_tuning("gemm_tile", None)
+            got[tile] = pair
+        assert bool(torch.isfinite(got[mode]).all()) and helpers.same_bits(got["128"], got[mode]), (n, incoming)
+
+
 @pytest.mark.parametrize("n", [48, 72, 384])
 def test_triangle_multiplication_block_on_each_gated_projection_kernel(torch_cuda, n):
     """The block's two gated projections go out in one launch.  Its default kernel (weights in registers, both sides in
