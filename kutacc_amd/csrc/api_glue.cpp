@@ -197,23 +197,17 @@ int kutacc_hip_triangle_attention(const kutacc_hip_triangle_attention_args_t *a,
     const kutacc_hip_attention_args_t g = triangle_attention_call(a, ws, w, fused_ln);
     if (streamed) {
         // LayerNorm + pair bias, with the tiles the attention reads where the producer can write them; the operator, which
-        // forms the mask bias from the pair mask itself; residual sum (transposed back for the ending node).
-        kutacc_hip_attention_args_t t = g;
-        t.out = ws + w.out;
+        // forms the mask bias from the pair mask itself and adds its result to the pair activation (transposed back for the
+        // ending node).
         kutacc_launch::FusedAttentionOptions opt;
+        opt.out_mode = ending ? kutacc_launch::FUSED_OUT_ADD_TRANSPOSED : kutacc_launch::FUSED_OUT_ADD;
         opt.bias_is_mask = true, opt.bias_stride_k = ending ? n : 1;
         const int nb_blocks = (int)((n + 31) / 32);
         opt.nb_tiles_ready = kutacc_launch::pair_bias_writes_fragments(a->pair_act, a->bias_w, ws + w.z_norm, n, n, c, heads, KUTACC_DTYPE_BF16);
         int rc = kutacc_launch::pair_bias(a->pair_act, a->ln_gamma, a->ln_beta, a->bias_w, ws + w.nb, ws + w.z_norm, n, n, c, heads,
                                           a->ln_eps, KUTACC_DTYPE_BF16, ending, s, opt.nb_tiles_ready ? ws + w.q : nullptr, nb_blocks,
                                           (nb_blocks + 1) & ~1, 1);
-        if (rc == 0) {
-            rc = kutacc_launch::gating_attention_streamed(t, opt, ws + w.q, w.avg - w.q, s);
-        }
-        if (rc == 0) {
-            rc = kutacc_launch::residual_add(a->pair_act, ws + w.out, n, n, c, ending, KUTACC_DTYPE_BF16, s);
-        }
-        return rc;
+        return rc != 0 ? rc : kutacc_launch::gating_attention_streamed(g, opt, ws + w.q, w.avg - w.q, ws + w.out, s);
     }
     if (tiled) {
         // Rows beyond the fused head kernels: the same chain as separate passes -- LayerNorm + pair bias (read transposed
@@ -594,9 +588,8 @@ int kutacc_hip_msa_attention(const kutacc_hip_msa_attention_args_t *a, void *str
     hipStream_t s = kutacc_api::stream_or_default(stream);
     const kutacc_hip_attention_args_t g = msa_attention_call(a, ws, w, fused_ln);
     if (streamed) {
-        kutacc_hip_attention_args_t t = g;
-        t.out = ws + w.out;
         kutacc_launch::FusedAttentionOptions opt;
+        opt.out_mode = column ? kutacc_launch::FUSED_OUT_ADD_TRANSPOSED : kutacc_launch::FUSED_OUT_ADD;
         opt.bias_is_mask = true, opt.bias_stride_k = column ? n_res : 1;
         int rc = kutacc_launch::layernorm_rows(a->msa_act, c, a->ln_gamma, a->ln_beta, ws + w.m_norm, c, n_seq * n_res, c, a->ln_eps,
                                                KUTACC_DTYPE_BF16, s, column ? n_seq : 0);
@@ -608,13 +601,7 @@ int kutacc_hip_msa_attention(const kutacc_hip_msa_attention_args_t *a, void *str
                                           a->c_z, heads, a->ln_eps, KUTACC_DTYPE_BF16, 0, s, opt.nb_tiles_ready ? ws + w.q : nullptr,
                                           nb_blocks, (nb_blocks + 1) & ~1, 1);
         }
-        if (rc == 0) {
-            rc = kutacc_launch::gating_attention_streamed(t, opt, ws + w.q, w.avg - w.q, s);
-        }
-        if (rc == 0) {
-            rc = kutacc_launch::residual_add(a->msa_act, ws + w.out, n_seq, n_res, c, column ? 1 : 0, KUTACC_DTYPE_BF16, s);
-        }
-        return rc;
+        return rc != 0 ? rc : kutacc_launch::gating_attention_streamed(g, opt, ws + w.q, w.avg - w.q, ws + w.out, s);
     }
     if (tiled) {
         // Rows beyond the fused head kernels (more than 1024 keys): LayerNorm (read transposed column-wise), pair bias

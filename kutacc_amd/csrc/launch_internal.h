@@ -134,11 +134,12 @@ int pair_bias_tiles(const kutacc_hip_attention_args_t &args, void *tiles, hipStr
 
 // streamed_attention.hip: rows of any length, 128 or 256 channels in heads of 32, on a workspace of streamed_workspace_bytes()
 // (256-byte aligned) that starts with the tiles of the pair bias; opt.nb_tiles_ready: they lie there already.  args.q, k, v
-// and gate are not used; the result is stored (opt.out_mode FUSED_OUT_STORE).
+// and gate are not used; the result is added to args.out (opt.out_mode FUSED_OUT_ADD or FUSED_OUT_ADD_TRANSPOSED), by way of
+// `spare`, [batch * seq_len, channels], where the projection cannot do that itself.
 bool streamed_attention_supports(const kutacc_hip_attention_args_t &args);
 int64_t streamed_workspace_bytes(int64_t batch, int64_t seq_len, int64_t nheads, bool pair_bias);
 int gating_attention_streamed(const kutacc_hip_attention_args_t &args, const FusedAttentionOptions &opt, void *workspace, int64_t bytes,
-                              hipStream_t stream);
+                              void *spare, hipStream_t stream);
 bool streamed_attention_forced(); // the "streamed" hook: blocks of every size on these kernels
 int streamed_attention_tuning(const char *name, const char *value);
 
@@ -152,6 +153,9 @@ bool row_projection_supports(const void *a, int64_t a_ld, const void *w, const f
 int row_projection(const void *a, int64_t a_ld, const void *w, const float *bias, void *out, int64_t out_ld, int64_t m,
                    int64_t n, int64_t k, hipStream_t stream);
 
+// acc += the product's rows, row (i, j) of their [m / swap_n, swap_n] grid to row (j, i) of acc where swap_n is not zero (not timed)
+int row_projection_residual(const void *a, int64_t a_ld, const void *w, const float *bias, void *acc, int64_t acc_ld, int64_t m,
+                            int64_t n, int64_t k, int64_t swap_n, hipStream_t stream);
 int row_projection_gated_residual(const void *a, int64_t a_ld, const void *w, const float *bias, const void *gate,
                                   int64_t gate_ld, void *acc, int64_t acc_ld, int64_t m, int64_t n, int64_t k,
                                   hipStream_t stream);

@@ -308,6 +308,26 @@ def test_triangle_attention_block_on_the_streamed_kernels(torch_cuda, streamed_e
         helpers.check_close(helpers.to_numpy(got), block_oracle(c, ending), "bf16", f"streamed block n={n} heads={heads} ending={ending}")
 
 
+@pytest.mark.parametrize("n,heads", [(33, 4), (70, 8)])
+def test_streamed_block_adds_its_result_in_a_pass_of_its_own_where_it_must(torch_cuda, streamed_everywhere, n, heads):
+    """An output bias that does not start on 16 bytes keeps the projection from adding into the activation itself: the same
+    bits by way of the workspace."""
+    torch = torch_cuda
+    for ending in (False, True):
+        c = block_case(9450 + n, n, heads)
+        want = run_block(torch, c, ending)
+        dev = lambda a, dt=torch.bfloat16: torch.from_numpy(np.ascontiguousarray(a)).to(device="cuda", dtype=dt)  # noqa: E731
+        f32 = torch.float32
+        bo = torch.cat([torch.zeros(1, device="cuda"), dev(c["bo"], f32)])[1:]
+        pair = dev(c["z"])
+        blk = capi.TriangleAttentionBlock(pair, dev(c["mask"]), dev(c["gamma"], f32), dev(c["beta"], f32), dev(c["bias_w"]),
+                                          dev(c["wq"]), dev(c["wk"]), dev(c["wv"]), dev(c["wg"]), dev(c["bg"], f32), dev(c["wo"]),
+                                          bo, heads, ending)
+        assert bo.data_ptr() % 16 == 4 and blk.run() == 0
+        torch.cuda.synchronize()
+        assert helpers.same_bits(pair, want)
+
+
 def test_fused_layernorm_drops_the_normalised_copy_from_the_workspace(torch_cuda):
     """With the LayerNorm inside the attention kernel the blocks keep no normalised activation: the workspace is one
     activation smaller wherever the persistent kernel runs (384 residues), and unchanged where it does not (1024)."""
