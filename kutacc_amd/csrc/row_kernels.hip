@@ -222,6 +222,7 @@ __global__ __launch_bounds__(256) void layernorm_rows_bf16_kernel(const bf16_t *
 // fp32 accumulation), whose result has one z row per lane: every head's 32 values leave as one 64-byte store.
 // The vector ALU, which bounds this kernel, is left with the LayerNorm alone.
 constexpr int PAIR_BIAS_ROWS_PER_WAVE = 32; // a multiple of 32; LDS per workgroup = 1 KB per row
+constexpr int64_t PAIR_BIAS_MAX_ROWS = (int64_t)1 << 23; // rows and byte offsets are counted in 32 bits: 2 GiB of z
 
 template <int H>
 __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__restrict__ z, const float *__restrict__ gamma,
@@ -552,8 +553,7 @@ int launch_pair_bias(const void *z, const float *gamma, const float *beta, const
          frag_nb != rows_j / 32 || frag_nt != ((frag_nb + 1) & ~1))) {
         return KUTACC_HIP_EINVAL;
     }
-    // the MFMA kernel counts rows and byte offsets in 32 bits: at most 2^23 rows of 256 bytes
-    if (sizeof(T) == 2 && c_z == 128 && (nheads == 4 || nheads == 8) && rows <= ((int64_t)1 << 23) &&
+    if (sizeof(T) == 2 && c_z == 128 && (nheads == 4 || nheads == 8) && rows <= PAIR_BIAS_MAX_ROWS &&
         (reinterpret_cast<uintptr_t>(z) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(z_norm)) % 16 == 0) {
         const int64_t nblk = (rows + 4 * PAIR_BIAS_ROWS_PER_WAVE - 1) / (4 * PAIR_BIAS_ROWS_PER_WAVE);
         if (nblk > INT32_MAX) {
@@ -651,6 +651,7 @@ bool pair_bias_writes_fragments(const void *z, const void *w, const void *z_norm
     // the MFMA producer, whose waves own 32 consecutive rows: whole key tiles of one query when the grid is square
     // and its side a multiple of 32
     return dtype == KUTACC_DTYPE_BF16 && c_z == 128 && (nheads == 4 || nheads == 8) && rows_i == rows_j && rows_j % 32 == 0 &&
+           rows_i * rows_j <= PAIR_BIAS_MAX_ROWS &&
            (reinterpret_cast<uintptr_t>(z) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(z_norm)) % 16 == 0;
 }
 

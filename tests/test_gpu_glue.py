@@ -279,6 +279,35 @@ def test_triangle_attention_block_beyond_1024_residues(torch_cuda):
         helpers.check_close(helpers.to_numpy(sample.contiguous()), want, "bf16", f"block n={n} ending={ending}, sampled rows")
 
 
+def test_triangle_attention_block_past_the_pair_bias_producer_s_rows(torch_cuda):
+    """2912 residues: more rows than the producer of the pair bias counts in 32 bits, so the copy that the attention reads has to
+    come from a pass of its own.  Single queries against plain fp32 torch: a query of a row needs that row, its own row of the
+    pair activation for the bias, and nothing else."""
+    torch = torch_cuda
+    n, heads, C = 2912, 4, 128
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *s, scale=1.0: (torch.randn(*s, device="cuda", generator=g) * scale).to(torch.bfloat16)  # noqa: E731
+    act = rnd(n, n, C)
+    w = {k: rnd(C, C, scale=C ** -0.5) for k in ("q", "k", "v", "g", "o")}
+    bias_w, ones, zeros = rnd(heads, C, scale=4 * C ** -0.5), torch.ones(C, device="cuda"), torch.zeros(C, device="cuda")
+    picks = [(0, 5), (1234, 2900), (n - 1, 700)]
+    norm = lambda t: torch.nn.functional.layer_norm(t.float(), (C,)).to(torch.bfloat16).float()  # noqa: E731
+    want = []
+    for b, q in picks:
+        x = norm(act[b])
+        proj = lambda m, rows: (rows @ w[m].float().T).view(-1, heads, 32).transpose(0, 1)  # noqa: E731
+        nb = (norm(act[q]) @ bias_w.float().T).T
+        p = torch.softmax((proj("q", x[q:q + 1]) @ proj("k", x).transpose(1, 2))[:, 0] * 32 ** -0.5 + nb, dim=1)
+        avg = (p[:, None] @ proj("v", x))[:, 0].reshape(C) * torch.sigmoid(x[q] @ w["g"].float().T + 1.0)
+        want.append(act[b, q].float() + avg @ w["o"].float().T)
+    blk = capi.TriangleAttentionBlock(act, torch.ones(n, n, device="cuda", dtype=torch.bfloat16), ones, zeros, bias_w, w["q"], w["k"],
+                                      w["v"], w["g"], ones, w["o"], zeros, heads, False)
+    assert blk.run() == 0
+    torch.cuda.synchronize()
+    for (b, q), ref in zip(picks, want):
+        helpers.check_close(helpers.to_numpy(act[b, q]), ref.cpu().numpy(), "bf16", f"row {b}, query {q}")
+
+
 @pytest.mark.parametrize("n,heads", [(72, 3), (100, 5), (45, 1)])
 def test_triangle_attention_block_with_other_channel_counts(torch_cuda, n, heads):
     """96, 160 and 32 channels (heads of 32): no fused head kernel takes them, the block's tiled route does; whole result
