@@ -240,22 +240,38 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
     // Rows are counted in 32 bits and addressed by 32-bit byte offsets from the tensors' first elements (the launcher
     // sends at most 2^23 rows here: 2 GiB of z), not by 64-bit products per lane and row.
     const uint32_t nrows = (uint32_t)rows, ncol = (uint32_t)rows_j, nrow_i = (uint32_t)rows_i;
-    const uint32_t r0 = ((uint32_t)blockIdx.x * 4 + wave) * PAIR_BIAS_ROWS_PER_WAVE;
-    if (r0 >= nrows) {
-        return;
+    // A wave's rows: row0 and the `count` - 1 behind it.  Without the attention's copy they are 32 rows as they come.  With it they are
+    // key tile t of query q, on a grid of whole blocks of queries and whole tiles of keys: the last tile of a query has fewer
+    // rows (zeros take the place of the others in the copy), and queries past the last repeat that one, in the copy only.
+    uint32_t row0 = ((uint32_t)blockIdx.x * 4 + wave) * PAIR_BIAS_ROWS_PER_WAVE, count = 0;
+    int q = 0, t = 0;
+    if (nbf == nullptr) {
+        if (row0 >= nrows) {
+            return;
+        }
+        count = min(32u, nrows - row0);
+    } else {
+        const uint32_t tile_index = (uint32_t)blockIdx.x * 4 + wave;
+        q = (int)(tile_index / (uint32_t)frag_nb), t = (int)(tile_index % (uint32_t)frag_nb);
+        if (q >= 32 * frag_nb) {
+            return;
+        }
+        row0 = min((uint32_t)q, nrow_i - 1) * ncol + 32u * t;
+        count = min(32u, ncol - 32u * t);
     }
+    const bool stores = q < (int)nrow_i; // (nrow_i = ncol where there is a copy)
     const char *zbytes = reinterpret_cast<const char *>(z);
     uint4 *tile = tiles[wave];
     Pack16 in[STEPS];
     {
         // transposed: output row (i, j) is computed from row (j, i) of z, stored [rows_j, rows_i, c_z]; the walk
         // over consecutive output rows then steps through z with stride rows_i rows
-        uint32_t r = r0 + grp * STEPS;
+        uint32_t r = row0 + grp * STEPS;
         uint32_t i = transposed ? r / ncol : 0, j = transposed ? r % ncol : 0;
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
             uint32_t src = transposed ? j * nrow_i + i : r;
-            src = r < nrows ? src : 0;
+            src = grp * STEPS + s < (int)count ? src : 0;
             in[s].u = *reinterpret_cast<const uint4 *>(zbytes + (src * (2u * CZ) + 16u * sub));
             ++r;
             if (++j == ncol) {
@@ -285,7 +301,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
         const int row_local = grp * STEPS + s;
-        const uint32_t r = r0 + row_local;
+        const uint32_t r = row0 + row_local;
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -299,7 +315,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
         for (int e = 0; e < 8; ++e) {
             o.b[e] = (bf16_t)fmaf(fmaf(v[e], rstd, shift), gm[e], bt[e]);
         }
-        if (z_norm != nullptr && r < nrows) {
+        if (z_norm != nullptr && stores && row_local < (int)count) {
             *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(z_norm) + (r * (2u * CZ) + 16u * sub)) = o.u;
         }
         tile[((row_local >> 5) * 2 + (sub >> 3)) * 256 + kutacc_dev::panel_slot(row_local & 31, sub & 7)] = o.u;
@@ -314,9 +330,11 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
             const uint4 zf = tile[(rb * 2 + (ks >> 2)) * 256 + kutacc_dev::panel_slot(col, 2 * (ks & 3) + g)];
             acc = kutacc_dev::mfma(wf[ks], kutacc_dev::as_bf16x8(zf), acc);
         }
-        // accumulator v < 4 of lane (col, g) is head 4 g + v of z row r0 + 32 rb + col
-        const uint32_t r = r0 + rb * 32 + col;
-        if (r < nrows) {
+        // accumulator v < 4 of lane (col, g) is head 4 g + v of z row row0 + col
+        static_assert(RB == 1, "a wave is one key tile");
+        const uint32_t r = row0 + col;
+        const bool real = col < (int)count;
+        if (real && stores) {
             char *nbytes = reinterpret_cast<char *>(nb);
             const uint32_t first = 2u * (__umul24(4u * g, nrows) + r); // head 4 g of row r, in bytes; H * rows * 2 < 2^28
 #pragma unroll
@@ -336,7 +354,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 if (4 * g + v < H) {
-                    const float x = (float)(bf16_t)acc[v] * kutacc_dev::LOG2E;
+                    const float x = real ? (float)(bf16_t)acc[v] * kutacc_dev::LOG2E : 0.f;
                     t32[(4 * g + v) * 32 + col] = x < -3.0e38f ? -3.0e38f : x; // -inf: the most negative finite value
                 }
             }
@@ -344,8 +362,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
             if (lane < 8 * H) {
                 const int h = lane >> 3, c = lane & 7; // piece c: keys 4 c .. 4 c + 3 = half g' = c >> 2, piece a = c & 3
                 const uint4 val = *reinterpret_cast<const uint4 *>(t32 + h * 32 + c * 4);
-                const uint32_t r0b = r0 + rb * 32;
-                const int q = (int)(r0b / ncol), t = (int)(r0b % ncol) >> 5, qr = q & 31;
+                const int qr = q & 31;
                 const int qlane = (qr & 3) | (((qr >> 4) & 1) << 2) | (((qr >> 2) & 3) << 3);
                 uint4 *dst = nbf + ((((int64_t)h * frag_nb + (q >> 5)) * frag_nt + t) * 4 + (c & 3)) * 64 + qlane + 32 * (c >> 2);
                 *dst = val;
@@ -354,8 +371,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
                 }
             }
         } else if (nbf != nullptr) {
-            // The copy the attention kernels read (rows_j a multiple of 32: the wave's rows are key tile t of one query
-            // q): for head h, query block j, key tile t, 16-key half g' and 8-key half e the 16 bytes of lane
+            // The copy the attention kernels read: for head h, query block j, key tile t, 16-key half g' and 8-key half e the 16 bytes of lane
             // (pi^-1(q mod 32), g'), pi being the row order of the attention's accumulators; values in log2 units as
             // fp16 (the bf16 pair bias times log2(e), eleven significant bits kept).  Through the wave's tile, which nobody
             // reads any more: [head][32 keys].
@@ -364,15 +380,14 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 if (4 * g + v < H) {
-                    t16[(4 * g + v) * 32 + col] = kutacc_dev::pair_bias_log2_f16((float)(bf16_t)acc[v]);
+                    t16[(4 * g + v) * 32 + col] = real ? kutacc_dev::pair_bias_log2_f16((float)(bf16_t)acc[v]) : (uint16_t)0;
                 }
             }
             __builtin_amdgcn_wave_barrier(); // other lanes' stores: keep the loads below behind them
             if (lane < 4 * H) {
                 const int h = lane >> 2, c = lane & 3;
                 const uint4 val = *reinterpret_cast<const uint4 *>(t16 + h * 32 + c * 8);
-                const uint32_t r0b = r0 + rb * 32;
-                const int q = (int)(r0b / ncol), t = (int)(r0b % ncol) >> 5, qr = q & 31;
+                const int qr = q & 31;
                 const int qlane = (qr & 3) | (((qr >> 4) & 1) << 2) | (((qr >> 2) & 3) << 3);
                 uint4 *dst = nbf + ((((int64_t)h * frag_nb + (q >> 5)) * frag_nt + t) * 2 + (c & 1)) * 64 + qlane + 32 * (c >> 1);
                 *dst = val;
@@ -550,12 +565,13 @@ int launch_pair_bias(const void *z, const float *gamma, const float *beta, const
     if (fragments != nullptr &&
         (!kutacc_launch::pair_bias_writes_fragments(z, w, z_norm, rows_i, rows_j, c_z, nheads,
                                                     sizeof(T) == 2 ? KUTACC_DTYPE_BF16 : KUTACC_DTYPE_FP32) ||
-         frag_nb != rows_j / 32 || frag_nt != ((frag_nb + 1) & ~1))) {
+         frag_nb != (rows_j + 31) / 32 || frag_nt != ((frag_nb + 1) & ~1))) {
         return KUTACC_HIP_EINVAL;
     }
     if (sizeof(T) == 2 && c_z == 128 && (nheads == 4 || nheads == 8) && rows <= PAIR_BIAS_MAX_ROWS &&
         (reinterpret_cast<uintptr_t>(z) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(z_norm)) % 16 == 0) {
-        const int64_t nblk = (rows + 4 * PAIR_BIAS_ROWS_PER_WAVE - 1) / (4 * PAIR_BIAS_ROWS_PER_WAVE);
+        const int64_t wave_tiles = fragments != nullptr ? (int64_t)32 * frag_nb * frag_nb : (rows + PAIR_BIAS_ROWS_PER_WAVE - 1) / PAIR_BIAS_ROWS_PER_WAVE;
+        const int64_t nblk = (wave_tiles + 3) / 4;
         if (nblk > INT32_MAX) {
             return KUTACC_HIP_EUNSUPPORTED;
         }
@@ -648,9 +664,10 @@ int linear(int32_t dtype, const void *act, int64_t ld_act, const void *w, int64_
 bool pair_bias_writes_fragments(const void *z, const void *w, const void *z_norm, int64_t rows_i, int64_t rows_j, int64_t c_z,
                                 int64_t nheads, int32_t dtype)
 {
-    // the MFMA producer, whose waves own 32 consecutive rows: whole key tiles of one query when the grid is square
-    // and its side a multiple of 32
-    return dtype == KUTACC_DTYPE_BF16 && c_z == 128 && (nheads == 4 || nheads == 8) && rows_i == rows_j && rows_j % 32 == 0 &&
+    // The MFMA producer, on a square grid.  At lengths that are no multiple of 32 the whole tiles cost it some waves (77
+    // residues 48 %, 500 5 %) and the block saves a launch: triangle attention at 77 residues 27.2 -> 24.9 us,
+    // 301: 111.2 -> 107.7, 691: 543 -> 539; MSA rows 64 x 77: 42.3 -> 38.0, 508 x 259: 317.9 -> 312.6.
+    return dtype == KUTACC_DTYPE_BF16 && c_z == 128 && (nheads == 4 || nheads == 8) && rows_i == rows_j &&
            rows_i * rows_j <= PAIR_BIAS_MAX_ROWS &&
            (reinterpret_cast<uintptr_t>(z) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(z_norm)) % 16 == 0;
 }

@@ -260,6 +260,24 @@ def test_triangle_attention_block_full_size_sampled_rows(torch_cuda, n):
         helpers.check_close(helpers.to_numpy(sample.contiguous()), want, "bf16", f"block n={n} ending={ending}, sampled rows")
 
 
+@pytest.mark.parametrize("n", [33, 95, 290, 361, 385, 449])
+def test_producer_writes_the_attention_s_pair_bias_copy_at_ragged_lengths(torch_cuda, n):
+    """Lengths that are no multiple of 32 (one row past a tile, one short of it, odd and even tile counts), on the single-row, the
+    two-row and the long-row kernel: no pass of its own for the copy, and the last query block's and key tile's rows against the
+    oracle, both orientations."""
+    torch = torch_cuda
+    c = block_case(7500 + n, n, 4)
+    rows = sorted({0, 1, 31, 32, n // 2, n - 2, n - 1})
+    for ending in (False, True):
+        res = {}
+        names = profiled_kernels(torch, lambda: res.setdefault("z", run_block(torch, c, ending)))
+        got = res["z"]
+        assert "pair_bias_tiles_kernel" not in names and "pair_bias_fragments_kernel" not in names, names
+        assert bool(torch.isfinite(got).all())
+        sample = got[:, rows].transpose(0, 1) if ending else got[rows]
+        helpers.check_close(helpers.to_numpy(sample.contiguous()), block_oracle_rows(c, ending, rows), "bf16", f"block n={n} ending={ending}")
+
+
 def test_triangle_attention_block_beyond_1024_residues(torch_cuda):
     """1088 residues: past the fused head kernels' longest row, the block runs the same chain as separate passes with the
     operator on the tiled MFMA route.  Both orientations against the oracle on a sample of attention rows."""
