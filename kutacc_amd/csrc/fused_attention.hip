@@ -2281,7 +2281,7 @@ __global__ __launch_bounds__(64) void pair_bias_fragments_kernel(const bf16_t *_
 // Tuning hooks (kutacc_hip_set_tuning): a forced plan of the long-sequence kernel, the fragment-major pair bias switched
 // off, one line per call on stderr.  Plain atomics: set from a test or an experiment, read on every launch.
 std::atomic<int> g_forced_bpw{0}, g_forced_gw{0}, g_no_fragments{0}, g_debug{0};
-std::atomic<int> g_pair_mode{0}; // persistent_pair_kernel: 0 = where every workgroup has two batch rows or more, 1 = wherever it can run, 2 = never
+std::atomic<int> g_pair_mode{0}; // persistent_pair_kernel: 0 = where row_pairs_pay says so, 1 = wherever it can run, 2 = never
 
 bool fragments_disabled() { return g_no_fragments.load(std::memory_order_relaxed) != 0; }
 
@@ -2424,9 +2424,21 @@ void *fragment_home(const kutacc_hip_attention_args_t &a, int NB, const kutacc_l
     return (q_dense && nbf_bytes <= a.batch * a.seq_len * C * 2) ? a.q : nullptr;
 }
 
-// Two batch rows per step (persistent_pair_kernel): 128 channels, log2 units, a home for the fp32 tiles of the pair bias
+// Whether the rows of a workgroup are better walked in pairs.  With an odd number the last pair costs as much as a whole
+// one, which a pair's gain over two single rows (2 % with 128 channels, 5 to 10 % with 256) makes up for from some number on.
+// Operator, us, pairs against single rows.  128 channels, squares: 135 (three rows) 31.5 28.0, 180 (three) 36.4 32.2, 200
+// (four) 40.6 40.6, 290 (five) 74.7 66.2, 384 (six) 94.1 96.1; 448 x 200 (seven) 67.5 65.1, 576 x 200 (nine) 78.5 76.7, 704 x
+// 200 (eleven) 93.6 93.4.  256 channels: 96 x 250 (three) 58.7 51.4, 160 x 250 (five) 75.1 69.7, 224 x 128 and x 250 (seven)
+// 53.9 55.9 and 92.7 89.7, 352 x 128 (eleven) 71.8 75.9.
+bool row_pairs_pay(const kutacc_hip_attention_args_t &a)
+{
+    const int64_t sequences = 8 * (int64_t)persistent_groups((int)a.batch, (int)a.nheads), rows = (a.batch + sequences - 1) / sequences;
+    return a.batch >= 2 * sequences && (rows % 2 == 0 || rows >= (a.nheads * a.head_size == 128 ? 11 : 7));
+}
+
+// Two batch rows per step (persistent_pair_kernel): 128 or 256 channels, log2 units, a home for the fp32 tiles of the pair bias
 // (twice the fragments' bytes), no LayerNorm inside the kernel and no ready-made fp16 fragments; by default only where
-// every workgroup walks at least two rows.
+// that pays.
 bool pair_kernel_applies(const kutacc_hip_attention_args_t &a, const Plan &pl, const kutacc_launch::FusedAttentionOptions &opt)
 {
     const int pair_mode = g_pair_mode.load(std::memory_order_relaxed);
@@ -2434,7 +2446,7 @@ bool pair_kernel_applies(const kutacc_hip_attention_args_t &a, const Plan &pl, c
     return pl.persistent && (C == 128 || C == 256) && pair_mode != 2 && !fragments_disabled() && opt.ln_gamma == nullptr &&
            !opt.nb_fragments_ready && pair_kernel_lds((int)C, pl.NB) <= (size_t)max_lds_bytes() &&
            (a.nonbatched_bias == nullptr || fragment_home(a, pl.NB, opt, 2) != nullptr) &&
-           (pair_mode == 1 || a.batch >= 16 * (int64_t)persistent_groups((int)a.batch, (int)a.nheads));
+           (pair_mode == 1 || row_pairs_pay(a));
 }
 
 template <typename K>

@@ -278,6 +278,23 @@ def test_producer_writes_the_attention_s_pair_bias_copy_at_ragged_lengths(torch_
         helpers.check_close(helpers.to_numpy(sample.contiguous()), block_oracle_rows(c, ending, rows), "bf16", f"block n={n} ending={ending}")
 
 
+@pytest.mark.parametrize("n,pairs", [(129, False), (192, False), (193, True), (257, False)])
+def test_odd_numbers_of_rows_per_workgroup_take_the_single_row_kernel(torch_cuda, n, pairs):
+    """Three, three, four and five rows a workgroup (256 CUs), both orientations, first and last rows against the oracle."""
+    torch = torch_cuda
+    c = block_case(7700 + n, n, 4)
+    rows = [0, 1, n - 2, n - 1]
+    for ending in (False, True):
+        res = {}
+        names = profiled_kernels(torch, lambda: res.setdefault("z", run_block(torch, c, ending)))
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert ("persistent_pair_kernel" in names) == pairs, names
+        got = res["z"]
+        assert bool(torch.isfinite(got).all())
+        sample = got[:, rows].transpose(0, 1) if ending else got[rows]
+        helpers.check_close(helpers.to_numpy(sample.contiguous()), block_oracle_rows(c, ending, rows), "bf16", f"block n={n} ending={ending}")
+
+
 def test_triangle_attention_block_beyond_1024_residues(torch_cuda):
     """1088 residues: past the fused head kernels' longest row, the block runs the same chain as separate passes with the
     operator on the tiled MFMA route.  Both orientations against the oracle on a sample of attention rows."""
