@@ -2449,6 +2449,26 @@ bool pair_kernel_applies(const kutacc_hip_attention_args_t &a, const Plan &pl, c
            (pair_mode == 1 || row_pairs_pay(a));
 }
 
+// The plan of a call.  Short rows of 128 channels (two to four blocks) give the persistent kernel four waves a CU where a
+// workgroup per unit, with a third of the LDS, has twelve.  Staging the weights for every unit costs less than that as soon as
+// a workgroup of the persistent kernel would walk a second row.  Operator, us, persistent against one workgroup per unit: 66 x 96
+// 18.7 17.0, 96 x 60 17.9 17.2, 128 x 128 18.5 17.3, 190 x 80 22.9 20.5, 256 x 80 25.8 25.7, 500 x 128 42.7 38.5; one row a
+// workgroup, 60 x 128: 15.5 15.6; five blocks, 128 x 150: 24.1 26.9.
+bool make_call_plan(const kutacc_hip_attention_args_t &a, const kutacc_launch::FusedAttentionOptions &opt, Plan &pl)
+{
+    const int C = (int)(a.nheads * a.head_size);
+    if (!make_plan(a.seq_len, C, pl)) {
+        return false;
+    }
+    if (pl.persistent && C == 128 && pl.NB >= 2 && pl.NB <= 4 && a.batch > 8 * (int64_t)persistent_groups((int)a.batch, (int)a.nheads) &&
+        opt.ln_gamma == nullptr && g_pair_mode.load(std::memory_order_relaxed) != 1 && !fragments_disabled() &&
+        (a.nonbatched_bias == nullptr || fragment_home(a, pl.NB, opt) != nullptr)) {
+        pl.persistent = false;
+        pl.lds_bytes = head_kernel_lds(C, pl.NB, pl.GW, pl.NW, pl.BPW);
+    }
+    return true;
+}
+
 template <typename K>
 int opt_in_lds(K kern, size_t bytes, size_t *table)
 {
@@ -2592,7 +2612,7 @@ bool fused_attention_tile_layout(const kutacc_hip_attention_args_t &a, const Fus
 {
     Plan pl;
     if (a.nonbatched_bias == nullptr || opt.nb_fragments_ready || !fused_attention_supports(a) ||
-        !make_plan(a.seq_len, (int)(a.nheads * a.head_size), pl) || !pair_kernel_applies(a, pl, opt)) {
+        !make_call_plan(a, opt, pl) || !pair_kernel_applies(a, pl, opt)) {
         return false;
     }
     *nb = pl.NB, *nt = (pl.NB + 1) & ~1;
@@ -2660,7 +2680,7 @@ int gating_attention_fused(const kutacc_hip_attention_args_t &a, hipStream_t str
     const int residual = opt.out_mode;
     const int C = (int)(a.nheads * a.head_size);
     Plan pl;
-    if (!make_plan(a.seq_len, C, pl)) {
+    if (!make_call_plan(a, opt, pl)) {
         return KUTACC_HIP_EUNSUPPORTED;
     }
     if (opt.bias_stride_k < 0 || opt.bias_stride_k > (1 << 20) || a.input_ld <= 0 || a.input_ld > (1 << 19)) {

@@ -278,6 +278,19 @@ def test_producer_writes_the_attention_s_pair_bias_copy_at_ragged_lengths(torch_
         helpers.check_close(helpers.to_numpy(sample.contiguous()), block_oracle_rows(c, ending, rows), "bf16", f"block n={n} ending={ending}")
 
 
+@pytest.mark.parametrize("n", [65, 96, 97, 128])
+def test_short_rows_take_a_workgroup_per_unit(torch_cuda, n):
+    """Three and four blocks of 32, whole and ragged, with two rows to a CU and head: the long-row kernel, every row against the oracle."""
+    torch = torch_cuda
+    c = block_case(7800 + n, n, 4)
+    for ending in (False, True):
+        res = {}
+        names = profiled_kernels(torch, lambda: res.setdefault("z", run_block(torch, c, ending)))
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert "fused_head_kernel" in names, names
+        helpers.check_close(helpers.to_numpy(res["z"]), block_oracle(c, ending), "bf16", f"block n={n} ending={ending}")
+
+
 @pytest.mark.parametrize("n,pairs", [(129, False), (192, False), (193, True), (257, False)])
 def test_odd_numbers_of_rows_per_workgroup_take_the_single_row_kernel(torch_cuda, n, pairs):
     """Three, three, four and five rows a workgroup (256 CUs), both orientations, first and last rows against the oracle."""
