@@ -1,4 +1,4 @@
-// Gated attention for fp32 storage on the fp32 matrix core (v_mfma_f32_32x32x2_f32), head_size 32, short sequences.
+// Gated attention for fp32 storage on the fp32 matrix core (v_mfma_f32_16x16x4_f32), head_size 32, short sequences.
 //
 // The reference serves every call through its GEMM (src/linear/mm.cpp:77-86); the bf16 kernels of fused_attention.hip
 // take bf16 storage only, and an fp32 tensor rounded to bf16 operands would miss the fp32 bar (1e-4 relative).  The

@@ -3,8 +3,9 @@
 // them lies the equation, one n x n product per channel (pair_stack.hip).
 //
 // Layout of the intermediates.  The projections and the centre are channel-first, one plane per channel, and a plane's
-// rows are n positions padded to a pitch of np = n rounded up to 8: every row then starts on 16 bytes, whatever n is, and
-// the products run on the matrix cores with vector loads at every length.  The projections write zeros into the padding
+// rows are n positions padded to a pitch of np, n rounded up to 8 (to 32, and for incoming edges the rows too, where the
+// product takes whole steps of that): every row then starts on 16 bytes, whatever n is, and the products run on the matrix
+// cores with vector loads at every length.  The projections write zeros into the padding
 // (their mask is zero there), so a contraction over np positions is one over n.  With dense rows an n that is no multiple
 // of 8 left the product to scalar loads: 217 ms for the block at 691 residues, 0.39 ms so.
 //
