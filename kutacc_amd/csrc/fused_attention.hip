@@ -2453,14 +2453,17 @@ bool pair_kernel_applies(const kutacc_hip_attention_args_t &a, const Plan &pl, c
 // workgroup per unit, with a third of the LDS, has twelve.  Staging the weights for every unit costs less than that as soon as
 // a workgroup of the persistent kernel would walk a second row.  Operator, us, persistent against one workgroup per unit: 66 x 96
 // 18.7 17.0, 96 x 60 17.9 17.2, 128 x 128 18.5 17.3, 190 x 80 22.9 20.5, 256 x 80 25.8 25.7, 500 x 128 42.7 38.5; one row a
-// workgroup, 60 x 128: 15.5 15.6; five blocks, 128 x 150: 24.1 26.9.
+// workgroup, 60 x 128: 15.5 15.6; five blocks, 128 x 150: 24.1 26.9.  With 256 channels the weights are four times as many, and it
+// pays where some workgroups would walk two rows and none more: 40 x 77 30.3 29.0, 60 x 64 28.5 27.1, 60 x 110 31.4 30.6; two
+// rows each, in pairs, 64 x 128: 29.7 30.0; three, 90 x 80: 35.9 37.5.
 bool make_call_plan(const kutacc_hip_attention_args_t &a, const kutacc_launch::FusedAttentionOptions &opt, Plan &pl)
 {
     const int C = (int)(a.nheads * a.head_size);
     if (!make_plan(a.seq_len, C, pl)) {
         return false;
     }
-    if (pl.persistent && C == 128 && pl.NB >= 2 && pl.NB <= 4 && a.batch > 8 * (int64_t)persistent_groups((int)a.batch, (int)a.nheads) &&
+    const int64_t sequences = 8 * (int64_t)persistent_groups((int)a.batch, (int)a.nheads); // of rows, one per workgroup and head
+    if (pl.persistent && pl.NB >= 2 && pl.NB <= 4 && a.batch > sequences && (C == 128 || a.batch < 2 * sequences) &&
         opt.ln_gamma == nullptr && g_pair_mode.load(std::memory_order_relaxed) != 1 && !fragments_disabled() &&
         (a.nonbatched_bias == nullptr || fragment_home(a, pl.NB, opt) != nullptr)) {
         pl.persistent = false;

@@ -291,6 +291,26 @@ def test_short_rows_take_a_workgroup_per_unit(torch_cuda, n):
         helpers.check_close(helpers.to_numpy(res["z"]), block_oracle(c, ending), "bf16", f"block n={n} ending={ending}")
 
 
+@pytest.mark.parametrize("n_seq,n_res", [(33, 64), (63, 33), (40, 127)])
+def test_short_msa_rows_take_a_workgroup_per_unit(torch_cuda, n_seq, n_res):
+    """256 channels, two to four blocks, two rows to a CU and head: the long-row kernel, the whole block against the oracle."""
+    torch = torch_cuda
+    c = msa_case(9600 + n_seq + n_res, n_seq, n_res, 8, 128)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
+        device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
+    msa = dev(c["m"])
+    w = {k: dev(c[k]) for k in ("ln_gamma", "ln_beta", "wq", "wk", "wv", "wg", "bg", "wo", "bo")}
+    pair = {"pair_act": dev(c["z"]), "pair_ln_gamma": dev(c["pair_ln_gamma"]), "pair_ln_beta": dev(c["pair_ln_beta"]), "bias_w": dev(c["bias_w"])}
+    blk = capi.MsaAttentionBlock(msa, dev(c["mask"]), w, 8, pair)
+    res = {}
+    names = profiled_kernels(torch, lambda: res.setdefault("rc", blk.run()))
+    torch.cuda.synchronize()
+    assert res["rc"] == 0
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert "fused_head_kernel" in names, names
+    helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, False), "bf16", f"msa rows {n_seq}x{n_res}")
+
+
 @pytest.mark.parametrize("n,pairs", [(129, False), (192, False), (193, True), (257, False)])
 def test_odd_numbers_of_rows_per_workgroup_take_the_single_row_kernel(torch_cuda, n, pairs):
     """Three, three, four and five rows a workgroup (256 CUs), both orientations, first and last rows against the oracle."""
