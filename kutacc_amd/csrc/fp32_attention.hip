@@ -86,8 +86,9 @@ __global__ __launch_bounds__(512, 2) void fp32_head_kernel(Fp32Params p)
     const int r = lane & 15, g = lane >> 4;
     constexpr int C = 16 * PIECES;
     const int S = p.S, NB = (S + 31) / 32, S32 = NB * 32;
-    const int part = blockIdx.x % p.parts, bh = blockIdx.x / p.parts;
-    const int b = bh / p.H, h = bh % p.H;
+    // neighbouring workgroups, dealt to different XCDs, take different heads: with eight each L2 holds one head's weights
+    const int h = blockIdx.x % p.H, rest = blockIdx.x / p.H;
+    const int part = rest % p.parts, b = rest / p.parts;
     const int t_lo = NB * part / p.parts, t_hi = NB * (part + 1) / p.parts; // query tiles of this workgroup
     const int XP = C + 4, VP = S32 + 4; // odd multiples of 16 bytes, as LDP
 
