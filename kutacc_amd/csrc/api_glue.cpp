@@ -199,6 +199,9 @@ int kutacc_hip_triangle_attention(const kutacc_hip_triangle_attention_args_t *a,
         // LayerNorm + pair bias, with the tiles the attention reads where the producer can write them; the operator, which
         // forms the mask bias from the pair mask itself and adds its result to the pair activation (transposed back for the
         // ending node).
+        if (!kutacc_launch::streamed_attention_supports(g)) {
+            return KUTACC_HIP_EUNSUPPORTED;
+        }
         kutacc_launch::FusedAttentionOptions opt;
         opt.out_mode = ending ? kutacc_launch::FUSED_OUT_ADD_TRANSPOSED : kutacc_launch::FUSED_OUT_ADD;
         opt.bias_is_mask = true, opt.bias_stride_k = ending ? n : 1;
@@ -588,6 +591,9 @@ int kutacc_hip_msa_attention(const kutacc_hip_msa_attention_args_t *a, void *str
     hipStream_t s = kutacc_api::stream_or_default(stream);
     const kutacc_hip_attention_args_t g = msa_attention_call(a, ws, w, fused_ln);
     if (streamed) {
+        if (!kutacc_launch::streamed_attention_supports(g)) {
+            return KUTACC_HIP_EUNSUPPORTED;
+        }
         kutacc_launch::FusedAttentionOptions opt;
         opt.out_mode = column ? kutacc_launch::FUSED_OUT_ADD_TRANSPOSED : kutacc_launch::FUSED_OUT_ADD;
         opt.bias_is_mask = true, opt.bias_stride_k = column ? n_res : 1;

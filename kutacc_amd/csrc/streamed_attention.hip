@@ -118,8 +118,7 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
 #pragma unroll
         for (int ks = 0; ks < CK; ++ks) {
             const int at = (h * HEAD + r) * C + ks * 16 + g * 8;
-            w0[ks] = *reinterpret_cast<const bf16x8 *>(m0 + at);
-            w1[ks] = *reinterpret_cast<const bf16x8 *>(m1 + at);
+            w0[ks] = as_bf16x8(load8_any(m0, at)), w1[ks] = as_bf16x8(load8_any(m1, at)); // once per workgroup: on any address
         }
     }
     park(0, rows);
@@ -164,7 +163,8 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
                 const float *bg = p.bg + h * HEAD + 4 * g;
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
-                    const f32x4 bv = *reinterpret_cast<const f32x4 *>(bg + 8 * a);
+                    f32x4 bv;
+                    __builtin_memcpy(&bv, bg + 8 * a, 16); // on any address
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
                         a0[4 * a + c] *= p.qmul;
@@ -553,9 +553,8 @@ bool streamed_attention_supports(const kutacc_hip_attention_args_t &a)
     const int64_t C = a.nheads * a.head_size;
     return a.dtype == KUTACC_DTYPE_BF16 && a.head_size == HEAD && (C == 128 || C == 256) && a.seq_len > 0 && a.seq_len <= (1 << 20) &&
            a.batch > 0 && a.batch <= (1 << 24) && a.batch * blocks_of(a.seq_len) <= INT32_MAX / 4 && a.input_ld % 8 == 0 &&
-           kutacc_hip_aligned16(a.input) && kutacc_hip_aligned16(a.query_w) && kutacc_hip_aligned16(a.key_w) && kutacc_hip_aligned16(a.value_w) &&
-           kutacc_hip_aligned16(a.gating_w) && kutacc_hip_aligned16(a.gating_b) && a.avg_stride_h == HEAD && a.avg_stride_s % 8 == 0 &&
-           a.avg_stride_b == a.seq_len * a.avg_stride_s && kutacc_hip_aligned16(a.avg);
+           kutacc_hip_aligned16(a.input) && a.avg_stride_h == HEAD && a.avg_stride_s % 8 == 0 && a.avg_stride_b == a.seq_len * a.avg_stride_s &&
+           kutacc_hip_aligned16(a.avg);
 }
 
 int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedAttentionOptions &opt, void *workspace, int64_t bytes,

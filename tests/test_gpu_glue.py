@@ -425,6 +425,47 @@ def test_streamed_block_adds_its_result_in_a_pass_of_its_own_where_it_must(torch
         assert helpers.same_bits(pair, want)
 
 
+def drawn_block(torch, seed, kind, n_seq, n_res, heads):
+    """A block whose inputs are drawn on the device: kind "triangle" (n_res residues, ending node), "row" or "column" (MSA).  Returns
+    the activation, its weights as a dict and a function (activation, weights) -> block."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *s, scale=1.0: (torch.randn(*s, device="cuda", generator=g) * scale).to(torch.bfloat16)  # noqa: E731
+    around = lambda centre, size: centre + 0.1 * torch.randn(size, device="cuda", generator=g)  # noqa: E731
+    C = 32 * heads
+    act = rnd(n_res if kind == "triangle" else n_seq, n_res, C)
+    w = {k: rnd(C, C, scale=C ** -0.5) for k in ("wq", "wk", "wv", "wg", "wo")}
+    w.update(ln_gamma=around(1.0, C), ln_beta=around(0.0, C), bg=around(1.0, C), bo=around(0.0, C))
+    mask = (torch.rand(act.shape[:2], device="cuda", generator=g) > 0.1).to(torch.bfloat16)
+    if kind == "triangle":
+        bias_w = rnd(heads, C, scale=C ** -0.5)
+        return act, w, lambda z, v: capi.TriangleAttentionBlock(z, mask, v["ln_gamma"], v["ln_beta"], bias_w, v["wq"], v["wk"], v["wv"], v["wg"],
+                                                                v["bg"], v["wo"], v["bo"], heads, True)
+    pair = None
+    if kind == "row":
+        pair = dict(pair_act=rnd(n_res, n_res, 64), pair_ln_gamma=around(1.0, 64), pair_ln_beta=around(0.0, 64), bias_w=rnd(heads, 64, scale=0.125))
+    return act, w, lambda z, v: capi.MsaAttentionBlock(z, mask, v, heads, pair)
+
+
+@pytest.mark.parametrize("kind,n_seq,n_res,heads", [("triangle", 0, 1025, 4), ("row", 3, 1050, 8), ("column", 1030, 2, 4)])
+def test_blocks_beyond_1024_keys_take_weights_on_any_address(torch_cuda, kind, n_seq, n_res, heads):
+    """The route of these blocks asks nothing of the weights' alignment: the same bits with every matrix and both biases one element
+    past a 16-byte boundary."""
+    torch = torch_cuda
+    act, w, block = drawn_block(torch, 77 + n_res, kind, n_seq, n_res, heads)
+    moved = {k: t if k.startswith("ln_") else torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape) for k, t in w.items()}
+    assert all(moved[k].data_ptr() % 16 == w[k].element_size() for k in ("wq", "wk", "wv", "wg", "wo", "bg", "bo"))
+    res = []
+    for weights in (w, moved):
+        z = act.clone()
+        print(f"{kind} {n_seq}x{n_res} heads={heads} moved={weights is moved}", flush=True)
+        rc = block(z, weights).run()
+        torch.cuda.synchronize()
+        assert rc == 0, rc
+        res.append(z)
+    assert bool(torch.isfinite(res[0]).all()) and not helpers.same_bits(res[0], act)
+    assert helpers.same_bits(res[0], res[1])
+
+
 def test_fused_layernorm_drops_the_normalised_copy_from_the_workspace(torch_cuda):
     """With the LayerNorm inside the attention kernel the blocks keep no normalised activation: the workspace is one
     activation smaller wherever the persistent kernel runs (384 residues), and unchanged where it does not (1024)."""
