@@ -247,7 +247,7 @@ int kutacc_hip_triangle_attention(const kutacc_hip_triangle_attention_args_t *a,
     }
     // 1. LayerNorm + pair-bias projection in one pass over the pair tensor; the ending node reads it transposed
     //    -- and, where the grid allows it, writes the copy the attention kernel will read as well: fp32 tiles where
-    //    the operator takes the two-row kernel, fp16 fragments otherwise
+    //    the workgroups walk two rows or more, fp16 fragments otherwise
     void *z_norm = fused_ln ? nullptr : ws + w.z_norm;
     int frag_nb = 0, frag_nt = 0;
     const bool writes = kutacc_launch::pair_bias_writes_fragments(a->pair_act, a->bias_w, z_norm, n, n, c, heads, KUTACC_DTYPE_BF16);
@@ -652,8 +652,8 @@ int kutacc_hip_msa_attention(const kutacc_hip_msa_attention_args_t *a, void *str
         opt.input_stride_b = column ? c : n_res * c;
     }
     // 2. pair bias from the pair activation (row-wise form only)
-    //    -- with the copy the attention kernel will read, where the grid allows it: fp32 tiles for the two-row kernel,
-    //    fp16 fragments otherwise
+    //    -- with the copy the attention kernel will read, where the grid allows it: fp32 tiles or fp16
+    //    fragments
     if (rc == 0 && !column) {
         int frag_nb = 0, frag_nt = 0;
         const bool writes = kutacc_launch::pair_bias_writes_fragments(a->pair_act, a->bias_w, nullptr, n_res, n_res, a->c_z, heads,

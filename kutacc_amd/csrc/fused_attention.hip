@@ -75,7 +75,7 @@ struct FusedParams {
     int nb_vec;   // pair-bias rows may be read with 16-byte loads
     float qscale; // 1 / sqrt(head_size)
     int ngrp;     // persistent kernel: batch-row groups per XCD
-    const uint4 *nbf; // pair bias * log2(e), fp16, in fragment-major order (pair_bias_fragments_kernel), or nullptr
+    const uint4 *nbf; // pair bias * log2(e): fp16, in fragment-major order (pair_bias_fragments_kernel), or fp32 tiles, or nullptr
     int NT;           // key tiles the LDS arrays are laid out for: NB rounded up to an even number (the log2-unit
                       // loop walks tile pairs; a phantom tile is all zeros behind a -inf mask)
     int l2mode;       // logits in log2 units (attend_block_l2); needs nbf when there is a pair bias
@@ -448,7 +448,9 @@ __device__ __forceinline__ void attend_block(const uint4 *lds_k, const uint4 *ld
 // loads per tile and wave).  The 8 MFMAs of a tile sit, fenced, between the exp/convert pieces of the
 // neighbouring tile's softmax.  The loop runs one extra (clamped) logits computation at the end
 // instead of a peeled epilogue.  Requires an even number of key tiles.
-//   nbf : this wave's fragment-major pair bias, already offset by the lane: tile t at nbf[(2t+m)*64]
+// TILES: the pair bias comes as fp32 tiles in accumulator order (pair_bias_tiles_kernel), which seed the logits MFMAs: twice the
+// bytes of the fragments, no selector MFMAs, and no second rounding of the bias.
+//   nbf : this wave's fragment-major pair bias, already offset by the lane: tile t at nbf[(2t+m)*64] (TILES: nbf[(4t+a)*64])
 //   returns the row sum of every lane's query in l_out
 
 // Issue priority of a wave among the (up to three) waves of its workgroup on one SIMD, by time slices of the clock they
@@ -479,7 +481,22 @@ __device__ __forceinline__ void timeslice_priority(uint32_t turn, int shift)
                  : "scc");
 }
 
-template <bool HAS_NB, bool WITH_MASK, bool SHIFT>
+// fp32 tile t of the pair bias, from a pointer offset by the lane
+__device__ __forceinline__ f32x16 pair_bias_tile(const uint4 *nbf, int t)
+{
+    f32x16 c;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(nbf + (t * 4 + a) * 64);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            c[4 * a + e] = v[e];
+        }
+    }
+    return c;
+}
+
+template <bool HAS_NB, bool WITH_MASK, bool SHIFT, bool TILES = false>
 __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 *lds_v, const f32x4 *mask4,
                                                 const uint4 *nbf, bf16x8 q0, bf16x8 q1, f16x8 sel0, f16x8 sel1,
                                                 bf16x8 sumsel, int NB, int lane, float shift, f32x16 &o_out, float &l_out,
@@ -506,10 +523,22 @@ __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 
         return x;
     };
     auto clampt = [&](int t) { return t < NB ? t : NB - 1; };
+    auto load_tile = [&](int t) { return pair_bias_tile(nbf, t); };
+    auto seed = [&](int t, const f32x16 &C) { // of the logits, where the mask has to be added to the tile
+        f32x16 x = init(t);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            x[v] += C[v];
+        }
+        return x;
+    };
 
-    // pair-bias words: wa* belong to even tiles, wb* to odd tiles
+    // pair-bias words: wa* belong to even tiles, wb* to odd tiles; tiles Ca and Cb likewise
     uint4 wa0 = {}, wa1 = {}, wb0 = {}, wb1 = {}, k0, k1, v0, v1;
-    if (HAS_NB) {
+    f32x16 Ca, Cb;
+    if constexpr (TILES) {
+        Ca = load_tile(0), Cb = load_tile(clampt(1));
+    } else if (HAS_NB) {
         wa0 = nbf[0], wa1 = nbf[64];
         wb0 = nbf[2 * 64], wb1 = nbf[3 * 64];
         // Pinned in this order, ahead of the reload of wa below: the loop then finds the loads in flight in the order it
@@ -519,7 +548,10 @@ __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 
     }
     k0 = kp[0], k1 = kp[64];
     f32x16 xa = init(0), xb;
-    if (HAS_NB) {
+    if constexpr (TILES) {
+        xa = seed(0, Ca);
+        Ca = load_tile(clampt(2));
+    } else if (HAS_NB) {
         xa = mfma_f16(sel0, as_f16x8(wa0), xa);
         xa = mfma_f16(sel1, as_f16x8(wa1), xa);
         wa0 = nbf[clampt(2) * 128], wa1 = nbf[clampt(2) * 128 + 64];
@@ -542,8 +574,30 @@ __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 
     // One half step: the softmax and P.V of the finished tile `xc`, with the logits MFMAs of the
     // following tile `xn` (pair-bias words w0, w1) spread between its pieces; t_w is the tile whose
     // pair-bias words replace w0, w1 once consumed, t_k the tile whose K fragments replace k0, k1.
-    auto half_step = [&](f32x16 &xc, f32x16 &xn, int t_next, uint4 &w0, uint4 &w1, int t_w, int t_k) {
+    auto half_step = [&](f32x16 &xc, f32x16 &xn, int t_next, uint4 &w0, uint4 &w1, f32x16 &C, int t_w, int t_k) {
         bf16x8 p0, p1;
+        if constexpr (TILES) {
+            xn = WITH_MASK ? seed(t_next, C) : C;
+            exp4(xc, 0);
+            exp4(xc, 4);
+            p0 = pack8(xc, 0);
+            fence();
+            xn = mfma(as_bf16x8(k0), q0, xn);
+            asm volatile("" ::"v"(C)); // C stays live past its reader: the logits get registers of their own
+            o = mfma(as_bf16x8(v0), p0, o);
+            C = load_tile(t_w);
+            exp4(xc, 8);
+            fence();
+            xn = mfma(as_bf16x8(k1), q1, xn);
+            lacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sumsel, p0, lacc, 0, 0, 0);
+            k0 = kp[(t_k * 2 + 0) * 64], k1 = kp[(t_k * 2 + 1) * 64];
+            exp4(xc, 12);
+            p1 = pack8(xc, 8);
+            fence();
+            o = mfma(as_bf16x8(v1), p1, o);
+            lacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sumsel, p1, lacc, 0, 0, 0);
+            return;
+        }
         xn = init(t_next);
         if (HAS_NB) {
             xn = mfma_f16(sel0, as_f16x8(w0), xn);
@@ -590,11 +644,11 @@ __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 
         const int t1 = 2 * pair + 1;
         const int tn = pair + 1 < npairs ? 2 * pair + 2 : 2 * pair; // next pair's first tile, clamped
         // ---- odd tile's logits under the even tile's softmax ----
-        half_step(xa, xb, t1, wb0, wb1, clampt(t1 + 2), tn);
+        half_step(xa, xb, t1, wb0, wb1, Cb, clampt(t1 + 2), tn);
         v0 = vp[(t1 * 2 + 0) * 64], v1 = vp[(t1 * 2 + 1) * 64];
         fence();
         // ---- next pair's even tile under the odd tile's softmax ----
-        half_step(xb, xa, tn, wa0, wa1, clampt(tn + 2), tn + 1);
+        half_step(xb, xa, tn, wa0, wa1, Ca, clampt(tn + 2), tn + 1);
         v0 = vp[(tn * 2 + 0) * 64], v1 = vp[(tn * 2 + 1) * 64];
         fence();
     }
@@ -607,7 +661,7 @@ __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 
 
 // Row maxima of the logits (log2 units) of one 32-query block over all key tiles: the shift for the
 // repeat of attend_block_l2 after an overflow or underflow.  Not a hot path: operands are loaded at use.
-template <bool HAS_NB>
+template <bool HAS_NB, bool TILES = false>
 __device__ __forceinline__ float row_max_l2(const uint4 *lds_k, const f32x4 *mask4, const uint4 *nbf, bf16x8 q0, bf16x8 q1,
                                             f16x8 sel0, f16x8 sel1, int NB, int lane)
 {
@@ -622,7 +676,13 @@ __device__ __forceinline__ float row_max_l2(const uint4 *lds_k, const f32x4 *mas
                 x[4 * a + c] = mv[c];
             }
         }
-        if (HAS_NB) {
+        if constexpr (TILES) {
+            const f32x16 C = pair_bias_tile(nbf, t);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                x[v] += C[v];
+            }
+        } else if (HAS_NB) {
             x = mfma_f16(sel0, as_f16x8(nbf[t * 128]), x);
             x = mfma_f16(sel1, as_f16x8(nbf[t * 128 + 64]), x);
         }
@@ -801,12 +861,13 @@ __device__ inline void stage_weight_fragments(uint4 *lds_w, const FusedParams &p
 // and keeps them in registers until then.  At 1024 keys that leaves room for all four weight matrices of a
 // 128-channel head (two of a 256-channel one) beside K and V, so the input rows are read once (twice).
 // ------------------------------------------------------------------------------------------------
-template <int C, int BPW, bool HAS_NB>
+template <int C, int BPW, bool HAS_NB, bool TILES>
 __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(FusedParams p)
 {
     constexpr int CK = C / 16;
     constexpr bool V_ALIAS = C == 256 && BPW == 4; // second LDS layout, below
     constexpr bool ONE_GROUP = V_ALIAS || C == 128; // all four weight matrices staged at once, always (see make_plan)
+    const bool l2mode = TILES || p.l2mode != 0;
     extern __shared__ uint4 lds[];
 
     // XCD-aware unit mapping: consecutive workgroup ids land on different XCDs (8 of them), so the H
@@ -859,7 +920,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
         mask_raw[q] = mask_bias_fetch(p.bias + (int64_t)b * p.bias_sb, S, (wave + q * NW) * 64 + lane, p.bias_sk);
     }
 
-    const float qmul = p.l2mode ? p.qscale * LOG2E : p.qscale;
+    const float qmul = l2mode ? p.qscale * LOG2E : p.qscale;
     // ---- projections, in groups of GW weight matrices staged through LDS ----
     bf16x8 qf[BPW][2];   // Q^T fragments (B operand of the logits MFMA), scaled by 1/sqrt(d)
     bf16x8 gate[BPW][2]; // sigmoid(gate) in accumulator order, packed
@@ -1092,7 +1153,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
     for (int q = 0; q < MASK_PARTS; ++q) {
         const int part = wave + q * NW;
         if (part * 64 < NT * 32) {
-            const float mv = mask_bias_finish(mask_raw[q], part * 64 + lane < S, p.l2mode ? LOG2E : 1.0f, p.bias_is_mask != 0);
+            const float mv = mask_bias_finish(mask_raw[q], part * 64 + lane < S, l2mode ? LOG2E : 1.0f, p.bias_is_mask != 0);
             mask[part * 64 + lane] = mv;
             const unsigned long long nz = __ballot(mv != 0.f);
             if (lane == 0) {
@@ -1110,7 +1171,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
     const f32x4 *mask4 = reinterpret_cast<const f32x4 *>(mask + 16 * g);
     // one pair of selector fragments, as bits: fp16 ones for the log2-unit loop (fp16 pair-bias fragments), bf16 ones otherwise
     uint4 selw0, selw1;
-    if (p.l2mode) {
+    if (l2mode) {
         f16x8 a, b;
         make_selectors_f16(lane, a, b);
         selw0 = as_uint4(a), selw1 = as_uint4(b);
@@ -1131,20 +1192,20 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
         const int qrow = qpos < S ? qpos : S - 1;
         f32x16 o;
         float l;
-        if (p.l2mode) {
-            const uint4 *nbf = HAS_NB ? p.nbf + ((int64_t)(h * NB + j) * NT * 2) * 64 + lane : nullptr;
+        if (l2mode) {
+            const uint4 *nbf = HAS_NB ? p.nbf + ((int64_t)(h * NB + j) * NT * (TILES ? 4 : 2)) * 64 + lane : nullptr;
             if (flags == 0u) {
-                attend_block_l2<HAS_NB, false, false>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel, NT,
+                attend_block_l2<HAS_NB, false, false, TILES>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel, NT,
                                                       lane, 0.f, o, l, (wave >> 2) & 1);
             } else {
-                attend_block_l2<HAS_NB, true, false>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel, NT,
+                attend_block_l2<HAS_NB, true, false, TILES>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel, NT,
                                                      lane, 0.f, o, l, (wave >> 2) & 1);
             }
             __builtin_amdgcn_s_setprio(0);
             if (__any(!(l > 1e-30f && l < 1e30f))) {
                 // some probability overflowed or a whole row underflowed: shift by the true row maxima
-                const float m = row_max_l2<HAS_NB>(lds_k, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), NT, lane);
-                attend_block_l2<HAS_NB, true, true>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel, NT,
+                const float m = row_max_l2<HAS_NB, TILES>(lds_k, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), NT, lane);
+                attend_block_l2<HAS_NB, true, true, TILES>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel, NT,
                                                     lane, m, o, l);
             }
         } else {
@@ -1177,7 +1238,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
 // on the next row's loads and projections while the slower waves of its SIMD still attend, so the
 // latency- and MFMA-bound projection phase overlaps the VALU-heavy attention phase.
 // ------------------------------------------------------------------------------------------------
-template <int C, bool HAS_NB, bool L2MODE, bool FUSED_LN>
+template <int C, bool HAS_NB, bool L2MODE, bool FUSED_LN, bool TILES>
 __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_head_kernel(FusedParams p)
 {
     constexpr int CK = C / 16;
@@ -1427,19 +1488,19 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_head_kernel(F
         const uint32_t flags = *flag_word;
         const bf16_t *nb_head = HAS_NB ? p.nb + (int64_t)h * p.nb_sh : nullptr;
         if constexpr (L2MODE) {
-            const uint4 *nbf = HAS_NB ? p.nbf + ((int64_t)(h * NB + j) * NT * 2) * 64 + lane : nullptr;
+            const uint4 *nbf = HAS_NB ? p.nbf + ((int64_t)(h * NB + j) * NT * (TILES ? 4 : 2)) * 64 + lane : nullptr;
             if (flags == 0u) {
-                attend_block_l2<HAS_NB, false, false>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
+                attend_block_l2<HAS_NB, false, false, TILES>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
                                                       l, -1, fair_turn);
             } else {
-                attend_block_l2<HAS_NB, true, false>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
+                attend_block_l2<HAS_NB, true, false, TILES>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
                                                      l, -1, fair_turn);
             }
             const bool ok = !__any(!(l > 1e-30f && l < 1e30f));
             if (!ok) {
                 // some probability overflowed or a whole row underflowed: shift by the true row maxima
-                const float m = row_max_l2<HAS_NB>(lds_k, mask4, nbf, q0, q1, sel0, sel1, NT, lane);
-                attend_block_l2<HAS_NB, true, true>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, m, o, l);
+                const float m = row_max_l2<HAS_NB, TILES>(lds_k, mask4, nbf, q0, q1, sel0, sel1, NT, lane);
+                attend_block_l2<HAS_NB, true, true, TILES>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, m, o, l);
             }
         } else {
             attend_block<HAS_NB>(lds_k, lds_v, mask4, flags, nb_head, p.nb_sq, j * 32, p.nb_vec != 0, panel, q0, q1, sel0,
@@ -2289,6 +2350,7 @@ struct Plan {
     bool persistent;
     int NB, NW, BPW, GW;
     size_t lds_bytes;
+    bool tiles; // of a call: the pair bias as fp32 tiles instead of fp16 fragments
 };
 
 int max_lds_bytes()
@@ -2351,7 +2413,7 @@ bool make_plan(int64_t S, int C, Plan &pl)
         return false;
     }
     pl.NB = (int)NB;
-    pl.persistent = false;
+    pl.persistent = pl.tiles = false;
     const size_t cap = (size_t)max_lds_bytes();
     const int forced_bpw = g_forced_bpw.load(std::memory_order_relaxed), forced_gw = g_forced_gw.load(std::memory_order_relaxed);
     // persistent kernel: one wave per sequence block, everything of one head resident in LDS
@@ -2426,10 +2488,10 @@ void *fragment_home(const kutacc_hip_attention_args_t &a, int NB, const kutacc_l
 
 // Whether the rows of a workgroup are better walked in pairs.  With an odd number the last pair costs as much as a whole
 // one, which a pair's gain over two single rows (2 % with 128 channels, 5 to 10 % with 256) makes up for from some number on.
-// Operator, us, pairs against single rows.  128 channels, squares: 135 (three rows) 31.5 28.0, 180 (three) 36.4 32.2, 200
-// (four) 40.6 40.6, 290 (five) 74.7 66.2, 384 (six) 94.1 96.1; 448 x 200 (seven) 67.5 65.1, 576 x 200 (nine) 78.5 76.7, 704 x
-// 200 (eleven) 93.6 93.4.  256 channels: 96 x 250 (three) 58.7 51.4, 160 x 250 (five) 75.1 69.7, 224 x 128 and x 250 (seven)
-// 53.9 55.9 and 92.7 89.7, 352 x 128 (eleven) 71.8 75.9.
+// Operator, us, pairs against single rows on the same fp32 tiles.  128 channels: 187 x 200 (three rows) 38.6 34.4, 187 x 384 59.4
+// 54.9, 315 x 290 (five) 75.5 69.0, 443 x 200 (seven) 65.0 63.1, 443 x 384 104.2 105.4, 571 x 200 (nine) 79.5 79.1, 699 x 200
+// (eleven) 91.8 92.1, 699 x 384 159 163.  256 channels: 93 x 250 (three) 55.2 50.9, 157 x 250 (five) 70.8 69.3, 221 x 250
+// (seven) 88.4 88.5, 285 x 250 (nine) 109.6 112.7, 349 x 128 (eleven) 69.8 70.5.
 bool row_pairs_pay(const kutacc_hip_attention_args_t &a)
 {
     const int64_t sequences = 8 * (int64_t)persistent_groups((int)a.batch, (int)a.nheads), rows = (a.batch + sequences - 1) / sequences;
@@ -2452,10 +2514,14 @@ bool pair_kernel_applies(const kutacc_hip_attention_args_t &a, const Plan &pl, c
 // The plan of a call.  Short rows of 128 channels (two to four blocks) give the persistent kernel four waves a CU where a
 // workgroup per unit, with a third of the LDS, has twelve.  Staging the weights for every unit costs less than that as soon as
 // a workgroup of the persistent kernel would walk a second row.  Operator, us, persistent against one workgroup per unit: 66 x 96
-// 18.7 17.0, 96 x 60 17.9 17.2, 128 x 128 18.5 17.3, 190 x 80 22.9 20.5, 256 x 80 25.8 25.7, 500 x 128 42.7 38.5; one row a
-// workgroup, 60 x 128: 15.5 15.6; five blocks, 128 x 150: 24.1 26.9.  With 256 channels the weights are four times as many, and it
+// 18.7 17.0, 96 x 60 17.9 17.2; in pairs, both on fp32 tiles, 128 x 128 17.8 17.2, 190 x 80 24.4 20.0, 256 x 80 25.5 24.7, 500 x
+// 128 41.4 39.8; one row a workgroup, 60 x 128: 15.5 15.6; five blocks, 128 x 150: 24.1 26.9.  With 256 channels the weights are four times as many, and it
 // pays where some workgroups would walk two rows and none more: 40 x 77 30.3 29.0, 60 x 64 28.5 27.1, 60 x 110 31.4 30.6; two
-// rows each, in pairs, 64 x 128: 29.7 30.0; three, 90 x 80: 35.9 37.5.
+// two rows each, in pairs, 64 x 128: 29.7 30.0; three, 90 x 80: 35.9 37.5.
+//
+// The pair bias: from two rows a workgroup on, where the persistent kernel fits, as fp32 tiles wherever those have a home, for pairs
+// and for single rows alike (the 11 bits of the fragments were off by 1.1 % in the average at a bias of 50, the tiles by 0.3 %;
+// single rows 2 to 4 % slower: 135 x 135 27.8 28.6, 290 x 290 64.2 66.8, 96 x 250 with 256 channels 49.7 51.3).
 bool make_call_plan(const kutacc_hip_attention_args_t &a, const kutacc_launch::FusedAttentionOptions &opt, Plan &pl)
 {
     const int C = (int)(a.nheads * a.head_size);
@@ -2463,6 +2529,7 @@ bool make_call_plan(const kutacc_hip_attention_args_t &a, const kutacc_launch::F
         return false;
     }
     const int64_t sequences = 8 * (int64_t)persistent_groups((int)a.batch, (int)a.nheads); // of rows, one per workgroup and head
+    pl.tiles = pl.persistent && a.batch >= 2 * sequences && opt.ln_gamma == nullptr && !opt.nb_fragments_ready && fragment_home(a, pl.NB, opt, 2) != nullptr;
     if (pl.persistent && pl.NB >= 2 && pl.NB <= 4 && a.batch > sequences && (C == 128 || a.batch < 2 * sequences) &&
         opt.ln_gamma == nullptr && g_pair_mode.load(std::memory_order_relaxed) != 1 && !fragments_disabled() &&
         (a.nonbatched_bias == nullptr || fragment_home(a, pl.NB, opt) != nullptr)) {
@@ -2478,10 +2545,10 @@ int opt_in_lds(K kern, size_t bytes, size_t *table)
     return (int)kutacc_opt_in_lds(reinterpret_cast<const void *>(kern), bytes, table);
 }
 
-template <int C, int BPW, bool HAS_NB>
+template <int C, int BPW, bool HAS_NB, bool TILES = false>
 int launch_head_kernel(const FusedParams &p, const Plan &pl, hipStream_t stream)
 {
-    auto kern = fused_head_kernel<C, BPW, HAS_NB>;
+    auto kern = fused_head_kernel<C, BPW, HAS_NB, TILES>;
     static size_t configured[KUTACC_DEVICE_SLOTS] = {}; // per instantiation and device: dynamic LDS opted into so far
     if (const int rc = opt_in_lds(kern, pl.lds_bytes, configured)) {
         return rc;
@@ -2491,10 +2558,10 @@ int launch_head_kernel(const FusedParams &p, const Plan &pl, hipStream_t stream)
     return kutacc_hip_status(hipGetLastError());
 }
 
-template <int C, bool HAS_NB, bool L2MODE, bool FUSED_LN = false>
+template <int C, bool HAS_NB, bool L2MODE, bool FUSED_LN = false, bool TILES = false>
 int launch_persistent_kernel(FusedParams p, const Plan &pl, hipStream_t stream)
 {
-    auto kern = persistent_head_kernel<C, HAS_NB, L2MODE, FUSED_LN>;
+    auto kern = persistent_head_kernel<C, HAS_NB, L2MODE, FUSED_LN, TILES>;
     static size_t configured[KUTACC_DEVICE_SLOTS] = {};
     if (const int rc = opt_in_lds(kern, pl.lds_bytes, configured)) {
         return rc;
@@ -2527,10 +2594,18 @@ int dispatch_head_kernel(const FusedParams &p, const Plan &pl, hipStream_t strea
             return nb ? launch_persistent_kernel<C, true, true, true>(p, pl, stream)
                       : launch_persistent_kernel<C, false, true, true>(p, pl, stream);
         }
+        if (pl.tiles) {
+            return launch_persistent_kernel<C, true, true, false, true>(p, pl, stream);
+        }
         if (p.l2mode) {
             return nb ? launch_persistent_kernel<C, true, true>(p, pl, stream) : launch_persistent_kernel<C, false, true>(p, pl, stream);
         }
         return nb ? launch_persistent_kernel<C, true, false>(p, pl, stream) : launch_persistent_kernel<C, false, false>(p, pl, stream);
+    }
+    if constexpr (C == 128) {
+        if (pl.tiles) { // the short rows that make_call_plan takes from the persistent kernel: one block per wave
+            return launch_head_kernel<C, 1, true, true>(p, pl, stream);
+        }
     }
     switch (pl.BPW) {
         case 1: return nb ? launch_head_kernel<C, 1, true>(p, pl, stream) : launch_head_kernel<C, 1, false>(p, pl, stream);
@@ -2615,7 +2690,7 @@ bool fused_attention_tile_layout(const kutacc_hip_attention_args_t &a, const Fus
 {
     Plan pl;
     if (a.nonbatched_bias == nullptr || opt.nb_fragments_ready || !fused_attention_supports(a) ||
-        !make_call_plan(a, opt, pl) || !pair_kernel_applies(a, pl, opt)) {
+        !make_call_plan(a, opt, pl) || !(pl.tiles || pair_kernel_applies(a, pl, opt))) {
         return false;
     }
     *nb = pl.NB, *nt = (pl.NB + 1) & ~1;
@@ -2720,13 +2795,13 @@ int gating_attention_fused(const kutacc_hip_attention_args_t &a, hipStream_t str
     }
     void *const tiles = fragment_home(a, pl.NB, opt, 2);
     const bool pair_kernel = pair_kernel_applies(a, pl, opt);
-    if (opt.nb_tiles_ready && (!pair_kernel || p.nb == nullptr)) {
+    if (opt.nb_tiles_ready && (!(pl.tiles || pair_kernel) || p.nb == nullptr)) {
         return KUTACC_HIP_EINVAL; // the caller asks fused_attention_tile_layout under the same options and tuning first
     }
 
     const double BS = (double)a.batch * (double)a.seq_len;
     int rc;
-    if (pair_kernel) {
+    if (pair_kernel || pl.tiles) {
         if (p.nb != nullptr && opt.nb_tiles_ready) {
             p.nbf = (const uint4 *)tiles; // the producer of the pair bias wrote the tiles
         } else if (p.nb != nullptr) {

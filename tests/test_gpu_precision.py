@@ -1,0 +1,61 @@
+"""What is computed in 32 bits stays so: calls whose inputs make one operand's rounding the largest error by far, against float64 on
+the same bf16 inputs.  A value rounded to bf16 is off by 2^-9 / sqrt(3) = 0.11 % of itself in the root mean square; a result behind n
+such roundings, each independent, by 0.11 % sqrt(n).  The bars are somewhat under twice that, below what one more
+rounding of the operand in question would give."""
+import numpy as np
+import pytest
+
+import helpers
+from kutacc_amd import capi
+from kutacc_amd.workloads import MASK_BIAS, round_to_bf16
+from test_gpu_tiled_attention import draw_workload
+
+pytestmark = pytest.mark.gpu
+
+BF16_RMS = 2.0 ** -9 / 3 ** 0.5
+
+
+@pytest.fixture(scope="module")
+def torch_cuda():
+    import torch
+    assert torch.cuda.is_available(), "these tests need the GPU"
+    capi.set_stream(None)
+    capi.set_blocking(True)
+    return torch
+
+
+def gated_average_f64(w):
+    """softmax(q.k^T / sqrt(d) + bias + nb) . v * sigmoid(gate) of a workload, [B, S, C]."""
+    f = lambda a: np.asarray(a, dtype=np.float64)  # noqa: E731
+    heads = lambda m: (f(w.x) @ f(m).T).reshape(w.B, w.S, w.H, w.d).transpose(0, 2, 1, 3)  # noqa: E731
+    x = heads(w.wq) @ heads(w.wk).transpose(0, 1, 3, 2) / w.d ** 0.5 + f(w.bias)[:, None, None, :]
+    x = x + (f(w.nb)[None] if w.nb is not None else 0.0)
+    p = np.exp(x - x.max(axis=-1, keepdims=True))
+    avg = (p / p.sum(axis=-1, keepdims=True)) @ heads(w.wv)
+    return avg.transpose(0, 2, 1, 3).reshape(w.B, w.S, w.C) / (1.0 + np.exp(-(f(w.x) @ f(w.wg).T + f(w.bg))))
+
+
+def relative_error(got, want):
+    return float(np.linalg.norm(got - want) / np.linalg.norm(want))
+
+
+@pytest.mark.parametrize("B,S,H", [
+    (135, 135, 4),  # three rows a workgroup, one at a time
+    (140, 33, 4), (190, 80, 4), (130, 97, 4), (128, 128, 4),  # short rows, a workgroup per row and head
+    (70, 100, 8), (96, 256, 8),  # 256 channels, three rows a workgroup
+    (128, 160, 4),  # two rows, together
+])
+def test_pair_bias_keeps_32_bits(torch_cuda, B, S, H):
+    """A pair bias around 50, whose bf16 steps are a quarter: times log2(e) in 11 bits the probabilities would be off by 0.6 %.  Two
+    queries sit at 200 and -200, where the softmax is repeated with the row maxima subtracted, and some keys are masked."""
+    w = draw_workload(40 + B + S, B, S, H, 32, masked=0.05)
+    w.nb = w.nb * np.float32(0.5) + np.float32(50.0)
+    w.nb[:, S // 2, :] += np.float32(150.0)
+    w.nb[:, S - 1, :] -= np.float32(250.0)
+    w.nb = round_to_bf16(w.nb)
+    print(f"B={B} S={S} H={H}", flush=True)
+    ten, scratch = helpers.to_device(w)
+    assert helpers.run_hip(w, ten, scratch) == 0 and capi.last_path() == "fused_mfma"
+    err = relative_error(helpers.to_numpy(scratch["avg"]).reshape(B, S, -1), gated_average_f64(w))
+    # q, k, v, probabilities, gate and result are rounded; q and k move a logit by 0.002 of its size, which is about one
+    assert err < 1.8 * 6 ** 0.5 * BF16_RMS, err
