@@ -168,7 +168,7 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
                         a0[4 * a + c] *= p.qmul;
-                        a1[4 * a + c] = sigmoid_fast(a1[4 * a + c] + bv[c]);
+                        a1[4 * a + c] += bv[c]; // the gate is rounded in front of its sigmoid, as where the reference stores it
                     }
                 }
                 p.q[at] = as_uint4(pack8(a0, 0)), p.q[at + 64] = as_uint4(pack8(a0, 8));
@@ -477,9 +477,9 @@ __global__ __launch_bounds__(768) void streamed_attention_kernel(const StreamedP
             f32x16 gv;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                gv[i] = to_f32(g0[i]), gv[8 + i] = to_f32(g1[i]);
+                gv[i] = sigmoid_f32(to_f32(g0[i])), gv[8 + i] = sigmoid_f32(to_f32(g1[i]));
             }
-            store_gated(p.avg + (int64_t)b * p.avg_sb + (int64_t)qpos * p.avg_ss + h * HEAD + 4 * (lane >> 5), o, __builtin_amdgcn_rcpf(l), gv);
+            store_gated(p.avg + (int64_t)b * p.avg_sb + (int64_t)qpos * p.avg_ss + h * HEAD + 4 * (lane >> 5), o, 1.0f / l, gv);
         };
         store(bA, rowA, oA, lA);
         if (bB != bA) {
