@@ -270,6 +270,15 @@ __device__ __forceinline__ uint4 transpose8x8_lanes(uint4 v, uint32_t sel)
     return make_uint4(d[0], d[1], d[2], d[3]);
 }
 
+// 4 x 4 transposition of dwords over the four lanes that differ in lane bits 4 and 5: before, lane with index c = lane >> 4 holds
+// dwords (c, 0 .. 3), after, dwords (0 .. 3, c)
+__device__ __forceinline__ uint4 transpose4x4_lanes(const uint32_t (&v)[4])
+{
+    const auto a = __builtin_amdgcn_permlane16_swap(v[0], v[1], false, false), b = __builtin_amdgcn_permlane16_swap(v[2], v[3], false, false);
+    const auto lo = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false), hi = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+    return make_uint4(lo[0], hi[0], lo[1], hi[1]);
+}
+
 // LDS transposing read of gfx950 (ds_read_b64_tr_b16).  Within 16 lanes, lane i receives element (i & 3) of the 8-byte
 // chunks that lanes 4j + (i >> 2), j = 0..3, point at.  With lane s of a group pointing at row k0 + (s >> 2), columns
 // m0 + 4 (s & 3) .. +3 of a tile stored [k][m], lane i ends up with k0..k0+3 of column m0 + i: a 4 x 16 block

@@ -1,19 +1,17 @@
 // Attention with heads of 8 (the extra-MSA row attention: 64 channels, eight heads) for gfx950: the middle step of the tiled
 // route (tiled_attention.hip), reading q, k, v and gate as its projections leave them.
 //
-// A head of 8 leaves the matrix cores a quarter of a product's rows: 33 M logits take 4 % of a GFLOP and the exponential
-// decides.  What the vector ALU does per logit is therefore kept to that exponential, half a packed conversion and a fourth
-// of the pair bias's conversion:
-//   * logits in log2 units straight from the MFMA.  q * log2(e)/sqrt(d) needs more than the eight bits of a bf16 operand to
-//     keep the reference's product of bf16 q and k: the unused half of the 16 k-slots carries the rest, q = hi + lo
-//     against the same keys, exact to 2^-17;
-//   * the pair bias is the C operand of four batch rows' logits (a wave attends the same 32 queries of four rows at once);
-//   * a row's mask is one more MFMA, only for key tiles that have one; ragged ends are keys at -inf;
-//   * p.v with 16x16x32 MFMAs whose sixteen rows are the eight values of queries n and of queries n + 16 (the probability
-//     fragment of the 32-query layout holds both): half the matrix-pipe time of the 32x32 form and four registers
-//     instead of sixteen; row sums likewise (rowsum_selector).
-// K, V and masks of a head's four rows lie in the LDS for the whole workgroup (128 bytes per key and 16 of mask words).
-// Measured on 1024 rows x 301 keys x 8 heads: 505 us on the general attention_tiles_kernel, 200 us here (exponentials alone: 85).
+// A head of 8 fills little of a matrix product: the 742 M logits of 1024 rows x 301 keys x 8 heads are 24 GFLOP of products, 71 as
+// they fill the tiles, 57 us of the matrix cores; their exponentials take 85 us of the vector ALU.  What that does per logit is
+// kept to the exponential, half a packed conversion and a fourth of the pair bias's conversion:
+//   * logits in log2 units straight from a 16x16x32 MFMA.  q * log2(e)/sqrt(d) has 24 significant bits: three parts of eight, exact,
+//     in three of the four chunks of k-slots, against the same keys in each;
+//   * the pair bias is the C operand of four batch rows' logits (a wave attends the same 32 queries of four rows at once), with the
+//     keys past the end at -inf; masks are added to it in fp32, only in key tiles that have one;
+//   * p.v with 16x16x32 MFMAs of 32 keys whose rows are the eight values and ones, which give the sums of the probabilities.
+// K, V and masks of a head's four rows lie in the LDS for the whole workgroup (128 bytes per key and 16 of masks).
+// Measured on 1024 rows x 301 keys x 8 heads: 505 us on the general attention_tiles_kernel, 203 us here.  With the queries and
+// the masks in two parts (16 bits, an error of up to 8 % in a probability at logits of 11 000) and 32x32x16 products it was 199.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -39,8 +37,9 @@ struct SmallHeadParams {
     float scale2;                  // log2(e) / sqrt(8)
 };
 
-// slot of key i of a tile of 32: accumulator row r of the logits stands for key pi(r), so that a lane holds 16 consecutive keys
-__device__ __forceinline__ int key_slot(int i) { return (i & 3) | (((i >> 4) & 1) << 2) | (((i >> 2) & 3) << 3); }
+// slot of key i of a tile of 32: row m of half a of the logits products stands for key 8 (m / 4) + 4 a + m % 4, so that a lane's
+// four accumulator rows of both halves are eight consecutive keys, the chunk of p.v's k-slots that the lane supplies
+__device__ __forceinline__ int key_slot(int i) { return 16 * ((i >> 2) & 1) + 4 * (i >> 3) + (i & 3); }
 
 template <bool HAS_NB>
 __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const SmallHeadParams p)
@@ -59,11 +58,13 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
     auto row_of = [&](int i) { return min(b0 + i, p.B - 1); }; // past the last row: that one again
 
     // LDS, a tile's four rows together so that a lane's one offset serves them all: K [tile][row][32] (in key_slot order), V
-    // [tile][row][k-step][half][value], a tile of zeros, mask words [tile][row][32]
-    uint4 *ks = lds, *vs = lds + ROWS * keys, *zeros = vs + ROWS * keys;
-    uint32_t *words = reinterpret_cast<uint32_t *>(zeros + TILE), *first_masked = words + ROWS * keys;
+    // [tile][row][chunk of eight keys][value], a tile of constants (slots 32 i zeros, 32 i + 1 ones), masks in log2 units [tile][row][32]
+    uint4 *ks = lds, *vs = lds + ROWS * keys, *constants = vs + ROWS * keys;
+    float *masks = reinterpret_cast<float *>(constants + TILE);
+    uint32_t *first_masked = reinterpret_cast<uint32_t *>(masks + ROWS * keys);
     for (int idx = tid; idx < TILE; idx += 64 * waves) {
-        zeros[idx] = zero_u4();
+        const uint32_t one = idx % 32 == 1 ? 0x3f803f80u : 0u;
+        constants[idx] = make_uint4(one, one, one, one);
     }
     if (tid == 0) {
         *first_masked = (uint32_t)NB;
@@ -73,11 +74,11 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         const int i = idx / keys, key = idx % keys, b = row_of(i);
         const int64_t pos = (int64_t)b * S + min(key, S - 1);
         const uint4 kv = *reinterpret_cast<const uint4 *>(p.k + pos * p.k_ss + h * D);
-        const int slot = (key >> 5) * TILE + i * 32 + key_slot(key & 31);
-        ks[slot] = key < S ? kv : zero_u4();
-        const float mv = key < S ? to_f32(p.bias[(int64_t)b * p.bias_sb + key]) * LOG2E : -INFINITY;
-        words[slot] = mask_word(mv);
-        if (mv != 0.f) {
+        const int tile_row = (key >> 5) * TILE + i * 32;
+        ks[tile_row + key_slot(key & 31)] = key < S ? kv : zero_u4();
+        const float mask = key < S ? to_f32(p.bias[(int64_t)b * p.bias_sb + key]) * LOG2E : 0.f;
+        masks[tile_row + (key & 31)] = mask;
+        if (mask != 0.f) {
             atomicMin(first_masked, (uint32_t)(key >> 5));
         }
     }
@@ -87,112 +88,144 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         if (key < S) {
             vv = load8_checked(p.v + (int64_t)(h * D + d) * p.v_se + (int64_t)row_of(i) * S, key, S);
         }
-        vs[(kp >> 2) * TILE + i * 32 + ((kp & 1) * 2 + ((kp >> 1) & 1)) * 8 + d] = vv;
+        vs[(kp >> 2) * TILE + i * 32 + (kp & 3) * 8 + d] = vv;
     }
     __syncthreads();
     const int masked_from = (int)*first_masked;
 
-    const int r = lane & 31, g = lane >> 5;
-    const uint32_t lower = lane < 32 ? 0xffffffffu : 0u;
-    const bf16x8 onesf = as_bf16x8(make_uint4(0x3f803f80u & lower, 0u, 0u, 0u)), ones_rows = rowsum_selector(lane);
-    // V operand of the 16x16x32 MFMA: lane (row i, chunk c) of the 64; rows 0-7 are the values for queries n, which chunks 0
-    // and 2 of the probabilities belong to, rows 8-15 those for queries n + 16 (chunks 1 and 3); elsewhere zeros
-    const int vi = lane & 15, vc = lane >> 4;
-    const bool v_real = (vi >> 3) == (vc & 1);
-    const uint32_t v_first = v_real ? 8u * (vc >> 1) + (vi & 7) : (uint32_t)(zeros - vs), v_tile = v_real ? (uint32_t)TILE : 0u;
+    // Operands of the 16x16x32 MFMA: lane (row or column n, chunk c of eight k-slots).
+    //   logits: rows are sixteen keys, columns sixteen queries; chunks 0, 1, 2 hold the same keys against the three parts of the
+    //           queries, chunk 3 nothing (zeros in the queries);
+    //   p.v:    rows 0-7 are the values, row 8 ones (the row sums), the rest zeros; the k-slots of chunk c are keys 8 c .. 8 c + 7.
+    const int n = lane & 15, c = lane >> 4;
+    const uint32_t v_first = n < D ? 8u * c + n : (uint32_t)(constants - vs) + (n == D ? 1u : 0u), v_tile = n < D ? (uint32_t)TILE : 0u;
+    auto product = [](bf16x8 a, bf16x8 b, f32x4 x) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, x, 0, 0, 0); };
 
     for (int j = split * waves + wave; j < NB; j += waves * p.splits) {
         int lv = lane; // opaque: the addresses of a query block's rows are formed where they are used, not kept over the keys
         asm volatile("" : "+v"(lv));
-        const int query = min(32 * j + (lv & 31), S - 1);
-        bf16x8 q[ROWS];
+        bf16x8 q[ROWS][2]; // queries 32 j + 16 u + n
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
-            const bf16x8 raw = *reinterpret_cast<const bf16x8 *>(p.q + ((int64_t)row_of(i) * S + query) * p.q_ss + h * D);
 #pragma unroll
-            for (int e = 0; e < D; ++e) {
-                const float x = to_f32(raw[e]) * p.scale2;
-                const bf16_t hi = (bf16_t)x;
-                q[i][e] = g == 0 ? hi : (bf16_t)(x - to_f32(hi));
+            for (int u = 0; u < 2; ++u) {
+                // a lane splits dims 2 c and 2 c + 1 of its query, then the four lanes of the query exchange: parts for dims
+                const int query = min(32 * j + 16 * u + (lv & 15), S - 1);
+                const uint32_t raw = *reinterpret_cast<const uint32_t *>(p.q + ((int64_t)row_of(i) * S + query) * p.q_ss + h * D + 2 * (lv >> 4));
+                uint32_t part[4] = {0u, 0u, 0u, 0u};
+                float x0 = __uint_as_float(raw << 16) * p.scale2, x1 = __uint_as_float(raw & 0xffff0000u) * p.scale2;
+#pragma unroll
+                for (int w = 0; w < 3; ++w) {
+                    part[w] = __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u); // the upper halves
+                    x0 -= __uint_as_float(__float_as_uint(x0) & 0xffff0000u), x1 -= __uint_as_float(__float_as_uint(x1) & 0xffff0000u);
+                }
+                q[i][u] = as_bf16x8(transpose4x4_lanes(part));
             }
         }
         const bf16_t *nb_head = HAS_NB ? p.nb + (int64_t)h * p.nb_sh : nullptr;
-        const uint32_t nb_row = HAS_NB ? (uint32_t)query * (uint32_t)p.nb_sq : 0u; // elements, within 2^30 (the launcher checks)
+        uint32_t nb_row[2] = {0u, 0u}; // elements, within 2^30 (the launcher checks)
+#pragma unroll
+        for (int u = 0; HAS_NB && u < 2; ++u) {
+            nb_row[u] = (uint32_t)min(32 * j + 16 * u + (lv & 15), S - 1) * (uint32_t)p.nb_sq;
+        }
         struct Raw {
-            uint4 lo, hi; // 16 consecutive keys of this lane's query
+            uint4 r[2]; // keys 8 c .. 8 c + 7 of this lane's two queries
         };
         auto load_nb = [&](int t) {
             Raw w = {zero_u4(), zero_u4()};
             if constexpr (HAS_NB) {
-                const int key = 32 * min(t, NB - 1) + 16 * g;
-                if (32 * t + 32 <= S) {
-                    w.lo = load8_any(nb_head, nb_row + key), w.hi = load8_any(nb_head, nb_row + key + 8);
-                } else {
-                    w.lo = load8_checked(nb_head + nb_row, key, S), w.hi = load8_checked(nb_head + nb_row, key + 8, S);
+                const int key = 32 * min(t, NB - 1) + 8 * c;
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    w.r[u] = 32 * t + 32 <= S ? load8_any(nb_head, nb_row[u] + key) : load8_checked(nb_head + nb_row[u], key, S);
                 }
             }
             return w;
         };
-        auto convert_nb = [&](const Raw &w) {
-            f32x16 c = zero16();
-            if constexpr (HAS_NB) {
-                const bf16x8 lo = as_bf16x8(w.lo), hi = as_bf16x8(w.hi);
+        struct Tile {
+            f32x4 x[2][2]; // [query half][key half]
+        };
+        auto seeds = [&](const Raw &w, int t) { // of the four rows' logits: the pair bias, -inf past the last key
+            Tile s;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const bf16x8 raw = as_bf16x8(w.r[u]);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    c[e] = to_f32(lo[e]) * LOG2E, c[8 + e] = to_f32(hi[e]) * LOG2E;
+                    s.x[u][e >> 2][e & 3] = HAS_NB ? to_f32(raw[e]) * LOG2E : 0.f;
                 }
             }
-            return c;
+            if (32 * t + 32 > S) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    if (32 * t + 8 * c + e >= S) {
+                        s.x[0][e >> 2][e & 3] = s.x[1][e >> 2][e & 3] = -INFINITY;
+                    }
+                }
+            }
+            return s;
         };
-        auto logits = [&](int i, int t, const f32x16 &C) { // of row i, tile t, without the mask
-            return mfma(as_bf16x8(ks[t * TILE + i * 32 + r]), q[i], C);
+        auto logits = [&](int i, int t, const Tile &C, auto masked) { // of row i, tile t
+            Tile l;
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                const bf16x8 k = as_bf16x8(ks[t * TILE + i * 32 + a * 16 + n]);
+                f32x4 c0 = C.x[0][a], c1 = C.x[1][a];
+                if constexpr (decltype(masked)::value) {
+                    const f32x4 m = *reinterpret_cast<const f32x4 *>(masks + t * TILE + i * 32 + 8 * c + 4 * a);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        c0[e] += m[e], c1[e] += m[e];
+                    }
+                }
+                l.x[0][a] = product(k, q[i][0], c0);
+                l.x[1][a] = product(k, q[i][1], c1);
+            }
+            return l;
         };
-        auto add_mask = [&](int i, int t, f32x16 x) {
-            return mfma(as_bf16x8(make_uint4(words[t * TILE + i * 32 + r] & lower, 0u, 0u, 0u)), onesf, x);
-        };
-        f32x4 o[ROWS], sums[ROWS];
+        // rows 0-7: the values' sums, in lanes of chunks 0 and 1; row 8: the sums of the probabilities, in lanes of chunk 2
+        f32x4 o[ROWS][2];
+        auto clear = [&](int i) { o[i][0] = o[i][1] = f32x4{0.f, 0.f, 0.f, 0.f}; };
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
-            o[i] = sums[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            clear(i);
         }
-        auto values = [&](int i, int t, int s) { return as_bf16x8(vs[v_first + t * v_tile + i * 32 + s * 16]); };
-        auto finish = [&](int i, int t, f32x16 &x, float shift, auto shifted) { // softmax and p.v of row i, tile t
+        auto finish = [&](int i, int t, const Tile &l, const float (&shift)[2], auto shifted) { // softmax and p.v of row i, tile t
+            const bf16x8 v = as_bf16x8(vs[v_first + t * v_tile + i * 32]);
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                x[e] = __builtin_amdgcn_exp2f(decltype(shifted)::value ? x[e] - shift : x[e]);
+            for (int u = 0; u < 2; ++u) {
+                bf16x8 pr;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float x = l.x[u][e >> 2][e & 3];
+                    pr[e] = (bf16_t)__builtin_amdgcn_exp2f(decltype(shifted)::value ? x - shift[u] : x);
+                }
+                o[i][u] = product(v, pr, o[i][u]);
             }
-            const bf16x8 p0 = pack8(x, 0), p1 = pack8(x, 8);
-            o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(values(i, t, 0), p0, o[i], 0, 0, 0);
-            sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p0, sums[i], 0, 0, 0);
-            o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(values(i, t, 1), p1, o[i], 0, 0, 0);
-            sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p1, sums[i], 0, 0, 0);
         };
+        const float unshifted[2] = {0.f, 0.f};
         Raw raw = load_nb(0);
         for (int t = 0; t < NB; ++t) {
-            const f32x16 C = convert_nb(raw);
+            const Tile C = seeds(raw, t);
             if (t + 1 < NB) {
                 raw = load_nb(t + 1);
             }
             // Two rows in flight: the logits of one are in the matrix pipe while the other's exponentials run.  The fences keep
-            // it at two: left to itself the compiler starts all four and needs 235 registers, two waves per SIMD.
+            // it at two: left to itself the compiler starts all four and needs registers for two waves per SIMD only.
             auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
             auto rows = [&](auto masked) {
-                auto next = [&](int i) {
-                    const f32x16 x = logits(i, t, C);
-                    return decltype(masked)::value ? add_mask(i, t, x) : x;
-                };
-                f32x16 xa = next(0);
+                Tile xa = logits(0, t, C, masked);
                 fence();
-                f32x16 xb = next(1);
-                finish(0, t, xa, 0.f, std::false_type{});
+                Tile xb = logits(1, t, C, masked);
+                finish(0, t, xa, unshifted, std::false_type{});
                 fence();
-                xa = next(2);
-                finish(1, t, xb, 0.f, std::false_type{});
+                xa = logits(2, t, C, masked);
+                finish(1, t, xb, unshifted, std::false_type{});
                 fence();
-                xb = next(3);
-                finish(2, t, xa, 0.f, std::false_type{});
+                xb = logits(3, t, C, masked);
+                finish(2, t, xa, unshifted, std::false_type{});
                 fence();
-                finish(3, t, xb, 0.f, std::false_type{});
+                finish(3, t, xb, unshifted, std::false_type{});
                 fence();
             };
             if (t < masked_from) {
@@ -203,41 +236,55 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         }
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
-            float l = rowsum_fetch(sums[i], lane);
+            // the two query halves side by side: lane l then has values 4 (l / 16 % 2) .. + 3 of query 16 (l / 32) + l % 16
+            int le = lane;
+            asm volatile("" : "+v"(le));
+            f32x4 values;
+            float l;
+            auto collect = [&] {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[i][0][e]), __float_as_uint(o[i][1][e]), false, false);
+                    values[e] = __uint_as_float(sw[0]);
+                    if (e == 0) {
+                        l = __shfl(__uint_as_float(sw[1]), le & 47, 64);
+                    }
+                }
+            };
+            collect();
             if (__any(!(l > 1e-30f && l < 1e30f))) {
                 // Some probability overflowed or a whole row underflowed (every key masked: -1e9 log2(e) everywhere, which is
                 // finite): the row's true maxima first, then the probabilities with them subtracted.
-                float mx = -INFINITY;
+                float mx[2] = {-INFINITY, -INFINITY};
                 for (int t = 0; t < NB; ++t) {
-                    const f32x16 x = add_mask(i, t, logits(i, t, convert_nb(load_nb(t))));
+                    const Tile x = logits(i, t, seeds(load_nb(t), t), std::true_type{});
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
-                        mx = fmaxf(mx, x[e]);
+                        mx[e >> 3] = fmaxf(mx[e >> 3], x.x[e >> 3][(e >> 2) & 1][e & 3]);
                     }
                 }
-                mx = half_swap_max(mx);
-                mx = mx == -INFINITY ? 0.f : mx;
-                o[i] = sums[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-                for (int t = 0; t < NB; ++t) {
-                    f32x16 x = add_mask(i, t, logits(i, t, convert_nb(load_nb(t))));
-                    finish(i, t, x, mx, std::true_type{});
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    mx[u] = half_swap_max(mx[u]);
+                    mx[u] = fmaxf(mx[u], __shfl_xor(mx[u], 16, 64));
+                    mx[u] = mx[u] == -INFINITY ? 0.f : mx[u];
                 }
-                l = rowsum_fetch(sums[i], lane);
+                clear(i);
+                for (int t = 0; t < NB; ++t) {
+                    finish(i, t, logits(i, t, seeds(load_nb(t), t), std::true_type{}), mx, std::true_type{});
+                }
+                collect();
             }
-            // o: lane (column n, group c) holds values 4 (c & 1) .. + 3 of query n + 16 (c >> 1); its sum lies in the lane of
-            // that query
-            int le = lane;
-            asm volatile("" : "+v"(le));
-            const int qi = (le & 15) + 16 * (le >> 5), pos = 32 * j + qi, d0 = 4 * ((le >> 4) & 1);
-            const float inv = 1.0f / __shfl(l, qi, 64);
+            const int pos = 32 * j + 16 * (le >> 5) + (le & 15), d0 = 4 * ((le >> 4) & 1);
+            const float inv = 1.0f / l;
             if (pos < S && b0 + i < p.B) {
                 const int64_t row = (int64_t)(b0 + i) * S + pos;
                 const bf16x4 gv = *reinterpret_cast<const bf16x4 *>(p.gate + row * p.g_ss + h * D + d0);
                 bf16x4 ov;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const float wavg = to_f32((bf16_t)(o[i][c] * inv));
-                    ov[c] = (bf16_t)(wavg * sigmoid_f32(to_f32(gv[c])));
+                for (int e = 0; e < 4; ++e) {
+                    const float wavg = to_f32((bf16_t)(values[e] * inv));
+                    ov[e] = (bf16_t)(wavg * sigmoid_f32(to_f32(gv[e])));
                 }
                 *reinterpret_cast<bf16x4 *>(p.avg + row * p.a_ss + h * D + d0) = ov;
             }

@@ -82,3 +82,39 @@ def test_gate_of_long_rows_keeps_32_bits(torch_cuda, heads):
     want = v.double() * torch.sigmoid(gate.double())
     err = float(((act.double() - want).abs() / want).max())
     assert err < 2.0 ** -8 * (1 + 2.0 ** -7), err  # 2^-15: what 32-bit sums, sigmoid and quotient add, and to spare
+
+
+def run_heads_of_eight(w):
+    print(w.name, flush=True)
+    ten, scratch = helpers.to_device(w)
+    assert helpers.run_hip(w, ten, scratch) == 0 and capi.last_path() == "tiled_mfma"
+    err = relative_error(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), gated_average_f64(w))
+    # q, k, v, probabilities, gate, weighted average and result are rounded
+    assert err < 1.25 * 7 ** 0.5 * BF16_RMS, err
+
+
+@pytest.mark.parametrize("S", [33, 128, 301])
+def test_queries_of_heads_of_eight_keep_32_bits(torch_cuda, S):
+    """The first channel of every query is 127, that of the keys a whole number below 256: logits of up to 11 000, which the pair bias and
+    the mask together take back to within 0.1, leaving those of the other seven channels.  127 log2(e) / sqrt(8) in 16 bits is off
+    by enough to move a probability by up to 8 %."""
+    w = draw_workload(700 + S, 5, S, 8, 8, masked=0.0)
+    c = np.random.Generator(np.random.PCG64(S)).integers(1, 256, S).astype(np.float32)
+    for m in (w.wq, w.wk, w.wv, w.wg):
+        m[:, :2] = 0.0
+    w.wq[::8], w.wk[::8] = 0.0, 0.0
+    w.wq[::8, 0], w.wk[::8, 1] = 1.0, 1.0
+    w.x[:, :, 0], w.x[:, :, 1] = 127.0, c
+    logit = 127.0 * c.astype(np.float64) / 8.0 ** 0.5
+    nb = round_to_bf16(-logit.astype(np.float32))
+    w.nb[:], w.bias[:] = nb, round_to_bf16((-logit - nb).astype(np.float32))
+    run_heads_of_eight(w)
+
+
+@pytest.mark.parametrize("S", [33, 128, 301])
+def test_masks_of_heads_of_eight_keep_32_bits(torch_cuda, S):
+    """Mask biases of up to 4000 on all keys, one set for all rows, which the pair bias takes back: the softmax of the logits alone."""
+    w = draw_workload(800 + S, 5, S, 8, 8, masked=0.0)
+    w.bias[:] = round_to_bf16(np.random.Generator(np.random.PCG64(S)).uniform(-4000.0, 4000.0, S).astype(np.float32))
+    w.nb[:] = -w.bias[0]
+    run_heads_of_eight(w)
