@@ -408,7 +408,7 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
             const float nch = (float)C;
             const float mean = s1 / nch + x0;
             const float var = fmaxf((s2 - s1 * s1 / nch) / nch, 0.f);
-            const float rstd = __builtin_amdgcn_rsqf(var + eps);
+            const float rstd = 1.0f / sqrtf(var + eps);
             const float shift = -rstd * mean;
 #pragma unroll
             for (int t = 0; t < 2; ++t) {

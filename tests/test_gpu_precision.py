@@ -118,3 +118,26 @@ def test_masks_of_heads_of_eight_keep_32_bits(torch_cuda, S):
     w.bias[:] = round_to_bf16(np.random.Generator(np.random.PCG64(S)).uniform(-4000.0, 4000.0, S).astype(np.float32))
     w.nb[:] = -w.bias[0]
     run_heads_of_eight(w)
+
+
+def test_centre_layernorm_of_the_triangle_multiplication_is_exact_to_32_bits(torch_cuda):
+    """One residue whose normalised row is the input LayerNorm's beta, small whole numbers, as are then the left projections and, with
+    ones to the right, the centre: its sums are exact, and gamma = 2^20 with beta = -2^20 t, t the centre normalised in 32 bits
+    with a correctly rounded square root and quotient, leaves zeros, where one bit more or less would leave 1/16."""
+    torch = torch_cuda
+    C, f = 128, np.float32
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda")  # noqa: E731
+    vec = lambda value: torch.full((C,), float(value), device="cuda")  # noqa: E731
+    eye, zeros = torch.eye(C, device="cuda").to(torch.bfloat16), torch.zeros(C, C, device="cuda", dtype=torch.bfloat16)
+    for seed in range(24):
+        row = np.random.Generator(np.random.PCG64(seed)).integers(-9, 10, C).astype(f)
+        mean, var = f(row.mean(dtype=np.float64)), f(row.var(dtype=np.float64))
+        rstd = f(1) / np.sqrt(var + f(1e-5))
+        t = (row.astype(np.float64) * rstd + (-rstd * mean)).astype(f)
+        w = dict(ln_in_gamma=vec(0), ln_in_beta=dev(row), ln_center_gamma=vec(2.0 ** 20), ln_center_beta=dev(-t * f(2.0 ** 20)),
+                 left_proj_w=eye, left_proj_b=vec(0), right_proj_w=zeros, right_proj_b=vec(1), output_w=eye, output_b=vec(0),
+                 left_gate_w=zeros, right_gate_w=zeros, gating_w=zeros, left_gate_b=vec(100), right_gate_b=vec(100), gating_b=vec(100))
+        act = torch.zeros(1, 1, C, device="cuda", dtype=torch.bfloat16)
+        assert capi.TriangleMultiplicationBlock(act, torch.ones(1, 1, device="cuda", dtype=torch.bfloat16), w, False).run() == 0
+        torch.cuda.synchronize()
+        assert not bool(act.any()), (seed, float(act.abs().max()))
