@@ -134,12 +134,12 @@ int pair_bias_tiles(const kutacc_hip_attention_args_t &args, void *tiles, hipStr
 
 // streamed_attention.hip: rows of any length, 128 or 256 channels in heads of 32, on a workspace of streamed_workspace_bytes()
 // (256-byte aligned) that starts with the tiles of the pair bias; opt.nb_tiles_ready: they lie there already.  args.q, k, v
-// and gate are not used, weights and biases may lie on any address; the result is added to args.out (opt.out_mode FUSED_OUT_ADD or FUSED_OUT_ADD_TRANSPOSED), by way of
-// `spare`, [batch * seq_len, channels], where the projection cannot do that itself.
+// and gate are not used, weights and biases may lie on any address; the result is added to args.out (opt.out_mode FUSED_OUT_ADD or
+// FUSED_OUT_ADD_TRANSPOSED).
 bool streamed_attention_supports(const kutacc_hip_attention_args_t &args);
 int64_t streamed_workspace_bytes(int64_t batch, int64_t seq_len, int64_t nheads, bool pair_bias);
 int gating_attention_streamed(const kutacc_hip_attention_args_t &args, const FusedAttentionOptions &opt, void *workspace, int64_t bytes,
-                              void *spare, hipStream_t stream);
+                              hipStream_t stream);
 bool streamed_attention_forced(); // the "streamed" hook: blocks of every size on these kernels
 int streamed_attention_tuning(const char *name, const char *value);
 

@@ -561,7 +561,7 @@ bool streamed_attention_supports(const kutacc_hip_attention_args_t &a)
 }
 
 int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedAttentionOptions &opt, void *workspace, int64_t bytes,
-                              void *spare, hipStream_t stream)
+                              hipStream_t stream)
 {
     const int64_t C = a.nheads * a.head_size, S = a.seq_len;
     const bool has_nb = a.nonbatched_bias != nullptr;
@@ -598,7 +598,8 @@ int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedA
         return rc;
     }
     // The projection adds its result to the activation on the way out (2048 residues: 411 us and 674 us of residual pass
-    // before, 664 us together now); an activation it cannot address so (not 16-byte aligned) is added to afterwards.
+    // before, 664 us together now).  Where it cannot (the activation, the output weights or bias not on 16 bytes), it leaves its result
+    // where q was, which no kernel reads any more, and a pass of its own adds it.
     const int64_t M = a.batch * S;
     const bool transposed = opt.out_mode == FUSED_OUT_ADD_TRANSPOSED;
     if (row_projection_supports(a.avg, a.avg_stride_s, a.output_w, a.output_b, a.out, a.out_ld, M, C, C)) {
@@ -609,9 +610,9 @@ int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedA
     kutacc_hip_gemm_args_t g = {};
     g.m = M, g.n = g.k = C, g.batches = 1, g.dtype = KUTACC_DTYPE_BF16, g.path = KUTACC_HIP_PATH_AUTO;
     g.a = a.avg, g.a_stride_m = a.avg_stride_s, g.a_stride_k = 1, g.b = a.output_w, g.b_stride_n = C, g.b_stride_k = 1;
-    g.c = spare, g.c_stride_m = C, g.bias = a.output_b, g.bias_axis = 1;
+    g.c = p.q, g.c_stride_m = C, g.bias = a.output_b, g.bias_axis = 1;
     rc = pair_gemm(g, stream);
-    return rc != 0 ? rc : residual_add(a.out, spare, transposed ? S : a.batch, transposed ? a.batch : S, C, transposed, KUTACC_DTYPE_BF16, stream);
+    return rc != 0 ? rc : residual_add(a.out, p.q, transposed ? S : a.batch, transposed ? a.batch : S, C, transposed, KUTACC_DTYPE_BF16, stream);
 }
 
 } // namespace kutacc_launch
