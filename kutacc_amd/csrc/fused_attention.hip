@@ -2911,6 +2911,7 @@ int row_projection_residual(const void *a, int64_t a_ld, const void *w, const fl
     if (!row_projection_supports(a, a_ld, w, bias, acc, acc_ld, m, n, k)) {
         return KUTACC_HIP_EUNSUPPORTED;
     }
+    kutacc_prof::KernelTimer t("output_projection_kernel<residual>", 2.0 * (double)m * (double)n * (double)k, stream);
     return k == 128 ? launch_output_projection<128, EPILOGUE_RESIDUAL>(a, a_ld, w, bias, acc, acc_ld, m, n, stream, nullptr, 0, swap_n)
                     : launch_output_projection<256, EPILOGUE_RESIDUAL>(a, a_ld, w, bias, acc, acc_ld, m, n, stream, nullptr, 0, swap_n);
 }

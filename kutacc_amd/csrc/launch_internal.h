@@ -153,7 +153,7 @@ bool row_projection_supports(const void *a, int64_t a_ld, const void *w, const f
 int row_projection(const void *a, int64_t a_ld, const void *w, const float *bias, void *out, int64_t out_ld, int64_t m,
                    int64_t n, int64_t k, hipStream_t stream);
 
-// acc += the product's rows, row (i, j) of their [m / swap_n, swap_n] grid to row (j, i) of acc where swap_n is not zero (not timed)
+// acc += the product's rows, row (i, j) of their [m / swap_n, swap_n] grid to row (j, i) of acc where swap_n is not zero
 int row_projection_residual(const void *a, int64_t a_ld, const void *w, const float *bias, void *acc, int64_t acc_ld, int64_t m,
                             int64_t n, int64_t k, int64_t swap_n, hipStream_t stream);
 int row_projection_gated_residual(const void *a, int64_t a_ld, const void *w, const float *bias, const void *gate,

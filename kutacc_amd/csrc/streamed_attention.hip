@@ -517,8 +517,7 @@ int launch_attention(StreamedParams p, hipStream_t stream)
     p.pair_groups = (pairs + p.group_rows - 1) / p.group_rows;
     p.groups = p.pair_groups * p.H * parts;
     const int64_t blocks = (int64_t)(p.groups + 7) / 8 * 8 * p.group_rows * together;
-    // the name this stage has in the profile of a block beyond 1024 keys, whichever kernel serves it
-    kutacc_prof::KernelTimer t("attention_tiles_kernel", 4.0 * (double)p.B * p.S * p.S * p.H * HEAD, stream);
+    kutacc_prof::KernelTimer t("streamed_attention_kernel", 4.0 * (double)p.B * p.S * p.S * p.H * HEAD, stream);
     streamed_attention_kernel<HAS_NB><<<dim3((unsigned)blocks), 64 * WAVES, lds_bytes, stream>>>(p);
     return kutacc_hip_status(hipGetLastError());
 }
@@ -603,8 +602,6 @@ int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedA
     const int64_t M = a.batch * S;
     const bool transposed = opt.out_mode == FUSED_OUT_ADD_TRANSPOSED;
     if (row_projection_supports(a.avg, a.avg_stride_s, a.output_w, a.output_b, a.out, a.out_ld, M, C, C)) {
-        // (again the stage's name in the profile, whichever kernel serves it)
-        kutacc_prof::KernelTimer t("residual_add_kernel", 2.0 * (double)M * C * C, stream);
         return row_projection_residual(a.avg, a.avg_stride_s, a.output_w, a.output_b, a.out, a.out_ld, M, C, C, transposed ? S : 0, stream);
     }
     kutacc_hip_gemm_args_t g = {};

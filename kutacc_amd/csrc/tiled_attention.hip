@@ -607,8 +607,10 @@ int gating_attention_tiled(const kutacc_hip_attention_args_t &a, hipStream_t str
         return rc;
     }
     if (small_head_attention_supports(a)) {
-        kutacc_prof::KernelTimer t("attention_tiles_kernel", 4.0 * (double)B * (double)S * (double)S * (double)C, stream);
-        rc = small_head_attention(a, stream);
+        {
+            kutacc_prof::KernelTimer t("small_head_attention_kernel", 4.0 * (double)B * (double)S * (double)S * (double)C, stream);
+            rc = small_head_attention(a, stream);
+        }
         return rc != 0 ? rc : project(a.avg, a.avg_stride_s, M, a.output_w, C, C, C, a.out, a.out_ld, a.output_b, stream);
     }
     TileParams p;

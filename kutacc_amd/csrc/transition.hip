@@ -479,9 +479,13 @@ hipError_t launch_split(const TransitionParams &p, hipStream_t stream)
 template <bool BLOCK>
 hipError_t launch(const TransitionParams &p, int64_t c_o, hipStream_t stream)
 {
+    const double flops = 4.0 * (double)p.rows * (double)c_o * (double)p.c_i;
     // The split kernel while its workgroups of 32 rows fit one round on the chip: in a second round it takes as long as the
     // other kernel (12000 rows, 256 -> 1024: 39 and 38 us; 128 -> 512: 18 and 14).  With 64 channels all is within 7 us.
-    const bool few = (p.rows + 31) / 32 <= kutacc_cu_count();
+    const bool few = c_o != 64 && (p.rows + 31) / 32 <= kutacc_cu_count();
+    kutacc_prof::KernelTimer t(few ? (BLOCK ? "transition_split_kernel<block>" : "transition_split_kernel")
+                                   : (BLOCK ? "transition_rows_kernel<block>" : "transition_rows_kernel"),
+                               flops, stream);
     if (c_o == 256) {
         return few ? launch_split<256, BLOCK, 4>(p, stream) : launch_rows<256, BLOCK, 32, 2, 4, 2>(p, stream);
     }
@@ -515,7 +519,6 @@ int transition_fused(const void *x, const void *w1, const float *b1, const void 
     if (!transition_fused_supports(rows, c_o, c_i, x, w1, b1, w2, b2, out)) {
         return KUTACC_HIP_EUNSUPPORTED;
     }
-    kutacc_prof::KernelTimer t("transition_fused_kernel", 4.0 * (double)rows * (double)c_o * (double)c_i, stream);
     const TransitionParams p = {(const bf16_t *)x, (const bf16_t *)w1, (const bf16_t *)w2, b1, b2, nullptr, nullptr, (bf16_t *)out, rows, (int)c_i, 0.f};
     return kutacc_hip_status(launch<false>(p, c_o, stream));
 }
@@ -528,7 +531,6 @@ int transition_block_fused(void *act, const float *ln_gamma, const float *ln_bet
     if (!ln_gamma || !ln_beta || (c_o != 64 && c_o != 128 && c_o != 256) || !operands_fit(rows, c_i, act, w1, b1, w2, b2, act)) {
         return KUTACC_HIP_EUNSUPPORTED;
     }
-    kutacc_prof::KernelTimer t("transition_fused_kernel<block>", 4.0 * (double)rows * (double)c_o * (double)c_i, stream);
     const TransitionParams p = {(const bf16_t *)act, (const bf16_t *)w1, (const bf16_t *)w2, b1, b2, ln_gamma, ln_beta, (bf16_t *)act, rows, (int)c_i, ln_eps};
     return kutacc_hip_status(launch<true>(p, c_o, stream));
 }

@@ -497,7 +497,7 @@ int triangle_front(const kutacc_hip_triangle_multiplication_args_t &a, void *lef
     if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&triangle_front_kernel), FRONT_LDS, configured)) {
         return kutacc_hip_status(e);
     }
-    kutacc_prof::KernelTimer t("gated_projection_blocks_kernel<2>", 8.0 * (double)(a.n_res * a.n_res) * C * C, stream);
+    kutacc_prof::KernelTimer t("triangle_front_kernel", 8.0 * (double)(a.n_res * a.n_res) * C * C, stream);
     const Split s = split_steps(rows, np, kutacc_cu_count());
     const Side l = {(const bf16_t *)a.left_proj_w, (const bf16_t *)a.left_gate_w, a.left_proj_b, a.left_gate_b, (bf16_t *)left};
     const Side r = {(const bf16_t *)a.right_proj_w, (const bf16_t *)a.right_gate_w, a.right_proj_b, a.right_gate_b, (bf16_t *)right};

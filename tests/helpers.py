@@ -90,6 +90,24 @@ def oracle_out(w: Workload, return_avg=False):
                                        return_avg=return_avg)
 
 
+def profiled_kernels(torch, fn):
+    """Names of the kernels the library timed while fn ran."""
+    lib = capi.lib()
+    lib.kutacc_hip_profile_enable(1)
+    try:
+        fn()
+        torch.cuda.synchronize()
+        names, i = [], 0
+        name = ctypes.create_string_buffer(128)
+        ms, cnt, fl = ctypes.c_double(), ctypes.c_int64(), ctypes.c_double()
+        while lib.kutacc_hip_profile_read(i, name, 128, ctypes.byref(ms), ctypes.byref(cnt), ctypes.byref(fl)) == 0:
+            names.append(name.value.decode())
+            i += 1
+        return names
+    finally:
+        lib.kutacc_hip_profile_enable(0)
+
+
 def check_close(got, ref, dtype: str, what=""):
     """The parity bar: fp32 path within 1e-4 relative (plus 1e-5 absolute floor); bf16 path within
     2e-2 absolute + 1e-2 relative of the fp32 oracle."""

@@ -164,23 +164,7 @@ def test_triangle_attention_block_against_the_oracle(torch_cuda, layernorm_place
     helpers.check_close(helpers.to_numpy(got), block_oracle(c, ending), "bf16", f"block n={n} ending={ending}")
 
 
-def profiled_kernels(torch, fn):
-    """Names of the kernels the library timed while fn ran."""
-    import ctypes
-    lib = capi.lib()
-    lib.kutacc_hip_profile_enable(1)
-    try:
-        fn()
-        torch.cuda.synchronize()
-        names, i = [], 0
-        name = ctypes.create_string_buffer(128)
-        ms, cnt, fl = ctypes.c_double(), ctypes.c_int64(), ctypes.c_double()
-        while lib.kutacc_hip_profile_read(i, name, 128, ctypes.byref(ms), ctypes.byref(cnt), ctypes.byref(fl)) == 0:
-            names.append(name.value.decode())
-            i += 1
-        return names
-    finally:
-        lib.kutacc_hip_profile_enable(0)
+profiled_kernels = helpers.profiled_kernels
 
 
 @pytest.mark.parametrize("ending", [False, True], ids=["starting node", "ending node"])
@@ -329,8 +313,8 @@ def test_odd_numbers_of_rows_per_workgroup_take_the_single_row_kernel(torch_cuda
 
 
 def test_triangle_attention_block_beyond_1024_residues(torch_cuda):
-    """1088 residues: past the fused head kernels' longest row, the block runs the same chain as separate passes with the
-    operator on the tiled MFMA route.  Both orientations against the oracle on a sample of attention rows."""
+    """1088 residues: past the fused head kernels' longest row, the block runs the same chain with the attention that keeps q, k, v
+    and gate in memory.  Both orientations against the oracle on a sample of attention rows."""
     torch = torch_cuda
     n = 1088
     c = block_case(9100, n, 4)
@@ -340,7 +324,7 @@ def test_triangle_attention_block_beyond_1024_residues(torch_cuda):
         res = {}
         names = profiled_kernels(torch, lambda: res.setdefault("z", run_block(torch, c, ending)))
         got = res["z"]
-        assert "attention_tiles_kernel" in names and "residual_add_kernel" in names, names
+        assert "streamed_attention_kernel" in names and "output_projection_kernel<residual>" in names, names
         assert bool(torch.isfinite(got).all())
         want = block_oracle_rows(c, ending, rows)
         sample = got[:, rows].transpose(0, 1) if ending else got[rows]
@@ -645,7 +629,7 @@ def test_triangle_multiplication_block_on_each_gated_projection_kernel(torch_cud
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
         device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
     w = {k: dev(v) for k, v in case.items() if k not in ("z", "mask")}
-    want = {None: "gated_projection_blocks_kernel<2>", "streaming": "gated_projection_kernel<2>", "tiled": "pair_gemm_kernel<gated>"}
+    want = {None: "triangle_front_kernel", "streaming": "gated_projection_kernel<2>", "tiled": "pair_gemm_kernel<gated>"}
     res = {}
     for mode in want:
         assert capi.set_tuning("gated_projection", mode) == 0
@@ -787,9 +771,13 @@ def test_transition_block_at_the_edges_of_its_kernels(torch_cuda, rows, c_o, c_i
     L = capi.lib()
     nbytes = L.kutacc_hip_transition_block_workspace(rows, c_o, c_i)
     ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device="cuda")
-    assert L.kutacc_hip_transition_block(act.data_ptr(), gamma.data_ptr(), beta.data_ptr(), 1e-5, w1.data_ptr(), b1.data_ptr(),
-                                         w2.data_ptr(), b2.data_ptr(), ws.data_ptr(), nbytes, rows, c_o, c_i, capi.K_BF16, None) == 0
-    torch.cuda.synchronize()
+    res = {}
+    names = profiled_kernels(torch, lambda: res.setdefault("rc", L.kutacc_hip_transition_block(
+        act.data_ptr(), gamma.data_ptr(), beta.data_ptr(), 1e-5, w1.data_ptr(), b1.data_ptr(), w2.data_ptr(), b2.data_ptr(), ws.data_ptr(),
+        nbytes, rows, c_o, c_i, capi.K_BF16, None)))
+    assert res["rc"] == 0
+    few = c_o != 64 and (rows + 31) // 32 <= torch.cuda.get_device_properties(0).multi_processor_count
+    assert names == ["transition_split_kernel<block>" if few else "transition_rows_kernel<block>"], names
     helpers.check_close(num(act), want, "bf16", f"transition block {rows}x{c_o}->{c_i}")
 
 
@@ -941,8 +929,8 @@ def test_pair_stack_blocks_replay_from_a_hip_graph(torch_cuda):
 @pytest.mark.parametrize("column,n_seq,n_res,heads", [(True, 1088, 24, 8), (False, 20, 1040, 8), (False, 24, 56, 3), (True, 40, 24, 5)])
 def test_msa_attention_blocks_on_the_tiled_route(torch_cuda, column, n_seq, n_res, heads):
     """Attention rows of more than 1024 keys (column-wise over 1088 sequences, row-wise over 1040 residues) and channel
-    counts other than 128 and 256: the block's separate passes with the operator on the tiled MFMA route, whole result
-    against the oracle's composition."""
+    counts other than 128 and 256: the attention that keeps q, k, v and gate in memory for the former, the block's separate passes with
+    the operator on the tiled MFMA route for the latter; whole result against the oracle's composition."""
     torch = torch_cuda
     c = msa_case(9300 + n_seq + n_res, n_seq, n_res, heads, 128)
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
@@ -955,7 +943,7 @@ def test_msa_attention_blocks_on_the_tiled_route(torch_cuda, column, n_seq, n_re
     res = {}
     names = profiled_kernels(torch, lambda: res.setdefault("rc", blk.run()))
     torch.cuda.synchronize()
-    assert res["rc"] == 0 and "attention_tiles_kernel" in names, (res, names)
+    assert res["rc"] == 0 and ("streamed_attention_kernel" if heads == 8 else "attention_tiles_kernel") in names, (res, names)
     helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, column), "bf16", f"msa block {n_seq}x{n_res} heads={heads} column={column}")
 
 

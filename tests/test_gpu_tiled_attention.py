@@ -158,7 +158,8 @@ def test_heads_of_eight_at_tile_edges(torch_cuda, B, S, pair_bias):
         w.nb[:, S - 1, :] -= np.float32(150.0)
         w.nb = round_to_bf16(w.nb)
     w.bias = round_to_bf16(w.bias)
-    run_and_check(w)
+    names = helpers.profiled_kernels(torch_cuda, lambda: run_and_check(w))
+    assert ("small_head_attention_kernel" if S <= 1120 else "attention_tiles_kernel") in names, names
 
 
 def test_pair_bias_entries_of_minus_infinity(torch_cuda):
