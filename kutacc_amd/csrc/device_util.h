@@ -72,6 +72,33 @@ __device__ __forceinline__ float group_sum(float v)
     return v;
 }
 
+// LayerNorm's scale and shift from a row's sum and sum of squares, both of x - x0 with x0 the row's first element: y = x * rstd + shift,
+// then gamma and beta (reference src/normalization/layernorm_kernel.h:21-53).  ROUNDED: correctly rounded square root and quotient;
+// otherwise the hardware's reciprocal square root (1 ulp), for rows of which every lane forms it: the two rounded operations
+// expand to some 25 instructions per lane and row.
+template <bool ROUNDED>
+__device__ __forceinline__ void norm_from_sums(float s1, float s2, float x0, float n, float eps, float &rstd, float &shift)
+{
+    const float mean = s1 / n + x0;
+    const float var = fmaxf((s2 - s1 * s1 / n) / n, 0.f);
+    rstd = ROUNDED ? 1.0f / sqrtf(var + eps) : __builtin_amdgcn_rsqf(var + eps);
+    shift = -rstd * mean;
+}
+
+// the same of one row held as 8 values per lane of LPR consecutive lanes; x0 = first element of the row
+template <int LPR>
+__device__ __forceinline__ void group_stats(const float (&x)[8], float x0, float n, float eps, float &rstd, float &shift)
+{
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float v = x[e] - x0;
+        s1 += v;
+        s2 = fmaf(v, v, s2);
+    }
+    norm_from_sums<false>(group_sum<LPR>(s1), group_sum<LPR>(s2), x0, n, eps, rstd, shift);
+}
+
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
 } // namespace kutacc_dev

@@ -1359,12 +1359,8 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_head_kernel(F
                         s2 = fmaf(d, d, s2);
                     }
                 }
-                s1 = group_sum<8>(s1), s2 = group_sum<8>(s2);
-                const float nch = (float)C;
-                const float mean = s1 / nch + x0;
-                const float var = fmaxf((s2 - s1 * s1 / nch) / nch, 0.f);
-                const float rstd = __builtin_amdgcn_rsqf(var + p.ln_eps); // as the row kernels form it
-                const float shift = -rstd * mean;
+                float rstd, shift;
+                norm_from_sums<false>(group_sum<8>(s1), group_sum<8>(s2), x0, (float)C, p.ln_eps, rstd, shift); // as the row kernels form it
 #pragma unroll
                 for (int c = 0; c < NP; ++c) {
                     bf16x8 o;
@@ -2359,18 +2355,12 @@ int max_lds_bytes()
     return kutacc_device_attribute(hipDeviceAttributeMaxSharedMemoryPerBlock, 64 * 1024, table);
 }
 
-int num_cus()
-{
-    static int table[KUTACC_DEVICE_SLOTS] = {};
-    return kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, table);
-}
-
 // batch-row groups per XCD of the persistent kernels: one workgroup per CU at most; groups of 8*H workgroups share
 // batch-row sequences across the XCDs
 int persistent_groups(int B, int H)
 {
     const int per_ring = 8 * H;
-    int ngrp = num_cus() / per_ring;
+    int ngrp = kutacc_cu_count() / per_ring;
     const int need = (B + 7) / 8;
     ngrp = ngrp < 1 ? 1 : ngrp;
     return ngrp > need ? need : ngrp;
@@ -2624,7 +2614,7 @@ inline void output_projection_split(int C, int64_t M, int64_t &gx, int64_t &rpw)
     const int waves = 4 * (C / 128);
     const int64_t tiles = (M + 31) / 32;
     gx = (tiles + waves - 1) / waves;
-    const int64_t cap = (int64_t)num_cus() * (C == 128 ? 2 : 1);
+    const int64_t cap = (int64_t)kutacc_cu_count() * (C == 128 ? 2 : 1);
     gx = gx > cap ? cap : gx;
     rpw = ((M + gx * waves - 1) / (gx * waves) + 7) / 8 * 8;
 }
@@ -2834,7 +2824,7 @@ int gating_attention_fused(const kutacc_hip_attention_args_t &a, hipStream_t str
         fprintf(stderr,
                 "[kutacc] fused plan: persistent=%d C=%d NB=%d NT=%d NW=%d BPW=%d GW=%d lds=%zu max_lds=%d cus=%d log2_units=%d "
                 "fragments=%d row_pairs=%d\n",
-                (int)pl.persistent, C, pl.NB, p.NT, pl.NW, pl.BPW, pl.GW, pl.lds_bytes, max_lds_bytes(), num_cus(), p.l2mode,
+                (int)pl.persistent, C, pl.NB, p.NT, pl.NW, pl.BPW, pl.GW, pl.lds_bytes, max_lds_bytes(), kutacc_cu_count(), p.l2mode,
                 p.nbf != nullptr ? 1 : 0, (int)pair_kernel);
     }
     {

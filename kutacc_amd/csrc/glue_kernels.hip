@@ -113,11 +113,8 @@ __global__ __launch_bounds__(256) void layernorm_channel_first_bf16_kernel(const
             s2 = fmaf(d, d, s2);
         }
     }
-    const float n = (float)C;
-    const float mean = s1 / n + x0;
-    const float var = fmaxf((s2 - s1 * s1 / n) / n, 0.f);
-    const float rstd = 1.0f / sqrtf(var + eps);
-    const float shift = -rstd * mean;
+    float rstd, shift;
+    norm_from_sums<true>(s1, s2, x0, (float)C, eps, rstd, shift);
     uint4 *rows = tile[wave];
     const int lds_row = kk * 8 + mc; // 16 consecutive lanes write 16 consecutive rows: no bank conflicts
 #pragma unroll
@@ -161,11 +158,8 @@ __global__ __launch_bounds__(256) void layernorm_channel_first_kernel(const T *_
         s1 += d;
         s2 = fmaf(d, d, s2);
     }
-    const float n = (float)channels;
-    const float mean = s1 / n + x0;
-    const float var = fmaxf((s2 - s1 * s1 / n) / n, 0.f);
-    const float rstd = 1.0f / sqrtf(var + eps);
-    const float shift = -rstd * mean;
+    float rstd, shift;
+    norm_from_sums<true>(s1, s2, x0, (float)channels, eps, rstd, shift);
     for (int64_t c = 0; c < channels; ++c) {
         out[p * ld_out + c] = from_f32<T>(fmaf(fmaf(to_f32(x[c * ld_x + p]), rstd, shift), gamma[c], beta[c]));
     }

@@ -1352,13 +1352,7 @@ hipError_t launch_big_tiles(const GemmParams &p, int64_t blocks, hipStream_t str
     if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&pair_gemm_big_kernel<MM, BW>), BIG_GEMM_LDS, configured)) {
         return e;
     }
-    int device = 0, cus = 0;
-    if (hipError_t e = hipGetDevice(&device)) {
-        return e;
-    }
-    if (hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device)) {
-        return e;
-    }
+    const int cus = kutacc_cu_count();
     // one workgroup per CU; a multiple of 8, so that a workgroup's tiles stay on its XCD's share of the walk
     const int64_t grid = blocks < cus ? blocks : (cus >= 8 ? cus / 8 * 8 : cus);
     pair_gemm_big_kernel<MM, BW><<<dim3((unsigned)grid), 256, BIG_GEMM_LDS, stream>>>(p, blocks);
@@ -1372,13 +1366,7 @@ hipError_t launch_direct_tiles(const GemmParams &p, int64_t blocks, hipStream_t 
     if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&pair_gemm_direct_kernel<MM>), DIRECT_GEMM_LDS, configured)) {
         return e;
     }
-    int device = 0, cus = 0;
-    if (hipError_t e = hipGetDevice(&device)) {
-        return e;
-    }
-    if (hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device)) {
-        return e;
-    }
+    const int cus = kutacc_cu_count();
     const int64_t grid = blocks < cus ? blocks : (cus >= 8 ? cus / 8 * 8 : cus);
     pair_gemm_direct_kernel<MM><<<dim3((unsigned)grid), 256, DIRECT_GEMM_LDS, stream>>>(p, blocks);
     return hipGetLastError();
@@ -1413,11 +1401,10 @@ hipError_t launch_gated_projection(const kutacc_hip_gemm_args_t &g, const kutacc
     constexpr int WAVES = 4 * SIDES;
     constexpr size_t lds_bytes = (size_t)SIDES * 2 * 4 * 8 * 64 * 16 + WAVES * 4096;
     static size_t configured[KUTACC_DEVICE_SLOTS] = {};
-    static int cu_table[KUTACC_DEVICE_SLOTS] = {};
     if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&gated_projection_kernel<SIDES>), lds_bytes, configured)) {
         return e;
     }
-    const int cus = kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, cu_table);
+    const int cus = kutacc_cu_count();
     // eight resident waves per CU (two workgroups of four, or one of eight), every wave an equal range of positions (a
     // multiple of 8; the last step of a range may be partial)
     const int64_t tiles = (g.n + 63) / 64;
@@ -1440,11 +1427,10 @@ hipError_t launch_gated_projection_blocks(const kutacc_hip_gemm_args_t &g, hipSt
     constexpr int WAVES = 4, RING = 3;
     constexpr size_t lds_bytes = (size_t)(RING * 1024 + WAVES * (256 + RING * 16)) * 16;
     static size_t configured[KUTACC_DEVICE_SLOTS] = {};
-    static int cu_table[KUTACC_DEVICE_SLOTS] = {};
     if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&gated_projection_blocks_kernel), lds_bytes, configured)) {
         return e;
     }
-    const int cus = kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, cu_table);
+    const int cus = kutacc_cu_count();
     // two resident workgroups per CU; every workgroup an equal run of steps
     const int64_t steps = (g.n + 63) / 64;
     const int64_t cap = (int64_t)cus * 2;

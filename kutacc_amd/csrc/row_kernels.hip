@@ -32,11 +32,7 @@ __device__ __forceinline__ void row_stats(const T *__restrict__ row, int64_t siz
     }
     s1 = wave_sum(s1);
     s2 = wave_sum(s2);
-    const float n = (float)size;
-    const float mean = s1 / n + delta;
-    const float var = fmaxf((s2 - s1 * s1 / n) / n, 0.f);
-    rstd = 1.0f / sqrtf(var + eps);
-    shift = -rstd * mean;
+    norm_from_sums<true>(s1, s2, delta, (float)size, eps, rstd, shift);
 }
 
 template <typename T>
@@ -129,28 +125,6 @@ union Pack16 {
     bf16x8 b;
     bf16x2 p[4];
 };
-
-// statistics of one row held as 8 values per lane; x0 = first element of the row
-template <int LPR>
-__device__ __forceinline__ void group_stats(const float (&x)[8], float x0, float n, float eps, float &rstd, float &shift)
-{
-    float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float v = x[e] - x0;
-        s1 += v;
-        s2 = fmaf(v, v, s2);
-    }
-    s1 = group_sum<LPR>(s1);
-    s2 = group_sum<LPR>(s2);
-    const float mean = s1 / n + x0;
-    const float var = fmaxf((s2 - s1 * s1 / n) / n, 0.f);
-    // The hardware's reciprocal square root (1 ulp) instead of an IEEE square root and division: every lane of a row
-    // forms it, the two correctly rounded operations expand to some 25 instructions per lane and row, and the normalised
-    // value is rounded to bf16 afterwards.
-    rstd = __builtin_amdgcn_rsqf(var + eps);
-    shift = -rstd * mean;
-}
 
 // NEAR: fewer than 2^24 rows, row pitches below 2^23 elements and less than 2^31 bytes from the first row to the end of
 // the last (the launcher checks): rows are counted in 32 bits and addressed by 32-bit byte offsets from the tensors'
@@ -627,8 +601,7 @@ int linear(int32_t dtype, const void *act, int64_t ld_act, const void *w, int64_
             // (all 256 outputs of 256 features at once, 62 899 rows: 39 us against 31 in slices; 3 313 rows x 128: 15 against 9).
             const int slice = (int)(n < 16384 / k ? n : 16384 / k), slices = (int)((n + slice - 1) / slice);
             const size_t lds_bytes = (size_t)((slice + 31) / 32 * (k / 16) * 64 + 4 * 256) * 16 + 256 * sizeof(float);
-            static int cu_table[KUTACC_DEVICE_SLOTS] = {};
-            const int cus = kutacc_device_attribute(hipDeviceAttributeMultiprocessorCount, 256, cu_table);
+            const int cus = kutacc_cu_count();
             // as many workgroups as are resident at once, at most eight per CU; each stages the weights once
             const int64_t resident = (int64_t)(160 * 1024) / (int64_t)lds_bytes;
             const int64_t cap = (cus * (resident > 8 ? 8 : resident) + slices - 1) / slices, blocks = (m + 127) / 128;

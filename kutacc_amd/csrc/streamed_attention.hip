@@ -304,7 +304,7 @@ __global__ __launch_bounds__(768) void streamed_attention_kernel(const StreamedP
             const int t = min(first_tile + (u >> 3), NB - 1);
             const uint4 *src = ((u & 2) ? p.v : p.k) + (((u & 4) ? rowB : rowA) + t) * BLOCK_SLOTS + (u & 1) * 64;
             const uint32_t to = ring + (uint32_t)(place * TILES_PER_GROUP) * TILE_BYTES + (uint32_t)u * 1024u;
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(lane_bytes), "s"(src) : "memory");
+            load_to_lds(to, src, lane_bytes);
         }
     };
     request(0, 0);

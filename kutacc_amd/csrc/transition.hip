@@ -95,13 +95,8 @@ __device__ __forceinline__ XFragments<CO> fragments(Rows<CO> t, const Transition
                     s2 = fmaf(d, d, s2);
                 }
             }
-            s1 = group_sum<8>(s1);
-            s2 = group_sum<8>(s2);
-            const float n = (float)CO;
-            const float mean = s1 / n + x0;
-            const float var = fmaxf((s2 - s1 * s1 / n) / n, 0.f);
-            const float rstd = 1.0f / sqrtf(var + p.ln_eps);
-            const float shift = -rstd * mean;
+            float rstd, shift;
+            norm_from_sums<true>(group_sum<8>(s1), group_sum<8>(s2), x0, (float)CO, p.ln_eps, rstd, shift);
 #pragma unroll
             for (int cp = 0; cp < CP; ++cp) {
                 const bf16x8 b = as_bf16x8(*regs[cp]);

@@ -57,21 +57,8 @@ __device__ __forceinline__ uint4 normalise_row(uint4 raw, int lane, const float 
     for (int e = 0; e < 8; ++e) {
         v[e] = to_f32(b[e]);
     }
-    const float x0 = __shfl(v[0], lane & ~15, 64);
-    float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float d = v[e] - x0;
-        s1 += d;
-        s2 = fmaf(d, d, s2);
-    }
-    s1 = group_sum<16>(s1);
-    s2 = group_sum<16>(s2);
-    const float n = (float)C;
-    const float mean = s1 / n + x0;
-    const float var = fmaxf((s2 - s1 * s1 / n) / n, 0.f);
-    const float rstd = __builtin_amdgcn_rsqf(var + eps);
-    const float shift = -rstd * mean;
+    float rstd, shift;
+    group_stats<16>(v, __shfl(v[0], lane & ~15, 64), (float)C, eps, rstd, shift);
     bf16x8 o;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -404,12 +391,8 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
                     s2 = fmaf(d, d, s2);
                 }
             }
-            s1 = group_sum<8>(s1), s2 = group_sum<8>(s2);
-            const float nch = (float)C;
-            const float mean = s1 / nch + x0;
-            const float var = fmaxf((s2 - s1 * s1 / nch) / nch, 0.f);
-            const float rstd = 1.0f / sqrtf(var + eps);
-            const float shift = -rstd * mean;
+            float rstd, shift;
+            norm_from_sums<true>(group_sum<8>(s1), group_sum<8>(s2), x0, (float)C, eps, rstd, shift);
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const float *gm = params + 2 * C + 64 * t + 8 * c8, *bt = gm + C;
