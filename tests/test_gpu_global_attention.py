@@ -98,6 +98,34 @@ def test_global_attention_rows_past_the_kept_tiles(torch_cuda, B, S, H, d):
     helpers.assert_within(helpers.to_numpy(scratch["avg"]), ref_qavg, 2.0 ** -8 * np.abs(ref_qavg) + 1e-6, "masked mean q_avg")
 
 
+def test_global_attention_replays_from_a_hip_graph(torch_cuda):
+    """Rows past the kept tiles, whose rest comes through the ring in the LDS: captured on a side stream and replayed three times, with
+    eager work (the results overwritten) between the replays; every replay gives the eager result bit for bit."""
+    torch = torch_cuda
+    c = make_case(11, 3, 2590, 8, 8)
+    op, ten, scratch = device_op(torch, c)
+    op.run()
+    torch.cuda.synchronize()
+    want, want_avg = ten["out"].clone(), scratch["avg"].clone()
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    capi.set_blocking(False)
+    try:
+        with torch.cuda.graph(graph, stream=side):
+            capi.set_stream(torch.cuda.current_stream().cuda_stream)
+            op.run()
+    finally:
+        capi.set_stream(None)
+        capi.set_blocking(True)
+    assert not capi.error_flag()
+    for _ in range(3):
+        ten["out"].fill_(7.0)
+        scratch["avg"].fill_(-3.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert helpers.same_bits(ten["out"], want) and helpers.same_bits(scratch["avg"], want_avg)
+
+
 def test_global_attention_full_extra_msa_shape(torch_cuda):
     """An extra-MSA sized call (N_res = 256 batch rows of 1024 extra sequences): spot-check rows against the oracle."""
     c = make_case(7, 256, 1024, 8, 8, "random")

@@ -430,6 +430,67 @@ def drawn_block(torch, seed, kind, n_seq, n_res, heads):
     return act, w, lambda z, v: capi.MsaAttentionBlock(z, mask, v, heads, pair)
 
 
+@pytest.mark.parametrize("kind,n_seq,n_res,heads", [("triangle", 0, 1025, 4), ("row", 3, 1057, 4), ("column", 1056, 3, 8)])
+def test_blocks_beyond_1024_keys_replay_from_a_hip_graph(torch_cuda, kind, n_seq, n_res, heads):
+    """Captured on a side stream and replayed three times, with eager work (the activation and the workspace overwritten) between the
+    replays: every replay gives the eager result bit for bit."""
+    torch = torch_cuda
+    act, w, block = drawn_block(torch, 177 + n_res, kind, n_seq, n_res, heads)
+    z = act.clone()
+    blk = block(z, w)
+    print(f"graph {kind} {n_seq}x{n_res} heads={heads}", flush=True)
+    assert blk.run() == 0  # eager; also takes first-call set-up out of the capture
+    torch.cuda.synchronize()
+    want = z.clone()
+    assert bool(torch.isfinite(want).all()) and not helpers.same_bits(want, act)
+    z.copy_(act)
+    torch.cuda.synchronize()
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        assert blk.run(torch.cuda.current_stream().cuda_stream) == 0
+    for _ in range(3):
+        z.copy_(act)
+        blk.workspace.fill_(255)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert helpers.same_bits(z, want)
+
+
+def test_triangle_attention_block_of_1025_residues(torch_cuda):
+    """The first length past the fused head kernels' longest row, one key into its last tile and one row without a partner: both
+    orientations against the oracle on a sample of attention rows."""
+    torch = torch_cuda
+    n = 1025
+    c = block_case(9150, n, 4)
+    rows = [0, 1, 31, 32, 512, n - 3, n - 2, n - 1]
+    for ending in (False, True):
+        got = run_block(torch, c, ending)
+        assert bool(torch.isfinite(got).all())
+        sample = got[:, rows].transpose(0, 1) if ending else got[rows]
+        helpers.check_close(helpers.to_numpy(sample.contiguous()), block_oracle_rows(c, ending, rows), "bf16", f"block n={n} ending={ending}, sampled rows")
+
+
+# rows without a partner; whole tiles and one key more or less; four and five query blocks to the last workgroup; sixteen workgroups
+# and one more to a row; a pair bias whose producer does not write the tiles
+@pytest.mark.parametrize("column,n_seq,n_res,heads,c_z", [(False, 1, 1056, 4, 128), (True, 1055, 3, 4, 1), (True, 1057, 5, 8, 1), (True, 1152, 2, 4, 1),
+                                                          (True, 1153, 1, 8, 1), (True, 2048, 2, 8, 1), (True, 2049, 3, 4, 1), (False, 2, 1281, 8, 16)])
+def test_msa_attention_blocks_beyond_1024_keys(torch_cuda, column, n_seq, n_res, heads, c_z):
+    torch = torch_cuda
+    c = msa_case(9700 + n_seq + n_res, n_seq, n_res, heads, c_z)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
+        device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
+    msa = dev(c["m"])
+    w = {k: dev(c[k]) for k in ("ln_gamma", "ln_beta", "wq", "wk", "wv", "wg", "bg", "wo", "bo")}
+    pair = None if column else {"pair_act": dev(c["z"]), "pair_ln_gamma": dev(c["pair_ln_gamma"]),
+                                "pair_ln_beta": dev(c["pair_ln_beta"]), "bias_w": dev(c["bias_w"])}
+    res = {}
+    names = profiled_kernels(torch, lambda: res.setdefault("rc", capi.MsaAttentionBlock(msa, dev(c["mask"]), w, heads, pair).run()))
+    torch.cuda.synchronize()
+    assert res["rc"] == 0 and "streamed_attention_kernel" in names and ("pair_bias_tiles_kernel" in names) == (c_z == 16), (res, names)
+    helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, column), "bf16", f"msa block {n_seq}x{n_res} heads={heads} column={column}")
+
+
 @pytest.mark.parametrize("kind,n_seq,n_res,heads", [("triangle", 0, 1025, 4), ("row", 3, 1050, 8), ("column", 1030, 2, 4)])
 def test_blocks_beyond_1024_keys_take_weights_on_any_address(torch_cuda, kind, n_seq, n_res, heads):
     """The route of these blocks asks nothing of the weights' alignment: the same bits with every matrix and both biases one element
@@ -589,8 +650,12 @@ def test_triangle_multiplication_block_at_any_length(torch_cuda, n):
         assert capi.TriangleMultiplicationBlock(pair, dev(case["mask"]), w, incoming).run() == 0
         torch.cuda.synchronize()
         want = tm_block_oracle(case, incoming)
-        # half as much again as the usual bar: six bf16 roundings in a chain, up to five million values per orientation
-        helpers.assert_within(helpers.to_numpy(pair), want, 3e-2 + 1.5e-2 * np.abs(want), f"TM block n={n} incoming={incoming}")
+        # Values behind the roundings of the normalised row, projections, their products and the centre (0.2 % each, two sides): the
+        # normalised centre, of order one, is off by 0.5 % rms, and so is the update at most; 5 million of them lie within five
+        # times that.  The sum with the activation is rounded once more, by at most 2^-8.
+        got = helpers.to_numpy(pair)
+        helpers.assert_within(got, want, 2.5e-2 + 2.0 ** -8 * np.abs(want), f"TM block n={n} incoming={incoming}")
+        assert np.sqrt(np.mean((got - want) ** 2)) < 5e-3
         assert bool((guarded[n * n:] == 7.0).all())
 
 

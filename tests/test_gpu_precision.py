@@ -141,3 +141,22 @@ def test_centre_layernorm_of_the_triangle_multiplication_is_exact_to_32_bits(tor
         assert capi.TriangleMultiplicationBlock(act, torch.ones(1, 1, device="cuda", dtype=torch.bfloat16), w, False).run() == 0
         torch.cuda.synchronize()
         assert not bool(act.any()), (seed, float(act.abs().max()))
+
+
+@pytest.mark.parametrize("B,S,H", [(130, 97, 4), (135, 135, 4), (70, 100, 8)])
+def test_infinite_pair_bias_and_masked_rows_on_fp32_tiles(torch_cuda, B, S, H):
+    """The single-row kernels that read the pair bias as fp32 tiles: pairs excluded by -inf, a row with every key masked, a query whose
+    logits leave the range of the unshifted softmax."""
+    w = draw_workload(60 + B, B, S, H, 32)
+    drop = np.random.Generator(np.random.PCG64(B)).random(w.nb.shape) < 0.3
+    drop[:, :, 0] = False
+    w.nb[:, S // 2, :] += np.float32(150.0)
+    w.nb = round_to_bf16(w.nb)
+    w.nb[drop] = -np.inf
+    w.bias[B // 2, :] = round_to_bf16(np.full(S, MASK_BIAS, dtype=np.float32))
+    print(f"B={B} S={S} H={H}", flush=True)
+    ten, scratch = helpers.to_device(w)
+    assert helpers.run_hip(w, ten, scratch) == 0 and capi.last_path() == "fused_mfma"
+    ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
+    helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(B, S, -1), ref_avg, "bf16", "gated average")
+    helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, "bf16", "out")
