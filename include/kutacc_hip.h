@@ -78,7 +78,7 @@ typedef struct kutacc_hip_attention_args {
     int64_t nb_stride_q;
 
     /* Caller scratch.  k/v/gate are written only by the generic and the tiled path; q is written by those
-     * and may be used as workspace by the fused path (a fragment-major copy of the pair bias), so
+     * and may be used as workspace by the fused path (a re-ordered copy of the pair bias), so
      * its contents are unspecified after any call; avg (gated weighted average, [B,S,H,d]) is
      * written by every path.  Element (b,s,h,e) of q,k,gate,avg lives at
      * b*stride_b + s*stride_s + h*stride_h + e; v is [H,d,B,S]: (h,e,b,s) at
@@ -101,7 +101,7 @@ kutacc_export int kutacc_hip_gating_attention(const kutacc_hip_attention_args_t 
 /*
  * kutacc_hip_gating_attention for callers that cannot allocate device memory or lend scratch: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.  The one
- * scratch buffer of the MFMA kernels, a fragment-major copy of the pair bias, lives in a device array inside the
+ * scratch buffer of the MFMA kernels, a re-ordered copy of the pair bias, lives in a device array inside the
  * library image (KUTACC_HIP_STATIC_SCRATCH_BYTES; each GPU the library runs on holds it until the process ends), so
  * args->q, k, v and gate are neither read nor written and may be NULL.  Nothing on this path calls hipMalloc, hipFree
  * or any allocating routine; per-kernel profiling events are not recorded for it.  Only shapes the MFMA kernels take
@@ -450,7 +450,8 @@ kutacc_export int kutacc_hip_profile_read(int index, char *name, int name_len, d
  *   "debug"     "1": one line per fused call on stderr with the plan taken; "0": default
  *   "row_pairs" "0": never the attention kernel that walks two batch rows per step (128 channels up to 384 positions,
  *               256 channels up to 256);
- *               "1": wherever it can run; anything else (default): where every workgroup has at least two batch rows
+ *               "1": wherever it can run; anything else (default): where every workgroup has at least two batch rows, and
+ *               an even number of them or many
  *   "streamed"  "1": kutacc_hip_triangle_attention and kutacc_hip_msa_attention with 128 or 256 channels run every length, not
  *               only those beyond 1024, on the attention kernels that keep q, k, v and gate in memory (the workspace functions
  *               answer for the setting in force when they are called); anything else: default

@@ -7,7 +7,7 @@
 //       the attention loads -- 1 KB per store instruction, no layout change anywhere after it.
 //   streamed_attention_kernel softmax(q.k^T + mask + pair bias).v * gate.  A wave owns the same 32 queries of two batch rows,
 //       which share the pair bias (fp32 tiles in accumulator order, the C operand of both rows' logits MFMAs, as in
-//       persistent_pair_kernel); a workgroup of three to six waves walks all keys of the two rows, its K and V staged
+//       persistent_pair_kernel); a workgroup of four waves walks all keys of the two rows, its K and V staged
 //       through a ring of three key tiles in the LDS.
 //
 // Against fused_head_kernel (one workgroup per row and head, K and V of the whole row in the LDS, projections in front):

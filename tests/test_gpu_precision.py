@@ -46,7 +46,7 @@ def relative_error(got, want):
     (128, 160, 4),  # two rows, together
 ])
 def test_pair_bias_keeps_32_bits(torch_cuda, B, S, H):
-    """A pair bias around 50, whose bf16 steps are a quarter: times log2(e) in 11 bits the probabilities would be off by 0.6 %.  Two
+    """A pair bias around 50, whose bf16 steps are a quarter: times log2(e) in 11 bits the probabilities would be off by 1.2 %.  Two
     queries sit at 200 and -200, where the softmax is repeated with the row maxima subtracted, and some keys are masked."""
     w = draw_workload(40 + B + S, B, S, H, 32, masked=0.05)
     w.nb = w.nb * np.float32(0.5) + np.float32(50.0)
