@@ -2893,19 +2893,6 @@ int row_projection_gated_residual(const void *a, int64_t a_ld, const void *w, co
                     : launch_output_projection<256, EPILOGUE_GATED_RESIDUAL>(a, a_ld, w, bias, acc, acc_ld, m, n, stream, gate, gate_ld);
 }
 
-// acc[m, n] += bf16(sum_k a[m, k] * w[n, k] + bias[n]), row (i, j) of the product's [m / swap_n, swap_n] grid going to row (j, i) of
-// acc where swap_n is not zero: same shapes as row_projection
-int row_projection_residual(const void *a, int64_t a_ld, const void *w, const float *bias, void *acc, int64_t acc_ld, int64_t m,
-                            int64_t n, int64_t k, int64_t swap_n, hipStream_t stream)
-{
-    if (!row_projection_supports(a, a_ld, w, bias, acc, acc_ld, m, n, k)) {
-        return KUTACC_HIP_EUNSUPPORTED;
-    }
-    kutacc_prof::KernelTimer t("output_projection_kernel<residual>", 2.0 * (double)m * (double)n * (double)k, stream);
-    return k == 128 ? launch_output_projection<128, EPILOGUE_RESIDUAL>(a, a_ld, w, bias, acc, acc_ld, m, n, stream, nullptr, 0, swap_n)
-                    : launch_output_projection<256, EPILOGUE_RESIDUAL>(a, a_ld, w, bias, acc, acc_ld, m, n, stream, nullptr, 0, swap_n);
-}
-
 } // namespace kutacc_launch
 
 // ------------------------------------------------------------------------------------------------

@@ -133,8 +133,8 @@ int gating_attention_fused(const kutacc_hip_attention_args_t &args, hipStream_t 
 int pair_bias_tiles(const kutacc_hip_attention_args_t &args, void *tiles, hipStream_t stream);
 
 // streamed_attention.hip: rows of any length, 128 or 256 channels in heads of 32, on a workspace of streamed_workspace_bytes()
-// (256-byte aligned) that starts with the tiles of the pair bias; opt.nb_tiles_ready: they lie there already.  args.q, k, v
-// and gate are not used, weights and biases may lie on any address; the result is added to args.out (opt.out_mode FUSED_OUT_ADD or
+// (256-byte aligned) that starts with the tiles of the pair bias; opt.nb_tiles_ready: they lie there already.  args.q, k, v,
+// gate and avg are not used, weights, biases and args.out may lie on any address; the result is added to args.out (opt.out_mode FUSED_OUT_ADD or
 // FUSED_OUT_ADD_TRANSPOSED).
 bool streamed_attention_supports(const kutacc_hip_attention_args_t &args);
 int64_t streamed_workspace_bytes(int64_t batch, int64_t seq_len, int64_t nheads, bool pair_bias);
@@ -153,9 +153,6 @@ bool row_projection_supports(const void *a, int64_t a_ld, const void *w, const f
 int row_projection(const void *a, int64_t a_ld, const void *w, const float *bias, void *out, int64_t out_ld, int64_t m,
                    int64_t n, int64_t k, hipStream_t stream);
 
-// acc += the product's rows, row (i, j) of their [m / swap_n, swap_n] grid to row (j, i) of acc where swap_n is not zero
-int row_projection_residual(const void *a, int64_t a_ld, const void *w, const float *bias, void *acc, int64_t acc_ld, int64_t m,
-                            int64_t n, int64_t k, int64_t swap_n, hipStream_t stream);
 int row_projection_gated_residual(const void *a, int64_t a_ld, const void *w, const float *bias, const void *gate,
                                   int64_t gate_ld, void *acc, int64_t acc_ld, int64_t m, int64_t n, int64_t k,
                                   hipStream_t stream);

@@ -1,19 +1,20 @@
 // Gated attention of long batch rows for gfx950, bf16 storage, head size 32, 128 or 256 channels: the rows whose keys and
 // values do not fit the LDS twice beside a head's weights (persistent_pair_kernel), in batches that fill the chip.
 //
-// Two kernels share the work, with K, V, Q and the gate in memory between them:
+// Three kernels share the work, with K, V, Q, the gate and the gated average in memory between them:
 //
 //   qkvg_projection_kernel    reads the input rows once, forms all four projections and writes them as the MFMA fragments
 //       the attention loads -- 1 KB per store instruction, no layout change anywhere after it.
-//   streamed_attention_kernel softmax(q.k^T + mask + pair bias).v * gate.  A wave owns the same 32 queries of two batch rows,
-//       which share the pair bias (fp32 tiles in accumulator order, the C operand of both rows' logits MFMAs, as in
-//       persistent_pair_kernel); a workgroup of four waves walks all keys of the two rows, its K and V staged
-//       through a ring of three key tiles in the LDS.
+//   streamed_attention_kernel softmax(q.k^T + mask + pair bias).v * gate.  A wave owns the same 32 queries of several batch rows,
+//       which share the pair bias (fp32 tiles in accumulator order, the C operand of every row's logits MFMAs, as in
+//       persistent_pair_kernel); a workgroup of four waves walks all keys of the rows, their K and V staged
+//       through a ring of key tiles in the LDS.
+//   output_projection_kernel  multiplies the gated average, fragments as well, and adds the result to the activation.
 //
 // Against fused_head_kernel (one workgroup per row and head, K and V of the whole row in the LDS, projections in front):
-// the pair bias costs no MFMAs and half the bytes, three waves per SIMD at every length instead of two, the projections
+// the pair bias costs no MFMAs and half the bytes, waves of every length work alike, the projections
 // run at the rate of the memory instead of behind one barrier per workgroup, and a row's length decides nothing.  The price
-// is the four projections through memory, 8 bytes per channel and position.
+// is the four projections and the average through memory, 10 bytes per channel and position.
 //
 // The order of positions, keys and head dims inside a fragment is that of the fused kernels (fused_attention.hip): lane r
 // of a block of 32 positions stands for position pi(r), Q and K share their order of head dims, V and the probabilities
@@ -24,6 +25,7 @@
 #include <atomic>
 #include <climits>
 #include <cstring>
+#include <type_traits>
 
 #include "attention_util.h"
 #include "launch_internal.h"
@@ -34,6 +36,7 @@ namespace {
 using namespace kutacc_dev;
 
 constexpr int HEAD = 32;
+constexpr uint32_t MIXED_WORDS = 1; // no word a row shares: a denormal mask bias
 constexpr int BLOCK_SLOTS = 128; // 16-byte slots of a fragment pair: 32 positions x 32 head dims
 
 struct StreamedParams {
@@ -45,17 +48,18 @@ struct StreamedParams {
     int64_t bias_sb, bias_sk;
     int bias_is_mask;
     float qmul; // log2(e) / sqrt(head size)
-    uint4 *q, *g, *k, *v; // [batch row][head][block of 32 positions][2 k-steps][64 lanes]
+    // [batch row][head][block of 32 positions][2 k-steps][64 lanes]; the gated average takes the place of the queries it was formed from
+    uint4 *q, *g, *k, *v;
     // [batch row][block][32]: mask bias of key pi(i) in log2 units as two bf16 (mask_word).  Their 2^-17 moves no probability: the bias
     // is formed from a bf16 mask, so it is 0, or at least 3.9e6 in size and 2^-8 of that from any other.  (A third part was 7 %
     // slower at 2048 residues, a tenth of them masked.)
     uint32_t *words;
-    uint32_t *flags;      // [batch row][block]: some word of the block is not zero
+    // [batch row][block]: 0, no key of the block has a mask; the word that all its keys have (those of the row, the tail is at -inf);
+    // MIXED_WORDS otherwise
+    uint32_t *flags;
     const f32x4 *tiles;   // pair bias: [head][query block][NT][4][64 lanes] (pair_bias_tiles_kernel)
-    bf16_t *avg;          // first batch row of the slice
-    int64_t avg_sb, avg_ss;
     int B, S, H, NB, NT; // batch rows of the slice, positions, heads, blocks, key tiles of `tiles` per query block
-    int query_groups, pair_groups, groups, group_rows; // placement of the attention's workgroups
+    int query_groups, set_groups, groups, group_rows; // placement of the attention's workgroups
 };
 
 // ---- the projections ----
@@ -187,12 +191,13 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
                     }
                     mv *= LOG2E;
                 }
+                const uint32_t word = mask_word(mv), first_word = __builtin_amdgcn_readfirstlane(word); // lane 0: key 32 j
                 if (lane < 32) {
-                    p.words[((int64_t)b * p.NB + j) * 32 + lane] = mask_word(mv);
+                    p.words[((int64_t)b * p.NB + j) * 32 + lane] = word;
                 }
-                const bool any = __ballot(mv != 0.f) != 0;
+                const bool any = __ballot(mv != 0.f) != 0, mixed = __ballot(key < p.S && word != first_word) != 0 || first_word == 0;
                 if (lane == 0) {
-                    p.flags[(int64_t)b * p.NB + j] = any ? 1u : 0u;
+                    p.flags[(int64_t)b * p.NB + j] = !any ? 0u : (mixed ? MIXED_WORDS : first_word);
                 }
             }
             if (++j == p.NB) {
@@ -204,20 +209,41 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
 }
 
 // ---- the attention ----
-constexpr int WAVES = 4;                      // query blocks per workgroup
-constexpr int TILES_PER_GROUP = WAVES / 2;    // key tiles per barrier: four pieces of 1 KB for every wave
-constexpr int RING = 3;                       // groups of tiles in the LDS
-constexpr int TOGETHER = 8, MEMBERS = 64;     // query groups and workgroups of a placement group, at most
-constexpr int TILE_SLOTS = 4 * BLOCK_SLOTS;   // K and V of one key tile of the two rows: [row][K, V][2][64]
-constexpr int TILE_BYTES = TILE_SLOTS * 16;
+constexpr int WAVES = 4;                  // query blocks per workgroup
+constexpr int RING = 3;                   // groups of tiles in the LDS
+constexpr int TOGETHER = 8, MEMBERS = 64; // query groups and workgroups of a placement group, at most
 
-// Repeat of one row's 32 queries after an overflow or underflow of the unshifted exponentials (a sum outside 1e-30 .. 1e30, a
-// row with every key masked): the true row maxima first, then the probabilities with them subtracted.  Not a hot path:
-// one row, operands straight from memory, no barrier.
-template <bool HAS_NB>
-__device__ __forceinline__ void attend_shifted(const uint4 *k, const uint4 *v, const uint32_t *words, const f32x4 *nbc, bf16x8 q0, bf16x8 q1,
-                                               int NB, int lane, f32x16 &o_out, float &l_out)
+// What a wave attends with one set of 32 queries' positions: ROWS batch rows, which share a tile of the pair bias.  A tile's keys and
+// values are ROWS x 4 KB; tiles come in groups of which every wave brings four pieces of 1 KB.
+template <int ROWS>
+struct Walk {
+    static constexpr int TILES_PER_GROUP = 4 / ROWS, TILE_SLOTS = ROWS * 2 * BLOCK_SLOTS, TILE_BYTES = TILE_SLOTS * 16;
+    static constexpr int GROUP_BYTES = TILES_PER_GROUP * TILE_BYTES; // 4 KB a wave
+    static constexpr size_t LDS = (size_t)RING * GROUP_BYTES;
+};
+
+// The gated average of 32 queries of one row in the place of their queries: o / l * sigmoid(gate).  Positions past the row's end are
+// stored like the others: nobody reads them.
+__device__ __forceinline__ void store_average(uint4 *dst, uint4 gate0, uint4 gate1, const f32x16 &o, float l)
 {
+    const bf16x8 g0 = as_bf16x8(gate0), g1 = as_bf16x8(gate1);
+    const float inv = 1.0f / l;
+    f32x16 out;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        out[i] = o[i] * inv * sigmoid_fast(to_f32(g0[i])), out[8 + i] = o[8 + i] * inv * sigmoid_fast(to_f32(g1[i]));
+    }
+    dst[0] = as_uint4(pack8(out, 0)), dst[64] = as_uint4(pack8(out, 8));
+}
+
+// Repeat of one row's 32 queries after an overflow or underflow of the unshifted exponentials (a sum outside 1e-30 .. 1e30): the
+// true row maxima first, then the probabilities with them subtracted.  Not a hot path: one row, operands straight from memory, no
+// barrier.  q: the queries, whose place the result takes.
+template <bool HAS_NB>
+__device__ __forceinline__ void attend_shifted(const uint4 *k, const uint4 *v, const uint32_t *words, const f32x4 *nbc, uint4 *q, const uint4 *gate,
+                                               int NB, int lane)
+{
+    const bf16x8 q0 = as_bf16x8(q[lane]), q1 = as_bf16x8(q[64 + lane]);
     auto logits = [&](int t) {
         f32x16 x;
 #pragma unroll
@@ -259,23 +285,27 @@ __device__ __forceinline__ void attend_shifted(const uint4 *k, const uint4 *v, c
             sums = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, pv, sums, 0, 0, 0);
         }
     }
-    o_out = o;
-    l_out = rowsum_fetch(sums, lane);
+    store_average(q + lane, gate[lane], gate[64 + lane], o, rowsum_fetch(sums, lane));
 }
 
-// Keys and values come straight into the LDS (global_load_lds_dwordx4), two key tiles at a time, so that every wave brings
-// four pieces of 1 KB per group of tiles: a ring of three groups, one barrier per group.  At the barrier in front of group G,
-// group G + 1 has landed and group G - 1 has been left by every wave; its place takes group G + 2.  Three workgroups share
-// a CU: three waves per SIMD (the launch bound asks for 168 registers), 48 KB of ring each.
-template <bool HAS_NB>
-__global__ __launch_bounds__(768) void streamed_attention_kernel(const StreamedParams p)
+// Bound by the issue of the softmax (16 exponentials and 8 packs per lane, row and tile: 201 of the 268 clocks that a tile of 32 x 32
+// logits takes a SIMD with no load in the loop) and next to it by what the loop loads.  Four rows a wave halve the loads of
+// the pair bias, 4 KB a tile, and leave 256 registers to the two waves of a SIMD, against two rows on three waves of 168: 2048
+// residues without padding 6.56 -> 5.84 ms, 1024 residues 1.00 -> 0.79 ms.  Without a pair bias rows share nothing: two rows on three waves.
+//
+// Keys and values come straight into the LDS (global_load_lds_dwordx4), a group of tiles at a time, of which every wave brings four
+// pieces of 1 KB: a ring of three groups, one barrier per group.  At the barrier in front of group G, group G + 1 has landed and group
+// G - 1 has been left by every wave; its place takes group G + 2.
+template <bool HAS_NB, int ROWS>
+__global__ __launch_bounds__(ROWS == 4 || HAS_NB ? 512 : 768) void streamed_attention_kernel(const StreamedParams p)
 {
+    using W = Walk<ROWS>;
     typedef __attribute__((address_space(3))) void *lds_ptr;
     extern __shared__ uint4 lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int NB = p.NB;
 
-    // Workgroup ids are dealt round robin over the 8 XCDs; an XCD works on one group at a time: group_rows pairs of rows x
+    // Workgroup ids are dealt round robin over the 8 XCDs; an XCD works on one group at a time: group_rows sets of rows x
     // up to eight query groups of one head, which sweep the keys together, so that the group's K and V and pair bias come
     // from memory once and from the XCD's L2 after that.
     const int members = p.group_rows * min(p.query_groups, TOGETHER);
@@ -284,39 +314,59 @@ __global__ __launch_bounds__(768) void streamed_attention_kernel(const StreamedP
     if (group >= p.groups) {
         return;
     }
-    const int pair_group = group % p.pair_groups, rest = group / p.pair_groups;
+    const int set_group = group % p.set_groups, rest = group / p.set_groups;
     const int h = rest % p.H, query_part = rest / p.H;
-    const int pair = pair_group * p.group_rows + member % p.group_rows, qg = query_part * TOGETHER + member / p.group_rows;
-    if (2 * pair >= p.B || qg >= p.query_groups) {
+    const int set = set_group * p.group_rows + member % p.group_rows, qg = query_part * TOGETHER + member / p.group_rows;
+    if (ROWS * set >= p.B || qg >= p.query_groups) {
         return;
     }
-    const int bA = 2 * pair, bB = min(bA + 1, p.B - 1);
     const int j = qg * WAVES + wave;
-    const int64_t rowA = ((int64_t)bA * p.H + h) * NB, rowB = ((int64_t)bB * p.H + h) * NB; // first fragment block of either row
+    int b[ROWS]; // past the last row: that one again, not stored
+    int64_t row[ROWS]; // first fragment block
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        b[i] = min(ROWS * set + i, p.B - 1);
+        row[i] = ((int64_t)b[i] * p.H + h) * NB;
+    }
 
-    // The pieces u = 4 wave + i of a group of tiles: tile u / 8, piece u % 8 = [row][K, V][k-step].  Written out: as a builtin
+    // The pieces u = 4 wave + i of a group of tiles: tile u / (4 ROWS), piece u % (4 ROWS) = [row][K, V][k-step].  Written out: as a builtin
     // the compiler takes every LDS read behind it for a reader of its data and waits for all loads in flight.
     const uint32_t ring = (uint32_t)(uintptr_t)(lds_ptr)lds, lane_bytes = 16u * (uint32_t)lane;
+    const int own_row = ROWS == 4 ? wave : wave & 1; // all four pieces of a wave are of one row and tile
+    const int64_t own = ((int64_t)min(ROWS * set + own_row, p.B - 1) * p.H + h) * NB;
     auto request = [&](int first_tile, int place) { // tiles first_tile .. into group `place` of the ring
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int u = 4 * wave + i;
-            const int t = min(first_tile + (u >> 3), NB - 1);
-            const uint4 *src = ((u & 2) ? p.v : p.k) + (((u & 4) ? rowB : rowA) + t) * BLOCK_SLOTS + (u & 1) * 64;
-            const uint32_t to = ring + (uint32_t)(place * TILES_PER_GROUP) * TILE_BYTES + (uint32_t)u * 1024u;
-            load_to_lds(to, src, lane_bytes);
-        }
+        const int64_t from = (own + min(first_tile + (ROWS == 4 ? 0 : wave >> 1), NB - 1)) * BLOCK_SLOTS;
+        const uint32_t to = ring + (uint32_t)place * W::GROUP_BYTES + (uint32_t)wave * 4096u;
+        load_to_lds(to, p.k + from, lane_bytes);
+        load_to_lds(to + 1024u, p.k + from + 64, lane_bytes);
+        load_to_lds(to + 2048u, p.v + from, lane_bytes);
+        load_to_lds(to + 3072u, p.v + from + 64, lane_bytes);
     };
     request(0, 0);
-    request(TILES_PER_GROUP, 1);
-    int fill = 2, fill_tile = 2 * TILES_PER_GROUP; // the next group to ask for: its place in the ring, its first tile
+    request(W::TILES_PER_GROUP, 1);
+    int fill = 2, fill_tile = 2 * W::TILES_PER_GROUP; // the next group to ask for: its place in the ring, its first tile
+    // Behind the last keys each wave asks for the gates of its own queries, two rows at a time, four pieces as well, so that they wait
+    // in the ring when the loop ends (asked for there, they were a round trip at the end of every workgroup).
+    int gates = 0, gate_place = 0; // rows asked for; the place of the first two
     auto refill = [&] {
-        request(fill_tile, fill);
-        fill = fill == 2 ? 0 : fill + 1;
-        fill_tile += TILES_PER_GROUP;
+        if (fill_tile < NB) {
+            request(fill_tile, fill);
+        } else if (gates < ROWS && j < NB) {
+            gate_place = gates == 0 ? fill : gate_place;
+            const uint32_t to = ring + (uint32_t)fill * W::GROUP_BYTES + (uint32_t)wave * 4096u;
+            const uint4 *first = p.g + ((gates == 0 ? row[0] : row[ROWS - 2]) + j) * BLOCK_SLOTS;
+            const uint4 *second = p.g + ((gates == 0 ? row[1] : row[ROWS - 1]) + j) * BLOCK_SLOTS;
+            load_to_lds(to, first, lane_bytes);
+            load_to_lds(to + 1024u, first + 64, lane_bytes);
+            load_to_lds(to + 2048u, second, lane_bytes);
+            load_to_lds(to + 3072u, second + 64, lane_bytes);
+            gates += 2;
+        }
+        fill = fill == RING - 1 ? 0 : fill + 1;
+        fill_tile += W::TILES_PER_GROUP;
     };
     if (j >= NB) { // a wave without queries brings its share of the keys
-        for (int t = 0; t < NB; t += TILES_PER_GROUP) {
+        for (int t = 0; t < NB; t += W::TILES_PER_GROUP) {
             asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
             refill();
         }
@@ -324,17 +374,20 @@ __global__ __launch_bounds__(768) void streamed_attention_kernel(const StreamedP
         return;
     }
 
-    const uint4 *qa = p.q + (rowA + j) * BLOCK_SLOTS, *qb = p.q + (rowB + j) * BLOCK_SLOTS;
-    const bf16x8 qA0 = as_bf16x8(qa[lane]), qA1 = as_bf16x8(qa[64 + lane]), qB0 = as_bf16x8(qb[lane]), qB1 = as_bf16x8(qb[64 + lane]);
+    bf16x8 q[ROWS][2];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        const uint4 *src = p.q + (row[i] + j) * BLOCK_SLOTS;
+        q[i][0] = as_bf16x8(src[lane]), q[i][1] = as_bf16x8(src[64 + lane]);
+    }
     const f32x4 *nbc = HAS_NB ? p.tiles + ((int64_t)h * NB + j) * p.NT * 256 : nullptr;
-    const uint32_t *wordsA = p.words + (int64_t)bA * NB * 32, *wordsB = p.words + (int64_t)bB * NB * 32;
     auto load_nb = [&](int t) {
         f32x16 c = zero16();
         if constexpr (HAS_NB) {
-            const int tc = min(t, NB - 1);
+            const char *tile = reinterpret_cast<const char *>(nbc + min(t, NB - 1) * 256); // uniform; the lane's part in 32 bits
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
-                const f32x4 v = nbc[(tc * 4 + a) * 64 + lane];
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(tile + (lane_bytes + 1024u * a));
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     c[4 * a + e] = v[e];
@@ -345,11 +398,14 @@ __global__ __launch_bounds__(768) void streamed_attention_kernel(const StreamedP
     };
     f32x16 C0 = load_nb(0), C1 = load_nb(1);
 
-    // first key tile in which either row has a mask (the ragged tail of a row counts: its keys are at -inf)
+    // first key tile in which a row has a mask (the ragged tail of a row counts: its keys are at -inf)
     int masked_from = NB;
     for (int t0 = 0; t0 < NB; t0 += 64) {
-        const int t = t0 + lane;
-        const uint32_t f = t < NB ? (p.flags[(int64_t)bA * NB + t] | p.flags[(int64_t)bB * NB + t]) : 0u;
+        uint32_t f = 0;
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+            f |= t0 + lane < NB ? p.flags[(int64_t)b[i] * NB + t0 + lane] : 0u;
+        }
         const unsigned long long any = __ballot(f != 0u);
         if (any != 0) {
             masked_from = t0 + __builtin_ctzll(any);
@@ -357,10 +413,29 @@ __global__ __launch_bounds__(768) void streamed_attention_kernel(const StreamedP
         }
     }
 
+    // A row whose keys all have one mask (a padded residue's: -1e9 everywhere) would end with every exponential at zero.  Its logits
+    // are taken against that mask from the start: x = (q.k + bias + mask) - mask, each sum rounded, so that the mask absorbs what
+    // it absorbs in the reference.  shift: the word of the -mask, 0 for other rows.  Such rows used to be attended twice more, by
+    // attend_shifted: 2048 residues, 4 % of them padding, 1.4 ms of 8.0.
+    uint32_t shift[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        shift[i] = 0;
+        if (masked_from == 0) {
+            const uint32_t *flags = p.flags + (int64_t)b[i] * NB;
+            const uint32_t f = flags[0];
+            bool differs = f == MIXED_WORDS || f == 0;
+            for (int t0 = 0; t0 < NB && !differs; t0 += 64) {
+                differs = __any(flags[min(t0 + lane, NB - 1)] != f);
+            }
+            shift[i] = __builtin_amdgcn_readfirstlane(differs ? 0u : f ^ 0x80008000u);
+        }
+    }
+
     // The mask of a row as a rank-one MFMA: A holds (hi, lo) of the key of accumulator row i in k-slots 0 and 1, B ones there,
     // all else zero, also in the lanes of the upper half, so that an infinite mask value never meets a zero.
     const uint32_t lower = lane < 32 ? 0xffffffffu : 0u;
-    auto mask_word_of = [&](const uint32_t *words, int t) { return words[min(t, NB - 1) * 32 + (lane & 31)] & lower; };
+    auto mask_word_of = [&](int i, int t) { return p.words[((int64_t)b[i] * NB + min(t, NB - 1)) * 32 + (lane & 31)] & lower; };
     auto add_mask = [&](f32x16 x, uint32_t w) {
         const bf16x8 ones = as_bf16x8(make_uint4(0x3f803f80u & lower, 0u, 0u, 0u));
         return mfma(as_bf16x8(make_uint4(w, 0u, 0u, 0u)), ones, x);
@@ -368,85 +443,95 @@ __global__ __launch_bounds__(768) void streamed_attention_kernel(const StreamedP
 
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); // groups 0 and 1 have landed, every wave's part of them
     refill();
-    int left = TILES_PER_GROUP;                              // tiles of the current group still to come, this one included
-    const uint4 *cur = lds, *const end = lds + RING * TILES_PER_GROUP * TILE_SLOTS, *next = lds + TILE_SLOTS; // tiles t and t + 1
-    next = next == end ? lds : next;
-    uint4 k0 = cur[lane], k1 = cur[64 + lane], v0, v1;
-    f32x16 xa, xb;
-    xa = mfma(as_bf16x8(k0), qA0, C0);
-    xa = mfma(as_bf16x8(k1), qA1, xa);
-    k0 = cur[2 * BLOCK_SLOTS + lane], k1 = cur[2 * BLOCK_SLOTS + 64 + lane];
-    v0 = cur[BLOCK_SLOTS + lane], v1 = cur[BLOCK_SLOTS + 64 + lane];
-    f32x16 oA = zero16(), oB = zero16();
-    f32x4 sumsA = {0.f, 0.f, 0.f, 0.f}, sumsB = {0.f, 0.f, 0.f, 0.f}; // the row sums on the matrix pipe: see rowsum_selector
+    int left = W::TILES_PER_GROUP; // tiles of the current group still to come, this one included
+    const uint4 *cur = lds, *const end = lds + RING * W::TILES_PER_GROUP * W::TILE_SLOTS, *next = lds + W::TILE_SLOTS; // tiles t and t + 1
+    auto keys = [&](const uint4 *tile, int i) { return tile + i * 2 * BLOCK_SLOTS + lane; };
+    auto values = [&](const uint4 *tile, int i) { return tile + i * 2 * BLOCK_SLOTS + BLOCK_SLOTS + lane; };
+    uint4 k0 = keys(cur, 0)[0], k1 = keys(cur, 0)[64], v0, v1;
+    f32x16 x[2]; // logits: of row i in x[i & 1]
+    x[0] = mfma(as_bf16x8(k0), q[0][0], C0);
+    x[0] = mfma(as_bf16x8(k1), q[0][1], x[0]);
+    k0 = keys(cur, 1)[0], k1 = keys(cur, 1)[64];
+    v0 = values(cur, 0)[0], v1 = values(cur, 0)[64];
+    f32x16 o[ROWS];
+    f32x4 sums[ROWS]; // the row sums on the matrix pipe: see rowsum_selector
+    uint32_t m[ROWS]; // the mask words of a row's next logits
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        o[i] = zero16(), sums[i] = f32x4{0.f, 0.f, 0.f, 0.f}, m[i] = 0;
+    }
     const bf16x8 ones_rows = rowsum_selector(lane);
-    uint32_t mA = 0, mB = 0; // mask words of (A, t + 1) and (B, t)
 
     auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
-    // softmax and P.V of the finished logits xc (into o, sums); the logits of the next row and tile into xn from seed C with
-    // query fragments q0, q1; then k0, k1 <- knext.  The fences deal the exponentials between the MFMAs.  The empty asm keeps C
-    // live past the MFMA that reads it, so that xn gets registers of its own.
-    auto half_step = [&](f32x16 &xc, f32x16 &xn, const f32x16 &C, bf16x8 q0, bf16x8 q1, f32x16 &o, f32x4 &sums, const uint4 *knext,
-                         uint32_t mask_next, auto masked) {
-        auto exp4 = [&](int base) {
+    // Tile t with seed C: finishes row i = 0 .. ROWS - 1, each time softmax and P.V of the finished logits, the logits of the next row (of
+    // the first one and tile t + 1, from seed Cn, behind the last), and the fragments of the row behind that.  The fences deal the
+    // exponentials between the MFMAs.  The empty asm keeps C live past the MFMA that reads it, so that the logits get registers of their own.
+    auto tile = [&](int t, f32x16 &C, f32x16 &Cn, auto masked) __attribute__((always_inline)) {
 #pragma unroll
-            for (int e = base; e < base + 4; ++e) {
-                xc[e] = __builtin_amdgcn_exp2f(xc[e]);
+        for (int i = 0; i < ROWS; ++i) {
+            constexpr int LAST = ROWS - 1;
+            const int n = i == LAST ? 0 : i + 1, nn = (i + 2) % ROWS; // the next row, the one behind it
+            f32x16 &xc = x[i & 1], &xn = x[n & 1];
+            auto exp4 = [&](int base) {
+#pragma unroll
+                for (int e = base; e < base + 4; ++e) {
+                    xc[e] = __builtin_amdgcn_exp2f(xc[e]);
+                }
+            };
+            exp4(0);
+            if (i == LAST) {
+                xn = mfma(as_bf16x8(k0), q[n][0], Cn);
+                asm volatile("" ::"v"(Cn));
+            } else {
+                xn = mfma(as_bf16x8(k0), q[n][0], C);
+                asm volatile("" ::"v"(C));
             }
-        };
-        exp4(0);
-        xn = mfma(as_bf16x8(k0), q0, C);
-        asm volatile("" ::"v"(C));
-        fence();
-        exp4(4);
-        const bf16x8 p0 = pack8(xc, 0);
-        xn = mfma(as_bf16x8(k1), q1, xn);
-        if constexpr (decltype(masked)::value) {
-            xn = add_mask(xn, mask_next);
-        }
-        k0 = knext[lane], k1 = knext[64 + lane];
-        fence();
-        exp4(8);
-        o = mfma(as_bf16x8(v0), p0, o);
-        fence();
-        exp4(12);
-        const bf16x8 p1 = pack8(xc, 8);
-        sums = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p0, sums, 0, 0, 0);
-        o = mfma(as_bf16x8(v1), p1, o);
-        sums = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p1, sums, 0, 0, 0);
-        fence();
-    };
-    // Tile t: finishes (A, t) and (B, t), forms the logits of (B, t) from C and of (A, t + 1) from Cn
-    auto tile = [&](int t, f32x16 &C, f32x16 &Cn, auto masked) {
-        half_step(xa, xb, C, qB0, qB1, oA, sumsA, next, mB, masked);
-        v0 = cur[3 * BLOCK_SLOTS + lane], v1 = cur[3 * BLOCK_SLOTS + 64 + lane];
-        fence(); // the loads stay behind the last reader of the registers they fill
-        C = load_nb(t + 2);
-        if constexpr (decltype(masked)::value) {
-            mB = mask_word_of(wordsB, t + 1);
-        }
-        fence();
-        half_step(xb, xa, Cn, qA0, qA1, oB, sumsB, next + 2 * BLOCK_SLOTS, mA, masked);
-        v0 = next[BLOCK_SLOTS + lane], v1 = next[BLOCK_SLOTS + 64 + lane];
-        if constexpr (decltype(masked)::value) {
-            mA = mask_word_of(wordsA, t + 2);
+            fence();
+            exp4(4);
+            const bf16x8 p0 = pack8(xc, 0);
+            xn = mfma(as_bf16x8(k1), q[n][1], xn);
+            if constexpr (decltype(masked)::value) {
+                xn = add_mask(add_mask(xn, m[n]), shift[n] & lower);
+            }
+            const uint4 *kf = keys(i + 2 < ROWS ? cur : next, nn);
+            k0 = kf[0], k1 = kf[64];
+            fence();
+            exp4(8);
+            o[i] = mfma(as_bf16x8(v0), p0, o[i]);
+            fence();
+            exp4(12);
+            const bf16x8 p1 = pack8(xc, 8);
+            sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p0, sums[i], 0, 0, 0);
+            o[i] = mfma(as_bf16x8(v1), p1, o[i]);
+            sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p1, sums[i], 0, 0, 0);
+            fence();
+            const uint4 *vf = values(i == LAST ? next : cur, n);
+            v0 = vf[0], v1 = vf[64];
+            fence(); // the loads stay behind the last reader of the registers they fill
+            if (i == LAST - 1) {
+                C = load_nb(t + 2);
+            }
+            if constexpr (decltype(masked)::value) {
+                m[n] = mask_word_of(n, t + (i == LAST ? 2 : 1));
+            }
+            fence();
         }
         cur = next;
-        next += TILE_SLOTS;
+        next += W::TILE_SLOTS;
         next = next == end ? lds : next;
         if (--left == 0) {
             // This wave's pieces of the group behind the next one have landed: it asked for them a group ago, and with a
-            // pair bias its eight youngest loads are those of the last two tiles' bias, issued since.
+            // pair bias its youngest loads are those of the group's tiles' bias, issued since.
             if constexpr (HAS_NB) {
-                asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+                asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(4 * W::TILES_PER_GROUP) : "memory");
             } else {
                 asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
             }
             refill();
-            left = TILES_PER_GROUP;
+            left = W::TILES_PER_GROUP;
         }
     };
-    auto run = [&](int from, int to, auto masked) {
+    auto run = [&](int from, int to, auto masked) __attribute__((always_inline)) {
         int t = from;
         for (; t + 1 < to; t += 2) {
             tile(t, C0, C1, masked);
@@ -460,33 +545,140 @@ __global__ __launch_bounds__(768) void streamed_attention_kernel(const StreamedP
     };
     run(0, masked_from, std::false_type{});
     if (masked_from < NB) {
-        mB = mask_word_of(wordsB, masked_from), mA = mask_word_of(wordsA, masked_from + 1);
-        xa = add_mask(xa, mask_word_of(wordsA, masked_from));
+        x[0] = add_mask(add_mask(x[0], mask_word_of(0, masked_from)), shift[0] & lower);
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+            m[i] = mask_word_of(i, masked_from + (i == 0 ? 1 : 0));
+        }
         run(masked_from, NB, std::true_type{});
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // requests past the last tile: let them land before the LDS is given back
-    float lA = rowsum_fetch(sumsA, lane), lB = rowsum_fetch(sumsB, lane);
-    if (__any(!(lA > 1e-30f && lA < 1e30f))) {
-        attend_shifted<HAS_NB>(p.k + rowA * BLOCK_SLOTS, p.v + rowA * BLOCK_SLOTS, wordsA, nbc, qA0, qA1, NB, lane, oA, lA);
-    }
-    if (__any(!(lB > 1e-30f && lB < 1e30f))) {
-        attend_shifted<HAS_NB>(p.k + rowB * BLOCK_SLOTS, p.v + rowB * BLOCK_SLOTS, wordsB, nbc, qB0, qB1, NB, lane, oB, lB);
-    }
-    const int qpos = j * 32 + pi_row(lane & 31);
-    if (qpos < p.S) {
-        auto store = [&](int b, int64_t row, const f32x16 &o, float l) {
-            const uint4 *gf = p.g + (row + j) * BLOCK_SLOTS;
-            const bf16x8 g0 = as_bf16x8(gf[lane]), g1 = as_bf16x8(gf[64 + lane]);
-            f32x16 gv;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the gates, and requests past the last tile before the LDS is given back
+    uint32_t again = 0; // rows whose sums ran out of range
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                gv[i] = sigmoid_f32(to_f32(g0[i])), gv[8 + i] = sigmoid_f32(to_f32(g1[i]));
+    for (int i = 0; i < ROWS; ++i) {
+        const float l = rowsum_fetch(sums[i], lane);
+        const bool stored = i == 0 || ROWS * set + i < p.B;
+        if (__any(!(l > 1e-30f && l < 1e30f))) {
+            again |= stored ? 1u << i : 0u;
+        } else if (stored) {
+            const int place = i < 2 ? gate_place : (gate_place == RING - 1 ? 0 : gate_place + 1);
+            const uint4 *gate = lds + place * (W::GROUP_BYTES / 16) + wave * 256 + (i & 1) * 128 + lane;
+            store_average(p.q + (row[i] + j) * BLOCK_SLOTS + lane, gate[0], gate[64], o[i], l);
+        }
+    }
+    while (again != 0) {
+        const int i = __builtin_ctz(again), bi = ROWS * set + i;
+        again &= again - 1;
+        const int64_t at = ((int64_t)bi * p.H + h) * NB;
+        attend_shifted<HAS_NB>(p.k + at * BLOCK_SLOTS, p.v + at * BLOCK_SLOTS, p.words + (int64_t)bi * NB * 32, nbc, p.q + (at + j) * BLOCK_SLOTS,
+                               p.g + (at + j) * BLOCK_SLOTS, NB, lane);
+    }
+}
+
+// ---- the output projection ----
+//
+// act += avg . Wo^T + bo, row (b, s) of the product to row (b, s) of act, or transposed to row (s, b).  Bound by HBM: 2 C bytes a
+// position in, and 4 C of act.  The gated average arrives as MFMA fragments, 1 KB a load instruction, requested a block ahead; the
+// weights stay in the LDS with their head dims in the order of those fragments; the product (rows = features, columns =
+// positions) crosses the wave's panel to meet the activation in whole cache lines.  act, weights and bias lie on any address.
+template <int C>
+struct OutputShape {
+    static constexpr int SLABS = C / 128, WAVES = 4 * SLABS; // 128 features of Wo per slab; two workgroups a CU, or one of both slabs
+    static constexpr size_t LDS = (size_t)(SLABS * 4 * (C / 16) * 64 + WAVES * 256) * 16;
+};
+
+template <int C>
+__global__ __launch_bounds__(64 * OutputShape<C>::WAVES, C == 128 ? 2 : 1) void output_projection_kernel(
+    const uint4 *__restrict__ avg, const bf16_t *__restrict__ wo, const float *__restrict__ bo, bf16_t *__restrict__ act, int64_t ld,
+    int B, int S, int H, int NB, int transposed)
+{
+    constexpr int CK = C / 16, SLABS = OutputShape<C>::SLABS, W = OutputShape<C>::WAVES, THREADS = 64 * W;
+    extern __shared__ uint4 lds[]; // [4 SLABS feature blocks][CK][64 lanes], a panel per wave
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 31, g = lane >> 5;
+    uint4 *panel = lds + SLABS * 4 * CK * 64 + wave * 256;
+    const int blocks = B * NB, stride = (int)gridDim.x * W;
+    int block = (int)blockIdx.x * W + wave;
+    struct Rows {
+        uint4 f[CK];
+    };
+    auto load = [&](int at) { // the fragments of block `at` (of the last one past the end), k-steps 2 h and 2 h + 1 = head h
+        const int bl = min(at, blocks - 1), b = bl / NB, j = bl - b * NB;
+        const uint4 *src = avg + ((int64_t)b * H * NB + j) * BLOCK_SLOTS + lane;
+        Rows t;
+#pragma unroll
+        for (int h = 0; h < CK / 2; ++h) {
+            t.f[2 * h] = src[(int64_t)h * NB * BLOCK_SLOTS], t.f[2 * h + 1] = src[(int64_t)h * NB * BLOCK_SLOTS + 64];
+        }
+        return t;
+    };
+    Rows next = load(block);
+    for (int at = tid; at < SLABS * 4 * CK * 64; at += THREADS) {
+        // elements e of lane half g: head dims 16 ks + 4 g + e (e < 4), 16 ks + 8 + 4 g + e - 4
+        const int ln = at & 63, ks = (at >> 6) % CK, row = (at >> 6) / CK * 32 + (ln & 31);
+        const bf16_t *src = wo + row * C + ks * 16 + 4 * (ln >> 5);
+        uint64_t lo, hi;
+        __builtin_memcpy(&lo, src, 8);
+        __builtin_memcpy(&hi, src + 8, 8);
+        lds[at] = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+    }
+    __syncthreads();
+    // row (b, position) of the activation
+    const int64_t step = (transposed ? (int64_t)B : 1) * ld * 2, lane_part = (lane >> 3) * step + 16 * (lane & 7);
+    for (; block < blocks; block += stride) {
+        const Rows rows = next;
+        next = load(block + stride);
+        const int b = block / NB, j = block - b * NB;
+        char *base = reinterpret_cast<char *>(act) + (transposed ? (int64_t)32 * j * B + b : (int64_t)b * S + 32 * j) * ld * 2 + lane_part;
+        const int last = S - 1 - 32 * j; // last position of the block that is one, counted in it
+#pragma unroll 1
+        for (int slab = 0; slab < SLABS; ++slab) {
+#pragma unroll
+            for (int half = 0; half < 2; ++half) { // 64 features per panel
+                const int n0 = slab * 128 + half * 64;
+                uint4 z[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (8 * i + (lane >> 3) <= last) {
+                        __builtin_memcpy(&z[i], base + 8 * i * step + 2 * n0, 16);
+                    }
+                }
+                f32x16 acc[2];
+                acc[0] = zero16(), acc[1] = zero16();
+                const uint4 *w = lds + (slab * 4 + 2 * half) * CK * 64 + lane;
+#pragma unroll
+                for (int ks = 0; ks < CK; ++ks) {
+                    acc[0] = mfma(as_bf16x8(w[ks * 64]), as_bf16x8(rows.f[ks]), acc[0]);
+                    acc[1] = mfma(as_bf16x8(w[(CK + ks) * 64]), as_bf16x8(rows.f[ks]), acc[1]);
+                }
+#pragma unroll
+                for (int n = 0; n < 2; ++n) {
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) {
+                        f32x4 bv;
+                        __builtin_memcpy(&bv, bo + n0 + n * 32 + 8 * a + 4 * g, 16);
+                        bf16x4 ov;
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            ov[c] = (bf16_t)(acc[n][4 * a + c] + bv[c]);
+                        }
+                        *(reinterpret_cast<bf16x4 *>(panel + panel_slot(pi_row(r), n * 4 + a)) + g) = ov;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int pos = 8 * i + (lane >> 3);
+                    const bf16x8 o = as_bf16x8(panel[panel_slot(pos, lane & 7)]), x = as_bf16x8(z[i]);
+                    bf16x8 sum;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        sum[e] = (bf16_t)(to_f32(x[e]) + to_f32(o[e]));
+                    }
+                    if (pos <= last) {
+                        __builtin_memcpy(base + 8 * i * step + 2 * n0, &sum, 16);
+                    }
+                }
             }
-            store_gated(p.avg + (int64_t)b * p.avg_sb + (int64_t)qpos * p.avg_ss + h * HEAD + 4 * (lane >> 5), o, 1.0f / l, gv);
-        };
-        store(bA, rowA, oA, lA);
-        if (bB != bA) {
-            store(bB, rowB, oB, lB);
         }
     }
 }
@@ -506,19 +698,33 @@ int launch_projection(const StreamedParams &p, hipStream_t stream)
     return kutacc_hip_status(hipGetLastError());
 }
 
-template <bool HAS_NB>
+template <bool HAS_NB, int ROWS>
 int launch_attention(StreamedParams p, hipStream_t stream)
 {
-    constexpr size_t lds_bytes = (size_t)RING * TILES_PER_GROUP * TILE_BYTES;
-    const int pairs = (p.B + 1) / 2;
+    const int sets = (p.B + ROWS - 1) / ROWS;
     p.query_groups = (p.NB + WAVES - 1) / WAVES;
     const int parts = (p.query_groups + TOGETHER - 1) / TOGETHER, together = std::min(p.query_groups, TOGETHER);
-    p.group_rows = std::min(pairs, MEMBERS / together);
-    p.pair_groups = (pairs + p.group_rows - 1) / p.group_rows;
-    p.groups = p.pair_groups * p.H * parts;
+    p.group_rows = std::min(sets, MEMBERS / together);
+    p.set_groups = (sets + p.group_rows - 1) / p.group_rows;
+    p.groups = p.set_groups * p.H * parts;
     const int64_t blocks = (int64_t)(p.groups + 7) / 8 * 8 * p.group_rows * together;
     kutacc_prof::KernelTimer t("streamed_attention_kernel", 4.0 * (double)p.B * p.S * p.S * p.H * HEAD, stream);
-    streamed_attention_kernel<HAS_NB><<<dim3((unsigned)blocks), 64 * WAVES, lds_bytes, stream>>>(p);
+    streamed_attention_kernel<HAS_NB, ROWS><<<dim3((unsigned)blocks), 64 * WAVES, Walk<ROWS>::LDS, stream>>>(p);
+    return kutacc_hip_status(hipGetLastError());
+}
+
+template <int C>
+int launch_output(const StreamedParams &p, const void *wo, const float *bo, void *act, int64_t ld, bool transposed, hipStream_t stream)
+{
+    using Shape = OutputShape<C>;
+    static size_t configured[KUTACC_DEVICE_SLOTS] = {};
+    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&output_projection_kernel<C>), Shape::LDS, configured)) {
+        return kutacc_hip_status(e);
+    }
+    const int64_t blocks = (int64_t)p.B * p.NB, full = kutacc_cu_count() * (C == 128 ? 2 : 1);
+    kutacc_prof::KernelTimer t("output_projection_kernel<residual>", 2.0 * (double)p.B * p.S * C * C, stream);
+    output_projection_kernel<C><<<dim3((unsigned)std::min(full, (blocks + Shape::WAVES - 1) / Shape::WAVES)), 64 * Shape::WAVES, Shape::LDS, stream>>>(
+        p.q, (const bf16_t *)wo, bo, (bf16_t *)act, ld, p.B, p.S, p.H, p.NB, transposed ? 1 : 0);
     return kutacc_hip_status(hipGetLastError());
 }
 } // namespace
@@ -555,8 +761,7 @@ bool streamed_attention_supports(const kutacc_hip_attention_args_t &a)
     const int64_t C = a.nheads * a.head_size;
     return a.dtype == KUTACC_DTYPE_BF16 && a.head_size == HEAD && (C == 128 || C == 256) && a.seq_len > 0 && a.seq_len <= (1 << 20) &&
            a.batch > 0 && a.batch <= (1 << 24) && a.batch * blocks_of(a.seq_len) <= INT32_MAX / 4 && a.input_ld % 8 == 0 &&
-           kutacc_hip_aligned16(a.input) && a.avg_stride_h == HEAD && a.avg_stride_s % 8 == 0 && a.avg_stride_b == a.seq_len * a.avg_stride_s &&
-           kutacc_hip_aligned16(a.avg);
+           kutacc_hip_aligned16(a.input);
 }
 
 int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedAttentionOptions &opt, void *workspace, int64_t bytes,
@@ -586,30 +791,23 @@ int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedA
     const int64_t each = a.batch * row_bytes(S, C);
     p.q = (uint4 *)data, p.k = (uint4 *)(data + each), p.v = (uint4 *)(data + 2 * each), p.g = (uint4 *)(data + 3 * each);
     p.tiles = has_nb ? (const f32x4 *)ws : nullptr;
-    p.avg = (bf16_t *)a.avg, p.avg_sb = a.avg_stride_b, p.avg_ss = a.avg_stride_s;
     p.B = (int)a.batch, p.S = (int)S, p.H = (int)a.nheads, p.NB = (int)blocks_of(S), p.NT = (p.NB + 1) & ~1;
     p.words = (uint32_t *)words, p.flags = p.words + (int64_t)p.B * p.NB * 32;
     rc = C == 128 ? launch_projection<128>(p, stream) : launch_projection<256>(p, stream);
     if (rc == 0) {
-        rc = has_nb ? launch_attention<true>(p, stream) : launch_attention<false>(p, stream);
+        // Two rows a wave where four would leave CUs idle, below three workgroups to two CUs (8 heads of 1100 residues, whole block: 4, 8
+        // and 16 sequences 155, 167 and 187 us against 165, 172 and 192 on four rows a wave; 24 and 64: 223 and 347 against 206 and 336).
+        const int64_t fours = (a.batch + 3) / 4 * a.nheads * ((p.NB + WAVES - 1) / WAVES);
+        rc = !has_nb                             ? launch_attention<false, 2>(p, stream)
+             : 2 * fours >= 3 * kutacc_cu_count() ? launch_attention<true, 4>(p, stream)
+                                                  : launch_attention<true, 2>(p, stream);
     }
     if (rc != 0) {
         return rc;
     }
-    // The projection adds its result to the activation on the way out (2048 residues: 411 us and 674 us of residual pass
-    // before, 664 us together now).  Where it cannot (the activation, the output weights or bias not on 16 bytes), it leaves its result
-    // where q was, which no kernel reads any more, and a pass of its own adds it.
-    const int64_t M = a.batch * S;
     const bool transposed = opt.out_mode == FUSED_OUT_ADD_TRANSPOSED;
-    if (row_projection_supports(a.avg, a.avg_stride_s, a.output_w, a.output_b, a.out, a.out_ld, M, C, C)) {
-        return row_projection_residual(a.avg, a.avg_stride_s, a.output_w, a.output_b, a.out, a.out_ld, M, C, C, transposed ? S : 0, stream);
-    }
-    kutacc_hip_gemm_args_t g = {};
-    g.m = M, g.n = g.k = C, g.batches = 1, g.dtype = KUTACC_DTYPE_BF16, g.path = KUTACC_HIP_PATH_AUTO;
-    g.a = a.avg, g.a_stride_m = a.avg_stride_s, g.a_stride_k = 1, g.b = a.output_w, g.b_stride_n = C, g.b_stride_k = 1;
-    g.c = p.q, g.c_stride_m = C, g.bias = a.output_b, g.bias_axis = 1;
-    rc = pair_gemm(g, stream);
-    return rc != 0 ? rc : residual_add(a.out, p.q, transposed ? S : a.batch, transposed ? a.batch : S, C, transposed, KUTACC_DTYPE_BF16, stream);
+    return C == 128 ? launch_output<128>(p, a.output_w, a.output_b, a.out, a.out_ld, transposed, stream)
+                    : launch_output<256>(p, a.output_w, a.output_b, a.out, a.out_ld, transposed, stream);
 }
 
 } // namespace kutacc_launch

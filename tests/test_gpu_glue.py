@@ -491,6 +491,29 @@ def test_msa_attention_blocks_beyond_1024_keys(torch_cuda, column, n_seq, n_res,
     helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, column), "bf16", f"msa block {n_seq}x{n_res} heads={heads} column={column}")
 
 
+# two rows a wave (with and without pair bias), four (at least three workgroups to two CUs), one to three of a set's rows missing
+@pytest.mark.parametrize("column,n_seq,n_res,heads", [(False, 6, 70, 8), (True, 70, 7, 4), (False, 193, 33, 8), (False, 194, 65, 8), (False, 195, 32, 8)])
+def test_streamed_rows_of_one_mask_beside_others(torch_cuda, streamed_everywhere, column, n_seq, n_res, heads):
+    """Rows whose every key is masked attend uniformly, beside rows with some keys masked, or none, in one wave."""
+    torch = torch_cuda
+    c = msa_case(9800 + n_seq + n_res, n_seq, n_res, heads, 128)
+    mask = c["mask"].T if column else c["mask"]
+    mask[:] = 1.0
+    mask[1::3] = 0.0
+    mask[2::4, -(mask.shape[1] // 3):] = 0.0
+    mask[-1] = 0.0
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
+        device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
+    msa = dev(c["m"])
+    w = {k: dev(c[k]) for k in ("ln_gamma", "ln_beta", "wq", "wk", "wv", "wg", "bg", "wo", "bo")}
+    pair = None if column else {"pair_act": dev(c["z"]), "pair_ln_gamma": dev(c["pair_ln_gamma"]),
+                                "pair_ln_beta": dev(c["pair_ln_beta"]), "bias_w": dev(c["bias_w"])}
+    print(f"streamed rows of one mask {n_seq}x{n_res} heads={heads} column={column}", flush=True)
+    assert capi.MsaAttentionBlock(msa, dev(c["mask"]), w, heads, pair).run() == 0
+    torch.cuda.synchronize()
+    helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, column), "bf16", f"rows of one mask {n_seq}x{n_res} heads={heads} column={column}")
+
+
 @pytest.mark.parametrize("kind,n_seq,n_res,heads", [("triangle", 0, 1025, 4), ("row", 3, 1050, 8), ("column", 1030, 2, 4)])
 def test_blocks_beyond_1024_keys_take_weights_on_any_address(torch_cuda, kind, n_seq, n_res, heads):
     """The route of these blocks asks nothing of the weights' alignment: the same bits with every matrix and both biases one element
