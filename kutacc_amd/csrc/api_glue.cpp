@@ -196,18 +196,20 @@ int kutacc_hip_triangle_attention(const kutacc_hip_triangle_attention_args_t *a,
 
     const kutacc_hip_attention_args_t g = triangle_attention_call(a, ws, w, fused_ln);
     if (streamed) {
-        // LayerNorm + pair bias, with the tiles the attention reads where the producer can write them; the operator, which
-        // forms the mask bias from the pair mask itself and adds its result to the pair activation (transposed back for the
-        // ending node).
+        // Pair bias, with the tiles the attention reads where the producer can write them; the operator, which normalises the
+        // pair activation and forms the mask bias from the pair mask itself, and adds its result to the pair activation (transposed
+        // back for the ending node).
+        kutacc_hip_attention_args_t g = triangle_attention_call(a, ws, w, true);
         if (!kutacc_launch::streamed_attention_supports(g)) {
             return KUTACC_HIP_EUNSUPPORTED;
         }
         kutacc_launch::FusedAttentionOptions opt;
         opt.out_mode = ending ? kutacc_launch::FUSED_OUT_ADD_TRANSPOSED : kutacc_launch::FUSED_OUT_ADD;
         opt.bias_is_mask = true, opt.bias_stride_k = ending ? n : 1;
+        opt.ln_gamma = a->ln_gamma, opt.ln_beta = a->ln_beta, opt.ln_eps = a->ln_eps, opt.input_stride_b = ending ? c : n * c;
         const int nb_blocks = (int)((n + 31) / 32);
-        opt.nb_tiles_ready = kutacc_launch::pair_bias_writes_fragments(a->pair_act, a->bias_w, ws + w.z_norm, n, n, c, heads, KUTACC_DTYPE_BF16);
-        int rc = kutacc_launch::pair_bias(a->pair_act, a->ln_gamma, a->ln_beta, a->bias_w, ws + w.nb, ws + w.z_norm, n, n, c, heads,
+        opt.nb_tiles_ready = kutacc_launch::pair_bias_writes_fragments(a->pair_act, a->bias_w, nullptr, n, n, c, heads, KUTACC_DTYPE_BF16);
+        int rc = kutacc_launch::pair_bias(a->pair_act, a->ln_gamma, a->ln_beta, a->bias_w, ws + w.nb, nullptr, n, n, c, heads,
                                           a->ln_eps, KUTACC_DTYPE_BF16, ending, s, opt.nb_tiles_ready ? ws + w.q : nullptr, nb_blocks,
                                           (nb_blocks + 1) & ~1, 1);
         return rc != 0 ? rc : kutacc_launch::gating_attention_streamed(g, opt, ws + w.q, w.avg - w.q, s);
@@ -591,15 +593,16 @@ int kutacc_hip_msa_attention(const kutacc_hip_msa_attention_args_t *a, void *str
     hipStream_t s = kutacc_api::stream_or_default(stream);
     const kutacc_hip_attention_args_t g = msa_attention_call(a, ws, w, fused_ln);
     if (streamed) {
+        const kutacc_hip_attention_args_t g = msa_attention_call(a, ws, w, true);
         if (!kutacc_launch::streamed_attention_supports(g)) {
             return KUTACC_HIP_EUNSUPPORTED;
         }
         kutacc_launch::FusedAttentionOptions opt;
         opt.out_mode = column ? kutacc_launch::FUSED_OUT_ADD_TRANSPOSED : kutacc_launch::FUSED_OUT_ADD;
         opt.bias_is_mask = true, opt.bias_stride_k = column ? n_res : 1;
-        int rc = kutacc_launch::layernorm_rows(a->msa_act, c, a->ln_gamma, a->ln_beta, ws + w.m_norm, c, n_seq * n_res, c, a->ln_eps,
-                                               KUTACC_DTYPE_BF16, s, column ? n_seq : 0);
-        if (rc == 0 && !column) {
+        opt.ln_gamma = a->ln_gamma, opt.ln_beta = a->ln_beta, opt.ln_eps = a->ln_eps, opt.input_stride_b = column ? c : n_res * c;
+        int rc = 0;
+        if (!column) {
             const int nb_blocks = (int)((n_res + 31) / 32);
             opt.nb_tiles_ready =
                 kutacc_launch::pair_bias_writes_fragments(a->pair_act, a->bias_w, nullptr, n_res, n_res, a->c_z, heads, KUTACC_DTYPE_BF16);

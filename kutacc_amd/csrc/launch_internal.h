@@ -132,9 +132,10 @@ int gating_attention_fused(const kutacc_hip_attention_args_t &args, hipStream_t 
 // pair bias -> fp32 tiles in log2 units, [nheads][ceil(S/32)][ceil(S/32) rounded up to even][4][64 lanes] x 16 bytes
 int pair_bias_tiles(const kutacc_hip_attention_args_t &args, void *tiles, hipStream_t stream);
 
-// streamed_attention.hip: rows of any length, 128 or 256 channels in heads of 32, on a workspace of streamed_workspace_bytes()
+// streamed_attention.hip: rows of any length, 128 or 256 channels in heads of 32, normalised on the way in (opt.ln_gamma, ln_beta and
+// ln_eps; args.input with its strides is the un-normalised tensor), on a workspace of streamed_workspace_bytes()
 // (256-byte aligned) that starts with the tiles of the pair bias; opt.nb_tiles_ready: they lie there already.  args.q, k, v,
-// gate and avg are not used, weights, biases and args.out may lie on any address; the result is added to args.out (opt.out_mode FUSED_OUT_ADD or
+// gate and avg are not used, activations, weights and biases may lie on any address; the result is added to args.out (opt.out_mode FUSED_OUT_ADD or
 // FUSED_OUT_ADD_TRANSPOSED).
 bool streamed_attention_supports(const kutacc_hip_attention_args_t &args);
 int64_t streamed_workspace_bytes(int64_t batch, int64_t seq_len, int64_t nheads, bool pair_bias);

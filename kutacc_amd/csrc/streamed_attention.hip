@@ -40,8 +40,10 @@ constexpr uint32_t MIXED_WORDS = 1; // no word a row shares: a denormal mask bia
 constexpr int BLOCK_SLOTS = 128; // 16-byte slots of a fragment pair: 32 positions x 32 head dims
 
 struct StreamedParams {
-    const bf16_t *x; // first batch row of the slice
+    const bf16_t *x; // un-normalised
     int64_t x_ld, x_sb;
+    const float *ln_gamma, *ln_beta;
+    float ln_eps;
     const bf16_t *wq, *wk, *wv, *wg;
     const float *bg;
     const bf16_t *bias;
@@ -58,7 +60,7 @@ struct StreamedParams {
     // MIXED_WORDS otherwise
     uint32_t *flags;
     const f32x4 *tiles;   // pair bias: [head][query block][NT][4][64 lanes] (pair_bias_tiles_kernel)
-    int B, S, H, NB, NT; // batch rows of the slice, positions, heads, blocks, key tiles of `tiles` per query block
+    int B, S, H, NB, NT; // batch rows, positions, heads, blocks, key tiles of `tiles` per query block
     int query_groups, set_groups, groups, group_rows; // placement of the attention's workgroups
 };
 
@@ -66,15 +68,17 @@ struct StreamedParams {
 //
 // Bound by HBM: per position 2 C bytes in and 8 C out.  Eight waves, one workgroup per CU (and per 128 channels of outputs); a
 // wave owns one head's two matrices -- Q and gate, or K and V -- whose 32 x C blocks stay in its registers, and stages
-// eight of the 64 positions of a step into the shared stage, requested a step ahead.
+// eight of the 64 positions of a step into the shared stage, requested a step ahead and normalised on the way (a row's pieces lie
+// in neighbouring lanes), so that no pass writes and reads a normalised copy.
 template <int C>
-constexpr size_t projection_lds() { return (size_t)2 * 64 * (C / 8) * 16; }
+constexpr size_t projection_lds() { return (size_t)2 * 64 * (C / 8) * 16 + 12 * C; }
 
 template <int C>
 __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedParams p, int steps_per_group)
 {
     constexpr int CK = C / 16, SLOTS = C / 8, LOADS = 8 * SLOTS / 64, ROWS = 64 / SLOTS; // rows per load instruction
-    extern __shared__ uint4 lds[];                                                      // two stages of [64 positions][SLOTS]
+    extern __shared__ uint4 lds[]; // two stages of [64 positions][SLOTS], gamma, beta, gating bias
+    float *gamma = reinterpret_cast<float *>(lds + 2 * 64 * SLOTS), *beta = gamma + C, *gating = beta + C;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
     const int h = (int)blockIdx.y * 4 + (wave & 3);
@@ -107,18 +111,47 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
 #pragma unroll
         for (int u = 0; u < LOADS; ++u) {
             const int pos = min(32 * load_j + 8 * (wave & 3) + ROWS * u + lane / SLOTS, p.S - 1);
-            t.r[u] = *reinterpret_cast<const uint4 *>(base + ((int64_t)pos * p.x_ld * 2 + 16 * (lane % SLOTS)));
+            __builtin_memcpy(&t.r[u], base + ((int64_t)pos * p.x_ld * 2 + 16 * (lane % SLOTS)), 16); // on any address
         }
         advance(load_b, load_j);
         return t;
     };
-    auto park = [&](int s, const Rows &t) {
+    auto park = [&](int s, const Rows &t, int lane) {
 #pragma unroll
         for (int u = 0; u < LOADS; ++u) {
-            lds[s * 64 * SLOTS + slot(8 * wave + ROWS * u + lane / SLOTS, lane % SLOTS)] = t.r[u];
+            const bf16x8 in = as_bf16x8(t.r[u]);
+            float v[8], rstd, shift;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                v[e] = to_f32(in[e]);
+            }
+            group_stats<SLOTS>(v, __shfl(v[0], lane & ~(SLOTS - 1), 64), (float)C, p.ln_eps, rstd, shift);
+            bf16x8 out;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                out[e] = (bf16_t)fmaf(fmaf(v[e], rstd, shift), gamma[lane % SLOTS * 8 + e], beta[lane % SLOTS * 8 + e]);
+            }
+            lds[s * 64 * SLOTS + slot(8 * wave + ROWS * u + lane / SLOTS, lane % SLOTS)] = as_uint4(out);
         }
     };
+    // The masks of a step's two blocks are the business of waves 0 and 3, one each.  Whatever a step uses is asked for a step ahead and in
+    // front of the next rows: loads return in order, and a later one waited for would make the rows' wait a whole round trip.
+    const bool forms_masks = blockIdx.y == 0 && (wave == 0 || wave == 3);
+    int mask_b = (2 * first + (wave == 3)) / p.NB, mask_j = (2 * first + (wave == 3)) % p.NB;
+    auto load_mask = [&] {
+        const int key = min(32 * mask_j + pi_row(r), p.S - 1);
+        const bf16_t m = p.bias[(int64_t)min(mask_b, p.B - 1) * p.bias_sb + (int64_t)key * p.bias_sk];
+        advance(mask_b, mask_j);
+        return m;
+    };
+    bf16_t mask = (bf16_t)0.f;
+    if (forms_masks) {
+        mask = load_mask();
+    }
     Rows rows = load();
+    for (int c = tid; c < C; c += 512) {
+        gamma[c] = p.ln_gamma[c], beta[c] = p.ln_beta[c], gating[c] = p.bg[c];
+    }
     bf16x8 w0[CK], w1[CK]; // Q and gate, or K and V
     {
         const bf16_t *m0 = forms_kv ? p.wk : p.wq, *m1 = forms_kv ? p.wv : p.wg;
@@ -128,83 +161,115 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
             w0[ks] = as_bf16x8(load8_any(m0, at)), w1[ks] = as_bf16x8(load8_any(m1, at)); // once per workgroup: on any address
         }
     }
-    park(0, rows);
+    __syncthreads();
+    park(0, rows, lane);
+    bf16_t next_mask = (bf16_t)0.f;
     if (first + 1 < stop) {
+        next_mask = forms_masks ? load_mask() : next_mask;
         rows = load();
     }
     __syncthreads();
+    // The weights are waited for here: waits that the compiler leaves to their first uses stand in the loop, where they are waits for
+    // every load and store on its way (with the stores of a step counted below, 2048 residues 1289 -> 1165 us, 5.4 GB
+    // at 4.6 TB/s; 1024 sequences x 384 residues of 256 channels 261 -> 240 us).
+#pragma unroll
+    for (int ks = 0; ks < CK; ++ks) {
+        asm volatile("" ::"v"(w0[ks]), "v"(w1[ks]));
+    }
 
     int b = (2 * first) / p.NB, j = (2 * first) % p.NB; // the block being multiplied
-    for (int step = first; step < stop; ++step) {
-        const int s = (step - first) & 1;
-        if (step + 1 < stop) {
-            park(s ^ 1, rows);
-            if (step + 2 < stop) {
-                rows = load();
+    auto steps = [&](auto kv) {
+        for (int step = first; step < stop; ++step) {
+            const int s = (step - first) & 1;
+            // With 256 channels the lane index is opaque to the optimiser, so that addresses are formed per step: kept across the loop
+            // beside the weights they would be spilled, and a reload waits for every load on its way.
+            int lv = tid & 63;
+            if constexpr (C == 256) {
+                asm volatile("" : "+v"(lv));
             }
-        }
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            if (2 * step + half >= blocks) {
-                break;
+            const int r = lv & 31, g = lv >> 5, lane = lv;
+            bf16_t after_next = (bf16_t)0.f;
+            auto stage_next = [&] {
+                if (step + 1 < stop) {
+                    park(s ^ 1, rows, lane);
+                    after_next = forms_masks ? load_mask() : after_next;
+                    rows = load();
+                }
+            };
+            // The two waves of a SIMD start a step together: one normalises while the other multiplies.
+            if constexpr (!decltype(kv)::value) {
+                stage_next();
             }
-            const uint4 *stage = lds + (s * 64 + 32 * half) * SLOTS;
-            f32x16 a0 = zero16(), a1 = zero16();
-            const int64_t at = (((int64_t)b * p.H + h) * p.NB + j) * BLOCK_SLOTS + lane;
-            if (forms_kv) {
 #pragma unroll
-                for (int ks = 0; ks < CK; ++ks) {
-                    const bf16x8 xf = as_bf16x8(stage[slot(pi_row(r), 2 * ks + g)]);
-                    a0 = mfma(w0[ks], xf, a0);
-                    a1 = mfma(xf, w1[ks], a1); // V: rows = keys, columns = head dims
+            for (int half = 0; half < 2; ++half) {
+                // Behind an odd number of blocks the last one again: every step has the same stores, so that the wait for the next rows lets
+                // them be on their way.
+                const uint4 *stage = lds + (s * 64 + (2 * step + half < blocks ? 32 * half : 0)) * SLOTS;
+                f32x16 a0 = zero16(), a1 = zero16();
+                const int64_t at = (((int64_t)b * p.H + h) * p.NB + j) * BLOCK_SLOTS + lane;
+                if constexpr (decltype(kv)::value) {
+#pragma unroll
+                    for (int ks = 0; ks < CK; ++ks) {
+                        const bf16x8 xf = as_bf16x8(stage[slot(pi_row(r), 2 * ks + g)]);
+                        a0 = mfma(w0[ks], xf, a0);
+                        a1 = mfma(xf, w1[ks], a1); // V: rows = keys, columns = head dims
+                    }
+                    p.k[at] = as_uint4(pack8(a0, 0)), p.k[at + 64] = as_uint4(pack8(a0, 8));
+                    p.v[at] = as_uint4(pack8(a1, 0)), p.v[at + 64] = as_uint4(pack8(a1, 8));
+                } else {
+#pragma unroll
+                    for (int ks = 0; ks < CK; ++ks) {
+                        const bf16x8 xf = as_bf16x8(stage[slot(pi_row(r), 2 * ks + g)]);
+                        a0 = mfma(w0[ks], xf, a0);
+                        a1 = mfma(w1[ks], xf, a1);
+                    }
+                    const float *bg = gating + h * HEAD + 4 * g;
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) {
+                        const f32x4 bv = *reinterpret_cast<const f32x4 *>(bg + 8 * a);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            a0[4 * a + c] *= p.qmul;
+                            a1[4 * a + c] += bv[c]; // the gate is rounded in front of its sigmoid, as where the reference stores it
+                        }
+                    }
+                    p.q[at] = as_uint4(pack8(a0, 0)), p.q[at + 64] = as_uint4(pack8(a0, 8));
+                    p.g[at] = as_uint4(pack8(a1, 0)), p.g[at + 64] = as_uint4(pack8(a1, 8));
                 }
-                p.k[at] = as_uint4(pack8(a0, 0)), p.k[at + 64] = as_uint4(pack8(a0, 8));
-                p.v[at] = as_uint4(pack8(a1, 0)), p.v[at + 64] = as_uint4(pack8(a1, 8));
-            } else {
-#pragma unroll
-                for (int ks = 0; ks < CK; ++ks) {
-                    const bf16x8 xf = as_bf16x8(stage[slot(pi_row(r), 2 * ks + g)]);
-                    a0 = mfma(w0[ks], xf, a0);
-                    a1 = mfma(w1[ks], xf, a1);
-                }
-                const float *bg = p.bg + h * HEAD + 4 * g;
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    f32x4 bv;
-                    __builtin_memcpy(&bv, bg + 8 * a, 16); // on any address
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        a0[4 * a + c] *= p.qmul;
-                        a1[4 * a + c] += bv[c]; // the gate is rounded in front of its sigmoid, as where the reference stores it
+                if (!decltype(kv)::value && forms_masks && wave == 3 * half && 2 * step + half < blocks) {
+                    const int key = 32 * j + pi_row(r);
+                    float mv = -INFINITY;
+                    if (key < p.S) {
+                        mv = to_f32(mask);
+                        if (p.bias_is_mask) {
+                            mv = to_f32((bf16_t)fmaf(mv, 1e9f, -1e9f));
+                        }
+                        mv *= LOG2E;
+                    }
+                    const uint32_t word = mask_word(mv), first_word = __builtin_amdgcn_readfirstlane(word); // lane 0: key 32 j
+                    if (lane < 32) {
+                        p.words[((int64_t)b * p.NB + j) * 32 + lane] = word;
+                    }
+                    const bool any = __ballot(mv != 0.f) != 0, mixed = __ballot(key < p.S && word != first_word) != 0 || first_word == 0;
+                    if (lane == 0) {
+                        p.flags[(int64_t)b * p.NB + j] = !any ? 0u : (mixed ? MIXED_WORDS : first_word);
                     }
                 }
-                p.q[at] = as_uint4(pack8(a0, 0)), p.q[at + 64] = as_uint4(pack8(a0, 8));
-                p.g[at] = as_uint4(pack8(a1, 0)), p.g[at + 64] = as_uint4(pack8(a1, 8));
-            }
-            if (wave == 3 * half && blockIdx.y == 0) { // the mask of the block, by two waves in turn
-                const int key = 32 * j + pi_row(r);
-                float mv = -INFINITY;
-                if (key < p.S) {
-                    mv = to_f32(p.bias[(int64_t)b * p.bias_sb + (int64_t)key * p.bias_sk]);
-                    if (p.bias_is_mask) {
-                        mv = to_f32((bf16_t)fmaf(mv, 1e9f, -1e9f));
-                    }
-                    mv *= LOG2E;
-                }
-                const uint32_t word = mask_word(mv), first_word = __builtin_amdgcn_readfirstlane(word); // lane 0: key 32 j
-                if (lane < 32) {
-                    p.words[((int64_t)b * p.NB + j) * 32 + lane] = word;
-                }
-                const bool any = __ballot(mv != 0.f) != 0, mixed = __ballot(key < p.S && word != first_word) != 0 || first_word == 0;
-                if (lane == 0) {
-                    p.flags[(int64_t)b * p.NB + j] = !any ? 0u : (mixed ? MIXED_WORDS : first_word);
+                if (2 * step + half + 1 < blocks && ++j == p.NB) {
+                    j = 0, ++b;
                 }
             }
-            if (++j == p.NB) {
-                j = 0, ++b;
+            if constexpr (decltype(kv)::value) {
+                stage_next();
             }
+            mask = next_mask, next_mask = after_next;
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); // the next stage is complete, this one no longer read
         }
-        __syncthreads(); // the next stage is complete, this one no longer read
+    };
+    if (forms_kv) { // two loops, so that the waits of each are those of its own loads and stores
+        steps(std::true_type{});
+    } else {
+        steps(std::false_type{});
     }
 }
 
@@ -227,11 +292,11 @@ struct Walk {
 __device__ __forceinline__ void store_average(uint4 *dst, uint4 gate0, uint4 gate1, const f32x16 &o, float l)
 {
     const bf16x8 g0 = as_bf16x8(gate0), g1 = as_bf16x8(gate1);
-    const float inv = 1.0f / l;
     f32x16 out;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        out[i] = o[i] * inv * sigmoid_fast(to_f32(g0[i])), out[8 + i] = o[8 + i] * inv * sigmoid_fast(to_f32(g1[i]));
+    for (int i = 0; i < 16; ++i) { // l (1 + 2^(-gate log2 e)): one reciprocal for the sum and the sigmoid
+        const float e = __builtin_amdgcn_exp2f(to_f32(i < 8 ? g0[i & 7] : g1[i & 7]) * -LOG2E);
+        out[i] = o[i] * __builtin_amdgcn_rcpf(fmaf(e, l, l));
     }
     dst[0] = as_uint4(pack8(out, 0)), dst[64] = as_uint4(pack8(out, 8));
 }
@@ -597,13 +662,16 @@ __global__ __launch_bounds__(64 * OutputShape<C>::WAVES, C == 128 ? 2 : 1) void 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
     uint4 *panel = lds + SLABS * 4 * CK * 64 + wave * 256;
-    const int blocks = B * NB, stride = (int)gridDim.x * W;
-    int block = (int)blockIdx.x * W + wave;
+    // A unit is a block of positions and a slab.  With two slabs a wave takes a run of units: what some waves have more than others is
+    // half a block.  With one, neighbouring waves take neighbouring blocks (1024 residues 137 us, in runs 150).
+    const int units = B * NB * SLABS, waves = (int)gridDim.x * W, me = (int)blockIdx.x * W + wave;
+    const int stride = SLABS == 1 ? waves : 1, first = SLABS == 1 ? me : (int)((int64_t)units * me / waves);
+    const int stop = SLABS == 1 ? units : (int)((int64_t)units * (me + 1) / waves);
     struct Rows {
         uint4 f[CK];
     };
-    auto load = [&](int at) { // the fragments of block `at` (of the last one past the end), k-steps 2 h and 2 h + 1 = head h
-        const int bl = min(at, blocks - 1), b = bl / NB, j = bl - b * NB;
+    auto load = [&](int unit) { // the fragments of a unit's block, k-steps 2 h and 2 h + 1 = head h
+        const int block = min(unit, units - 1) / SLABS, b = block / NB, j = block - b * NB;
         const uint4 *src = avg + ((int64_t)b * H * NB + j) * BLOCK_SLOTS + lane;
         Rows t;
 #pragma unroll
@@ -612,7 +680,31 @@ __global__ __launch_bounds__(64 * OutputShape<C>::WAVES, C == 128 ? 2 : 1) void 
         }
         return t;
     };
-    Rows next = load(block);
+    // a unit's 64 features `half` of the activation: row (b, position), pieces of lane / 8 + 8 i
+    const int64_t step = (transposed ? (int64_t)B : 1) * ld * 2;
+    struct Where {
+        char *base; // lane's piece of position 32 j
+        int last;   // last position of the block that is one, counted in it
+    };
+    auto where = [&](int unit) {
+        const int at = min(unit, units - 1), block = at / SLABS, b = block / NB, j = block - b * NB;
+        const int64_t row = transposed ? (int64_t)32 * j * B + b : (int64_t)b * S + 32 * j;
+        return Where{reinterpret_cast<char *>(act) + row * ld * 2 + (at % SLABS) * 256 + 16 * (lane & 7), min(31, S - 1 - 32 * j)};
+    };
+    struct Piece {
+        uint4 z[4];
+    };
+    auto load_act = [&](const Where &w, int half) {
+        Piece t;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            __builtin_memcpy(&t.z[i], w.base + min(8 * i + (lane >> 3), w.last) * step + 128 * half, 16);
+        }
+        return t;
+    };
+    Rows next = load(first);
+    Where here = where(first);
+    Piece z = load_act(here, 0); // the activation arrives a half ahead of the result it is added to
     for (int at = tid; at < SLABS * 4 * CK * 64; at += THREADS) {
         // elements e of lane half g: head dims 16 ks + 4 g + e (e < 4), 16 ks + 8 + 4 g + e - 4
         const int ln = at & 63, ks = (at >> 6) % CK, row = (at >> 6) / CK * 32 + (ln & 31);
@@ -623,60 +715,62 @@ __global__ __launch_bounds__(64 * OutputShape<C>::WAVES, C == 128 ? 2 : 1) void 
         lds[at] = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
     }
     __syncthreads();
-    // row (b, position) of the activation
-    const int64_t step = (transposed ? (int64_t)B : 1) * ld * 2, lane_part = (lane >> 3) * step + 16 * (lane & 7);
-    for (; block < blocks; block += stride) {
+    for (int unit = first; unit < stop; unit += stride) {
         const Rows rows = next;
-        next = load(block + stride);
-        const int b = block / NB, j = block - b * NB;
-        char *base = reinterpret_cast<char *>(act) + (transposed ? (int64_t)32 * j * B + b : (int64_t)b * S + 32 * j) * ld * 2 + lane_part;
-        const int last = S - 1 - 32 * j; // last position of the block that is one, counted in it
-#pragma unroll 1
-        for (int slab = 0; slab < SLABS; ++slab) {
+        const Where at = here;
+        const int slab = unit % SLABS;
+        here = where(unit + stride);
 #pragma unroll
-            for (int half = 0; half < 2; ++half) { // 64 features per panel
-                const int n0 = slab * 128 + half * 64;
-                uint4 z[4];
+        for (int half = 0; half < 2; ++half) { // 64 features per panel
+            f32x16 acc[2]; // from the bias; its loads in front of those for the next half, which are still on their way when it is used
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if (8 * i + (lane >> 3) <= last) {
-                        __builtin_memcpy(&z[i], base + 8 * i * step + 2 * n0, 16);
+            for (int n = 0; n < 2; ++n) {
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    f32x4 bv;
+                    __builtin_memcpy(&bv, bo + slab * 128 + half * 64 + n * 32 + 8 * a + 4 * g, 16);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        acc[n][4 * a + c] = bv[c];
                     }
                 }
-                f32x16 acc[2];
-                acc[0] = zero16(), acc[1] = zero16();
-                const uint4 *w = lds + (slab * 4 + 2 * half) * CK * 64 + lane;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const Piece in = z;
+            z = half == 0 ? load_act(at, 1) : load_act(here, 0);
+            if (half == 0 && (SLABS == 1 || slab == SLABS - 1)) { // else the next unit is of the same block
+                next = load(unit + stride);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const uint4 *w = lds + (slab * 4 + 2 * half) * CK * 64 + lane;
 #pragma unroll
-                for (int ks = 0; ks < CK; ++ks) {
-                    acc[0] = mfma(as_bf16x8(w[ks * 64]), as_bf16x8(rows.f[ks]), acc[0]);
-                    acc[1] = mfma(as_bf16x8(w[(CK + ks) * 64]), as_bf16x8(rows.f[ks]), acc[1]);
+            for (int ks = 0; ks < CK; ++ks) {
+                acc[0] = mfma(as_bf16x8(w[ks * 64]), as_bf16x8(rows.f[ks]), acc[0]);
+                acc[1] = mfma(as_bf16x8(w[(CK + ks) * 64]), as_bf16x8(rows.f[ks]), acc[1]);
+            }
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    bf16x4 ov;
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        ov[c] = (bf16_t)acc[n][4 * a + c];
+                    }
+                    *(reinterpret_cast<bf16x4 *>(panel + panel_slot(pi_row(r), n * 4 + a)) + g) = ov;
                 }
+            }
 #pragma unroll
-                for (int n = 0; n < 2; ++n) {
+            for (int i = 0; i < 4; ++i) {
+                const int pos = 8 * i + (lane >> 3);
+                const bf16x8 o = as_bf16x8(panel[panel_slot(pos, lane & 7)]), x = as_bf16x8(in.z[i]);
+                bf16x8 sum;
 #pragma unroll
-                    for (int a = 0; a < 4; ++a) {
-                        f32x4 bv;
-                        __builtin_memcpy(&bv, bo + n0 + n * 32 + 8 * a + 4 * g, 16);
-                        bf16x4 ov;
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) {
-                            ov[c] = (bf16_t)(acc[n][4 * a + c] + bv[c]);
-                        }
-                        *(reinterpret_cast<bf16x4 *>(panel + panel_slot(pi_row(r), n * 4 + a)) + g) = ov;
-                    }
+                for (int e = 0; e < 8; ++e) {
+                    sum[e] = (bf16_t)(to_f32(x[e]) + to_f32(o[e]));
                 }
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int pos = 8 * i + (lane >> 3);
-                    const bf16x8 o = as_bf16x8(panel[panel_slot(pos, lane & 7)]), x = as_bf16x8(z[i]);
-                    bf16x8 sum;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        sum[e] = (bf16_t)(to_f32(x[e]) + to_f32(o[e]));
-                    }
-                    if (pos <= last) {
-                        __builtin_memcpy(base + 8 * i * step + 2 * n0, &sum, 16);
-                    }
+                if (pos <= at.last) {
+                    __builtin_memcpy(at.base + pos * step + 128 * half, &sum, 16);
                 }
             }
         }
@@ -721,9 +815,9 @@ int launch_output(const StreamedParams &p, const void *wo, const float *bo, void
     if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&output_projection_kernel<C>), Shape::LDS, configured)) {
         return kutacc_hip_status(e);
     }
-    const int64_t blocks = (int64_t)p.B * p.NB, full = kutacc_cu_count() * (C == 128 ? 2 : 1);
+    const int64_t units = (int64_t)p.B * p.NB * Shape::SLABS, full = kutacc_cu_count() * (C == 128 ? 2 : 1);
     kutacc_prof::KernelTimer t("output_projection_kernel<residual>", 2.0 * (double)p.B * p.S * C * C, stream);
-    output_projection_kernel<C><<<dim3((unsigned)std::min(full, (blocks + Shape::WAVES - 1) / Shape::WAVES)), 64 * Shape::WAVES, Shape::LDS, stream>>>(
+    output_projection_kernel<C><<<dim3((unsigned)std::min(full, (units + Shape::WAVES - 1) / Shape::WAVES)), 64 * Shape::WAVES, Shape::LDS, stream>>>(
         p.q, (const bf16_t *)wo, bo, (bf16_t *)act, ld, p.B, p.S, p.H, p.NB, transposed ? 1 : 0);
     return kutacc_hip_status(hipGetLastError());
 }
@@ -760,8 +854,7 @@ bool streamed_attention_supports(const kutacc_hip_attention_args_t &a)
 {
     const int64_t C = a.nheads * a.head_size;
     return a.dtype == KUTACC_DTYPE_BF16 && a.head_size == HEAD && (C == 128 || C == 256) && a.seq_len > 0 && a.seq_len <= (1 << 20) &&
-           a.batch > 0 && a.batch <= (1 << 24) && a.batch * blocks_of(a.seq_len) <= INT32_MAX / 4 && a.input_ld % 8 == 0 &&
-           kutacc_hip_aligned16(a.input);
+           a.batch > 0 && a.batch <= (1 << 24) && a.batch * blocks_of(a.seq_len) <= INT32_MAX / 4;
 }
 
 int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedAttentionOptions &opt, void *workspace, int64_t bytes,
@@ -769,7 +862,7 @@ int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedA
 {
     const int64_t C = a.nheads * a.head_size, S = a.seq_len;
     const bool has_nb = a.nonbatched_bias != nullptr;
-    if (!streamed_attention_supports(a) || opt.out_mode == FUSED_OUT_STORE || opt.ln_gamma != nullptr) {
+    if (!streamed_attention_supports(a) || opt.out_mode == FUSED_OUT_STORE || opt.ln_gamma == nullptr) {
         return KUTACC_HIP_EUNSUPPORTED;
     }
     if (bytes < streamed_workspace_bytes(a.batch, S, a.nheads, has_nb)) {
@@ -783,6 +876,7 @@ int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedA
     StreamedParams p;
     std::memset(&p, 0, sizeof(p));
     p.x = (const bf16_t *)a.input, p.x_ld = a.input_ld, p.x_sb = opt.input_stride_b != 0 ? opt.input_stride_b : S * a.input_ld;
+    p.ln_gamma = opt.ln_gamma, p.ln_beta = opt.ln_beta, p.ln_eps = opt.ln_eps;
     p.wq = (const bf16_t *)a.query_w, p.wk = (const bf16_t *)a.key_w, p.wv = (const bf16_t *)a.value_w, p.wg = (const bf16_t *)a.gating_w;
     p.bg = a.gating_b;
     p.bias = (const bf16_t *)a.bias, p.bias_sb = a.bias_stride_b, p.bias_sk = opt.bias_stride_k, p.bias_is_mask = opt.bias_is_mask ? 1 : 0;
