@@ -107,7 +107,8 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
     // repeats the row's last position, steps past the end repeat the last row: valid addresses, results masked or dropped.
     struct Rows {
         uint4 r[2];
-        uint16_t m; // mask of position lane % 8 of the eight
+        uint16_t m; // mask of position lane % 8 of the eight, if there is such a position
+        bool there;
     };
     Place at = place_of((uint32_t)(first * STEP + 8 * wave), (uint32_t)np);
     auto load = [&](Rows &t) {
@@ -120,8 +121,8 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
             t.r[u] = *reinterpret_cast<const uint4 *>(row + ((uint32_t)j * (2u * C) + 16u * (lane & 15)));
         }
         const int jm = at.j + (lane & 7);
-        const uint16_t m = reinterpret_cast<const uint16_t *>(mask)[(int64_t)i * n + min(jm, n - 1)];
-        t.m = there && jm < n ? m : (uint16_t)0;
+        t.m = reinterpret_cast<const uint16_t *>(mask)[(int64_t)i * n + min(jm, n - 1)];
+        t.there = there && jm < n;
         advance(at, np);
     };
     float gm[8], bt[8];
@@ -131,7 +132,7 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
             lds[s * FRONT_STAGE + row_slot(8 * wave + 4 * u + (lane >> 4), lane & 15)] = normalise_row(t.r[u], lane, gm, bt, eps);
         }
         if (lane < 8) {
-            mask_rows[s * STEP + 8 * wave + lane] = t.m;
+            mask_rows[s * STEP + 8 * wave + lane] = t.there ? t.m : (uint16_t)0;
         }
     };
 
@@ -152,11 +153,18 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
     bf16_t *out = sd.out + (int64_t)cb * 32 * plane;
     stage_rows(even, 0);
     __syncthreads();
+    // The weights are waited for here: the waits that the compiler leaves to their first uses stand in the loop, where they are waits for
+    // all rows and stores on their way.  With them, a mask that was waited for where it was loaded, and loads and stores that some steps
+    // did without, 384 residues 42.0 -> 38.4 us (2.9 TB/s), 691 residues 127 -> 106 us (3.5 TB/s); what is left is the vector
+    // work of two waves a SIMD.
+#pragma unroll
+    for (int ks = 0; ks < CK; ++ks) {
+        asm volatile("" ::"v"(wp[ks]), "v"(wg[ks]));
+    }
+    asm volatile("" ::"v"(pbias), "v"(gneg));
 
     auto do_step = [&](int step, int s, Rows &next, Rows &after) {
-        if (step + 2 < stop) {
-            load(after);
-        }
+        load(after); // (behind the last step as well: every step has the same loads and stores, and the wait for `next` lets them fly)
         if (step + 1 < stop) {
             stage_rows(next, s ^ 1);
         }
@@ -214,14 +222,12 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
                 *(reinterpret_cast<bf16x4 *>(panel + panel_slot(rv, rb * 4 + a)) + gv) = ov;
             }
         }
-        // 32 channels x eight 16-byte pieces of 8 positions
-        const int piece = lane & 7;
-        if (step * STEP + 8 * piece < positions) {
+        // 32 channels x eight 16-byte pieces of 8 positions; pieces past the last one repeat it
+        const int piece = min(lane & 7, (positions - 1 - step * STEP) >> 3);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int ch = 8 * i + (lane >> 3);
-                *reinterpret_cast<uint4 *>(out + (int64_t)ch * plane + step * STEP + 8 * piece) = panel[panel_slot(ch, piece)];
-            }
+        for (int i = 0; i < 4; ++i) {
+            const int ch = 8 * i + (lane >> 3);
+            *reinterpret_cast<uint4 *>(out + (int64_t)ch * plane + step * STEP + 8 * piece) = panel[panel_slot(ch, piece)];
         }
         __syncthreads(); // the other stage is complete, this one no longer read
     };
