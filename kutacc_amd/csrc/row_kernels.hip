@@ -378,9 +378,12 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
 // row and writes 16), so the weights stay in the LDS as MFMA fragments, padded with zeros to whole blocks of 32 outputs, and every
 // wave streams 32 rows at a time: whole cache lines in through its panel, the next rows requested before the current ones are
 // multiplied, 64 outputs at a time out through the same panel.  A lane ends up with one row and four consecutive outputs per
-// accumulator group.  147 456 rows x 128 -> 8: 54.5 us on the scalar kernel, 11.1 us here.
-template <int K>
-__global__ __launch_bounds__(256) void linear_rows_kernel(const bf16_t *__restrict__ act, int64_t ld_act, const bf16_t *__restrict__ w,
+// accumulator group.  The addition of beta * result is a kernel of its own (its sixteen guarded loads per block of outputs are sixteen
+// branches, taken or not), groups of eight outputs past n are skipped, and with 128 registers four workgroups share a CU up to 128
+// features.  The call, us: 147 456 rows x 128 -> 8 54.5 on the scalar kernel, 9.8 without these, 8.0 here (5.0 TB/s); 100 000
+// x 128 -> 128 19.1 -> 15.7; 300 000 x 256 -> 256 105.5 -> 98.2.
+template <int K, bool BETA>
+__global__ __launch_bounds__(256, K == 256 ? 2 : 4) void linear_rows_kernel(const bf16_t *__restrict__ act, int64_t ld_act, const bf16_t *__restrict__ w,
                                                           int64_t ld_w, const float *__restrict__ bias, bf16_t *__restrict__ out, int64_t m,
                                                           int ld_out, int slice, float beta, int piece)
 {
@@ -462,14 +465,17 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(const bf16_t *__restri
                 }
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
+                    if (fb + 8 * a >= n) {
+                        break;
+                    }
                     const int f = fb + 8 * a + 4 * g;
                     const kutacc_dev::f32x4 bv = *reinterpret_cast<const kutacc_dev::f32x4 *>(bias_s + f);
                     kutacc_dev::bf16x4 ov;
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
                         float v = acc[4 * a + c] + bv[c];
-                        if (beta != 0.f && f + c < n && r < rows) {
-                            v += beta * to_f32(dst[r * ld_out + f + c]);
+                        if constexpr (BETA) {
+                            v += f + c < n && r < rows ? beta * to_f32(dst[r * ld_out + f + c]) : 0.f;
                         }
                         ov[c] = (bf16_t)v;
                     }
@@ -616,9 +622,13 @@ int linear(int32_t dtype, const void *act, int64_t ld_act, const void *w, int64_
                     (const bf16_t *)act, ld_act, (const bf16_t *)w, ld_w, bias, (bf16_t *)result, m, (int)n, slice, beta, piece);
                 return kutacc_hip_status(hipGetLastError());
             };
-            static size_t configured[3][KUTACC_DEVICE_SLOTS] = {};
-            return k == 64 ? launch(linear_rows_kernel<64>, configured[0])
-                           : (k == 128 ? launch(linear_rows_kernel<128>, configured[1]) : launch(linear_rows_kernel<256>, configured[2]));
+            static size_t configured[6][KUTACC_DEVICE_SLOTS] = {};
+            if (beta != 0.f) {
+                return k == 64 ? launch(linear_rows_kernel<64, true>, configured[0])
+                               : (k == 128 ? launch(linear_rows_kernel<128, true>, configured[1]) : launch(linear_rows_kernel<256, true>, configured[2]));
+            }
+            return k == 64 ? launch(linear_rows_kernel<64, false>, configured[3])
+                           : (k == 128 ? launch(linear_rows_kernel<128, false>, configured[4]) : launch(linear_rows_kernel<256, false>, configured[5]));
         }
         if (beta == 0.f) {
             kutacc_hip_gemm_args_t g = {};
