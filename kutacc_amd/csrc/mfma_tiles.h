@@ -131,11 +131,27 @@ __device__ __forceinline__ uint4 load8_any(const bf16_t *row, uint32_t at)
     return v;
 }
 
-__device__ __forceinline__ uint4 load8_checked(const bf16_t *row, int at, int length)
+// eight elements without the first `drop` <= 8, zeros behind the others
+__device__ __forceinline__ uint4 drop_first(uint4 v, int drop)
 {
     union {
         uint4 u;
         uint64_t q[2];
+    } c;
+    c.u = v;
+    const int bits = 16 * (drop & 3);
+    if (drop >= 4) {
+        c.q[0] = drop == 8 ? 0 : c.q[1] >> bits, c.q[1] = 0;
+    } else if (drop > 0) {
+        c.q[0] = c.q[0] >> bits | c.q[1] << (64 - bits), c.q[1] >>= bits;
+    }
+    return c.u;
+}
+
+__device__ __forceinline__ uint4 load8_checked(const bf16_t *row, int at, int length)
+{
+    union {
+        uint4 u;
         bf16_t e[8];
     } c;
     if (length < 8) {
@@ -149,14 +165,7 @@ __device__ __forceinline__ uint4 load8_checked(const bf16_t *row, int at, int le
         return c.u;
     }
     const int from = min(at, length - 8), drop = min(at - from, 8);
-    c.u = load8_any(row, from);
-    const int bits = 16 * (drop & 3);
-    if (drop >= 4) {
-        c.q[0] = drop == 8 ? 0 : c.q[1] >> bits, c.q[1] = 0;
-    } else if (drop > 0) {
-        c.q[0] = c.q[0] >> bits | c.q[1] << (64 - bits), c.q[1] >>= bits;
-    }
-    return c.u;
+    return drop_first(load8_any(row, from), drop);
 }
 
 // Wave-private staging panel in LDS: 32 rows x 128 bytes, in 16-byte slots.  A panel is filled with

@@ -10,7 +10,7 @@
 //     keys past the end at -inf; masks are added to it in fp32, only in key tiles that have one;
 //   * p.v with 16x16x32 MFMAs of 32 keys whose rows are the eight values and ones, which give the sums of the probabilities.
 // K, V and masks of a head's four rows lie in the LDS for the whole workgroup (128 bytes per key and 16 of masks).
-// Measured on 1024 rows x 301 keys x 8 heads: 505 us on the general attention_tiles_kernel, 203 us here.  With the queries and
+// Measured on 1024 rows x 301 keys x 8 heads: 505 us on the general attention_tiles_kernel, 184 us here (vector ALU busy 65 %).  With the queries and
 // the masks in two parts (16 bits, an error of up to 8 % in a probability at logits of 11 000) and 32x32x16 products it was 199.
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -131,13 +131,24 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         struct Raw {
             uint4 r[2]; // keys 8 c .. 8 c + 7 of this lane's two queries
         };
+        // eight keys of a row of the bias, the row's last eight where it ends before them (and rows of fewer than eight are not read here)
         auto load_nb = [&](int t) {
             Raw w = {zero_u4(), zero_u4()};
             if constexpr (HAS_NB) {
-                const int key = 32 * min(t, NB - 1) + 8 * c;
+                const int key = min(32 * t + 8 * c, S - 8);
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    w.r[u] = 32 * t + 32 <= S ? load8_any(nb_head, nb_row[u] + key) : load8_checked(nb_head + nb_row[u], key, S);
+                    w.r[u] = load8_any(nb_head, nb_row[u] + (uint32_t)key);
+                }
+            }
+            return w;
+        };
+        auto load_tail = [&] { // of the last tile, where it has fewer than 32 keys; keys past the end zero
+            Raw w = {zero_u4(), zero_u4()};
+            if constexpr (HAS_NB) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    w.r[u] = load8_checked(nb_head + nb_row[u], 32 * (NB - 1) + 8 * c, S);
                 }
             }
             return w;
@@ -145,7 +156,7 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         struct Tile {
             f32x4 x[2][2]; // [query half][key half]
         };
-        auto seeds = [&](const Raw &w, int t) { // of the four rows' logits: the pair bias, -inf past the last key
+        auto seeds = [&](const Raw &w, auto tail) { // of the four rows' logits: the pair bias, -inf past the last key
             Tile s;
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
@@ -155,10 +166,10 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
                     s.x[u][e >> 2][e & 3] = HAS_NB ? to_f32(raw[e]) * LOG2E : 0.f;
                 }
             }
-            if (32 * t + 32 > S) {
+            if constexpr (decltype(tail)::value) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    if (32 * t + 8 * c + e >= S) {
+                    if (32 * (NB - 1) + 8 * c + e >= S) {
                         s.x[0][e >> 2][e & 3] = s.x[1][e >> 2][e & 3] = -INFINITY;
                     }
                 }
@@ -204,35 +215,51 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
             }
         };
         const float unshifted[2] = {0.f, 0.f};
-        Raw raw = load_nb(0);
-        for (int t = 0; t < NB; ++t) {
-            const Tile C = seeds(raw, t);
-            if (t + 1 < NB) {
+        // Two rows in flight: the logits of one are in the matrix pipe while the other's exponentials run.  The fences keep
+        // it at two: left to itself the compiler starts all four and needs registers for two waves per SIMD only.
+        auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+        auto rows = [&](int t, const Tile &C, auto masked) __attribute__((always_inline)) {
+            Tile xa = logits(0, t, C, masked);
+            fence();
+            Tile xb = logits(1, t, C, masked);
+            finish(0, t, xa, unshifted, std::false_type{});
+            fence();
+            xa = logits(2, t, C, masked);
+            finish(1, t, xb, unshifted, std::false_type{});
+            fence();
+            xb = logits(3, t, C, masked);
+            finish(2, t, xa, unshifted, std::false_type{});
+            fence();
+            finish(3, t, xb, unshifted, std::false_type{});
+            fence();
+        };
+        // Tiles without a mask, tiles with one, and the ragged last one, each in a loop of its own: with their choice inside one loop
+        // a tile cost 76 vector instructions and 16 moves of register pairs more than the 160 that it needs (the whole operator, us: 1024
+        // rows of 301 237 -> 221, 1000 of 420 432 -> 381; with one-instruction reciprocals behind the loop 217 and 374).
+        const int full = S >> 5, plain = min(masked_from, full);
+        Raw raw = {zero_u4(), zero_u4()};
+        if (S >= 8) {
+            raw = load_nb(0);
+        }
+        auto run = [&](int from, int to, auto masked) __attribute__((always_inline)) {
+            for (int t = from; t < to; ++t) {
+                const Tile C = seeds(raw, std::false_type{});
                 raw = load_nb(t + 1);
+                rows(t, C, masked);
             }
-            // Two rows in flight: the logits of one are in the matrix pipe while the other's exponentials run.  The fences keep
-            // it at two: left to itself the compiler starts all four and needs registers for two waves per SIMD only.
-            auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
-            auto rows = [&](auto masked) {
-                Tile xa = logits(0, t, C, masked);
-                fence();
-                Tile xb = logits(1, t, C, masked);
-                finish(0, t, xa, unshifted, std::false_type{});
-                fence();
-                xa = logits(2, t, C, masked);
-                finish(1, t, xb, unshifted, std::false_type{});
-                fence();
-                xb = logits(3, t, C, masked);
-                finish(2, t, xa, unshifted, std::false_type{});
-                fence();
-                finish(3, t, xb, unshifted, std::false_type{});
-                fence();
-            };
-            if (t < masked_from) {
-                rows(std::false_type{});
-            } else {
-                rows(std::true_type{});
+        };
+        run(0, plain, std::false_type{});
+        run(plain, full, std::true_type{});
+        if (full < NB) {
+            if constexpr (HAS_NB) {
+                if (S >= 8) {
+                    const int drop = min(max(32 * full + 8 * c - (S - 8), 0), 8);
+                    raw.r[0] = drop_first(raw.r[0], drop), raw.r[1] = drop_first(raw.r[1], drop);
+                } else {
+                    raw = load_tail();
+                }
             }
+            rows(full, seeds(raw, std::true_type{}), std::true_type{});
         }
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
@@ -255,9 +282,10 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
             if (__any(!(l > 1e-30f && l < 1e30f))) {
                 // Some probability overflowed or a whole row underflowed (every key masked: -1e9 log2(e) everywhere, which is
                 // finite): the row's true maxima first, then the probabilities with them subtracted.
+                auto again = [&](int t) { return logits(i, t, t < full ? seeds(load_nb(t), std::false_type{}) : seeds(load_tail(), std::true_type{}), std::true_type{}); };
                 float mx[2] = {-INFINITY, -INFINITY};
                 for (int t = 0; t < NB; ++t) {
-                    const Tile x = logits(i, t, seeds(load_nb(t), t), std::true_type{});
+                    const Tile x = again(t);
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
                         mx[e >> 3] = fmaxf(mx[e >> 3], x.x[e >> 3][(e >> 2) & 1][e & 3]);
@@ -271,12 +299,12 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
                 }
                 clear(i);
                 for (int t = 0; t < NB; ++t) {
-                    finish(i, t, logits(i, t, seeds(load_nb(t), t), std::true_type{}), mx, std::true_type{});
+                    finish(i, t, again(t), mx, std::true_type{});
                 }
                 collect();
             }
             const int pos = 32 * j + 16 * (le >> 5) + (le & 15), d0 = 4 * ((le >> 4) & 1);
-            const float inv = 1.0f / l;
+            const float inv = __builtin_amdgcn_rcpf(l);
             if (pos < S && b0 + i < p.B) {
                 const int64_t row = (int64_t)(b0 + i) * S + pos;
                 const bf16x4 gv = *reinterpret_cast<const bf16x4 *>(p.gate + row * p.g_ss + h * D + d0);
@@ -284,7 +312,7 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float wavg = to_f32((bf16_t)(values[e] * inv));
-                    ov[e] = (bf16_t)(wavg * sigmoid_f32(to_f32(gv[e])));
+                    ov[e] = (bf16_t)(wavg * sigmoid_fast(to_f32(gv[e])));
                 }
                 *reinterpret_cast<bf16x4 *>(p.avg + row * p.a_ss + h * D + d0) = ov;
             }
