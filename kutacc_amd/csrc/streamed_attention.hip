@@ -9,6 +9,7 @@
 //       which share the pair bias (fp32 tiles in accumulator order, the C operand of every row's logits MFMAs, as in
 //       persistent_pair_kernel); a workgroup of four waves walks all keys of the rows, their K and V staged
 //       through a ring of key tiles in the LDS.
+//   streamed_plain_kernel     the same without a pair bias, where a wave owns two blocks of queries of one row.
 //   output_projection_kernel  multiplies the gated average, fragments as well, and adds the result to the activation.
 //
 // Against fused_head_kernel (one workgroup per row and head, K and V of the whole row in the LDS, projections in front):
@@ -61,7 +62,7 @@ struct StreamedParams {
     uint32_t *flags;
     const f32x4 *tiles;   // pair bias: [head][query block][NT][4][64 lanes] (pair_bias_tiles_kernel)
     int B, S, H, NB, NT; // batch rows, positions, heads, blocks, key tiles of `tiles` per query block
-    int query_groups, set_groups, groups, group_rows; // placement of the attention's workgroups
+    int query_groups, set_groups, groups, group_rows, plain_waves; // the attention's workgroups
 };
 
 // ---- the projections ----
@@ -275,6 +276,7 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
 
 // ---- the attention ----
 constexpr int WAVES = 4;                  // query blocks per workgroup
+constexpr int PLAIN_BLOCKS = 2;           // query blocks of a wave without a pair bias
 constexpr int RING = 3;                   // groups of tiles in the LDS
 constexpr int TOGETHER = 8, MEMBERS = 64; // query groups and workgroups of a placement group, at most
 
@@ -356,13 +358,13 @@ __device__ __forceinline__ void attend_shifted(const uint4 *k, const uint4 *v, c
 // Bound by the issue of the softmax (16 exponentials and 8 packs per lane, row and tile: 201 of the 268 clocks that a tile of 32 x 32
 // logits takes a SIMD with no load in the loop) and next to it by what the loop loads.  Four rows a wave halve the loads of
 // the pair bias, 4 KB a tile, and leave 256 registers to the two waves of a SIMD, against two rows on three waves of 168: 2048
-// residues without padding 6.56 -> 5.84 ms, 1024 residues 1.00 -> 0.79 ms.  Without a pair bias rows share nothing: two rows on three waves.
+// residues without padding 6.56 -> 5.84 ms, 1024 residues 1.00 -> 0.79 ms.
 //
 // Keys and values come straight into the LDS (global_load_lds_dwordx4), a group of tiles at a time, of which every wave brings four
 // pieces of 1 KB: a ring of three groups, one barrier per group.  At the barrier in front of group G, group G + 1 has landed and group
 // G - 1 has been left by every wave; its place takes group G + 2.
-template <bool HAS_NB, int ROWS>
-__global__ __launch_bounds__(ROWS == 4 || HAS_NB ? 512 : 768) void streamed_attention_kernel(const StreamedParams p)
+template <int ROWS>
+__global__ __launch_bounds__(512) void streamed_attention_kernel(const StreamedParams p)
 {
     using W = Walk<ROWS>;
     typedef __attribute__((address_space(3))) void *lds_ptr;
@@ -445,18 +447,16 @@ __global__ __launch_bounds__(ROWS == 4 || HAS_NB ? 512 : 768) void streamed_atte
         const uint4 *src = p.q + (row[i] + j) * BLOCK_SLOTS;
         q[i][0] = as_bf16x8(src[lane]), q[i][1] = as_bf16x8(src[64 + lane]);
     }
-    const f32x4 *nbc = HAS_NB ? p.tiles + ((int64_t)h * NB + j) * p.NT * 256 : nullptr;
+    const f32x4 *nbc = p.tiles + ((int64_t)h * NB + j) * p.NT * 256;
     auto load_nb = [&](int t) {
-        f32x16 c = zero16();
-        if constexpr (HAS_NB) {
-            const char *tile = reinterpret_cast<const char *>(nbc + min(t, NB - 1) * 256); // uniform; the lane's part in 32 bits
+        f32x16 c;
+        const char *tile = reinterpret_cast<const char *>(nbc + min(t, NB - 1) * 256); // uniform; the lane's part in 32 bits
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(tile + (lane_bytes + 1024u * a));
+        for (int a = 0; a < 4; ++a) {
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(tile + (lane_bytes + 1024u * a));
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    c[4 * a + e] = v[e];
-                }
+            for (int e = 0; e < 4; ++e) {
+                c[4 * a + e] = v[e];
             }
         }
         return c;
@@ -585,13 +585,9 @@ __global__ __launch_bounds__(ROWS == 4 || HAS_NB ? 512 : 768) void streamed_atte
         next += W::TILE_SLOTS;
         next = next == end ? lds : next;
         if (--left == 0) {
-            // This wave's pieces of the group behind the next one have landed: it asked for them a group ago, and with a
-            // pair bias its youngest loads are those of the group's tiles' bias, issued since.
-            if constexpr (HAS_NB) {
-                asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(4 * W::TILES_PER_GROUP) : "memory");
-            } else {
-                asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-            }
+            // This wave's pieces of the group behind the next one have landed: it asked for them a group ago, and its
+            // youngest loads are those of the group's tiles' bias, issued since.
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(4 * W::TILES_PER_GROUP) : "memory");
             refill();
             left = W::TILES_PER_GROUP;
         }
@@ -635,8 +631,199 @@ __global__ __launch_bounds__(ROWS == 4 || HAS_NB ? 512 : 768) void streamed_atte
         const int i = __builtin_ctz(again), bi = ROWS * set + i;
         again &= again - 1;
         const int64_t at = ((int64_t)bi * p.H + h) * NB;
-        attend_shifted<HAS_NB>(p.k + at * BLOCK_SLOTS, p.v + at * BLOCK_SLOTS, p.words + (int64_t)bi * NB * 32, nbc, p.q + (at + j) * BLOCK_SLOTS,
+        attend_shifted<true>(p.k + at * BLOCK_SLOTS, p.v + at * BLOCK_SLOTS, p.words + (int64_t)bi * NB * 32, nbc, p.q + (at + j) * BLOCK_SLOTS,
                                p.g + (at + j) * BLOCK_SLOTS, NB, lane);
+    }
+}
+
+// The same without a pair bias, where batch rows share nothing: a wave attends two blocks of 32 queries of one row, which share its
+// keys, values and masks.  A workgroup walks the row's keys once for all its blocks; each of its waves brings one tile (4 KB) of a group.
+// Bound by issue and power: 1024 sequences x 384 residues x 8 heads 520 us, 295 clocks a tile of 32 x 32 logits and SIMD, at the
+// 1.8 GHz that the chip holds under it.  Two rows a wave, which share nothing, 541 us; four blocks a wave on two waves a SIMD 526; two
+// blocks on four waves of 128 registers 523.  3000 x 60 685 -> 605, 700 x 256 211 -> 192, 300 x 100 25.2 -> 26.2 us.
+__global__ __launch_bounds__(768) void streamed_plain_kernel(const StreamedParams p)
+{
+    typedef __attribute__((address_space(3))) void *lds_ptr;
+    extern __shared__ uint4 lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int NB = p.NB, W = p.plain_waves;
+    constexpr int BLOCKS = PLAIN_BLOCKS, TILE = 2 * BLOCK_SLOTS; // slots of a tile in the LDS: K, V
+
+    // Workgroup ids are dealt round robin over the 8 XCDs: a row and head's workgroups run side by side on one, whose L2 has its keys.
+    const int local = (int)(blockIdx.x >> 3), part = local % p.query_groups;
+    const int row_head = (local / p.query_groups) * 8 + (int)(blockIdx.x & 7);
+    if (row_head >= p.groups) {
+        return;
+    }
+    const int b = row_head / p.H;
+    const int64_t row = (int64_t)row_head * NB; // first fragment block
+    const int j = (part * W + wave) * BLOCKS;
+
+    const uint32_t ring = (uint32_t)(uintptr_t)(lds_ptr)lds, lane_bytes = 16u * (uint32_t)lane;
+    auto request = [&](uint32_t place, int first_tile) { // this wave's one of the tiles first_tile ..
+        const int64_t from = (row + min(first_tile + wave, NB - 1)) * BLOCK_SLOTS;
+        const uint32_t to = ring + (place * W + wave) * 4096u;
+        load_to_lds(to, p.k + from, lane_bytes);
+        load_to_lds(to + 1024u, p.k + from + 64, lane_bytes);
+        load_to_lds(to + 2048u, p.v + from, lane_bytes);
+        load_to_lds(to + 3072u, p.v + from + 64, lane_bytes);
+    };
+    request(0, 0);
+    request(1, W);
+    int fill = 2, fill_tile = 2 * W;
+    int gate_place = -1; // of this wave's gates, which follow the last keys as in streamed_attention_kernel
+    auto refill = [&] {
+        if (fill_tile < NB) {
+            request(fill, fill_tile);
+        } else if (gate_place < 0 && j < NB) {
+            gate_place = fill;
+            const uint32_t to = ring + (uint32_t)(fill * W + wave) * 4096u;
+            const uint4 *first = p.g + (row + j) * BLOCK_SLOTS, *second = p.g + (row + min(j + 1, NB - 1)) * BLOCK_SLOTS;
+            load_to_lds(to, first, lane_bytes);
+            load_to_lds(to + 1024u, first + 64, lane_bytes);
+            load_to_lds(to + 2048u, second, lane_bytes);
+            load_to_lds(to + 3072u, second + 64, lane_bytes);
+        }
+        fill = fill == RING - 1 ? 0 : fill + 1;
+        fill_tile += W;
+    };
+    if (j >= NB) { // a wave without queries brings its share of the keys
+        for (int t = 0; t < NB; t += W) {
+            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+            refill();
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
+    }
+
+    bf16x8 q[BLOCKS][2]; // past the last block: that one again, not stored
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i) {
+        const uint4 *src = p.q + (row + min(j + i, NB - 1)) * BLOCK_SLOTS;
+        q[i][0] = as_bf16x8(src[lane]), q[i][1] = as_bf16x8(src[64 + lane]);
+    }
+
+    const uint32_t *flags = p.flags + (int64_t)b * NB;
+    int masked_from = NB; // first key tile that has a mask (the ragged tail counts: its keys are at -inf)
+    for (int t0 = 0; t0 < NB; t0 += 64) {
+        const unsigned long long any = __ballot(t0 + lane < NB && flags[min(t0 + lane, NB - 1)] != 0u);
+        if (any != 0) {
+            masked_from = t0 + __builtin_ctzll(any);
+            break;
+        }
+    }
+    uint32_t shift = 0; // one mask on all keys: see streamed_attention_kernel
+    if (masked_from == 0) {
+        const uint32_t f = flags[0];
+        bool differs = f == MIXED_WORDS;
+        for (int t0 = 0; t0 < NB && !differs; t0 += 64) {
+            differs = __any(flags[min(t0 + lane, NB - 1)] != f);
+        }
+        shift = __builtin_amdgcn_readfirstlane(differs ? 0u : f ^ 0x80008000u);
+    }
+    const uint32_t lower = lane < 32 ? 0xffffffffu : 0u; // the mask as a rank-one MFMA
+    auto mask_word_of = [&](int t) { return p.words[((int64_t)b * NB + min(t, NB - 1)) * 32 + (lane & 31)] & lower; };
+    auto add_mask = [&](f32x16 x, uint32_t w) {
+        const bf16x8 ones = as_bf16x8(make_uint4(0x3f803f80u & lower, 0u, 0u, 0u));
+        return mfma(as_bf16x8(make_uint4(w, 0u, 0u, 0u)), ones, x);
+    };
+
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); // groups 0 and 1 have landed, every wave's part of them
+    refill();
+    int left = W; // tiles of the current group still to come, this one included
+    const uint4 *const end = lds + RING * W * TILE, *next = lds + TILE; // tile t + 1
+    uint4 k0 = lds[lane], k1 = lds[64 + lane], v0 = lds[128 + lane], v1 = lds[192 + lane];
+    f32x16 x[2]; // logits: of block i in x[i & 1]
+    x[0] = mfma(as_bf16x8(k0), q[0][0], zero16());
+    x[0] = mfma(as_bf16x8(k1), q[0][1], x[0]);
+    f32x16 o[BLOCKS];
+    f32x4 sums[BLOCKS];
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i) {
+        o[i] = zero16(), sums[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    uint32_t m = 0, mn = 0; // mask words of this tile and of the next
+    const bf16x8 ones_rows = rowsum_selector(lane);
+
+    auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+    auto tile = [&](int t, auto masked) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < BLOCKS; ++i) {
+            constexpr int LAST = BLOCKS - 1;
+            const int n = i == LAST ? 0 : i + 1;
+            f32x16 &xc = x[i & 1], &xn = x[n & 1];
+            auto exp4 = [&](int base) {
+#pragma unroll
+                for (int e = base; e < base + 4; ++e) {
+                    xc[e] = __builtin_amdgcn_exp2f(xc[e]);
+                }
+            };
+            exp4(0);
+            xn = mfma(as_bf16x8(k0), q[n][0], zero16());
+            fence();
+            exp4(4);
+            const bf16x8 p0 = pack8(xc, 0);
+            xn = mfma(as_bf16x8(k1), q[n][1], xn);
+            if constexpr (decltype(masked)::value) {
+                xn = add_mask(add_mask(xn, i == LAST ? mn : m), shift & lower);
+            }
+            if (i == LAST - 1) {
+                k0 = next[lane], k1 = next[64 + lane];
+            }
+            fence();
+            exp4(8);
+            o[i] = mfma(as_bf16x8(v0), p0, o[i]);
+            fence();
+            exp4(12);
+            const bf16x8 p1 = pack8(xc, 8);
+            sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p0, sums[i], 0, 0, 0);
+            o[i] = mfma(as_bf16x8(v1), p1, o[i]);
+            sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p1, sums[i], 0, 0, 0);
+            fence();
+            if (i == LAST) {
+                v0 = next[128 + lane], v1 = next[192 + lane];
+                if constexpr (decltype(masked)::value) {
+                    m = mn, mn = mask_word_of(t + 2);
+                }
+            }
+            fence();
+        }
+        next += TILE;
+        next = next == end ? lds : next;
+        if (--left == 0) {
+            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); // this wave's tile of the group behind the next one: asked for a group ago
+            refill();
+            left = W;
+        }
+    };
+    for (int t = 0; t < masked_from; ++t) {
+        tile(t, std::false_type{});
+    }
+    if (masked_from < NB) {
+        m = mask_word_of(masked_from), mn = mask_word_of(masked_from + 1);
+        x[0] = add_mask(add_mask(x[0], m), shift & lower);
+        for (int t = masked_from; t < NB; ++t) {
+            tile(t, std::true_type{});
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the gates, and requests past the last tile before the LDS is given back
+    uint32_t again = 0; // blocks whose sums ran out of range
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i) {
+        const float l = rowsum_fetch(sums[i], lane);
+        const bool stored = j + i < NB;
+        if (__any(!(l > 1e-30f && l < 1e30f))) {
+            again |= stored ? 1u << i : 0u;
+        } else if (stored) {
+            const uint4 *gate = lds + (gate_place * W + wave) * TILE + i * BLOCK_SLOTS + lane;
+            store_average(p.q + (row + j + i) * BLOCK_SLOTS + lane, gate[0], gate[64], o[i], l);
+        }
+    }
+    while (again != 0) {
+        const int i = __builtin_ctz(again);
+        again &= again - 1;
+        attend_shifted<false>(p.k + row * BLOCK_SLOTS, p.v + row * BLOCK_SLOTS, p.words + (int64_t)b * NB * 32, nullptr,
+                              p.q + (row + j + i) * BLOCK_SLOTS, p.g + (row + j + i) * BLOCK_SLOTS, NB, lane);
     }
 }
 
@@ -792,7 +979,7 @@ int launch_projection(const StreamedParams &p, hipStream_t stream)
     return kutacc_hip_status(hipGetLastError());
 }
 
-template <bool HAS_NB, int ROWS>
+template <int ROWS>
 int launch_attention(StreamedParams p, hipStream_t stream)
 {
     const int sets = (p.B + ROWS - 1) / ROWS;
@@ -803,7 +990,21 @@ int launch_attention(StreamedParams p, hipStream_t stream)
     p.groups = p.set_groups * p.H * parts;
     const int64_t blocks = (int64_t)(p.groups + 7) / 8 * 8 * p.group_rows * together;
     kutacc_prof::KernelTimer t("streamed_attention_kernel", 4.0 * (double)p.B * p.S * p.S * p.H * HEAD, stream);
-    streamed_attention_kernel<HAS_NB, ROWS><<<dim3((unsigned)blocks), 64 * WAVES, Walk<ROWS>::LDS, stream>>>(p);
+    streamed_attention_kernel<ROWS><<<dim3((unsigned)blocks), 64 * WAVES, Walk<ROWS>::LDS, stream>>>(p);
+    return kutacc_hip_status(hipGetLastError());
+}
+
+int launch_plain(StreamedParams p, hipStream_t stream)
+{
+    // Three waves a workgroup instead of four where that leaves a tenth fewer queries past the row's end, as 9 .. 12 blocks do (300
+    // sequences x 100 residues 27.9 -> 26.2 us; 900 x 300, 30 blocks for 32, 373 -> 382).
+    const auto slots = [&](int waves) { return (p.NB + PLAIN_BLOCKS * waves - 1) / (PLAIN_BLOCKS * waves) * waves; };
+    p.plain_waves = 10 * slots(3) < 9 * slots(4) ? 3 : 4;
+    p.query_groups = slots(p.plain_waves) / p.plain_waves;
+    p.groups = p.B * p.H;
+    const int64_t blocks = ((int64_t)p.groups + 7) / 8 * 8 * p.query_groups;
+    kutacc_prof::KernelTimer t("streamed_attention_kernel", 4.0 * (double)p.B * p.S * p.S * p.H * HEAD, stream);
+    streamed_plain_kernel<<<dim3((unsigned)blocks), 64 * p.plain_waves, (size_t)RING * p.plain_waves * 4096, stream>>>(p);
     return kutacc_hip_status(hipGetLastError());
 }
 
@@ -892,9 +1093,9 @@ int gating_attention_streamed(const kutacc_hip_attention_args_t &a, const FusedA
         // Two rows a wave where four would leave CUs idle, below three workgroups to two CUs (8 heads of 1100 residues, whole block: 4, 8
         // and 16 sequences 155, 167 and 187 us against 165, 172 and 192 on four rows a wave; 24 and 64: 223 and 347 against 206 and 336).
         const int64_t fours = (a.batch + 3) / 4 * a.nheads * ((p.NB + WAVES - 1) / WAVES);
-        rc = !has_nb                             ? launch_attention<false, 2>(p, stream)
-             : 2 * fours >= 3 * kutacc_cu_count() ? launch_attention<true, 4>(p, stream)
-                                                  : launch_attention<true, 2>(p, stream);
+        rc = !has_nb                             ? launch_plain(p, stream)
+             : 2 * fours >= 3 * kutacc_cu_count() ? launch_attention<4>(p, stream)
+                                                  : launch_attention<2>(p, stream);
     }
     if (rc != 0) {
         return rc;

@@ -514,6 +514,26 @@ def test_streamed_rows_of_one_mask_beside_others(torch_cuda, streamed_everywhere
     helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, column), "bf16", f"rows of one mask {n_seq}x{n_res} heads={heads} column={column}")
 
 
+# without a pair bias: one block of queries and two a wave, three waves a workgroup (3 to 6, 9 to 12, 17 and 18 blocks) and four, the
+# last workgroup full, with an odd block, and with waves that have none
+@pytest.mark.parametrize("n_seq,n_res,heads", [(1, 5, 8), (33, 3, 4), (96, 2, 8), (193, 3, 4), (256, 2, 8), (257, 3, 8), (390, 2, 4), (520, 2, 8)])
+def test_streamed_rows_without_pair_bias_at_the_edges_of_a_workgroup(torch_cuda, streamed_everywhere, n_seq, n_res, heads):
+    torch = torch_cuda
+    c = msa_case(9900 + n_seq, n_seq, n_res, heads, 128)
+    c["mask"][:] = 1.0
+    c["mask"][-(n_seq // 4):, n_res // 2] = 0.0  # masked keys at the end of one residue's row, anywhere in the next, everywhere in the last
+    c["mask"][::3, (n_res // 2 + 1) % n_res] = 0.0
+    c["mask"][:, -1] = 0.0
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
+        device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
+    msa = dev(c["m"])
+    w = {k: dev(c[k]) for k in ("ln_gamma", "ln_beta", "wq", "wk", "wv", "wg", "bg", "wo", "bo")}
+    print(f"streamed column {n_seq}x{n_res} heads={heads}", flush=True)
+    assert capi.MsaAttentionBlock(msa, dev(c["mask"]), w, heads, None).run() == 0
+    torch.cuda.synchronize()
+    helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, True), "bf16", f"streamed column {n_seq}x{n_res} heads={heads}")
+
+
 @pytest.mark.parametrize("kind,n_seq,n_res,heads", [("triangle", 0, 1025, 4), ("row", 3, 1050, 8), ("column", 1030, 2, 4)])
 def test_blocks_beyond_1024_keys_take_weights_on_any_address(torch_cuda, kind, n_seq, n_res, heads):
     """The route of these blocks asks nothing of the weights' alignment: the same bits with every matrix and both biases one element
