@@ -485,20 +485,19 @@ struct MsaWorkspace {
 };
 
 // fused_ln: the head kernel normalises the msa rows itself, so no normalised copy is kept; tiled: as for the
-// triangle-attention block
+// triangle-attention block; streamed: neither a normalised copy nor an average beside the attention's own workspace at q
 MsaWorkspace msa_layout(int64_t n_seq, int64_t n_res, int64_t heads, bool column, bool fused_ln, bool tiled = false, bool streamed = false)
 {
     const int64_t act = align256(n_seq * n_res * heads * HEAD * 2);
     MsaWorkspace w;
     w.m_norm = 0;
-    w.nb = w.m_norm + (fused_ln ? 0 : act);
+    w.nb = w.m_norm + (fused_ln || streamed ? 0 : act);
     w.bias = w.nb + (column ? 0 : align256(heads * n_res * n_res * 2));
     w.q = w.bias + align256(n_seq * n_res * 2);
     w.avg = w.q + act;
     w.k = w.v = w.gate = w.out = w.total = w.avg + act;
     if (streamed) {
-        w.avg = w.q + align256(kutacc_launch::streamed_workspace_bytes(column ? n_res : n_seq, column ? n_seq : n_res, heads, !column));
-        w.total = w.avg + act;
+        w.total = w.q + align256(kutacc_launch::streamed_workspace_bytes(column ? n_res : n_seq, column ? n_seq : n_res, heads, !column));
     } else if (tiled) {
         w.v = w.k + act, w.gate = w.v + act, w.out = w.gate + act, w.total = w.out + act;
     }
@@ -540,6 +539,25 @@ bool msa_block_is_tiled(int64_t n_seq, int64_t n_res, int64_t heads, bool column
     return beyond_fused_kernels(column ? n_seq : n_res, heads) || block_is_streamed(column ? n_seq : n_res, heads);
 }
 
+// Blocks that both the fused and the streamed kernels take, and the streamed ones faster: 256 channels, more than 256 keys.
+// Up to 256 keys the fused kernel needs half the waves' registers for K and V and wins (508 sequences x 192 residues 155 against
+// 168 us); beyond, whole blocks of 508 sequences: 259 residues 313 -> 278 us, 512: 575 -> 518, 1000: 1498 -> 1354.
+// Column-wise more than 32 residues (40 x 512 68 -> 61, 256 x 1024 612 -> 577, 384 x 1024 910 -> 853): up to there the fused kernel has one
+// workgroup a CU for its 8 heads a residue, all in one turn (32 x 512 48 against 52).  Row-wise more than 128 sequences (144 x 384 138 -> 131,
+// 192 x 512 238 -> 215; worst 192 x 330 150 against 152): there four rows a wave leave the streamed kernel short of work
+// (128 x 384 112 against 119, 64 x 640 131 against 142).
+// Not with the LayerNorm inside the fused kernel, which is asked for to have the smaller workspace.
+bool msa_block_prefers_streamed(int64_t n_seq, int64_t n_res, int64_t heads, bool column)
+{
+    return heads == 8 && (column ? n_seq : n_res) > 256 && (column ? n_res > 32 : n_seq > 128) && !msa_block_is_tiled(n_seq, n_res, heads, column) &&
+           !layernorm_policy_allows(heads * HEAD);
+}
+
+MsaWorkspace msa_streamed_layout(int64_t n_seq, int64_t n_res, int64_t heads, bool column)
+{
+    return msa_layout(n_seq, n_res, heads, column, false, false, true);
+}
+
 bool msa_block_fuses_layernorm(int64_t n_seq, int64_t n_res, int64_t heads, bool column)
 {
     if (!layernorm_policy_allows(heads * HEAD) || msa_block_is_tiled(n_seq, n_res, heads, column)) {
@@ -563,6 +581,9 @@ int64_t kutacc_hip_msa_attention_workspace(int64_t n_seq, int64_t n_res, int64_t
     if (n_seq <= 0 || n_res <= 0 || nheads <= 0 || n_seq > 1 << 20 || n_res > 65536 || nheads > 64) {
         return -1;
     }
+    if (msa_block_prefers_streamed(n_seq, n_res, nheads, column != 0)) {
+        return msa_streamed_layout(n_seq, n_res, nheads, column != 0).total;
+    }
     return msa_layout(n_seq, n_res, nheads, column != 0, msa_block_fuses_layernorm(n_seq, n_res, nheads, column != 0),
                       msa_block_is_tiled(n_seq, n_res, nheads, column != 0), block_is_streamed(column ? n_seq : n_res, nheads))
         .total;
@@ -584,14 +605,21 @@ int kutacc_hip_msa_attention(const kutacc_hip_msa_attention_args_t *a, void *str
     const int64_t n_seq = a->n_seq, n_res = a->n_res, heads = a->nheads, c = heads * HEAD;
     // where the persistent head kernel takes the call it normalises the msa rows itself: no normalised copy, no LayerNorm pass
     const bool fused_ln = msa_block_fuses_layernorm(n_seq, n_res, heads, column), tiled = msa_block_is_tiled(n_seq, n_res, heads, column);
-    const bool streamed = block_is_streamed(column ? n_seq : n_res, heads);
-    const MsaWorkspace w = msa_layout(n_seq, n_res, heads, column, fused_ln, tiled, streamed);
+    bool streamed = block_is_streamed(column ? n_seq : n_res, heads);
+    MsaWorkspace w = msa_layout(n_seq, n_res, heads, column, fused_ln, tiled, streamed);
     if (a->workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(a->workspace) & 255u) != 0) {
         return KUTACC_HIP_EINVAL;
     }
     char *ws = static_cast<char *>(a->workspace);
     hipStream_t s = kutacc_api::stream_or_default(stream);
     const kutacc_hip_attention_args_t g = msa_attention_call(a, ws, w, fused_ln);
+    if (msa_block_prefers_streamed(n_seq, n_res, heads, column) && kutacc_launch::fused_attention_supports(g)) {
+        // a workspace that only the fused kernels fit in is enough for them
+        const MsaWorkspace larger = msa_streamed_layout(n_seq, n_res, heads, column);
+        if (a->workspace_bytes >= larger.total) {
+            streamed = true, w = larger;
+        }
+    }
     if (streamed) {
         const kutacc_hip_attention_args_t g = msa_attention_call(a, ws, w, true);
         if (!kutacc_launch::streamed_attention_supports(g)) {
@@ -610,7 +638,7 @@ int kutacc_hip_msa_attention(const kutacc_hip_msa_attention_args_t *a, void *str
                                           a->c_z, heads, a->ln_eps, KUTACC_DTYPE_BF16, 0, s, opt.nb_tiles_ready ? ws + w.q : nullptr,
                                           nb_blocks, (nb_blocks + 1) & ~1, 1);
         }
-        return rc != 0 ? rc : kutacc_launch::gating_attention_streamed(g, opt, ws + w.q, w.avg - w.q, s);
+        return rc != 0 ? rc : kutacc_launch::gating_attention_streamed(g, opt, ws + w.q, w.total - w.q, s);
     }
     if (tiled) {
         // Rows beyond the fused head kernels (more than 1024 keys): LayerNorm (read transposed column-wise), pair bias

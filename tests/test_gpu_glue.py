@@ -534,6 +534,53 @@ def test_streamed_rows_without_pair_bias_at_the_edges_of_a_workgroup(torch_cuda,
     helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, True), "bf16", f"streamed column {n_seq}x{n_res} heads={heads}")
 
 
+# both sides of each line: more than 256 keys, more than 128 sequences row-wise, more than 32 residues column-wise, 8 heads
+@pytest.mark.parametrize("column,n_seq,n_res,heads,streamed", [
+    (False, 129, 257, 8, True), (False, 128, 257, 8, False), (False, 129, 256, 8, False), (False, 129, 257, 4, False), (False, 130, 1024, 8, True),
+    (True, 257, 33, 8, True), (True, 257, 32, 8, False), (True, 256, 33, 8, False), (True, 257, 33, 4, False), (True, 1023, 34, 8, True)])
+def test_msa_blocks_that_prefer_the_streamed_kernels(torch_cuda, column, n_seq, n_res, heads, streamed):
+    """The workspace decides where both kernels take a block: three activations are still enough, for the fused kernels, less is
+    refused as before, and so are weights that the fused kernels refuse.  Both give the oracle's result within the parity bar, and so each
+    other's within twice that."""
+    torch = torch_cuda
+    c = msa_case(9950 + n_seq + n_res, n_seq, n_res, heads, 64)
+    c["mask"][1::2] *= np.where(c["mask"][1::2].cumsum(1) % 5 == 0, 0.5, 1.0).astype(np.float32)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
+        device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
+    w = {k: dev(c[k]) for k in ("ln_gamma", "ln_beta", "wq", "wk", "wv", "wg", "bg", "wo", "bo")}
+    pair = None if column else {"pair_act": dev(c["z"]), "pair_ln_gamma": dev(c["pair_ln_gamma"]),
+                                "pair_ln_beta": dev(c["pair_ln_beta"]), "bias_w": dev(c["bias_w"])}
+    up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    fused_bytes = 3 * up(n_seq * n_res * heads * 64) + up(n_seq * n_res * 2) + (0 if column else up(heads * n_res * n_res * 2))
+    mask = dev(c["mask"])
+    res = []
+    for size in (None, fused_bytes, fused_bytes - 256):
+        msa = dev(c["m"])
+        blk = capi.MsaAttentionBlock(msa, mask, w, heads, pair)
+        assert (blk.args.workspace_bytes > fused_bytes) == streamed and blk.args.workspace_bytes >= fused_bytes
+        if size is not None:
+            blk.args.workspace_bytes = size
+        rc = {}
+        print(f"msa {n_seq}x{n_res} heads={heads} column={column} workspace={size}", flush=True)
+        names = profiled_kernels(torch, lambda: rc.setdefault("rc", blk.run()))  # noqa: B023
+        torch.cuda.synchronize()
+        if size == fused_bytes - 256:
+            assert rc["rc"] == capi.EINVAL and helpers.same_bits(msa, dev(c["m"]))
+            continue
+        assert rc["rc"] == 0 and ("streamed_attention_kernel" in names) == (streamed and size is None), (rc, names)
+        res.append(helpers.to_numpy(msa))
+    if n_seq * n_res < 40000:
+        want = msa_oracle(c, column)
+        for got in res:
+            helpers.check_close(got, want, "bf16", f"msa {n_seq}x{n_res} heads={heads} column={column}")
+    helpers.assert_within(res[0], res[1], 2 * (2e-2 + 1e-2 * np.abs(res[1])), f"routes {n_seq}x{n_res} heads={heads} column={column}")
+    moved = {k: t if k.startswith("ln_") else torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape) for k, t in w.items()}
+    msa = dev(c["m"])
+    assert capi.MsaAttentionBlock(msa, mask, moved, heads, pair).run() == capi.EUNSUPPORTED
+    torch.cuda.synchronize()
+    assert helpers.same_bits(msa, dev(c["m"]))
+
+
 @pytest.mark.parametrize("kind,n_seq,n_res,heads", [("triangle", 0, 1025, 4), ("row", 3, 1050, 8), ("column", 1030, 2, 4)])
 def test_blocks_beyond_1024_keys_take_weights_on_any_address(torch_cuda, kind, n_seq, n_res, heads):
     """The route of these blocks asks nothing of the weights' alignment: the same bits with every matrix and both biases one element
