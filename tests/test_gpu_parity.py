@@ -229,6 +229,31 @@ def test_seeded_shape_sweep_matches_oracle(torch_cuda, index, config, batch, seq
     helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, w.dtype, f"sweep {index} out")
 
 
+# one, two, three and four query blocks a wave, the persistent kernels of one row and of two
+@pytest.mark.parametrize("lifted", [False, True])
+@pytest.mark.parametrize("config,seq", [(5, 40), (5, 128), (5, 200), (5, 290), (5, 384), (5, 420), (5, 700), (5, 1000), (4, 200), (4, 300), (4, 1000)])
+def test_rows_whose_keys_all_have_one_mask(torch_cuda, config, seq, lifted):
+    """Their logits are taken against that mask from the start.  lifted: a pair bias of 444, which -1e9 absorbs to 448 in the oracle's
+    units and to 640 / log2(e) in the kernels': the exponentials overflow all the same and the row is repeated with its true maxima."""
+    w = make_workload(config, batch=9, seq_len=seq)
+    w.bias[:] = 0.0
+    w.bias[0, :] = round_to_bf16(np.full(seq, -1e9, dtype=np.float32))
+    w.bias[1, :] = round_to_bf16(np.full(seq, -1e9, dtype=np.float32))
+    w.bias[2, : seq - 1] = round_to_bf16(np.full(seq - 1, -1e9, dtype=np.float32))  # all but the last key
+    w.bias[4, 1:] = round_to_bf16(np.full(seq - 1, -1e9, dtype=np.float32))         # all but the first
+    w.bias[5, :] = -3.0
+    w.bias[6, seq // 2:] = round_to_bf16(np.full(seq - seq // 2, -1e9, dtype=np.float32))
+    w.bias[8, :] = w.bias[0, 0]
+    if lifted:
+        w.nb = np.full((w.H, seq, seq), 444.0, dtype=np.float32)
+    print(f"one mask: config {config} S={seq} lifted={lifted}", flush=True)
+    ten, scratch = helpers.to_device(w)
+    assert helpers.run_hip(w, ten, scratch, capi.PATH_FUSED) == 0
+    ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
+    helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), ref_avg, w.dtype, "gated average")
+    helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, w.dtype, "out")
+
+
 # ---- the two-row persistent kernel (128 channels, up to 384 keys), forced wherever it can run --------------------------
 @pytest.fixture
 def row_pairs_forced():
