@@ -10,7 +10,7 @@
 //     keys past the end at -inf; masks are added to it in fp32, only in key tiles that have one;
 //   * p.v with 16x16x32 MFMAs of 32 keys whose rows are the eight values and ones, which give the sums of the probabilities.
 // K, V and masks of a head's four rows lie in the LDS for the whole workgroup (128 bytes per key and 16 of masks).
-// Measured on 1024 rows x 301 keys x 8 heads: 505 us on the general attention_tiles_kernel, 184 us here (vector ALU busy 65 %).  With the queries and
+// Measured on 1024 rows x 301 keys x 8 heads: 505 us on the general attention_tiles_kernel, 180 us here (vector ALU busy 66 %).  With the queries and
 // the masks in two parts (16 bits, an error of up to 8 % in a probability at logits of 11 000) and 32x32x16 products it was 199.
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -70,25 +70,42 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         *first_masked = (uint32_t)NB;
     }
     __syncthreads();
-    for (int idx = tid; idx < ROWS * keys; idx += 64 * waves) {
-        const int i = idx / keys, key = idx % keys, b = row_of(i);
-        const int64_t pos = (int64_t)b * S + min(key, S - 1);
-        const uint4 kv = *reinterpret_cast<const uint4 *>(p.k + pos * p.k_ss + h * D);
-        const int tile_row = (key >> 5) * TILE + i * 32;
-        ks[tile_row + key_slot(key & 31)] = key < S ? kv : zero_u4();
-        const float mask = key < S ? to_f32(p.bias[(int64_t)b * p.bias_sb + key]) * LOG2E : 0.f;
-        masks[tile_row + (key & 31)] = mask;
+    // A wave brings 64 keys of one row at a time, the next ones requested before these are stored: of K and the mask a key a lane, of V
+    // eight keys of one value.  (Keys dealt to threads by division, K and V in loops of their own, one round trip after the other: whole
+    // operator 2000 rows of 384 660 us, 627 so, of 170 206 and 200.)
+    struct Piece {
+        uint4 k, v;
+        bf16_t mask;
+    };
+    const int units = ROWS * ((NB + 1) / 2); // row unit % 4, keys 64 (unit / 4) ..
+    const bf16_t *v_lane = p.v + (int64_t)(h * D + (lane >> 3)) * p.v_se;
+    auto fetch = [&](int unit) {
+        const int64_t pos = (int64_t)row_of(unit & 3) * S;
+        const int key0 = 64 * (unit >> 2), key = min(key0 + lane, S - 1);
+        Piece w;
+        w.k = *reinterpret_cast<const uint4 *>(p.k + pos * p.k_ss + h * D + (uint32_t)key * (uint32_t)p.k_ss);
+        w.mask = (p.bias + (int64_t)row_of(unit & 3) * p.bias_sb)[(uint32_t)key];
+        w.v = load8_checked(v_lane + pos, min(key0 + 8 * (lane & 7), S), S);
+        return w;
+    };
+    Piece piece = fetch(min(wave, units - 1));
+    for (int unit = wave; unit < units; unit += waves) {
+        const Piece w = piece;
+        piece = fetch(min(unit + waves, units - 1));
+        const int i = unit & 3, key = 64 * (unit >> 2) + lane;
+        const float mask = key < S ? to_f32(w.mask) * LOG2E : 0.f;
+        if (key < keys) {
+            const int tile_row = (key >> 5) * TILE + i * 32;
+            ks[tile_row + key_slot(key & 31)] = key < S ? w.k : zero_u4();
+            masks[tile_row + (key & 31)] = mask;
+        }
+        const int kp = 8 * (unit >> 2) + (lane & 7);
+        if (8 * kp < keys) {
+            vs[(kp >> 2) * TILE + i * 32 + (kp & 3) * 8 + (lane >> 3)] = w.v;
+        }
         if (mask != 0.f) {
             atomicMin(first_masked, (uint32_t)(key >> 5));
         }
-    }
-    for (int idx = tid; idx < ROWS * keys; idx += 64 * waves) { // eight keys of one value: as many pieces as keys
-        const int i = idx / keys, rest = idx % keys, d = rest / (keys >> 3), kp = rest % (keys >> 3), key = 8 * kp;
-        uint4 vv = zero_u4();
-        if (key < S) {
-            vv = load8_checked(p.v + (int64_t)(h * D + d) * p.v_se + (int64_t)row_of(i) * S, key, S);
-        }
-        vs[(kp >> 2) * TILE + i * 32 + (kp & 3) * 8 + d] = vv;
     }
     __syncthreads();
     const int masked_from = (int)*first_masked;
@@ -105,13 +122,18 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         int lv = lane; // opaque: the addresses of a query block's rows are formed where they are used, not kept over the keys
         asm volatile("" : "+v"(lv));
         bf16x8 q[ROWS][2]; // queries 32 j + 16 u + n
+        uint32_t query[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            query[u] = (uint32_t)min(32 * j + 16 * u + (lv & 15), S - 1);
+        }
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 // a lane splits dims 2 c and 2 c + 1 of its query, then the four lanes of the query exchange: parts for dims
-                const int query = min(32 * j + 16 * u + (lv & 15), S - 1);
-                const uint32_t raw = *reinterpret_cast<const uint32_t *>(p.q + ((int64_t)row_of(i) * S + query) * p.q_ss + h * D + 2 * (lv >> 4));
+                const uint32_t raw = *reinterpret_cast<const uint32_t *>(p.q + (int64_t)row_of(i) * S * p.q_ss + h * D +
+                                                                         (query[u] * (uint32_t)p.q_ss + 2u * (uint32_t)(lv >> 4)));
                 uint32_t part[4] = {0u, 0u, 0u, 0u};
                 float x0 = __uint_as_float(raw << 16) * p.scale2, x1 = __uint_as_float(raw & 0xffff0000u) * p.scale2;
 #pragma unroll
@@ -126,7 +148,7 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         uint32_t nb_row[2] = {0u, 0u}; // elements, within 2^30 (the launcher checks)
 #pragma unroll
         for (int u = 0; HAS_NB && u < 2; ++u) {
-            nb_row[u] = (uint32_t)min(32 * j + 16 * u + (lv & 15), S - 1) * (uint32_t)p.nb_sq;
+            nb_row[u] = query[u] * (uint32_t)p.nb_sq;
         }
         struct Raw {
             uint4 r[2]; // keys 8 c .. 8 c + 7 of this lane's two queries
@@ -261,11 +283,18 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
             }
             rows(full, seeds(raw, std::true_type{}), std::true_type{});
         }
+        // the two query halves side by side: lane l then has values 4 (l / 16 % 2) .. + 3 of query 16 (l / 32) + l % 16
+        int le = lane;
+        asm volatile("" : "+v"(le));
+        const int pos = 32 * j + 16 * (le >> 5) + (le & 15);
+        const uint32_t d0 = 4 * ((le >> 4) & 1), gate_at = (uint32_t)min(pos, S - 1) * (uint32_t)p.g_ss + d0, avg_at = (uint32_t)pos * (uint32_t)p.a_ss + d0;
+        bf16x4 gates[ROWS]; // of all rows at once, one round trip (2000 rows of 384 627 -> 622 us, of 170 200 -> 195)
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
-            // the two query halves side by side: lane l then has values 4 (l / 16 % 2) .. + 3 of query 16 (l / 32) + l % 16
-            int le = lane;
-            asm volatile("" : "+v"(le));
+            gates[i] = *reinterpret_cast<const bf16x4 *>(p.gate + (int64_t)row_of(i) * S * p.g_ss + h * D + gate_at);
+        }
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
             f32x4 values;
             float l;
             auto collect = [&] {
@@ -303,18 +332,16 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
                 }
                 collect();
             }
-            const int pos = 32 * j + 16 * (le >> 5) + (le & 15), d0 = 4 * ((le >> 4) & 1);
             const float inv = __builtin_amdgcn_rcpf(l);
             if (pos < S && b0 + i < p.B) {
-                const int64_t row = (int64_t)(b0 + i) * S + pos;
-                const bf16x4 gv = *reinterpret_cast<const bf16x4 *>(p.gate + row * p.g_ss + h * D + d0);
+                const bf16x4 gv = gates[i];
                 bf16x4 ov;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float wavg = to_f32((bf16_t)(values[e] * inv));
                     ov[e] = (bf16_t)(wavg * sigmoid_fast(to_f32(gv[e])));
                 }
-                *reinterpret_cast<bf16x4 *>(p.avg + row * p.a_ss + h * D + d0) = ov;
+                *reinterpret_cast<bf16x4 *>(p.avg + (int64_t)(b0 + i) * S * p.a_ss + h * D + avg_at) = ov;
             }
         }
     }
@@ -347,9 +374,10 @@ namespace kutacc_launch {
 bool small_head_attention_supports(const kutacc_hip_attention_args_t &a)
 {
     static int table[KUTACC_DEVICE_SLOTS] = {};
+    const auto in_reach = [&](int64_t stride) { return stride >= 0 && stride < (1 << 30) && a.seq_len * stride < (1 << 30); }; // of 32-bit byte offsets
     const int64_t NB = (a.seq_len + 31) / 32, sets = (a.batch + ROWS - 1) / ROWS;
     return a.head_size == D && NB <= 64 && lds_bytes((int)NB) <= (size_t)kutacc_device_attribute(hipDeviceAttributeMaxSharedMemoryPerBlock, 64 * 1024, table) &&
-           a.nb_stride_q >= 0 && a.seq_len * a.nb_stride_q < (1 << 30) && (sets + 7) * a.nheads * 8 <= INT32_MAX;
+           in_reach(a.nb_stride_q) && in_reach(a.q_stride_s) && in_reach(a.k_stride_s) && in_reach(a.gate_stride_s) && in_reach(a.avg_stride_s) && (sets + 7) * a.nheads * 8 <= INT32_MAX;
 }
 
 int small_head_attention(const kutacc_hip_attention_args_t &a, hipStream_t stream)

@@ -162,6 +162,13 @@ def test_heads_of_eight_at_tile_edges(torch_cuda, B, S, pair_bias):
     assert ("small_head_attention_kernel" if S <= 1120 else "attention_tiles_kernel") in names, names
 
 
+@pytest.mark.parametrize("B,S", [(1, 9), (2, 63), (3, 64), (4, 65), (5, 97), (6, 193)])
+def test_heads_of_eight_stage_their_keys_in_units_of_64(torch_cuda, B, S):
+    """Units whole, short of a key and with one, half units behind an odd number of tiles, fewer waves than rows, and the last eight keys
+    of a row read in one piece."""
+    test_heads_of_eight_at_tile_edges(torch_cuda, B, S, True)
+
+
 def test_pair_bias_entries_of_minus_infinity(torch_cuda):
     """Pairs excluded by a -inf pair bias get zero weight; a row keeps at least one finite key."""
     w = draw_workload(9, 2, 140, 4, 16)
