@@ -12,9 +12,9 @@
 // Both kernels take the padded positions p = i np + j in steps of 64.  Eight consecutive positions share the row i, because
 // np is a multiple of 8: a wave follows (i, j) of its eights with scalar additions.
 //
-// Both are bound by vector issue at two waves per SIMD (254 and 248 registers) as much as by HBM: at 384 residues each moves its 113 MB
-// (front: 256 bytes in, 512 out per position; back: 512 in, 256 out) in 41 to 46 us, half the rate of a copy, with the vector ALU
-// taken for 55 to 59 % of the clocks and the matrix cores for 23 and 11.  Neither reads a normalised copy of the pair activation: the front kernel normalises the rows on their way into the LDS, the back kernel does it again for
+// Both are bound by vector issue at two waves per SIMD (246 and 237 registers) as much as by HBM: at 384 residues each moves its 113 MB
+// (front: 256 bytes in, 512 out per position; back: 512 in, 256 out) in 38 to 39 us, 60 % of the rate of a copy, with the vector ALU
+// taken for 45 % of the clocks and the matrix cores for 18 and 9.  Neither reads a normalised copy of the pair activation: the front kernel normalises the rows on their way into the LDS, the back kernel does it again for
 // its gate, from the same rows that its residual needs.  At 384 residues that saves a pass of 76 MB and a read of 38 MB.
 #include <hip/hip_runtime.h>
 
@@ -247,8 +247,9 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
 // x[i, j] += bf16(bf16(centre' . wo^T + bo) * sigmoid(bf16(y . wg^T + bg))), centre' the normalised centre of (i, j), y its
 // normalised row of x.  Four waves, two workgroups per CU (the three barriers of a step of one are covered by the
 // other); a wave owns 32 output features, keeps both 32 x 128 weight blocks in 64 registers and moves 16 of the step's 64
-// positions: it normalises their rows of x, transposes and normalises their centre (a lane holds 8 positions of a
-// channel as it lies in memory; transpose8x8_lanes turns them into 8 channels of one position), and finishes them with the
+// positions: it normalises their rows of x, normalises their centre (which lies channel by channel in the stage; transposing
+// LDS reads give a lane 32 channels of one position: exchanged between lanes the whole block took 94.7 us at 384 residues,
+// 93.6 so, and 92.8 with the biases as the products' seeds), and finishes them with the
 // residual, for which the rows of x have stayed in its registers.
 constexpr int BACK_STAGE = STEP * ROW_SLOTS; // slots of each of the four stages: centre as it lies, y, centre', result
 constexpr size_t BACK_LDS = (size_t)4 * BACK_STAGE * 16 + 6 * C * sizeof(float);
@@ -318,20 +319,15 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
         params[4 * C + tid] = bo[tid], params[5 * C + tid] = bg[tid];
     }
     __syncthreads();
-    const uint32_t sel = transpose8x8_selector(lane);
 
     for (int step = first; step < stop; ++step) {
         int lv = lane; // opaque: LDS addresses are formed per step, not kept across the loop
         asm volatile("" : "+v"(lv));
-        // the centre as it lies: [128 channels][8 slots], the slot XOR-ed with channel / 8 % 8, under which the reads below
-        // (eight lanes: channels 8 apart, one slot) and these writes are free of bank conflicts
+        // the centre as it lies: [128 channels][8 slots], the slot XOR-ed with 2 (channel % 4) + channel / 4 % 2, under which the
+        // transposing reads below (16 lanes: four channels, two slots) and these writes are free of bank conflicts
         {
-            uint4 *mine = raw + (32 * wave + (lv >> 3)) * 8;
-            const int f = 4 * (wave & 1); // channel / 8 % 8 of this wave's first eight channels
-            mine[(lv & 7) ^ f] = ct.r0;
-            mine[64 + ((lv & 7) ^ (f + 1))] = ct.r1;
-            mine[128 + ((lv & 7) ^ (f + 2))] = ct.r2;
-            mine[192 + ((lv & 7) ^ (f + 3))] = ct.r3;
+            uint4 *mine = raw + (32 * wave + (lv >> 3)) * 8 + ((lv & 7) ^ (2 * ((lv >> 3) & 3) + (lv >> 5)));
+            mine[0] = ct.r0, mine[64] = ct.r1, mine[128] = ct.r2, mine[192] = ct.r3;
         }
         if (step + 1 < stop) {
             ct = load_centre(step + 1);
@@ -353,10 +349,23 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
             load_eight(next_hi, at_hi);
         }
         __syncthreads();
+        auto biases = [&](int which) { // of this wave's 32 features, in accumulator order: the seed of their products
+            f32x16 b;
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(params + which * C + wave * 32 + 8 * a + 4 * (lv >> 5));
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    b[4 * a + c] = v[c];
+                }
+            }
+            return b;
+        };
         // gate: this wave's 32 features of all 64 positions, rounded to bf16
         bf16x8 gate[2][2];
         {
-            f32x16 acc[2] = {zero16(), zero16()};
+            f32x16 acc[2];
+            acc[0] = acc[1] = biases(5);
 #pragma unroll
             for (int ks = 0; ks < CK; ++ks) {
 #pragma unroll
@@ -365,32 +374,23 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
                 }
             }
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const f32x4 bv = *reinterpret_cast<const f32x4 *>(params + 5 * C + wave * 32 + 8 * a + 4 * (lv >> 5));
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-#pragma unroll
-                    for (int pb = 0; pb < 2; ++pb) {
-                        gate[pb][a >> 1][4 * (a & 1) + c] = (bf16_t)(acc[pb][4 * a + c] + bv[c]);
-                    }
-                }
+            for (int pb = 0; pb < 2; ++pb) {
+                gate[pb][0] = pack8(acc[pb], 0), gate[pb][1] = pack8(acc[pb], 8);
             }
         }
-        // the centre of this wave's positions, eight at a time: lane (k, c) has channel 8 c + k (+ 64 t) of all eight, after
-        // the exchange channels 8 c .. + 7 (+ 64 t) of position k; a position's channels lie in eight consecutive lanes
+        // the centre of this wave's positions: lane l takes channels 8 (l / 16) .. + 7 (+ 32 t) of position l % 16
+        {
+            const lds_char *from = (const lds_char *)raw + (lv >> 4) * 1024 + ((lv >> 2) & 3) * 128 + 8 * (lv & 1);
+            const int slot = (2 * wave + ((lv >> 1) & 1)) ^ (2 * ((lv >> 2) & 3));
+            bf16x8 v[4];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int k8 = lv >> 3, c8 = lv & 7;
-            bf16x8 v[2];
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int ch = 64 * t + 8 * c8 + k8;
-                v[t] = as_bf16x8(transpose8x8_lanes(raw[ch * 8 + ((2 * wave + q) ^ c8)], sel));
+            for (int t = 0; t < 4; ++t) {
+                v[t] = lds_transposed_fragment(from + t * 4096 + 16 * slot, from + t * 4096 + 512 + 16 * (slot ^ 1));
             }
-            const float x0 = __shfl(to_f32(v[0][0]), lv & ~7, 64);
+            const float x0 = __shfl(to_f32(v[0][0]), lv & 15, 64);
             float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
+            for (int t = 0; t < 4; ++t) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const float d = to_f32(v[t][e]) - x0;
@@ -399,21 +399,22 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
                 }
             }
             float rstd, shift;
-            norm_from_sums<true>(group_sum<8>(s1), group_sum<8>(s2), x0, (float)C, eps, rstd, shift);
+            norm_from_sums<true>(half_swap_sum(quarter_swap_sum(s1)), half_swap_sum(quarter_swap_sum(s2)), x0, (float)C, eps, rstd, shift);
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const float *gm = params + 2 * C + 64 * t + 8 * c8, *bt = gm + C;
+            for (int t = 0; t < 4; ++t) {
+                const float *gm = params + 2 * C + 32 * t + 8 * (lv >> 4), *bt = gm + C;
                 bf16x8 o;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     o[e] = (bf16_t)fmaf(fmaf(to_f32(v[t][e]), rstd, shift), gm[e], bt[e]);
                 }
-                cs[row_slot(16 * wave + 8 * q + k8, 8 * t + c8)] = as_uint4(o);
+                cs[row_slot(16 * wave + (lv & 15), 4 * t + (lv >> 4))] = as_uint4(o);
             }
         }
         __syncthreads();
         {
-            f32x16 acc[2] = {zero16(), zero16()};
+            f32x16 acc[2];
+            acc[0] = acc[1] = biases(4);
 #pragma unroll
             for (int ks = 0; ks < CK; ++ks) {
 #pragma unroll
@@ -422,15 +423,14 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
                 }
             }
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const f32x4 bv = *reinterpret_cast<const f32x4 *>(params + 4 * C + wave * 32 + 8 * a + 4 * (lv >> 5));
+            for (int pb = 0; pb < 2; ++pb) {
 #pragma unroll
-                for (int pb = 0; pb < 2; ++pb) {
+                for (int a = 0; a < 4; ++a) {
                     bf16x4 ov;
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
                         // bf16(out) * sigmoid(bf16(gate)), rounded to bf16: the reference's rounding points
-                        const float o = to_f32((bf16_t)(acc[pb][4 * a + c] + bv[c]));
+                        const float o = to_f32((bf16_t)acc[pb][4 * a + c]);
                         ov[c] = (bf16_t)(o * sigmoid_fast(to_f32(gate[pb][a >> 1][4 * (a & 1) + c])));
                     }
                     *(reinterpret_cast<bf16x4 *>(res + row_slot(32 * pb + (lv & 31), 4 * wave + a)) + (lv >> 5)) = ov;
