@@ -539,6 +539,12 @@ hipError_t launch_tiles(const TileParams &p, int64_t blocks, hipStream_t stream)
 int project(const void *a, int64_t a_sm, int64_t m, const void *b, int64_t b_sn, int64_t n, int64_t k, void *c, int64_t c_sm,
             const float *bias, hipStream_t stream)
 {
+    // 64 channels: the row kernel of kutacc_af2_linear keeps the weights in the LDS and streams the rows (whole operator, heads of 8: 1024
+    // rows of 301 210.0 -> 202.9 us, 64 of 48 21.3 -> 20.2).  With 128 and 256 channels its slices of outputs read the rows more than
+    // once, and it loses to the product's tiles (10 rows of 1100, 4 heads of 32: 75.0 against 81.6; 100 of 1200, 8 heads: 573 against 613).
+    if (k == 64 && n == 64 && c_sm == n && a_sm % 8 == 0 && b_sn % 8 == 0 && aligned16(a) && aligned16(b)) {
+        return kutacc_launch::linear(KUTACC_DTYPE_BF16, a, a_sm, b, b_sn, bias, c, m, n, k, 0.f, stream);
+    }
     kutacc_hip_gemm_args_t g = {};
     g.m = m, g.n = n, g.k = k, g.batches = 1;
     g.dtype = KUTACC_DTYPE_BF16, g.path = KUTACC_HIP_PATH_AUTO;

@@ -234,6 +234,35 @@ def test_replays_from_a_hip_graph(torch_cuda):
         assert helpers.same_bits(ten["out"], want_out) and helpers.same_bits(scratch["avg"], want_avg)
 
 
+@pytest.mark.parametrize("B,S,H,d", [(1, 1, 8, 8), (3, 33, 8, 8), (5, 77, 4, 16)])
+def test_output_projection_of_64_channels_on_every_form_of_its_operands(torch_cuda, B, S, H, d):
+    """Dense results on any address take the row kernel; a wider pitch, weights off the 16-byte grid the products' kernels.  All within
+    the parity bar, and so within twice that of each other."""
+    import ctypes
+    torch = torch_cuda
+    w = draw_workload(70 + S, B, S, H, d)
+    want = helpers.oracle_out(w)
+    for form in ("dense", "dense, one element on", "pitch 72", "weights one element on"):
+        ten, scratch = helpers.to_device(w)
+        a = helpers.hip_args(w, ten, scratch, capi.PATH_TILED)
+        room = torch.full((B * S * 72 + 8,), 5.0, device="cuda", dtype=torch.bfloat16)
+        shift, pitch = int(form == "dense, one element on"), 72 if form == "pitch 72" else 64
+        a.out, a.out_ld = room.data_ptr() + 2 * shift, pitch
+        moved = torch.cat([ten["wo"].new_zeros(1), ten["wo"].flatten()])
+        if form == "weights one element on":
+            a.output_w = moved.data_ptr() + 2
+        print(f"64 channels B={B} S={S} H={H} d={d} {form}", flush=True)
+        names = helpers.profiled_kernels(torch, lambda: expect_success(capi.lib().kutacc_hip_gating_attention(ctypes.byref(a), None)))  # noqa: B023
+        assert ("linear_rows_kernel" in names) == form.startswith("dense"), (form, names)
+        used = room[shift:shift + B * S * pitch].view(B, S, pitch)
+        helpers.check_close(helpers.to_numpy(used[..., :64]), want, "bf16", form)
+        assert bool((room[:shift] == 5.0).all()) and bool((room[shift + B * S * pitch:] == 5.0).all()) and bool((used[..., 64:] == 5.0).all())
+
+
+def expect_success(rc):
+    assert rc == 0, rc
+
+
 def test_unsupported_layouts_fall_back_to_the_generic_kernels(torch_cuda):
     """A head size that is no multiple of 8 is not this route's: the automatic choice takes the scalar kernels, the forced
     routes refuse."""
