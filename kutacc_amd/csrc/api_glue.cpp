@@ -324,7 +324,7 @@ int kutacc_hip_triangle_multiplication(const kutacc_hip_triangle_multiplication_
         // as rows.  Its last tiles read on past a plane's edges, into what follows in the workspace, and drop the results.
         const auto plane_of = [](int64_t r, int64_t p) { return (r * p + 63) / 64 * 64 + TM_PLANE_PAD; };
         const int64_t n32 = (n + 31) / 32 * 32;
-        const bool whole_steps = kutacc_launch::triangle_equation_whole_steps(n, ci) && 3 * align256(ci * plane_of(n32, n32) * 2) <= need;
+        const bool whole_steps = kutacc_launch::triangle_equation_whole_steps(n, ci, a->incoming != 0) && 3 * align256(ci * plane_of(n32, n32) * 2) <= need;
         const int64_t np = whole_steps ? n32 : (n + 7) / 8 * 8, lines = whole_steps && a->incoming ? n32 : n;
         const int64_t padded = plane_of(lines, np);
         void *left = ws, *right = ws + align256(ci * padded * 2), *centre = ws + 2 * align256(ci * padded * 2);

@@ -165,9 +165,9 @@ int global_attention(const kutacc_hip_global_attention_args_t &args, hipStream_t
 // nothing launched, when the two cannot share one: the caller then makes two calls)
 int pair_gemm(const kutacc_hip_gemm_args_t &args, hipStream_t stream, const kutacc_hip_gemm_args_t *second = nullptr);
 int gated_projection_mode(); // 0: the default rule (see pair_gemm_tuning)
-// whole_steps, where triangle_equation_whole_steps(n, channels) says so: np a multiple of 32 and, for incoming edges, rows as well, with
+// whole_steps, where triangle_equation_whole_steps says so: np a multiple of 32 and, for incoming edges, rows as well, with
 // zeros past n; 255 rows (columns, incoming) past a plane's end are readable
-bool triangle_equation_whole_steps(int64_t n, int64_t channels);
+bool triangle_equation_whole_steps(int64_t n, int64_t channels, bool incoming);
 int triangle_equation(const void *left, const void *right, void *centre, int64_t n, int64_t rows, int64_t np, int64_t plane, int64_t channels,
                       bool incoming, bool whole_steps, hipStream_t stream);
 // transition.hip

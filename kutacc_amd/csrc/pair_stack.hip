@@ -1642,15 +1642,18 @@ int pair_gemm(const kutacc_hip_gemm_args_t &g, hipStream_t stream, const kutacc_
 int gated_projection_mode() { return g_gated_mode.load(); }
 
 // A length that is no multiple of 256 on the direct kernel, whose last tiles then run over the planes' edges.  Its tiles take
-// half the time of as much work on the 128 x 128 ones but pad more: by default three tiles a side and at most 14 % of
-// padding.  The whole block, us, 128 x 128 tiles against these, outgoing and incoming:
-//   691: 397 358, 384 361    760: 469 414, 453 410    900: 730 693, 716 638    1000: 873 764, 851 749    1250: 1480 1298, 1450 1228
-// and beyond the rule: 508: 173 177, 177 177    640: 300 323, 294 309    800: 534 563, 526 510    1100: 1088 1101, 1071 989
-bool triangle_equation_whole_steps(int64_t n, int64_t channels)
+// half the time of as much work on the 128 x 128 ones, but may pad more.  From three tiles a side on it runs where they pad no more
+// (an even number of 128 x 128 tiles a side), the whole block, us, 128 x 128 tiles against these, outgoing and incoming:
+//   641: 330 328, 320 304    660: 349 334, 341 315    740: 426 383, 414 379    1010: 836 721, 813 687    1180: 1234 1162, 1231 1051
+// and where they do, for incoming edges from four tiles on, for outgoing ones up to 14 % of padding or from six:
+//   800: 505 524, 499 475    896: 579 586, 582 566    1056: 941 968, 944 863    1130: 1082 1019, 1061 969    1290: 1576 1525, 1550 1394
+// Beyond the rule: 508: 159 162, 162 165    560: 228 233, 222 238    620: 282 293, 274 292    640: 276 297, 273 284.
+bool triangle_equation_whole_steps(int64_t n, int64_t channels, bool incoming)
 {
     const int mode = g_big_tile_mode.load();
     const int64_t side = (n + BIG_TILE - 1) / BIG_TILE;
-    const bool pays = side >= 3 && 100 * side * BIG_TILE <= 114 * n;
+    const bool pads_no_more = (n + 127) / 128 == 2 * side;
+    const bool pays = side >= 3 && (pads_no_more || (incoming ? side >= 4 : side >= 6 || 100 * side * BIG_TILE <= 114 * n));
     return n % BIG_TILE != 0 && n > BIG_TILE && n < (1 << 22) && side * side * channels <= INT32_MAX && (mode == 4 || (mode == 0 && pays));
 }
 

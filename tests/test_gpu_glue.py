@@ -774,6 +774,39 @@ def test_triangle_multiplication_block_on_tiles_over_the_edge(torch_cuda, n, mod
         assert bool(torch.isfinite(got[mode]).all()) and helpers.same_bits(got["128"], got[mode]), (n, incoming)
 
 
+# three tiles a side with an even number of 128 x 128 tiles and with an odd one, four with an odd one up to whole tiles, 14 % of padding
+# with an odd number, six
+@pytest.mark.parametrize("n,outgoing,incoming", [(640, False, False), (641, True, True), (769, False, True), (896, False, True), (1122, False, True),
+                                                 (1130, True, True), (1281, True, True)])
+def test_lengths_at_which_the_equation_runs_over_the_edge(torch_cuda, n, outgoing, incoming):
+    """The same bits on either tiles, in a workspace that holds NaN beforehand."""
+    torch = torch_cuda
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *sh, scale=1.0: torch.randn(*sh, device="cuda", generator=g) * scale  # noqa: E731
+    case = tm_block_case(3700 + n, 8, 128, 128)
+    w = {k: torch.from_numpy(np.ascontiguousarray(v)).to(device="cuda", dtype=torch.bfloat16 if v.ndim >= 2 else torch.float32)
+         for k, v in case.items() if k not in ("z", "mask")}
+    act = rnd(n, n, 128).to(torch.bfloat16)
+    mask = (torch.rand(n, n, device="cuda", generator=g) > 0.1).to(torch.bfloat16)
+    for edge, direct in ((False, outgoing), (True, incoming)):
+        got = []
+        for tile in (None, "128"):
+            assert capi.set_tuning("gemm_tile", tile) == 0
+            try:
+                pair = act.clone()
+                blk = capi.TriangleMultiplicationBlock(pair, mask, w, edge)
+                blk.workspace.fill_(255)
+                print(f"n={n} incoming={edge} tile={tile}", flush=True)
+                names = profiled_kernels(torch, lambda: blk.run())  # noqa: B023
+                torch.cuda.synchronize()
+            finally:
+                capi.set_tuning("gemm_tile", None)
+            assert any(k.startswith("pair_gemm_direct_kernel") for k in names) == (direct and tile is None), names
+            got.append(pair)
+        assert bool(torch.isfinite(got[0]).all()) and helpers.same_bits(got[0], got[1]), (n, edge)
+        assert not helpers.same_bits(got[0], act)
+
+
 @pytest.mark.parametrize("n", [48, 72, 384])
 def test_triangle_multiplication_block_on_each_gated_projection_kernel(torch_cuda, n):
     """The block's two gated projections go out in one launch.  Its default kernel (weights in registers, both sides in
