@@ -455,7 +455,7 @@ kutacc_export int kutacc_hip_profile_read(int index, char *name, int name_len, d
  *               "1": wherever it can run; anything else (default): where every workgroup has at least two batch rows, and
  *               an even number of them or many
  *   "streamed"  "1": kutacc_hip_triangle_attention and kutacc_hip_msa_attention with 128 or 256 channels run every length, not
- *               only those beyond 1024, on the attention kernels that keep q, k, v and gate in memory (the workspace functions
+ *               only those beyond 1024 and the larger MSA blocks, on the attention kernels that keep q, k, v and gate in memory (the workspace functions
  *               answer for the setting in force when they are called); anything else: default
  *   "gemm_tile" "128" / "256" / "192" / "direct": the batched products of kutacc_af2_triangle_multiplication_equation
  *               always on 128 x 128 tiles / on 256 x 256 tiles staged through registers wherever the shape has whole

@@ -1167,7 +1167,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
             const float mv = mask_bias_finish(mask_raw[q], part * 64 + lane < S, l2mode ? LOG2E : 1.0f, p.bias_is_mask != 0);
             mask[part * 64 + lane] = mv;
             const unsigned long long nz = __ballot(mv != 0.f);
-            const bool differ = __any(part * 64 + lane < S && (mv == 0.f || mv != __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(mv)))));
+            const bool differ = BPW > 1 && __any(part * 64 + lane < S && (mv == 0.f || mv != __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(mv)))));
             if (lane == 0) {
                 part_flags[part] = ((uint32_t)nz != 0u ? 1u : 0u) | ((uint32_t)(nz >> 32) != 0u ? 2u : 0u) | (differ ? 4u : 0u);
             }
@@ -1179,14 +1179,18 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
     uint32_t flags = 0; // bit t: key tile t needs the mask added (non-zero bias or ragged tail)
     uint32_t differ = 0;
     for (int part = 0; part * 64 < NT * 32; ++part) {
-        flags |= (part_flags[part] & 3u) << (2 * part);
+        flags |= (BPW > 1 ? part_flags[part] & 3u : part_flags[part]) << (2 * part);
         differ |= part_flags[part] & 4u;
     }
     // A row whose keys all have one mask (a padded residue's: -1e9 everywhere) would end with every exponential at zero: its logits are
-    // taken against that mask from the start, which absorbs in each sum what it absorbs in the reference.  Such rows used to be attended
-    // three times (triangle attention of 450 residues, 5 % of them padding, whole block 218 -> 203 us, 203 without padding; 128: 22.9 -> 21.2).
+    // taken against that mask, which absorbs in each sum what it absorbs in the reference, with several blocks a wave from the start.  Such
+    // rows used to be attended three times (triangle attention of 450 residues, 5 % of them padding, whole block 218 -> 203 us, 203 without
+    // padding).  With one block a wave, and in persistent_head_kernel, the choice in front of the loops slows rows without such a mask
+    // (77 residues 22.0 -> 22.15 us, 320 74.4 -> 77.9); there the first pass is made in vain (128 residues 22.9 -> 22.3, 320 85.0 -> 83.3).
+    // persistent_pair_kernel has no register left for either (three more spilled: the operator at 384 residues 88.1 -> 89.5).
+    constexpr bool ONE_PASS = BPW > 1;
     constexpr uint32_t ONE_MASK = 2;
-    if (l2mode && flags != 0u) { // whose loops know no mask, masks, and one mask
+    if (ONE_PASS && l2mode && flags != 0u) { // whose loops know no mask, masks, and one mask
         flags = differ == 0u && one_mask_of(mask, S, lane) != 0.f ? ONE_MASK : 1u;
     }
     const f32x4 *mask4 = reinterpret_cast<const f32x4 *>(mask + 16 * g);
@@ -1215,8 +1219,8 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
         float l;
         if (l2mode) {
             const uint4 *nbf = HAS_NB ? p.nbf + ((int64_t)(h * NB + j) * NT * (TILES ? 4 : 2)) * 64 + lane : nullptr;
-            bool again = false; // shifted by the true row maxima, as some probability overflowed or a whole row underflowed
-            if (flags != ONE_MASK) {
+            bool again = true; // some probability overflowed or a whole row underflowed
+            if (!ONE_PASS || flags != ONE_MASK) {
                 if (flags == 0u) {
                     attend_block_l2<HAS_NB, false, false, TILES>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel,
                                                           NT, lane, 0.f, o, l, (wave >> 2) & 1);
@@ -1227,15 +1231,16 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
                 __builtin_amdgcn_s_setprio(0);
                 again = __any(!(l > 1e-30f && l < 1e30f));
             }
-            while (again || flags == ONE_MASK) {
-                const float shift = again ? row_max_l2<HAS_NB, TILES>(lds_k, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), NT, lane)
-                                          : mask[0];
+            float shift = again ? one_mask_of(mask, S, lane) : 0.f;
+            while (again) { // shifted by the row's one mask, if it has one, or by the true row maxima
+                const bool maxima = shift == 0.f;
+                if (maxima) {
+                    shift = row_max_l2<HAS_NB, TILES>(lds_k, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), NT, lane);
+                }
                 attend_block_l2<HAS_NB, true, true, TILES>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel, NT,
                                                     lane, shift, o, l);
-                if (again || !__any(!(l > 1e-30f && l < 1e30f))) {
-                    break;
-                }
-                again = true;
+                again = !maxima && __any(!(l > 1e-30f && l < 1e30f));
+                shift = 0.f;
             }
         } else {
             const bf16_t *nbrow = HAS_NB ? p.nb + (int64_t)h * p.nb_sh + (int64_t)qrow * p.nb_sq + 16 * g : nullptr;
@@ -1805,12 +1810,11 @@ __device__ __forceinline__ void attend_pair_l2(const uint4 *lds_kA, const uint4 
 }
 
 // The repeat of one row's block after an overflow or underflow of the unshifted exponentials, with the pair bias as fp32
-// tiles: a pass over the key tiles for the true row maxima, and one with them subtracted.  A row whose keys all have one mask (a padded
-// residue's: -1e9 everywhere) does without the first: its logits are taken against that mask, which absorbs in each sum what it
-// absorbs in the reference.  Not a hot path: one row, nothing prefetched, few registers.
+// tiles: a first pass over the key tiles for the true row maxima, a second one with them subtracted.  Not a hot path:
+// one row, nothing prefetched, few registers.
 template <bool HAS_NB>
 __device__ __forceinline__ void attend_row_shifted(const uint4 *lds_k, const uint4 *lds_v, const uint32_t *words, const f32x4 *nbc, bf16x8 q0,
-                                                bf16x8 q1, int NB, int S, int lane, f32x16 &o_out, float &l_out)
+                                                bf16x8 q1, int NB, int lane, f32x16 &o_out, float &l_out)
 {
     // words: the row's mask words (stage_mask_words), offset by 16 (lane >> 5): register 4 a + c stands for key 4 a + c of them
     auto logits = [&](int t) {
@@ -1834,53 +1838,39 @@ __device__ __forceinline__ void attend_row_shifted(const uint4 *lds_k, const uin
         x = mfma(as_bf16x8(lds_k[(t * 2 + 0) * 64 + lane]), q0, x);
         return mfma(as_bf16x8(lds_k[(t * 2 + 1) * 64 + lane]), q1, x);
     };
+    float mx = -INFINITY;
+    for (int t = 0; t < NB; ++t) {
+        const f32x16 x = logits(t);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            mx = fmaxf(mx, x[v]);
+        }
+    }
+    mx = half_swap_max(mx); // finite: a fully masked row has -1e9*log2(e) everywhere
+    f32x16 o = zero16();
+    float lsum = 0.f;
     bf16x2 one2;
     one2[0] = (bf16_t)1.0f, one2[1] = (bf16_t)1.0f;
-    bool differ = false;
-    for (int k = lane & 31; k < S; k += 32) {
-        differ |= (words - 16 * (lane >> 5))[k] != words[-16 * (lane >> 5)];
+    for (int t = 0; t < NB; ++t) {
+        f32x16 x = logits(t);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            x[v] = __builtin_amdgcn_exp2f(x[v] - mx);
+        }
+        const bf16x8 p0 = pack8(x, 0), p1 = pack8(x, 8);
+        o = mfma(as_bf16x8(lds_v[(t * 2 + 0) * 64 + lane]), p0, o);
+        o = mfma(as_bf16x8(lds_v[(t * 2 + 1) * 64 + lane]), p1, o);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            bf16x2 a, c;
+            a[0] = p0[2 * v], a[1] = p0[2 * v + 1];
+            c[0] = p1[2 * v], c[1] = p1[2 * v + 1];
+            lsum = __builtin_amdgcn_fdot2_f32_bf16(a, one2, lsum, false);
+            lsum = __builtin_amdgcn_fdot2_f32_bf16(c, one2, lsum, false);
+        }
     }
-    float shift = __any(differ) ? 0.f : mask_word_value(words[-16 * (lane >> 5)]);
-    bool maxima = false;
-    for (;;) {
-        if (shift == 0.f || maxima) {
-            float mx = -INFINITY;
-            for (int t = 0; t < NB; ++t) {
-                const f32x16 x = logits(t);
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    mx = fmaxf(mx, x[v]);
-                }
-            }
-            shift = half_swap_max(mx), maxima = true; // finite: a row of which every key is masked has at least -1e9*log2(e)
-        }
-        f32x16 o = zero16();
-        float lsum = 0.f;
-        for (int t = 0; t < NB; ++t) {
-            f32x16 x = logits(t);
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                x[v] = __builtin_amdgcn_exp2f(x[v] - shift);
-            }
-            const bf16x8 p0 = pack8(x, 0), p1 = pack8(x, 8);
-            o = mfma(as_bf16x8(lds_v[(t * 2 + 0) * 64 + lane]), p0, o);
-            o = mfma(as_bf16x8(lds_v[(t * 2 + 1) * 64 + lane]), p1, o);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                bf16x2 a, c;
-                a[0] = p0[2 * v], a[1] = p0[2 * v + 1];
-                c[0] = p1[2 * v], c[1] = p1[2 * v + 1];
-                lsum = __builtin_amdgcn_fdot2_f32_bf16(a, one2, lsum, false);
-                lsum = __builtin_amdgcn_fdot2_f32_bf16(c, one2, lsum, false);
-            }
-        }
-        o_out = o;
-        l_out = half_swap_sum(lsum);
-        if (maxima || !__any(!(l_out > 1e-30f && l_out < 1e30f))) {
-            return;
-        }
-        maxima = true;
-    }
+    o_out = o;
+    l_out = half_swap_sum(lsum);
 }
 
 template <int C, bool HAS_NB>
@@ -2079,10 +2069,10 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_pair_kernel(F
         }
         // some probability overflowed or a whole row underflowed: repeat that row shifted by its true row maxima
         if (__any(!(lA > 1e-30f && lA < 1e30f))) {
-            attend_row_shifted<HAS_NB>(kA, vA, mask + 16 * g, nbc, qA0, qA1, NT, S, lane_a, oA, lA);
+            attend_row_shifted<HAS_NB>(kA, vA, mask + 16 * g, nbc, qA0, qA1, NT, lane_a, oA, lA);
         }
         if (__any(!(lB > 1e-30f && lB < 1e30f))) {
-            attend_row_shifted<HAS_NB>(kB, vB, mask + NT * 32 + 16 * g, nbc, qB0, qB1, NT, S, lane_a, oB, lB);
+            attend_row_shifted<HAS_NB>(kB, vB, mask + NT * 32 + 16 * g, nbc, qB0, qB1, NT, lane_a, oB, lB);
         }
         int lane_o = lane; // as above: the addresses of the epilogue are not worth a register during the attention loop
         asm volatile("" : "+v"(lane_o));
