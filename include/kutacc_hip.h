@@ -389,8 +389,8 @@ kutacc_export int kutacc_hip_layernorm_rows_transposed(const void *x, const floa
  *                transposed, the output projection adds its result back transposed).
  * bf16.  With c_m in {128, 256} mask bias and residual update happen inside the operator; any other size runs them as passes
  * of their own around the operator on the tiled MFMA route, with four more activation-sized buffers in the workspace.
- * An attended axis beyond 1024, and for c_m = 256 one beyond 256 with more than 128 sequences (row-wise) or 32 residues
- * (column-wise), runs on the attention kernels that keep q, k, v and gate in memory; for the latter the workspace function asks
+ * An attended axis beyond 1024, and for c_m = 256 one beyond 256 with many sequences (row-wise) or residues (column-wise),
+ * runs on the attention kernels that keep q, k, v and gate in memory; for the latter the workspace function asks
  * for one more activation, and a workspace without it is still enough: the call then runs on the fused kernels.
  * pair_act [n_res, n_res, c_z], its LayerNorm parameters and bias_w [nheads, c_z] are read by the row-wise form only.
  */

@@ -542,14 +542,17 @@ bool msa_block_is_tiled(int64_t n_seq, int64_t n_res, int64_t heads, bool column
 // Blocks that both the fused and the streamed kernels take, and the streamed ones faster: 256 channels, more than 256 keys.
 // Up to 256 keys the fused kernel needs half the waves' registers for K and V and wins (508 sequences x 192 residues 155 against
 // 168 us); beyond, whole blocks of 508 sequences: 259 residues 313 -> 278 us, 512: 575 -> 518, 1000: 1498 -> 1354.
-// Column-wise more than 32 residues (40 x 512 68 -> 61, 256 x 1024 612 -> 577, 384 x 1024 910 -> 853): up to there the fused kernel has one
-// workgroup a CU for its 8 heads a residue, all in one turn (32 x 512 48 against 52).  Row-wise more than 128 sequences (144 x 384 138 -> 131,
-// 192 x 512 238 -> 215; worst 192 x 330 150 against 152): there four rows a wave leave the streamed kernel short of work
-// (128 x 384 112 against 119, 64 x 640 131 against 142).
+// Beyond 256 batch rows always (384 residues x 1024 sequences 910 -> 853).  Up to there where the fused kernel, one workgroup a CU for
+// a row and head, ends with a turn that is at most half full (32 rows of 8 heads fill one): column-wise from 33 residues on (40 x 512 68 -> 61, 104 x 512
+// 119 -> 105), row-wise from 129 sequences on (136 x 384 138 -> 125; 200 x 512 252 -> 240), below which the streamed kernel is short of work
+// (128 x 384 112 against 119, 64 x 640 131 against 142).  With fuller last turns the two are within 3 % of each other while everything lies in the
+// last-level cache, and the streamed kernels, which move four more activations, lose where it does not (91 x 501 96 against 101).
 // Not with the LayerNorm inside the fused kernel, which is asked for to have the smaller workspace.
 bool msa_block_prefers_streamed(int64_t n_seq, int64_t n_res, int64_t heads, bool column)
 {
-    return heads == 8 && (column ? n_seq : n_res) > 256 && (column ? n_res > 32 : n_seq > 128) && !msa_block_is_tiled(n_seq, n_res, heads, column) &&
+    const int64_t rows = column ? n_res : n_seq;
+    return heads == 8 && (column ? n_seq : n_res) > 256 && (rows > 256 || (rows > (column ? 32 : 128) && (rows - 1) % 32 < 16)) &&
+           !msa_block_is_tiled(n_seq, n_res, heads, column) &&
            !layernorm_policy_allows(heads * HEAD);
 }
 

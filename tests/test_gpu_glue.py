@@ -534,10 +534,13 @@ def test_streamed_rows_without_pair_bias_at_the_edges_of_a_workgroup(torch_cuda,
     helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, True), "bf16", f"streamed column {n_seq}x{n_res} heads={heads}")
 
 
-# both sides of each line: more than 256 keys, more than 128 sequences row-wise, more than 32 residues column-wise, 8 heads
+# both sides of each line: more than 256 keys, from 129 sequences row-wise and 33 residues column-wise the first sixteen of every 32, from 257
+# on all, 8 heads
 @pytest.mark.parametrize("column,n_seq,n_res,heads,streamed", [
     (False, 129, 257, 8, True), (False, 128, 257, 8, False), (False, 129, 256, 8, False), (False, 129, 257, 4, False), (False, 130, 1024, 8, True),
-    (True, 257, 33, 8, True), (True, 257, 32, 8, False), (True, 256, 33, 8, False), (True, 257, 33, 4, False), (True, 1023, 34, 8, True)])
+    (True, 257, 33, 8, True), (True, 257, 32, 8, False), (True, 256, 33, 8, False), (True, 257, 33, 4, False), (True, 1023, 34, 8, True),
+    (True, 257, 48, 8, True), (True, 257, 49, 8, False), (True, 257, 256, 8, False), (True, 257, 257, 8, True), (False, 145, 257, 8, False),
+    (False, 281, 257, 8, True)])
 def test_msa_blocks_that_prefer_the_streamed_kernels(torch_cuda, column, n_seq, n_res, heads, streamed):
     """The workspace decides where both kernels take a block: three activations are still enough, for the fused kernels, less is
     refused as before, and so are weights that the fused kernels refuse.  Both give the oracle's result within the parity bar, and so each
