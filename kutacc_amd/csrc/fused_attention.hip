@@ -878,6 +878,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
     constexpr int CK = C / 16;
     constexpr bool V_ALIAS = C == 256 && BPW == 4; // second LDS layout, below
     constexpr bool ONE_GROUP = V_ALIAS || C == 128; // all four weight matrices staged at once, always (see make_plan)
+    constexpr bool ONE_PASS = C == 128 && BPW > 1;  // rows of one mask attended once: see below
     const bool l2mode = TILES || p.l2mode != 0;
     extern __shared__ uint4 lds[];
 
@@ -1167,7 +1168,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
             const float mv = mask_bias_finish(mask_raw[q], part * 64 + lane < S, l2mode ? LOG2E : 1.0f, p.bias_is_mask != 0);
             mask[part * 64 + lane] = mv;
             const unsigned long long nz = __ballot(mv != 0.f);
-            const bool differ = BPW > 1 && __any(part * 64 + lane < S && (mv == 0.f || mv != __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(mv)))));
+            const bool differ = ONE_PASS && __any(part * 64 + lane < S && (mv == 0.f || mv != __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(mv)))));
             if (lane == 0) {
                 part_flags[part] = ((uint32_t)nz != 0u ? 1u : 0u) | ((uint32_t)(nz >> 32) != 0u ? 2u : 0u) | (differ ? 4u : 0u);
             }
@@ -1179,16 +1180,15 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
     uint32_t flags = 0; // bit t: key tile t needs the mask added (non-zero bias or ragged tail)
     uint32_t differ = 0;
     for (int part = 0; part * 64 < NT * 32; ++part) {
-        flags |= (BPW > 1 ? part_flags[part] & 3u : part_flags[part]) << (2 * part);
+        flags |= (ONE_PASS ? part_flags[part] & 3u : part_flags[part]) << (2 * part);
         differ |= part_flags[part] & 4u;
     }
     // A row whose keys all have one mask (a padded residue's: -1e9 everywhere) would end with every exponential at zero: its logits are
-    // taken against that mask, which absorbs in each sum what it absorbs in the reference, with several blocks a wave from the start.  Such
+    // taken against that mask, which absorbs in each sum what it absorbs in the reference; with 128 channels and several blocks a wave from the start.  Such
     // rows used to be attended three times (triangle attention of 450 residues, 5 % of them padding, whole block 218 -> 203 us, 203 without
-    // padding).  With one block a wave, and in persistent_head_kernel, the choice in front of the loops slows rows without such a mask
+    // padding).  With 256 channels (columns of 501 sequences x 91 95.6 -> 96.9), with one block a wave, and in persistent_head_kernel, the choice in front of the loops slows rows without such a mask
     // (77 residues 22.0 -> 22.15 us, 320 74.4 -> 77.9); there the first pass is made in vain (128 residues 22.9 -> 22.3, 320 85.0 -> 83.3).
     // persistent_pair_kernel has no register left for either (three more spilled: the operator at 384 residues 88.1 -> 89.5).
-    constexpr bool ONE_PASS = BPW > 1;
     constexpr uint32_t ONE_MASK = 2;
     if (ONE_PASS && l2mode && flags != 0u) { // whose loops know no mask, masks, and one mask
         flags = differ == 0u && one_mask_of(mask, S, lane) != 0.f ? ONE_MASK : 1u;
