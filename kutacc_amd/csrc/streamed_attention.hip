@@ -290,15 +290,21 @@ struct Walk {
 };
 
 // The gated average of 32 queries of one row in the place of their queries: o / l * sigmoid(gate).  Positions past the row's end are
-// stored like the others: nobody reads them.
+// stored like the others: nobody reads them.  l lies within 1e-30 .. 1e30, or is of a repeated row: 1 .. 2^20.
 __device__ __forceinline__ void store_average(uint4 *dst, uint4 gate0, uint4 gate1, const f32x16 &o, float l)
 {
     const bf16x8 g0 = as_bf16x8(gate0), g1 = as_bf16x8(gate1);
+    const float inv = reciprocal(l);
+    float sigmoid[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        sigmoid[i] = to_f32(i < 8 ? g0[i & 7] : g1[i & 7]);
+    }
+    sigmoids_f32(sigmoid);
     f32x16 out;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) { // l (1 + 2^(-gate log2 e)): one reciprocal for the sum and the sigmoid
-        const float e = __builtin_amdgcn_exp2f(to_f32(i < 8 ? g0[i & 7] : g1[i & 7]) * -LOG2E);
-        out[i] = o[i] * __builtin_amdgcn_rcpf(fmaf(e, l, l));
+    for (int i = 0; i < 16; ++i) {
+        out[i] = o[i] * inv * sigmoid[i];
     }
     dst[0] = as_uint4(pack8(out, 0)), dst[64] = as_uint4(pack8(out, 8));
 }

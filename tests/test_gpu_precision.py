@@ -84,6 +84,78 @@ def test_gate_of_long_rows_keeps_32_bits(torch_cuda, heads):
     assert err < 2.0 ** -8 * (1 + 2.0 ** -7), err  # 2^-15: what 32-bit sums, sigmoid and quotient add, and to spare
 
 
+def halves_to_the_nearest_even(kept):
+    """Averages of `kept` values, half of them 1 and half 1 + 2^-7, or 1 + 2^-7 and 1 + 2^-6: halfway between two bf16.  As the sum (exact)
+    times the rounded reciprocal of the sum of the probabilities gives them, [low, high][row]."""
+    n = np.asarray(kept, dtype=np.float32)
+    inv = np.float32(1.0) / n
+    return [round_to_bf16(n * np.float32(1.0 + k / 256.0) * inv) for k in (1, 3)]
+
+
+@pytest.mark.parametrize("heads,n_seq,n_res,column", [
+    (4, 1030, 512, True), (8, 1030, 512, True), (8, 400, 300, True),  # two blocks of queries a wave
+    (8, 24, 1030, False), (8, 64, 1030, False), (4, 128, 1030, False),  # two rows a wave, four
+])
+def test_sums_of_long_rows_keep_32_bits(torch_cuda, heads, n_seq, n_res, column):
+    """Every probability is one, every average halfway between two bf16: one unit of 32 bits more or less in 1 / sum, as a hardware
+    reciprocal has it, is a bf16 more or less.  Normalised rows are 1, -1, s, -s over and over, s the parity of the key."""
+    torch = torch_cuda
+    C, keys, rows = 32 * heads, n_seq if column else n_res, n_res if column else n_seq
+    kept = np.minimum(2 * (1 + np.arange(rows)), keys // 2 * 2)
+    zeros = torch.zeros(C, C, device="cuda", dtype=torch.bfloat16)
+    wv = zeros.clone()
+    wv[:, 0], wv[:, 2], wv[:, 4] = 1.0, 2.0 ** -8, 2.0 ** -8
+    wv[C // 2:, 4] = 3.0 * 2.0 ** -8
+    w = dict(ln_gamma=torch.ones(C, device="cuda"), ln_beta=torch.zeros(C, device="cuda"), wq=zeros, wk=zeros, wv=wv, wg=zeros,
+             bg=torch.full((C,), 100.0, device="cuda"), wo=torch.eye(C, device="cuda").to(torch.bfloat16), bo=torch.zeros(C, device="cuda"))
+    parity = 1.0 - 2.0 * (torch.arange(keys, device="cuda") % 2)
+    x = torch.ones(keys, C // 4, 4, device="cuda")
+    x[:, :, 1], x[:, :, 2], x[:, :, 3] = -1.0, parity[:, None], -parity[:, None]
+    there = torch.arange(keys, device="cuda")[None, :] < torch.from_numpy(kept).to("cuda")[:, None]
+    act = x.reshape(1, keys, C).expand(rows, keys, C).to(torch.bfloat16)
+    if column:
+        act, there = act.transpose(0, 1), there.transpose(0, 1)
+    act, mask, pair = act.contiguous(), there.to(torch.bfloat16).contiguous(), None
+    if not column:
+        pair = dict(pair_act=torch.zeros(keys, keys, 128, device="cuda", dtype=torch.bfloat16), pair_ln_gamma=torch.ones(128, device="cuda"),
+                    pair_ln_beta=torch.zeros(128, device="cuda"), bias_w=torch.zeros(heads, 128, device="cuda", dtype=torch.bfloat16))
+    print(f"heads={heads} n_seq={n_seq} n_res={n_res} column={column}", flush=True)
+    assert capi.MsaAttentionBlock(act, mask, w, heads, pair).run() == 0
+    torch.cuda.synchronize()
+    got = helpers.to_numpy(act.transpose(0, 1) if column else act)[:, :, 1::4] + 1.0  # channels of -1: the sum with the average is exact
+    for half, want in enumerate(halves_to_the_nearest_even(kept)):
+        wrong = (got[:, :, half * C // 8:(half + 1) * C // 8] != want[:, None, None]).any(axis=(1, 2))
+        assert not wrong.any(), (half, kept[wrong])
+
+
+@pytest.mark.parametrize("heads,n_seq,n_res,column", [(4, 1030, 3, True), (8, 300, 300, True), (8, 24, 1030, False)])
+def test_small_gates_of_long_rows_beside_large_sums(torch_cuda, heads, n_seq, n_res, column):
+    """Logits of 45 on all keys, sums of 2^75, and gates of -45: the average times 3e-20, which the output weights take back to 0.5.
+    Every fourth gate is -100, whose sigmoid is no normal number: no update."""
+    torch = torch_cuda
+    C, keys = 32 * heads, n_seq if column else n_res
+    wq = torch.zeros(C, C, device="cuda", dtype=torch.bfloat16)
+    wq[::32, 0] = 16.0
+    wv = torch.zeros(C, C, device="cuda", dtype=torch.bfloat16)
+    wv[:, 0] = 1.0
+    bg = torch.full((C,), -45.0, device="cuda")
+    bg[3::4] = -100.0
+    w = dict(ln_gamma=torch.ones(C, device="cuda"), ln_beta=torch.zeros(C, device="cuda"), wq=wq, wk=wq, wv=wv, wg=torch.zeros_like(wv),
+             bg=bg, wo=(torch.eye(C, device="cuda") * 2.0 ** 64).to(torch.bfloat16), bo=torch.zeros(C, device="cuda"))
+    x = torch.ones(n_seq, n_res, C, device="cuda", dtype=torch.bfloat16)
+    x[:, :, 1::2] = -1.0
+    act, pair = x.clone(), None
+    if not column:
+        pair = dict(pair_act=torch.zeros(keys, keys, 128, device="cuda", dtype=torch.bfloat16), pair_ln_gamma=torch.ones(128, device="cuda"),
+                    pair_ln_beta=torch.zeros(128, device="cuda"), bias_w=torch.zeros(heads, 128, device="cuda", dtype=torch.bfloat16))
+    print(f"heads={heads} n_seq={n_seq} n_res={n_res} column={column}", flush=True)
+    assert capi.MsaAttentionBlock(act, torch.ones(n_seq, n_res, device="cuda", dtype=torch.bfloat16), w, heads, pair).run() == 0
+    torch.cuda.synchronize()
+    update = 2.0 ** 64 * torch.sigmoid(bg.double())
+    err = float(((act.double() - (x.double() + update)).abs() / (1.0 + 2.0 * update)).max())
+    assert err < 2.0 ** -8, err  # the update and the sum, each rounded once to bf16
+
+
 def run_heads_of_eight(w):
     print(w.name, flush=True)
     ten, scratch = helpers.to_device(w)
