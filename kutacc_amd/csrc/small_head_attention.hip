@@ -257,7 +257,7 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         };
         // Tiles without a mask, tiles with one, and the ragged last one, each in a loop of its own: with their choice inside one loop
         // a tile cost 76 vector instructions and 16 moves of register pairs more than the 160 that it needs (the whole operator, us: 1024
-        // rows of 301 237 -> 221, 1000 of 420 432 -> 381; with one-instruction reciprocals behind the loop 217 and 374).
+        // rows of 301 237 -> 221, 1000 of 420 432 -> 381).
         const int full = S >> 5, plain = min(masked_from, full);
         Raw raw = {zero_u4(), zero_u4()};
         if (S >= 8) {
@@ -332,14 +332,19 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
                 }
                 collect();
             }
-            const float inv = __builtin_amdgcn_rcpf(l);
+            const float inv = reciprocal(l);
             if (pos < S && b0 + i < p.B) {
-                const bf16x4 gv = gates[i];
+                float gate[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    gate[e] = to_f32(gates[i][e]);
+                }
+                sigmoids_f32(gate);
                 bf16x4 ov;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float wavg = to_f32((bf16_t)(values[e] * inv));
-                    ov[e] = (bf16_t)(wavg * sigmoid_fast(to_f32(gv[e])));
+                    ov[e] = (bf16_t)(wavg * gate[e]);
                 }
                 *reinterpret_cast<bf16x4 *>(p.avg + (int64_t)(b0 + i) * S * p.a_ss + h * D + avg_at) = ov;
             }

@@ -192,6 +192,27 @@ def test_masks_of_heads_of_eight_keep_32_bits(torch_cuda, S):
     run_heads_of_eight(w)
 
 
+def test_sums_of_heads_of_eight_keep_32_bits(torch_cuda):
+    """As for the long rows: averages halfway between two bf16, 200 rows of 2 .. 400 keys.  The fourth gate of every head is -100: zero."""
+    B, S = 200, 401
+    w = draw_workload(900, B, S, 8, 8, masked=0.0)
+    kept = 2 * (1 + np.arange(B))
+    for m in (w.wq, w.wk, w.wv, w.wg):
+        m[:] = 0.0
+    w.x[:, :, 0], w.x[:, :, 1] = 1.0, 1.0 - 2.0 * (np.arange(S) % 2)
+    w.wv[:, 0], w.wv[:, 1] = 1.0 + 2.0 ** -7, 2.0 ** -8
+    w.x[:, :, 2], w.wv[:32, 2], w.wv[32:, 2] = 1.0, -(2.0 ** -8), 2.0 ** -8
+    w.bg[:], w.bg[3::8], w.nb[:] = 100.0, -100.0, 0.0
+    w.bias[:] = np.where(np.arange(S)[None, :] < kept[:, None], np.float32(0.0), round_to_bf16(np.full(1, MASK_BIAS, dtype=np.float32)))
+    ten, scratch = helpers.to_device(w)
+    assert helpers.run_hip(w, ten, scratch) == 0 and capi.last_path() == "tiled_mfma"
+    got = helpers.to_numpy(scratch["avg"])
+    assert not got[:, :, :, 3].any()
+    for half, want in enumerate(halves_to_the_nearest_even(kept)):
+        wrong = (got[:, :, 4 * half:4 * half + 4, [0, 1, 2, 4, 5, 6, 7]] != want[:, None, None, None]).any(axis=(1, 2, 3))
+        assert not wrong.any(), (half, kept[wrong])
+
+
 def test_centre_layernorm_of_the_triangle_multiplication_is_exact_to_32_bits(torch_cuda):
     """One residue whose normalised row is the input LayerNorm's beta, small whole numbers, as are then the left projections and, with
     ones to the right, the centre: its sums are exact, and gamma = 2^20 with beta = -2^20 t, t the centre normalised in 32 bits
