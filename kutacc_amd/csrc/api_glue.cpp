@@ -29,20 +29,20 @@ struct Workspace {
 // fused_ln: the head kernel normalises the rows of the pair tensor itself, so no normalised copy is kept.
 // tiled: rows beyond the fused head kernels (more than 1024 residues) -- the operator runs on the tiled MFMA route, which
 // forms k, v and gate in memory, and its result is added to the pair activation by a pass of its own.
-// streamed: the same for 128 and 256 channels -- the attention's own workspace lies at q; k, v, gate and out do not exist
+// streamed: the same for 128 and 256 channels -- the attention's own workspace lies at q, and neither a normalised copy nor
+// an average beside it
 Workspace layout(int64_t n, int64_t heads, bool fused_ln, bool tiled = false, bool streamed = false)
 {
     const int64_t c = heads * HEAD, act = align256(n * n * c * 2);
     Workspace w;
     w.z_norm = 0;
-    w.nb = w.z_norm + (fused_ln ? 0 : act);
+    w.nb = w.z_norm + (fused_ln || streamed ? 0 : act);
     w.bias = w.nb + align256(heads * n * n * 2);
     w.q = w.bias + align256(n * n * 2);
     w.avg = w.q + act;
     w.k = w.v = w.gate = w.out = w.total = w.avg + act;
     if (streamed) {
-        w.avg = w.q + align256(kutacc_launch::streamed_workspace_bytes(n, n, heads, true));
-        w.total = w.avg + act;
+        w.total = w.q + align256(kutacc_launch::streamed_workspace_bytes(n, n, heads, true));
     } else if (tiled) {
         w.v = w.k + act, w.gate = w.v + act, w.out = w.gate + act, w.total = w.out + act;
     }
@@ -212,7 +212,7 @@ int kutacc_hip_triangle_attention(const kutacc_hip_triangle_attention_args_t *a,
         int rc = kutacc_launch::pair_bias(a->pair_act, a->ln_gamma, a->ln_beta, a->bias_w, ws + w.nb, nullptr, n, n, c, heads,
                                           a->ln_eps, KUTACC_DTYPE_BF16, ending, s, opt.nb_tiles_ready ? ws + w.q : nullptr, nb_blocks,
                                           (nb_blocks + 1) & ~1, 1);
-        return rc != 0 ? rc : kutacc_launch::gating_attention_streamed(g, opt, ws + w.q, w.avg - w.q, s);
+        return rc != 0 ? rc : kutacc_launch::gating_attention_streamed(g, opt, ws + w.q, w.total - w.q, s);
     }
     if (tiled) {
         // Rows beyond the fused head kernels: the same chain as separate passes -- LayerNorm + pair bias (read transposed

@@ -287,11 +287,11 @@ def test_glue_launch_layer_rejects_bad_arguments_without_a_device():
     act = n * n * h * 32 * 2
     assert L.kutacc_hip_triangle_attention_workspace(n, h) == 3 * act + h * n * n * 2 + n * n * 2
     assert L.kutacc_hip_triangle_attention_workspace(-1, h) == -1
-    # beyond 1024 residues: normalised copy, q, k, v, gate and average, no seventh activation for the result; the pair bias as bf16 and
-    # as fp32 tiles, mask biases as bf16 and as words with a flag per 32
+    # beyond 1024 residues: q, k, v and gate, no further activation for a normalised copy, the average or the result; the pair bias as
+    # bf16 and as fp32 tiles, mask biases as bf16 and as words with a flag per 32
     n = 2048
     act = n * n * h * 32 * 2
-    assert L.kutacc_hip_triangle_attention_workspace(n, h) == 6 * act + h * n * n * (2 + 4) + n * n * 2 + n * n // 32 * 132
+    assert L.kutacc_hip_triangle_attention_workspace(n, h) == 4 * act + h * n * n * (2 + 4) + n * n * 2 + n * n // 32 * 132
 
 
 def test_global_attention_launch_layer_rejects_long_rows_before_any_launch():

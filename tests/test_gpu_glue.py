@@ -319,7 +319,7 @@ def test_triangle_attention_block_beyond_1024_residues(torch_cuda):
     n = 1088
     c = block_case(9100, n, 4)
     rows = sorted({0, 1, 31, 32, 127, 128, n // 2, n - 65, n - 64, n - 2, n - 1})
-    assert capi.lib().kutacc_hip_triangle_attention_workspace(n, 4) > capi.lib().kutacc_hip_triangle_attention_workspace(1024, 4) * 2
+    assert capi.lib().kutacc_hip_triangle_attention_workspace(n, 4) > 4 * n * n * 128 * 2  # q, k, v and gate
     for ending in (False, True):
         res = {}
         names = profiled_kernels(torch, lambda: res.setdefault("z", run_block(torch, c, ending)))
@@ -473,6 +473,31 @@ def test_triangle_attention_block_of_1025_residues(torch_cuda):
 
 # rows without a partner; whole tiles and one key more or less; four and five query blocks to the last workgroup; sixteen workgroups
 # and one more to a row; a pair bias whose producer does not write the tiles
+@pytest.mark.parametrize("n,ending", [(1, False), (33, True), (1025, True), (1056, False)])
+def test_streamed_triangle_block_stays_within_its_workspace(torch_cuda, streamed_everywhere, n, ending):
+    """The size asked for, NaN beforehand and a guard behind it: the same bits as with any other contents, and the guard untouched; a
+    byte less is refused."""
+    torch = torch_cuda
+    act, w, block = drawn_block(torch, 400 + n, "triangle", 0, n, 4)
+    blk = block(act, w)
+    blk.args.ending_node = int(ending)
+    start, size = act.clone(), blk.args.workspace_bytes
+    res = []
+    for fill in (255, 0):
+        act.copy_(start)
+        room = torch.full((size + 4096,), fill, dtype=torch.uint8, device="cuda")
+        room[size:] = 90
+        blk.args.workspace = room.data_ptr()
+        print(f"n={n} ending={ending} fill={fill}", flush=True)
+        assert blk.run() == 0
+        torch.cuda.synchronize()
+        assert bool((room[size:] == 90).all())
+        res.append(act.clone())
+    assert bool(torch.isfinite(res[0]).all()) and helpers.same_bits(res[0], res[1]) and not helpers.same_bits(res[0], start)
+    blk.args.workspace_bytes = size - 1
+    assert blk.run() == capi.EINVAL
+
+
 @pytest.mark.parametrize("column,n_seq,n_res,heads,c_z", [(False, 1, 1056, 4, 128), (True, 1055, 3, 4, 1), (True, 1057, 5, 8, 1), (True, 1152, 2, 4, 1),
                                                           (True, 1153, 1, 8, 1), (True, 2048, 2, 8, 1), (True, 2049, 3, 4, 1), (False, 2, 1281, 8, 16)])
 def test_msa_attention_blocks_beyond_1024_keys(torch_cuda, column, n_seq, n_res, heads, c_z):
