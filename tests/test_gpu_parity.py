@@ -19,6 +19,7 @@ from kutacc_amd import capi
 from kutacc_amd.workloads import CONFIGS, Workload, bf16_bits, make_workload, round_to_bf16
 
 import helpers
+from test_gpu_tiled_attention import draw_workload
 
 pytestmark = pytest.mark.gpu
 
@@ -229,11 +230,12 @@ def test_seeded_shape_sweep_matches_oracle(torch_cuda, index, config, batch, seq
     helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, w.dtype, f"sweep {index} out")
 
 
-# one, two, three and four query blocks a wave, the persistent kernels of one row and of two
+# one row a workgroup: the persistent kernel, and several query blocks a wave
 @pytest.mark.parametrize("lifted", [False, True])
 @pytest.mark.parametrize("config,seq", [(5, 40), (5, 128), (5, 200), (5, 290), (5, 384), (5, 420), (5, 700), (5, 1000), (4, 200), (4, 300), (4, 1000)])
 def test_rows_whose_keys_all_have_one_mask(torch_cuda, config, seq, lifted):
-    """Their logits are taken against that mask from the start.  lifted: a pair bias of 444, which -1e9 absorbs to 448 in the oracle's
+    """Their logits are taken against that mask, with 128 channels and several blocks a wave from the start, elsewhere when the first pass
+    has run out of range.  lifted: a pair bias of 444, which -1e9 absorbs to 448 in the oracle's
     units and to 640 / log2(e) in the kernels': the exponentials overflow all the same and the row is repeated with its true maxima."""
     w = make_workload(config, batch=9, seq_len=seq)
     w.bias[:] = 0.0
@@ -252,6 +254,42 @@ def test_rows_whose_keys_all_have_one_mask(torch_cuda, config, seq, lifted):
     ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
     helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), ref_avg, w.dtype, "gated average")
     helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, w.dtype, "out")
+
+
+# kernels that take over from a second row a workgroup on, whose rows of one mask are repeated: a workgroup per row and head with one block a
+# wave, on fp16 fragments of the pair bias (66 x 96, 256 channels 40 x 77) and on fp32 tiles (130 x 97); the persistent one on fp32 tiles (rows by
+# themselves) and the one of two rows
+@pytest.mark.parametrize("lifted", [False, True])
+@pytest.mark.parametrize("heads,batch,seq,pair_bias,kernel", [
+    (4, 66, 96, True, "fused_head_kernel"), (8, 40, 77, True, "fused_head_kernel"), (8, 40, 77, False, "fused_head_kernel"),
+    (4, 130, 97, True, "fused_head_kernel"), (4, 135, 135, True, "persistent_head_kernel"), (8, 70, 100, True, "persistent_head_kernel"),
+    (4, 128, 160, True, "persistent_pair_kernel"), (8, 64, 200, True, "persistent_pair_kernel")])
+def test_rows_whose_keys_all_have_one_mask_in_larger_batches(torch_cuda, heads, batch, seq, pair_bias, kernel, lifted):
+    w = draw_workload(1200 + batch + seq, batch, seq, heads, 32, pair_bias, masked=0.0)
+    masked = round_to_bf16(np.full(seq, -1e9, dtype=np.float32))
+    w.bias[:] = 0.0
+    w.bias[::3, :] = masked
+    w.bias[1::9, :] = -3.0
+    w.bias[2::9, : seq - 1] = masked[1:]  # all but the last key
+    w.bias[4::9, 1:] = masked[1:]         # all but the first
+    w.bias[5::9, seq // 2:] = masked[seq // 2:]
+    w.bias[batch - 1, :] = masked
+    if lifted and w.nb is not None:
+        w.nb = np.full((w.H, seq, seq), 444.0, dtype=np.float32)
+    want_out, want_avg = helpers.oracle_out(w, return_avg=True)
+    for pairs in (None, "0", "1"):
+        ten, scratch = helpers.to_device(w)
+        assert capi.set_tuning("row_pairs", pairs) == 0
+        print(f"one mask: heads={heads} {batch} x {seq} lifted={lifted} row_pairs={pairs}", flush=True)
+        try:
+            rc = {}
+            names = helpers.profiled_kernels(torch_cuda, lambda: rc.setdefault("rc", helpers.run_hip(w, ten, scratch, capi.PATH_FUSED)))  # noqa: B023
+        finally:
+            capi.set_tuning("row_pairs", None)
+        runs = {None: kernel, "0": kernel.replace("pair", "head"), "1": "persistent_pair_kernel"}[pairs]
+        assert rc["rc"] == 0 and [k for k in names if k.endswith(("head_kernel", "pair_kernel"))] == [runs], (rc, names)
+        helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), want_avg, w.dtype, f"gated average, row_pairs={pairs}")
+        helpers.check_close(helpers.to_numpy(ten["out"]), want_out, w.dtype, f"out, row_pairs={pairs}")
 
 
 # ---- the two-row persistent kernel (128 channels, up to 384 keys), forced wherever it can run --------------------------
