@@ -271,9 +271,10 @@ kutacc_export int kutacc_hip_residual_add(void *acc, const void *delta, int64_t 
  * on the transposed pair tensor, result transposed back).  Four device passes on `stream`: LayerNorm + pair-bias
  * projection (one read of pair_act), mask bias, the attention operator, residual update.  bf16, head_size 32,
  * c_z = nheads * 32.  With c_z in {128, 256} and n_res <= 1024 (the shapes of the fused MFMA attention kernels) the
- * mask bias and the residual update happen inside the operator: three launches.  Any other size runs the chain as
- * separate passes with the operator on the tiled MFMA route (KUTACC_HIP_PATH_TILED), which needs four more
- * activation-sized buffers -- the workspace function answers for the size it is asked about.  `workspace`: device memory,
+ * mask bias and the residual update happen inside the operator: three launches.  Longer chains of these channels run on
+ * the attention kernels that keep q, k, v and gate in memory: one more activation-sized buffer and a second copy of the pair
+ * bias.  Any other number of channels runs the chain as separate passes with the operator on the tiled MFMA route
+ * (KUTACC_HIP_PATH_TILED), which needs four more -- the workspace function answers for the size it is asked about.  `workspace`: device memory,
  * 256-byte aligned, at least kutacc_hip_triangle_attention_workspace(n_res, nheads) bytes; contents unspecified afterwards.
  */
 typedef struct kutacc_hip_triangle_attention_args {

@@ -539,11 +539,15 @@ bool msa_block_is_tiled(int64_t n_seq, int64_t n_res, int64_t heads, bool column
     return beyond_fused_kernels(column ? n_seq : n_res, heads) || block_is_streamed(column ? n_seq : n_res, heads);
 }
 
+// Batch rows of 8 heads whose workgroups of the fused kernel, one a CU, fill the chip once: the 256 CUs of an MI355X by 8.  A constant,
+// because the workspace functions answer without a device; with another number of CUs the rule below is still right, only not the faster one.
+constexpr int64_t FUSED_TURN_ROWS = 32;
+
 // Blocks that both the fused and the streamed kernels take, and the streamed ones faster: 256 channels, more than 256 keys.
 // Up to 256 keys the fused kernel needs half the waves' registers for K and V and wins (508 sequences x 192 residues 155 against
 // 168 us); beyond, whole blocks of 508 sequences: 259 residues 313 -> 278 us, 512: 575 -> 518, 1000: 1498 -> 1354.
 // Beyond 256 batch rows always (384 residues x 1024 sequences 910 -> 853).  Up to there where the fused kernel, one workgroup a CU for
-// a row and head, ends with a turn that is at most half full (32 rows of 8 heads fill one): column-wise from 33 residues on (40 x 512 68 -> 61, 104 x 512
+// a row and head, ends with a turn that is at most half full: column-wise from 33 residues on (40 x 512 68 -> 61, 104 x 512
 // 119 -> 105), row-wise from 129 sequences on (136 x 384 138 -> 125; 200 x 512 252 -> 240), below which the streamed kernel is short of work
 // (128 x 384 112 against 119, 64 x 640 131 against 142).  With fuller last turns the two are within 3 % of each other while everything lies in the
 // last-level cache, and the streamed kernels, which move four more activations, lose where it does not (91 x 501 96 against 101).
@@ -551,7 +555,8 @@ bool msa_block_is_tiled(int64_t n_seq, int64_t n_res, int64_t heads, bool column
 bool msa_block_prefers_streamed(int64_t n_seq, int64_t n_res, int64_t heads, bool column)
 {
     const int64_t rows = column ? n_res : n_seq;
-    return heads == 8 && (column ? n_seq : n_res) > 256 && (rows > 256 || (rows > (column ? 32 : 128) && (rows - 1) % 32 < 16)) &&
+    return heads == 8 && (column ? n_seq : n_res) > 256 && (rows > 8 * FUSED_TURN_ROWS ||
+            (rows > (column ? 1 : 4) * FUSED_TURN_ROWS && (rows - 1) % FUSED_TURN_ROWS < FUSED_TURN_ROWS / 2)) &&
            !msa_block_is_tiled(n_seq, n_res, heads, column) &&
            !layernorm_policy_allows(heads * HEAD);
 }

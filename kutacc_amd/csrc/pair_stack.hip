@@ -1646,7 +1646,7 @@ int gated_projection_mode() { return g_gated_mode.load(); }
 // (an even number of 128 x 128 tiles a side), the whole block, us, 128 x 128 tiles against these, outgoing and incoming:
 //   641: 330 328, 320 304    660: 349 334, 341 315    740: 426 383, 414 379    1010: 836 721, 813 687    1180: 1234 1162, 1231 1051
 // and where they do, for incoming edges from four tiles on, for outgoing ones up to 14 % of padding or from six:
-//   800: 505 524, 499 475    896: 579 586, 582 566    1056: 941 968, 944 863    1130: 1082 1019, 1061 969    1290: 1576 1525, 1550 1394
+//   769: 486 511, 469 459    800: 505 524, 499 475    896: 579 586, 582 566    1056: 941 968, 944 863    1130: 1082 1019, 1061 969    1290: 1576 1525, 1550 1394
 // Beyond the rule: 508: 159 162, 162 165    560: 228 233, 222 238    620: 282 293, 274 292    640: 276 297, 273 284.
 bool triangle_equation_whole_steps(int64_t n, int64_t channels, bool incoming)
 {

@@ -380,8 +380,8 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
 // multiplied, 64 outputs at a time out through the same panel.  A lane ends up with one row and four consecutive outputs per
 // accumulator group.  The addition of beta * result is a kernel of its own (its sixteen guarded loads per block of outputs are sixteen
 // branches, taken or not), groups of eight outputs past n are skipped, and with 128 registers four workgroups share a CU up to 128
-// features.  The call, us: 147 456 rows x 128 -> 8 54.5 on the scalar kernel, 9.8 without these, 8.0 here (5.0 TB/s); 100 000
-// x 128 -> 128 19.1 -> 15.7; 300 000 x 256 -> 256 105.5 -> 98.2.
+// features.  The call on new rows, us: 147 456 x 128 -> 8 11.1 without these, 9.1 here (4.4 TB/s; the kernel alone 8.1 on average), 54.5 on
+// the scalar kernel; over and over on the same rows, 100 000 x 128 -> 128 19.1 -> 15.7; 300 000 x 256 -> 256 105.5 -> 98.2.
 template <int K, bool BETA>
 __global__ __launch_bounds__(256, K == 256 ? 2 : 4) void linear_rows_kernel(const bf16_t *__restrict__ act, int64_t ld_act, const bf16_t *__restrict__ w,
                                                           int64_t ld_w, const float *__restrict__ bias, bf16_t *__restrict__ out, int64_t m,

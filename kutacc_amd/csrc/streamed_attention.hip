@@ -1,7 +1,7 @@
 // Gated attention of long batch rows for gfx950, bf16 storage, head size 32, 128 or 256 channels: the rows whose keys and
 // values do not fit the LDS twice beside a head's weights (persistent_pair_kernel), in batches that fill the chip.
 //
-// Three kernels share the work, with K, V, Q, the gate and the gated average in memory between them:
+// Four kernels, of which a call runs three, with K, V, Q, the gate and the gated average in memory between them:
 //
 //   qkvg_projection_kernel    reads the input rows once, forms all four projections and writes them as the MFMA fragments
 //       the attention loads -- 1 KB per store instruction, no layout change anywhere after it.
@@ -54,8 +54,9 @@ struct StreamedParams {
     // [batch row][head][block of 32 positions][2 k-steps][64 lanes]; the gated average takes the place of the queries it was formed from
     uint4 *q, *g, *k, *v;
     // [batch row][block][32]: mask bias of key pi(i) in log2 units as two bf16 (mask_word).  Their 2^-17 moves no probability: the bias
-    // is formed from a bf16 mask, so it is 0, or at least 3.9e6 in size and 2^-8 of that from any other.  (A third part was 7 %
-    // slower at 2048 residues, a tenth of them masked.)
+    // is formed from a bf16 mask, so it is 0, or at least 3.9e6 in size and 2^-8 of that from any other: two keys' masks differ by
+    // thousands or by nothing.  The fused kernels keep the bias in fp32; blocks of up to 1024 keys that run here instead get the same
+    // probabilities.  (A third part was 7 % slower at 2048 residues, a tenth of them masked.)
     uint32_t *words;
     // [batch row][block]: 0, no key of the block has a mask; the word that all its keys have (those of the row, the tail is at -inf);
     // MIXED_WORDS otherwise
@@ -487,7 +488,8 @@ __global__ __launch_bounds__(512) void streamed_attention_kernel(const StreamedP
     // A row whose keys all have one mask (a padded residue's: -1e9 everywhere) would end with every exponential at zero.  Its logits
     // are taken against that mask from the start: x = (q.k + bias + mask) - mask, each sum rounded, so that the mask absorbs what
     // it absorbs in the reference.  shift: the word of the -mask, 0 for other rows.  Such rows used to be attended twice more, by
-    // attend_shifted: 2048 residues, 4 % of them padding, 1.4 ms of 8.0.
+    // attend_shifted: 2048 residues, 4 % of them padding, 1.4 ms of 8.0.  The masked loop adds the shift of every row, zero or not (2048
+    // residues without the first one 9.46 ms, whole 7.83; two rows a wave with one product 10.9 and 8.78).
     uint32_t shift[ROWS];
 #pragma unroll
     for (int i = 0; i < ROWS; ++i) {
@@ -645,7 +647,7 @@ __global__ __launch_bounds__(512) void streamed_attention_kernel(const StreamedP
 // The same without a pair bias, where batch rows share nothing: a wave attends two blocks of 32 queries of one row, which share its
 // keys, values and masks.  A workgroup walks the row's keys once for all its blocks; each of its waves brings one tile (4 KB) of a group.
 // Bound by issue and power: 1024 sequences x 384 residues x 8 heads 520 us, 295 clocks a tile of 32 x 32 logits and SIMD, at the
-// 1.8 GHz that the chip holds under it.  Two rows a wave, which share nothing, 541 us; four blocks a wave on two waves a SIMD 526; two
+// 1.8 GHz that the chip holds under it (some 10 us more with the rounded quotients behind the loop).  Two rows a wave, which share nothing, 541 us; four blocks a wave on two waves a SIMD 526; two
 // blocks on four waves of 128 registers 523.  3000 x 60 685 -> 605, 700 x 256 211 -> 192, 300 x 100 25.2 -> 26.2 us.
 __global__ __launch_bounds__(768) void streamed_plain_kernel(const StreamedParams p)
 {

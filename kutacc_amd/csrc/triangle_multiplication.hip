@@ -13,8 +13,8 @@
 // np is a multiple of 8: a wave follows (i, j) of its eights with scalar additions.
 //
 // Both are bound by vector issue at two waves per SIMD (246 and 237 registers) as much as by HBM: at 384 residues each moves its 113 MB
-// (front: 256 bytes in, 512 out per position; back: 512 in, 256 out) in 38 to 39 us, 60 % of the rate of a copy, with the vector ALU
-// taken for 45 % of the clocks and the matrix cores for 18 and 9.  Neither reads a normalised copy of the pair activation: the front kernel normalises the rows on their way into the LDS, the back kernel does it again for
+// (front: 256 bytes in, 512 out per position; back: 512 in, 256 out) in 40 to 41 us on average and 38 at best, 60 % of the rate of a copy,
+// with the vector issue ports taken for 63 and 56 % of the clocks and the matrix cores for 26 and 12.  Neither reads a normalised copy of the pair activation: the front kernel normalises the rows on their way into the LDS, the back kernel does it again for
 // its gate, from the same rows that its residual needs.  At 384 residues that saves a pass of 76 MB and a read of 38 MB.
 #include <hip/hip_runtime.h>
 
