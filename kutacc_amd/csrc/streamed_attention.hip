@@ -394,15 +394,6 @@ __global__ __launch_bounds__(512) void streamed_attention_kernel(const StreamedP
     if (ROWS * set >= p.B || qg >= p.query_groups) {
         return;
     }
-    const int j = qg * WAVES + wave;
-    int b[ROWS]; // past the last row: that one again, not stored
-    int64_t row[ROWS]; // first fragment block
-#pragma unroll
-    for (int i = 0; i < ROWS; ++i) {
-        b[i] = min(ROWS * set + i, p.B - 1);
-        row[i] = ((int64_t)b[i] * p.H + h) * NB;
-    }
-
     // The pieces u = 4 wave + i of a group of tiles: tile u / (4 ROWS), piece u % (4 ROWS) = [row][K, V][k-step].  Written out: as a builtin
     // the compiler takes every LDS read behind it for a reader of its data and waits for all loads in flight.
     const uint32_t ring = (uint32_t)(uintptr_t)(lds_ptr)lds, lane_bytes = 16u * (uint32_t)lane;
@@ -418,230 +409,253 @@ __global__ __launch_bounds__(512) void streamed_attention_kernel(const StreamedP
     };
     request(0, 0);
     request(W::TILES_PER_GROUP, 1);
-    int fill = 2, fill_tile = 2 * W::TILES_PER_GROUP; // the next group to ask for: its place in the ring, its first tile
-    // Behind the last keys each wave asks for the gates of its own queries, two rows at a time, four pieces as well, so that they wait
-    // in the ring when the loop ends (asked for there, they were a round trip at the end of every workgroup).
-    int gates = 0, gate_place = 0; // rows asked for; the place of the first two
-    auto refill = [&] {
-        if (fill_tile < NB) {
-            request(fill_tile, fill);
-        } else if (gates < ROWS && j < NB) {
-            gate_place = gates == 0 ? fill : gate_place;
-            const uint32_t to = ring + (uint32_t)fill * W::GROUP_BYTES + (uint32_t)wave * 4096u;
-            const uint4 *first = p.g + ((gates == 0 ? row[0] : row[ROWS - 2]) + j) * BLOCK_SLOTS;
-            const uint4 *second = p.g + ((gates == 0 ? row[1] : row[ROWS - 1]) + j) * BLOCK_SLOTS;
-            load_to_lds(to, first, lane_bytes);
-            load_to_lds(to + 1024u, first + 64, lane_bytes);
-            load_to_lds(to + 2048u, second, lane_bytes);
-            load_to_lds(to + 3072u, second + 64, lane_bytes);
-            gates += 2;
+    // Rows first .. first + N - 1 of the set, the queries of block j.
+    auto attend = [&](int j, int first, auto rows_attended) __attribute__((always_inline)) {
+        constexpr int N = decltype(rows_attended)::value;
+        int b[N]; // past the last row: that one again, not stored
+        int64_t row[N]; // first fragment block
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            b[i] = min(ROWS * set + first + i, p.B - 1);
+            row[i] = ((int64_t)b[i] * p.H + h) * NB;
         }
-        fill = fill == RING - 1 ? 0 : fill + 1;
-        fill_tile += W::TILES_PER_GROUP;
-    };
-    if (j >= NB) { // a wave without queries brings its share of the keys
-        for (int t = 0; t < NB; t += W::TILES_PER_GROUP) {
-            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-            refill();
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        return;
-    }
 
-    bf16x8 q[ROWS][2];
-#pragma unroll
-    for (int i = 0; i < ROWS; ++i) {
-        const uint4 *src = p.q + (row[i] + j) * BLOCK_SLOTS;
-        q[i][0] = as_bf16x8(src[lane]), q[i][1] = as_bf16x8(src[64 + lane]);
-    }
-    const f32x4 *nbc = p.tiles + ((int64_t)h * NB + j) * p.NT * 256;
-    auto load_nb = [&](int t) {
-        f32x16 c;
-        const char *tile = reinterpret_cast<const char *>(nbc + min(t, NB - 1) * 256); // uniform; the lane's part in 32 bits
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            const f32x4 v = *reinterpret_cast<const f32x4 *>(tile + (lane_bytes + 1024u * a));
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                c[4 * a + e] = v[e];
+        int fill = 2, fill_tile = 2 * W::TILES_PER_GROUP; // the next group to ask for: its place in the ring, its first tile
+        // Behind the last keys each wave asks for the gates of its own queries, two rows at a time, four pieces as well, so that they wait
+        // in the ring when the loop ends (asked for there, they were a round trip at the end of every workgroup).
+        int gates = 0, gate_place = 0; // rows asked for; the place of the first two
+        auto refill = [&] {
+            if (fill_tile < NB) {
+                request(fill_tile, fill);
+            } else if (gates < N && j < NB) {
+                gate_place = gates == 0 ? fill : gate_place;
+                const uint32_t to = ring + (uint32_t)fill * W::GROUP_BYTES + (uint32_t)wave * 4096u;
+                const uint4 *first = p.g + ((gates == 0 ? row[0] : row[N - 2]) + j) * BLOCK_SLOTS;
+                const uint4 *second = p.g + ((gates == 0 ? row[1] : row[N - 1]) + j) * BLOCK_SLOTS;
+                load_to_lds(to, first, lane_bytes);
+                load_to_lds(to + 1024u, first + 64, lane_bytes);
+                load_to_lds(to + 2048u, second, lane_bytes);
+                load_to_lds(to + 3072u, second + 64, lane_bytes);
+                gates += 2;
             }
-        }
-        return c;
-    };
-    f32x16 C0 = load_nb(0), C1 = load_nb(1);
-
-    // first key tile in which a row has a mask (the ragged tail of a row counts: its keys are at -inf)
-    int masked_from = NB;
-    for (int t0 = 0; t0 < NB; t0 += 64) {
-        uint32_t f = 0;
-#pragma unroll
-        for (int i = 0; i < ROWS; ++i) {
-            f |= t0 + lane < NB ? p.flags[(int64_t)b[i] * NB + t0 + lane] : 0u;
-        }
-        const unsigned long long any = __ballot(f != 0u);
-        if (any != 0) {
-            masked_from = t0 + __builtin_ctzll(any);
-            break;
-        }
-    }
-
-    // A row whose keys all have one mask (a padded residue's: -1e9 everywhere) would end with every exponential at zero.  Its logits
-    // are taken against that mask from the start: x = (q.k + bias + mask) - mask, each sum rounded, so that the mask absorbs what
-    // it absorbs in the reference.  shift: the word of the -mask, 0 for other rows.  Such rows used to be attended twice more, by
-    // attend_shifted: 2048 residues, 4 % of them padding, 1.4 ms of 8.0.  The masked loop adds the shift of every row, zero or not (2048
-    // residues without the first one 9.46 ms, whole 7.83; two rows a wave with one product 10.9 and 8.78).
-    uint32_t shift[ROWS];
-#pragma unroll
-    for (int i = 0; i < ROWS; ++i) {
-        shift[i] = 0;
-        if (masked_from == 0) {
-            const uint32_t *flags = p.flags + (int64_t)b[i] * NB;
-            const uint32_t f = flags[0];
-            bool differs = f == MIXED_WORDS || f == 0;
-            for (int t0 = 0; t0 < NB && !differs; t0 += 64) {
-                differs = __any(flags[min(t0 + lane, NB - 1)] != f);
+            fill = fill == RING - 1 ? 0 : fill + 1;
+            fill_tile += W::TILES_PER_GROUP;
+        };
+        if (j >= NB) { // a wave without queries brings its share of the keys
+            for (int t = 0; t < NB; t += W::TILES_PER_GROUP) {
+                asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+                refill();
             }
-            shift[i] = __builtin_amdgcn_readfirstlane(differs ? 0u : f ^ 0x80008000u);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            return;
         }
-    }
 
-    // The mask of a row as a rank-one MFMA: A holds (hi, lo) of the key of accumulator row i in k-slots 0 and 1, B ones there,
-    // all else zero, also in the lanes of the upper half, so that an infinite mask value never meets a zero.
-    const uint32_t lower = lane < 32 ? 0xffffffffu : 0u;
-    auto mask_word_of = [&](int i, int t) { return p.words[((int64_t)b[i] * NB + min(t, NB - 1)) * 32 + (lane & 31)] & lower; };
-    auto add_mask = [&](f32x16 x, uint32_t w) {
-        const bf16x8 ones = as_bf16x8(make_uint4(0x3f803f80u & lower, 0u, 0u, 0u));
-        return mfma(as_bf16x8(make_uint4(w, 0u, 0u, 0u)), ones, x);
-    };
-
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); // groups 0 and 1 have landed, every wave's part of them
-    refill();
-    int left = W::TILES_PER_GROUP; // tiles of the current group still to come, this one included
-    const uint4 *cur = lds, *const end = lds + RING * W::TILES_PER_GROUP * W::TILE_SLOTS, *next = lds + W::TILE_SLOTS; // tiles t and t + 1
-    auto keys = [&](const uint4 *tile, int i) { return tile + i * 2 * BLOCK_SLOTS + lane; };
-    auto values = [&](const uint4 *tile, int i) { return tile + i * 2 * BLOCK_SLOTS + BLOCK_SLOTS + lane; };
-    uint4 k0 = keys(cur, 0)[0], k1 = keys(cur, 0)[64], v0, v1;
-    f32x16 x[2]; // logits: of row i in x[i & 1]
-    x[0] = mfma(as_bf16x8(k0), q[0][0], C0);
-    x[0] = mfma(as_bf16x8(k1), q[0][1], x[0]);
-    k0 = keys(cur, 1)[0], k1 = keys(cur, 1)[64];
-    v0 = values(cur, 0)[0], v1 = values(cur, 0)[64];
-    f32x16 o[ROWS];
-    f32x4 sums[ROWS]; // the row sums on the matrix pipe: see rowsum_selector
-    uint32_t m[ROWS]; // the mask words of a row's next logits
+        bf16x8 q[N][2];
 #pragma unroll
-    for (int i = 0; i < ROWS; ++i) {
-        o[i] = zero16(), sums[i] = f32x4{0.f, 0.f, 0.f, 0.f}, m[i] = 0;
-    }
-    const bf16x8 ones_rows = rowsum_selector(lane);
-
-    auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
-    // Tile t with seed C: finishes row i = 0 .. ROWS - 1, each time softmax and P.V of the finished logits, the logits of the next row (of
-    // the first one and tile t + 1, from seed Cn, behind the last), and the fragments of the row behind that.  The fences deal the
-    // exponentials between the MFMAs.  The empty asm keeps C live past the MFMA that reads it, so that the logits get registers of their own.
-    auto tile = [&](int t, f32x16 &C, f32x16 &Cn, auto masked) __attribute__((always_inline)) {
+        for (int i = 0; i < N; ++i) {
+            const uint4 *src = p.q + (row[i] + j) * BLOCK_SLOTS;
+            q[i][0] = as_bf16x8(src[lane]), q[i][1] = as_bf16x8(src[64 + lane]);
+        }
+        const f32x4 *nbc = p.tiles + ((int64_t)h * NB + j) * p.NT * 256;
+        auto load_nb = [&](int t) {
+            f32x16 c;
+            const char *tile = reinterpret_cast<const char *>(nbc + min(t, NB - 1) * 256); // uniform; the lane's part in 32 bits
 #pragma unroll
-        for (int i = 0; i < ROWS; ++i) {
-            constexpr int LAST = ROWS - 1;
-            const int n = i == LAST ? 0 : i + 1, nn = (i + 2) % ROWS; // the next row, the one behind it
-            f32x16 &xc = x[i & 1], &xn = x[n & 1];
-            auto exp4 = [&](int base) {
+            for (int a = 0; a < 4; ++a) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(tile + (lane_bytes + 1024u * a));
 #pragma unroll
-                for (int e = base; e < base + 4; ++e) {
-                    xc[e] = __builtin_amdgcn_exp2f(xc[e]);
+                for (int e = 0; e < 4; ++e) {
+                    c[4 * a + e] = v[e];
                 }
-            };
-            exp4(0);
-            if (i == LAST) {
-                xn = mfma(as_bf16x8(k0), q[n][0], Cn);
-                asm volatile("" ::"v"(Cn));
-            } else {
-                xn = mfma(as_bf16x8(k0), q[n][0], C);
-                asm volatile("" ::"v"(C));
             }
-            fence();
-            exp4(4);
-            const bf16x8 p0 = pack8(xc, 0);
-            xn = mfma(as_bf16x8(k1), q[n][1], xn);
-            if constexpr (decltype(masked)::value) {
-                xn = add_mask(add_mask(xn, m[n]), shift[n] & lower);
+            return c;
+        };
+        f32x16 C0 = load_nb(0), C1 = load_nb(1);
+
+        // first key tile in which a row has a mask (the ragged tail of a row counts: its keys are at -inf)
+        int masked_from = NB;
+        for (int t0 = 0; t0 < NB; t0 += 64) {
+            uint32_t f = 0;
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                f |= t0 + lane < NB ? p.flags[(int64_t)b[i] * NB + t0 + lane] : 0u;
             }
-            const uint4 *kf = keys(i + 2 < ROWS ? cur : next, nn);
-            k0 = kf[0], k1 = kf[64];
-            fence();
-            exp4(8);
-            o[i] = mfma(as_bf16x8(v0), p0, o[i]);
-            fence();
-            exp4(12);
-            const bf16x8 p1 = pack8(xc, 8);
-            sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p0, sums[i], 0, 0, 0);
-            o[i] = mfma(as_bf16x8(v1), p1, o[i]);
-            sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p1, sums[i], 0, 0, 0);
-            fence();
-            const uint4 *vf = values(i == LAST ? next : cur, n);
-            v0 = vf[0], v1 = vf[64];
-            fence(); // the loads stay behind the last reader of the registers they fill
-            if (i == LAST - 1) {
-                C = load_nb(t + 2);
+            const unsigned long long any = __ballot(f != 0u);
+            if (any != 0) {
+                masked_from = t0 + __builtin_ctzll(any);
+                break;
             }
-            if constexpr (decltype(masked)::value) {
-                m[n] = mask_word_of(n, t + (i == LAST ? 2 : 1));
-            }
-            fence();
         }
-        cur = next;
-        next += W::TILE_SLOTS;
-        next = next == end ? lds : next;
-        if (--left == 0) {
-            // This wave's pieces of the group behind the next one have landed: it asked for them a group ago, and its
-            // youngest loads are those of the group's tiles' bias, issued since.
-            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(4 * W::TILES_PER_GROUP) : "memory");
-            refill();
-            left = W::TILES_PER_GROUP;
+
+        // A row whose keys all have one mask (a padded residue's: -1e9 everywhere) would end with every exponential at zero.  Its logits
+        // are taken against that mask from the start: x = (q.k + bias + mask) - mask, each sum rounded, so that the mask absorbs what
+        // it absorbs in the reference.  shift: the word of the -mask, 0 for other rows.  Such rows used to be attended twice more, by
+        // attend_shifted: 2048 residues, 4 % of them padding, 1.4 ms of 8.0.  The masked loop adds the shift of every row, zero or not (2048
+        // residues without the first one 9.46 ms, whole 7.83; two rows a wave with one product 10.9 and 8.78).
+        uint32_t shift[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            shift[i] = 0;
+            if (masked_from == 0) {
+                const uint32_t *flags = p.flags + (int64_t)b[i] * NB;
+                const uint32_t f = flags[0];
+                bool differs = f == MIXED_WORDS || f == 0;
+                for (int t0 = 0; t0 < NB && !differs; t0 += 64) {
+                    differs = __any(flags[min(t0 + lane, NB - 1)] != f);
+                }
+                shift[i] = __builtin_amdgcn_readfirstlane(differs ? 0u : f ^ 0x80008000u);
+            }
+        }
+
+        // The mask of a row as a rank-one MFMA: A holds (hi, lo) of the key of accumulator row i in k-slots 0 and 1, B ones there,
+        // all else zero, also in the lanes of the upper half, so that an infinite mask value never meets a zero.
+        const uint32_t lower = lane < 32 ? 0xffffffffu : 0u;
+        auto mask_word_of = [&](int i, int t) { return p.words[((int64_t)b[i] * NB + min(t, NB - 1)) * 32 + (lane & 31)] & lower; };
+        auto add_mask = [&](f32x16 x, uint32_t w) {
+            const bf16x8 ones = as_bf16x8(make_uint4(0x3f803f80u & lower, 0u, 0u, 0u));
+            return mfma(as_bf16x8(make_uint4(w, 0u, 0u, 0u)), ones, x);
+        };
+
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); // groups 0 and 1 have landed, every wave's part of them
+        refill();
+        int left = W::TILES_PER_GROUP; // tiles of the current group still to come, this one included
+        const uint4 *cur = lds, *const end = lds + RING * W::TILES_PER_GROUP * W::TILE_SLOTS, *next = lds + W::TILE_SLOTS; // tiles t and t + 1
+        auto keys = [&](const uint4 *tile, int i) { return tile + (first + i) * 2 * BLOCK_SLOTS + lane; };
+        auto values = [&](const uint4 *tile, int i) { return tile + (first + i) * 2 * BLOCK_SLOTS + BLOCK_SLOTS + lane; };
+        uint4 k0 = keys(cur, 0)[0], k1 = keys(cur, 0)[64], v0, v1;
+        f32x16 x[2]; // logits: of row i in x[i & 1]
+        x[0] = mfma(as_bf16x8(k0), q[0][0], C0);
+        x[0] = mfma(as_bf16x8(k1), q[0][1], x[0]);
+        k0 = keys(cur, 1)[0], k1 = keys(cur, 1)[64];
+        v0 = values(cur, 0)[0], v1 = values(cur, 0)[64];
+        f32x16 o[N];
+        f32x4 sums[N]; // the row sums on the matrix pipe: see rowsum_selector
+        uint32_t m[N]; // the mask words of a row's next logits
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            o[i] = zero16(), sums[i] = f32x4{0.f, 0.f, 0.f, 0.f}, m[i] = 0;
+        }
+        const bf16x8 ones_rows = rowsum_selector(lane);
+
+        auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+        // Tile t with seed C: finishes row i = 0 .. N - 1, each time softmax and P.V of the finished logits, the logits of the next row (of
+        // the first one and tile t + 1, from seed Cn, behind the last), and the fragments of the row behind that.  The fences deal the
+        // exponentials between the MFMAs.  The empty asm keeps C live past the MFMA that reads it, so that the logits get registers of their own.
+        auto tile = [&](int t, f32x16 &C, f32x16 &Cn, auto masked) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                constexpr int LAST = N - 1;
+                const int n = i == LAST ? 0 : i + 1, nn = (i + 2) % N; // the next row, the one behind it
+                f32x16 &xc = x[i & 1], &xn = x[n & 1];
+                auto exp4 = [&](int base) {
+#pragma unroll
+                    for (int e = base; e < base + 4; ++e) {
+                        xc[e] = __builtin_amdgcn_exp2f(xc[e]);
+                    }
+                };
+                exp4(0);
+                if (i == LAST) {
+                    xn = mfma(as_bf16x8(k0), q[n][0], Cn);
+                    asm volatile("" ::"v"(Cn));
+                } else {
+                    xn = mfma(as_bf16x8(k0), q[n][0], C);
+                    asm volatile("" ::"v"(C));
+                }
+                fence();
+                exp4(4);
+                const bf16x8 p0 = pack8(xc, 0);
+                xn = mfma(as_bf16x8(k1), q[n][1], xn);
+                if constexpr (decltype(masked)::value) {
+                    xn = add_mask(add_mask(xn, m[n]), shift[n] & lower);
+                }
+                const uint4 *kf = keys(i + 2 < N ? cur : next, nn);
+                k0 = kf[0], k1 = kf[64];
+                fence();
+                exp4(8);
+                o[i] = mfma(as_bf16x8(v0), p0, o[i]);
+                fence();
+                exp4(12);
+                const bf16x8 p1 = pack8(xc, 8);
+                sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p0, sums[i], 0, 0, 0);
+                o[i] = mfma(as_bf16x8(v1), p1, o[i]);
+                sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_rows, p1, sums[i], 0, 0, 0);
+                fence();
+                const uint4 *vf = values(i == LAST ? next : cur, n);
+                v0 = vf[0], v1 = vf[64];
+                fence(); // the loads stay behind the last reader of the registers they fill
+                if (i == LAST - 1) {
+                    C = load_nb(t + 2);
+                }
+                if constexpr (decltype(masked)::value) {
+                    m[n] = mask_word_of(n, t + (i == LAST ? 2 : 1));
+                }
+                fence();
+            }
+            cur = next;
+            next += W::TILE_SLOTS;
+            next = next == end ? lds : next;
+            if (--left == 0) {
+                // This wave's pieces of the group behind the next one have landed: it asked for them a group ago, and its
+                // youngest loads are those of the group's tiles' bias, issued since.
+                asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(4 * W::TILES_PER_GROUP) : "memory");
+                refill();
+                left = W::TILES_PER_GROUP;
+            }
+        };
+        auto run = [&](int from, int to, auto masked) __attribute__((always_inline)) {
+            int t = from;
+            for (; t + 1 < to; t += 2) {
+                tile(t, C0, C1, masked);
+                tile(t + 1, C1, C0, masked);
+            }
+            if (t < to) {
+                tile(t, C0, C1, masked);
+                const f32x16 swap = C0;
+                C0 = C1, C1 = swap;
+            }
+        };
+        run(0, masked_from, std::false_type{});
+        if (masked_from < NB) {
+            x[0] = add_mask(add_mask(x[0], mask_word_of(0, masked_from)), shift[0] & lower);
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                m[i] = mask_word_of(i, masked_from + (i == 0 ? 1 : 0));
+            }
+            run(masked_from, NB, std::true_type{});
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the gates, and requests past the last tile before the LDS is given back
+        uint32_t again = 0; // rows whose sums ran out of range
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float l = rowsum_fetch(sums[i], lane);
+            const bool stored = ROWS * set + first + i < p.B;
+            if (__any(!(l > 1e-30f && l < 1e30f))) {
+                again |= stored ? 1u << i : 0u;
+            } else if (stored) {
+                const int place = i < 2 ? gate_place : (gate_place == RING - 1 ? 0 : gate_place + 1);
+                const uint4 *gate = lds + place * (W::GROUP_BYTES / 16) + wave * 256 + (i & 1) * 128 + lane;
+                store_average(p.q + (row[i] + j) * BLOCK_SLOTS + lane, gate[0], gate[64], o[i], l);
+            }
+        }
+        while (again != 0) {
+            const int i = __builtin_ctz(again), bi = ROWS * set + first + i;
+            again &= again - 1;
+            const int64_t at = ((int64_t)bi * p.H + h) * NB;
+            attend_shifted<true>(p.k + at * BLOCK_SLOTS, p.v + at * BLOCK_SLOTS, p.words + (int64_t)bi * NB * 32, nbc, p.q + (at + j) * BLOCK_SLOTS,
+                                   p.g + (at + j) * BLOCK_SLOTS, NB, lane);
         }
     };
-    auto run = [&](int from, int to, auto masked) __attribute__((always_inline)) {
-        int t = from;
-        for (; t + 1 < to; t += 2) {
-            tile(t, C0, C1, masked);
-            tile(t + 1, C1, C0, masked);
-        }
-        if (t < to) {
-            tile(t, C0, C1, masked);
-            const f32x16 swap = C0;
-            C0 = C1, C1 = swap;
-        }
-    };
-    run(0, masked_from, std::false_type{});
-    if (masked_from < NB) {
-        x[0] = add_mask(add_mask(x[0], mask_word_of(0, masked_from)), shift[0] & lower);
-#pragma unroll
-        for (int i = 0; i < ROWS; ++i) {
-            m[i] = mask_word_of(i, masked_from + (i == 0 ? 1 : 0));
-        }
-        run(masked_from, NB, std::true_type{});
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the gates, and requests past the last tile before the LDS is given back
-    uint32_t again = 0; // rows whose sums ran out of range
-#pragma unroll
-    for (int i = 0; i < ROWS; ++i) {
-        const float l = rowsum_fetch(sums[i], lane);
-        const bool stored = i == 0 || ROWS * set + i < p.B;
-        if (__any(!(l > 1e-30f && l < 1e30f))) {
-            again |= stored ? 1u << i : 0u;
-        } else if (stored) {
-            const int place = i < 2 ? gate_place : (gate_place == RING - 1 ? 0 : gate_place + 1);
-            const uint4 *gate = lds + place * (W::GROUP_BYTES / 16) + wave * 256 + (i & 1) * 128 + lane;
-            store_average(p.q + (row[i] + j) * BLOCK_SLOTS + lane, gate[0], gate[64], o[i], l);
+    // One or two query blocks behind the last whole workgroup: its waves share out the rows, two each, and are done in half the time; with four
+    // rows a wave two or three of the four only brought keys.  508 sequences x 259 residues (nine blocks) 281 -> 276 us and padded
+    // 296 -> 283, 300 x 420 301 -> 289, triangle attention of 1200 residues 2139 -> 2080.
+    if constexpr (ROWS == 4) {
+        const int left = NB % WAVES;
+        if (qg == p.query_groups - 1 && (left == 1 || left == 2)) {
+            attend(qg * WAVES + (wave >> 1), 2 * (wave & 1), std::integral_constant<int, 2>{});
+            return;
         }
     }
-    while (again != 0) {
-        const int i = __builtin_ctz(again), bi = ROWS * set + i;
-        again &= again - 1;
-        const int64_t at = ((int64_t)bi * p.H + h) * NB;
-        attend_shifted<true>(p.k + at * BLOCK_SLOTS, p.v + at * BLOCK_SLOTS, p.words + (int64_t)bi * NB * 32, nbc, p.q + (at + j) * BLOCK_SLOTS,
-                               p.g + (at + j) * BLOCK_SLOTS, NB, lane);
-    }
+    attend(qg * WAVES + wave, 0, std::integral_constant<int, ROWS>{});
 }
 
 // The same without a pair bias, where batch rows share nothing: a wave attends two blocks of 32 queries of one row, which share its

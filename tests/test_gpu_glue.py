@@ -539,6 +539,13 @@ def test_streamed_rows_of_one_mask_beside_others(torch_cuda, streamed_everywhere
     helpers.check_close(helpers.to_numpy(msa), msa_oracle(c, column), "bf16", f"rows of one mask {n_seq}x{n_res} heads={heads} column={column}")
 
 
+# five and six blocks of queries: one and two left over, whose rows the last workgroup's waves share; three, which they do not; sets of four rows and
+# of one to three
+@pytest.mark.parametrize("n_seq,n_res", [(97, 129), (98, 160), (99, 161), (100, 190), (99, 192), (98, 200)])
+def test_streamed_rows_of_left_over_query_blocks(torch_cuda, streamed_everywhere, n_seq, n_res):
+    test_streamed_rows_of_one_mask_beside_others(torch_cuda, streamed_everywhere, False, n_seq, n_res, 8)
+
+
 # without a pair bias: one block of queries and two a wave, three waves a workgroup (3 to 6, 9 to 12, 17 and 18 blocks) and four, the
 # last workgroup full, with an odd block, and with waves that have none
 @pytest.mark.parametrize("n_seq,n_res,heads", [(1, 5, 8), (33, 3, 4), (96, 2, 8), (193, 3, 4), (256, 2, 8), (257, 3, 8), (390, 2, 4), (520, 2, 8)])
