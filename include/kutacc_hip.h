@@ -77,7 +77,8 @@ typedef struct kutacc_hip_attention_args {
     int64_t nb_stride_h;
     int64_t nb_stride_q;
 
-    /* Caller scratch.  k/v/gate are written only by the generic and the tiled path; q is written by those
+    /* Caller scratch.  k/v/gate are written only by the generic and the tiled path (the latter, with eight heads of 8 and
+     * KUTACC_HIP_PATH_AUTO, uses q, k and gate as workspace and leaves v); q is written by those
      * and may be used as workspace by the fused path (a re-ordered copy of the pair bias), so
      * its contents are unspecified after any call; avg (gated weighted average, [B,S,H,d]) is
      * written by every path.  Element (b,s,h,e) of q,k,gate,avg lives at

@@ -82,7 +82,9 @@ int gating_attention_tiled(const kutacc_hip_attention_args_t &args, hipStream_t 
 
 // small_head_attention.hip: the attention step of that route for heads of 8, on the same tensors
 bool small_head_attention_supports(const kutacc_hip_attention_args_t &args);
-int small_head_attention(const kutacc_hip_attention_args_t &args, hipStream_t stream);
+// whether it can form the projections itself, from the input rows (q, k, v and gate stay as they are)
+bool small_head_attention_projects(const kutacc_hip_attention_args_t &args);
+int small_head_attention(const kutacc_hip_attention_args_t &args, bool projects, hipStream_t stream);
 
 // fp32_attention.hip: fp32 storage on the fp32 matrix core (head_size 32, up to 256 channels, up to 224 positions)
 bool fp32_attention_supports(const kutacc_hip_attention_args_t &args);

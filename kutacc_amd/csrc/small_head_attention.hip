@@ -1,5 +1,5 @@
 // Attention with heads of 8 (the extra-MSA row attention: 64 channels, eight heads) for gfx950: the middle step of the tiled
-// route (tiled_attention.hip), reading q, k, v and gate as its projections leave them.
+// route (tiled_attention.hip), reading q, k, v and gate as its projections leave them, or forming them itself (64 channels).
 //
 // A head of 8 fills little of a matrix product: the 742 M logits of 1024 rows x 301 keys x 8 heads are 24 GFLOP of products, 71 as
 // they fill the tiles, 57 us of the matrix cores; their exponentials take 85 us of the vector ALU.  What that does per logit is
@@ -27,11 +27,18 @@ namespace {
 using namespace kutacc_dev;
 
 constexpr int CU_LDS_BYTES = 160 * 1024;
+constexpr int PROJECTED = 64; // channels of the calls whose projections are formed here
 constexpr int D = 8, ROWS = 4, TILE = ROWS * 32; // slots of a key tile's rows
 
 struct SmallHeadParams {
     const bf16_t *q, *k, *v, *gate, *bias, *nb;
     bf16_t *avg;
+    // ... and its queries and gates: of a set and head [row][tile][queries, gates][64 lanes] of 8 bytes, in one of three of the scratch tensors
+    uint2 *stash[3];
+    int stash_each; // sets and heads per tensor
+    const bf16_t *x, *wq, *wk, *wv, *wg; // the kernel that projects: input rows of 64 channels, weights
+    const float *bg;
+    int64_t x_ss;
     int64_t q_ss, k_ss, g_ss, a_ss; // rows of the [batch * seq, channels] matrices
     int64_t v_se, bias_sb, nb_sh, nb_sq;
     int B, S, H, NB, sets, splits; // blocks of 32 positions, sets of four rows, workgroups that share a set's queries
@@ -42,7 +49,7 @@ struct SmallHeadParams {
 // four accumulator rows of both halves are eight consecutive keys, the chunk of p.v's k-slots that the lane supplies
 __device__ __forceinline__ int key_slot(int i) { return 16 * ((i >> 2) & 1) + 4 * (i >> 3) + (i & 3); }
 
-template <bool HAS_NB>
+template <bool HAS_NB, bool PROJECTS>
 __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const SmallHeadParams p)
 {
     extern __shared__ uint4 lds[];
@@ -71,53 +78,142 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         *first_masked = (uint32_t)NB;
     }
     __syncthreads();
-    // A wave brings 64 keys of one row at a time, the next ones requested before these are stored: of K and the mask a key a lane, of V
-    // eight keys of one value.  (Keys dealt to threads by division, K and V in loops of their own, one round trip after the other: whole
-    // operator 2000 rows of 384 660 us, 627 so, of 170 206 and 200.)
-    struct Piece {
-        uint4 k, v;
-        bf16_t mask;
-    };
-    const int units = ROWS * ((NB + 1) / 2); // row unit % 4, keys 64 (unit / 4) ..
-    const bf16_t *v_lane = p.v + (int64_t)(h * D + (lane >> 3)) * p.v_se;
-    auto fetch = [&](int unit) {
-        const int64_t pos = (int64_t)row_of(unit & 3) * S;
-        const int key0 = 64 * (unit >> 2), key = min(key0 + lane, S - 1);
-        Piece w;
-        w.k = *reinterpret_cast<const uint4 *>(p.k + pos * p.k_ss + h * D + (uint32_t)key * (uint32_t)p.k_ss);
-        w.mask = (p.bias + (int64_t)row_of(unit & 3) * p.bias_sb)[(uint32_t)key];
-        w.v = load8_checked(v_lane + pos, min(key0 + 8 * (lane & 7), S), S);
-        return w;
-    };
-    Piece piece = fetch(min(wave, units - 1));
-    for (int unit = wave; unit < units; unit += waves) {
-        const Piece w = piece;
-        piece = fetch(min(unit + waves, units - 1));
-        const int i = unit & 3, key = 64 * (unit >> 2) + lane;
-        const float mask = key < S ? to_f32(w.mask) * LOG2E : 0.f;
-        if (key < keys) {
-            const int tile_row = (key >> 5) * TILE + i * 32;
-            ks[tile_row + key_slot(key & 31)] = key < S ? w.k : zero_u4();
-            masks[tile_row + (key & 31)] = mask;
+    // Operands of the 16x16x32 MFMA: lane (row or column n, chunk c of eight k-slots); results: lane (column n, rows 4 c .. 4 c + 3).
+    const int n = lane & 15, c = lane >> 4;
+    const int unit_of_stash = set * p.H + h;
+    uint2 *const stash = PROJECTS ? p.stash[unit_of_stash / p.stash_each] + (int64_t)(unit_of_stash % p.stash_each) * ROWS * NB * 128 : nullptr;
+    auto product = [](bf16x8 a, bf16x8 b, f32x4 x) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, x, 0, 0, 0); };
+    if constexpr (PROJECTS) {
+        // The head's four projections from the input rows, 16 features as they fill a product.  Keys and values go to the LDS: the
+        // keys from rows of a product, so that a lane has four dims of a position, the values from the columns of the product the other
+        // way round, so that it has four positions of a value.  Queries and gates wait in memory, as the lanes that use them hold
+        // them (1 KB a row and tile in two stores; four bytes a lane in the layout of q and gate cost 25 us of 209): rows 4 c, 4 c + 1 of a third
+        // product are the queries' dims 2 c, 2 c + 1, rows 4 c + 2, 4 c + 3 the gates' dims 2 d, 2 d + 1, d being c with its two bits exchanged, which an
+        // exchange of the halves of the wave turns into the order of the average.
+        // A wave takes the tiles whose queries it attends later, all four rows of them, a row's inputs of the next tile requested where those
+        // of this one have been multiplied.
+        struct Inputs {
+            uint4 x[2][2]; // positions 16 u + n of a tile of 32, channels 32 ks + 8 c .. + 7
+            bf16_t mask;
+        };
+        auto load = [&](int i, int tile) {
+            Inputs t;
+            const bf16_t *rows = p.x + (int64_t)row_of(i) * S * p.x_ss;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const uint32_t at = (uint32_t)min(32 * tile + 16 * u + n, S - 1) * (uint32_t)p.x_ss + 8u * (uint32_t)c;
+                t.x[u][0] = *reinterpret_cast<const uint4 *>(rows + at), t.x[u][1] = *reinterpret_cast<const uint4 *>(rows + at + 32);
+            }
+            t.mask = (p.bias + (int64_t)row_of(i) * p.bias_sb)[(uint32_t)min(32 * tile + (lane & 31), S - 1)];
+            return t;
+        };
+        Inputs in[ROWS];
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+            in[i] = load(i, min(wave, NB - 1));
         }
-        const int kp = 8 * (unit >> 2) + (lane & 7);
-        if (8 * kp < keys) {
-            vs[(kp >> 2) * TILE + i * 32 + (kp & 3) * 8 + (lane >> 3)] = w.v;
+        bf16x8 kv[2], qg[2];
+        {
+            const int pair = n >> 2, dim = 2 * ((n & 2) == 0 ? pair : 2 * (pair & 1) + (pair >> 1)) + (n & 1);
+            const bf16_t *from_kv = n < D ? p.wk + (h * D + n) * PROJECTED : p.wv + (h * D + n - D) * PROJECTED;
+            const bf16_t *from_qg = ((n & 2) == 0 ? p.wq : p.wg) + (h * D + dim) * PROJECTED;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                kv[ks] = as_bf16x8(*reinterpret_cast<const uint4 *>(from_kv + 32 * ks + 8 * c));
+                qg[ks] = as_bf16x8(*reinterpret_cast<const uint4 *>(from_qg + 32 * ks + 8 * c));
+            }
         }
-        if (mask != 0.f) {
-            atomicMin(first_masked, (uint32_t)(key >> 5));
+        const int gate_pair = 2 * (c & 1) + (c >> 1);
+        const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f}, gate_bias = {0.f, 0.f, p.bg[h * D + 2 * gate_pair], p.bg[h * D + 2 * gate_pair + 1]};
+        for (int t = wave; t < NB; t += waves) {
+#pragma unroll
+            for (int i = 0; i < ROWS; ++i) {
+                uint32_t q2[2], g2[2];
+                uint4 *k_tile = ks + t * TILE + i * 32, *v_tile = vs + t * TILE + i * 32;
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    f32x4 kk = zero4, vv = zero4, qq = gate_bias;
+#pragma unroll
+                    for (int ks = 0; ks < 2; ++ks) {
+                        const bf16x8 x = as_bf16x8(in[i].x[u][ks]);
+                        kk = product(kv[ks], x, kk);
+                        vv = product(x, kv[ks], vv);
+                        qq = product(qg[ks], x, qq);
+                    }
+                    bf16x4 k4, v4;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) { // zeros past the last key
+                        k4[e] = (bf16_t)(32 * t + 16 * u + n < S ? kk[e] : 0.f), v4[e] = (bf16_t)(32 * t + 16 * u + 4 * c + e < S ? vv[e] : 0.f);
+                    }
+                    if (c < 2) {
+                        reinterpret_cast<bf16x4 *>(k_tile + key_slot(16 * u + n))[c] = k4;
+                    }
+                    if (n >= D) {
+                        reinterpret_cast<bf16x4 *>(v_tile + (2 * u + (c >> 1)) * 8 + n - D)[c & 1] = v4;
+                    }
+                    const bf16x2 qp = {(bf16_t)qq[0], (bf16_t)qq[1]}, gp = {(bf16_t)qq[2], (bf16_t)qq[3]};
+                    q2[u] = __builtin_bit_cast(uint32_t, qp), g2[u] = __builtin_bit_cast(uint32_t, gp);
+                }
+                const auto sw = __builtin_amdgcn_permlane32_swap(g2[0], g2[1], false, false);
+                uint2 *to = stash + (i * NB + t) * 128;
+                to[lane] = make_uint2(q2[0], q2[1]), to[64 + lane] = make_uint2(sw[0], sw[1]);
+                const int key = 32 * t + lane;
+                const float mask = key < S ? to_f32(in[i].mask) * LOG2E : 0.f;
+                if (lane < 32) {
+                    masks[t * TILE + i * 32 + lane] = mask;
+                    if (mask != 0.f) {
+                        atomicMin(first_masked, (uint32_t)t);
+                    }
+                }
+                in[i] = load(i, min(t + waves, NB - 1));
+            }
+        }
+    } else {
+        // A wave brings 64 keys of one row at a time, the next ones requested before these are stored: of K and the mask a key a lane, of V
+        // eight keys of one value.  (Keys dealt to threads by division, K and V in loops of their own, one round trip after the other: whole
+        // operator 2000 rows of 384 660 us, 627 so, of 170 206 and 200.)
+        struct Piece {
+            uint4 k, v;
+            bf16_t mask;
+        };
+        const int units = ROWS * ((NB + 1) / 2); // row unit % 4, keys 64 (unit / 4) ..
+        const bf16_t *v_lane = p.v + (int64_t)(h * D + (lane >> 3)) * p.v_se;
+        auto fetch = [&](int unit) {
+            const int64_t pos = (int64_t)row_of(unit & 3) * S;
+            const int key0 = 64 * (unit >> 2), key = min(key0 + lane, S - 1);
+            Piece w;
+            w.k = *reinterpret_cast<const uint4 *>(p.k + pos * p.k_ss + h * D + (uint32_t)key * (uint32_t)p.k_ss);
+            w.mask = (p.bias + (int64_t)row_of(unit & 3) * p.bias_sb)[(uint32_t)key];
+            w.v = load8_checked(v_lane + pos, min(key0 + 8 * (lane & 7), S), S);
+            return w;
+        };
+        Piece piece = fetch(min(wave, units - 1));
+        for (int unit = wave; unit < units; unit += waves) {
+            const Piece w = piece;
+            piece = fetch(min(unit + waves, units - 1));
+            const int i = unit & 3, key = 64 * (unit >> 2) + lane;
+            const float mask = key < S ? to_f32(w.mask) * LOG2E : 0.f;
+            if (key < keys) {
+                const int tile_row = (key >> 5) * TILE + i * 32;
+                ks[tile_row + key_slot(key & 31)] = key < S ? w.k : zero_u4();
+                masks[tile_row + (key & 31)] = mask;
+            }
+            const int kp = 8 * (unit >> 2) + (lane & 7);
+            if (8 * kp < keys) {
+                vs[(kp >> 2) * TILE + i * 32 + (kp & 3) * 8 + (lane >> 3)] = w.v;
+            }
+            if (mask != 0.f) {
+                atomicMin(first_masked, (uint32_t)(key >> 5));
+            }
         }
     }
     __syncthreads();
     const int masked_from = (int)*first_masked;
 
-    // Operands of the 16x16x32 MFMA: lane (row or column n, chunk c of eight k-slots).
     //   logits: rows are sixteen keys, columns sixteen queries; chunks 0, 1, 2 hold the same keys against the three parts of the
     //           queries, chunk 3 nothing (zeros in the queries);
     //   p.v:    rows 0-7 are the values, row 8 ones (the row sums), the rest zeros; the k-slots of chunk c are keys 8 c .. 8 c + 7.
-    const int n = lane & 15, c = lane >> 4;
     const uint32_t v_first = n < D ? 8u * c + n : (uint32_t)(constants - vs) + (n == D ? 1u : 0u), v_tile = n < D ? (uint32_t)TILE : 0u;
-    auto product = [](bf16x8 a, bf16x8 b, f32x4 x) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, x, 0, 0, 0); };
 
     for (int j = split * waves + wave; j < NB; j += waves * p.splits) {
         int lv = lane; // opaque: the addresses of a query block's rows are formed where they are used, not kept over the keys
@@ -128,12 +224,19 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         for (int u = 0; u < 2; ++u) {
             query[u] = (uint32_t)min(32 * j + 16 * u + (lv & 15), S - 1);
         }
+        uint2 kept[ROWS];
+        if constexpr (PROJECTS) {
+#pragma unroll
+            for (int i = 0; i < ROWS; ++i) {
+                kept[i] = stash[(i * NB + j) * 128 + lv];
+            }
+        }
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 // a lane splits dims 2 c and 2 c + 1 of its query, then the four lanes of the query exchange: parts for dims
-                const uint32_t raw = *reinterpret_cast<const uint32_t *>(p.q + (int64_t)row_of(i) * S * p.q_ss + h * D +
+                const uint32_t raw = PROJECTS ? (u == 0 ? kept[i].x : kept[i].y) : *reinterpret_cast<const uint32_t *>(p.q + (int64_t)row_of(i) * S * p.q_ss + h * D +
                                                                          (query[u] * (uint32_t)p.q_ss + 2u * (uint32_t)(lv >> 4)));
                 uint32_t part[4] = {0u, 0u, 0u, 0u};
                 float x0 = __uint_as_float(raw << 16) * p.scale2, x1 = __uint_as_float(raw & 0xffff0000u) * p.scale2;
@@ -292,7 +395,8 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         bf16x4 gates[ROWS]; // of all rows at once, one round trip (2000 rows of 384 627 -> 622 us, of 170 200 -> 195)
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
-            gates[i] = *reinterpret_cast<const bf16x4 *>(p.gate + (int64_t)row_of(i) * S * p.g_ss + h * D + gate_at);
+            gates[i] = PROJECTS ? __builtin_bit_cast(bf16x4, stash[(i * NB + j) * 128 + 64 + le])
+                                : *reinterpret_cast<const bf16x4 *>(p.gate + (int64_t)row_of(i) * S * p.g_ss + h * D + gate_at);
         }
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
@@ -355,12 +459,12 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
 
 size_t lds_bytes(int NB) { return (size_t)(2 * NB + 1) * TILE * 16 + (size_t)(TILE * NB + 1) * 4; }
 
-template <bool HAS_NB>
+template <bool HAS_NB, bool PROJECTS>
 int launch(SmallHeadParams p, hipStream_t stream)
 {
     static size_t configured[KUTACC_DEVICE_SLOTS] = {};
     const size_t lds = lds_bytes(p.NB);
-    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&small_head_attention_kernel<HAS_NB>), lds, configured)) {
+    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&small_head_attention_kernel<HAS_NB, PROJECTS>), lds, configured)) {
         return kutacc_hip_status(e);
     }
     // Four waves while three workgroups' keys fit a CU (the registers' limit of 12 waves), else eight.  A number that is no
@@ -370,7 +474,7 @@ int launch(SmallHeadParams p, hipStream_t stream)
     const int turns = (p.NB + waves - 1) / waves, room = 2 * kutacc_cu_count() / std::max(1, p.sets * p.H);
     p.splits = std::max(1, std::min(turns, room));
     const int64_t blocks = (int64_t)(p.sets + 7) / 8 * 8 * p.H * p.splits;
-    small_head_attention_kernel<HAS_NB><<<dim3((unsigned)blocks), 64 * waves, lds, stream>>>(p);
+    small_head_attention_kernel<HAS_NB, PROJECTS><<<dim3((unsigned)blocks), 64 * waves, lds, stream>>>(p);
     return kutacc_hip_status(hipGetLastError());
 }
 } // namespace
@@ -386,7 +490,34 @@ bool small_head_attention_supports(const kutacc_hip_attention_args_t &a)
            in_reach(a.nb_stride_q) && in_reach(a.q_stride_s) && in_reach(a.k_stride_s) && in_reach(a.gate_stride_s) && in_reach(a.avg_stride_s) && (sets + 7) * a.nheads * 8 <= INT32_MAX;
 }
 
-int small_head_attention(const kutacc_hip_attention_args_t &a, hipStream_t stream)
+namespace {
+// sets (of one head) whose queries and gates one scratch tensor of the call holds
+int64_t stash_capacity(const kutacc_hip_attention_args_t &a)
+{
+    return std::min<int64_t>(INT32_MAX, a.batch * a.seq_len * a.nheads * D * 2 / (ROWS * ((a.seq_len + 31) / 32) * 1024));
+}
+} // namespace
+
+// The projections inside: no pass that writes and reads four activations (1024 rows of 301 215 -> 181-191 us, of 107 3576 rows 199 -> 175, 5120 of
+// 128 353 -> 281, 64 of 60 20.4 -> 12.8, whole operator), where the inputs are what projections_kernel takes, the scratch tensors are dense and hold
+// the queries and gates (not where padding makes three times as much of the rows), and no other workgroup
+// reads what one of them writes.  KUTACC_HIP_PATH_TILED asks for q, k, v and gate as the reference leaves them.
+bool small_head_attention_projects(const kutacc_hip_attention_args_t &a)
+{
+    const int64_t C = a.nheads * D, M = a.batch * a.seq_len;
+    const auto apart = [&](const void *from, int64_t bytes) { // of the average, which other workgroups write while these operands are read
+        const uintptr_t at = reinterpret_cast<uintptr_t>(from), avg = reinterpret_cast<uintptr_t>(a.avg);
+        return at + (uintptr_t)bytes <= avg || avg + (uintptr_t)(((M - 1) * a.avg_stride_s + C) * 2) <= at;
+    };
+    return a.path != KUTACC_HIP_PATH_TILED && C == PROJECTED && a.q_stride_s == C && a.k_stride_s == C && a.gate_stride_s == C &&
+           3 * stash_capacity(a) >= (a.batch + ROWS - 1) / ROWS * a.nheads && small_head_attention_supports(a) && a.input_ld % 8 == 0 && a.input_ld < (1 << 30) &&
+           a.seq_len * a.input_ld < (1 << 30) && kutacc_hip_aligned16(a.input) && kutacc_hip_aligned16(a.query_w) && kutacc_hip_aligned16(a.key_w) &&
+           kutacc_hip_aligned16(a.value_w) && kutacc_hip_aligned16(a.gating_w) && apart(a.input, ((M - 1) * a.input_ld + C) * 2) &&
+           apart(a.query_w, 2 * C * C) && apart(a.key_w, 2 * C * C) && apart(a.value_w, 2 * C * C) && apart(a.gating_w, 2 * C * C) &&
+           apart(a.gating_b, 4 * C);
+}
+
+int small_head_attention(const kutacc_hip_attention_args_t &a, bool projects, hipStream_t stream)
 {
     SmallHeadParams p;
     p.q = (const bf16_t *)a.q, p.k = (const bf16_t *)a.k, p.v = (const bf16_t *)a.v, p.gate = (const bf16_t *)a.gate;
@@ -396,7 +527,14 @@ int small_head_attention(const kutacc_hip_attention_args_t &a, hipStream_t strea
     p.B = (int)a.batch, p.S = (int)a.seq_len, p.H = (int)a.nheads, p.NB = (p.S + 31) / 32, p.sets = (p.B + ROWS - 1) / ROWS, p.splits = 1;
     // (float)(1 / sqrt(head_size)) as the reference forms it (gating_attention.cpp:68)
     p.scale2 = (float)(1.0 / sqrt((double)D)) * LOG2E;
-    return p.nb ? launch<true>(p, stream) : launch<false>(p, stream);
+    if (!projects) {
+        return p.nb ? launch<true, false>(p, stream) : launch<false, false>(p, stream);
+    }
+    p.x = (const bf16_t *)a.input, p.x_ss = a.input_ld;
+    p.wq = (const bf16_t *)a.query_w, p.wk = (const bf16_t *)a.key_w, p.wv = (const bf16_t *)a.value_w, p.wg = (const bf16_t *)a.gating_w;
+    p.bg = a.gating_b;
+    p.stash[0] = (uint2 *)a.q, p.stash[1] = (uint2 *)a.k, p.stash[2] = (uint2 *)a.gate, p.stash_each = (int)stash_capacity(a);
+    return p.nb ? launch<true, true>(p, stream) : launch<false, true>(p, stream);
 }
 
 } // namespace kutacc_launch

@@ -2,6 +2,8 @@
 head kernels do not take -- rows longer than 1024 positions, head sizes other than 32, channel counts other than 128 and
 256 -- against the fp32 oracle, to the bf16 bar (2e-2 absolute + 1e-2 relative); the scratch tensors it leaves against
 the oracle's bf16 model of the reference (reference src/attention/gating_attention.cpp:47-66)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -167,6 +169,48 @@ def test_heads_of_eight_stage_their_keys_in_units_of_64(torch_cuda, B, S):
     """Units whole, short of a key and with one, half units behind an odd number of tiles, fewer waves than rows, and the last eight keys
     of a row read in one piece."""
     test_heads_of_eight_at_tile_edges(torch_cuda, B, S, True)
+
+
+# sets of four rows, whole and with one to three; one tile and several, ragged and not, a wave with one tile, two and three, eight waves; rows and averages
+# with a pitch.  projects: whether the kernel forms the projections itself: no where the scratch does not hold its queries and gates (5 rows of
+# 64, rows of 40), is not dense, or the average lies where the input does
+@pytest.mark.parametrize("B,S,form,projects", [(8, 64, "", True), (65, 48, "", True), (12, 97, "", True), (11, 128, "", True), (33, 150, "", True), (8, 301, "", True),
+                                               (12, 385, "", True), (10, 77, "pitch", True), (5, 64, "", False), (40, 40, "", False), (10, 77, "q", False), (10, 77, "k", False),
+                                               (10, 77, "in place", False)])
+@pytest.mark.parametrize("pair_bias", [True, False])
+def test_heads_of_eight_with_the_projections_inside(torch_cuda, B, S, form, projects, pair_bias):
+    """The kernel that projects against the one that reads q, k, v and gate: the same roundings, sums of products in another order."""
+    torch = torch_cuda
+    w = draw_workload(300 + S, B, S, 8, 8, pair_bias=pair_bias)
+    w.bias[B - 1, :] = MASK_BIAS
+    w.bias = round_to_bf16(w.bias)
+    got = {}
+    for path in (capi.PATH_TILED, capi.PATH_AUTO):
+        ten, scratch = helpers.to_device(w)
+        a = helpers.hip_args(w, ten, scratch, path)
+        wide = torch.full((B, S, 72), 7.0, device="cuda", dtype=torch.bfloat16)
+        out_wide, avg = wide.clone(), scratch["avg"].view(B, S, 64)
+        if form == "pitch":
+            wide[..., :64] = ten["x"]
+            a.input, a.input_ld = wide.data_ptr(), 72
+            a.avg, a.avg_stride_b, a.avg_stride_s, avg = out_wide.data_ptr(), 72 * S, 72, out_wide[..., :64]
+        elif form in ("q", "k"):
+            setattr(a, form, wide.data_ptr()), setattr(a, form + "_stride_b", 72 * S), setattr(a, form + "_stride_s", 72)
+        elif form == "in place":
+            a.avg, avg = ten["x"].data_ptr(), ten["x"]
+        print(f"{w.name} {form} path={path}", flush=True)
+        names = helpers.profiled_kernels(torch, lambda: capi.lib().kutacc_hip_gating_attention(ctypes.byref(a), None))  # noqa: B023
+        torch.cuda.synchronize()
+        assert capi.last_path() == "tiled_mfma" and "small_head_attention_kernel" in names
+        assert ("projections_kernel" in names) == (path == capi.PATH_TILED or not projects), names
+        assert form != "pitch" or bool((out_wide[..., 64:] == 7.0).all())
+        got[path] = (ten["out"].float(), avg.float().clone())
+    ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
+    helpers.check_close(helpers.to_numpy(got[capi.PATH_AUTO][0]), ref_out, "bf16", "out")
+    helpers.check_close(helpers.to_numpy(got[capi.PATH_AUTO][1]), ref_avg, "bf16", "gated average")
+    for x, y in zip(*got.values()):
+        # q, k, v and gate are rounded to bf16 on both sides: a sum in another order moves a few of them, and the results with them, by a unit (2^-8)
+        assert float((x - y).norm() / y.norm()) <= 2.0 ** -9 and float((x - y).abs().max()) <= 2.0 ** -6 * float(y.abs().max())
 
 
 def test_pair_bias_entries_of_minus_infinity(torch_cuda):
