@@ -79,15 +79,20 @@ template <int C>
 __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedParams p, int steps_per_group)
 {
     constexpr int CK = C / 16, SLOTS = C / 8, LOADS = 8 * SLOTS / 64, ROWS = 64 / SLOTS; // rows per load instruction
+    constexpr int AHEAD = 2; // fragments of the stage on their way to the products
     extern __shared__ uint4 lds[]; // two stages of [64 positions][SLOTS], gamma, beta, gating bias
     float *gamma = reinterpret_cast<float *>(lds + 2 * 64 * SLOTS), *beta = gamma + C, *gating = beta + C;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
-    const int h = (int)blockIdx.y * 4 + (wave & 3);
+    // Workgroup ids are dealt round robin over the 8 XCDs: with 256 channels the two workgroups that read the same rows, eight ids apart,
+    // share an L2 whatever the number of runs (508 x 259, 127 runs: 279.5 -> 276 us).
+    constexpr int HALVES = C / 128;
+    const int id = (int)blockIdx.x, run = HALVES == 1 ? id : (id & 7) + 8 * (id >> 4), half_of_heads = HALVES == 1 ? 0 : (id >> 3) & 1;
+    const int h = half_of_heads * 4 + (wave & 3);
     const bool forms_kv = wave >= 4;
 
     const int blocks = p.B * p.NB, total_steps = (blocks + 1) / 2;
-    const int first = (int)blockIdx.x * steps_per_group;
+    const int first = run * steps_per_group;
     const int stop = min(first + steps_per_group, total_steps);
     if (first >= stop) {
         return;
@@ -119,6 +124,11 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
         return t;
     };
     auto park = [&](int s, const Rows &t, int lane) {
+        float gm[8], bt[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            gm[e] = gamma[lane % SLOTS * 8 + e], bt[e] = beta[lane % SLOTS * 8 + e];
+        }
 #pragma unroll
         for (int u = 0; u < LOADS; ++u) {
             const bf16x8 in = as_bf16x8(t.r[u]);
@@ -131,14 +141,14 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
             bf16x8 out;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                out[e] = (bf16_t)fmaf(fmaf(v[e], rstd, shift), gamma[lane % SLOTS * 8 + e], beta[lane % SLOTS * 8 + e]);
+                out[e] = (bf16_t)fmaf(fmaf(v[e], rstd, shift), gm[e], bt[e]);
             }
             lds[s * 64 * SLOTS + slot(8 * wave + ROWS * u + lane / SLOTS, lane % SLOTS)] = as_uint4(out);
         }
     };
     // The masks of a step's two blocks are the business of waves 0 and 3, one each.  Whatever a step uses is asked for a step ahead and in
     // front of the next rows: loads return in order, and a later one waited for would make the rows' wait a whole round trip.
-    const bool forms_masks = blockIdx.y == 0 && (wave == 0 || wave == 3);
+    const bool forms_masks = half_of_heads == 0 && (wave == 0 || wave == 3);
     int mask_b = (2 * first + (wave == 3)) / p.NB, mask_j = (2 * first + (wave == 3)) % p.NB;
     auto load_mask = [&] {
         const int key = min(32 * mask_j + pi_row(r), p.S - 1);
@@ -207,23 +217,44 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
                 // Behind an odd number of blocks the last one again: every step has the same stores, so that the wait for the next rows lets
                 // them be on their way.
                 const uint4 *stage = lds + (s * 64 + (2 * step + half < blocks ? 32 * half : 0)) * SLOTS;
+                // Fragment ks lies in slot(pi_row(r), 2 ks + g): four lane offsets, the rest of the slot is the same for all lanes.  With an
+                // offset for each of 16 fragments and one fragment on its way, as the compiler had it, a pair of products waited for its operand:
+                // 508 sequences x 259 residues 274.5 -> 269.4 us (projections 94.6 -> 90.0), 1024 x 384 843 -> 833.5 (236 -> 223); four, six and
+                // eight on their way 90.3, 90.5 and 91.5 us.
+                const uint4 *lane_slot[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    lane_slot[i] = stage + slot(pi_row(r), 2 * i + g);
+                }
+                bf16x8 xf[CK];
+                auto fragment = [&](int ks) { xf[ks] = as_bf16x8(lane_slot[ks & 3][8 * (ks >> 2)]); };
+#pragma unroll
+                for (int ks = 0; ks < AHEAD; ++ks) {
+                    fragment(ks);
+                }
                 f32x16 a0 = zero16(), a1 = zero16();
                 const int64_t at = (((int64_t)b * p.H + h) * p.NB + j) * BLOCK_SLOTS + lane;
                 if constexpr (decltype(kv)::value) {
 #pragma unroll
                     for (int ks = 0; ks < CK; ++ks) {
-                        const bf16x8 xf = as_bf16x8(stage[slot(pi_row(r), 2 * ks + g)]);
-                        a0 = mfma(w0[ks], xf, a0);
-                        a1 = mfma(xf, w1[ks], a1); // V: rows = keys, columns = head dims
+                        a0 = mfma(w0[ks], xf[ks], a0);
+                        a1 = mfma(xf[ks], w1[ks], a1); // V: rows = keys, columns = head dims
+                        if (ks + AHEAD < CK) {
+                            fragment(ks + AHEAD);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
                     p.k[at] = as_uint4(pack8(a0, 0)), p.k[at + 64] = as_uint4(pack8(a0, 8));
                     p.v[at] = as_uint4(pack8(a1, 0)), p.v[at + 64] = as_uint4(pack8(a1, 8));
                 } else {
 #pragma unroll
                     for (int ks = 0; ks < CK; ++ks) {
-                        const bf16x8 xf = as_bf16x8(stage[slot(pi_row(r), 2 * ks + g)]);
-                        a0 = mfma(w0[ks], xf, a0);
-                        a1 = mfma(w1[ks], xf, a1);
+                        a0 = mfma(w0[ks], xf[ks], a0);
+                        a1 = mfma(w1[ks], xf[ks], a1);
+                        if (ks + AHEAD < CK) {
+                            fragment(ks + AHEAD);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
                     const float *bg = gating + h * HEAD + 4 * g;
 #pragma unroll
@@ -997,7 +1028,8 @@ int launch_projection(const StreamedParams &p, hipStream_t stream)
     const int64_t steps = ((int64_t)p.B * p.NB + 1) / 2, cap = std::max(1, kutacc_cu_count() / halves);
     const int64_t per = (steps + cap - 1) / cap;
     kutacc_prof::KernelTimer t("qkvg_projection_kernel", 8.0 * (double)p.B * p.S * C * C, stream);
-    qkvg_projection_kernel<C><<<dim3((unsigned)((steps + per - 1) / per), halves), 512, projection_lds<C>(), stream>>>(p, (int)per);
+    const int64_t runs = (steps + per - 1) / per;
+    qkvg_projection_kernel<C><<<dim3((unsigned)(halves == 1 ? runs : (runs + 7) / 8 * 16)), 512, projection_lds<C>(), stream>>>(p, (int)per);
     return kutacc_hip_status(hipGetLastError());
 }
 
