@@ -8,7 +8,7 @@
 //   wavg[h,:] = sum_s p[h,s] (Wv x[s]);  out[s,:] = (sigmoid(x[s].Wg^T + bg) * wavg).Wo^T + bo
 // One workgroup owns a batch row and walks it in 32-token tiles in three phases: (A) masked mean, (B) logits, online
 // softmax and weighted average, (C) gate, gating and output projection.  A wave keeps the fragments of its first tiles in
-// registers after phase A -- all of them up to 1024 tokens, 64 tiles of a longer row's -- and what is left of a longer row
+// registers after phase A -- all of them up to 1024 tokens, 80 tiles of a longer row's -- and what is left of a longer row
 // is read again in phases B and C, straight into the LDS.  Nothing but q_avg and out is written to memory.  All
 // contractions are v_mfma_f32_32x32x16_bf16:
 //   B: logits^T[s, h] = X[s, :] . QK^T with QK[h, :] = q[h].Wk / sqrt(d) folded per batch row (heads are the
@@ -22,6 +22,7 @@
 // is all zero attends uniformly, as in the reference.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "device_util.h"
@@ -34,6 +35,7 @@ using namespace kutacc_dev;
 namespace {
 
 constexpr int GC = 64;        // channels
+constexpr int MAX_PARTS = 8;  // workgroups of a batch row
 constexpr int PANEL_SLOTS = 288; // of a wave: 32 rows of 128 bytes, or 64 lanes of MERGE_LD floats
 constexpr int MERGE_LD = 18;  // floats per lane in the cross-wave merge area: m, l, 16 accumulators
 
@@ -43,6 +45,7 @@ struct GlobalParams {
     bf16_t *q_avg, *out;
     int64_t x_sb, x_ss, mask_sb, qavg_sb, out_sb, out_ss;
     int B, S, H, d, NT;
+    int whole, parts; // batch rows that have one workgroup each; workgroups of each row behind them
     float scale;
 };
 
@@ -57,7 +60,8 @@ __device__ __forceinline__ int gate_channel(int rb, int v, int g)
 // NW * KEEP; the rest is read again in every phase, straight into the LDS, two tiles of a wave ahead.
 // What bounds it: in phase C the vector ALU (two transcendentals per gate element, 67 % busy on a row that has the chip to
 // itself), in phases A and B the memory.  Measured at 5120 tokens x 384 rows: phases 48 + 36 + 100 us; 220 us with every
-// phase streaming the whole row through registers, 184 with 64 of its 160 tiles kept.  1508 x 107: 32.4 -> 24.9 us.
+// phase streaming the whole row through registers, 189 with 64 of its 160 tiles kept, 186.5 with 80, for which gate bias and average are read
+// from the LDS per tile (4000 x 300 146.5 -> 144).  1508 x 107: 32.4 -> 24.9 us.
 template <int NW, int KEEP, bool STREAM>
 __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalParams p)
 {
@@ -66,8 +70,19 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     extern __shared__ uint4 lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
-    const int b = blockIdx.x;
     const int S = p.S, NT = p.NT, H = p.H, d = p.d;
+    // Workgroup ids are dealt round robin over the 8 XCDs: the parts of a row are eight ids apart, so that its tiles come from one L2.
+    int b = (int)blockIdx.x, turn = 0, own = NT;
+    if (b >= p.whole) {
+        const int idx = b - p.whole, part = (idx >> 3) % p.parts;
+        b = p.whole + (idx >> 3) / p.parts * 8 + (idx & 7);
+        if (b >= p.B) {
+            return;
+        }
+        turn = NT * part / p.parts, own = NT * (part + 1) / p.parts - turn;
+    }
+    // A part takes the row's tiles in an order that begins with those it puts out, so that these are the ones it keeps.
+    auto place = [&](int t) { return t + turn < NT ? t + turn : t + turn - NT; };
     const int spad = NT * 32;
 
     uint4 *qk_frag = lds;            // [4 k-steps][64 lanes]
@@ -84,6 +99,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     float *qv = qavg + GC;                                  // [64] q, bf16-rounded
     float *wavg = qv + GC;                                  // [64]
     float *bos = wavg + GC;                                 // [64] output bias
+    float *bgs = bos + GC;                                  // [64] gate bias
     float *merge = reinterpret_cast<float *>(panels);       // [NW waves][64 lanes][MERGE_LD]
 
     const bf16_t *xb = p.x + (int64_t)b * p.x_sb;
@@ -92,26 +108,27 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     // Requested before anything else, so that their latency passes under the staging of the weights: the first tiles of
     // the row (all of a wave's tiles when they are kept in registers and there are at most four) and this thread's slice
     // of the query weights (output o = tid / TPR, channels part * 64 / TPR ...).
-    constexpr int PRE = KEEP < 4 ? KEEP : 4;
+    constexpr int PRE = KEEP > 8 ? 2 : 4; // beside eight tiles and less there are registers for four
     PanelRegs ahead[PRE];
 #pragma unroll
     for (int i = 0; i < PRE; ++i) {
         const int t = wave + NW * i;
-        ahead[i] = panel_load_near(xb, x_pitch, (t < NT ? t : NT - 1) * 32, S - 1, 0, lane);
+        ahead[i] = panel_load_near(xb, x_pitch, place(t < NT ? t : NT - 1) * 32, S - 1, 0, lane);
     }
     const int first = wave + NW * KEEP; // first of the wave's tiles that are not kept
     const uint32_t ring_lds = (uint32_t)(uintptr_t)(const lds_char *)ring;
     auto ask = [&](int slot, int t) { // tile t into a slot of the ring, in the panel's layout
+        const int at = place(t);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int rl = lane >> 3, row = min(t * 32 + 8 * i + rl, S - 1);
+            const int rl = lane >> 3, row = min(at * 32 + 8 * i + rl, S - 1);
             load_to_lds(ring_lds + slot * 4096u + i * 1024u, xb, __umul24((uint32_t)row, 2u * x_pitch) + 16u * (uint32_t)((lane & 7) ^ rl ^ (i >> 1)));
         }
     };
-    auto stream_start = [&]() {
-        if (STREAM && first < NT) {
+    auto stream_start = [&](int end) { // of the tiles up to `end`
+        if (STREAM && first < end) {
             ask(0, first);
-            if (first + NW < NT) {
+            if (first + NW < end) {
                 ask(1, first + NW);
             }
         }
@@ -119,19 +136,19 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     struct Tile {
         bf16x8 f[4];
     };
-    auto ring_tile = [&](int slot, int t) { // out of the ring, and the tile after the next one asked for in its place
+    auto ring_tile = [&](int slot, int t, int end) { // out of the ring, and the tile after the next one asked for in its place
         Tile x;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             x.f[ks] = as_bf16x8(ring[slot * 256 + panel_slot(r, 2 * ks + g)]);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (t + 2 * NW < NT) {
+        if (t + 2 * NW < end) {
             ask(slot, t + 2 * NW);
         }
         return x;
     };
-    stream_start();
+    stream_start(NT);
     constexpr int TPR = NTHR / GC, WQV = GC / TPR / 8; // threads per output of q, 16-byte pieces per thread
     uint4 wq_part[WQV];
 #pragma unroll
@@ -162,7 +179,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         mask16[s] = s < S ? p.mask[(int64_t)b * p.mask_sb + s] : (bf16_t)-INFINITY;
     }
     if (tid < GC) {
-        bos[tid] = p.bo[tid];
+        bos[tid] = p.bo[tid], bgs[tid] = p.bg[tid];
     }
     __syncthreads();
 
@@ -178,7 +195,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         }
         float msum = 0.f;
         auto add_tile = [&](int t, const bf16x8 (&xf)[4]) {
-            float m = to_f32(mask16[t * 32 + r]);
+            float m = to_f32(mask16[place(t) * 32 + r]);
             m = m == -INFINITY ? 0.f : m;
             msum += g == 0 ? m : 0.f;
 #pragma unroll
@@ -199,13 +216,14 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
             panel_store(panel, lane, ahead[i % PRE]);
             if (i + PRE < KEEP) {
                 const int tn = t + NW * PRE;
-                ahead[i % PRE] = panel_load_near(xb, x_pitch, (tn < NT ? tn : NT - 1) * 32, S - 1, 0, lane);
+                ahead[i % PRE] = panel_load_near(xb, x_pitch, place(tn < NT ? tn : NT - 1) * 32, S - 1, 0, lane);
             }
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
                 xs[i][ks] = as_bf16x8(panel[panel_slot(r, 2 * ks + g)]);
             }
             add_tile(t, xs[i]);
+            __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (STREAM) {
             int slot = 0;
@@ -215,10 +233,10 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
                 } else {
                     wait_for_loads<0>();
                 }
-                const Tile x = ring_tile(slot, t);
+                const Tile x = ring_tile(slot, t, NT);
                 add_tile(t, x.f);
             }
-            stream_start();
+            stream_start(NT);
         }
         // sum over the 32 lanes of each half (they hold different tokens of the same channels)
         msum = group_sum<32>(msum);
@@ -252,7 +270,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         }
         const bf16_t qa = (bf16_t)(tot * (1.0f / (ms + 1e-10f))); // reference :66-74
         qavg[tid] = to_f32(qa);
-        if (p.q_avg != nullptr) {
+        if (p.q_avg != nullptr && turn == 0) {
             p.q_avg[(int64_t)b * p.qavg_sb + tid] = qa;
         }
     }
@@ -305,8 +323,11 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         f32x16 o = zero16();
         float m_run = -1e30f, lsum = 0.f;
         auto attend = [&](int t, const bf16x8 (&xf)[4]) {
+            int lane = tid & 63; // opaque, here and in put_out: constants and weights are read per tile, not kept beside the row
+            asm volatile("" : "+v"(lane));
+            const int g = lane >> 5;
             f32x16 x1, vv = zero16();
-            const bf16x4 *mb4 = reinterpret_cast<const bf16x4 *>(mask16 + t * 32 + 4 * g);
+            const bf16x4 *mb4 = reinterpret_cast<const bf16x4 *>(mask16 + place(t) * 32 + 4 * g);
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
                 const bf16x4 mv = mb4[2 * a];
@@ -343,6 +364,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
             }
             o = mfma(pack8(vv, 0), p0, o);
             o = mfma(pack8(vv, 8), p1, o);
+            __builtin_amdgcn_sched_barrier(0);
         };
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
@@ -359,10 +381,10 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
                 } else {
                     wait_for_loads<0>();
                 }
-                const Tile x = ring_tile(slot, t);
+                const Tile x = ring_tile(slot, t, NT);
                 attend(t, x.f);
             }
-            stream_start();
+            stream_start(own);
         }
         float *mine = merge + (wave * 64 + lane) * MERGE_LD;
         mine[0] = m_run;
@@ -406,35 +428,39 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
 
     // ---- phase C: gate, gating, output projection ----
     {
-        // per-channel constants of the gating, in the order the accumulators hold them
-        float bgv[32], wv_[32];
-#pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            const int ch = gate_channel(i >> 4, i & 15, g);
-            bgv[i] = p.bg[ch];
-            wv_[i] = wavg[ch];
-        }
         auto put_out = [&](int t, const bf16x8 (&xf)[4]) {
+            int lane = tid & 63;
+            asm volatile("" : "+v"(lane));
+            const int r = lane & 31, g = lane >> 5;
             bf16x8 gf[4];
 #pragma unroll
             for (int rb = 0; rb < 2; ++rb) {
+                // the lane's channels of the row block, gate_channel(rb, v, g): 32 rb + 8 g + 16 (v / 8) + v % 8
                 f32x16 ga;
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    ga[v] = bgv[rb * 16 + v];
+                for (int a = 0; a < 4; ++a) {
+                    const f32x4 bv = *reinterpret_cast<const f32x4 *>(bgs + 32 * rb + 8 * g + 16 * (a >> 1) + 4 * (a & 1));
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        ga[4 * a + c] = bv[c];
+                    }
                 }
 #pragma unroll
                 for (int ks = 0; ks < 4; ++ks) {
                     ga = mfma(as_bf16x8(wg_frag[(rb * 4 + ks) * 64 + lane]), xf[ks], ga);
                 }
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    ga[v] = wv_[rb * 16 + v] * sigmoid_fast(ga[v]);
+                for (int a = 0; a < 4; ++a) {
+                    const f32x4 wv = *reinterpret_cast<const f32x4 *>(wavg + 32 * rb + 8 * g + 16 * (a >> 1) + 4 * (a & 1));
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        ga[4 * a + c] = wv[c] * sigmoid_fast(ga[4 * a + c]);
+                    }
                 }
                 gf[2 * rb] = pack8(ga, 0);
                 gf[2 * rb + 1] = pack8(ga, 8);
             }
-            const int s = t * 32 + r;
+            const int s = place(t) * 32 + r;
 #pragma unroll
             for (int ob = 0; ob < 2; ++ob) {
                 f32x16 oa;
@@ -457,21 +483,22 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
                     dst[1] = as_uint4(pack8(oa, 8));
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);
         };
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
-            if (wave + NW * i >= NT) {
+            if (wave + NW * i >= own) {
                 break;
             }
             put_out(wave + NW * i, xs[i]);
         }
         if constexpr (STREAM) {
             int slot = 0;
-            for (int t = first; t < NT; t += NW, slot ^= 1) {
+            for (int t = first; t < own; t += NW, slot ^= 1) {
                 // younger than the tile's loads are the stores of the two tiles before it, four each (of kept ones, for the
                 // first two tiles)
                 wait_for_loads<8>();
-                const Tile x = ring_tile(slot, t);
+                const Tile x = ring_tile(slot, t, own);
                 put_out(t, x.f);
             }
         }
@@ -483,7 +510,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
 constexpr size_t LDS_PER_WORKGROUP = 160 * 1024;
 constexpr size_t lds_bytes_for(int nw, bool stream, int nt)
 {
-    return (size_t)(256 + 256 + 512 + 512 + 256 + nw * (PANEL_SLOTS + (stream ? 512 : 0))) * 16 + (size_t)nt * 64 + (size_t)(nw * 68 + 4 * GC) * 4;
+    return (size_t)(256 + 256 + 512 + 512 + 256 + nw * (PANEL_SLOTS + (stream ? 512 : 0))) * 16 + (size_t)nt * 64 + (size_t)(nw * 68 + 5 * GC) * 4;
 }
 constexpr int MAX_SEQ_LEN = 12288;
 static_assert(lds_bytes_for(8, true, MAX_SEQ_LEN / 32) <= LDS_PER_WORKGROUP);
@@ -497,7 +524,8 @@ hipError_t launch(const GlobalParams &p, hipStream_t stream)
     if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(kernel), lds_bytes, configured)) {
         return e;
     }
-    kernel<<<dim3((unsigned)p.B), 64 * NW, lds_bytes, stream>>>(p);
+    const int64_t rest = p.B - p.whole;
+    kernel<<<dim3((unsigned)(p.whole + (rest + 7) / 8 * 8 * p.parts)), 64 * NW, lds_bytes, stream>>>(p);
     return hipGetLastError();
 }
 
@@ -542,11 +570,23 @@ int global_attention(const kutacc_hip_global_attention_args_t &a, hipStream_t st
     // overlaps them is other rows on the same CU.  With the row kept in registers (up to 1024 positions) four waves hold
     // 128 + 107 registers and two rows share a CU; eight waves hold half the tiles each (171 registers) and one row has the
     // CU to itself, which is faster only while there is no second row to put there -- batch <= CUs: 28.1 against 30.7 us at
-    // 256 x 1024, 48.3 against 39.3 us at 384 x 1024.  Longer rows take eight waves with 64 tiles kept.
+    // 256 x 1024, 48.3 against 39.3 us at 384 x 1024.  Longer rows take eight waves with 80 tiles kept.
     const double BS = (double)a.batch * (double)a.seq_len;
     kutacc_prof::KernelTimer t("global_attention_kernel", BS * (4.0 * GC * a.head_size + 4.0 * GC * GC + 4.0 * GC), stream);
-    const hipError_t e = p.NT > 32 ? launch<8, 8, true>(p, stream)
-                         : p.NT >= 16 && a.batch <= kutacc_cu_count() ? launch<8, 4, false>(p, stream) : launch<4, 8, false>(p, stream);
+    const bool eight_waves = p.NT > 32 || (p.NT >= 16 && a.batch <= kutacc_cu_count());
+    // Rows of eight waves that would leave half of the CUs or more without one are shared by up to eight workgroups each: all form the
+    // mean and the average, from one L2, and a part of the result (us, one workgroup a row against this: 5120 positions x 384 rows 186.5 -> 183.5,
+    // x 128 82 -> 77.7, x 60 66.5 -> 52.3; 4000 x 300 144 -> 126, 2500 x 100 36.7 -> 31.8, 1024 x 128 21.1 -> 18.9, x 60 19.4 -> 15.8, 700 x 100 17.1
+    // -> 14.7).  Two rows of four waves a CU gain nothing (400 x 200 16.4 -> 17.3).  Not where the result lies over the input: one
+    // workgroup would put out what another still reads.
+    const int64_t room = kutacc_cu_count(), rest = eight_waves ? a.batch % room : 0;
+    const uintptr_t in = reinterpret_cast<uintptr_t>(a.q_data), out = reinterpret_cast<uintptr_t>(a.out);
+    const int64_t in_bytes = 2 * ((a.batch - 1) * a.q_data_stride_b + (a.seq_len - 1) * a.q_data_stride_s + GC);
+    const int64_t out_bytes = 2 * ((a.batch - 1) * a.out_stride_b + (a.seq_len - 1) * a.out_stride_s + GC);
+    const bool apart = a.q_data_stride_b >= 0 && a.out_stride_b >= 0 && (in + (uintptr_t)in_bytes <= out || out + (uintptr_t)out_bytes <= in);
+    p.parts = rest > 0 && apart ? (int)std::min<int64_t>(MAX_PARTS, std::max<int64_t>(1, room / rest)) : 1;
+    p.whole = (int)(p.parts > 1 ? a.batch - rest : a.batch);
+    const hipError_t e = p.NT > 32 ? launch<8, 10, true>(p, stream) : eight_waves ? launch<8, 4, false>(p, stream) : launch<4, 8, false>(p, stream);
     return kutacc_hip_status(e);
 }
 

@@ -98,6 +98,64 @@ def test_global_attention_rows_past_the_kept_tiles(torch_cuda, B, S, H, d):
     helpers.assert_within(helpers.to_numpy(scratch["avg"]), ref_qavg, 2.0 ** -8 * np.abs(ref_qavg) + 1e-6, "masked mean q_avg")
 
 
+def device_case(torch, B, S, H, d):
+    """make_case on the device, for batches too large to draw and convert on the host quickly."""
+    g = torch.Generator(device="cuda").manual_seed(B * 10007 + S)
+    bf = lambda *s, scale=1.0: (torch.randn(*s, device="cuda", generator=g) * scale).to(torch.bfloat16)  # noqa: E731
+    C = H * d
+    mask = (torch.rand(B, S, device="cuda", generator=g) > 0.25).to(torch.bfloat16)
+    mask[:, 0] = 1
+    mask[B - 1] = 0
+    ten = dict(x=bf(B, S, C), mask=mask[..., None].contiguous(), wq=bf(C, C, scale=C ** -0.5), wk=bf(d, C, scale=C ** -0.5), wv=bf(d, C, scale=C ** -0.5),
+               wg=bf(C, C, scale=C ** -0.5), bg=torch.ones(C, device="cuda"), wo=bf(C, C, scale=C ** -0.5), bo=torch.randn(C, device="cuda", generator=g))
+    return ten, torch.full((B, S, C), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((B, C), -3.0, dtype=torch.bfloat16, device="cuda")
+
+
+def run_device_case(torch, ten, out, avg, H):
+    small = torch.zeros(1, out.shape[2], dtype=torch.bfloat16, device="cuda")  # the device library leaves these alone
+    op = capi.GlobalAttention(ten["x"], ten["mask"], ten["wq"], ten["wk"], ten["wv"], ten["wg"], ten["bg"], ten["wo"], ten["bo"], H, out,
+                              dict(q=small, k=small, v=small, gate=small, avg=avg))
+    op.run()
+    assert not capi.error_flag() and capi.last_path() == "global_mfma"
+
+
+@pytest.mark.parametrize("rows,S", [
+    (-1, 513), (-1, 2561),                 # one row short of the CUs: a workgroup each
+    (0.5, 481), (0.5, 1024), (0.5, 1057), (0.5, 5121),  # two workgroups a row: first and last length kept whole, first read again, most with tiles of
+                                           # the first part all kept and one wave of the second with one more
+    (0.3, 2600), (0.2, 700), (7, 2600),    # three, five, eight
+    (1.25, 1100), (1.004, 1056),           # rows with a workgroup each, and a rest that shares four, and eight
+])
+def test_global_attention_rows_shared_by_workgroups(torch_cuda, rows, S):
+    torch = torch_cuda
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    B = rows if isinstance(rows, int) and rows > 0 else cus + rows if isinstance(rows, int) else int(rows * cus)
+    ten, out, avg = device_case(torch, B, S, 8, 8)
+    run_device_case(torch, ten, out, avg, 8)
+    checked = sorted({0, 1, B // 2, B - 7, B - 2, B - 1} if B > 7 else set(range(B)))
+    c = dict(nheads=8, **{k: helpers.to_numpy(ten[k]) for k in ("wq", "wk", "wv", "wg", "bg", "wo", "bo")})
+    c["x"], c["mask"] = helpers.to_numpy(ten["x"][checked]), helpers.to_numpy(ten["mask"][checked][..., 0])
+    ref, ref_qavg = oracle_out(c)
+    helpers.check_close(helpers.to_numpy(out[checked]), ref, "bf16", "global attention out")
+    helpers.assert_within(helpers.to_numpy(avg[checked]), ref_qavg, 2.0 ** -8 * np.abs(ref_qavg) + 1e-6, "masked mean q_avg")
+    # every row alone against the call: a workgroup's sums may be in another order, nothing else
+    assert bool(torch.isfinite(out).all()) and bool(torch.isfinite(avg).all())
+    one_out, one_avg = torch.empty_like(out[:1]), torch.empty_like(avg[:1])
+    for b in checked:
+        run_device_case(torch, dict(ten, x=ten["x"][b:b + 1].clone(), mask=ten["mask"][b:b + 1].clone()), one_out, one_avg, 8)
+        helpers.check_close(helpers.to_numpy(out[b]), helpers.to_numpy(one_out[0]), "bf16", "a row among others and alone")
+
+
+def test_global_attention_in_place_keeps_a_workgroup_per_row(torch_cuda):
+    """The result over the input: the same as into memory of its own, within the order of the sums."""
+    torch = torch_cuda
+    ten, out, avg = device_case(torch, 20, 2600, 8, 8)
+    run_device_case(torch, ten, out, avg, 8)
+    again = ten["x"].clone()
+    run_device_case(torch, dict(ten, x=again), again, avg, 8)
+    helpers.check_close(helpers.to_numpy(again), helpers.to_numpy(out), "bf16", "global attention in place")
+
+
 def test_global_attention_replays_from_a_hip_graph(torch_cuda):
     """Rows past the kept tiles, whose rest comes through the ring in the LDS: captured on a side stream and replayed three times, with
     eager work (the results overwritten) between the replays; every replay gives the eager result bit for bit."""
