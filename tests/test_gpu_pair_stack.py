@@ -738,3 +738,54 @@ def test_triangle_multiplication_host_pointers_match_device_pointers(torch_cuda,
         assert not capi.error_flag()
     np.testing.assert_array_equal(h_out, _bits(d_out))
     assert np.any(h_out != 0)
+
+
+def row_projection_args(a, w, bias, out):
+    """out[m, n] = a[m, k] . w[n, k]^T + bias[n], rows of a and out at their own pitches."""
+    g = capi.HipGemmArgs()
+    g.m, g.n, g.k, g.batches, g.dtype, g.path = a.shape[0], w.shape[0], w.shape[1], 1, capi.K_BF16, capi.PATH_AUTO
+    g.a, g.a_stride_m, g.a_stride_k = a.data_ptr(), a.stride(0), 1
+    g.b, g.b_stride_n, g.b_stride_k = w.data_ptr(), w.stride(0), 1
+    g.c, g.c_stride_m = out.data_ptr(), out.stride(0)
+    g.bias, g.bias_axis = bias.data_ptr(), 1
+    return g
+
+
+@pytest.mark.parametrize("k,n", [(128, 128), (128, 384), (256, 128), (256, 256), (256, 512)])
+def test_row_projections_on_either_side_of_the_tile_kernel_s_rows(torch_cuda, k, n):
+    """Rows of 128 and 256 features against a dense matrix: one row, a tile of 32 less and more one, the last number of rows whose 32 x 128
+    tiles are a workgroup each (five a CU), and one more; rows wider than the product, nothing written between them."""
+    torch = torch_cuda
+    limit = 32 * (5 * torch.cuda.get_device_properties(0).multi_processor_count // (n // 128))
+    g = torch.Generator(device="cuda").manual_seed(k + n)
+    w = (torch.randn(n, k, device="cuda", generator=g) * k ** -0.5).to(torch.bfloat16)
+    bias = torch.randn(n, device="cuda", generator=g)
+    full = torch.randn(limit + 1, k + 8, device="cuda", generator=g).to(torch.bfloat16)
+    results = {}
+    for m in (1, 31, 33, limit, limit + 1):
+        a, out = full[:m, :k], torch.full((m, n + 16), 3.0, device="cuda", dtype=torch.bfloat16)
+        rc = capi.lib().kutacc_hip_gemm(ctypes.byref(row_projection_args(a, w, bias, out)), None)
+        torch.cuda.synchronize()
+        assert rc == 0, rc
+        want = a.float() @ w.float().T + bias
+        helpers.check_close(helpers.to_numpy(out[:, :n]), helpers.to_numpy(want), "bf16", f"row projection {m} x {n} x {k}")
+        assert bool((out[:, n:] == 3.0).all())
+        results[m] = out
+    # the same products in the same order: rows of either kernel are the same bits
+    for m in (1, 31, 33, limit):
+        assert helpers.same_bits(results[m], results[limit + 1][:m].contiguous())
+
+
+@pytest.mark.parametrize("n", [256])
+def test_row_projection_over_its_own_rows(torch_cuda, n):
+    """The result in the place of the rows it was formed from: all features of a row by the workgroup that has read it."""
+    torch = torch_cuda
+    g = torch.Generator(device="cuda").manual_seed(n)
+    w = (torch.randn(n, n, device="cuda", generator=g) * n ** -0.5).to(torch.bfloat16)
+    bias = torch.randn(n, device="cuda", generator=g)
+    a = torch.randn(777, n, device="cuda", generator=g).to(torch.bfloat16)
+    want = a.float() @ w.float().T + bias
+    rc = capi.lib().kutacc_hip_gemm(ctypes.byref(row_projection_args(a, w, bias, a)), None)
+    torch.cuda.synchronize()
+    assert rc == 0, rc
+    helpers.check_close(helpers.to_numpy(a), helpers.to_numpy(want), "bf16", "row projection in place")
