@@ -216,7 +216,10 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
     const uint32_t nrows = (uint32_t)rows, ncol = (uint32_t)rows_j, nrow_i = (uint32_t)rows_i;
     // A wave's rows: row0 and the `count` - 1 behind it.  Without the attention's copy they are 32 rows as they come.  With it they are
     // key tile t of query q, on a grid of whole blocks of queries and whole tiles of keys: the last tile of a query has fewer
-    // rows (zeros take the place of the others in the copy), and queries past the last repeat that one, in the copy only.
+    // rows (zeros take the place of the others in the copy), and queries past the last repeat that one, in the copy only.  A workgroup's
+    // waves take four queries that follow each other: their pieces of 16 bytes in the copy are neighbours, and so are their rows of z for the
+    // ending node.  (Four tiles of one query: triangle attention of 128 residues 22.2 us, now 21.1; of 384 116.1 and 114.4, ending node 121.3
+    // and 119.2; 508 x 259 with eight heads, this kernel, 12.8 and 10.6.)
     uint32_t row0 = ((uint32_t)blockIdx.x * 4 + wave) * PAIR_BIAS_ROWS_PER_WAVE, count = 0;
     int q = 0, t = 0;
     if (nbf == nullptr) {
@@ -225,8 +228,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
         }
         count = min(32u, nrows - row0);
     } else {
-        const uint32_t tile_index = (uint32_t)blockIdx.x * 4 + wave;
-        q = (int)(tile_index / (uint32_t)frag_nb), t = (int)(tile_index % (uint32_t)frag_nb);
+        q = (int)(blockIdx.x / (uint32_t)frag_nb * 4) + wave, t = (int)(blockIdx.x % (uint32_t)frag_nb);
         if (q >= 32 * frag_nb) {
             return;
         }
