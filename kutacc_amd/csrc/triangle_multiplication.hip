@@ -12,9 +12,9 @@
 // Both kernels take the padded positions p = i np + j in steps of 64.  Eight consecutive positions share the row i, because
 // np is a multiple of 8: a wave follows (i, j) of its eights with scalar additions.
 //
-// Both are bound by vector issue at two waves per SIMD (246 and 237 registers) as much as by HBM: at 384 residues each moves its 113 MB
-// (front: 256 bytes in, 512 out per position; back: 512 in, 256 out) in 40 to 41 us on average and 38 at best, 60 % of the rate of a copy,
-// with the vector issue ports taken for 63 and 56 % of the clocks and the matrix cores for 26 and 12.  Neither reads a normalised copy of the pair activation: the front kernel normalises the rows on their way into the LDS, the back kernel does it again for
+// Both are bound by vector issue as much as by HBM, and by power: at 384 residues each moves its 113 MB
+// (front: 256 bytes in, 512 out per position; back: 512 in, 256 out) in 37 to 38 us, 60 % of the rate of a copy,
+// with the vector issue ports taken for some 60 % of the clocks and the matrix cores for 29 and 15.  Neither reads a normalised copy of the pair activation: the front kernel normalises the rows on their way into the LDS, the back kernel does it again for
 // its gate, from the same rows that its residual needs.  At 384 residues that saves a pass of 76 MB and a read of 38 MB.
 #include <hip/hip_runtime.h>
 
@@ -77,26 +77,33 @@ struct Side {
 };
 
 // LayerNorm and both gated projections: out[c][p] = bf16(bf16(y . wp[c] + bp[c]) * mask * sigmoid(y . wg[c] + bg[c])), y the
-// normalised row of position p.  Eight waves, one workgroup per CU; a wave owns 32 channels of one side and keeps its two
-// 32 x 128 weight blocks in 64 registers.  Per step it normalises eight of the 64 rows, loaded two steps ahead, into the
-// shared stage, multiplies the whole stage and writes 32 channels x 128 bytes.  Same arithmetic in the same order as
-// LayerNorm followed by gated_projection_kernel: the results are bit-identical.
-constexpr int FRONT_WAVES = 8;
+// normalised row of position p.  Sixteen waves, one workgroup per CU; a wave owns 16 channels of one side and keeps its two
+// 16 x 128 weight blocks in 32 registers.  Per step it normalises four of the 64 rows, loaded two steps ahead, into the
+// shared stage, multiplies the whole stage and writes 16 channels x 128 bytes.  Same arithmetic in the same order as
+// LayerNorm followed by gated_projection_kernel: the results are bit-identical (a 16x16x32 product sums as two 32x32x16 ones do).
+//
+// Four waves a SIMD of 16 channels instead of two of 32: the older of two waves was through a step in 5500 clocks and waited 2000 at the
+// barrier for the younger, which it had kept from issuing; products whose rows are channels leave a lane one mask a product and 18 % fewer
+// vector instructions.  This kernel, us: 691 residues 101.4 -> 97.5, 1024 213.5 -> 205.7, 384 38.4 -> 38.2.  No barrier at all, with the weights of
+// both sides in the LDS and 32 positions x 256 outputs a wave: 116, 213 and 41.6; one of two waves half a step behind the other: no difference.
+constexpr int FRONT_WAVES = 16;
 constexpr int FRONT_STAGE = STEP * ROW_SLOTS;
-constexpr size_t FRONT_LDS = (size_t)(2 * FRONT_STAGE + FRONT_WAVES * 256) * 16 + 2 * STEP * 2;
+constexpr int FRONT_PANEL = STEP * 32; // bytes of a wave's panel: 64 positions x 16 channels
+constexpr size_t FRONT_LDS = (size_t)2 * FRONT_STAGE * 16 + FRONT_WAVES * FRONT_PANEL + 2 * C * sizeof(float) + 2 * STEP * 2;
 
 __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(const bf16_t *__restrict__ x, const float *__restrict__ gamma,
                                                                              const float *__restrict__ beta, float eps, Side s0, Side s1,
                                                                              const bf16_t *__restrict__ mask, int64_t plane, int n, int rows,
                                                                              int np, int steps_per_group)
 {
-    extern __shared__ uint4 lds[]; // two stages, a panel per wave, two mask rows
+    extern __shared__ uint4 lds[]; // two stages, a panel per wave, gamma and beta, two mask rows
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int rv = lane & 31, gv = lane >> 5;
-    const Side &sd = wave >= 4 ? s1 : s0;
-    const int cb = wave & 3; // this wave's 32 channels
-    uint4 *panel = lds + 2 * FRONT_STAGE + wave * 256;
-    uint16_t *mask_rows = reinterpret_cast<uint16_t *>(lds + 2 * FRONT_STAGE + FRONT_WAVES * 256);
+    const int col = lane & 15, chunk = lane >> 4; // operands: row or column, eight k; results: column, rows 4 chunk .. + 3
+    const Side &sd = wave >= 8 ? s1 : s0;
+    const int cb = wave & 7; // this wave's 16 channels
+    char *const panel = reinterpret_cast<char *>(lds + 2 * FRONT_STAGE) + wave * FRONT_PANEL;
+    float *norm = reinterpret_cast<float *>(reinterpret_cast<char *>(lds + 2 * FRONT_STAGE) + FRONT_WAVES * FRONT_PANEL);
+    uint16_t *mask_rows = reinterpret_cast<uint16_t *>(norm + 2 * C);
 
     const int positions = rows * np, total_steps = (positions + STEP - 1) / STEP;
     const int first = (int)blockIdx.x * steps_per_group;
@@ -105,131 +112,108 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
         return;
     }
 
-    // This wave's eight rows of a step: lane (l / 16, l % 16) holds chunk l % 16 of rows l / 16 and 4 + l / 16.  Padding
+    // This wave's four rows of a step, half of an eight: lane (l / 16, l % 16) holds chunk l % 16 of row l / 16.  Padding
     // repeats the row's last position, steps past the end repeat the last row: valid addresses, results masked or dropped.
     struct Rows {
-        uint4 r[2];
-        uint16_t m; // mask of position lane % 8 of the eight, if there is such a position
+        uint4 r;
+        uint16_t m; // mask of the lane's position, if there is such a position
         bool there;
     };
-    Place at = place_of((uint32_t)(first * STEP + 8 * wave), (uint32_t)np);
-    auto load = [&](Rows &t) {
-        const bool there = at.i < n;
-        const int i = there ? at.i : n - 1;
+    Place at = place_of((uint32_t)(first * STEP + 8 * (wave >> 1)), (uint32_t)np);
+    auto load = [&](Rows &t) __attribute__((always_inline)) {
+        const int i = min(at.i, n - 1), j = at.j + 4 * (wave & 1) + chunk;
+        t.there = at.i < n && j < n;
+        const uint32_t here = (uint32_t)min(j, n - 1);
         const char *row = reinterpret_cast<const char *>(x + (int64_t)i * n * C);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int j = min(at.j + 4 * u + (lane >> 4), n - 1);
-            t.r[u] = *reinterpret_cast<const uint4 *>(row + ((uint32_t)j * (2u * C) + 16u * (lane & 15)));
-        }
-        const int jm = at.j + (lane & 7);
-        t.m = reinterpret_cast<const uint16_t *>(mask)[(int64_t)i * n + min(jm, n - 1)];
-        t.there = there && jm < n;
+        t.r = *reinterpret_cast<const uint4 *>(row + (here * (2u * C) + 16u * col));
+        t.m = reinterpret_cast<const uint16_t *>(mask + (int64_t)i * n)[here];
         advance(at, np);
     };
-    float gm[8], bt[8];
-    auto stage_rows = [&](const Rows &t, int s) {
+    auto stage_rows = [&](const Rows &t, int s) __attribute__((always_inline)) {
+        float gm[8], bt[8];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            lds[s * FRONT_STAGE + row_slot(8 * wave + 4 * u + (lane >> 4), lane & 15)] = normalise_row(t.r[u], lane, gm, bt, eps);
+        for (int e = 0; e < 8; ++e) {
+            gm[e] = norm[8 * col + e], bt[e] = norm[C + 8 * col + e];
         }
-        if (lane < 8) {
-            mask_rows[s * STEP + 8 * wave + lane] = t.there ? t.m : (uint16_t)0;
+        lds[s * FRONT_STAGE + row_slot(4 * wave + chunk, col)] = normalise_row(t.r, lane, gm, bt, eps);
+        if (col == 0) {
+            mask_rows[s * STEP + 4 * wave + chunk] = t.there ? t.m : (uint16_t)0;
         }
     };
 
     Rows even, odd;
     load(even);
     load(odd);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        gm[e] = gamma[(lane & 15) * 8 + e], bt[e] = beta[(lane & 15) * 8 + e];
+    if (tid < C) {
+        norm[tid] = gamma[tid], norm[C + tid] = beta[tid];
     }
-    bf16x8 wp[CK], wg[CK];
+    bf16x8 wp[4], wg[4];
+    f32x4 pbias, gneg;
 #pragma unroll
-    for (int ks = 0; ks < CK; ++ks) {
-        wp[ks] = *reinterpret_cast<const bf16x8 *>(sd.wp + (cb * 32 + rv) * C + ks * 16 + gv * 8);
-        wg[ks] = *reinterpret_cast<const bf16x8 *>(sd.wg + (cb * 32 + rv) * C + ks * 16 + gv * 8);
+    for (int ks = 0; ks < 4; ++ks) {
+        wp[ks] = *reinterpret_cast<const bf16x8 *>(sd.wp + (cb * 16 + col) * C + ks * 32 + chunk * 8);
+        wg[ks] = *reinterpret_cast<const bf16x8 *>(sd.wg + (cb * 16 + col) * C + ks * 32 + chunk * 8);
     }
-    const float pbias = sd.bp[cb * 32 + rv], gneg = -LOG2E * sd.bg[cb * 32 + rv];
-    bf16_t *out = sd.out + (int64_t)cb * 32 * plane;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        pbias[v] = sd.bp[cb * 16 + 4 * chunk + v], gneg[v] = -LOG2E * sd.bg[cb * 16 + 4 * chunk + v];
+    }
+    char *out = reinterpret_cast<char *>(sd.out + (int64_t)cb * 16 * plane);
+    __syncthreads();
     stage_rows(even, 0);
     __syncthreads();
     // The weights are waited for here: the waits that the compiler leaves to their first uses stand in the loop, where they are waits for
-    // all rows and stores on their way.  With them, a mask that was waited for where it was loaded, and loads and stores that some steps
-    // did without, 384 residues 42.0 -> 38.4 us (2.9 TB/s), 691 residues 127 -> 106 us (3.5 TB/s); what is left is the vector
-    // work of two waves a SIMD.
+    // all rows and stores on their way.
 #pragma unroll
-    for (int ks = 0; ks < CK; ++ks) {
+    for (int ks = 0; ks < 4; ++ks) {
         asm volatile("" ::"v"(wp[ks]), "v"(wg[ks]));
     }
     asm volatile("" ::"v"(pbias), "v"(gneg));
+    auto product = [](bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); };
 
-    auto do_step = [&](int step, int s, Rows &next, Rows &after) {
+    auto do_step = [&](int step, int s, Rows &next, Rows &after) __attribute__((always_inline)) {
         load(after); // (behind the last step as well: every step has the same loads and stores, and the wait for `next` lets them fly)
         if (step + 1 < stop) {
             stage_rows(next, s ^ 1);
         }
         const uint4 *stage = lds + s * FRONT_STAGE;
-        const char *mrow = reinterpret_cast<const char *>(mask_rows + s * STEP);
-        bf16x8 af[2][CK];
+        const uint16_t *mask_row = mask_rows + s * STEP;
+        // The panel: [64 positions][4 chunks of 4 channels], the chunk XOR-ed with 2 (position / 4 % 2), under which these writes and the
+        // transposing reads below are free of bank conflicts.
+        const uint32_t write_at = 32u * col + 8u * (uint32_t)(chunk ^ (2 * ((col >> 2) & 1)));
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
+        for (int pb = 0; pb < 4; ++pb) { // 16 positions
+            f32x4 pa = {0.f, 0.f, 0.f, 0.f}, ga = pa;
 #pragma unroll
-            for (int ks = 0; ks < CK; ++ks) {
-                af[rb][ks] = as_bf16x8(stage[row_slot(rb * 32 + rv, 2 * ks + gv)]);
+            for (int ks = 0; ks < 4; ++ks) {
+                const bf16x8 y = as_bf16x8(stage[row_slot(16 * pb + col, 4 * ks + chunk)]);
+                pa = product(wp[ks], y, pa);
+                ga = product(wg[ks], y, ga);
             }
+            const float mk = __uint_as_float((uint32_t)mask_row[16 * pb + col] << 16);
+            bf16x4 pp, ov;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                pp[v] = (bf16_t)(pa[v] + pbias[v]);
+            }
+            asm volatile("" : "+v"(pp)); // else each value is rounded by itself
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                // sigmoid(gate + bias) = 1 / (1 + 2^-(gate*log2e + bias*log2e)); the gate stays in fp32
+                const float e = __builtin_amdgcn_exp2f(fmaf(ga[v], -LOG2E, gneg[v]));
+                ov[v] = (bf16_t)(to_f32(pp[v]) * mk * __builtin_amdgcn_rcpf(1.0f + e));
+            }
+            *reinterpret_cast<bf16x4 *>(panel + write_at + 512 * pb) = ov;
         }
-        // projection first, rounded to bf16 and parked as packed pairs, then the gate: half the accumulators live
-        bf16x8 pp[2][2];
-        {
-            f32x16 pa[2] = {zero16(), zero16()};
+        // 16 channels x eight 16-byte pieces of 8 positions; pieces past the last one repeat it.  A store: 16 channels x four pieces.
+        const int last_piece = (positions - 1 - step * STEP) >> 3;
+        char *const to = out + (int64_t)step * (2 * STEP);
 #pragma unroll
-            for (int ks = 0; ks < CK; ++ks) {
-#pragma unroll
-                for (int rb = 0; rb < 2; ++rb) {
-                    pa[rb] = mfma(af[rb][ks], wp[ks], pa[rb]);
-                }
-            }
-#pragma unroll
-            for (int rb = 0; rb < 2; ++rb) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    pa[rb][v] += pbias;
-                }
-                pp[rb][0] = pack8(pa[rb], 0), pp[rb][1] = pack8(pa[rb], 8);
-            }
-        }
-        f32x16 ga[2] = {zero16(), zero16()};
-#pragma unroll
-        for (int ks = 0; ks < CK; ++ks) {
-#pragma unroll
-            for (int rb = 0; rb < 2; ++rb) {
-                ga[rb] = mfma(af[rb][ks], wg[ks], ga[rb]);
-            }
-        }
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const bf16x4 mk = *reinterpret_cast<const bf16x4 *>(mrow + 2 * (rb * 32 + 8 * a + 4 * gv)); // the lane's four positions
-                bf16x4 ov;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const float pv = to_f32(pp[rb][a >> 1][4 * (a & 1) + c]) * to_f32(mk[c]);
-                    // sigmoid(gate + bias) = 1 / (1 + 2^-(gate*log2e + bias*log2e)); the gate stays in fp32
-                    const float e = __builtin_amdgcn_exp2f(fmaf(ga[rb][4 * a + c], -LOG2E, gneg));
-                    ov[c] = (bf16_t)(pv * __builtin_amdgcn_rcpf(1.0f + e));
-                }
-                *(reinterpret_cast<bf16x4 *>(panel + panel_slot(rv, rb * 4 + a)) + gv) = ov;
-            }
-        }
-        // 32 channels x eight 16-byte pieces of 8 positions; pieces past the last one repeat it
-        const int piece = min(lane & 7, (positions - 1 - step * STEP) >> 3);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int ch = 8 * i + (lane >> 3);
-            *reinterpret_cast<uint4 *>(out + (int64_t)ch * plane + step * STEP + 8 * piece) = panel[panel_slot(ch, piece)];
+        for (int half = 0; half < 2; ++half) {
+            const uint32_t piece = (uint32_t)min(4 * half + chunk, last_piece);
+            const lds_char *from = (const lds_char *)panel + (256u * piece + 32u * (col >> 2));
+            const bf16x8 v = lds_transposed_fragment(from + 8 * (col & 3), from + (128 + 8 * ((col & 3) ^ 2)));
+            *reinterpret_cast<uint4 *>(to + ((uint32_t)col * (uint32_t)plane * 2u + 16u * piece)) = as_uint4(v);
         }
         __syncthreads(); // the other stage is complete, this one no longer read
     };
