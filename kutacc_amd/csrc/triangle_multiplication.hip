@@ -237,6 +237,9 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
 // LDS reads give a lane 32 channels of one position: exchanged between lanes the whole block took 94.7 us at 384 residues,
 // 93.6 so, and 92.8 with the biases as the products' seeds), and finishes them with the
 // residual, for which the rows of x have stayed in its registers.
+// Four lanes hold a row of x: with sixteen, four rows a lane, their sums, scales, addresses and bounds were formed four times by each
+// (1006 vector instructions a step and wave, 873 now, the pairs of rounded values among them).  This kernel, us: 384 residues 39.2 -> 37.5, 691
+// 97.7 -> 93.3, 1024 203 -> 194.
 constexpr int BACK_STAGE = STEP * ROW_SLOTS; // slots of each of the four stages: centre as it lies, y, centre', result
 constexpr size_t BACK_LDS = (size_t)4 * BACK_STAGE * 16 + 6 * C * sizeof(float);
 
@@ -259,19 +262,22 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
         return;
     }
 
-    // rows of x: this wave's 16 positions of a step, in two eights: 16 wave + 4 u + lane / 16
-    struct Eight {
-        uint4 r0, r1; // named members, so that they always live in registers
-        Place at;
+    // rows of x: this wave's 16 positions of a step, four lanes each: lane l holds pieces l % 4 + 4 u of position 16 wave + l / 4
+    struct RowOfX {
+        uint4 r0, r1, r2, r3; // named members, so that they always live in registers
+        uint32_t at;          // i n + j, of the position itself or of the last one in its place
+        bool there;
     };
     Place at_lo = place_of((uint32_t)(first * STEP + 16 * wave), (uint32_t)np), at_hi = place_of((uint32_t)(first * STEP + 16 * wave + 8), (uint32_t)np);
-    auto load_eight = [&](Eight &t, Place &at) {
-        t.at = at;
-        const char *row = reinterpret_cast<const char *>(x + (int64_t)(at.i < n ? at.i : n - 1) * n * C);
-        const int j = at.j + (lane >> 4);
-        t.r0 = *reinterpret_cast<const uint4 *>(row + ((uint32_t)min(j, n - 1) * (2u * C) + 16u * (lane & 15)));
-        t.r1 = *reinterpret_cast<const uint4 *>(row + ((uint32_t)min(j + 4, n - 1) * (2u * C) + 16u * (lane & 15)));
-        advance(at, np);
+    auto row_of_x = [&](uint32_t at, int ln) { return reinterpret_cast<char *>(x) + ((uint64_t)at * (2 * C) + 16u * (ln & 3)); };
+    auto load_row = [&](RowOfX &t) {
+        const int i = lane < 32 ? at_lo.i : at_hi.i, j = (lane < 32 ? at_lo.j : at_hi.j) + ((lane >> 2) & 7);
+        t.there = i < n && j < n;
+        t.at = (uint32_t)min(i, n - 1) * (uint32_t)n + (uint32_t)min(j, n - 1);
+        const char *row = row_of_x(t.at, lane);
+        t.r0 = *reinterpret_cast<const uint4 *>(row), t.r1 = *reinterpret_cast<const uint4 *>(row + 64);
+        t.r2 = *reinterpret_cast<const uint4 *>(row + 128), t.r3 = *reinterpret_cast<const uint4 *>(row + 192);
+        advance(at_lo, np), advance(at_hi, np);
     };
     // the centre: channels 32 wave + 8 i + lane / 8, positions 8 (lane % 8) .. + 7 of the step; past the end the last eight
     const uint32_t lane_plane = (uint32_t)(lane >> 3) * (uint32_t)plane * 2u;
@@ -288,11 +294,10 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
         return t;
     };
 
-    Eight lo, hi, next_lo, next_hi;
+    RowOfX row, next_row;
     PanelRegs ct = load_centre(first);
-    load_eight(lo, at_lo);
-    load_eight(hi, at_hi);
-    next_lo = lo, next_hi = hi;
+    load_row(row);
+    next_row = row;
     bf16x8 wof[CK], wgf[CK];
 #pragma unroll
     for (int ks = 0; ks < CK; ++ks) {
@@ -305,6 +310,11 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
         params[4 * C + tid] = bo[tid], params[5 * C + tid] = bg[tid];
     }
     __syncthreads();
+    // waited for here, not at their first uses in the loop, where that is a wait for the next step's loads
+#pragma unroll
+    for (int ks = 0; ks < CK; ++ks) {
+        asm volatile("" ::"v"(wof[ks]), "v"(wgf[ks]));
+    }
 
     for (int step = first; step < stop; ++step) {
         int lv = lane; // opaque: LDS addresses are formed per step, not kept across the loop
@@ -319,20 +329,35 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
             ct = load_centre(step + 1);
         }
         {
-            float gm[8], bt[8];
+            const bf16x8 v[4] = {as_bf16x8(row.r0), as_bf16x8(row.r1), as_bf16x8(row.r2), as_bf16x8(row.r3)};
+            // the row's first element, in the first of its four lanes
+            const float x0 = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(to_f32(v[0][0])), 0x00, 0xf, 0xf, false));
+            float s1 = 0.f, s2 = 0.f, rstd, shift;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                gm[e] = params[(lv & 15) * 8 + e], bt[e] = params[C + (lv & 15) * 8 + e];
+            for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float d = to_f32(v[t][e]) - x0;
+                    s1 += d;
+                    s2 = fmaf(d, d, s2);
+                }
             }
-            const int pos = 16 * wave + (lv >> 4);
-            ys[row_slot(pos, lv & 15)] = normalise_row(lo.r0, lv, gm, bt, eps);
-            ys[row_slot(pos + 4, lv & 15)] = normalise_row(lo.r1, lv, gm, bt, eps);
-            ys[row_slot(pos + 8, lv & 15)] = normalise_row(hi.r0, lv, gm, bt, eps);
-            ys[row_slot(pos + 12, lv & 15)] = normalise_row(hi.r1, lv, gm, bt, eps);
+            s1 = dpp_add<0x4E>(dpp_add<0xB1>(s1)), s2 = dpp_add<0x4E>(dpp_add<0xB1>(s2)); // lanes ^ 1, ^ 2
+            norm_from_sums<false>(s1, s2, x0, (float)C, eps, rstd, shift);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int chunk = 4 * t + (lv & 3);
+                const float *gm = params + 8 * chunk, *bt = gm + C;
+                bf16x8 o;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    o[e] = (bf16_t)fmaf(fmaf(to_f32(v[t][e]), rstd, shift), gm[e], bt[e]);
+                }
+                ys[row_slot(16 * wave + (lv >> 2), chunk)] = as_uint4(o);
+            }
         }
         if (step + 1 < stop) {
-            load_eight(next_lo, at_lo);
-            load_eight(next_hi, at_hi);
+            load_row(next_row);
         }
         __syncthreads();
         auto biases = [&](int which) { // of this wave's 32 features, in accumulator order: the seed of their products
@@ -362,6 +387,7 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
 #pragma unroll
             for (int pb = 0; pb < 2; ++pb) {
                 gate[pb][0] = pack8(acc[pb], 0), gate[pb][1] = pack8(acc[pb], 8);
+                asm volatile("" : "+v"(gate[pb][0]), "+v"(gate[pb][1])); // else each value is rounded by itself
             }
         }
         // the centre of this wave's positions: lane l takes channels 8 (l / 16) .. + 7 (+ 32 t) of position l % 16
@@ -410,13 +436,15 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
             }
 #pragma unroll
             for (int pb = 0; pb < 2; ++pb) {
+                bf16x8 rounded[2] = {pack8(acc[pb], 0), pack8(acc[pb], 8)};
+                asm volatile("" : "+v"(rounded[0]), "+v"(rounded[1])); // else each value is rounded by itself
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
                     bf16x4 ov;
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
                         // bf16(out) * sigmoid(bf16(gate)), rounded to bf16: the reference's rounding points
-                        const float o = to_f32((bf16_t)acc[pb][4 * a + c]);
+                        const float o = to_f32(rounded[a >> 1][4 * (a & 1) + c]);
                         ov[c] = (bf16_t)(o * sigmoid_fast(to_f32(gate[pb][a >> 1][4 * (a & 1) + c])));
                     }
                     *(reinterpret_cast<bf16x4 *>(res + row_slot(32 * pb + (lv & 31), 4 * wave + a)) + (lv >> 5)) = ov;
@@ -424,23 +452,28 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
             }
         }
         __syncthreads();
-        auto finish = [&](const Place &at, uint4 raw_row, int local) { // position `local` of the eight at `at`
-            const int j = at.j + (local & 7);
-            const bf16x8 d = as_bf16x8(res[row_slot(16 * wave + local, lv & 15)]), z = as_bf16x8(raw_row);
-            bf16x8 o;
+        {
+            char *to = row_of_x(row.at, lv);
+            const uint4 raw_row[4] = {row.r0, row.r1, row.r2, row.r3};
+            uint4 sum[4];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                o[e] = (bf16_t)(to_f32(z[e]) + to_f32(d[e]));
+            for (int t = 0; t < 4; ++t) {
+                const bf16x8 d = as_bf16x8(res[row_slot(16 * wave + (lv >> 2), 4 * t + (lv & 3))]), z = as_bf16x8(raw_row[t]);
+                bf16x8 o;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    o[e] = (bf16_t)(to_f32(z[e]) + to_f32(d[e]));
+                }
+                sum[t] = as_uint4(o);
             }
-            if (at.i < n && j < n) {
-                *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(x + (int64_t)at.i * n * C) + ((uint32_t)j * (2u * C) + 16u * (lv & 15))) = as_uint4(o);
+            if (row.there) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    *reinterpret_cast<uint4 *>(to + 64 * t) = sum[t];
+                }
             }
-        };
-        finish(lo.at, lo.r0, lv >> 4);
-        finish(lo.at, lo.r1, 4 + (lv >> 4));
-        finish(hi.at, hi.r0, 8 + (lv >> 4));
-        finish(hi.at, hi.r1, 12 + (lv >> 4));
-        lo = next_lo, hi = next_hi;
+        }
+        row = next_row;
     }
 }
 
