@@ -507,12 +507,15 @@ __device__ __forceinline__ f32x16 pair_bias_tile(const uint4 *nbf, int t)
     return c;
 }
 
-template <bool HAS_NB, bool WITH_MASK, bool SHIFT, bool TILES = false>
+template <bool HAS_NB, bool WITH_MASK, bool SHIFT, bool TILES = false, bool ODD = false>
 __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 *lds_v, const f32x4 *mask4,
                                                 const uint4 *nbf, bf16x8 q0, bf16x8 q1, f16x8 sel0, f16x8 sel1,
                                                 bf16x8 sumsel, int NB, int lane, float shift, f32x16 &o_out, float &l_out,
                                                 int prio_phase = -1, int fair_turn = -1)
 {
+    // ODD: the last tile is the one of zeros behind an odd number of them, and left out (us, triangle attention of 77 residues 18.9 -> 18.4, 150
+    // 33.6 -> 32.4, 288 70.9 -> 67.9, 450 211.5 -> 206, 600 391 -> 382; MSA rows, two rows a step, 512 x 224 186.3 -> 184.1).  A loop of its own: decided
+    // inside one, even numbers lost 0.5 to 1 %.
     const int npairs = NB >> 1;
     const uint4 *kp = lds_k + lane;
     const uint4 *vp = lds_v + lane;
@@ -639,7 +642,7 @@ __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 
         lacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sumsel, p1, lacc, 0, 0, 0);
     };
 
-    for (int pair = 0; pair < npairs; ++pair) {
+    for (int pair = 0; pair < (ODD ? npairs - 1 : npairs); ++pair) {
         if (fair_turn >= 0) {
             timeslice_priority((uint32_t)fair_turn, FAIR_SLICE_SHIFT);
         }
@@ -662,6 +665,16 @@ __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 
         half_step(xb, xa, tn, wa0, wa1, Ca, clampt(tn + 2), tn + 1);
         v0 = vp[(tn * 2 + 0) * 64], v1 = vp[(tn * 2 + 1) * 64];
         fence();
+    }
+    if constexpr (ODD) { // the last tile by itself: its logits are there
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            exp4(xa, 8 * k);
+            exp4(xa, 8 * k + 4);
+            const bf16x8 pv = pack8(xa, 8 * k);
+            o = mfma(as_bf16x8(k == 0 ? v0 : v1), pv, o);
+            lacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sumsel, pv, lacc, 0, 0, 0);
+        }
     }
     if (fair_turn >= 0) {
         __builtin_amdgcn_s_setprio(0);
@@ -1224,6 +1237,9 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
                 if (flags == 0u) {
                     attend_block_l2<HAS_NB, false, false, TILES>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel,
                                                           NT, lane, 0.f, o, l, (wave >> 2) & 1);
+                } else if (NB < NT) { // (always here with an odd number of tiles: the one of zeros has a mask)
+                    attend_block_l2<HAS_NB, true, false, TILES, true>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1),
+                                                         sumsel, NT, lane, 0.f, o, l, (wave >> 2) & 1);
                 } else {
                     attend_block_l2<HAS_NB, true, false, TILES>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel,
                                                          NT, lane, 0.f, o, l, (wave >> 2) & 1);
@@ -1522,6 +1538,9 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_head_kernel(F
             if (flags == 0u) {
                 attend_block_l2<HAS_NB, false, false, TILES>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
                                                       l, -1, fair_turn);
+            } else if (NB < NT) { // (always here with an odd number of tiles: the one of zeros has a mask)
+                attend_block_l2<HAS_NB, true, false, TILES, true>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
+                                                     l, -1, fair_turn);
             } else {
                 attend_block_l2<HAS_NB, true, false, TILES>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
                                                      l, -1, fair_turn);
@@ -1657,9 +1676,11 @@ __global__ __launch_bounds__(64) void pair_bias_tiles_kernel(const bf16_t *__res
 //                     lane's accumulator row stands for; one more MFMA per tile adds them (WITH_MASK only)
 //   nbc             : fp32 pair-bias tiles of this head and query block, offset by the lane: tile t, piece a at
 //                     nbc[(4 t + a) * 64]; nullptr without a pair bias
+//   ODD             : the last tile is the one of zeros behind an odd number of them, and left out.  Not with 128 channels, where the
+//                     branch costs nine registers more than there are (352 residues 104.6 us with it and without)
 //   MFMA_SUMS       : the row sums on the matrix pipe (one 16x16x32 MFMA per 16 keys and row) instead of four dot products
 //                     on the vector ALU; costs ten more registers, which the 256-channel kernel (two waves per SIMD) has
-template <bool HAS_NB, bool WITH_MASK, bool MFMA_SUMS>
+template <bool HAS_NB, bool WITH_MASK, bool MFMA_SUMS, bool ODD = false>
 __device__ __forceinline__ void attend_pair_l2(const uint4 *lds_kA, const uint4 *lds_vA, const uint4 *lds_kB, const uint4 *lds_vB,
                                                const uint32_t *mwA, const uint32_t *mwB, const f32x4 *nbc, bf16x8 qA0, bf16x8 qA1,
                                                bf16x8 qB0, bf16x8 qB1, int NB, int lane, f32x16 &oA_out,
@@ -1790,6 +1811,9 @@ __device__ __forceinline__ void attend_pair_l2(const uint4 *lds_kA, const uint4 
         // (B, t0) finished; logits of (A, t1) from C1
         half_step(xb, xa, C1, qA0, qA1, oB, lsumB, sumsB, kB + t1 * 128, mwA, t1);
         v0 = vA[t1 * 128], v1 = vA[t1 * 128 + 64];
+        if (ODD && pair == npairs - 1) {
+            break;
+        }
         // (A, t1) finished; logits of (B, t1) from C1
         half_step(xa, xb, C1, qB0, qB1, oA, lsumA, sumsA, kA + tn * 128, mwB, t1);
         v0 = vB[t1 * 128], v1 = vB[t1 * 128 + 64];
@@ -2064,6 +2088,8 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_pair_kernel(F
         float lA, lB;
         if ((flagsA | flagsB) == 0u) {
             attend_pair_l2<HAS_NB, false, true>(kA, vA, kB, vB, mwA, mwB, nbc, qA0, qA1, qB0, qB1, NT, lane_a, oA, lA, oB, lB, fair_turn);
+        } else if (C == 256 && NB < NT) { // (a row of an odd number of tiles is always here: the one of zeros has a mask)
+            attend_pair_l2<HAS_NB, true, PAIR_MFMA_SUMS, C == 256>(kA, vA, kB, vB, mwA, mwB, nbc, qA0, qA1, qB0, qB1, NT, lane_a, oA, lA, oB, lB, fair_turn);
         } else {
             attend_pair_l2<HAS_NB, true, PAIR_MFMA_SUMS>(kA, vA, kB, vB, mwA, mwB, nbc, qA0, qA1, qB0, qB1, NT, lane_a, oA, lA, oB, lB, fair_turn);
         }

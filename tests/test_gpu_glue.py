@@ -224,6 +224,37 @@ def block_oracle_rows(c, ending, rows):
     return z[rows] + out
 
 
+@pytest.mark.parametrize("n", [17, 32, 65, 96, 129, 160, 257, 288, 321, 385, 544])
+def test_triangle_attention_block_of_odd_numbers_of_key_tiles(torch_cuda, n):
+    """1, 3, 5, 9, 11, 13 and 17 tiles of 32 keys, whole and of one key: behind them the kernels have a tile of zeros that is not attended.  The
+    oracle on a sample of rows, every other entry checked for finiteness."""
+    torch = torch_cuda
+    c = block_case(7300 + n, n, 4)
+    rows = sorted({0, 1, n // 2, n - 2, n - 1})
+    for ending in (False, True):
+        got = run_block(torch, c, ending)
+        assert bool(torch.isfinite(got).all())
+        sample = got[:, rows].transpose(0, 1) if ending else got[rows]
+        helpers.check_close(helpers.to_numpy(sample.contiguous()), block_oracle_rows(c, ending, rows), "bf16", f"block n={n} ending={ending}")
+
+
+@pytest.mark.parametrize("n_seq,n_res", [(40, 32), (40, 33), (40, 96), (130, 65), (130, 160), (64, 161), (600, 224), (24, 257)])
+def test_msa_row_attention_of_odd_numbers_of_key_tiles(torch_cuda, n_seq, n_res):
+    torch = torch_cuda
+    c = msa_case(7700 + n_seq + n_res, n_seq, n_res, 8, 128)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
+        device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
+    msa = dev(c["m"])
+    w = {k: dev(c[k]) for k in ("ln_gamma", "ln_beta", "wq", "wk", "wv", "wg", "bg", "wo", "bo")}
+    pair = {"pair_act": dev(c["z"]), "pair_ln_gamma": dev(c["pair_ln_gamma"]), "pair_ln_beta": dev(c["pair_ln_beta"]), "bias_w": dev(c["bias_w"])}
+    assert capi.MsaAttentionBlock(msa, dev(c["mask"]), w, 8, pair).run() == 0
+    torch.cuda.synchronize()
+    rows = sorted({0, 1, n_seq // 2, n_seq - 2, n_seq - 1})
+    want = msa_oracle(dict(c, m=np.ascontiguousarray(c["m"][rows]), mask=np.ascontiguousarray(c["mask"][rows])), False)
+    assert bool(torch.isfinite(msa).all())
+    helpers.check_close(helpers.to_numpy(msa[rows].contiguous()), want, "bf16", f"msa rows {n_seq}x{n_res}")
+
+
 @pytest.mark.parametrize("n", [384, 1024])
 def test_triangle_attention_block_full_size_sampled_rows(torch_cuda, n):
     """The pair sizes the block is benchmarked at, both orientations: the oracle on a sample of attention rows (first,
