@@ -15,9 +15,11 @@
 // What bounds it: the fp32 matrix rate (64 multiply-adds per cycle and SIMD: 16 positions x 32 features x 256 channels
 // take 4096 cycles) once loads are out of the way.  The smaller 16x16x4 form has the rate of 32x32x2 and twice the
 // pieces to deal out: two waves per SIMD cover each other's LDS reads, and 64 queries occupy four SIMDs instead of two.
-// A wave's whole weight block is in flight before the first position arrives.
-// 16 rows x 64 positions x 256 channels, whole operator: 40.9 us with four waves of 32x32x2 and weights
-// loaded as they were used, 21.9 now; 64 x 200 x 256: 235 and 151.
+// A wave's whole weight block is in flight before the first position arrives.  In front of the first product stand the loads:
+// whole lines (load_rows below) brought 16 rows x 64 positions x 256 channels from 21.8 to 19.1 us and 64 x 200 x 256 from 151 to 131,
+// of which the output projection's are 30 and 17.4: its floor, the matrix cores', is 10.7.  (With four waves of 32x32x2 and weights
+// loaded as they were used they were 40.9 and 235.)  Two tiles of positions in the LDS, in turn or both at once, gave the first
+// projections under 1 % or cost 4 %.
 //
 // Operand and accumulator layouts of the 16x16x4 MFMA: A is 16 x 4, lane l holds A[l % 16][l / 16]; B is 4 x 16, lane l
 // holds B[l / 16][l % 16]; D[4 g + v][j] sits in lane j + 16 g, register v.  A lane reads four consecutive k with one
@@ -45,12 +47,37 @@ typedef f32x4 f32x4_any __attribute__((aligned(4))); // global loads and stores 
 constexpr int HEAD = 32;
 constexpr int LDP = 36;            // row pitch of the [position][feature] arrays in LDS, in floats: 16 rows' 16-byte pieces in 16 bank groups
 constexpr int MAX_SEQ = 224;       // what the LDS holds of K, V, Q and gate of one head in fp32
+constexpr int64_t GEMM_WORKGROUPS_PER_CU = 3; // 64 x 200 x 256 positions' projection 17.4 us, with 2 or 4 a CU 18.8 and 20.3, with one tile each 20.3
 constexpr int MAX_CHANNELS = 256;  // input rows are staged 32 positions x C channels at a time
 constexpr float LOG2E_F = 1.44269504088896340736f;
 
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 __device__ __forceinline__ f32x4 load4(const float *ptr) { return *reinterpret_cast<const f32x4 *>(ptr); }
+
+// A wave's 16 rows of 16 PIECES values, loaded in whole lines (eight rows of 32 values a load), put into operand order: the
+// four values 16 i + 4 g of row r for lane r + 16 g, through 2 KB of the LDS that are the wave's own.  (Loaded in operand
+// order, a 16-byte piece of another row in every lane, each load takes the address path some 50 cycles instead of 16.)
+template <int PIECES>
+__device__ __forceinline__ void load_rows(f32x4 (&w)[PIECES], const float *rows, int64_t ld, int lane)
+{
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        w[i] = load4(rows + (int64_t)((lane >> 3) + 8 * (i & 1)) * ld + 32 * (i / 2) + 4 * (lane & 7));
+    }
+}
+template <int PIECES>
+__device__ __forceinline__ void to_operand_order(f32x4 (&w)[PIECES], float *own, int lane)
+{
+    const auto slot = [](int row, int piece) { return 4 * (8 * row + (piece ^ ((row >> 1) & 7))); }; // 16 rows' in 16 bank groups
+#pragma unroll
+    for (int i = 0; i < PIECES; i += 2) {
+        *reinterpret_cast<f32x4 *>(own + slot(lane >> 3, lane & 7)) = w[i];
+        *reinterpret_cast<f32x4 *>(own + slot(8 + (lane >> 3), lane & 7)) = w[i + 1];
+        w[i] = load4(own + slot(lane & 15, lane >> 4));
+        w[i + 1] = load4(own + slot(lane & 15, 4 + (lane >> 4)));
+    }
+}
 
 // the four lanes that hold one query's keys: l, l ^ 16, l ^ 32, l ^ 48
 __device__ __forceinline__ float quad_max(float x)
@@ -103,7 +130,6 @@ __global__ __launch_bounds__(512, 2) void fp32_head_kernel(Fp32Params p)
     // every SIMD has one of k, v (all positions) and one of q, gate (this workgroup's) ----
     const int half = wave >> 2, mat = (wave + 2 * half) & 3; // 0 k, 1 v, 2 q, 3 gate
     const float *wmat = mat == 0 ? p.wk : mat == 1 ? p.wv : mat == 2 ? p.wq : p.wg;
-    const float *wrow = wmat + (int64_t)(h * HEAD + 16 * half + r) * C + 4 * g;
     // the next 32 positions wait in registers while the staged ones are used
     const float *xb = p.x + (int64_t)b * S * p.x_ld;
     constexpr int c4 = C / 4, pieces = 32 * c4, LOADS = (pieces + 511) / 512;
@@ -124,17 +150,12 @@ __global__ __launch_bounds__(512, 2) void fp32_head_kernel(Fp32Params p)
     };
     fetch(0);
     f32x4 w[PIECES];
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-        w[i] = load4(wrow + 16 * i);
-    }
+    load_rows<PIECES>(w, wmat + (int64_t)(h * HEAD + 16 * half) * C, C, lane);
     f32x4 start = {0.f, 0.f, 0.f, 0.f};
     if (mat == 3) {
         start = *reinterpret_cast<const f32x4_any *>(p.bg + h * HEAD + 16 * half + 4 * g);
     }
-    for (int k = tid; k < S32; k += 512) {
-        ms[k] = k < S ? p.bias[(int64_t)b * p.bias_sb + k] : -INFINITY;
-    }
+    const float mask = tid < S ? p.bias[(int64_t)b * p.bias_sb + tid] : -INFINITY;
     // four keys' pair bias of query q0 + r; a step's is requested one step ahead, the first one's before the projections
     const auto pair_bias = [&](int q0, int key0) {
         f32x4 nv = {0.f, 0.f, 0.f, 0.f};
@@ -153,8 +174,12 @@ __global__ __launch_bounds__(512, 2) void fp32_head_kernel(Fp32Params p)
     };
     const int q_first = 32 * t_lo + 16 * wave, q_end = 32 * t_hi < S ? 32 * t_hi : S;
     f32x4 next0 = pair_bias(q_first, 4 * g), next1 = pair_bias(q_first, 16 + 4 * g);
+    to_operand_order<PIECES>(w, lds_f + 512 * wave, lane); // on the arrays, which are empty still
+    if (tid < S32) {
+        ms[tid] = mask;
+    }
     for (int t = 0; t < NB; ++t) {
-        __syncthreads(); // the previous tile's readers are done with xs
+        __syncthreads(); // the weights' places, or the previous tile, have been read
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
             if (tid + 512 * i < pieces) {
@@ -294,78 +319,65 @@ __global__ __launch_bounds__(512, 2) void fp32_head_kernel(Fp32Params p)
     }
 }
 
-// out[m, n] = sum_k a[m, k] * w[n, k] + bias[n] over 16 PIECES k; 16 T x 16 T outputs per wave, four waves along n.  Rows
-// of a and w are 16-byte aligned.  P pieces of 16 k are fetched at a time, the next P while these are used.  T = 1 with a
-// whole row in flight is bound by one memory latency; T = 2 reads half as much per product.
-template <int PIECES, int T, int P>
+// out[m, n] = sum_k a[m, k] * w[n, k] + bias[n] over 16 PIECES k.  A workgroup keeps 64 rows of w, 16 a wave, in registers and walks
+// tiles of 16 rows of a, which lie in the LDS for its four waves; the next tile's wait in registers meanwhile.  Rows of a and
+// w are 16-byte aligned.
+template <int PIECES>
 __global__ __launch_bounds__(256, 2) void fp32_rows_gemm_kernel(const float *__restrict__ a, int64_t a_ld, const float *__restrict__ w,
                                                                 const float *__restrict__ bias, float *__restrict__ out,
                                                                 int64_t out_ld, int64_t M, int N)
 {
-    static_assert(PIECES % P == 0, "whole steps");
-    constexpr int K = 16 * PIECES;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int K = 16 * PIECES, AP = K + 4, LOADS = (4 * K + 255) / 256;
+    __shared__ __attribute__((aligned(16))) float rows[16 * AP], own[4][512];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, g = lane >> 4;
-    const int64_t m0 = (int64_t)blockIdx.x * 16 * T;
-    const int n0 = (blockIdx.y * 4 + wave) * 16 * T;
-    if (n0 >= N) {
-        return;
-    }
-    const float *ap[T], *wp[T];
-    f32x4 acc[T][T]; // [n][m]: D[output feature][row]
+    const int n0 = (blockIdx.y * 4 + wave) * 16;
+    const bool live = n0 < N; // N is a multiple of 32
+    f32x4 av[LOADS], wv[PIECES];
+    const auto fetch = [&](int64_t m0) {
 #pragma unroll
-    for (int i = 0; i < T; ++i) {
-        const int64_t arow = m0 + 16 * i + r < M ? m0 + 16 * i + r : M - 1;
-        ap[i] = a + arow * a_ld + 4 * g;
-        wp[i] = w + (int64_t)(n0 + 16 * i + r) * K + 4 * g; // n0 + 16 T <= N: N is a multiple of 32
-#pragma unroll
-        for (int j = 0; j < T; ++j) {
-            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-    f32x4 av[2][T][P], wv[2][T][P];
-    const auto fetch = [&](int step) {
-#pragma unroll
-        for (int s = 0; s < P; ++s) {
-#pragma unroll
-            for (int i = 0; i < T; ++i) {
-                wv[step & 1][i][s] = load4(wp[i] + 16 * (step * P + s));
-                av[step & 1][i][s] = load4(ap[i] + 16 * (step * P + s));
-            }
+        for (int i = 0; i < LOADS; ++i) {
+            const int idx = tid + 256 * i < 4 * K ? tid + 256 * i : 4 * K - 1;
+            const int64_t row = m0 + idx / (K / 4) < M ? m0 + idx / (K / 4) : M - 1;
+            av[i] = load4(a + row * a_ld + 4 * (idx % (K / 4)));
         }
     };
-    fetch(0);
-#pragma unroll
-    for (int step = 0; step < PIECES / P; ++step) {
-        if (step + 1 < PIECES / P) {
-            fetch(step + 1);
+    fetch((int64_t)blockIdx.x * 16);
+    f32x4 bv = {0.f, 0.f, 0.f, 0.f};
+    if (live) {
+        load_rows<PIECES>(wv, w + (int64_t)n0 * K, K, lane);
+        if (bias != nullptr) {
+            bv = *reinterpret_cast<const f32x4_any *>(bias + n0 + 4 * g);
         }
-        __builtin_amdgcn_sched_barrier(0); // the loads stay ahead of the products
+        to_operand_order<PIECES>(wv, own[wave], lane);
+    }
+    for (int64_t m0 = (int64_t)blockIdx.x * 16; m0 < M; m0 += (int64_t)gridDim.x * 16) {
+        if (m0 != (int64_t)blockIdx.x * 16) {
+            __syncthreads(); // the previous tile has been read
+        }
 #pragma unroll
-        for (int s = 0; s < P; ++s) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-#pragma unroll
-                for (int i = 0; i < T; ++i) {
-#pragma unroll
-                    for (int j = 0; j < T; ++j) {
-                        acc[i][j] = mfma_f32(wv[step & 1][i][s][e], av[step & 1][j][s][e], acc[i][j]);
-                    }
-                }
+        for (int i = 0; i < LOADS; ++i) {
+            const int idx = tid + 256 * i;
+            if (idx < 4 * K) {
+                *reinterpret_cast<f32x4 *>(rows + idx / (K / 4) * AP + 4 * (idx % (K / 4))) = av[i];
             }
         }
-    }
-#pragma unroll
-    for (int i = 0; i < T; ++i) {
-        f32x4 bv = {0.f, 0.f, 0.f, 0.f};
-        if (bias != nullptr) {
-            bv = *reinterpret_cast<const f32x4_any *>(bias + n0 + 16 * i + 4 * g);
+        __syncthreads();
+        if (m0 + (int64_t)gridDim.x * 16 < M) {
+            fetch(m0 + (int64_t)gridDim.x * 16);
         }
+        if (live) {
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f}; // D[output feature][row]
 #pragma unroll
-        for (int j = 0; j < T; ++j) {
-            const int64_t m = m0 + 16 * j + r;
-            if (m < M) {
-                *reinterpret_cast<f32x4_any *>(out + m * out_ld + n0 + 16 * i + 4 * g) = acc[i][j] + bv;
+            for (int i = 0; i < PIECES; ++i) {
+                const f32x4 x = load4(rows + r * AP + 16 * i + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    acc = mfma_f32(wv[i][e], x[e], acc);
+                }
+            }
+            if (m0 + r < M) {
+                *reinterpret_cast<f32x4_any *>(out + (m0 + r) * out_ld + n0 + 4 * g) = acc + bv;
             }
         }
     }
@@ -377,15 +389,6 @@ size_t head_kernel_lds(int S, int C)
 {
     const int S32 = (S + 31) / 32 * 32;
     return (size_t)(32 * (C + 4) + 3 * S32 * LDP + HEAD * (S32 + 4) + S32) * sizeof(float);
-}
-
-template <int PIECES, int T, int P>
-void launch_rows_gemm(const kutacc_hip_attention_args_t &a, int64_t M, hipStream_t stream)
-{
-    constexpr int C = 16 * PIECES;
-    const dim3 grid((unsigned)((M + 16 * T - 1) / (16 * T)), (unsigned)((C / (16 * T) + 3) / 4));
-    fp32_rows_gemm_kernel<PIECES, T, P><<<grid, 256, 0, stream>>>((const float *)a.avg, a.avg_stride_s, (const float *)a.output_w,
-                                                                  a.output_b, (float *)a.out, a.out_ld, M, C);
 }
 
 template <int PIECES>
@@ -409,12 +412,10 @@ int launch(const kutacc_hip_attention_args_t &a, const Fp32Params &p, hipStream_
     }
     const int64_t M = a.batch * a.seq_len;
     kutacc_prof::KernelTimer t("fp32_rows_gemm_kernel", 2.0 * BS * C * C, stream);
-    // 32 x 32 outputs per wave where that gives every SIMD a wave
-    if ((M + 31) / 32 * (C / 32) >= 4 * (int64_t)kutacc_cu_count()) {
-        launch_rows_gemm<PIECES, 2, 2>(a, M, stream);
-    } else {
-        launch_rows_gemm<PIECES, 1, PIECES>(a, M, stream);
-    }
+    const int64_t columns = (C + 63) / 64, cap = GEMM_WORKGROUPS_PER_CU * (int64_t)kutacc_cu_count() / columns;
+    const dim3 grid((unsigned)std::min<int64_t>((M + 15) / 16, std::max<int64_t>(cap, 1)), (unsigned)columns);
+    fp32_rows_gemm_kernel<PIECES><<<grid, 256, 0, stream>>>((const float *)a.avg, a.avg_stride_s, (const float *)a.output_w,
+                                                            a.output_b, (float *)a.out, a.out_ld, M, C);
     return kutacc_hip_status(hipGetLastError());
 }
 

@@ -161,6 +161,19 @@ def test_fp32_storage_shared_queries_and_projection_tiles(torch_cuda, config, ba
     helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, "fp32", "out")
 
 
+@pytest.mark.parametrize("heads,batch,seq", [(1, 1, 1), (1, 161, 80), (2, 60, 209), (3, 45, 96), (5, 31, 97), (6, 26, 128), (7, 15, 224), (8, 49, 64)])
+def test_fp32_storage_at_every_width(torch_cuda, heads, batch, seq):
+    """Whole-line loads of weights of 32 to 256 channels; the output projection with its last columns missing (an odd number of
+    heads), with one and with several tiles of rows per workgroup, the last one short."""
+    w = draw_workload(7, batch, seq, heads, 32)
+    w.dtype = "fp32"
+    ten, scratch = helpers.to_device(w)
+    assert helpers.run_hip(w, ten, scratch, capi.PATH_FUSED) == 0 and capi.last_path() == "fp32_mfma"
+    ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
+    helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), ref_avg, "fp32", "gated average")
+    helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, "fp32", "out")
+
+
 def test_fp32_storage_beyond_the_matrix_core_path_takes_the_generic_kernels(torch_cuda):
     w = make_workload(1, batch=2, seq_len=225)
     ten, scratch = helpers.to_device(w)
