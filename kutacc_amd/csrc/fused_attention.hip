@@ -874,6 +874,41 @@ __device__ inline void stage_weight_fragments(uint4 *lds_w, const FusedParams &p
     }
 }
 
+// The same in whole lines, eight rows by 64 channels a copy: in fragment order, a 16-byte piece of another row in every
+// lane, a load takes the address path 42 cycles instead of 16, and a workgroup of one unit waits for them all.  Lane l's place of
+// fragment ks is weight_slot(l, ks), so that eight pieces of two rows go to 16 bank groups.
+__device__ inline int weight_slot(int lane, int ks) { return lane ^ (4 * (ks & 3) + 2 * (lane >> 5)); }
+template <int C>
+__device__ inline void stage_weight_lines(uint4 *lds_w, const FusedParams &p, int first, int count, int h, int wave, int nwaves, int lane)
+{
+    constexpr int CK = C / 16;
+    const int nfrag = count * CK, q = lane & 7;
+    auto line = [&](int f) {
+        const int m = first + f / CK, k = f % CK;
+        const bf16_t *w = m == 0 ? p.w[0] : m == 1 ? p.w[1] : m == 2 ? p.w[2] : p.w[3];
+        return *reinterpret_cast<const uint4 *>(w + (int64_t)(h * HEAD + 8 * (k & 3) + (lane >> 3)) * C + (k >> 2) * 64 + q * 8);
+    };
+    auto put = [&](int f, uint4 v) {
+        const int row = 8 * (f & 3) + (lane >> 3), ks0 = f & ~3; // CK is a multiple of 4
+        lds_w[(ks0 + (q >> 1)) * 64 + weight_slot(32 * (q & 1) + row, q >> 1)] = v;
+    };
+    int f = wave;
+    for (; f + (WEIGHT_LOADS_IN_FLIGHT - 1) * nwaves < nfrag; f += WEIGHT_LOADS_IN_FLIGHT * nwaves) {
+        uint4 t[WEIGHT_LOADS_IN_FLIGHT];
+#pragma unroll
+        for (int k = 0; k < WEIGHT_LOADS_IN_FLIGHT; ++k) {
+            t[k] = line(f + k * nwaves);
+        }
+#pragma unroll
+        for (int k = 0; k < WEIGHT_LOADS_IN_FLIGHT; ++k) {
+            put(f + k * nwaves, t[k]);
+        }
+    }
+    for (; f < nfrag; f += nwaves) {
+        put(f, line(f));
+    }
+}
+
 // ------------------------------------------------------------------------------------------------
 // fused_head_kernel: one workgroup per (b, h) unit
 // LDS carve-up, in 16-byte units unless noted:
@@ -964,7 +999,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
             __syncthreads(); // previous group's fragments are no longer being read
         } else {
         }
-        stage_weight_fragments<C>(lds_w, p, pass * GW, GW, h, wave, NW, lane);
+        stage_weight_lines<C>(lds_w, p, pass * GW, GW, h, wave, NW, lane);
         __syncthreads();
         if (pi == 0) {
         }
@@ -1014,12 +1049,12 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
                 }
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
-                    const uint4 *wsrc = lds_w + m * CK * 64 + lane;
+                    const uint4 *wsrc = lds_w + m * CK * 64;
                     f32x16 acc[PAIR];
                     acc[0] = zero16(), acc[1] = zero16();
 #pragma unroll
                     for (int ks = 0; ks < CK; ++ks) {
-                        const bf16x8 wf = as_bf16x8(wsrc[ks * 64]);
+                        const bf16x8 wf = as_bf16x8(wsrc[ks * 64 + weight_slot(lane, ks)]);
 #pragma unroll
                         for (int n = 0; n < PAIR; ++n) {
                             // V[s][d]: rows = sequence positions; the others W_h . x^T: rows = head-dim
@@ -1111,13 +1146,13 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
             }
             for (int mm = 0; mm < GW; ++mm) {
                 const int m = pass * GW + mm;
-                const uint4 *wsrc = lds_w + mm * CK * 64 + lane;
+                const uint4 *wsrc = lds_w + mm * CK * 64;
                 f32x16 acc = zero16();
                 if (m == PROJ_V) {
                     // V[s][d]: rows = sequence positions, so a lane ends up with 16 keys of one head-dim
 #pragma unroll
                     for (int ks = 0; ks < CK; ++ks) {
-                        acc = mfma(xf[ks], as_bf16x8(wsrc[ks * 64]), acc);
+                        acc = mfma(xf[ks], as_bf16x8(wsrc[ks * 64 + weight_slot(lane, ks)]), acc);
                     }
                     if constexpr (V_ALIAS) {
                         vpark[i][0] = as_uint4(pack8(acc, 0));
@@ -1130,7 +1165,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
                     // W_h . x^T: rows = head-dim, columns = sequence positions
 #pragma unroll
                     for (int ks = 0; ks < CK; ++ks) {
-                        acc = mfma(as_bf16x8(wsrc[ks * 64]), xf[ks], acc);
+                        acc = mfma(as_bf16x8(wsrc[ks * 64 + weight_slot(lane, ks)]), xf[ks], acc);
                     }
                     if (m == PROJ_K) {
                         lds_k[(j * 2 + 0) * 64 + lane] = as_uint4(pack8(acc, 0));
