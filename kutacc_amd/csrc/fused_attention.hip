@@ -2390,87 +2390,127 @@ __global__ __launch_bounds__(C == 128 ? 256 : 512, C == 128 ? 2 : 1) void output
     }
 }
 
-// The same product of few rows, of which output_projection_kernel makes a few dozen workgroups, each waiting for its weights, then for
-// the later channels of its rows and for `out` several times in turn.  Here a workgroup takes 32 rows x 128 features, a wave 32 of those, and asks
-// for rows, weights, bias and the rows of `out` at the start: bound by that one round trip, and by the weights that every 32 rows fetch again
-// as there come more of them.  Same products in the same order: the same bits.  Whole calls, us: triangle attention of 50, 77, 128 and 200
-// residues 19.3 -> 16.5, 22.0 -> 19.2, 24.7 -> 22.7, 48.4 -> 47.2 (1250 workgroups), of 256 (2048) 52 -> 54; MSA rows, 64 x 100 38.2 -> 29.0,
-// 128 x 128 48.4 -> 43.4 (1024), 200 x 200 (2500) 92 -> 97.5.
-constexpr int TILE_WORKGROUPS_PER_CU = 5;
+// The same product by tiles of 32 rows x 128 features, a wave 32 of those; same products in the same order: the same bits.  A workgroup asks
+// for rows, weights, bias and the rows of `out` at once, where output_projection_kernel waits for its weights, then for the later channels of
+// its rows and for `out` in turn, with a few dozen workgroups where rows are few.  With 128 channels it keeps its weights in registers and walks
+// the tiles, three workgroups a CU, the next tile's rows and `out` under way: faster than output_projection_kernel at every size.
+// With 256 there are no registers for that (walking 128 sequences x 128 residues 39.5 -> 42): a tile each, the weights fetched for every tile,
+// and no gain is left past some twelve workgroups a CU.
+// Whole calls, us, output_projection_kernel's -> now: triangle attention of 50, 77, 128 and 200 residues 19.3 -> 15.3, 22.0 -> 18.0,
+// 24.7 -> 21.9, 48.4 -> 44.3, of 256, 400, 450 and 691 52 -> 50, 174 -> 166, 218 -> 208, 504 -> 500; attention of 384 x 384, 4 heads
+// 98.5 -> 93.2; MSA rows, 64 x 100 38.2 -> 27.0, 128 x 128 48.4 -> 39.5, 150 x 150 63.5 -> 57.7, 200 x 200 (2500 tiles) 89.8 -> 88.5; MSA
+// columns, 500 x 100 (3126) 113.8 and 113.9.
+constexpr int WALKERS_PER_CU = 3, TILE_WORKGROUPS_PER_CU = 12;
 template <int C, int EPILOGUE>
-__global__ __launch_bounds__(256) void output_projection_tile_kernel(const bf16_t *__restrict__ avg, int64_t avg_ld, const bf16_t *__restrict__ wo,
+__global__ __launch_bounds__(256, C == 128 ? 3 : 2) void output_projection_tile_kernel(const bf16_t *__restrict__ avg, int64_t avg_ld, const bf16_t *__restrict__ wo,
                                                                      const float *__restrict__ bo, bf16_t *__restrict__ out, int64_t out_ld, int M, int swap_n)
 {
+    constexpr bool WALK = C == 128;
     constexpr int CK = C / 16, SLOTS = C / 8, LOADS = 32 * SLOTS / 256;
     __shared__ uint4 rows[32 * SLOTS], result[32 * 16]; // slots XOR-ed with row % 16
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
-    const int row0 = (int)blockIdx.x * 32, last = min(M - 1 - row0, 31); // its last row that is one
     const int n0 = (int)blockIdx.y * 128, f0 = n0 + 32 * wave;
-    uint4 in[LOADS];
+    const int tiles = (M + 31) / 32;
+    bf16x8 in[LOADS];
+    bf16_t *to[2], *next_to[2]; // the thread's two pieces of 8 features of `out`
+    bf16x8 z[2], next_z[2];
+    const auto fetch = [&](int tile) {
+        const int row0 = tile * 32, last = min(M - 1 - row0, 31); // its last row that is one
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-        const int idx = tid + 256 * i;
-        in[i] = *reinterpret_cast<const uint4 *>(avg + (int64_t)(row0 + min(idx / SLOTS, last)) * avg_ld + idx % SLOTS * 8);
-    }
+        for (int i = 0; i < LOADS; ++i) {
+            const int idx = tid + 256 * i;
+            in[i] = *reinterpret_cast<const bf16x8 *>(avg + (int64_t)(row0 + min(idx / SLOTS, last)) * avg_ld + idx % SLOTS * 8);
+        }
+    };
+    const auto fetch_out = [&](int tile) {
+        const int row0 = tile * 32, last = min(M - 1 - row0, 31);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int at = (tid >> 4) + 16 * i;
+            const int row = row0 + min(at, last);
+            const int target = EPILOGUE == EPILOGUE_RESIDUAL && swap_n ? (int)((uint32_t)row % (uint32_t)swap_n) * (M / swap_n) + (int)((uint32_t)row / (uint32_t)swap_n) : row;
+            next_to[i] = out + (int64_t)target * out_ld + n0 + (tid & 15) * 8;
+            if constexpr (EPILOGUE == EPILOGUE_RESIDUAL) {
+                next_z[i] = *reinterpret_cast<const bf16x8 *>(next_to[i]);
+            }
+        }
+    };
+    fetch(blockIdx.x);
+    // weights in half lines, 16 rows by 32 channels a load, put into fragment order below through 2 KB of `result` that are the
+    // wave's own: loaded in fragment order, each takes the address path 42 cycles instead of 16
     bf16x8 w[CK];
 #pragma unroll
     for (int ks = 0; ks < CK; ++ks) {
-        w[ks] = *reinterpret_cast<const bf16x8 *>(wo + (int64_t)(f0 + r) * C + ks * 16 + g * 8);
+        w[ks] = *reinterpret_cast<const bf16x8 *>(wo + (int64_t)(f0 + 16 * (ks & 1) + (lane >> 2)) * C + (ks >> 1) * 32 + (lane & 3) * 8);
     }
-    bf16_t *to[2]; // the thread's two pieces of 8 features of `out`
-    uint4 z[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int at = (tid >> 4) + 16 * i;
-        const int row = row0 + min(at, last);
-        const int target = EPILOGUE == EPILOGUE_RESIDUAL && swap_n ? (int)((uint32_t)row % (uint32_t)swap_n) * (M / swap_n) + (int)((uint32_t)row / (uint32_t)swap_n) : row;
-        to[i] = out + (int64_t)target * out_ld + n0 + (tid & 15) * 8;
-        if constexpr (EPILOGUE == EPILOGUE_RESIDUAL) {
-            z[i] = *reinterpret_cast<const uint4 *>(to[i]);
-        }
-    }
+    fetch_out(blockIdx.x);
     f32x4 bv[4];
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
         bv[a] = *reinterpret_cast<const f32x4 *>(bo + f0 + 8 * a + 4 * g);
     }
+    {
+        uint4 *own = result + 128 * wave;
+        const auto slot = [](int row, int piece) { return 4 * row + (piece ^ ((row >> 2) & 3)); };
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-        const int idx = tid + 256 * i, row = idx / SLOTS;
-        rows[row * SLOTS + (idx % SLOTS ^ (row & 15))] = in[i];
-    }
-    __syncthreads();
-    f32x16 acc = zero16();
-#pragma unroll
-    for (int ks = 0; ks < CK; ++ks) {
-        acc = mfma(w[ks], as_bf16x8(rows[r * SLOTS + ((2 * ks + g) ^ (r & 15))]), acc);
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        bf16x4 ov;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            ov[c] = (bf16_t)(acc[4 * a + c] + bv[a][c]);
+        for (int ks = 0; ks < CK; ks += 2) {
+            own[slot(lane >> 2, lane & 3)] = as_uint4(w[ks]);
+            own[slot(16 + (lane >> 2), lane & 3)] = as_uint4(w[ks + 1]);
+            w[ks] = as_bf16x8(own[slot(r, g)]);
+            w[ks + 1] = as_bf16x8(own[slot(r, 2 + g)]);
         }
-        *(reinterpret_cast<bf16x4 *>(result + r * 16 + ((4 * wave + a) ^ (r & 15))) + g) = ov;
     }
-    __syncthreads();
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int at = (tid >> 4) + 16 * i;
-        uint4 v = result[at * 16 + ((tid & 15) ^ (at & 15))];
-        if constexpr (EPILOGUE == EPILOGUE_RESIDUAL) {
-            const bf16x8 o = as_bf16x8(v), zz = as_bf16x8(z[i]);
-            bf16x8 sum;
+        for (int i = 0; i < LOADS; ++i) {
+            const int idx = tid + 256 * i, row = idx / SLOTS;
+            rows[row * SLOTS + (idx % SLOTS ^ (row & 15))] = as_uint4(in[i]);
+        }
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                sum[e] = (bf16_t)(to_f32(zz[e]) + to_f32(o[e]));
+        for (int i = 0; i < 2; ++i) {
+            to[i] = next_to[i];
+            z[i] = next_z[i];
+        }
+        __syncthreads(); // (the previous result has been read, too)
+        if (WALK && tile + (int)gridDim.x < tiles) {
+            fetch(tile + gridDim.x);
+            fetch_out(tile + gridDim.x);
+        }
+        f32x16 acc = zero16();
+#pragma unroll
+        for (int ks = 0; ks < CK; ++ks) {
+            acc = mfma(w[ks], as_bf16x8(rows[r * SLOTS + ((2 * ks + g) ^ (r & 15))]), acc);
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            bf16x4 ov;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                ov[c] = (bf16_t)(acc[4 * a + c] + bv[a][c]);
             }
-            v = as_uint4(sum);
+            *(reinterpret_cast<bf16x4 *>(result + r * 16 + ((4 * wave + a) ^ (r & 15))) + g) = ov;
         }
-        if (at <= last) {
-            *reinterpret_cast<uint4 *>(to[i]) = v;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int at = (tid >> 4) + 16 * i;
+            uint4 v = result[at * 16 + ((tid & 15) ^ (at & 15))];
+            if constexpr (EPILOGUE == EPILOGUE_RESIDUAL) {
+                const bf16x8 o = as_bf16x8(v), zz = z[i];
+                bf16x8 sum;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    sum[e] = (bf16_t)(to_f32(zz[e]) + to_f32(o[e]));
+                }
+                v = as_uint4(sum);
+            }
+            if (tile * 32 + at < M) {
+                *reinterpret_cast<uint4 *>(to[i]) = v;
+            }
+        }
+        if (!WALK) {
+            return;
         }
     }
 }
@@ -2833,8 +2873,10 @@ int launch_output_projection(const void *a, int64_t a_ld, const void *w, const f
         // not where the result lies over the rows: one workgroup's features would be written while another still reads them
         const uintptr_t from = reinterpret_cast<uintptr_t>(a), to = reinterpret_cast<uintptr_t>(out);
         const bool apart = from + (uintptr_t)(2 * ((M - 1) * a_ld + C)) <= to || to + (uintptr_t)(2 * ((M - 1) * out_ld + N)) <= from;
-        if (apart && tiles * slabs <= TILE_WORKGROUPS_PER_CU * (int64_t)kutacc_cu_count()) {
-            output_projection_tile_kernel<C, EPILOGUE><<<dim3((unsigned)tiles, (unsigned)slabs), 256, 0, stream>>>(
+        const int64_t cus = kutacc_cu_count();
+        if (apart && M < (1 << 30) && (C == 128 || tiles * slabs <= TILE_WORKGROUPS_PER_CU * cus)) {
+            const int64_t gx = C == 128 ? std::min(tiles, std::max<int64_t>(WALKERS_PER_CU * cus / slabs, 1)) : tiles;
+            output_projection_tile_kernel<C, EPILOGUE><<<dim3((unsigned)gx, (unsigned)slabs), 256, 0, stream>>>(
                 (const bf16_t *)a, a_ld, (const bf16_t *)w, bias, (bf16_t *)out, out_ld, (int)M, (int)swap_n);
             return kutacc_hip_status(hipGetLastError());
         }

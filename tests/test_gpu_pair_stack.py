@@ -754,15 +754,16 @@ def row_projection_args(a, w, bias, out):
 @pytest.mark.parametrize("k,n", [(128, 128), (128, 384), (256, 128), (256, 256), (256, 512)])
 def test_row_projections_on_either_side_of_the_tile_kernel_s_rows(torch_cuda, k, n):
     """Rows of 128 and 256 features against a dense matrix: one row, a tile of 32 less and more one, the last number of rows whose 32 x 128
-    tiles are a workgroup each (five a CU), and one more; rows wider than the product, nothing written between them."""
+    tiles are a workgroup each (three a CU, and with 256 features twelve), one more, and several tiles a workgroup; rows wider than the
+    product, nothing written between them."""
     torch = torch_cuda
-    limit = 32 * (5 * torch.cuda.get_device_properties(0).multi_processor_count // (n // 128))
+    limit = 32 * ((3 if k == 128 else 12) * torch.cuda.get_device_properties(0).multi_processor_count // (n // 128))
     g = torch.Generator(device="cuda").manual_seed(k + n)
     w = (torch.randn(n, k, device="cuda", generator=g) * k ** -0.5).to(torch.bfloat16)
     bias = torch.randn(n, device="cuda", generator=g)
-    full = torch.randn(limit + 1, k + 8, device="cuda", generator=g).to(torch.bfloat16)
+    full = torch.randn(2 * limit + 45, k + 8, device="cuda", generator=g).to(torch.bfloat16)
     results = {}
-    for m in (1, 31, 33, limit, limit + 1):
+    for m in (1, 31, 33, limit, limit + 1, 2 * limit + 45):
         a, out = full[:m, :k], torch.full((m, n + 16), 3.0, device="cuda", dtype=torch.bfloat16)
         rc = capi.lib().kutacc_hip_gemm(ctypes.byref(row_projection_args(a, w, bias, out)), None)
         torch.cuda.synchronize()
@@ -772,8 +773,8 @@ def test_row_projections_on_either_side_of_the_tile_kernel_s_rows(torch_cuda, k,
         assert bool((out[:, n:] == 3.0).all())
         results[m] = out
     # the same products in the same order: rows of either kernel are the same bits
-    for m in (1, 31, 33, limit):
-        assert helpers.same_bits(results[m], results[limit + 1][:m].contiguous())
+    for m in (1, 31, 33, limit, limit + 1):
+        assert helpers.same_bits(results[m], results[2 * limit + 45][:m].contiguous())
 
 
 @pytest.mark.parametrize("n", [256])
