@@ -2394,23 +2394,24 @@ __global__ __launch_bounds__(C == 128 ? 256 : 512, C == 128 ? 2 : 1) void output
 // for rows, weights, bias and the rows of `out` at once, where output_projection_kernel waits for its weights, then for the later channels of
 // its rows and for `out` in turn, with a few dozen workgroups where rows are few.  With 128 channels it keeps its weights in registers and walks
 // the tiles, three workgroups a CU, the next tile's rows and `out` under way: faster than output_projection_kernel at every size.
-// With 256 there are no registers for that (walking 128 sequences x 128 residues 39.5 -> 42): a tile each, the weights fetched for every tile,
-// and no gain is left past some twelve workgroups a CU.
+// With 256 four waves have no registers for that (128 sequences x 128 residues 39.5 -> 42); there eight waves walk for all 256 features, one
+// workgroup a CU, where that gives each more than one tile and no half of its features is missing.  Fewer tiles, or an odd number
+// of 128 features, have a workgroup of four waves each, which fetches the weights again: no gain is left past some twelve a CU (300000 rows
+// to 128 features 43 in either kernel).
 // Whole calls, us, output_projection_kernel's -> now: triangle attention of 50, 77, 128 and 200 residues 19.3 -> 15.3, 22.0 -> 18.0,
 // 24.7 -> 21.9, 48.4 -> 44.3, of 256, 400, 450 and 691 52 -> 50, 174 -> 166, 218 -> 208, 504 -> 500; attention of 384 x 384, 4 heads
-// 98.5 -> 93.2; MSA rows, 64 x 100 38.2 -> 27.0, 128 x 128 48.4 -> 39.5, 150 x 150 63.5 -> 57.7, 200 x 200 (2500 tiles) 89.8 -> 88.5; MSA
-// columns, 500 x 100 (3126) 113.8 and 113.9.
-constexpr int WALKERS_PER_CU = 3, TILE_WORKGROUPS_PER_CU = 12;
-template <int C, int EPILOGUE>
-__global__ __launch_bounds__(256, C == 128 ? 3 : 2) void output_projection_tile_kernel(const bf16_t *__restrict__ avg, int64_t avg_ld, const bf16_t *__restrict__ wo,
+// 98.5 -> 93.2, of 256 x 384, 8 heads 190 -> 179; MSA rows, 64 x 100 38.2 -> 27.0, 128 x 128 48.4 -> 39.5, 150 x 150 63.5 -> 56,
+// 200 x 200 89.8 -> 85.5; MSA columns, 600 x 160 222 -> 207.
+constexpr int TILE_WORKGROUPS_PER_CU = 12;
+template <int C, int EPILOGUE, int F, bool WALK>
+__global__ __launch_bounds__(2 * F, WALK && F == 128 ? 3 : 2) void output_projection_tile_kernel(const bf16_t *__restrict__ avg, int64_t avg_ld, const bf16_t *__restrict__ wo,
                                                                      const float *__restrict__ bo, bf16_t *__restrict__ out, int64_t out_ld, int M, int swap_n)
 {
-    constexpr bool WALK = C == 128;
-    constexpr int CK = C / 16, SLOTS = C / 8, LOADS = 32 * SLOTS / 256;
-    __shared__ uint4 rows[32 * SLOTS], result[32 * 16]; // slots XOR-ed with row % 16
+    constexpr int CK = C / 16, SLOTS = C / 8, THREADS = 2 * F, LOADS = 32 * SLOTS / THREADS, PIECES = F / 8;
+    __shared__ uint4 rows[32 * SLOTS], result[32 * PIECES]; // slots XOR-ed with row % 16
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
-    const int n0 = (int)blockIdx.y * 128, f0 = n0 + 32 * wave;
+    const int n0 = (int)blockIdx.y * F, f0 = n0 + 32 * wave;
     const int tiles = (M + 31) / 32;
     bf16x8 in[LOADS];
     bf16_t *to[2], *next_to[2]; // the thread's two pieces of 8 features of `out`
@@ -2419,7 +2420,7 @@ __global__ __launch_bounds__(256, C == 128 ? 3 : 2) void output_projection_tile_
         const int row0 = tile * 32, last = min(M - 1 - row0, 31); // its last row that is one
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
-            const int idx = tid + 256 * i;
+            const int idx = tid + THREADS * i;
             in[i] = *reinterpret_cast<const bf16x8 *>(avg + (int64_t)(row0 + min(idx / SLOTS, last)) * avg_ld + idx % SLOTS * 8);
         }
     };
@@ -2427,10 +2428,10 @@ __global__ __launch_bounds__(256, C == 128 ? 3 : 2) void output_projection_tile_
         const int row0 = tile * 32, last = min(M - 1 - row0, 31);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int at = (tid >> 4) + 16 * i;
+            const int at = tid / PIECES + 16 * i;
             const int row = row0 + min(at, last);
             const int target = EPILOGUE == EPILOGUE_RESIDUAL && swap_n ? (int)((uint32_t)row % (uint32_t)swap_n) * (M / swap_n) + (int)((uint32_t)row / (uint32_t)swap_n) : row;
-            next_to[i] = out + (int64_t)target * out_ld + n0 + (tid & 15) * 8;
+            next_to[i] = out + (int64_t)target * out_ld + n0 + tid % PIECES * 8;
             if constexpr (EPILOGUE == EPILOGUE_RESIDUAL) {
                 next_z[i] = *reinterpret_cast<const bf16x8 *>(next_to[i]);
             }
@@ -2464,7 +2465,7 @@ __global__ __launch_bounds__(256, C == 128 ? 3 : 2) void output_projection_tile_
     for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
-            const int idx = tid + 256 * i, row = idx / SLOTS;
+            const int idx = tid + THREADS * i, row = idx / SLOTS;
             rows[row * SLOTS + (idx % SLOTS ^ (row & 15))] = as_uint4(in[i]);
         }
 #pragma unroll
@@ -2489,13 +2490,13 @@ __global__ __launch_bounds__(256, C == 128 ? 3 : 2) void output_projection_tile_
             for (int c = 0; c < 4; ++c) {
                 ov[c] = (bf16_t)(acc[4 * a + c] + bv[a][c]);
             }
-            *(reinterpret_cast<bf16x4 *>(result + r * 16 + ((4 * wave + a) ^ (r & 15))) + g) = ov;
+            *(reinterpret_cast<bf16x4 *>(result + r * PIECES + ((4 * wave + a) ^ (r & 15))) + g) = ov;
         }
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int at = (tid >> 4) + 16 * i;
-            uint4 v = result[at * 16 + ((tid & 15) ^ (at & 15))];
+            const int at = tid / PIECES + 16 * i;
+            uint4 v = result[at * PIECES + (tid % PIECES ^ (at & 15))];
             if constexpr (EPILOGUE == EPILOGUE_RESIDUAL) {
                 const bf16x8 o = as_bf16x8(v), zz = z[i];
                 bf16x8 sum;
@@ -2874,11 +2875,22 @@ int launch_output_projection(const void *a, int64_t a_ld, const void *w, const f
         const uintptr_t from = reinterpret_cast<uintptr_t>(a), to = reinterpret_cast<uintptr_t>(out);
         const bool apart = from + (uintptr_t)(2 * ((M - 1) * a_ld + C)) <= to || to + (uintptr_t)(2 * ((M - 1) * out_ld + N)) <= from;
         const int64_t cus = kutacc_cu_count();
-        if (apart && M < (1 << 30) && (C == 128 || tiles * slabs <= TILE_WORKGROUPS_PER_CU * cus)) {
-            const int64_t gx = C == 128 ? std::min(tiles, std::max<int64_t>(WALKERS_PER_CU * cus / slabs, 1)) : tiles;
-            output_projection_tile_kernel<C, EPILOGUE><<<dim3((unsigned)gx, (unsigned)slabs), 256, 0, stream>>>(
+        const auto launch = [&](auto kern, int features, int64_t per_cu) {
+            const int64_t gx = std::min(tiles, std::max<int64_t>(per_cu * cus / (N / features), 1));
+            kern<<<dim3((unsigned)gx, (unsigned)(N / features)), 2 * features, 0, stream>>>(
                 (const bf16_t *)a, a_ld, (const bf16_t *)w, bias, (bf16_t *)out, out_ld, (int)M, (int)swap_n);
             return kutacc_hip_status(hipGetLastError());
+        };
+        if (apart && M < (1 << 30)) {
+            if (C == 128) {
+                return launch(output_projection_tile_kernel<C, EPILOGUE, 128, C == 128>, 128, 3);
+            }
+            if (N % 256 == 0 && tiles * (N / 256) > cus) {
+                return launch(output_projection_tile_kernel<C, EPILOGUE, C, true>, 256, 1);
+            }
+            if (tiles * slabs <= TILE_WORKGROUPS_PER_CU * cus) {
+                return launch(output_projection_tile_kernel<C, EPILOGUE, 128, C == 128>, 128, INT_MAX);
+            }
         }
     }
     // the transposing residual epilogue finds its rows of `out` with 32-bit arithmetic where the tensor allows (without

@@ -754,10 +754,10 @@ def row_projection_args(a, w, bias, out):
 @pytest.mark.parametrize("k,n", [(128, 128), (128, 384), (256, 128), (256, 256), (256, 512)])
 def test_row_projections_on_either_side_of_the_tile_kernel_s_rows(torch_cuda, k, n):
     """Rows of 128 and 256 features against a dense matrix: one row, a tile of 32 less and more one, the last number of rows whose 32 x 128
-    tiles are a workgroup each (three a CU, and with 256 features twelve), one more, and several tiles a workgroup; rows wider than the
-    product, nothing written between them."""
+    tiles are a workgroup each (three a CU; with 256 features one for every 256 of the result, or twelve for 128), one more, and several tiles
+    a workgroup; rows wider than the product, nothing written between them."""
     torch = torch_cuda
-    limit = 32 * ((3 if k == 128 else 12) * torch.cuda.get_device_properties(0).multi_processor_count // (n // 128))
+    limit = 32 * ((3 if k == 128 else 12 if n % 256 else 2) * torch.cuda.get_device_properties(0).multi_processor_count // (n // 128))
     g = torch.Generator(device="cuda").manual_seed(k + n)
     w = (torch.randn(n, k, device="cuda", generator=g) * k ** -0.5).to(torch.bfloat16)
     bias = torch.randn(n, device="cuda", generator=g)
