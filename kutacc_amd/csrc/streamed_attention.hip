@@ -883,135 +883,114 @@ __global__ __launch_bounds__(768) void streamed_plain_kernel(const StreamedParam
 // ---- the output projection ----
 //
 // act += avg . Wo^T + bo, row (b, s) of the product to row (b, s) of act, or transposed to row (s, b).  Bound by HBM: 2 C bytes a
-// position in, and 4 C of act.  The gated average arrives as MFMA fragments, 1 KB a load instruction, requested a block ahead; the
-// weights stay in the LDS with their head dims in the order of those fragments; the product (rows = features, columns =
-// positions) crosses the wave's panel to meet the activation in whole cache lines.  act, weights and bias lie on any address.
+// position in, and 4 C of act.  A wave keeps the weights of 32 features in registers, their head dims in the order of the fragments in which the
+// gated average arrives; a workgroup of all features walks blocks of 32 positions, which its waves share in the LDS, the next block
+// and its activations under way.  The product (rows = features, columns = positions) crosses the LDS to meet the activation in whole
+// cache lines.  act, weights and bias lie on any address.  With the weights in the LDS, read for every block by waves that walked
+// alone, MSA rows of 508 x 259 took 50 us of this kernel, now 43, 300 x 300 37 and 26, columns of 500 x 100 26 and 17.5,
+// triangle attention of 2048 residues 652 and 617, of 1000 141 and 141.
 template <int C>
-struct OutputShape {
-    static constexpr int SLABS = C / 128, WAVES = 4 * SLABS; // 128 features of Wo per slab; two workgroups a CU, or one of both slabs
-    static constexpr size_t LDS = (size_t)(SLABS * 4 * (C / 16) * 64 + WAVES * 256) * 16;
-};
-
-template <int C>
-__global__ __launch_bounds__(64 * OutputShape<C>::WAVES, C == 128 ? 2 : 1) void output_projection_kernel(
+__global__ __launch_bounds__(2 * C, 2) void output_projection_kernel(
     const uint4 *__restrict__ avg, const bf16_t *__restrict__ wo, const float *__restrict__ bo, bf16_t *__restrict__ act, int64_t ld,
     int B, int S, int H, int NB, int transposed)
 {
-    constexpr int CK = C / 16, SLABS = OutputShape<C>::SLABS, W = OutputShape<C>::WAVES, THREADS = 64 * W;
-    extern __shared__ uint4 lds[]; // [4 SLABS feature blocks][CK][64 lanes], a panel per wave
+    constexpr int CK = C / 16, THREADS = 2 * C, LOADS = CK * 64 / THREADS, PIECES = C / 8;
+    __shared__ uint4 block[CK * 64], result[32 * PIECES]; // a position's pieces XOR-ed with position % 16
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
-    uint4 *panel = lds + SLABS * 4 * CK * 64 + wave * 256;
-    // A unit is a block of positions and a slab.  With two slabs a wave takes a run of units: what some waves have more than others is
-    // half a block.  With one, neighbouring waves take neighbouring blocks (1024 residues 137 us, in runs 150).
-    const int units = B * NB * SLABS, waves = (int)gridDim.x * W, me = (int)blockIdx.x * W + wave;
-    const int stride = SLABS == 1 ? waves : 1, first = SLABS == 1 ? me : (int)((int64_t)units * me / waves);
-    const int stop = SLABS == 1 ? units : (int)((int64_t)units * (me + 1) / waves);
-    struct Rows {
-        uint4 f[CK];
-    };
-    auto load = [&](int unit) { // the fragments of a unit's block, k-steps 2 h and 2 h + 1 = head h
-        const int block = min(unit, units - 1) / SLABS, b = block / NB, j = block - b * NB;
-        const uint4 *src = avg + ((int64_t)b * H * NB + j) * BLOCK_SLOTS + lane;
-        Rows t;
-#pragma unroll
-        for (int h = 0; h < CK / 2; ++h) {
-            t.f[2 * h] = src[(int64_t)h * NB * BLOCK_SLOTS], t.f[2 * h + 1] = src[(int64_t)h * NB * BLOCK_SLOTS + 64];
-        }
-        return t;
-    };
-    // a unit's 64 features `half` of the activation: row (b, position), pieces of lane / 8 + 8 i
+    const int units = B * NB;
     const int64_t step = (transposed ? (int64_t)B : 1) * ld * 2;
-    struct Where {
-        char *base; // lane's piece of position 32 j
-        int last;   // last position of the block that is one, counted in it
-    };
-    auto where = [&](int unit) {
-        const int at = min(unit, units - 1), block = at / SLABS, b = block / NB, j = block - b * NB;
-        const int64_t row = transposed ? (int64_t)32 * j * B + b : (int64_t)b * S + 32 * j;
-        return Where{reinterpret_cast<char *>(act) + row * ld * 2 + (at % SLABS) * 256 + 16 * (lane & 7), min(31, S - 1 - 32 * j)};
-    };
-    struct Piece {
-        uint4 z[4];
-    };
-    auto load_act = [&](const Where &w, int half) {
-        Piece t;
+    const int pos[2] = {tid / PIECES, tid / PIECES + 16}; // the thread's pieces of 8 features of the activation
+    bf16x8 in[LOADS], z[2], next_z[2];
+    char *to[2], *next_to[2];
+    auto fetch = [&](int unit) {
+        const int b = unit / NB, j = unit - b * NB, last = min(31, S - 1 - 32 * j); // last position of the block that is one
+        const uint4 *src = avg + ((int64_t)b * H * NB + j) * BLOCK_SLOTS;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            __builtin_memcpy(&t.z[i], w.base + min(8 * i + (lane >> 3), w.last) * step + 128 * half, 16);
+        for (int i = 0; i < LOADS; ++i) { // k-steps 2 h and 2 h + 1 = head h
+            const int at = tid + THREADS * i;
+            in[i] = *reinterpret_cast<const bf16x8 *>(src + (int64_t)(at / BLOCK_SLOTS) * NB * BLOCK_SLOTS + at % BLOCK_SLOTS);
         }
-        return t;
+        const int64_t row = transposed ? (int64_t)32 * j * B + b : (int64_t)b * S + 32 * j;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            next_to[i] = reinterpret_cast<char *>(act) + row * ld * 2 + min(pos[i], last) * step + tid % PIECES * 16;
+            __builtin_memcpy(&next_z[i], next_to[i], 16);
+        }
     };
-    Rows next = load(first);
-    Where here = where(first);
-    Piece z = load_act(here, 0); // the activation arrives a half ahead of the result it is added to
-    for (int at = tid; at < SLABS * 4 * CK * 64; at += THREADS) {
-        // elements e of lane half g: head dims 16 ks + 4 g + e (e < 4), 16 ks + 8 + 4 g + e - 4
-        const int ln = at & 63, ks = (at >> 6) % CK, row = (at >> 6) / CK * 32 + (ln & 31);
-        const bf16_t *src = wo + row * C + ks * 16 + 4 * (ln >> 5);
-        uint64_t lo, hi;
-        __builtin_memcpy(&lo, src, 8);
-        __builtin_memcpy(&hi, src + 8, 8);
-        lds[at] = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+    fetch(blockIdx.x);
+    bf16x8 w[CK];
+#pragma unroll
+    for (int ks = 0; ks < CK; ++ks) { // in half lines, 16 rows by 32 channels a load
+        __builtin_memcpy(&w[ks], wo + (int64_t)(32 * wave + 16 * (ks & 1) + (lane >> 2)) * C + (ks >> 1) * 32 + (lane & 3) * 8, 16);
     }
-    __syncthreads();
-    for (int unit = first; unit < stop; unit += stride) {
-        const Rows rows = next;
-        const Where at = here;
-        const int slab = unit % SLABS;
-        here = where(unit + stride);
+    f32x4 bv[4];
 #pragma unroll
-        for (int half = 0; half < 2; ++half) { // 64 features per panel
-            f32x16 acc[2]; // from the bias; its loads in front of those for the next half, which are still on their way when it is used
+    for (int a = 0; a < 4; ++a) {
+        __builtin_memcpy(&bv[a], bo + 32 * wave + 8 * a + 4 * g, 16);
+    }
+    {
+        // elements e of lane half g: head dims 16 ks + 4 g + e (e < 4), 16 ks + 8 + 4 g + e - 4; through 2 KB that are the wave's own
+        uint4 *own = result + 128 * wave;
+        const auto slot = [](int row, int piece) { return 4 * row + (piece ^ ((row >> 2) & 3)); };
 #pragma unroll
-            for (int n = 0; n < 2; ++n) {
+        for (int ks = 0; ks < CK; ks += 2) {
+            own[slot(lane >> 2, lane & 3)] = as_uint4(w[ks]);
+            own[slot(16 + (lane >> 2), lane & 3)] = as_uint4(w[ks + 1]);
 #pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    f32x4 bv;
-                    __builtin_memcpy(&bv, bo + slab * 128 + half * 64 + n * 32 + 8 * a + 4 * g, 16);
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        acc[n][4 * a + c] = bv[c];
-                    }
-                }
+            for (int k = 0; k < 2; ++k) {
+                uint2 lo, hi;
+                __builtin_memcpy(&lo, reinterpret_cast<const char *>(own + slot(r, 2 * k)) + 8 * g, 8);
+                __builtin_memcpy(&hi, reinterpret_cast<const char *>(own + slot(r, 2 * k + 1)) + 8 * g, 8);
+                w[ks + k] = as_bf16x8(make_uint4(lo.x, lo.y, hi.x, hi.y));
             }
-            __builtin_amdgcn_sched_barrier(0);
-            const Piece in = z;
-            z = half == 0 ? load_act(at, 1) : load_act(here, 0);
-            if (half == 0 && (SLABS == 1 || slab == SLABS - 1)) { // else the next unit is of the same block
-                next = load(unit + stride);
+        }
+    }
+    for (int unit = blockIdx.x; unit < units; unit += gridDim.x) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            block[tid + THREADS * i] = as_uint4(in[i]);
+        }
+        const int last = min(31, S - 1 - 32 * (unit % NB));
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            to[i] = next_to[i];
+            z[i] = next_z[i];
+        }
+        __syncthreads(); // (the previous result has been read, too)
+        if (unit + (int)gridDim.x < units) {
+            fetch(unit + gridDim.x);
+        }
+        f32x16 acc;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            acc[v] = bv[v >> 2][v & 3];
+        }
+#pragma unroll
+        for (int ks = 0; ks < CK; ++ks) {
+            acc = mfma(w[ks], as_bf16x8(block[ks * 64 + lane]), acc);
+        }
+        const int p = pi_row(r);
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            bf16x4 ov;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                ov[c] = (bf16_t)acc[4 * a + c];
             }
-            __builtin_amdgcn_sched_barrier(0);
-            const uint4 *w = lds + (slab * 4 + 2 * half) * CK * 64 + lane;
+            *(reinterpret_cast<bf16x4 *>(result + p * PIECES + ((4 * wave + a) ^ (p & 15))) + g) = ov;
+        }
+        __syncthreads();
 #pragma unroll
-            for (int ks = 0; ks < CK; ++ks) {
-                acc[0] = mfma(as_bf16x8(w[ks * 64]), as_bf16x8(rows.f[ks]), acc[0]);
-                acc[1] = mfma(as_bf16x8(w[(CK + ks) * 64]), as_bf16x8(rows.f[ks]), acc[1]);
+        for (int i = 0; i < 2; ++i) {
+            const bf16x8 o = as_bf16x8(result[pos[i] * PIECES + (tid % PIECES ^ (pos[i] & 15))]);
+            bf16x8 sum;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                sum[e] = (bf16_t)(to_f32(z[i][e]) + to_f32(o[e]));
             }
-#pragma unroll
-            for (int n = 0; n < 2; ++n) {
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    bf16x4 ov;
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        ov[c] = (bf16_t)acc[n][4 * a + c];
-                    }
-                    *(reinterpret_cast<bf16x4 *>(panel + panel_slot(pi_row(r), n * 4 + a)) + g) = ov;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int pos = 8 * i + (lane >> 3);
-                const bf16x8 o = as_bf16x8(panel[panel_slot(pos, lane & 7)]), x = as_bf16x8(in.z[i]);
-                bf16x8 sum;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    sum[e] = (bf16_t)(to_f32(x[e]) + to_f32(o[e]));
-                }
-                if (pos <= at.last) {
-                    __builtin_memcpy(at.base + pos * step + 128 * half, &sum, 16);
-                }
+            if (pos[i] <= last) {
+                __builtin_memcpy(to[i], &sum, 16);
             }
         }
     }
@@ -1062,17 +1041,16 @@ int launch_plain(StreamedParams p, hipStream_t stream)
     return kutacc_hip_status(hipGetLastError());
 }
 
+// workgroups a CU, as the registers allow with 256 channels; with 128, columns of 2048 x 2048 pairs 621 us, with three 658, with four 682, and
+// no difference up to 1000 x 1000
+template <int C>
+constexpr int OUTPUT_PER_CU = C == 128 ? 2 : 1;
 template <int C>
 int launch_output(const StreamedParams &p, const void *wo, const float *bo, void *act, int64_t ld, bool transposed, hipStream_t stream)
 {
-    using Shape = OutputShape<C>;
-    static size_t configured[KUTACC_DEVICE_SLOTS] = {};
-    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&output_projection_kernel<C>), Shape::LDS, configured)) {
-        return kutacc_hip_status(e);
-    }
-    const int64_t units = (int64_t)p.B * p.NB * Shape::SLABS, full = kutacc_cu_count() * (C == 128 ? 2 : 1);
     kutacc_prof::KernelTimer t("output_projection_kernel<residual>", 2.0 * (double)p.B * p.S * C * C, stream);
-    output_projection_kernel<C><<<dim3((unsigned)std::min(full, (units + Shape::WAVES - 1) / Shape::WAVES)), 64 * Shape::WAVES, Shape::LDS, stream>>>(
+    const int64_t units = (int64_t)p.B * p.NB, full = (int64_t)kutacc_cu_count() * OUTPUT_PER_CU<C>;
+    output_projection_kernel<C><<<dim3((unsigned)std::min(full, units)), 2 * C, 0, stream>>>(
         p.q, (const bf16_t *)wo, bo, (bf16_t *)act, ld, p.B, p.S, p.H, p.NB, transposed ? 1 : 0);
     return kutacc_hip_status(hipGetLastError());
 }
