@@ -2438,30 +2438,15 @@ __global__ __launch_bounds__(2 * F, WALK && F == 128 ? 3 : 2) void output_projec
         }
     };
     fetch(blockIdx.x);
-    // weights in half lines, 16 rows by 32 channels a load, put into fragment order below through 2 KB of `result` that are the
-    // wave's own: loaded in fragment order, each takes the address path 42 cycles instead of 16
     bf16x8 w[CK];
-#pragma unroll
-    for (int ks = 0; ks < CK; ++ks) {
-        w[ks] = *reinterpret_cast<const bf16x8 *>(wo + (int64_t)(f0 + 16 * (ks & 1) + (lane >> 2)) * C + (ks >> 1) * 32 + (lane & 3) * 8);
-    }
+    load_half_lines<CK>(w, wo + (int64_t)f0 * C, C, lane);
     fetch_out(blockIdx.x);
     f32x4 bv[4];
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
         bv[a] = *reinterpret_cast<const f32x4 *>(bo + f0 + 8 * a + 4 * g);
     }
-    {
-        uint4 *own = result + 128 * wave;
-        const auto slot = [](int row, int piece) { return 4 * row + (piece ^ ((row >> 2) & 3)); };
-#pragma unroll
-        for (int ks = 0; ks < CK; ks += 2) {
-            own[slot(lane >> 2, lane & 3)] = as_uint4(w[ks]);
-            own[slot(16 + (lane >> 2), lane & 3)] = as_uint4(w[ks + 1]);
-            w[ks] = as_bf16x8(own[slot(r, g)]);
-            w[ks + 1] = as_bf16x8(own[slot(r, 2 + g)]);
-        }
-    }
+    half_lines_to_fragments<CK>(w, result + 128 * wave, lane);
     for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {

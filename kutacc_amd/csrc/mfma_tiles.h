@@ -128,6 +128,30 @@ __device__ __forceinline__ float quarter_swap_sum(float x)
 
 __device__ __forceinline__ uint4 zero_u4() { return make_uint4(0u, 0u, 0u, 0u); }
 
+// A wave's block of weights, 32 rows by 16 CK channels, as fragments of a 32x32x16 product: lane r + 32 g holds channels 16 ks + 8 g .. + 7
+// of row r.  Loaded in half lines, 16 rows by 32 channels a load -- in fragment order, 16 bytes of another row in every lane, a load takes
+// the address path 42 cycles instead of 16 -- and brought into that order through 2 KB of the LDS that are the wave's own.
+template <int CK>
+__device__ __forceinline__ void load_half_lines(bf16x8 (&w)[CK], const bf16_t *rows, int64_t ld, int lane)
+{
+#pragma unroll
+    for (int ks = 0; ks < CK; ++ks) { // on any address
+        __builtin_memcpy(&w[ks], rows + (int64_t)(16 * (ks & 1) + (lane >> 2)) * ld + (ks >> 1) * 32 + (lane & 3) * 8, 16);
+    }
+}
+__device__ __forceinline__ int half_line_slot(int row, int piece) { return 4 * row + (piece ^ ((row >> 2) & 3)); } // 16 rows' pieces in 16 bank groups
+template <int CK>
+__device__ __forceinline__ void half_lines_to_fragments(bf16x8 (&w)[CK], uint4 *own, int lane)
+{
+#pragma unroll
+    for (int ks = 0; ks < CK; ks += 2) {
+        own[half_line_slot(lane >> 2, lane & 3)] = as_uint4(w[ks]);
+        own[half_line_slot(16 + (lane >> 2), lane & 3)] = as_uint4(w[ks + 1]);
+        w[ks] = as_bf16x8(own[half_line_slot(lane & 31, lane >> 5)]);
+        w[ks + 1] = as_bf16x8(own[half_line_slot(lane & 31, 2 + (lane >> 5))]);
+    }
+}
+
 // Eight bf16 from a row of `length`, from element `at` on; elements past the end are zero (never read).  Rows start on any
 // even address: the hardware's unaligned 16-byte loads serve them, and the last piece of a row is the row's last eight
 // elements, shifted down.

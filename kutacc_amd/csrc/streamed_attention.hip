@@ -167,11 +167,10 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
     bf16x8 w0[CK], w1[CK]; // Q and gate, or K and V
     {
         const bf16_t *m0 = forms_kv ? p.wk : p.wq, *m1 = forms_kv ? p.wv : p.wg;
-#pragma unroll
-        for (int ks = 0; ks < CK; ++ks) {
-            const int at = (h * HEAD + r) * C + ks * 16 + g * 8;
-            w0[ks] = as_bf16x8(load8_any(m0, at)), w1[ks] = as_bf16x8(load8_any(m1, at)); // once per workgroup: on any address
-        }
+        load_half_lines<CK>(w0, m0 + h * HEAD * C, C, lane);
+        load_half_lines<CK>(w1, m1 + h * HEAD * C, C, lane);
+        half_lines_to_fragments<CK>(w0, lds + 128 * wave, lane); // on the stages, which are empty still
+        half_lines_to_fragments<CK>(w1, lds + 128 * wave, lane);
     }
     __syncthreads();
     park(0, rows, lane);
@@ -920,10 +919,7 @@ __global__ __launch_bounds__(2 * C, 2) void output_projection_kernel(
     };
     fetch(blockIdx.x);
     bf16x8 w[CK];
-#pragma unroll
-    for (int ks = 0; ks < CK; ++ks) { // in half lines, 16 rows by 32 channels a load
-        __builtin_memcpy(&w[ks], wo + (int64_t)(32 * wave + 16 * (ks & 1) + (lane >> 2)) * C + (ks >> 1) * 32 + (lane & 3) * 8, 16);
-    }
+    load_half_lines<CK>(w, wo + 32 * wave * C, C, lane);
     f32x4 bv[4];
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
@@ -932,16 +928,15 @@ __global__ __launch_bounds__(2 * C, 2) void output_projection_kernel(
     {
         // elements e of lane half g: head dims 16 ks + 4 g + e (e < 4), 16 ks + 8 + 4 g + e - 4; through 2 KB that are the wave's own
         uint4 *own = result + 128 * wave;
-        const auto slot = [](int row, int piece) { return 4 * row + (piece ^ ((row >> 2) & 3)); };
 #pragma unroll
         for (int ks = 0; ks < CK; ks += 2) {
-            own[slot(lane >> 2, lane & 3)] = as_uint4(w[ks]);
-            own[slot(16 + (lane >> 2), lane & 3)] = as_uint4(w[ks + 1]);
+            own[half_line_slot(lane >> 2, lane & 3)] = as_uint4(w[ks]);
+            own[half_line_slot(16 + (lane >> 2), lane & 3)] = as_uint4(w[ks + 1]);
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
                 uint2 lo, hi;
-                __builtin_memcpy(&lo, reinterpret_cast<const char *>(own + slot(r, 2 * k)) + 8 * g, 8);
-                __builtin_memcpy(&hi, reinterpret_cast<const char *>(own + slot(r, 2 * k + 1)) + 8 * g, 8);
+                __builtin_memcpy(&lo, reinterpret_cast<const char *>(own + half_line_slot(r, 2 * k)) + 8 * g, 8);
+                __builtin_memcpy(&hi, reinterpret_cast<const char *>(own + half_line_slot(r, 2 * k + 1)) + 8 * g, 8);
                 w[ks + k] = as_bf16x8(make_uint4(lo.x, lo.y, hi.x, hi.y));
             }
         }

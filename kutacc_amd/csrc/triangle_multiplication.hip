@@ -149,10 +149,13 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
     }
     bf16x8 wp[4], wg[4];
     f32x4 pbias, gneg;
+    // in half lines, 16 rows by 32 channels a load, and into operand order through the panel (one load in operand order takes the address
+    // path some 42 cycles instead of 16, and there are 128)
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-        wp[ks] = *reinterpret_cast<const bf16x8 *>(sd.wp + (cb * 16 + col) * C + ks * 32 + chunk * 8);
-        wg[ks] = *reinterpret_cast<const bf16x8 *>(sd.wg + (cb * 16 + col) * C + ks * 32 + chunk * 8);
+        const int at = (cb * 16 + (lane >> 2)) * C + ks * 32 + (lane & 3) * 8;
+        wp[ks] = *reinterpret_cast<const bf16x8 *>(sd.wp + at);
+        wg[ks] = *reinterpret_cast<const bf16x8 *>(sd.wg + at);
     }
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -161,6 +164,14 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
     char *out = reinterpret_cast<char *>(sd.out + (int64_t)cb * 16 * plane);
     __syncthreads();
     stage_rows(even, 0);
+    uint4 *own = reinterpret_cast<uint4 *>(panel);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        own[half_line_slot(lane >> 2, lane & 3)] = as_uint4(wp[ks]);
+        own[64 + half_line_slot(lane >> 2, lane & 3)] = as_uint4(wg[ks]);
+        wp[ks] = as_bf16x8(own[half_line_slot(col, chunk)]);
+        wg[ks] = as_bf16x8(own[64 + half_line_slot(col, chunk)]);
+    }
     __syncthreads();
     // The weights are waited for here: the waits that the compiler leaves to their first uses stand in the loop, where they are waits for
     // all rows and stores on their way.
@@ -299,11 +310,10 @@ __global__ __launch_bounds__(256, 2) void triangle_back_kernel(const bf16_t *__r
     load_row(row);
     next_row = row;
     bf16x8 wof[CK], wgf[CK];
-#pragma unroll
-    for (int ks = 0; ks < CK; ++ks) {
-        wof[ks] = *reinterpret_cast<const bf16x8 *>(wo + (wave * 32 + rv) * C + ks * 16 + gv * 8);
-        wgf[ks] = *reinterpret_cast<const bf16x8 *>(wg + (wave * 32 + rv) * C + ks * 16 + gv * 8);
-    }
+    load_half_lines<CK>(wof, wo + wave * 32 * C, C, lane);
+    load_half_lines<CK>(wgf, wg + wave * 32 * C, C, lane);
+    half_lines_to_fragments<CK>(wof, res + 128 * wave, lane);
+    half_lines_to_fragments<CK>(wgf, res + 128 * wave, lane);
     if (tid < C) {
         params[tid] = gamma[tid], params[C + tid] = beta[tid];
         params[2 * C + tid] = c_gamma[tid], params[3 * C + tid] = c_beta[tid];
