@@ -840,37 +840,33 @@ __device__ __forceinline__ void attend_block_direct(const uint4 *lds_k, const ui
     l_out = half_swap_sum(lsum);
 }
 
-// Copies head h's rows of `count` weight matrices (first, first + 1, ...) into LDS in MFMA fragment order.  One
-// fragment -- a matrix's 32 rows by 16 channels, 1 KB -- is one wave-wide copy, so the fragment index is wave-uniform
-// and the matrix pointer is picked with scalar selects (indexing the pointer array per lane made every copy wait for a
-// load of the pointer first).  Whole batches of eight fragments per wave go without a branch between the loads and the
-// stores: eight L2 round trips overlap instead of queueing (one at a time they were 9 % of the long-sequence kernel).
+// Copies head h's rows of the four weight matrices into LDS in MFMA fragment order.  A unit -- a matrix's 32 rows by 32 channels, two fragments
+// -- is two wave-wide loads of half lines, put in order through 2 KB of the LDS that are the wave's own: in fragment order, 16 bytes of another
+// row in every lane, a load takes the address path 42 cycles instead of 16.  The unit's index is wave-uniform and the matrix pointer
+// is picked with scalar selects (indexing the pointer array per lane made every copy wait for a load of the pointer
+// first).  Four units per wave are asked for at once: their round trips overlap instead of queueing (one at a time they were 9 % of
+// the long-sequence kernel).  Half lines against fragment order, 256 channels: MSA rows 200 x 200 84.2 -> 83.7 us, columns 128 x 200 52.9 ->
+// 52.2, attention of 128 x 256 48.7 -> 48.0; with 128 channels, half as many, no difference.
 // ------------------------------------------------------------------------------------------------
 template <int C>
-__device__ inline void stage_weight_fragments(uint4 *lds_w, const FusedParams &p, int first, int count, int h, int wave,
-                                              int nwaves, int lane)
+__device__ inline void stage_weight_fragments(uint4 *lds_w, uint4 *own, const FusedParams &p, int h, int wave, int nwaves, int lane)
 {
-    constexpr int CK = C / 16;
-    const int nfrag = count * CK;
-    auto fragment = [&](int f) {
-        const int m = first + f / CK, ks = f % CK;
-        const bf16_t *w = m == 0 ? p.w[0] : m == 1 ? p.w[1] : m == 2 ? p.w[2] : p.w[3];
-        return *reinterpret_cast<const uint4 *>(w + (int64_t)(h * HEAD + (lane & 31)) * C + ks * 16 + (lane >> 5) * 8);
-    };
-    int f = wave;
-    for (; f + (WEIGHT_LOADS_IN_FLIGHT - 1) * nwaves < nfrag; f += WEIGHT_LOADS_IN_FLIGHT * nwaves) {
-        uint4 t[WEIGHT_LOADS_IN_FLIGHT];
+    constexpr int CK = C / 16, UNITS = 2 * CK, TOGETHER = 4;
+    for (int u0 = wave; u0 < UNITS; u0 += TOGETHER * nwaves) {
+        bf16x8 t[TOGETHER][2];
 #pragma unroll
-        for (int k = 0; k < WEIGHT_LOADS_IN_FLIGHT; ++k) {
-            t[k] = fragment(f + k * nwaves);
+        for (int k = 0; k < TOGETHER; ++k) {
+            const int u = min(u0 + k * nwaves, UNITS - 1), m = u / (CK / 2);
+            const bf16_t *w = m == 0 ? p.w[0] : m == 1 ? p.w[1] : m == 2 ? p.w[2] : p.w[3];
+            load_half_lines<2>(t[k], w + (int64_t)h * HEAD * C + u % (CK / 2) * 32, C, lane);
         }
 #pragma unroll
-        for (int k = 0; k < WEIGHT_LOADS_IN_FLIGHT; ++k) {
-            lds_w[(f + k * nwaves) * 64 + lane] = t[k];
+        for (int k = 0; k < TOGETHER; ++k) {
+            const int u = min(u0 + k * nwaves, UNITS - 1); // (a unit of another wave's once more, the same values)
+            half_lines_to_fragments<2>(t[k], own, lane);
+            lds_w[2 * u * 64 + lane] = as_uint4(t[k][0]);
+            lds_w[(2 * u + 1) * 64 + lane] = as_uint4(t[k][1]);
         }
-    }
-    for (; f < nfrag; f += nwaves) {
-        lds_w[f * 64 + lane] = fragment(f);
     }
 }
 
@@ -1356,7 +1352,7 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_head_kernel(F
     uint32_t *flag_words = reinterpret_cast<uint32_t *>(mask_base + 2 * NT * 32);            // two, alternating by batch row
 
     // the head's rows of the four weight matrices, in fragment order, for the whole kernel
-    stage_weight_fragments<C>(lds_w, p, 0, 4, h, wave, nthreads >> 6, lane);
+    stage_weight_fragments<C>(lds_w, panel, p, h, wave, nthreads >> 6, lane);
     if (tid == 0) {
         flag_words[0] = 0;
         flag_words[1] = 0;
@@ -1962,7 +1958,7 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_pair_kernel(F
     uint32_t *mask_base = reinterpret_cast<uint32_t *>(lds_v + 2 * NT * 2 * 64 + NB * 128); // [pair parity][row of the pair][NT*32] mask words
     uint32_t *flag_words = mask_base + 4 * NT * 32;                                         // [pair parity][row of the pair]
 
-    stage_weight_fragments<C>(lds_w, p, 0, 4, h, wave, nthreads >> 6, lane);
+    stage_weight_fragments<C>(lds_w, panel, p, h, wave, nthreads >> 6, lane);
     if (tid < 4) {
         flag_words[tid] = 0;
     }
