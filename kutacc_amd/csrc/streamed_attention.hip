@@ -884,40 +884,47 @@ __global__ __launch_bounds__(768) void streamed_plain_kernel(const StreamedParam
 // act += avg . Wo^T + bo, row (b, s) of the product to row (b, s) of act, or transposed to row (s, b).  Bound by HBM: 2 C bytes a
 // position in, and 4 C of act.  A wave keeps the weights of 32 features in registers, their head dims in the order of the fragments in which the
 // gated average arrives; a workgroup of all features walks blocks of 32 positions, which its waves share in the LDS, the next block
-// and its activations under way.  The product (rows = features, columns = positions) crosses the LDS to meet the activation in whole
+// and its activations under way; with 256 channels, one workgroup a CU, the next two (MSA columns of 1024 x 384 126 -> 119 us of this kernel; with 128,
+// two workgroups a CU, 2048 residues 617 -> 638).  The product (rows = features, columns = positions) crosses the LDS to meet the activation in whole
 // cache lines.  act, weights and bias lie on any address.  With the weights in the LDS, read for every block by waves that walked
-// alone, MSA rows of 508 x 259 took 50 us of this kernel, now 43, 300 x 300 37 and 26, columns of 500 x 100 26 and 17.5,
+// alone, MSA rows of 508 x 259 took 50 us of this kernel, now 40, 300 x 300 37 and 26, columns of 500 x 100 26 and 17,
 // triangle attention of 2048 residues 652 and 617, of 1000 141 and 141.
 template <int C>
 __global__ __launch_bounds__(2 * C, 2) void output_projection_kernel(
     const uint4 *__restrict__ avg, const bf16_t *__restrict__ wo, const float *__restrict__ bo, bf16_t *__restrict__ act, int64_t ld,
     int B, int S, int H, int NB, int transposed)
 {
-    constexpr int CK = C / 16, THREADS = 2 * C, LOADS = CK * 64 / THREADS, PIECES = C / 8;
+    constexpr int CK = C / 16, THREADS = 2 * C, LOADS = CK * 64 / THREADS, PIECES = C / 8, AHEAD = C / 128;
     __shared__ uint4 block[CK * 64], result[32 * PIECES]; // a position's pieces XOR-ed with position % 16
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
     const int units = B * NB;
     const int64_t step = (transposed ? (int64_t)B : 1) * ld * 2;
     const int pos[2] = {tid / PIECES, tid / PIECES + 16}; // the thread's pieces of 8 features of the activation
-    bf16x8 in[LOADS], z[2], next_z[2];
-    char *to[2], *next_to[2];
-    auto fetch = [&](int unit) {
+    struct Block {
+        bf16x8 in[LOADS], z[2];
+        char *to[2];
+    };
+    auto fetch = [&](Block &t, int unit) __attribute__((always_inline)) {
         const int b = unit / NB, j = unit - b * NB, last = min(31, S - 1 - 32 * j); // last position of the block that is one
         const uint4 *src = avg + ((int64_t)b * H * NB + j) * BLOCK_SLOTS;
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) { // k-steps 2 h and 2 h + 1 = head h
             const int at = tid + THREADS * i;
-            in[i] = *reinterpret_cast<const bf16x8 *>(src + (int64_t)(at / BLOCK_SLOTS) * NB * BLOCK_SLOTS + at % BLOCK_SLOTS);
+            t.in[i] = *reinterpret_cast<const bf16x8 *>(src + (int64_t)(at / BLOCK_SLOTS) * NB * BLOCK_SLOTS + at % BLOCK_SLOTS);
         }
         const int64_t row = transposed ? (int64_t)32 * j * B + b : (int64_t)b * S + 32 * j;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            next_to[i] = reinterpret_cast<char *>(act) + row * ld * 2 + min(pos[i], last) * step + tid % PIECES * 16;
-            __builtin_memcpy(&next_z[i], next_to[i], 16);
+            t.to[i] = reinterpret_cast<char *>(act) + row * ld * 2 + min(pos[i], last) * step + tid % PIECES * 16;
+            __builtin_memcpy(&t.z[i], t.to[i], 16);
         }
     };
-    fetch(blockIdx.x);
+    Block even, odd;
+    fetch(even, blockIdx.x);
+    if (AHEAD == 2) {
+        fetch(odd, min((int)(blockIdx.x + gridDim.x), units - 1));
+    }
     bf16x8 w[CK];
     load_half_lines<CK>(w, wo + 32 * wave * C, C, lane);
     f32x4 bv[4];
@@ -941,20 +948,17 @@ __global__ __launch_bounds__(2 * C, 2) void output_projection_kernel(
             }
         }
     }
-    for (int unit = blockIdx.x; unit < units; unit += gridDim.x) {
+    auto do_block = [&](int unit, Block &now) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
-            block[tid + THREADS * i] = as_uint4(in[i]);
+            block[tid + THREADS * i] = as_uint4(now.in[i]);
         }
         const int last = min(31, S - 1 - 32 * (unit % NB));
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            to[i] = next_to[i];
-            z[i] = next_z[i];
-        }
+        const bf16x8 z[2] = {now.z[0], now.z[1]};
+        char *const to[2] = {now.to[0], now.to[1]};
         __syncthreads(); // (the previous result has been read, too)
-        if (unit + (int)gridDim.x < units) {
-            fetch(unit + gridDim.x);
+        if (unit + AHEAD * (int)gridDim.x < units) {
+            fetch(now, unit + AHEAD * gridDim.x);
         }
         f32x16 acc;
 #pragma unroll
@@ -987,6 +991,12 @@ __global__ __launch_bounds__(2 * C, 2) void output_projection_kernel(
             if (pos[i] <= last) {
                 __builtin_memcpy(to[i], &sum, 16);
             }
+        }
+    };
+    for (int unit = blockIdx.x; unit < units; unit += AHEAD * gridDim.x) {
+        do_block(unit, even);
+        if (AHEAD == 2 && unit + (int)gridDim.x < units) {
+            do_block(unit + gridDim.x, odd);
         }
     }
 }
