@@ -2163,31 +2163,20 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_pair_kernel(F
 // EPILOGUE 1 (gated residual): the rounded result is not stored but folded into `out`, out += result * sigmoid(gate),
 // with gate and out read in the order they are written, 16 bytes per lane -- the last two steps of the triangle
 // multiplication (reference src/attention/triangle_multiplication.cpp:129-150) and the residual update fused into
-// its output projection.  EPILOGUE 2 (residual): out += result, where row (i, j) of the result goes to row (j, i)
-// of `out` when swap_n != 0 (rows are pairs (i, j) of an [M / swap_n, swap_n] grid): the residual update of a triangle-attention block,
-// transposed back for the ending node.
+// its output projection.  EPILOGUE 2 (residual; output_projection_tile_kernel only): out += result, where row (i, j) of the result goes to
+// row (j, i) of `out` when swap_n != 0 (rows are pairs (i, j) of an [M / swap_n, swap_n] grid): the residual update of a
+// triangle-attention block, transposed back for the ending node.
 constexpr int EPILOGUE_STORE = 0, EPILOGUE_GATED_RESIDUAL = 1, EPILOGUE_RESIDUAL = 2;
 
 // With 256 input features a workgroup has eight waves and keeps two 128-feature slabs of Wo (128 KB, the whole matrix of
 // the attention's output projection), so a row is read once for all 256 output features; with 128 it has four waves,
 // one slab, and two workgroups share a CU.
-// NEAR_OUT (residual epilogue only): fewer than 2^24 rows, less than 2^31 bytes of `out`, swap_n zero or at least 32 (the
-// launcher checks): the rows of `out` are found with 32-bit arithmetic -- one division of a wave-uniform row index per
-// 32-row step and an add, a compare and two 24-bit multiplies per row -- where 64-bit division and remainder per lane
-// and row are some 300 quarter-rate instructions per step.
-template <int C, int EPILOGUE, bool NEAR_OUT = false>
+template <int C, int EPILOGUE>
 __global__ __launch_bounds__(C == 128 ? 256 : 512, C == 128 ? 2 : 1) void output_projection_kernel(
     const bf16_t *__restrict__ avg, int64_t avg_ld, const bf16_t *__restrict__ wo, const float *__restrict__ bo,
     bf16_t *__restrict__ out, int64_t out_ld, int64_t M, int N, int rows_per_wave, const bf16_t *__restrict__ gate,
-    int64_t gate_ld, int64_t swap_n)
+    int64_t gate_ld)
 {
-    // row of `out` that receives row `row` of the result
-    auto target_row = [&](int64_t row) -> int64_t {
-        if constexpr (EPILOGUE == EPILOGUE_RESIDUAL) {
-            return swap_n ? (row % swap_n) * (M / swap_n) + row / swap_n : row; // row (b, s) of [M / n, n] -> (s, b)
-        }
-        return row;
-    };
     constexpr int CK = C / 16;
     constexpr int NP = CK / 4;
     constexpr int SLABS = C / 128, WAVES = 4 * SLABS, THREADS = 64 * WAVES;
@@ -2271,27 +2260,6 @@ __global__ __launch_bounds__(C == 128 ? 256 : 512, C == 128 ? 2 : 1) void output
                 af[4 * c + k] = as_bf16x8(panel[panel_slot(rv, 2 * k + gv)]);
             }
         }
-        uint32_t out_off[4]; // NEAR_OUT: byte offsets of this lane's four rows of `out` (rows past the end: the last one)
-        if constexpr (EPILOGUE == EPILOGUE_RESIDUAL && NEAR_OUT) {
-            const uint32_t n32 = (uint32_t)swap_n, nb32 = n32 ? (uint32_t)M / n32 : 0u;
-            const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane(row0);
-            const uint32_t b0 = n32 ? first / n32 : 0u, s0 = first - b0 * n32; // row (b0, s0) of the [M / n, n] grid
-            const uint32_t last_rel = (uint32_t)(stop - 1 - rbase);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                uint32_t pr = 8u * i + ((uint32_t)lv >> 3);
-                pr = pr < last_rel ? pr : last_rel;
-                uint32_t target = first + pr;
-                if (n32) { // (b, s) -> (s, b); the 32 rows of a step wrap at most once (n >= 32)
-                    uint32_t sq = s0 + pr, bq = b0;
-                    if (sq >= n32) {
-                        sq -= n32, bq += 1;
-                    }
-                    target = __umul24(sq, nb32) + bq;
-                }
-                out_off[i] = __umul24(target, 2u * (uint32_t)out_ld) + 16u * ((uint32_t)lv & 7u);
-            }
-        }
         {
             // clamped to the last step instead of a branch: one harmless re-read at the end
             const int rnext = rbase + 32 < stop ? rel0 + 32 : rel0;
@@ -2306,20 +2274,14 @@ __global__ __launch_bounds__(C == 128 ? 256 : 512, C == 128 ? 2 : 1) void output
 #pragma unroll
         for (int half = 0; half < 2; ++half) { // 64 output features per panel
             uint4 gq[4], zq[4];
-            if constexpr (EPILOGUE != EPILOGUE_STORE) { // requested before the MFMAs, used after them
+            if constexpr (EPILOGUE == EPILOGUE_GATED_RESIDUAL) { // requested before the MFMAs, used after them
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     int64_t row = (int64_t)row0 + 8 * i + (lv >> 3);
                     row = row < stop ? row : stop - 1;
                     const int64_t col = n0 + half * 64 + (lv & 7) * 8;
-                    if constexpr (EPILOGUE == EPILOGUE_GATED_RESIDUAL) {
-                        gq[i] = *reinterpret_cast<const uint4 *>(gate + row * gate_ld + col);
-                    }
-                    if constexpr (EPILOGUE == EPILOGUE_RESIDUAL && NEAR_OUT) {
-                        zq[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(out + n0 + half * 64) + out_off[i]);
-                    } else {
-                        zq[i] = *reinterpret_cast<const uint4 *>(out + target_row(row) * out_ld + col);
-                    }
+                    gq[i] = *reinterpret_cast<const uint4 *>(gate + row * gate_ld + col);
+                    zq[i] = *reinterpret_cast<const uint4 *>(out + row * out_ld + col);
                 }
             }
             f32x16 acc[2];
@@ -2361,20 +2323,10 @@ __global__ __launch_bounds__(C == 128 ? 256 : 512, C == 128 ? 2 : 1) void output
                         res[e] = (bf16_t)(to_f32(z[e]) + upd);
                     }
                     v = as_uint4(res);
-                } else if constexpr (EPILOGUE == EPILOGUE_RESIDUAL) {
-                    const bf16x8 o = as_bf16x8(v), z = as_bf16x8(zq[i]);
-                    bf16x8 res;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        res[e] = (bf16_t)(to_f32(z[e]) + to_f32(o[e]));
-                    }
-                    v = as_uint4(res);
                 }
                 if (row < stop) {
-                    if constexpr (EPILOGUE == EPILOGUE_RESIDUAL && NEAR_OUT) {
-                        *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(out + n0 + half * 64) + out_off[i]) = v;
-                    } else if constexpr (EPILOGUE == EPILOGUE_RESIDUAL || !NEAR) {
-                        *reinterpret_cast<uint4 *>(out + target_row(row) * out_ld + n0 + half * 64 + (lv & 7) * 8) = v;
+                    if constexpr (!NEAR) {
+                        *reinterpret_cast<uint4 *>(out + row * out_ld + n0 + half * 64 + (lv & 7) * 8) = v;
                     } else {
                         char *out_w = reinterpret_cast<char *>(out + start * out_ld + n0 + half * 64);
                         *reinterpret_cast<uint4 *>(out_w + (__umul24((uint32_t)(rel0 + prow_), 2u * (uint32_t)out_ld) + 16u * (lv & 7))) = v;
@@ -2852,9 +2804,10 @@ int launch_output_projection(const void *a, int64_t a_ld, const void *w, const f
     }
     if constexpr (EPILOGUE != EPILOGUE_GATED_RESIDUAL) {
         const int64_t tiles = (M + 31) / 32, slabs = N / 128;
-        // not where the result lies over the rows: one workgroup's features would be written while another still reads them
+        // not where the result lies over the rows: one workgroup's features would be written while another still reads them (a residual is
+        // added to an activation, of which the rows are never part)
         const uintptr_t from = reinterpret_cast<uintptr_t>(a), to = reinterpret_cast<uintptr_t>(out);
-        const bool apart = from + (uintptr_t)(2 * ((M - 1) * a_ld + C)) <= to || to + (uintptr_t)(2 * ((M - 1) * out_ld + N)) <= from;
+        const bool apart = EPILOGUE == EPILOGUE_RESIDUAL || from + (uintptr_t)(2 * ((M - 1) * a_ld + C)) <= to || to + (uintptr_t)(2 * ((M - 1) * out_ld + N)) <= from;
         const int64_t cus = kutacc_cu_count();
         const auto launch = [&](auto kern, int features, int64_t per_cu) {
             const int64_t gx = std::min(tiles, std::max<int64_t>(per_cu * cus / (N / features), 1));
@@ -2874,24 +2827,22 @@ int launch_output_projection(const void *a, int64_t a_ld, const void *w, const f
             }
         }
     }
-    // the transposing residual epilogue finds its rows of `out` with 32-bit arithmetic where the tensor allows (without
-    // the transposition there is no division to save, and the 64-bit form measured 1 us faster at 384 x 384 rows)
-    const bool near_out = EPILOGUE == EPILOGUE_RESIDUAL && M < (1 << 24) && out_ld > 0 && out_ld < (1 << 22) &&
-                          M * out_ld * 2 < ((int64_t)1 << 31) && swap_n >= 32 && M % swap_n == 0;
-    auto kern = near_out ? output_projection_kernel<C, EPILOGUE, EPILOGUE == EPILOGUE_RESIDUAL> : output_projection_kernel<C, EPILOGUE, false>;
-    constexpr int SLABS = C / 128, WAVES = 4 * SLABS;
-    const size_t lds_bytes = (size_t)SLABS * 4 * (C / 16) * 64 * 16 + WAVES * 4096;
-    static size_t configured[2][KUTACC_DEVICE_SLOTS] = {}; // one table per kernel the pointer may hold
-    if (const int rc = opt_in_lds(kern, lds_bytes, configured[near_out ? 1 : 0])) {
-        return rc;
+    if constexpr (EPILOGUE != EPILOGUE_RESIDUAL) {
+        auto kern = output_projection_kernel<C, EPILOGUE>;
+        constexpr int SLABS = C / 128, WAVES = 4 * SLABS;
+        const size_t lds_bytes = (size_t)SLABS * 4 * (C / 16) * 64 * 16 + WAVES * 4096;
+        static size_t configured[KUTACC_DEVICE_SLOTS] = {};
+        if (const int rc = opt_in_lds(kern, lds_bytes, configured)) {
+            return rc;
+        }
+        int64_t gx, rpw;
+        output_projection_split(C, M, gx, rpw);
+        const int64_t gy = (N / 128 + SLABS - 1) / SLABS;
+        kern<<<dim3((unsigned)gx, (unsigned)gy), 64 * WAVES, lds_bytes, stream>>>(
+            (const bf16_t *)a, a_ld, (const bf16_t *)w, bias, (bf16_t *)out, out_ld, M, (int)N, (int)rpw, (const bf16_t *)gate, gate_ld);
+        return kutacc_hip_status(hipGetLastError());
     }
-    int64_t gx, rpw;
-    output_projection_split(C, M, gx, rpw);
-    const int64_t gy = (N / 128 + SLABS - 1) / SLABS;
-    kern<<<dim3((unsigned)gx, (unsigned)gy), 64 * WAVES, lds_bytes, stream>>>(
-        (const bf16_t *)a, a_ld, (const bf16_t *)w, bias, (bf16_t *)out, out_ld, M, (int)N, (int)rpw, (const bf16_t *)gate,
-        gate_ld, swap_n);
-    return kutacc_hip_status(hipGetLastError());
+    return KUTACC_HIP_EUNSUPPORTED; // (more rows than a device holds)
 }
 
 } // namespace
