@@ -16,7 +16,7 @@
 // maximum, pair bias from a fragment-major copy made by pair_bias_fragments_kernel, row sums on the
 // matrix core); attend_block and attend_block_direct are the general ones (running maximum with lazy
 // rescale, pair bias read in place) for calls whose pair bias cannot be copied.
-// A third kernel, output_projection_kernel, is the final GEMM with fp32 bias (reference :152-157).
+// The final GEMM with fp32 bias (reference :152-157) is output_projection_tile_kernel, or output_projection_kernel.
 //
 // All contractions are v_mfma_f32_32x32x16_bf16 (fp32 accumulate); fragment and accumulator layouts
 // are described in mfma_tiles.h.  Two consequences of those layouts are used everywhere below:
