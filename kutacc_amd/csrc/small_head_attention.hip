@@ -516,21 +516,36 @@ int64_t stash_capacity(const kutacc_hip_attention_args_t &a)
 
 // The projections inside: no pass that writes and reads four activations (1024 rows of 301 215 -> 181-191 us, of 107 3576 rows 199 -> 175, 5120 of
 // 128 353 -> 281, 64 of 60 20.4 -> 12.8, whole operator), where the inputs are what projections_kernel takes, the scratch tensors are dense and hold
-// the queries and gates (not where padding makes three times as much of the rows), and no other workgroup
-// reads what one of them writes.  KUTACC_HIP_PATH_TILED asks for q, k, v and gate as the reference leaves them.
+// the queries and gates (not where padding makes three times as much of the rows), and no workgroup writes what another one reads:
+// neither the average nor the queries and gates, which lie in the scratch tensors in an order of their own, over the operands of the
+// projections or over each other.  The kernel that reads q, k, v and gate takes those: it reads a position's queries and gates before it
+// writes the position's average.  KUTACC_HIP_PATH_TILED asks for q, k, v and gate as the reference leaves them.
 bool small_head_attention_projects(const kutacc_hip_attention_args_t &a)
 {
     const int64_t C = a.nheads * D, M = a.batch * a.seq_len;
-    const auto apart = [&](const void *from, int64_t bytes) { // of the average, which other workgroups write while these operands are read
-        const uintptr_t at = reinterpret_cast<uintptr_t>(from), avg = reinterpret_cast<uintptr_t>(a.avg);
-        return at + (uintptr_t)bytes <= avg || avg + (uintptr_t)(((M - 1) * a.avg_stride_s + C) * 2) <= at;
+    if (a.path == KUTACC_HIP_PATH_TILED || C != PROJECTED || a.q_stride_s != C || a.k_stride_s != C || a.gate_stride_s != C ||
+        3 * stash_capacity(a) < (a.batch + ROWS - 1) / ROWS * a.nheads || !small_head_attention_supports(a) || a.input_ld % 8 != 0 || a.input_ld >= (1 << 30) ||
+        a.seq_len * a.input_ld >= (1 << 30) || !kutacc_hip_aligned16(a.input) || !kutacc_hip_aligned16(a.query_w) || !kutacc_hip_aligned16(a.key_w) ||
+        !kutacc_hip_aligned16(a.value_w) || !kutacc_hip_aligned16(a.gating_w)) {
+        return false;
+    }
+    struct Range {
+        const void *from;
+        int64_t bytes;
     };
-    return a.path != KUTACC_HIP_PATH_TILED && C == PROJECTED && a.q_stride_s == C && a.k_stride_s == C && a.gate_stride_s == C &&
-           3 * stash_capacity(a) >= (a.batch + ROWS - 1) / ROWS * a.nheads && small_head_attention_supports(a) && a.input_ld % 8 == 0 && a.input_ld < (1 << 30) &&
-           a.seq_len * a.input_ld < (1 << 30) && kutacc_hip_aligned16(a.input) && kutacc_hip_aligned16(a.query_w) && kutacc_hip_aligned16(a.key_w) &&
-           kutacc_hip_aligned16(a.value_w) && kutacc_hip_aligned16(a.gating_w) && apart(a.input, ((M - 1) * a.input_ld + C) * 2) &&
-           apart(a.query_w, 2 * C * C) && apart(a.key_w, 2 * C * C) && apart(a.value_w, 2 * C * C) && apart(a.gating_w, 2 * C * C) &&
-           apart(a.gating_b, 4 * C);
+    const auto apart = [](const Range &x, const Range &y) {
+        const uintptr_t at = reinterpret_cast<uintptr_t>(x.from), other = reinterpret_cast<uintptr_t>(y.from);
+        return at + (uintptr_t)x.bytes <= other || other + (uintptr_t)y.bytes <= at;
+    };
+    const Range avg = {a.avg, ((M - 1) * a.avg_stride_s + C) * 2}, stash[3] = {{a.q, M * C * 2}, {a.k, M * C * 2}, {a.gate, M * C * 2}};
+    const Range read[] = {{a.input, ((M - 1) * a.input_ld + C) * 2}, {a.query_w, 2 * C * C}, {a.key_w, 2 * C * C}, {a.value_w, 2 * C * C},
+                          {a.gating_w, 2 * C * C}, {a.gating_b, 4 * C}};
+    for (const Range &operand : read) {
+        if (!apart(operand, avg) || !apart(operand, stash[0]) || !apart(operand, stash[1]) || !apart(operand, stash[2])) {
+            return false;
+        }
+    }
+    return apart(avg, stash[0]) && apart(avg, stash[1]) && apart(avg, stash[2]);
 }
 
 int small_head_attention(const kutacc_hip_attention_args_t &a, bool projects, hipStream_t stream)

@@ -173,10 +173,12 @@ def test_heads_of_eight_stage_their_keys_in_units_of_64(torch_cuda, B, S):
 
 # sets of four rows, whole and with one to three; one tile and several, ragged and not, a wave with one tile, two and three, eight waves; rows and averages
 # with a pitch.  projects: whether the kernel forms the projections itself: no where the scratch does not hold its queries and gates (5 rows of
-# 64, rows of 40), is not dense, or the average lies where the input does
+# 64, rows of 40), is not dense, or the average or the input lies where the other of the two or a scratch tensor does
 @pytest.mark.parametrize("B,S,form,projects", [(8, 64, "", True), (65, 48, "", True), (12, 97, "", True), (11, 128, "", True), (33, 150, "", True), (8, 301, "", True),
                                                (12, 385, "", True), (10, 77, "pitch", True), (5, 64, "", False), (40, 40, "", False), (10, 77, "q", False), (10, 77, "k", False),
-                                               (10, 77, "in place", False)])
+                                               (10, 77, "in place", False), (65, 96, "avg over q", False), (65, 96, "avg over k", False),
+                                               (65, 96, "avg over gate", False), (65, 96, "input over q", False), (65, 96, "input over k", False),
+                                               (65, 96, "input over gate", False)])
 @pytest.mark.parametrize("pair_bias", [True, False])
 def test_heads_of_eight_with_the_projections_inside(torch_cuda, B, S, form, projects, pair_bias):
     """The kernel that projects against the one that reads q, k, v and gate: the same roundings, sums of products in another order."""
@@ -198,6 +200,10 @@ def test_heads_of_eight_with_the_projections_inside(torch_cuda, B, S, form, proj
             setattr(a, form, wide.data_ptr()), setattr(a, form + "_stride_b", 72 * S), setattr(a, form + "_stride_s", 72)
         elif form == "in place":
             a.avg, avg = ten["x"].data_ptr(), ten["x"]
+        elif form.startswith("avg over"):
+            a.avg, avg = getattr(a, form.split()[2]), scratch[form.split()[2]].view(B, S, 64)
+        elif form.startswith("input over"):
+            setattr(a, form.split()[2], ten["x"].data_ptr())
         print(f"{w.name} {form} path={path}", flush=True)
         names = helpers.profiled_kernels(torch, lambda: capi.lib().kutacc_hip_gating_attention(ctypes.byref(a), None))  # noqa: B023
         torch.cuda.synchronize()
