@@ -73,7 +73,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     const int S = p.S, NT = p.NT, H = p.H, d = p.d;
     // Workgroup ids are dealt round robin over the 8 XCDs: the parts of a row are eight ids apart, so that its tiles come from one L2.
     int b = (int)blockIdx.x, turn = 0, own = NT;
-    if (b >= p.whole) {
+    if (NW == 8 && b >= p.whole) { // (rows of four waves are never shared)
         const int idx = b - p.whole, part = (idx >> 3) % p.parts;
         b = p.whole + (idx >> 3) / p.parts * 8 + (idx & 7);
         if (b >= p.B) {
@@ -84,6 +84,20 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     // A part takes the row's tiles in an order that begins with those it puts out, so that these are the ones it keeps.
     auto place = [&](int t) { return t + turn < NT ? t + turn : t + turn - NT; };
     const int spad = NT * 32;
+    // STREAM: ten tiles leave no registers beside them for constants and weights, which are read per tile, and tiles are kept from one another
+    // (rows that are kept whole have them, and lose by it: 300 tokens x 100 rows 11.3 -> 11.8 us, 512 x 300 19.5 -> 20.3, 1024 x 384 33.6 -> 34.2).
+    auto per_tile_lane = [&] {
+        int l = lane;
+        if constexpr (STREAM) {
+            asm volatile("" : "+v"(l)); // opaque: what is addressed with it stays where it is read
+        }
+        return l;
+    };
+    auto fence = [] {
+        if constexpr (STREAM) {
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
 
     uint4 *qk_frag = lds;            // [4 k-steps][64 lanes]
     uint4 *wv_frag = qk_frag + 256;  // [4][64]
@@ -99,7 +113,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     float *qv = qavg + GC;                                  // [64] q, bf16-rounded
     float *wavg = qv + GC;                                  // [64]
     float *bos = wavg + GC;                                 // [64] output bias
-    float *bgs = bos + GC;                                  // [64] gate bias
+    float *bgs = bos + GC;                                  // [64] gate bias (eight waves)
     float *merge = reinterpret_cast<float *>(panels);       // [NW waves][64 lanes][MERGE_LD]
 
     const bf16_t *xb = p.x + (int64_t)b * p.x_sb;
@@ -179,7 +193,10 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         mask16[s] = s < S ? p.mask[(int64_t)b * p.mask_sb + s] : (bf16_t)-INFINITY;
     }
     if (tid < GC) {
-        bos[tid] = p.bo[tid], bgs[tid] = p.bg[tid];
+        bos[tid] = p.bo[tid];
+        if constexpr (NW == 8) {
+            bgs[tid] = p.bg[tid];
+        }
     }
     __syncthreads();
 
@@ -223,7 +240,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
                 xs[i][ks] = as_bf16x8(panel[panel_slot(r, 2 * ks + g)]);
             }
             add_tile(t, xs[i]);
-            __builtin_amdgcn_sched_barrier(0);
+            fence();
         }
         if constexpr (STREAM) {
             int slot = 0;
@@ -323,9 +340,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         f32x16 o = zero16();
         float m_run = -1e30f, lsum = 0.f;
         auto attend = [&](int t, const bf16x8 (&xf)[4]) {
-            int lane = tid & 63; // opaque, here and in put_out: constants and weights are read per tile, not kept beside the row
-            asm volatile("" : "+v"(lane));
-            const int g = lane >> 5;
+            const int lane = per_tile_lane(), g = lane >> 5;
             f32x16 x1, vv = zero16();
             const bf16x4 *mb4 = reinterpret_cast<const bf16x4 *>(mask16 + place(t) * 32 + 4 * g);
 #pragma unroll
@@ -364,7 +379,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
             }
             o = mfma(pack8(vv, 0), p0, o);
             o = mfma(pack8(vv, 8), p1, o);
-            __builtin_amdgcn_sched_barrier(0);
+            fence();
         };
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
@@ -428,18 +443,34 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
 
     // ---- phase C: gate, gating, output projection ----
     {
+        // per-channel constants of the gating, in the order the accumulators hold them
+        constexpr int KEPT = STREAM ? 1 : 32;
+        float bgv[KEPT], wv_[KEPT];
+        if constexpr (!STREAM) {
+#pragma unroll
+            for (int i = 0; i < 32; ++i) {
+                const int ch = gate_channel(i >> 4, i & 15, g);
+                bgv[i] = NW == 8 ? bgs[ch] : p.bg[ch], wv_[i] = wavg[ch];
+            }
+        }
         auto put_out = [&](int t, const bf16x8 (&xf)[4]) {
-            int lane = tid & 63;
-            asm volatile("" : "+v"(lane));
-            const int r = lane & 31, g = lane >> 5;
+            const int lane = per_tile_lane(), r = lane & 31, g = lane >> 5;
+            auto four = [&](const float *at, const float (&kept)[KEPT], int rb, int a) { // constants 4 a .. 4 a + 3 of row block rb
+                f32x4 v;
+                if constexpr (STREAM) { // gate_channel(rb, 4 a, g) and the three behind it
+                    v = *reinterpret_cast<const f32x4 *>(at + 32 * rb + 8 * g + 16 * (a >> 1) + 4 * (a & 1));
+                } else {
+                    v = f32x4{kept[16 * rb + 4 * a], kept[16 * rb + 4 * a + 1], kept[16 * rb + 4 * a + 2], kept[16 * rb + 4 * a + 3]};
+                }
+                return v;
+            };
             bf16x8 gf[4];
 #pragma unroll
             for (int rb = 0; rb < 2; ++rb) {
-                // the lane's channels of the row block, gate_channel(rb, v, g): 32 rb + 8 g + 16 (v / 8) + v % 8
                 f32x16 ga;
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
-                    const f32x4 bv = *reinterpret_cast<const f32x4 *>(bgs + 32 * rb + 8 * g + 16 * (a >> 1) + 4 * (a & 1));
+                    const f32x4 bv = four(bgs, bgv, rb, a);
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
                         ga[4 * a + c] = bv[c];
@@ -451,7 +482,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
                 }
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
-                    const f32x4 wv = *reinterpret_cast<const f32x4 *>(wavg + 32 * rb + 8 * g + 16 * (a >> 1) + 4 * (a & 1));
+                    const f32x4 wv = four(wavg, wv_, rb, a);
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
                         ga[4 * a + c] = wv[c] * sigmoid_fast(ga[4 * a + c]);
@@ -483,7 +514,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
                     dst[1] = as_uint4(pack8(oa, 8));
                 }
             }
-            __builtin_amdgcn_sched_barrier(0);
+            fence();
         };
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
