@@ -72,17 +72,21 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     const int r = lane & 31, g = lane >> 5;
     const int S = p.S, NT = p.NT, H = p.H, d = p.d;
     // Workgroup ids are dealt round robin over the 8 XCDs: the parts of a row are eight ids apart, so that its tiles come from one L2.
-    int b = (int)blockIdx.x, turn = 0, own = NT;
+    int b = (int)blockIdx.x, put_from = 0, put_to = NT; // the tiles it puts out
     if (NW == 8 && b >= p.whole) { // (rows of four waves are never shared)
         const int idx = b - p.whole, part = (idx >> 3) % p.parts;
         b = p.whole + (idx >> 3) / p.parts * 8 + (idx & 7);
         if (b >= p.B) {
             return;
         }
-        turn = NT * part / p.parts, own = NT * (part + 1) / p.parts - turn;
+        put_from = NT * part / p.parts, put_to = NT * (part + 1) / p.parts;
     }
-    // A part takes the row's tiles in an order that begins with those it puts out, so that these are the ones it keeps.
-    auto place = [&](int t) { return t + turn < NT ? t + turn : t + turn - NT; };
+    // A wave's tiles are wave + NW * i.  All workgroups of a row take them in the same order, so that they have the same sums, and find in one L2
+    // what another has just read; a part keeps those from the first one on that it puts out (or the last KEEP).  Beginning with its own tiles, each
+    // part had sums of its own: tokens of a row differed by a bf16 unit of the average, 5120 x 60 took 52.5 us and takes 45.0, 4000 x 300 115.5 and 117.5.
+    const int count = (NT - wave + NW - 1) / NW;
+    const int kept_from = STREAM ? max(0, min((put_from - wave + NW - 1) / NW, count - KEEP)) : 0;
+    auto kept_tile = [&](int i) { return wave + NW * (kept_from + i); };
     const int spad = NT * 32;
     // STREAM: ten tiles leave no registers beside them for constants and weights, which are read per tile, and tiles are kept from one another
     // (rows that are kept whole have them, and lose by it: 300 tokens x 100 rows 11.3 -> 11.8 us, 512 x 300 19.5 -> 20.3, 1024 x 384 33.6 -> 34.2).
@@ -122,47 +126,64 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
     // Requested before anything else, so that their latency passes under the staging of the weights: the first tiles of
     // the row (all of a wave's tiles when they are kept in registers and there are at most four) and this thread's slice
     // of the query weights (output o = tid / TPR, channels part * 64 / TPR ...).
-    constexpr int PRE = KEEP > 8 ? 2 : 4; // beside eight tiles and less there are registers for four
+    constexpr int PRE = STREAM ? 1 : 4; // beside ten tiles there are no registers for more
     PanelRegs ahead[PRE];
 #pragma unroll
     for (int i = 0; i < PRE; ++i) {
-        const int t = wave + NW * i;
-        ahead[i] = panel_load_near(xb, x_pitch, place(t < NT ? t : NT - 1) * 32, S - 1, 0, lane);
+        const int t = kept_tile(i);
+        ahead[i] = panel_load_near(xb, x_pitch, (t < NT ? t : NT - 1) * 32, S - 1, 0, lane);
     }
-    const int first = wave + NW * KEEP; // first of the wave's tiles that are not kept
+    // The tiles that are not kept: the n-th of them.  In phases A and B they come through the ring around the kept ones, in phase C behind them.
+    const int streamed = max(0, count - KEEP);
+    auto streamed_tile = [&](int n) { return wave + NW * (n < kept_from ? n : n + KEEP); };
     const uint32_t ring_lds = (uint32_t)(uintptr_t)(const lds_char *)ring;
-    auto ask = [&](int slot, int t) { // tile t into a slot of the ring, in the panel's layout
-        const int at = place(t);
+    auto ask = [&](int n) { // the n-th streamed tile into its slot of the ring, in the panel's layout
+        const int at = streamed_tile(n), slot = n & 1;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int rl = lane >> 3, row = min(at * 32 + 8 * i + rl, S - 1);
             load_to_lds(ring_lds + slot * 4096u + i * 1024u, xb, __umul24((uint32_t)row, 2u * x_pitch) + 16u * (uint32_t)((lane & 7) ^ rl ^ (i >> 1)));
         }
     };
-    auto stream_start = [&](int end) { // of the tiles up to `end`
-        if (STREAM && first < end) {
-            ask(0, first);
-            if (first + NW < end) {
-                ask(1, first + NW);
+    auto stream_start = [&](int from, int end) {
+        if (STREAM && from < end) {
+            ask(from);
+            if (from + 1 < end) {
+                ask(from + 1);
             }
         }
     };
     struct Tile {
         bf16x8 f[4];
     };
-    auto ring_tile = [&](int slot, int t, int end) { // out of the ring, and the tile after the next one asked for in its place
+    auto ring_tile = [&](int n, int end) { // out of the ring, and the tile after the next one asked for in its place
+        const int slot = n & 1;
         Tile x;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             x.f[ks] = as_bf16x8(ring[slot * 256 + panel_slot(r, 2 * ks + g)]);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (t + 2 * NW < end) {
-            ask(slot, t + 2 * NW);
+        if (n + 2 < end) {
+            ask(n + 2);
         }
         return x;
     };
-    stream_start(NT);
+    // ... of which those up to this one are put out, from kept_from on: a part that has more than the kept tiles keeps its first ones
+    const int put_streamed = max(0, (put_to - wave + NW - 1) / NW - KEEP);
+    stream_start(0, streamed);
+    auto walk = [&](int from, int to, auto f) __attribute__((always_inline)) { // f(t, fragments) of streamed tiles, all of which are asked for in turn
+#pragma unroll 1
+        for (int n = from; n < to; ++n) {
+            if (n + 1 < streamed) {
+                wait_for_loads<4>(); // all but the next tile's
+            } else {
+                wait_for_loads<0>();
+            }
+            const Tile x = ring_tile(n, streamed);
+            f(streamed_tile(n), x.f);
+        }
+    };
     constexpr int TPR = NTHR / GC, WQV = GC / TPR / 8; // threads per output of q, 16-byte pieces per thread
     uint4 wq_part[WQV];
 #pragma unroll
@@ -212,7 +233,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         }
         float msum = 0.f;
         auto add_tile = [&](int t, const bf16x8 (&xf)[4]) {
-            float m = to_f32(mask16[place(t) * 32 + r]);
+            float m = to_f32(mask16[t * 32 + r]);
             m = m == -INFINITY ? 0.f : m;
             msum += g == 0 ? m : 0.f;
 #pragma unroll
@@ -223,17 +244,20 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
                 }
             }
         };
+        if constexpr (STREAM) {
+            walk(0, kept_from, add_tile);
+        }
         // the loads of the next PRE tiles are in flight while this one is summed
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
-            const int t = wave + NW * i;
+            const int t = kept_tile(i);
             if (t >= NT) {
                 break;
             }
             panel_store(panel, lane, ahead[i % PRE]);
             if (i + PRE < KEEP) {
                 const int tn = t + NW * PRE;
-                ahead[i % PRE] = panel_load_near(xb, x_pitch, place(tn < NT ? tn : NT - 1) * 32, S - 1, 0, lane);
+                ahead[i % PRE] = panel_load_near(xb, x_pitch, (tn < NT ? tn : NT - 1) * 32, S - 1, 0, lane);
             }
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
@@ -243,17 +267,8 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
             fence();
         }
         if constexpr (STREAM) {
-            int slot = 0;
-            for (int t = first; t < NT; t += NW, slot ^= 1) {
-                if (t + NW < NT) {
-                    wait_for_loads<4>(); // all but the next tile's
-                } else {
-                    wait_for_loads<0>();
-                }
-                const Tile x = ring_tile(slot, t, NT);
-                add_tile(t, x.f);
-            }
-            stream_start(NT);
+            walk(kept_from, streamed, add_tile);
+            stream_start(0, streamed);
         }
         // sum over the 32 lanes of each half (they hold different tokens of the same channels)
         msum = group_sum<32>(msum);
@@ -287,7 +302,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         }
         const bf16_t qa = (bf16_t)(tot * (1.0f / (ms + 1e-10f))); // reference :66-74
         qavg[tid] = to_f32(qa);
-        if (p.q_avg != nullptr && turn == 0) {
+        if (p.q_avg != nullptr && put_from == 0) {
             p.q_avg[(int64_t)b * p.qavg_sb + tid] = qa;
         }
     }
@@ -342,7 +357,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         auto attend = [&](int t, const bf16x8 (&xf)[4]) {
             const int lane = per_tile_lane(), g = lane >> 5;
             f32x16 x1, vv = zero16();
-            const bf16x4 *mb4 = reinterpret_cast<const bf16x4 *>(mask16 + place(t) * 32 + 4 * g);
+            const bf16x4 *mb4 = reinterpret_cast<const bf16x4 *>(mask16 + t * 32 + 4 * g);
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
                 const bf16x4 mv = mb4[2 * a];
@@ -381,25 +396,19 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
             o = mfma(pack8(vv, 8), p1, o);
             fence();
         };
+        if constexpr (STREAM) {
+            walk(0, kept_from, attend);
+        }
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
-            if (wave + NW * i >= NT) {
+            if (kept_tile(i) >= NT) {
                 break;
             }
-            attend(wave + NW * i, xs[i]);
+            attend(kept_tile(i), xs[i]);
         }
         if constexpr (STREAM) {
-            int slot = 0;
-            for (int t = first; t < NT; t += NW, slot ^= 1) {
-                if (t + NW < NT) {
-                    wait_for_loads<4>();
-                } else {
-                    wait_for_loads<0>();
-                }
-                const Tile x = ring_tile(slot, t, NT);
-                attend(t, x.f);
-            }
-            stream_start(own);
+            walk(kept_from, streamed, attend);
+            stream_start(kept_from, put_streamed);
         }
         float *mine = merge + (wave * 64 + lane) * MERGE_LD;
         mine[0] = m_run;
@@ -491,7 +500,7 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
                 gf[2 * rb] = pack8(ga, 0);
                 gf[2 * rb + 1] = pack8(ga, 8);
             }
-            const int s = place(t) * 32 + r;
+            const int s = t * 32 + r;
 #pragma unroll
             for (int ob = 0; ob < 2; ++ob) {
                 f32x16 oa;
@@ -518,19 +527,20 @@ __global__ __launch_bounds__(64 * NW, 2) void global_attention_kernel(GlobalPara
         };
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
-            if (wave + NW * i >= own) {
+            if (kept_tile(i) >= put_to) {
                 break;
             }
-            put_out(wave + NW * i, xs[i]);
+            if (NW == 4 || kept_tile(i) >= put_from) {
+                put_out(kept_tile(i), xs[i]);
+            }
         }
         if constexpr (STREAM) {
-            int slot = 0;
-            for (int t = first; t < own; t += NW, slot ^= 1) {
+            for (int n = kept_from; n < put_streamed; ++n) {
                 // younger than the tile's loads are the stores of the two tiles before it, four each (of kept ones, for the
                 // first two tiles)
                 wait_for_loads<8>();
-                const Tile x = ring_tile(slot, t, own);
-                put_out(t, x.f);
+                const Tile x = ring_tile(n, put_streamed);
+                put_out(streamed_tile(n), x.f);
             }
         }
     }
@@ -606,9 +616,9 @@ int global_attention(const kutacc_hip_global_attention_args_t &a, hipStream_t st
     kutacc_prof::KernelTimer t("global_attention_kernel", BS * (4.0 * GC * a.head_size + 4.0 * GC * GC + 4.0 * GC), stream);
     const bool eight_waves = p.NT > 32 || (p.NT >= 16 && a.batch <= kutacc_cu_count());
     // Rows of eight waves that would leave half of the CUs or more without one are shared by up to eight workgroups each: all form the
-    // mean and the average, from one L2, and a part of the result (us, one workgroup a row against this: 5120 positions x 384 rows 186.5 -> 183.5,
-    // x 128 82 -> 77.7, x 60 66.5 -> 52.3; 4000 x 300 144 -> 126, 2500 x 100 36.7 -> 31.8, 1024 x 128 21.1 -> 18.9, x 60 19.4 -> 15.8, 700 x 100 17.1
-    // -> 14.7).  Two rows of four waves a CU gain nothing (400 x 200 16.4 -> 17.3).  Not where the result lies over the input: one
+    // mean and the average, the same bits in each, from one L2, and a part of the result (us, one workgroup a row with 64 tiles kept against this: 5120
+    // positions x 384 rows 184 -> 173, x 128 69.1 -> 58.4, x 60 66.0 -> 45.0; 4000 x 300 136 -> 117, 2500 x 100 38.1 -> 30.1, 1024 x 128 19.4 -> 17.3,
+    // x 60 18.5 -> 14.6, 700 x 100 15.7 -> 14.2).  Two rows of four waves a CU gain nothing (400 x 200 16.4 -> 17.3).  Not where the result lies over the input: one
     // workgroup would put out what another still reads.
     const int64_t room = kutacc_cu_count(), rest = eight_waves ? a.batch % room : 0;
     const uintptr_t in = reinterpret_cast<uintptr_t>(a.q_data), out = reinterpret_cast<uintptr_t>(a.out);

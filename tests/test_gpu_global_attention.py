@@ -156,6 +156,23 @@ def test_global_attention_in_place_keeps_a_workgroup_per_row(torch_cuda):
     helpers.check_close(helpers.to_numpy(again), helpers.to_numpy(out), "bf16", "global attention in place")
 
 
+@pytest.mark.parametrize("rows,S", [(0.5, 1024), (0.5, 1057), (0.5, 5121), (0.3, 2600), (0.2, 700), (7, 2600), (1.25, 1100), (1.004, 1056)])
+def test_global_attention_rows_shared_by_workgroups_keep_their_bits(torch_cuda, rows, S):
+    """Rows of the same values, some of them shared by two to eight workgroups, have the same bits, and the bits of rows with a workgroup each
+    (the result over the input): every workgroup of a row forms the same mean and the same average."""
+    torch = torch_cuda
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    B = rows if isinstance(rows, int) else int(rows * cus)
+    ten, out, avg = device_case(torch, B, S, 8, 8)
+    ten["x"], ten["mask"] = ten["x"][:1].expand(B, -1, -1).contiguous(), ten["mask"][:1].expand(B, -1, -1).contiguous()
+    run_device_case(torch, ten, out, avg, 8)
+    alone, alone_avg = ten["x"].clone(), torch.empty_like(avg)
+    run_device_case(torch, dict(ten, x=alone), alone, alone_avg, 8)
+    for got, one in ((out, alone), (avg, alone_avg)):
+        assert helpers.same_bits(one, one[:1].expand_as(one).contiguous())
+        assert helpers.same_bits(got, one)
+
+
 def test_global_attention_replays_from_a_hip_graph(torch_cuda):
     """Rows past the kept tiles, whose rest comes through the ring in the LDS: captured on a side stream and replayed three times, with
     eager work (the results overwritten) between the replays; every replay gives the eager result bit for bit."""
