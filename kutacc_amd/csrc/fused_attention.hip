@@ -916,14 +916,14 @@ __device__ inline void stage_weight_lines(uint4 *lds_w, const FusedParams &p, in
 // and keeps them in registers until then.  At 1024 keys that leaves room for all four weight matrices of a
 // 128-channel head (two of a 256-channel one) beside K and V, so the input rows are read once (twice).
 // ------------------------------------------------------------------------------------------------
-template <int C, int BPW, bool HAS_NB, bool TILES>
+template <int C, int BPW, bool HAS_NB, bool TILES, bool ODD>
 __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(FusedParams p)
 {
     constexpr int CK = C / 16;
     constexpr bool V_ALIAS = C == 256 && BPW == 4; // second LDS layout, below
     constexpr bool ONE_GROUP = V_ALIAS || C == 128; // all four weight matrices staged at once, always (see make_plan)
     constexpr bool ONE_PASS = C == 128 && BPW > 1;  // rows of one mask attended once: see below
-    const bool l2mode = TILES || p.l2mode != 0;
+    const bool l2mode = TILES || ODD || p.l2mode != 0;
     extern __shared__ uint4 lds[];
 
     // XCD-aware unit mapping: consecutive workgroup ids land on different XCDs (8 of them), so the H
@@ -1265,14 +1265,11 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
             const uint4 *nbf = HAS_NB ? p.nbf + ((int64_t)(h * NB + j) * NT * (TILES ? 4 : 2)) * 64 + lane : nullptr;
             bool again = true; // some probability overflowed or a whole row underflowed
             if (!ONE_PASS || flags != ONE_MASK) {
-                if (flags == 0u) {
+                if (!ODD && flags == 0u) { // (the tile of zeros behind an odd number has a mask)
                     attend_block_l2<HAS_NB, false, false, TILES>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel,
                                                           NT, lane, 0.f, o, l, (wave >> 2) & 1);
-                } else if (NB < NT) { // (always here with an odd number of tiles: the one of zeros has a mask)
-                    attend_block_l2<HAS_NB, true, false, TILES, true>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1),
-                                                         sumsel, NT, lane, 0.f, o, l, (wave >> 2) & 1);
                 } else {
-                    attend_block_l2<HAS_NB, true, false, TILES>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel,
+                    attend_block_l2<HAS_NB, true, false, TILES, ODD>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel,
                                                          NT, lane, 0.f, o, l, (wave >> 2) & 1);
                 }
                 __builtin_amdgcn_s_setprio(0);
@@ -1319,7 +1316,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
 // on the next row's loads and projections while the slower waves of its SIMD still attend, so the
 // latency- and MFMA-bound projection phase overlaps the VALU-heavy attention phase.
 // ------------------------------------------------------------------------------------------------
-template <int C, bool HAS_NB, bool L2MODE, bool FUSED_LN, bool TILES>
+template <int C, bool HAS_NB, bool L2MODE, bool FUSED_LN, bool TILES, bool ODD>
 __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_head_kernel(FusedParams p)
 {
     constexpr int CK = C / 16;
@@ -1566,14 +1563,11 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_head_kernel(F
         const bf16_t *nb_head = HAS_NB ? p.nb + (int64_t)h * p.nb_sh : nullptr;
         if constexpr (L2MODE) {
             const uint4 *nbf = HAS_NB ? p.nbf + ((int64_t)(h * NB + j) * NT * (TILES ? 4 : 2)) * 64 + lane : nullptr;
-            if (flags == 0u) {
+            if (!ODD && flags == 0u) { // (the tile of zeros behind an odd number has a mask)
                 attend_block_l2<HAS_NB, false, false, TILES>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
                                                       l, -1, fair_turn);
-            } else if (NB < NT) { // (always here with an odd number of tiles: the one of zeros has a mask)
-                attend_block_l2<HAS_NB, true, false, TILES, true>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
-                                                     l, -1, fair_turn);
             } else {
-                attend_block_l2<HAS_NB, true, false, TILES>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
+                attend_block_l2<HAS_NB, true, false, TILES, ODD>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
                                                      l, -1, fair_turn);
             }
             // some probability overflowed or a whole row underflowed: shift by the row's one mask, if it has one, or by the true row maxima
@@ -2696,30 +2690,35 @@ int opt_in_lds(K kern, size_t bytes, size_t *table)
     return (int)kutacc_opt_in_lds(reinterpret_cast<const void *>(kern), bytes, table);
 }
 
-template <int C, int BPW, bool HAS_NB, bool TILES = false>
-int launch_head_kernel(const FusedParams &p, const Plan &pl, hipStream_t stream)
+template <typename K>
+int launch_rows_kernel(K kern, size_t *configured, int64_t workgroups, const FusedParams &p, const Plan &pl, hipStream_t stream)
 {
-    auto kern = fused_head_kernel<C, BPW, HAS_NB, TILES>;
-    static size_t configured[KUTACC_DEVICE_SLOTS] = {}; // per instantiation and device: dynamic LDS opted into so far
     if (const int rc = opt_in_lds(kern, pl.lds_bytes, configured)) {
         return rc;
     }
-    const int64_t units = ((int64_t)(p.B + 7) / 8) * 8 * p.H;
-    kern<<<dim3((unsigned)units), dim3((unsigned)(pl.NW * 64)), pl.lds_bytes, stream>>>(p);
+    kern<<<dim3((unsigned)workgroups), dim3((unsigned)(pl.NW * 64)), pl.lds_bytes, stream>>>(p);
     return kutacc_hip_status(hipGetLastError());
+}
+
+// The kernels of an odd number of key tiles have the loop that leaves out the tile of zeros, and no other without a shift: beside the
+// loops of even numbers it spilled registers that each pair of tiles then fetched back (eleven in the persistent kernel of 128 channels with fp32 tiles).
+template <int C, int BPW, bool HAS_NB, bool TILES = false>
+int launch_head_kernel(const FusedParams &p, const Plan &pl, hipStream_t stream)
+{
+    static size_t configured[2][KUTACC_DEVICE_SLOTS] = {}; // per instantiation and device: dynamic LDS opted into so far
+    const int64_t units = ((int64_t)(p.B + 7) / 8) * 8 * p.H;
+    return p.NB < p.NT && (TILES || p.l2mode) ? launch_rows_kernel(fused_head_kernel<C, BPW, HAS_NB, TILES, true>, configured[1], units, p, pl, stream)
+                                              : launch_rows_kernel(fused_head_kernel<C, BPW, HAS_NB, TILES, false>, configured[0], units, p, pl, stream);
 }
 
 template <int C, bool HAS_NB, bool L2MODE, bool FUSED_LN = false, bool TILES = false>
 int launch_persistent_kernel(FusedParams p, const Plan &pl, hipStream_t stream)
 {
-    auto kern = persistent_head_kernel<C, HAS_NB, L2MODE, FUSED_LN, TILES>;
-    static size_t configured[KUTACC_DEVICE_SLOTS] = {};
-    if (const int rc = opt_in_lds(kern, pl.lds_bytes, configured)) {
-        return rc;
-    }
+    static size_t configured[2][KUTACC_DEVICE_SLOTS] = {};
     p.ngrp = persistent_groups(p.B, p.H);
-    kern<<<dim3((unsigned)(8 * p.H * p.ngrp)), dim3((unsigned)(pl.NW * 64)), pl.lds_bytes, stream>>>(p);
-    return kutacc_hip_status(hipGetLastError());
+    const int64_t workgroups = 8 * (int64_t)p.H * p.ngrp;
+    return p.NB < p.NT && L2MODE ? launch_rows_kernel(persistent_head_kernel<C, HAS_NB, L2MODE, FUSED_LN, TILES, L2MODE>, configured[1], workgroups, p, pl, stream)
+                                 : launch_rows_kernel(persistent_head_kernel<C, HAS_NB, L2MODE, FUSED_LN, TILES, false>, configured[0], workgroups, p, pl, stream);
 }
 
 template <int C, bool HAS_NB>
