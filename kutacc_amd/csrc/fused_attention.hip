@@ -2801,6 +2801,7 @@ int launch_output_projection(const void *a, int64_t a_ld, const void *w, const f
     if (!output_projection_rows_fit(C, M, a_ld, out_ld)) {
         return KUTACC_HIP_EUNSUPPORTED; // the callers' support checks ask the same question first
     }
+    const double flops = 2.0 * (double)M * (double)N * C;
     if constexpr (EPILOGUE != EPILOGUE_GATED_RESIDUAL) {
         const int64_t tiles = (M + 31) / 32, slabs = N / 128;
         // not where the result lies over the rows: one workgroup's features would be written while another still reads them (a residual is
@@ -2808,7 +2809,11 @@ int launch_output_projection(const void *a, int64_t a_ld, const void *w, const f
         const uintptr_t from = reinterpret_cast<uintptr_t>(a), to = reinterpret_cast<uintptr_t>(out);
         const bool apart = EPILOGUE == EPILOGUE_RESIDUAL || from + (uintptr_t)(2 * ((M - 1) * a_ld + C)) <= to || to + (uintptr_t)(2 * ((M - 1) * out_ld + N)) <= from;
         const int64_t cus = kutacc_cu_count();
-        const auto launch = [&](auto kern, int features, int64_t per_cu) {
+        const auto launch = [&](auto kern, bool walks, int features, int64_t per_cu) {
+            kutacc_prof::KernelTimer t(EPILOGUE == EPILOGUE_RESIDUAL ? (walks ? "output_projection_tile_kernel<residual, walking>" : "output_projection_tile_kernel<residual>")
+                                       : walks                       ? "output_projection_tile_kernel<walking>"
+                                                                     : "output_projection_tile_kernel",
+                                       flops, stream);
             const int64_t gx = std::min(tiles, std::max<int64_t>(per_cu * cus / (N / features), 1));
             kern<<<dim3((unsigned)gx, (unsigned)(N / features)), 2 * features, 0, stream>>>(
                 (const bf16_t *)a, a_ld, (const bf16_t *)w, bias, (bf16_t *)out, out_ld, (int)M, (int)swap_n);
@@ -2816,13 +2821,13 @@ int launch_output_projection(const void *a, int64_t a_ld, const void *w, const f
         };
         if (apart && M < (1 << 30)) {
             if (C == 128) {
-                return launch(output_projection_tile_kernel<C, EPILOGUE, 128, C == 128>, 128, 3);
+                return launch(output_projection_tile_kernel<C, EPILOGUE, 128, C == 128>, true, 128, 3);
             }
             if (N % 256 == 0 && tiles * (N / 256) > cus) {
-                return launch(output_projection_tile_kernel<C, EPILOGUE, C, true>, 256, 1);
+                return launch(output_projection_tile_kernel<C, EPILOGUE, C, true>, true, 256, 1);
             }
             if (tiles * slabs <= TILE_WORKGROUPS_PER_CU * cus) {
-                return launch(output_projection_tile_kernel<C, EPILOGUE, 128, C == 128>, 128, INT_MAX);
+                return launch(output_projection_tile_kernel<C, EPILOGUE, 128, C == 128>, false, 128, INT_MAX);
             }
         }
     }
@@ -2837,6 +2842,7 @@ int launch_output_projection(const void *a, int64_t a_ld, const void *w, const f
         int64_t gx, rpw;
         output_projection_split(C, M, gx, rpw);
         const int64_t gy = (N / 128 + SLABS - 1) / SLABS;
+        kutacc_prof::KernelTimer t(EPILOGUE == EPILOGUE_GATED_RESIDUAL ? "output_projection_kernel<gated residual>" : "output_projection_kernel", flops, stream);
         kern<<<dim3((unsigned)gx, (unsigned)gy), 64 * WAVES, lds_bytes, stream>>>(
             (const bf16_t *)a, a_ld, (const bf16_t *)w, bias, (bf16_t *)out, out_ld, M, (int)N, (int)rpw, (const bf16_t *)gate, gate_ld);
         return kutacc_hip_status(hipGetLastError());
@@ -3025,13 +3031,11 @@ int gating_attention_fused(const kutacc_hip_attention_args_t &a, hipStream_t str
     if (residual != FUSED_OUT_STORE) {
         // out += result, row (b, s) of the result going to row (s, b) of out ([seq_len, batch, C]) in the transposed form
         const int64_t swap_n = residual == FUSED_OUT_ADD_TRANSPOSED ? a.seq_len : 0;
-        kutacc_prof::KernelTimer t("output_projection_kernel<residual>", 2.0 * BS * C * C, stream);
         return (C == 128) ? launch_output_projection<128, EPILOGUE_RESIDUAL>(a.avg, a.avg_stride_s, a.output_w, a.output_b, a.out,
                                                                              a.out_ld, M, C, stream, nullptr, 0, swap_n)
                           : launch_output_projection<256, EPILOGUE_RESIDUAL>(a.avg, a.avg_stride_s, a.output_w, a.output_b, a.out,
                                                                              a.out_ld, M, C, stream, nullptr, 0, swap_n);
     }
-    kutacc_prof::KernelTimer t("output_projection_kernel", 2.0 * BS * C * C, stream);
     return (C == 128) ? launch_output_projection<128>(a.avg, a.avg_stride_s, a.output_w, a.output_b, a.out, a.out_ld, M, C, stream)
                       : launch_output_projection<256>(a.avg, a.avg_stride_s, a.output_w, a.output_b, a.out, a.out_ld, M, C, stream);
 }
@@ -3058,7 +3062,6 @@ int row_projection(const void *a, int64_t a_ld, const void *w, const float *bias
     if (!row_projection_supports(a, a_ld, w, bias, out, out_ld, m, n, k)) {
         return KUTACC_HIP_EUNSUPPORTED;
     }
-    kutacc_prof::KernelTimer t("output_projection_kernel", 2.0 * (double)m * (double)n * (double)k, stream);
     return k == 128 ? launch_output_projection<128>(a, a_ld, w, bias, out, out_ld, m, n, stream)
                     : launch_output_projection<256>(a, a_ld, w, bias, out, out_ld, m, n, stream);
 }
@@ -3071,7 +3074,6 @@ int row_projection_gated_residual(const void *a, int64_t a_ld, const void *w, co
     if (!row_projection_supports(a, a_ld, w, bias, acc, acc_ld, m, n, k) || !gate || gate_ld % 8 != 0 || !aligned(gate, 16)) {
         return KUTACC_HIP_EUNSUPPORTED;
     }
-    kutacc_prof::KernelTimer t("output_projection_kernel<gated residual>", 2.0 * (double)m * (double)n * (double)k, stream);
     return k == 128 ? launch_output_projection<128, EPILOGUE_GATED_RESIDUAL>(a, a_ld, w, bias, acc, acc_ld, m, n, stream, gate, gate_ld)
                     : launch_output_projection<256, EPILOGUE_GATED_RESIDUAL>(a, a_ld, w, bias, acc, acc_ld, m, n, stream, gate, gate_ld);
 }
