@@ -779,16 +779,18 @@ def test_row_projections_on_either_side_of_the_tile_kernel_s_rows(torch_cuda, k,
         assert helpers.same_bits(results[m], results[2 * limit + 45][:m].contiguous())
 
 
-@pytest.mark.parametrize("n", [256])
-def test_row_projection_over_its_own_rows(torch_cuda, n):
-    """The result in the place of the rows it was formed from: all features of a row by the workgroup that has read it."""
+@pytest.mark.parametrize("n", [128, 256])
+@pytest.mark.parametrize("rows", [777, 100003])
+def test_row_projection_over_its_own_rows(torch_cuda, n, rows):
+    """The result in the place of the rows it was formed from: all features of a row by the workgroup that has read it, in one step of 32 rows a
+    wave and in several."""
     torch = torch_cuda
     g = torch.Generator(device="cuda").manual_seed(n)
     w = (torch.randn(n, n, device="cuda", generator=g) * n ** -0.5).to(torch.bfloat16)
     bias = torch.randn(n, device="cuda", generator=g)
-    a = torch.randn(777, n, device="cuda", generator=g).to(torch.bfloat16)
+    a = torch.randn(rows, n, device="cuda", generator=g).to(torch.bfloat16)
     want = a.float() @ w.float().T + bias
-    rc = capi.lib().kutacc_hip_gemm(ctypes.byref(row_projection_args(a, w, bias, a)), None)
-    torch.cuda.synchronize()
-    assert rc == 0, rc
+    rcs = []
+    names = helpers.profiled_kernels(torch, lambda: rcs.append(capi.lib().kutacc_hip_gemm(ctypes.byref(row_projection_args(a, w, bias, a)), None)))
+    assert rcs == [0] and names == ["output_projection_kernel"], (rcs, names)
     helpers.check_close(helpers.to_numpy(a), helpers.to_numpy(want), "bf16", "row projection in place")
