@@ -514,8 +514,9 @@ __device__ __forceinline__ void attend_block_l2(const uint4 *lds_k, const uint4 
                                                 int prio_phase = -1, int fair_turn = -1)
 {
     // ODD: the last tile is the one of zeros behind an odd number of them, and left out (us, triangle attention of 77 residues 18.9 -> 18.4, 150
-    // 33.6 -> 32.4, 288 70.9 -> 67.9, 450 211.5 -> 206, 600 391 -> 382; MSA rows, two rows a step, 512 x 224 186.3 -> 184.1).  A loop of its own: decided
-    // inside one, even numbers lost 0.5 to 1 %.
+    // 33.6 -> 32.4, 288 70.9 -> 67.9, 450 211.5 -> 206, 600 391 -> 382; MSA rows, two rows a step, 512 x 224 186.3 -> 184.1).  A loop of its own, and
+    // in the kernels of single rows a kernel of its own: decided inside one loop, even numbers lost 0.5 to 1 %, and both loops in one kernel spill
+    // registers (triangle attention of 185 padded residues 38.2 us so, 36.8 now, 300 83.0 and 75.7, 450 193 and 189).
     const int npairs = NB >> 1;
     const uint4 *kp = lds_k + lane;
     const uint4 *vp = lds_v + lane;

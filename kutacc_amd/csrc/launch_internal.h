@@ -82,7 +82,7 @@ int gating_attention_tiled(const kutacc_hip_attention_args_t &args, hipStream_t 
 
 // small_head_attention.hip: the attention step of that route for heads of 8, on the same tensors
 bool small_head_attention_supports(const kutacc_hip_attention_args_t &args);
-// whether it can form the projections itself, from the input rows (q, k, v and gate stay as they are)
+// whether it can form the projections itself, from the input rows (q, k and gate are its workspace, v is not touched)
 bool small_head_attention_projects(const kutacc_hip_attention_args_t &args);
 int small_head_attention(const kutacc_hip_attention_args_t &args, bool projects, hipStream_t stream);
 

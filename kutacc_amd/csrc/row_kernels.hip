@@ -218,8 +218,8 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
     // key tile t of query q, on a grid of whole blocks of queries and whole tiles of keys: the last tile of a query has fewer
     // rows (zeros take the place of the others in the copy), and queries past the last repeat that one, in the copy only.  A workgroup's
     // waves take four queries that follow each other: their pieces of 16 bytes in the copy are neighbours, and so are their rows of z for the
-    // ending node.  (Four tiles of one query: triangle attention of 128 residues 22.2 us, now 21.1; of 384 116.1 and 114.4, ending node 121.3
-    // and 119.2; 508 x 259 with eight heads, this kernel, 12.8 and 10.6.)
+    // ending node.  (Four tiles of one query, now: triangle attention of 160 residues 33.0 and 32.5 us, of 200 42.1 and 41.6, of 256 46.9 and 46.5, of 128 no
+    // difference, of 112 20.0 and 20.6; MSA rows 256 x 256 100.6 and 99.2; 508 x 259 with eight heads, this kernel, 12.8 and 10.6.)
     uint32_t row0 = ((uint32_t)blockIdx.x * 4 + wave) * PAIR_BIAS_ROWS_PER_WAVE, count = 0;
     int q = 0, t = 0;
     if (nbf == nullptr) {

@@ -10,9 +10,8 @@
 //     keys past the end at -inf; masks are added to it in fp32, only in key tiles that have one;
 //   * p.v with 16x16x32 MFMAs of 32 keys whose rows are the eight values and ones, which give the sums of the probabilities.
 // K, V and masks of a head's four rows lie in the LDS for the whole workgroup (128 bytes per key and 16 of masks).
-// Measured on 1024 rows x 301 keys x 8 heads: 505 us on the general attention_tiles_kernel, 177 to 189 us here (vector
-// issue 69 %).  With the queries and
-// the masks in two parts (16 bits, an error of up to 8 % in a probability at logits of 11 000) and 32x32x16 products it was 199.
+// Measured on 1024 rows x 301 keys x 8 heads: 505 us on the general attention_tiles_kernel, 177 to 189 us here behind a pass that
+// projects, 168 to 204 from card to card with the projections inside (vector issue 73 %).  With the queries and the masks in two parts (16 bits, an error of up to 8 % in a probability at logits of 11 000) and 32x32x16 products it was 199.
 #include <hip/hip_runtime.h>
 #include <math.h>
 

@@ -884,11 +884,11 @@ __global__ __launch_bounds__(768) void streamed_plain_kernel(const StreamedParam
 // act += avg . Wo^T + bo, row (b, s) of the product to row (b, s) of act, or transposed to row (s, b).  Bound by HBM: 2 C bytes a
 // position in, and 4 C of act.  A wave keeps the weights of 32 features in registers, their head dims in the order of the fragments in which the
 // gated average arrives; a workgroup of all features walks blocks of 32 positions, which its waves share in the LDS, the next block
-// and its activations under way; with 256 channels, one workgroup a CU, the next two (MSA columns of 1024 x 384 126 -> 119 us of this kernel; with 128,
-// two workgroups a CU, 2048 residues 617 -> 638).  The product (rows = features, columns = positions) crosses the LDS to meet the activation in whole
+// and its activations under way; with 256 channels, one workgroup a CU, the next two (medians of this kernel: MSA columns of
+// 1024 x 384 125 -> 119 us, of 2000 x 300 186 -> 176, rows of 508 x 259 47 -> 45; with 128, two workgroups a CU, 2048 residues 617 -> 638).  The product (rows = features, columns = positions) crosses the LDS to meet the activation in whole
 // cache lines.  act, weights and bias lie on any address.  With the weights in the LDS, read for every block by waves that walked
-// alone, MSA rows of 508 x 259 took 50 us of this kernel, now 40, 300 x 300 37 and 26, columns of 500 x 100 26 and 17,
-// triangle attention of 2048 residues 652 and 617, of 1000 141 and 141.
+// alone, MSA rows of 508 x 259 took 52 us of this kernel, now 45, 300 x 300 39 and 31, columns of 500 x 100 27 and 21, of 1024 x 384 122 and 119,
+// triangle attention of 2048 residues 650 and 618, of 1200 193 and 176.
 template <int C>
 __global__ __launch_bounds__(2 * C, 2) void output_projection_kernel(
     const uint4 *__restrict__ avg, const bf16_t *__restrict__ wo, const float *__restrict__ bo, bf16_t *__restrict__ act, int64_t ld,

@@ -504,7 +504,8 @@ namespace kutacc_launch {
 
 bool triangle_ends_support(const kutacc_hip_triangle_multiplication_args_t &a)
 {
-    // 16-byte loads of the activation's rows and of the weights; positions and a plane's bytes times eight in 32 bits
+    // 16-byte loads of the activation's rows and of the weights; positions and sixteen planes' bytes (2^31 at
+    // 8192 residues) in 32 bits
     return a.c_z == C && a.c_i == C && a.n_res <= 8192 && kutacc_hip_aligned16(a.pair_act) && kutacc_hip_aligned16(a.left_proj_w) &&
            kutacc_hip_aligned16(a.left_gate_w) && kutacc_hip_aligned16(a.right_proj_w) && kutacc_hip_aligned16(a.right_gate_w) &&
            kutacc_hip_aligned16(a.output_w) && kutacc_hip_aligned16(a.gating_w);
