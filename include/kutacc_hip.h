@@ -77,11 +77,11 @@ typedef struct kutacc_hip_attention_args {
     int64_t nb_stride_h;
     int64_t nb_stride_q;
 
-    /* Caller scratch.  k/v/gate are written only by the generic and the tiled path (the latter, with eight heads of 8 and
-     * KUTACC_HIP_PATH_AUTO, uses q, k and gate as workspace and leaves v); q is written by those
-     * and may be used as workspace by the fused path (a re-ordered copy of the pair bias), so
-     * its contents are unspecified after any call; avg (gated weighted average, [B,S,H,d]) is
-     * written by every path.  Element (b,s,h,e) of q,k,gate,avg lives at
+    /* Caller scratch.  KUTACC_HIP_PATH_TILED and KUTACC_HIP_PATH_GENERIC fill q, k, v and gate as the reference does.  After
+     * a call with another path their contents are unspecified: the fused kernels leave k, v and gate alone and may use q as
+     * workspace (a re-ordered copy of the pair bias), the tiled route with eight heads of 8 leaves v alone and uses q, k
+     * and gate as workspace (it fills all four where one of those three lies over input or avg).
+     * avg (gated weighted average, [B,S,H,d]) is written by every path.  Element (b,s,h,e) of q,k,gate,avg lives at
      * b*stride_b + s*stride_s + h*stride_h + e; v is [H,d,B,S]: (h,e,b,s) at
      * h*v_stride_h + e*v_stride_e + b*v_stride_b + s. */
     void *q, *k, *v, *gate, *avg;
@@ -122,6 +122,8 @@ kutacc_export int kutacc_hip_gating_attention_static(const kutacc_hip_attention_
  * shared by all heads.  bf16 storage, nheads*head_size == 64 (the reference hard-wires nchannels == 64,
  * :172), nheads <= 32, head_size <= 32.  The reference's scratch tensors q, k, v, gate are not needed and
  * not touched; q_avg ([B, 64], may be NULL) receives the masked mean as the reference leaves it in `avg`.
+ * A batch row's bits do not depend on the other rows of the call or on its place among them (a long row may be shared by several
+ * workgroups: each forms the same mean and the same average); they may depend on the number of rows and on the device.
  * seq_len <= 12288 (what a workgroup's LDS holds of a row's mask and logits; longer rows return
  * KUTACC_HIP_EUNSUPPORTED before anything is launched); the tokens of a batch row must lie within 2 GiB of its first one in q_data and in out (32-bit
  * offsets in the kernel), else KUTACC_HIP_EUNSUPPORTED. */
@@ -478,7 +480,8 @@ kutacc_export int kutacc_hip_profile_read(int index, char *name, int name_len, d
  *               shape-agnostic kernels where that route does not take the call), which fills the caller's q, k, v and
  *               gate tensors as the reference's kernel does (src/attention/gating_attention.cpp:47-66) -- for callers or
  *               tests that read them; about twice the time of the fused kernels.  Anything else (default): the fused MFMA
- *               kernels where they apply, which leave k, v and gate untouched and use q as workspace.
+ *               kernels where they apply, which leave k, v and gate untouched and use q as workspace, and with eight
+ *               heads of 8 the kernel that uses q, k and gate as workspace.
  *   "pointer_checks" "0": the handle-based attention entry points classify only `input` (host or device) and take the
  *               caller's word that every other operand lives in the same place, which saves about fifteen driver
  *               queries per call; "1": every operand is checked and mixed calls are rejected (default) */
