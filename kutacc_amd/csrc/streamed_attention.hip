@@ -781,6 +781,10 @@ __global__ __launch_bounds__(768) void streamed_plain_kernel(const StreamedParam
     };
 
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); // groups 0 and 1 have landed, every wave's part of them
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i) { // waited for here, not at their first uses in the loop, where that is a wait for the next tiles
+        asm volatile("" ::"v"(q[i][0]), "v"(q[i][1]));
+    }
     refill();
     int left = W; // tiles of the current group still to come, this one included
     const uint4 *const end = lds + RING * W * TILE, *next = lds + TILE; // tile t + 1
