@@ -7,18 +7,25 @@
 // second without leaving the registers.  For that, row i of a W1 block in the LDS is hidden unit sigma(i) (bits 2 and 3 of i
 // swapped), which makes the eight values a lane holds per k-step consecutive hidden units.
 //
-// What bounds it.  Every MFMA needs one weight fragment from the LDS, 8 cycles of the CU's 128 bytes a cycle for the 8
-// cycles of a SIMD that four SIMDs share: the matrix pipes and the LDS are saturated together.  What is left to win is to
-// keep them so: weights come straight into the LDS (global_load_lds_dwordx4, no registers, no LDS write instructions) into
-// a ring with one barrier per slice, and two waves or more on a SIMD hide each other's conversions and LDS round trips.
+// What bounds it: power.  With two waves a SIMD in their loops the matrix pipes work for 93 of 100 clocks, at the 1.6 to 1.7 GHz that
+// the chip holds under it; a third of a workgroup's time (of 103 000 clocks at 256 -> 1024) goes to its rows' way in and out, in
+// which the other workgroup of the CU has the pipes to itself.  Weights come straight into the LDS (global_load_lds_dwordx4, no
+// registers, no LDS write instructions) into a ring with one barrier per slice.
+// The two products of a slice are a step apart: while W1 of slice j runs, W2 of slice j - 1 runs between its products, whose sums
+// depend on each other; the hidden units of slice j are rounded beside the last products of W2, and every weight fragment leaves the LDS
+// AHEAD products before its own.  With both products of one slice in a step a wave waited for the end of the first product, for its
+// rounding and for most of its fragments.  A wave alone on its SIMD gains most: 20000 rows, 256 -> 1024 39.5 -> 34.1 us; 195072 rows 199
+// -> 186.5 (1097 TFLOP/s), 400000 rows, 256 -> 512 248 -> 229, 147456 rows, 128 -> 256 33.0 -> 31.8, 64 -> 256 19.2 -> 18.3.
 // Two workgroups or three per CU rather than one of twice the waves: one computes while the other fetches its rows or
-// stores its result (256 -> 512 at 147456 rows: 108 -> 98 us, 128 -> 256: 42 -> 34 us).
-//   195072 rows, 256 -> 1024, block: 328 us with weights through registers and one wave per SIMD, 198 here (1040 TFLOP/s,
-//   floor 165); 500000 rows, 128 -> 512: 175 -> 150 us (floor 106); 500000 rows, 64 -> 256: 200 us in three passes, 52 here.
+// stores its result (400000 rows, 256 -> 512 232 against 245 us, 147456 rows, 128 -> 512 48 and 51).  Two sets of rows a wave, for half the fragments,
+// leave no registers: 128 -> 512 70 us with 38 of them spilled.
+//   195072 rows, 256 -> 1024, block: 328 us with weights through registers and one wave per SIMD; 500000 rows, 64 -> 256: 200 us in three
+//   passes, 52 in this one.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "launch_internal.h"
 #include "mfma_tiles.h"
@@ -142,22 +149,34 @@ __device__ __forceinline__ bf16x8 hidden_operand(const f32x16 &h, int s)
     bf16x8 f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        f[e] = (bf16_t)fmaxf(h[8 * s + e], 0.f);
+        f[e] = (bf16_t)__builtin_amdgcn_fmed3f(h[8 * s + e], 0.f, INFINITY); // fmaxf without an instruction that quiets the value; a NaN gives 0 as well
     }
     return f;
 }
 
-// 64 channels of 32 rows: accumulators (+ b2) -> bf16 through the panel, out as whole 128-byte runs
-template <int CO, bool BLOCK>
-__device__ __forceinline__ void store_channels(const f32x16 &low, const f32x16 &high, const TransitionParams &p, int64_t row0, int last_local, int channel,
-                                               uint4 *panel, int lane)
+// 64 channels of 32 rows as store_channels adds to them and writes them: lane (lane >> 3, lane & 7) chunk lane & 7 of rows 8 i + (lane >> 3)
+struct Residual {
+    uint4 z[4];
+};
+template <int CO>
+__device__ __forceinline__ Residual load_residual(const bf16_t *rows, int last_local, int channel, int lane)
+{
+    const PanelRegs t = panel_load(rows, CO, 0, last_local, channel, lane);
+    return Residual{{t.r0, t.r1, t.r2, t.r3}};
+}
+
+// 64 channels of 32 rows: accumulators (+ b2) -> bf16 through the panel, out as whole 128-byte runs.  EARLY: the residual is there, else
+// it is read where it is added
+template <int CO, bool BLOCK, bool EARLY>
+__device__ __forceinline__ void store_channels(const f32x16 &low, const f32x16 &high, const float *b2, const Residual &residual, bf16_t *rows, int last_local,
+                                               int channel, uint4 *panel, int lane)
 {
     const int r = lane & 31, g = lane >> 5;
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
-            const f32x4 bv = *reinterpret_cast<const f32x4 *>(p.b2 + channel + n * 32 + 8 * a + 4 * g);
+            const f32x4 bv = *reinterpret_cast<const f32x4 *>(b2 + channel + n * 32 + 8 * a + 4 * g);
             bf16x4 ov;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
@@ -171,9 +190,9 @@ __device__ __forceinline__ void store_channels(const f32x16 &low, const f32x16 &
         const int prow = 8 * i + (lane >> 3);
         uint4 v = panel[panel_slot(prow, lane & 7)];
         if (prow <= last_local) {
-            bf16_t *dst = p.out + (row0 + prow) * CO + channel + (lane & 7) * 8;
+            uint4 *dst = reinterpret_cast<uint4 *>(rows + (int64_t)prow * CO + channel + (lane & 7) * 8);
             if constexpr (BLOCK) { // residual: the row as it was before the LayerNorm
-                const bf16x8 o = as_bf16x8(v), z = as_bf16x8(*reinterpret_cast<const uint4 *>(dst));
+                const bf16x8 o = as_bf16x8(v), z = as_bf16x8(EARLY ? residual.z[i] : *dst);
                 bf16x8 res;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
@@ -181,7 +200,7 @@ __device__ __forceinline__ void store_channels(const f32x16 &low, const f32x16 &
                 }
                 v = as_uint4(res);
             }
-            *reinterpret_cast<uint4 *>(dst) = v;
+            *dst = v;
         }
     }
 }
@@ -205,12 +224,17 @@ __global__ __launch_bounds__(64 * WAVES, GROUPS * WAVES / 4) void transition_row
     constexpr int UPW = STAGE_SLOTS / 64 / WAVES;  // loads of 1 KB a wave asks for per stage
     static_assert(SLICE == 32 || SLICE == 64, "layout of W2 slices");
     static_assert(WAVES * 256 <= STAGE_SLOTS && UPW >= 4, "the waves' panels lie in a stage; a wave's loads fill whole panels");
-    extern __shared__ uint4 lds[]; // [STAGES][W1 slice, W2 slice], b1
+    extern __shared__ uint4 lds[]; // [STAGES][W1 slice, W2 slice], b1, b2
+    static_assert(CO <= 64 * WAVES, "a thread brings one value of b2");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5, NJ = p.c_i / SLICE;
     float *b1s = reinterpret_cast<float *>(lds + STAGES * STAGE_SLOTS);
+    float *b2s = b1s + p.c_i;
     for (int i = tid; i < p.c_i; i += 64 * WAVES) {
         b1s[i] = p.b1[i]; // visible after the first barrier of the slice loop
+    }
+    if (CO == 64 * WAVES || tid < CO) {
+        b2s[tid] = p.b2[tid];
     }
 
     const int past = (int)blockIdx.x - p.full_groups;
@@ -236,7 +260,7 @@ __global__ __launch_bounds__(64 * WAVES, GROUPS * WAVES / 4) void transition_row
         } else if constexpr (SLICE == 64) {
             lane_bytes[hi] = 2u * (uint32_t)(rl * p.c_i + 8 * ((lane & 7) ^ rl ^ hi));
         } else {
-            lane_bytes[hi] = 2u * (uint32_t)((lane >> 2) * p.c_i + 8 * ((lane & 3) ^ ((lane >> 3) & 3)));
+            lane_bytes[hi] = 2u * (uint32_t)((lane >> 2) * p.c_i + 8 * ((lane & 3) ^ ((lane >> 4) & 3)));
         }
     }
     const char *unit_src[UPW];
@@ -261,8 +285,16 @@ __global__ __launch_bounds__(64 * WAVES, GROUPS * WAVES / 4) void transition_row
             unit_src[i] += slice_bytes;
         }
     };
-    for (int j = 0; j < STAGES - 1 && j < NJ; ++j) {
-        ask(j);
+    // Batch b of the loads: W1 of slice b and W2 of slice b - 1, which meet in step b of the loop.  A wave brings one matrix, so W1's
+    // batches are 0 .. NJ - 1 and W2's 1 .. NJ.
+    const int first_batch = first_matrix ? 0 : 1, last_batch = first_matrix ? NJ - 1 : NJ;
+    auto ask_batch = [&](int batch) {
+        if (batch >= first_batch && batch <= last_batch) {
+            ask((first_matrix ? batch : batch - 1) % STAGES);
+        }
+    };
+    for (int b = 0; b < STAGES - 1; ++b) {
+        ask_batch(b);
     }
 
     const XFragments<CO> x = fragments<CO, BLOCK>(t, p, lds + (STAGES - 1) * STAGE_SLOTS + wave * 256, lane);
@@ -272,12 +304,18 @@ __global__ __launch_bounds__(64 * WAVES, GROUPS * WAVES / 4) void transition_row
     for (int cb = 0; cb < CB; ++cb) {
         oacc[cb] = zero16();
     }
-    const int w1_lane = panel_slot(r, g), w2_lane = SLICE == 64 ? w1_lane : r * 4 + (g ^ ((r >> 1) & 3));
-    int at = STAGES - 1, given_up = STAGES - 2; // stages of the slice and of the one before it
-    for (int j = 0; j < NJ; ++j) {
-        given_up = at, at = at + 1 == STAGES ? 0 : at + 1;
-        // slice j has landed (the later ones may be under way), and every wave is done with the stage it gives up
-        const int behind = min(NJ - 1 - j, STAGES - 2);
+    const int w1_lane = panel_slot(r, g), w2_lane = SLICE == 64 ? w1_lane : r * 4 + (g ^ ((r >> 2) & 3));
+    f32x16 h[HB];
+    bf16x8 hf[HB][2];
+    constexpr bool EARLY = CO != 64; // with 64 channels there are no registers for it
+    Residual residual[CP];
+    // Step j: W1 of slice j (if FIRST) and W2 of slice j - 1 (if SECOND), PRODUCTS of each.  Their operands come from the LDS AHEAD of their
+    // use; the hidden units of slice j become operands while the last products of W2 run.
+    constexpr int PRODUCTS = HB * KS, AHEAD = CO == 64 ? 2 : 3;
+    auto step = [&](int j, auto has_first, auto has_second) __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(has_first)::value, SECOND = decltype(has_second)::value;
+        // batch j has landed (the later ones may be under way), and every wave is done with the stages of batch j - 1
+        const int behind = max(0, min(STAGES - 2, last_batch - j));
         if (behind == 2) {
             wait_and_barrier<2 * UPW>();
         } else if (behind == 1) {
@@ -285,39 +323,89 @@ __global__ __launch_bounds__(64 * WAVES, GROUPS * WAVES / 4) void transition_row
         } else {
             wait_and_barrier<0>();
         }
-        if (j + STAGES - 1 < NJ) {
-            ask(given_up);
-        }
+        ask_batch(j + STAGES - 1);
         if (!active) {
-            continue;
+            return;
         }
-        const uint4 *stage = lds + at * STAGE_SLOTS;
+        if constexpr (!FIRST && BLOCK && EARLY) { // the rows' place in the registers is free
+            int lane = tid & 63; // opaque: its part of the addresses is formed here, not kept over the loop
+            asm volatile("" : "+v"(lane));
 #pragma unroll
-        for (int hb = 0; hb < HB; ++hb) {
-            f32x16 h = hidden_bias(b1s + j * SLICE + hb * 32, g);
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                h = mfma(as_bf16x8(stage[(hb * CP + ks / 4) * 256 + (w1_lane ^ (2 * (ks % 4)))]), x.f[ks], h);
+            for (int cp = 0; cp < CP; ++cp) {
+                residual[cp] = load_residual<CO>(p.out + row0 * CO, last_local, cp * 64, lane);
             }
-            const bf16x8 hf[2] = {hidden_operand(h, 0), hidden_operand(h, 1)};
+        }
+        const uint4 *w1 = lds + j % STAGES * STAGE_SLOTS, *w2 = lds + (j + STAGES - 1) % STAGES * STAGE_SLOTS + W1_SLOTS;
+        if constexpr (FIRST) {
 #pragma unroll
-            for (int cb = 0; cb < CB; ++cb) {
+            for (int hb = 0; hb < HB; ++hb) {
+                h[hb] = hidden_bias(b1s + j * SLICE + hb * 32, g);
+            }
+        }
+        // product i of either matrix: of W1 k-step i / HB of hidden block i % HB, of W2 channels 32 (i % CB) by hidden units
+        // 16 (i / CB) .. + 15 of the slice
+        auto w1_fragment = [&](int i) {
+            const int hb = i % HB, ks = i / HB;
+            return as_bf16x8(w1[(hb * CP + ks / 4) * 256 + (w1_lane ^ (2 * (ks % 4)))]);
+        };
+        auto w2_fragment = [&](int i) {
+            const int cb = i % CB, s = i / CB;
+            return as_bf16x8(w2[SLICE == 64 ? cb * 256 + (w2_lane ^ (2 * s)) : cb * 128 + (w2_lane ^ (2 * s))]);
+        };
+        // the order: two of W1, one of W2, and so on, then the other half of W2's
+        constexpr int TOTAL = (FIRST ? PRODUCTS : 0) + (SECOND ? PRODUCTS : 0);
+        auto is_w1 = [](int m) { return FIRST && (!SECOND || (m < 3 * PRODUCTS / 2 && m % 3 != 2)); };
+        auto index_of = [&](int m) {
+            return !FIRST || !SECOND ? m : m >= 3 * PRODUCTS / 2 ? m - PRODUCTS : m % 3 == 2 ? m / 3 : m / 3 * 2 + m % 3;
+        };
+        auto fragment = [&](int m) { return is_w1(m) ? w1_fragment(index_of(m)) : w2_fragment(index_of(m)); };
+        bf16x8 w[TOTAL];
+#pragma unroll
+        for (int m = 0; m < AHEAD; ++m) {
+            w[m] = fragment(m);
+        }
+        bf16x8 next[HB][2];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < TOTAL; ++m) {
+            const int i = index_of(m);
+            if (is_w1(m)) {
+                h[i % HB] = mfma(w[m], x.f[i / HB], h[i % HB]);
+            } else {
+                oacc[i % CB] = mfma(w[m], hf[i / CB / 2][i / CB % 2], oacc[i % CB]);
+            }
+            if (m + AHEAD < TOTAL) {
+                w[m + AHEAD] = fragment(m + AHEAD);
+            }
+            if (FIRST && SECOND && m >= TOTAL - 2 * HB) { // one operand beside each of the last products
+                const int q = m - (TOTAL - 2 * HB);
+                next[q / 2][q % 2] = hidden_operand(h[q / 2], q % 2);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (FIRST) {
+#pragma unroll
+            for (int hb = 0; hb < HB; ++hb) {
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
-                    const int slot = SLICE == 64 ? cb * 256 + (w2_lane ^ (2 * (2 * hb + s))) : cb * 128 + (w2_lane ^ (2 * s));
-                    oacc[cb] = mfma(as_bf16x8(stage[W1_SLOTS + slot]), hf[s], oacc[cb]);
+                    hf[hb][s] = SECOND ? next[hb][s] : hidden_operand(h[hb], s);
                 }
             }
         }
+    };
+    step(0, std::true_type{}, std::false_type{});
+    for (int j = 1; j < NJ; ++j) {
+        step(j, std::true_type{}, std::true_type{});
     }
+    step(NJ, std::false_type{}, std::true_type{});
 
     if (!active) {
         return;
     }
-    uint4 *panel = lds + given_up * STAGE_SLOTS + wave * 256; // a stage that no wave reads any more
+    uint4 *panel = lds + NJ % STAGES * STAGE_SLOTS + wave * 256; // a stage that no wave reads any more
 #pragma unroll
-    for (int half = 0; half < CB / 2; ++half) {
-        store_channels<CO, BLOCK>(oacc[2 * half], oacc[2 * half + 1], p, row0, last_local, half * 64, panel, lane);
+    for (int cp = 0; cp < CP; ++cp) {
+        store_channels<CO, BLOCK, EARLY>(oacc[2 * cp], oacc[2 * cp + 1], b2s, residual[cp], p.out + row0 * CO, last_local, cp * 64, panel, lane);
     }
 }
 
@@ -347,7 +435,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void transition_split_kernel
     for (int hi = 0; hi < 2; ++hi) {
         w1_bytes[hi] = 2u * (uint32_t)(((rl & 3) | ((rl & 4) << 1)) * CO + 8 * ((lane & 7) ^ rl ^ hi));
     }
-    const uint32_t w2_bytes = 2u * (uint32_t)((lane >> 2) * p.c_i + 8 * ((lane & 3) ^ ((lane >> 3) & 3)));
+    const uint32_t w2_bytes = 2u * (uint32_t)((lane >> 2) * p.c_i + 8 * ((lane & 3) ^ ((lane >> 4) & 3)));
     auto ask_w1 = [&](int block) {
         const bf16_t *from = p.w1 + (int64_t)block * 32 * CO;
 #pragma unroll
@@ -377,7 +465,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void transition_split_kernel
     for (int cb = 0; cb < CB; ++cb) {
         oacc[cb] = zero16();
     }
-    const int w1_lane = panel_slot(r, g), w2_lane = r * 4 + (g ^ ((r >> 1) & 3));
+    const int w1_lane = panel_slot(r, g), w2_lane = r * 4 + (g ^ ((r >> 2) & 3));
     for (int block = wave; block < NB; block += WAVES) {
         const bool more = block + WAVES < NB;
         wait_for_loads<UNITS>(); // all but W2's
@@ -407,6 +495,10 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void transition_split_kernel
         }
     }
 
+    Residual residual;
+    if (BLOCK && wave < CB / 2) {
+        residual = load_residual<CO>(p.out + row0 * CO, last_local, wave * 64, lane);
+    }
     // the waves' sums, each in its own region, then 64 channels a wave
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
@@ -431,7 +523,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void transition_split_kernel
                 }
             }
         }
-        store_channels<CO, BLOCK>(sum[0], sum[1], p, row0, last_local, wave * 64, panel, lane);
+        store_channels<CO, BLOCK, true>(sum[0], sum[1], p.b2, residual, p.out + row0 * CO, last_local, wave * 64, panel, lane);
     }
 }
 
@@ -443,7 +535,7 @@ hipError_t launch_rows(TransitionParams p, hipStream_t stream)
     static size_t configured[KUTACC_DEVICE_SLOTS] = {};
     const size_t stages = (size_t)STAGES * SLICE * CO * 4;
     const auto kernel = &transition_rows_kernel<CO, BLOCK, SLICE, STAGES, WAVES, GROUPS>;
-    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(kernel), stages + MAX_HIDDEN * sizeof(float), configured)) {
+    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(kernel), stages + (MAX_HIDDEN + CO) * sizeof(float), configured)) {
         return e;
     }
     // Full rounds of workgroups, then the rest dealt evenly over the CUs, as few waves with rows per workgroup as that takes
@@ -455,7 +547,7 @@ hipError_t launch_rows(TransitionParams p, hipStream_t stream)
     const int64_t groups = (per_cu + WAVES - 1) / WAVES;
     p.tail_waves = (int)((per_cu + groups - 1) / groups);
     const int64_t blocks = p.full_groups + (rest + p.tail_waves - 1) / p.tail_waves;
-    kernel<<<dim3((unsigned)blocks), 64 * WAVES, stages + (size_t)p.c_i * sizeof(float), stream>>>(p);
+    kernel<<<dim3((unsigned)blocks), 64 * WAVES, stages + (size_t)(p.c_i + CO) * sizeof(float), stream>>>(p);
     return hipGetLastError();
 }
 

@@ -401,6 +401,21 @@ def test_transition_forced_paths(torch_cuda):
                                    2, 8, 8, capi.K_BF16, capi.PATH_AUTO, None) == capi.EINVAL  # needs the intermediate
 
 
+@pytest.mark.parametrize("rows,c_o,c_i", [(40, 256, 1024), (8200, 256, 64), (8200, 128, 128), (33, 128, 64)])
+def test_transition_of_a_row_that_is_no_number(torch_cuda, rows, c_o, c_i):
+    """ReLU takes a NaN for zero (as fmaxf does), in either kernel and at the fewest slices: such a row's result is b2, and no other row knows."""
+    torch = torch_cuda
+    c = transition_case(1400 + c_i, 1, rows, c_o, c_i)
+    out, _ = run_transition(torch, c)
+    x = c["x"].copy()
+    x[0, rows - 2, 3] = np.nan
+    other, _ = run_transition(torch, dict(c, x=x))
+    b2 = torch.from_numpy(c["b2"]).cuda().to(torch.bfloat16)
+    keep = [i for i in range(rows) if i != rows - 2]
+    assert helpers.same_bits(other.reshape(rows, c_o)[rows - 2], b2)
+    assert helpers.same_bits(other.reshape(rows, c_o)[keep], out.reshape(rows, c_o)[keep])
+
+
 def test_transition_full_pair_size(torch_cuda):
     """The pair transition of a 384-residue model at its real shape (147456 rows); the oracle checks a sample of
     rows (rows are independent), and a second call on a row permutation must give the permuted result bit for bit."""
