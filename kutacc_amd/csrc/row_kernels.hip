@@ -198,7 +198,9 @@ __global__ __launch_bounds__(256) void layernorm_rows_bf16_kernel(const bf16_t *
 constexpr int PAIR_BIAS_ROWS_PER_WAVE = 32; // a multiple of 32; LDS per workgroup = 1 KB per row
 constexpr int64_t PAIR_BIAS_MAX_ROWS = (int64_t)1 << 23; // rows and byte offsets are counted in 32 bits: 2 GiB of z
 
-template <int H>
+// SHARED: the four waves of a workgroup normalise eight of the 32 rows each and the first one goes on alone, so that fewer units than the
+// chip has SIMDs are not one wave's work each.
+template <int H, bool SHARED>
 __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__restrict__ z, const float *__restrict__ gamma,
                                                              const float *__restrict__ beta, const bf16_t *__restrict__ w,
                                                              bf16_t *__restrict__ nb, bf16_t *__restrict__ z_norm,
@@ -206,8 +208,8 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
                                                              int transposed, uint4 *__restrict__ nbf, int frag_nb,
                                                              int frag_nt, int frag_tiles)
 {
-    constexpr int LPR = 16, CZ = 128, STEPS = PAIR_BIAS_ROWS_PER_WAVE / 4, RB = PAIR_BIAS_ROWS_PER_WAVE / 32;
-    __shared__ uint4 tiles[4][RB * 2 * 256]; // per wave: its rows x 128 channels as 32 x 64 panels
+    constexpr int LPR = 16, CZ = 128, STEPS = PAIR_BIAS_ROWS_PER_WAVE / (SHARED ? 16 : 4), RB = PAIR_BIAS_ROWS_PER_WAVE / 32;
+    __shared__ uint4 tiles[SHARED ? 1 : 4][RB * 2 * 256]; // per wave (or of all four): its rows x 128 channels as 32 x 64 panels
     const int lane = threadIdx.x & 63;
     const int sub = lane & 15, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // uniform: the wave's first row stays in scalar registers
@@ -220,7 +222,8 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
     // waves take four queries that follow each other: their pieces of 16 bytes in the copy are neighbours, and so are their rows of z for the
     // ending node.  (Four tiles of one query, now: triangle attention of 160 residues 33.0 and 32.5 us, of 200 42.1 and 41.6, of 256 46.9 and 46.5, of 128 no
     // difference, of 112 20.0 and 20.6; MSA rows 256 x 256 100.6 and 99.2; 508 x 259 with eight heads, this kernel, 12.8 and 10.6.)
-    uint32_t row0 = ((uint32_t)blockIdx.x * 4 + wave) * PAIR_BIAS_ROWS_PER_WAVE, count = 0;
+    uint32_t row0 = (SHARED ? (uint32_t)blockIdx.x : (uint32_t)blockIdx.x * 4 + wave) * PAIR_BIAS_ROWS_PER_WAVE, count = 0;
+    const int first_row = (SHARED ? 8 * wave : 0) + grp * STEPS; // of this lane's group
     int q = 0, t = 0;
     if (nbf == nullptr) {
         if (row0 >= nrows) {
@@ -228,7 +231,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
         }
         count = min(32u, nrows - row0);
     } else {
-        q = (int)(blockIdx.x / (uint32_t)frag_nb * 4) + wave, t = (int)(blockIdx.x % (uint32_t)frag_nb);
+        q = SHARED ? (int)(blockIdx.x / (uint32_t)frag_nb) : (int)(blockIdx.x / (uint32_t)frag_nb * 4) + wave, t = (int)(blockIdx.x % (uint32_t)frag_nb);
         if (q >= 32 * frag_nb) {
             return;
         }
@@ -237,17 +240,17 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
     }
     const bool stores = q < (int)nrow_i; // (nrow_i = ncol where there is a copy)
     const char *zbytes = reinterpret_cast<const char *>(z);
-    uint4 *tile = tiles[wave];
+    uint4 *tile = tiles[SHARED ? 0 : wave];
     Pack16 in[STEPS];
     {
         // transposed: output row (i, j) is computed from row (j, i) of z, stored [rows_j, rows_i, c_z]; the walk
         // over consecutive output rows then steps through z with stride rows_i rows
-        uint32_t r = row0 + grp * STEPS;
+        uint32_t r = row0 + first_row;
         uint32_t i = transposed ? r / ncol : 0, j = transposed ? r % ncol : 0;
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
             uint32_t src = transposed ? j * nrow_i + i : r;
-            src = grp * STEPS + s < (int)count ? src : 0;
+            src = first_row + s < (int)count ? src : 0;
             in[s].u = *reinterpret_cast<const uint4 *>(zbytes + (src * (2u * CZ) + 16u * sub));
             ++r;
             if (++j == ncol) {
@@ -263,7 +266,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
     }
     // weight fragments, heads as MFMA rows (rows >= H are zero): lane (head, g) holds w[head][16 ks + 8 g .. + 8]
     kutacc_dev::bf16x8 wf[8];
-    {
+    if (!SHARED || wave == 0) {
         const int head = lane & 31, g = lane >> 5;
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) {
@@ -276,7 +279,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
     }
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
-        const int row_local = grp * STEPS + s;
+        const int row_local = first_row + s;
         const uint32_t r = row0 + row_local;
         float v[8];
 #pragma unroll
@@ -296,7 +299,13 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
         }
         tile[((row_local >> 5) * 2 + (sub >> 3)) * 256 + kutacc_dev::panel_slot(row_local & 31, sub & 7)] = o.u;
     }
-    // the tile is private to the wave and LDS operations of a wave complete in order: no barrier
+    if constexpr (SHARED) {
+        __syncthreads();
+        if (wave != 0) {
+            return;
+        }
+    }
+    // otherwise the tile is private to the wave and LDS operations of a wave complete in order: no barrier
     const int col = lane & 31, g = lane >> 5;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
@@ -553,18 +562,21 @@ int launch_pair_bias(const void *z, const float *gamma, const float *beta, const
     if (sizeof(T) == 2 && c_z == 128 && (nheads == 4 || nheads == 8) && rows <= PAIR_BIAS_MAX_ROWS &&
         (reinterpret_cast<uintptr_t>(z) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(z_norm)) % 16 == 0) {
         const int64_t wave_tiles = fragments != nullptr ? (int64_t)32 * frag_nb * frag_nb : (rows + PAIR_BIAS_ROWS_PER_WAVE - 1) / PAIR_BIAS_ROWS_PER_WAVE;
-        const int64_t nblk = (wave_tiles + 3) / 4;
+        // Up to one unit a SIMD.  Triangle attention, whole block, a wave a unit against four (us): 48 residues 14.9 and 13.7, 77 17.8 and 16.8, 96
+        // 19.2 and 17.5, 128 21.2 and 20.0, 160 (800 units) 32.6 and 30.6; beyond, 200 41.7 and 41.5, 256 45.5 and 45.4; MSA rows 32 x 64 20.1 and 18.9.
+        const bool shared = wave_tiles <= 4 * (int64_t)kutacc_cu_count();
+        const int64_t nblk = shared ? wave_tiles : (wave_tiles + 3) / 4;
         if (nblk > INT32_MAX) {
             return KUTACC_HIP_EUNSUPPORTED;
         }
+        const auto launch = [&](auto kernel) {
+            kernel<<<(unsigned)nblk, 256, 0, stream>>>((const bf16_t *)z, gamma, beta, (const bf16_t *)w, (bf16_t *)nb, (bf16_t *)z_norm, rows, eps, rows_i,
+                                                       rows_j, transposed, (uint4 *)fragments, frag_nb, frag_nt, frag_tiles);
+        };
         if (nheads == 4) {
-            pair_bias_bf16_kernel<4><<<(unsigned)nblk, 256, 0, stream>>>((const bf16_t *)z, gamma, beta, (const bf16_t *)w,
-                                                                        (bf16_t *)nb, (bf16_t *)z_norm, rows, eps, rows_i, rows_j,
-                                                                        transposed, (uint4 *)fragments, frag_nb, frag_nt, frag_tiles);
+            shared ? launch(pair_bias_bf16_kernel<4, true>) : launch(pair_bias_bf16_kernel<4, false>);
         } else {
-            pair_bias_bf16_kernel<8><<<(unsigned)nblk, 256, 0, stream>>>((const bf16_t *)z, gamma, beta, (const bf16_t *)w,
-                                                                        (bf16_t *)nb, (bf16_t *)z_norm, rows, eps, rows_i, rows_j,
-                                                                        transposed, (uint4 *)fragments, frag_nb, frag_nt, frag_tiles);
+            shared ? launch(pair_bias_bf16_kernel<8, true>) : launch(pair_bias_bf16_kernel<8, false>);
         }
         return kutacc_hip_status(hipGetLastError());
     }

@@ -100,6 +100,32 @@ def test_pair_bias_transposed_equals_pair_bias_of_the_swapped_tensor(torch_cuda,
     assert helpers.same_bits(res[0][0], res[1][0]) and helpers.same_bits(res[0][1], res[1][1])
 
 
+@pytest.mark.parametrize("n_i,n_j,heads", [(1, 1, 4), (5, 7, 8), (33, 31, 4), (64, 512, 8), (1024, 32, 4)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_pair_bias_of_few_rows_equals_that_of_many(torch_cuda, n_i, n_j, heads, transposed):
+    """Few rows of z are shared by the waves of a workgroup (up to 1024 units of 32 on 256 CUs: the last two sizes are the most), many are not:
+    the same bits for the rows that both have."""
+    torch = torch_cuda
+    more = n_i + 33000 // n_j + 1
+    g = torch.Generator(device="cuda").manual_seed(17)
+    z = torch.randn(more, n_j, 128, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(heads, 128, device="cuda", generator=g) / math.sqrt(128)).to(torch.bfloat16)
+    gamma = torch.rand(128, device="cuda", generator=g) + 0.5
+    beta = torch.randn(128, device="cuda", generator=g) * 0.1
+    L = capi.lib()
+    res = []
+    for rows in (n_i, more):
+        src = z[:rows].transpose(0, 1).contiguous() if transposed else z[:rows].contiguous()
+        nb = torch.full((heads, rows, n_j), 7.0, dtype=torch.bfloat16, device="cuda")
+        zn = torch.full((rows, n_j, 128), 7.0, dtype=torch.bfloat16, device="cuda")
+        fn = L.kutacc_hip_pair_bias_transposed if transposed else L.kutacc_hip_pair_bias
+        assert fn(src.data_ptr(), gamma.data_ptr(), beta.data_ptr(), w.data_ptr(), nb.data_ptr(), zn.data_ptr(), rows, n_j, 128, heads, 1e-5,
+                  capi.K_BF16, None) == 0
+        torch.cuda.synchronize()
+        res.append((nb, zn))
+    assert helpers.same_bits(res[0][0], res[1][0][:, :n_i].contiguous()) and helpers.same_bits(res[0][1], res[1][1][:n_i])
+
+
 # ---- the block ---------------------------------------------------------------------------------------------------
 @pytest.fixture(params=["fused", "separate"])
 def layernorm_placement(request):
