@@ -48,7 +48,6 @@ using namespace kutacc_dev;
 namespace {
 
 constexpr int HEAD = 32;            // head_size the MFMA kernels are written for
-constexpr int WEIGHT_LOADS_IN_FLIGHT = 8; // per wave, while the weight fragments of a head are copied into LDS
 constexpr int MAX_WAVES = 12;       // fused_head_kernel: 768 threads, 3 waves per SIMD, 168 VGPRs each
 constexpr int FAIR_SLICE_SHIFT = 11;  // log2 of the clocks a wave keeps one issue priority (timeslice_priority); 2^8 to 2^13 measured alike
 constexpr float RESCALE_GAP = 5.5f; // running max may lag the true max by this much (natural log units, ~8 octaves)
@@ -871,39 +870,30 @@ __device__ inline void stage_weight_fragments(uint4 *lds_w, uint4 *own, const Fu
     }
 }
 
-// The same in whole lines, eight rows by 64 channels a copy: in fragment order, a 16-byte piece of another row in every
-// lane, a load takes the address path 42 cycles instead of 16, and a workgroup of one unit waits for them all.  Lane l's place of
-// fragment ks is weight_slot(l, ks), so that eight pieces of two rows go to 16 bank groups.
-__device__ inline int weight_slot(int lane, int ks) { return lane ^ (4 * (ks & 3) + 2 * (lane >> 5)); }
+// The same in whole lines, eight rows by 64 channels a copy (in fragment order, a 16-byte piece of another row in every
+// lane, a load takes the address path 42 cycles instead of 16, and a workgroup of one unit waits for them all), straight into the LDS: no
+// registers, all copies of a wave on their way at once.  Through registers, most copies one after the other, the weights of 77 residues took 1.6 us of
+// that kernel's 7; with this and a wave's rows asked for before them the whole block takes 16.05 us, 16.8 before, 96 residues 17.5 and 16.9, 420 164 and
+// 160.5, 512 216 and 212; with 256 channels nothing to 2 %.  A matrix lies as panels of 32 rows x 64 channels (panel_slot); complete when the wave's
+// loads are and behind a barrier.
+__device__ inline int weight_slot(int lane, int ks) { return (ks >> 2) * 256 + (panel_slot(lane & 31, lane >> 5) ^ (2 * (ks & 3))); }
 template <int C>
 __device__ inline void stage_weight_lines(uint4 *lds_w, const FusedParams &p, int first, int count, int h, int wave, int nwaves, int lane)
 {
     constexpr int CK = C / 16;
-    const int nfrag = count * CK, q = lane & 7;
-    auto line = [&](int f) {
+    const uint32_t to = (uint32_t)(uintptr_t)(const lds_char *)reinterpret_cast<char *>(lds_w);
+    const int rl = lane >> 3;
+    uint32_t lane_bytes[2]; // rows 16 - 31 of a panel swizzle with bit 0 flipped
+#pragma unroll
+    for (int hi = 0; hi < 2; ++hi) {
+        lane_bytes[hi] = 2u * (uint32_t)(rl * C + 8 * ((lane & 7) ^ rl ^ hi));
+    }
+    for (int f = wave; f < count * CK; f += nwaves) {
         const int m = first + f / CK, k = f % CK;
         const bf16_t *w = m == 0 ? p.w[0] : m == 1 ? p.w[1] : m == 2 ? p.w[2] : p.w[3];
-        return *reinterpret_cast<const uint4 *>(w + (int64_t)(h * HEAD + 8 * (k & 3) + (lane >> 3)) * C + (k >> 2) * 64 + q * 8);
-    };
-    auto put = [&](int f, uint4 v) {
-        const int row = 8 * (f & 3) + (lane >> 3), ks0 = f & ~3; // CK is a multiple of 4
-        lds_w[(ks0 + (q >> 1)) * 64 + weight_slot(32 * (q & 1) + row, q >> 1)] = v;
-    };
-    int f = wave;
-    for (; f + (WEIGHT_LOADS_IN_FLIGHT - 1) * nwaves < nfrag; f += WEIGHT_LOADS_IN_FLIGHT * nwaves) {
-        uint4 t[WEIGHT_LOADS_IN_FLIGHT];
-#pragma unroll
-        for (int k = 0; k < WEIGHT_LOADS_IN_FLIGHT; ++k) {
-            t[k] = line(f + k * nwaves);
-        }
-#pragma unroll
-        for (int k = 0; k < WEIGHT_LOADS_IN_FLIGHT; ++k) {
-            put(f + k * nwaves, t[k]);
-        }
+        load_to_lds(to + f * 1024u, w + (int64_t)(h * HEAD + 8 * (k & 3)) * C + (k >> 2) * 64, k & 2 ? lane_bytes[1] : lane_bytes[0]);
     }
-    for (; f < nfrag; f += nwaves) {
-        put(f, line(f));
-    }
+    wait_for_loads<0>();
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -996,10 +986,23 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
             __syncthreads(); // previous group's fragments are no longer being read
         } else {
         }
+        // One block a wave: its rows and its gate's bias are asked for in front of the weights, one round trip for all (with 256 channels, columns of
+        // 500 sequences x 100 lose 1.8 % by it).
+        constexpr bool EARLY = BPW == 1 && C == 128;
+        PanelRegs early[EARLY ? CK / 4 : 1];
+        f32x4 early_bg[EARLY ? 4 : 1];
+        if constexpr (EARLY) {
+#pragma unroll
+            for (int c = 0; c < CK / 4; ++c) {
+                early[c] = panel_load(p.x + (int64_t)b * p.x_sb, p.x_ld, min(wave, NB - 1) * 32, S - 1, c * 64, lane);
+            }
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                early_bg[a] = *reinterpret_cast<const f32x4 *>(p.bg + h * HEAD + 4 * g + 8 * a);
+            }
+        }
         stage_weight_lines<C>(lds_w, p, pass * GW, GW, h, wave, NW, lane);
         __syncthreads();
-        if (pi == 0) {
-        }
         if constexpr (C == 128 && BPW >= 3) {
             // Two blocks of the wave per walk over the weight fragments: the input fragments of both stay in registers
             // (64 of them) and every fragment of the weights is read from LDS once for the pair (1 KB per MFMA when the
@@ -1051,7 +1054,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
                     acc[0] = zero16(), acc[1] = zero16();
 #pragma unroll
                     for (int ks = 0; ks < CK; ++ks) {
-                        const bf16x8 wf = as_bf16x8(wsrc[ks * 64 + weight_slot(lane, ks)]);
+                        const bf16x8 wf = as_bf16x8(wsrc[weight_slot(lane, ks)]);
 #pragma unroll
                         for (int n = 0; n < PAIR; ++n) {
                             // V[s][d]: rows = sequence positions; the others W_h . x^T: rows = head-dim
@@ -1117,14 +1120,20 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
                 }
                 const uint4 *fsrc = prow < 16 ? kslot : vslot;
                 const int srow8 = lane >> 3, chunk = lane & 7;
-                PanelRegs t = panel_load(xb, p.x_ld, j * 32, S - 1, 0, lane);
+                PanelRegs t;
+                if constexpr (!EARLY) {
+                    t = panel_load(xb, p.x_ld, j * 32, S - 1, 0, lane);
+                }
 #pragma unroll
                 for (int c = 0; c < CK / 4; ++c) {
+                    if constexpr (EARLY) {
+                        t = early[c];
+                    }
                     kslot[panel_slot(srow8, chunk)] = t.r0;
                     kslot[panel_slot(srow8 + 8, chunk)] = t.r1;
                     vslot[panel_slot(srow8 + 16, chunk)] = t.r2;
                     vslot[panel_slot(srow8 + 24, chunk)] = t.r3;
-                    if (c + 1 < CK / 4) {
+                    if (!EARLY && c + 1 < CK / 4) {
                         t = panel_load(xb, p.x_ld, j * 32, S - 1, (c + 1) * 64, lane);
                     }
 #pragma unroll
@@ -1149,7 +1158,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
                     // V[s][d]: rows = sequence positions, so a lane ends up with 16 keys of one head-dim
 #pragma unroll
                     for (int ks = 0; ks < CK; ++ks) {
-                        acc = mfma(xf[ks], as_bf16x8(wsrc[ks * 64 + weight_slot(lane, ks)]), acc);
+                        acc = mfma(xf[ks], as_bf16x8(wsrc[weight_slot(lane, ks)]), acc);
                     }
                     if constexpr (V_ALIAS) {
                         vpark[i][0] = as_uint4(pack8(acc, 0));
@@ -1162,7 +1171,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
                     // W_h . x^T: rows = head-dim, columns = sequence positions
 #pragma unroll
                     for (int ks = 0; ks < CK; ++ks) {
-                        acc = mfma(as_bf16x8(wsrc[ks * 64 + weight_slot(lane, ks)]), xf[ks], acc);
+                        acc = mfma(as_bf16x8(wsrc[weight_slot(lane, ks)]), xf[ks], acc);
                     }
                     if (m == PROJ_K) {
                         lds_k[(j * 2 + 0) * 64 + lane] = as_uint4(pack8(acc, 0));
@@ -1178,7 +1187,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
                         const float *bgp = p.bg + h * HEAD + 4 * g;
 #pragma unroll
                         for (int a = 0; a < 4; ++a) {
-                            const f32x4 bv = *reinterpret_cast<const f32x4 *>(bgp + 8 * a);
+                            const f32x4 bv = EARLY ? early_bg[EARLY ? a : 0] : *reinterpret_cast<const f32x4 *>(bgp + 8 * a);
 #pragma unroll
                             for (int c = 0; c < 4; ++c) {
                                 acc[4 * a + c] = sigmoid_fast(acc[4 * a + c] + bv[c]);
