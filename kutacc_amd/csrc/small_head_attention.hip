@@ -11,7 +11,8 @@
 //   * p.v with 16x16x32 MFMAs of 32 keys whose rows are the eight values and ones, which give the sums of the probabilities.
 // K, V and masks of a head's four rows lie in the LDS for the whole workgroup (128 bytes per key and 16 of masks).
 // Measured on 1024 rows x 301 keys x 8 heads: 505 us on the general attention_tiles_kernel, 177 to 189 us here behind a pass that
-// projects, 168 to 204 from card to card with the projections inside (vector issue 73 %).  With the queries and the masks in two parts (16 bits, an error of up to 8 % in a probability at logits of 11 000) and 32x32x16 products it was 199.
+// projects, 168 to 204 from card to card with the projections inside (vector issue 73 %), 4 to 8 % less of them with the bias's rows, which start on any
+// address, brought into the lanes' order by a pass of its own (seed_tiles_kernel).  With the queries and the masks in two parts (16 bits, an error of up to 8 % in a probability at logits of 11 000) and 32x32x16 products it was 199.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -35,6 +36,7 @@ struct SmallHeadParams {
     // ... and its queries and gates: of a set and head [row][tile][queries, gates][64 lanes] of 8 bytes, in one of three of the scratch tensors
     uint2 *stash[3];
     int stash_each; // sets and heads per tensor
+    f32x4 *tiles;   // pair bias, where it has been put in the logits' order (seed_tiles_kernel): [head][query block][key tile][4][64 lanes]
     const bf16_t *x, *wq, *wk, *wv, *wg; // the kernel that projects: input rows of 64 channels, weights
     const float *bg;
     int64_t x_ss;
@@ -48,7 +50,35 @@ struct SmallHeadParams {
 // four accumulator rows of both halves are eight consecutive keys, the chunk of p.v's k-slots that the lane supplies
 __device__ __forceinline__ int key_slot(int i) { return 16 * ((i >> 2) & 1) + 4 * (i >> 3) + (i & 3); }
 
-template <bool HAS_NB, bool PROJECTS>
+// The seeds of the logits of all batch rows: the pair bias in log2 units, -inf past the last key, tile by tile as the lanes hold them,
+// pieces 2 u + a of query half u and key half a.  5 us with the launch; 4 KB a tile instead of 2 in the attention's loop, but whole lines and no
+// conversion (a seventh of its vector instructions).
+__global__ __launch_bounds__(256) void seed_tiles_kernel(const SmallHeadParams p)
+{
+    const int lane = threadIdx.x & 63, n = lane & 15, c = lane >> 4;
+    const int tile = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), t = tile % p.NB, j = tile / p.NB % p.NB, h = tile / (p.NB * p.NB);
+    if (h >= p.H) {
+        return;
+    }
+    f32x4 *to = p.tiles + (int64_t)tile * 256 + lane;
+    const int key0 = 32 * t + 8 * c;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int query = min(32 * j + 16 * u + n, p.S - 1);
+        const bf16x8 raw = as_bf16x8(load8_checked(p.nb + (int64_t)h * p.nb_sh + (uint32_t)query * (uint32_t)p.nb_sq, min(key0, p.S), p.S));
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = key0 + 4 * a + e < p.S ? to_f32(raw[4 * a + e]) * LOG2E : -INFINITY;
+            }
+            to[(2 * u + a) * 64] = v;
+        }
+    }
+}
+
+template <bool HAS_NB, bool PROJECTS, bool TILES>
 __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const SmallHeadParams p)
 {
     extern __shared__ uint4 lds[];
@@ -324,7 +354,7 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
                 const bf16x8 k = as_bf16x8(ks[t * TILE + i * 32 + a * 16 + n]);
                 f32x4 c0 = C.x[0][a], c1 = C.x[1][a];
                 if constexpr (decltype(masked)::value) {
-                    const f32x4 m = *reinterpret_cast<const f32x4 *>(masks + t * TILE + i * 32 + 8 * c + 4 * a);
+                    const f32x4 m = *reinterpret_cast<const f32x4 *>(masks + t * TILE + i * 32 + 8 * (TILES ? lv >> 4 : c) + 4 * a);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         c0[e] += m[e], c1[e] += m[e];
@@ -359,7 +389,7 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         // Two rows in flight: the logits of one are in the matrix pipe while the other's exponentials run.  The fences keep
         // it at two: left to itself the compiler starts all four and needs registers for two waves per SIMD only.
         auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
-        auto rows = [&](int t, const Tile &C, auto masked) __attribute__((always_inline)) {
+        auto rows = [&](int t, Tile &C, auto masked, auto reload) __attribute__((always_inline)) {
             Tile xa = logits(0, t, C, masked);
             fence();
             Tile xb = logits(1, t, C, masked);
@@ -369,38 +399,70 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
             finish(1, t, xb, unshifted, std::false_type{});
             fence();
             xb = logits(3, t, C, masked);
+            reload();
             finish(2, t, xa, unshifted, std::false_type{});
             fence();
             finish(3, t, xb, unshifted, std::false_type{});
             fence();
         };
-        // Tiles without a mask, tiles with one, and the ragged last one, each in a loop of its own: with their choice inside one loop
-        // a tile cost 76 vector instructions and 16 moves of register pairs more than the 160 that it needs (the whole operator, us: 1024
-        // rows of 301 237 -> 221, 1000 of 420 432 -> 381).
-        const int full = S >> 5, plain = min(masked_from, full);
-        Raw raw = {zero_u4(), zero_u4()};
-        if (S >= 8) {
-            raw = load_nb(0);
-        }
-        auto run = [&](int from, int to, auto masked) __attribute__((always_inline)) {
-            for (int t = from; t < to; ++t) {
-                const Tile C = seeds(raw, std::false_type{});
-                raw = load_nb(t + 1);
-                rows(t, C, masked);
+        const f32x4 *tiles = TILES ? p.tiles + (int64_t)(h * NB + j) * NB * 256 : nullptr;
+        auto load_tile = [&](int t) {
+            Tile s;
+            const char *from = reinterpret_cast<const char *>(tiles + min(t, NB - 1) * 256); // uniform; the lane's part in 32 bits
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s.x[i >> 1][i & 1] = *reinterpret_cast<const f32x4 *>(from + (16u * (uint32_t)lv + 1024u * i));
             }
+            return s;
         };
-        run(0, plain, std::false_type{});
-        run(plain, full, std::true_type{});
-        if (full < NB) {
-            if constexpr (HAS_NB) {
-                if (S >= 8) {
-                    const int drop = min(max(32 * full + 8 * c - (S - 8), 0), 8);
-                    raw.r[0] = drop_first(raw.r[0], drop), raw.r[1] = drop_first(raw.r[1], drop);
-                } else {
-                    raw = load_tail();
+        const int full = S >> 5;
+        if constexpr (TILES) {
+            Tile C0 = load_tile(0), C1 = load_tile(1);
+            auto run = [&](int from, int to, auto masked) __attribute__((always_inline)) {
+                int t = from;
+                for (; t + 1 < to; t += 2) {
+                    rows(t, C0, masked, [&] { C0 = load_tile(t + 2); });
+                    rows(t + 1, C1, masked, [&] { C1 = load_tile(t + 3); });
                 }
+                if (t < to) {
+                    rows(t, C0, masked, [&] { C0 = load_tile(t + 2); });
+                    const Tile swap = C0;
+                    C0 = C1, C1 = swap;
+                }
+            };
+            const int plain = min(masked_from, NB);
+            run(0, plain, std::false_type{});
+            run(plain, NB, std::true_type{});
+        } else {
+            // Tiles without a mask, tiles with one, and the ragged last one, each in a loop of its own: with their choice inside one loop
+            // a tile cost 76 vector instructions and 16 moves of register pairs more than the 160 that it needs (the whole operator, us: 1024
+            // rows of 301 237 -> 221, 1000 of 420 432 -> 381).
+            const int plain = min(masked_from, full);
+            Raw raw = {zero_u4(), zero_u4()};
+            if (S >= 8) {
+                raw = load_nb(0);
             }
-            rows(full, seeds(raw, std::true_type{}), std::true_type{});
+            auto run = [&](int from, int to, auto masked) __attribute__((always_inline)) {
+                for (int t = from; t < to; ++t) {
+                    Tile C = seeds(raw, std::false_type{});
+                    raw = load_nb(t + 1);
+                    rows(t, C, masked, [] {});
+                }
+            };
+            run(0, plain, std::false_type{});
+            run(plain, full, std::true_type{});
+            if (full < NB) {
+                if constexpr (HAS_NB) {
+                    if (S >= 8) {
+                        const int drop = min(max(32 * full + 8 * c - (S - 8), 0), 8);
+                        raw.r[0] = drop_first(raw.r[0], drop), raw.r[1] = drop_first(raw.r[1], drop);
+                    } else {
+                        raw = load_tail();
+                    }
+                }
+                Tile C = seeds(raw, std::true_type{});
+                rows(full, C, std::true_type{}, [] {});
+            }
         }
         // the two query halves side by side: lane l then has values 4 (l / 16 % 2) .. + 3 of query 16 (l / 32) + l % 16
         int le = lane;
@@ -431,7 +493,13 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
             if (__any(!(l > 1e-30f && l < 1e30f))) {
                 // Some probability overflowed or a whole row underflowed (every key masked: -1e9 log2(e) everywhere, which is
                 // finite): the row's true maxima first, then the probabilities with them subtracted.
-                auto again = [&](int t) { return logits(i, t, t < full ? seeds(load_nb(t), std::false_type{}) : seeds(load_tail(), std::true_type{}), std::true_type{}); };
+                auto again = [&](int t) {
+                    if constexpr (TILES) {
+                        return logits(i, t, load_tile(t), std::true_type{});
+                    } else {
+                        return logits(i, t, t < full ? seeds(load_nb(t), std::false_type{}) : seeds(load_tail(), std::true_type{}), std::true_type{});
+                    }
+                };
                 float mx[2] = {-INFINITY, -INFINITY};
                 for (int t = 0; t < NB; ++t) {
                     const Tile x = again(t);
@@ -474,12 +542,12 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
 
 size_t lds_bytes(int NB) { return (size_t)(2 * NB + 1) * TILE * 16 + (size_t)(TILE * NB + 1) * 4; }
 
-template <bool HAS_NB, bool PROJECTS>
+template <bool HAS_NB, bool PROJECTS, bool TILES = false>
 int launch(SmallHeadParams p, hipStream_t stream)
 {
     static size_t configured[KUTACC_DEVICE_SLOTS] = {};
     const size_t lds = lds_bytes(p.NB);
-    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&small_head_attention_kernel<HAS_NB, PROJECTS>), lds, configured)) {
+    if (const hipError_t e = kutacc_opt_in_lds(reinterpret_cast<const void *>(&small_head_attention_kernel<HAS_NB, PROJECTS, TILES>), lds, configured)) {
         return kutacc_hip_status(e);
     }
     // Four waves while three workgroups' keys fit a CU (the registers' limit of 12 waves), else eight.  A number that is no
@@ -489,7 +557,10 @@ int launch(SmallHeadParams p, hipStream_t stream)
     const int turns = (p.NB + waves - 1) / waves, room = 2 * kutacc_cu_count() / std::max(1, p.sets * p.H);
     p.splits = std::max(1, std::min(turns, room));
     const int64_t blocks = (int64_t)(p.sets + 7) / 8 * 8 * p.H * p.splits;
-    small_head_attention_kernel<HAS_NB, PROJECTS><<<dim3((unsigned)blocks), 64 * waves, lds, stream>>>(p);
+    if constexpr (TILES) {
+        seed_tiles_kernel<<<dim3((unsigned)((p.H * p.NB * p.NB + 3) / 4)), 256, 0, stream>>>(p);
+    }
+    small_head_attention_kernel<HAS_NB, PROJECTS, TILES><<<dim3((unsigned)blocks), 64 * waves, lds, stream>>>(p);
     return kutacc_hip_status(hipGetLastError());
 }
 } // namespace
@@ -564,6 +635,19 @@ int small_head_attention(const kutacc_hip_attention_args_t &a, bool projects, hi
     p.wq = (const bf16_t *)a.query_w, p.wk = (const bf16_t *)a.key_w, p.wv = (const bf16_t *)a.value_w, p.wg = (const bf16_t *)a.gating_w;
     p.bg = a.gating_b;
     p.stash[0] = (uint2 *)a.q, p.stash[1] = (uint2 *)a.k, p.stash[2] = (uint2 *)a.gate, p.stash_each = (int)stash_capacity(a);
+    // The seeds as a pass of their own, behind the last stash where there is room for them: where the bias's rows start on any address, as they do
+    // at seven lengths of eight -- the kernel's loads of them then cross lines --, and where sets and tiles pay for the pass.  Operator, us, bias read
+    // in the kernel against this: 1024 rows of 301 171.5 164, of 253 122 118, of 381 240 235, 5120 of 127 274 254, 2000 of 199 196 186.5, of 319 438 330,
+    // 600 of 251 79.8 79.3; below the line 300 of 301 70.3 69.9, 256 of 317 57.6 59.0, 400 of 219 58.1 58.4, 1024 of 94 43.2 45.5.  Rows on 16 bytes gain
+    // nothing: 2000 of 320 327 329, 600 of 256 75.6 79.
+    const int64_t units = (int64_t)p.sets * p.H, last = std::max<int64_t>(0, units - 2 * (int64_t)p.stash_each), unit_bytes = (int64_t)ROWS * p.NB * 1024;
+    char *const gate = (char *)a.gate, *const seeds = (char *)(((uintptr_t)gate + (uintptr_t)(last * unit_bytes) + 15) / 16 * 16);
+    const int64_t seed_bytes = (int64_t)p.H * p.NB * p.NB * 4096, room = gate + a.batch * a.seq_len * a.nheads * D * 2 - seeds;
+    const bool any_address = !kutacc_hip_aligned16(p.nb) || p.nb_sh % 8 != 0 || p.nb_sq % 8 != 0;
+    if (p.nb && any_address && (int64_t)p.sets * p.NB * p.NB >= 7500 && seed_bytes <= room) {
+        p.tiles = (f32x4 *)seeds;
+        return launch<true, true, true>(p, stream);
+    }
     return p.nb ? launch<true, true>(p, stream) : launch<false, true>(p, stream);
 }
 
