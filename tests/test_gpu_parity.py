@@ -16,7 +16,7 @@ import numpy as np
 import pytest
 
 from kutacc_amd import capi
-from kutacc_amd.workloads import CONFIGS, Workload, bf16_bits, make_workload, round_to_bf16
+from kutacc_amd.workloads import CONFIGS, MASK_BIAS, Workload, bf16_bits, make_workload, round_to_bf16
 
 import helpers
 from test_gpu_tiled_attention import draw_workload
@@ -915,3 +915,28 @@ def test_pair_bias_producer_matches_oracle(torch_cuda, config):
     nb_ref = nb_ref.reshape(S, S, H).transpose(2, 0, 1)
     helpers.assert_within(helpers.to_numpy(zn), zn_ref, tol(zn_ref), "normalised z")
     helpers.assert_within(helpers.to_numpy(nb), nb_ref, tol(nb_ref), "pair bias")
+
+
+@pytest.mark.parametrize("B,S,heads", [(6, 130, 4), (5, 161, 4), (4, 191, 4), (3, 225, 4), (2, 353, 4), (4, 383, 4), (4, 129, 8), (3, 191, 8), (2, 223, 8), (4, 255, 8)])
+def test_two_row_kernel_at_ragged_lengths_without_a_mask(torch_cuda, B, S, heads):
+    """Keys past the end stand in the tiles of the pair bias, so that rows without a mask take the loop without one: odd and even numbers of
+    tiles, one key past a tile and one short of it; a row with a mask, and one masked throughout, beside them."""
+    torch = torch_cuda
+    assert capi.set_tuning("row_pairs", "1") == 0
+    try:
+        for masked_rows in ((), (1,), (0, B - 1)):
+            w = draw_workload(8100 + S, B, S, heads, 32, masked=0.0, nb_scale=3.0)
+            for i, b in enumerate(masked_rows):
+                w.bias[b, S // 2 if i == 0 else 0:] = MASK_BIAS
+            w.bias = round_to_bf16(w.bias)
+            w.x[:, S - 1] *= 4  # the last row is the one that the keys past the end repeat
+            w.x = round_to_bf16(w.x)
+            op, ten, scratch = helpers.make_op(w)
+            names = helpers.profiled_kernels(torch, op.run)
+            torch.cuda.synchronize()
+            assert not capi.error_flag() and "persistent_pair_kernel" in names, names
+            ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
+            helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), ref_avg, "bf16", "gated average")
+            helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, "bf16", "out")
+    finally:
+        capi.set_tuning("row_pairs", None)
