@@ -139,14 +139,13 @@ __device__ __forceinline__ float one_mask_of(const float *mask, int S, int lane)
 }
 
 // Mask bias of one batch row -> LDS as fp32 (keys past S get -inf), plus one flag bit per 32-key tile
-// saying "this tile needs the mask added" (non-zero bias or ragged tail).  Wave w covers keys
+// saying "this tile needs the mask added" (non-zero bias or ragged tail; keys from `flagged` on set none).  Wave w covers keys
 // [64w, 64w+64); *flag_word must have been zeroed before, with a barrier in between.
 // bias_row[k * stride_k] is the mask bias itself, or (from_mask) the 0/1 mask, turned into 1e9*(mask-1) here with the
 // same multiply-add and bf16 rounding as the stand-alone mask-bias pass.
 template <bool NEAR = false> // NEAR: S * stride_k < 2^31 and stride_k < 2^24 (checked on the host), 32-bit offsets
 __device__ __forceinline__ void stage_mask_part(const bf16_t *bias_row, float *mask, uint32_t *flag_word, int S, int NB,
-                                                int wave, int lane, float scale = 1.0f, int64_t stride_k = 1,
-                                                bool from_mask = false)
+                                                int flagged, int wave, int lane, float scale, int64_t stride_k, bool from_mask)
 {
     const int k = wave * 64 + lane;
     if (wave * 64 < NB * 32) {
@@ -161,7 +160,7 @@ __device__ __forceinline__ void stage_mask_part(const bf16_t *bias_row, float *m
         if (k < NB * 32) {
             mask[k] = mv;
         }
-        const unsigned long long nz = __ballot(k < NB * 32 && mv != 0.f);
+        const unsigned long long nz = __ballot(k < flagged && mv != 0.f);
         const uint32_t bits = (((uint32_t)nz != 0u ? 1u : 0u) | ((uint32_t)(nz >> 32) != 0u ? 2u : 0u)) << (2 * wave);
         if (lane == 0 && bits != 0u) {
             atomicOr(flag_word, bits);
@@ -1223,7 +1222,8 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
         if (part * 64 < NT * 32) {
             const float mv = mask_bias_finish(mask_raw[q], part * 64 + lane < S, l2mode ? LOG2E : 1.0f, p.bias_is_mask != 0);
             mask[part * 64 + lane] = mv;
-            const unsigned long long nz = __ballot(mv != 0.f);
+            // (in log2 units the copies of the pair bias take keys past the end out by themselves)
+            const unsigned long long nz = __ballot(mv != 0.f && (part * 64 + lane < S || !HAS_NB || !l2mode));
             const bool differ = ONE_PASS && __any(part * 64 + lane < S && (mv == 0.f || mv != __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(mv)))));
             if (lane == 0) {
                 part_flags[part] = ((uint32_t)nz != 0u ? 1u : 0u) | ((uint32_t)(nz >> 32) != 0u ? 2u : 0u) | (differ ? 4u : 0u);
@@ -1277,8 +1277,8 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
             const uint4 *nbf = HAS_NB ? p.nbf + ((int64_t)(h * NB + j) * NT * (TILES ? 4 : 2)) * 64 + lane : nullptr;
             bool again = true; // some probability overflowed or a whole row underflowed
             if (!ONE_PASS || flags != ONE_MASK) {
-                if (!ODD && flags == 0u) { // (the tile of zeros behind an odd number has a mask)
-                    attend_block_l2<HAS_NB, false, false, TILES>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel,
+                if ((HAS_NB || !ODD) && flags == 0u) { // (without a pair bias the tile of zeros behind an odd number has a mask)
+                    attend_block_l2<HAS_NB, false, false, TILES, ODD>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel,
                                                           NT, lane, 0.f, o, l, (wave >> 2) & 1);
                 } else {
                     attend_block_l2<HAS_NB, true, false, TILES, ODD>(lds_k, lds_v, mask4, nbf, qf[i][0], qf[i][1], as_f16x8(selw0), as_f16x8(selw1), sumsel,
@@ -1397,7 +1397,8 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_head_kernel(F
         // loop, where there is no register for them -- spilled, each costs a scratch round trip per batch row.
         int lane_x = lane;
         asm volatile("" : "+v"(lane_x));
-        stage_mask_part<true>(p.bias + (int64_t)b * p.bias_sb, mask, flag_word, S, NT, wave, lane_x, mask_scale, p.bias_sk,
+        // (in log2 units the copies of the pair bias take keys past the end out by themselves)
+        stage_mask_part<true>(p.bias + (int64_t)b * p.bias_sb, mask, flag_word, S, NT, HAS_NB && L2MODE ? S : NT * 32, wave, lane_x, mask_scale, p.bias_sk,
                               p.bias_is_mask != 0);
 
         // ---- input rows of the block -> fragments, 64 channels per staging panel ----
@@ -1575,8 +1576,8 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_head_kernel(F
         const bf16_t *nb_head = HAS_NB ? p.nb + (int64_t)h * p.nb_sh : nullptr;
         if constexpr (L2MODE) {
             const uint4 *nbf = HAS_NB ? p.nbf + ((int64_t)(h * NB + j) * NT * (TILES ? 4 : 2)) * 64 + lane : nullptr;
-            if (!ODD && flags == 0u) { // (the tile of zeros behind an odd number has a mask)
-                attend_block_l2<HAS_NB, false, false, TILES>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
+            if ((HAS_NB || !ODD) && flags == 0u) { // (without a pair bias the tile of zeros behind an odd number has a mask)
+                attend_block_l2<HAS_NB, false, false, TILES, ODD>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
                                                       l, -1, fair_turn);
             } else {
                 attend_block_l2<HAS_NB, true, false, TILES, ODD>(lds_k, lds_v, mask4, nbf, q0, q1, sel0, sel1, sumsel, NT, lane, 0.f, o,
@@ -2517,6 +2518,13 @@ __global__ __launch_bounds__(64) void pair_bias_fragments_kernel(const bf16_t *_
     for (int e = 0; e < 4; ++e) {
         d[e] = (uint32_t)pair_bias_log2_f16(to_f32(s0[2 * e])) | ((uint32_t)pair_bias_log2_f16(to_f32(s0[2 * e + 1])) << 16);
         d[4 + e] = (uint32_t)pair_bias_log2_f16(to_f32(s1[2 * e])) | ((uint32_t)pair_bias_log2_f16(to_f32(s1[2 * e + 1])) << 16);
+    }
+    if (key0 + 16 > S) { // keys past the end: 2^-65504 is zero
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t a0 = key0 + 2 * e < S ? d[e] & 0xffffu : PAST_THE_END_F16, a1 = key0 + 2 * e + 1 < S ? d[e] & 0xffff0000u : PAST_THE_END_F16 << 16;
+            d[e] = a0 | a1;
+        }
     }
     uint4 *dst = out + ((((int64_t)h * NB + j) * NT + t) * 2) * 64 + lane;
     dst[0] = make_uint4(d[0], d[1], d[2], d[3]);

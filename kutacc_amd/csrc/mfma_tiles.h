@@ -71,6 +71,10 @@ __device__ __forceinline__ uint16_t pair_bias_log2_f16(float nb)
     return c.u;
 }
 
+// -65504: what the copies of the pair bias hold for keys past the end, so that rows of a ragged length need no mask for them (operator, us: 301 residues
+// 66.9 -> 64.8, 511 197.6 -> 194.7, 1000 1155 -> 1137)
+constexpr uint32_t PAST_THE_END_F16 = 0xfbffu;
+
 __device__ __forceinline__ f32x16 zero16()
 {
     const f32x16 z = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};

@@ -366,7 +366,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 if (4 * g + v < H) {
-                    t16[(4 * g + v) * 32 + col] = real ? kutacc_dev::pair_bias_log2_f16((float)(bf16_t)acc[v]) : (uint16_t)0;
+                    t16[(4 * g + v) * 32 + col] = real ? kutacc_dev::pair_bias_log2_f16((float)(bf16_t)acc[v]) : (uint16_t)kutacc_dev::PAST_THE_END_F16;
                 }
             }
             __builtin_amdgcn_wave_barrier(); // other lanes' stores: keep the loads below behind them
@@ -378,7 +378,8 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
                 uint4 *dst = nbf + ((((int64_t)h * frag_nb + (q >> 5)) * frag_nt + t) * 2 + (c & 1)) * 64 + qlane + 32 * (c >> 1);
                 *dst = val;
                 if (t + 1 == frag_nb && frag_nt > frag_nb) { // the phantom tile that pads the key tiles to a pair
-                    dst[128] = make_uint4(0u, 0u, 0u, 0u);
+                    const uint32_t out = kutacc_dev::PAST_THE_END_F16 * 0x10001u;
+                    dst[128] = make_uint4(out, out, out, out);
                 }
             }
         }

@@ -938,3 +938,29 @@ def test_two_row_kernel_at_ragged_lengths_without_a_mask(torch_cuda, B, S, heads
             helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, "bf16", "out")
     finally:
         capi.set_tuning("row_pairs", None)
+
+
+@pytest.mark.parametrize("B,S,heads,pairs", [(70, 35, 4, "0"), (9, 63, 4, "0"), (9, 97, 4, "0"), (10, 225, 4, "0"), (17, 354, 4, "0"), (3, 385, 4, None), (2, 479, 4, None),
+                                             (2, 1023, 4, None), (3, 673, 4, None), (6, 33, 8, "0"), (9, 222, 8, "0"), (3, 289, 8, None), (2, 703, 8, None), (2, 993, 8, None)])
+def test_one_row_kernels_at_ragged_lengths_without_a_mask(torch_cuda, B, S, heads, pairs):
+    """The same of the kernels that walk one row, on fragments and on tiles of the pair bias; holes of -inf in it among the keys that are there."""
+    torch = torch_cuda
+    assert capi.set_tuning("row_pairs", pairs) == 0
+    try:
+        for masked_rows in ((), (1,), (0, B - 1)):
+            w = draw_workload(8300 + S, B, S, heads, 32, masked=0.0)
+            w.nb[:, S // 3, S // 2:] = -np.inf
+            for i, b in enumerate(masked_rows):
+                w.bias[b, S // 2 if i == 0 else 0:] = MASK_BIAS
+            w.bias = round_to_bf16(w.bias)
+            op, ten, scratch = helpers.make_op(w)
+            op.run()
+            torch.cuda.synchronize()
+            assert not capi.error_flag() and capi.last_path() == "fused_mfma"
+            got_avg, got = helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), helpers.to_numpy(ten["out"])
+            rows = [b for b in range(B) if b != B - 1 or len(masked_rows) < 2]  # (a row masked throughout: the holes of the reference stay holes)
+            ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
+            helpers.check_close(got_avg[rows], ref_avg[rows], "bf16", "gated average")
+            helpers.check_close(got[rows], ref_out[rows], "bf16", "out")
+    finally:
+        capi.set_tuning("row_pairs", None)
