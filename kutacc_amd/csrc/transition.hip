@@ -569,15 +569,21 @@ hipError_t launch(const TransitionParams &p, int64_t c_o, hipStream_t stream)
     const double flops = 4.0 * (double)p.rows * (double)c_o * (double)p.c_i;
     // The split kernel while its workgroups of 32 rows fit one round on the chip: in a second round it takes as long as the
     // other kernel (12000 rows, 256 -> 1024: 39 and 38 us; 128 -> 512: 18 and 14).  With 64 channels all is within 7 us.
-    const bool few = c_o != 64 && (p.rows + 31) / 32 <= kutacc_cu_count();
+    const int64_t blocks = (p.rows + 31) / 32, cus = kutacc_cu_count();
+    const bool few = c_o != 64 && blocks <= cus;
+    // While eight waves a CU take all rows, they are one workgroup, which brings the weights once, in four stages or in slices of twice the size.  Against
+    // two or three workgroups (us): 256 -> 1024 40000 rows 51.6 49.7, 50000 57.3 53.0, 65000 65.3 60.8, 128 -> 512 9000 rows 13.1 12.3, 30000 14.3 13.3,
+    // 65000 22.2 19.7, 128 -> 256 20000 9.9 9.9, 50000 14.3 13.2.  Beyond, a second round of it costs: 80000 89.5 94.2, 27.6 30.9.  With 256 channels and up
+    // to four waves a CU no gain: 256 -> 1024 20000 34.1 34.0, 256 -> 512 22.0 22.5.
+    const bool one_round = blocks <= 8 * cus && (c_o == 128 || blocks > 4 * cus);
     kutacc_prof::KernelTimer t(few ? (BLOCK ? "transition_split_kernel<block>" : "transition_split_kernel")
                                    : (BLOCK ? "transition_rows_kernel<block>" : "transition_rows_kernel"),
                                flops, stream);
     if (c_o == 256) {
-        return few ? launch_split<256, BLOCK, 4>(p, stream) : launch_rows<256, BLOCK, 32, 2, 4, 2>(p, stream);
+        return few ? launch_split<256, BLOCK, 4>(p, stream) : one_round ? launch_rows<256, BLOCK, 32, 4, 8, 1>(p, stream) : launch_rows<256, BLOCK, 32, 2, 4, 2>(p, stream);
     }
     if (c_o == 128) {
-        return few ? launch_split<128, BLOCK, 4>(p, stream) : launch_rows<128, BLOCK, 32, 3, 4, 3>(p, stream);
+        return few ? launch_split<128, BLOCK, 4>(p, stream) : one_round ? launch_rows<128, BLOCK, 64, 2, 8, 1>(p, stream) : launch_rows<128, BLOCK, 32, 3, 4, 3>(p, stream);
     }
     if constexpr (BLOCK) {
         return launch_rows<64, true, 64, 2, 4, 4>(p, stream);

@@ -401,6 +401,16 @@ def test_transition_forced_paths(torch_cuda):
                                    2, 8, 8, capi.K_BF16, capi.PATH_AUTO, None) == capi.EINVAL  # needs the intermediate
 
 
+@pytest.mark.parametrize("rows,c_o,c_i", [(32769, 256, 64), (40000, 256, 192), (65536, 256, 1024), (8193, 128, 64), (20011, 128, 128), (65536, 128, 2048)])
+def test_transition_of_one_round_equals_that_of_many_rows(torch_cuda, rows, c_o, c_i):
+    """The rows that one workgroup of eight waves a CU takes (with 256 channels from 32769 on, 128 from 8193, up to 65536 on 256 CUs): the same bits as
+    among more rows, at the fewest slices and the most."""
+    c = transition_case(1500 + c_i, 1, 70000, c_o, c_i)
+    many, _ = run_transition(torch_cuda, c)
+    out, _ = run_transition(torch_cuda, dict(c, x=np.ascontiguousarray(c["x"][:, :rows])))
+    assert helpers.same_bits(out.reshape(rows, c_o), many.reshape(70000, c_o)[:rows])
+
+
 @pytest.mark.parametrize("rows,c_o,c_i", [(40, 256, 1024), (8200, 256, 64), (8200, 128, 128), (33, 128, 64)])
 def test_transition_of_a_row_that_is_no_number(torch_cuda, rows, c_o, c_i):
     """ReLU takes a NaN for zero (as fmaxf does), in either kernel and at the fewest slices: such a row's result is b2, and no other row knows."""
