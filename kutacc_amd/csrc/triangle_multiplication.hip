@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "launch_internal.h"
 #include "mfma_tiles.h"
@@ -194,6 +195,7 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
         // The panel: [64 positions][4 chunks of 4 channels], the chunk XOR-ed with 2 (position / 4 % 2), under which these writes and the
         // transposing reads below are free of bank conflicts.
         const uint32_t write_at = 32u * col + 8u * (uint32_t)(chunk ^ (2 * ((col >> 2) & 1)));
+        auto multiply = [&](auto kept) __attribute__((always_inline)) {
 #pragma unroll
         for (int pb = 0; pb < 4; ++pb) { // 16 positions
             f32x4 pa = {0.f, 0.f, 0.f, 0.f}, ga = pa;
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
                 pa = product(wp[ks], y, pa);
                 ga = product(wg[ks], y, ga);
             }
-            const float mk = __uint_as_float((uint32_t)mask_row[16 * pb + col] << 16);
+            const float mk = decltype(kept)::value ? 1.0f : __uint_as_float((uint32_t)mask_row[16 * pb + col] << 16);
             bf16x4 pp, ov;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
@@ -214,9 +216,17 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
             for (int v = 0; v < 4; ++v) {
                 // sigmoid(gate + bias) = 1 / (1 + 2^-(gate*log2e + bias*log2e)); the gate stays in fp32
                 const float e = __builtin_amdgcn_exp2f(fmaf(ga[v], -LOG2E, gneg[v]));
-                ov[v] = (bf16_t)(to_f32(pp[v]) * mk * __builtin_amdgcn_rcpf(1.0f + e));
+                ov[v] = (bf16_t)((decltype(kept)::value ? to_f32(pp[v]) : to_f32(pp[v]) * mk) * __builtin_amdgcn_rcpf(1.0f + e));
             }
             *reinterpret_cast<bf16x4 *>(panel + write_at + 512 * pb) = ov;
+        }
+        };
+        // Positions that are all there are not multiplied by their masks: the same bits, 20 vector instructions of 370 a step and wave (whole block, us: 256
+        // residues 47.4 -> 46.5, 384 87.8 -> 86.8, 1024 685 -> 677).
+        if (__all(mask_row[lane] == 0x3f80)) {
+            multiply(std::true_type{});
+        } else {
+            multiply(std::false_type{});
         }
         // 16 channels x eight 16-byte pieces of 8 positions; pieces past the last one repeat it.  A store: 16 channels x four pieces.
         const int last_piece = (positions - 1 - step * STEP) >> 3;

@@ -899,6 +899,35 @@ def test_lengths_at_which_the_equation_runs_over_the_edge(torch_cuda, n, outgoin
         assert not helpers.same_bits(got[0], act)
 
 
+@pytest.mark.parametrize("n", [8, 64, 72, 200, 384])
+@pytest.mark.parametrize("kind", ["ones", "one zero", "padding", "halves"])
+def test_triangle_multiplication_block_of_steps_without_a_mask(torch_cuda, n, kind):
+    """Steps of 64 positions whose masks are all one are not multiplied by them: the streaming kernel's bits with no such step, with all, and with both."""
+    torch = torch_cuda
+    case = tm_block_case(3900 + n, n, 128, 128)
+    mask = np.ones((n, n), np.float32)
+    if kind == "one zero":
+        mask[n // 2, n // 3] = 0
+    elif kind == "padding":
+        mask[:, n - n // 10 - 1:] = mask[n - n // 10 - 1:, :] = 0
+    elif kind == "halves":
+        mask[n // 2:] = 0.5
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(  # noqa: E731
+        device="cuda", dtype=torch.bfloat16 if a.ndim >= 2 else torch.float32)
+    w = {k: dev(v) for k, v in case.items() if k not in ("z", "mask")}
+    got = []
+    for mode in (None, "streaming"):
+        assert capi.set_tuning("gated_projection", mode) == 0
+        try:
+            pair = dev(case["z"])
+            assert capi.TriangleMultiplicationBlock(pair, dev(mask), w, True).run() == 0
+            torch.cuda.synchronize()
+        finally:
+            capi.set_tuning("gated_projection", None)
+        got.append(pair)
+    assert bool(torch.isfinite(got[0]).all()) and helpers.same_bits(got[0], got[1])
+
+
 @pytest.mark.parametrize("n", [48, 72, 384])
 def test_triangle_multiplication_block_on_each_gated_projection_kernel(torch_cuda, n):
     """The block's two gated projections go out in one launch.  Its default kernel (weights in registers, both sides in
