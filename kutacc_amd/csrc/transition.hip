@@ -212,6 +212,11 @@ __device__ __forceinline__ void wait_and_barrier()
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
 }
 
+// b2 lies behind b1 where a CU has one workgroup; where several share its LDS, in the place of b1's slices before the last one, once these have been read
+// and if there are enough of them.  Always behind b1 it cost a CU its third workgroup at 128 -> 1088 and 1152 (300000 rows of the
+// latter 181 us, 174 so) and its fourth at 64 -> 2048 (156, 153).
+__host__ __device__ constexpr int b2_place(int c_o, int slice, int groups, int c_i) { return groups > 1 && c_i - slice >= c_o ? 0 : c_i; }
+
 // SLICE: hidden units per stage of the ring of STAGES; GROUPS: workgroups a CU is meant to hold.
 template <int CO, bool BLOCK, int SLICE, int STAGES, int WAVES, int GROUPS>
 __global__ __launch_bounds__(64 * WAVES, GROUPS * WAVES / 4) void transition_rows_kernel(const TransitionParams p)
@@ -224,17 +229,21 @@ __global__ __launch_bounds__(64 * WAVES, GROUPS * WAVES / 4) void transition_row
     constexpr int UPW = STAGE_SLOTS / 64 / WAVES;  // loads of 1 KB a wave asks for per stage
     static_assert(SLICE == 32 || SLICE == 64, "layout of W2 slices");
     static_assert(WAVES * 256 <= STAGE_SLOTS && UPW >= 4, "the waves' panels lie in a stage; a wave's loads fill whole panels");
-    extern __shared__ uint4 lds[]; // [STAGES][W1 slice, W2 slice], b1, b2
-    static_assert(CO <= 64 * WAVES, "a thread brings one value of b2");
+    extern __shared__ uint4 lds[]; // [STAGES][W1 slice, W2 slice], b1, and b2 (b2_place)
+    static_assert(CP <= WAVES, "a thread brings one value of b2");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5, NJ = p.c_i / SLICE;
     float *b1s = reinterpret_cast<float *>(lds + STAGES * STAGE_SLOTS);
-    float *b2s = b1s + p.c_i;
+    float *b2s = b1s + b2_place(CO, SLICE, GROUPS, p.c_i);
     for (int i = tid; i < p.c_i; i += 64 * WAVES) {
         b1s[i] = p.b1[i]; // visible after the first barrier of the slice loop
     }
-    if (CO == 64 * WAVES || tid < CO) {
-        b2s[tid] = p.b2[tid];
+    float b2_value = 0.f;
+    if (wave < CP) {
+        b2_value = p.b2[wave * 64 + lane];
+        if constexpr (GROUPS == 1) {
+            b2s[wave * 64 + lane] = b2_value;
+        }
     }
 
     const int past = (int)blockIdx.x - p.full_groups;
@@ -397,15 +406,22 @@ __global__ __launch_bounds__(64 * WAVES, GROUPS * WAVES / 4) void transition_row
     for (int j = 1; j < NJ; ++j) {
         step(j, std::true_type{}, std::true_type{});
     }
+    if (GROUPS > 1 && wave < CP) { // of b1, only the last slice may still be read
+        b2s[wave * 64 + lane] = b2_value;
+    }
     step(NJ, std::false_type{}, std::true_type{});
 
     if (!active) {
         return;
     }
     uint4 *panel = lds + NJ % STAGES * STAGE_SLOTS + wave * 256; // a stage that no wave reads any more
+    int lane_o = lane;
+    if constexpr (CO == 256) { // opaque, as above: no register to spare
+        asm volatile("" : "+v"(lane_o));
+    }
 #pragma unroll
     for (int cp = 0; cp < CP; ++cp) {
-        store_channels<CO, BLOCK, EARLY>(oacc[2 * cp], oacc[2 * cp + 1], b2s, residual[cp], p.out + row0 * CO, last_local, cp * 64, panel, lane);
+        store_channels<CO, BLOCK, EARLY>(oacc[2 * cp], oacc[2 * cp + 1], b2s, residual[cp], p.out + row0 * CO, last_local, cp * 64, panel, lane_o);
     }
 }
 
@@ -547,7 +563,7 @@ hipError_t launch_rows(TransitionParams p, hipStream_t stream)
     const int64_t groups = (per_cu + WAVES - 1) / WAVES;
     p.tail_waves = (int)((per_cu + groups - 1) / groups);
     const int64_t blocks = p.full_groups + (rest + p.tail_waves - 1) / p.tail_waves;
-    kernel<<<dim3((unsigned)blocks), 64 * WAVES, stages + (size_t)(p.c_i + CO) * sizeof(float), stream>>>(p);
+    kernel<<<dim3((unsigned)blocks), 64 * WAVES, stages + (size_t)std::max(p.c_i, b2_place(CO, SLICE, GROUPS, p.c_i) + CO) * sizeof(float), stream>>>(p);
     return hipGetLastError();
 }
 

@@ -2,8 +2,10 @@
 loops, where a wait for them is a wait for every load that was to stay on its way."""
 import os
 import re
+import shutil
 import struct
 import subprocess
+import sys
 
 import pytest
 
@@ -46,3 +48,52 @@ def test_attention_kernels_keep_their_registers(tmp_path):
     assert len(kernels) > 100 and any("fused_head_kernel" in k for k in kernels), len(kernels)
     spilled = {k: n for k, n in kernels.items() if n and not any(m in k for m in MEASURED)}
     assert not spilled, spilled
+
+
+# Launches that print what they ask for instead of starting anything, on a device of 256 CUs
+LAUNCHES = r"""
+#include <stddef.h>
+#include <stdint.h>
+#include <stdio.h>
+typedef struct { uint32_t x, y, z; } dim3;
+int hipGetDevice(int *d) { *d = 0; return 0; }
+int hipDeviceGetAttribute(int *v, int which, int d) { *v = 256; return 0; }
+int hipFuncSetAttribute(const void *f, int which, int v) { return 0; }
+int hipGetLastError(void) { return 0; }
+unsigned __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, void *stream)
+{
+    printf("launch %u %u %zu\n", grid.x, block.x, lds);
+    fflush(stdout);
+    return 1; // not 0: what <<<>>> expands to goes no further
+}
+"""
+CALL = """
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)  # in front of the runtime that the library brings
+L = ctypes.CDLL(sys.argv[2])
+v, i = ctypes.c_void_p, ctypes.c_int64
+L.kutacc_hip_transition_block.argtypes = [v, v, v, ctypes.c_float, v, v, v, v, v, i, i, i, i, ctypes.c_int32, v]
+at = 1 << 32  # an address that nothing reads
+rows, c_o, c_i, dtype = map(int, sys.argv[3:])
+print("rc", L.kutacc_hip_transition_block(at, at, at, 1e-5, at, at, at, at, at, 1 << 40, rows, c_o, c_i, dtype, None), flush=True)
+"""
+
+
+# The largest hidden layers that a CU's workgroups have room for, and the model's own.  The LDS comes in pieces of 1280 bytes.
+@pytest.mark.parametrize("c_o,c_i,per_cu", [(64, 256, 4), (64, 2048, 4), (128, 64, 3), (128, 512, 3), (128, 1088, 3), (128, 1152, 3), (256, 64, 2),
+                                            (256, 1024, 2), (256, 2048, 2)])
+def test_transition_fits_its_workgroups_into_the_lds(tmp_path, c_o, c_i, per_cu):
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None or not os.path.exists(build.LIB_PATH):
+        pytest.skip("needs the built library and a C compiler")
+    from kutacc_amd import capi
+    source, shim = tmp_path / "launches.c", tmp_path / "launches.so"
+    source.write_text(LAUNCHES)
+    subprocess.run([cc, "-shared", "-fPIC", "-O1", str(source), "-o", str(shim)], check=True)
+    out = subprocess.run([sys.executable, "-c", CALL, str(shim), build.LIB_PATH, "600000", str(c_o), str(c_i), str(capi.K_BF16)], capture_output=True,
+                         text=True, check=True).stdout
+    assert "rc 0" in out, out
+    launches = re.findall(r"launch (\d+) (\d+) (\d+)", out)
+    assert len(launches) == 1 and launches[0][1] == "256", out
+    pieces = -(-int(launches[0][2]) // 1280)
+    assert per_cu * pieces <= 160 * 1024 // 1280, f"{launches[0][2]} bytes: {160 * 1024 // 1280 // pieces} workgroups a CU"
