@@ -558,8 +558,11 @@ int launch(SmallHeadParams p, hipStream_t stream)
     p.splits = std::max(1, std::min(turns, room));
     const int64_t blocks = (int64_t)(p.sets + 7) / 8 * 8 * p.H * p.splits;
     if constexpr (TILES) {
+        kutacc_prof::KernelTimer t("seed_tiles_kernel", 0.0, stream);
         seed_tiles_kernel<<<dim3((unsigned)((p.H * p.NB * p.NB + 3) / 4)), 256, 0, stream>>>(p);
     }
+    const double C = (double)p.H * D, M = (double)p.B * p.S;
+    kutacc_prof::KernelTimer t("small_head_attention_kernel", (PROJECTS ? 8.0 * M * C * C : 0.0) + 4.0 * M * (double)p.S * C, stream);
     small_head_attention_kernel<HAS_NB, PROJECTS, TILES><<<dim3((unsigned)blocks), 64 * waves, lds, stream>>>(p);
     return kutacc_hip_status(hipGetLastError());
 }
@@ -636,15 +639,16 @@ int small_head_attention(const kutacc_hip_attention_args_t &a, bool projects, hi
     p.bg = a.gating_b;
     p.stash[0] = (uint2 *)a.q, p.stash[1] = (uint2 *)a.k, p.stash[2] = (uint2 *)a.gate, p.stash_each = (int)stash_capacity(a);
     // The seeds as a pass of their own, behind the last stash where there is room for them: where the bias's rows start on any address, as they do
-    // at seven lengths of eight -- the kernel's loads of them then cross lines --, and where sets and tiles pay for the pass.  Operator, us, bias read
-    // in the kernel against this: 1024 rows of 301 171.5 164, of 253 122 118, of 381 240 235, 5120 of 127 274 254, 2000 of 199 196 186.5, of 319 438 330,
-    // 600 of 251 79.8 79.3; below the line 300 of 301 70.3 69.9, 256 of 317 57.6 59.0, 400 of 219 58.1 58.4, 1024 of 94 43.2 45.5.  Rows on 16 bytes gain
-    // nothing: 2000 of 320 327 329, 600 of 256 75.6 79.
+    // at seven lengths of eight -- the kernel's loads of them then cross lines --, and where sets and tiles pay for the pass: tiles of all
+    // sets per CU, whose loads it makes cheaper, against its launch and its own tiles.  Operator, us, bias read in the kernel against this (256 CUs): 1024
+    // rows of 301 171.5 164, of 253 122 118, of 381 240 235, 5120 of 127 274 254, 2000 of 199 196 186.5, of 319 438 330, 600 of 251 79.8 79.3, 300 of 301, on
+    // the line, 70.3 69.9; below it 256 of 317 57.6 59.0, 400 of 219 58.1 58.4, 1024 of 94 43.2 45.5.  Rows on 16 bytes gain nothing: 2000 of 320 327 329, 600
+    // of 256 75.6 79.
     const int64_t units = (int64_t)p.sets * p.H, last = std::max<int64_t>(0, units - 2 * (int64_t)p.stash_each), unit_bytes = (int64_t)ROWS * p.NB * 1024;
     char *const gate = (char *)a.gate, *const seeds = (char *)(((uintptr_t)gate + (uintptr_t)(last * unit_bytes) + 15) / 16 * 16);
     const int64_t seed_bytes = (int64_t)p.H * p.NB * p.NB * 4096, room = gate + a.batch * a.seq_len * a.nheads * D * 2 - seeds;
     const bool any_address = !kutacc_hip_aligned16(p.nb) || p.nb_sh % 8 != 0 || p.nb_sq % 8 != 0;
-    if (p.nb && any_address && (int64_t)p.sets * p.NB * p.NB >= 7500 && seed_bytes <= room) {
+    if (p.nb && any_address && (int64_t)p.sets * p.NB * p.NB * 256 >= 7500 * (int64_t)kutacc_cu_count() && seed_bytes <= room) {
         p.tiles = (f32x4 *)seeds;
         return launch<true, true, true>(p, stream);
     }

@@ -593,10 +593,7 @@ int gating_attention_tiled(const kutacc_hip_attention_args_t &a, hipStream_t str
     const int64_t B = a.batch, S = a.seq_len, H = a.nheads, hd = a.head_size, C = H * hd, M = B * S;
     int rc;
     if (small_head_attention_projects(a)) {
-        {
-            kutacc_prof::KernelTimer t("small_head_attention_kernel", 8.0 * (double)M * (double)C * (double)C + 4.0 * (double)B * (double)S * (double)S * (double)C, stream);
-            rc = small_head_attention(a, true, stream);
-        }
+        rc = small_head_attention(a, true, stream);
         return rc != 0 ? rc : project(a.avg, a.avg_stride_s, M, a.output_w, C, C, C, a.out, a.out_ld, a.output_b, stream);
     }
     // 64 channels: one pass for all four (rows of 16-byte pieces on both sides, v of any pitch, offsets in 32 bits)
@@ -620,10 +617,7 @@ int gating_attention_tiled(const kutacc_hip_attention_args_t &a, hipStream_t str
         return rc;
     }
     if (small_head_attention_supports(a)) {
-        {
-            kutacc_prof::KernelTimer t("small_head_attention_kernel", 4.0 * (double)B * (double)S * (double)S * (double)C, stream);
-            rc = small_head_attention(a, false, stream);
-        }
+        rc = small_head_attention(a, false, stream);
         return rc != 0 ? rc : project(a.avg, a.avg_stride_s, M, a.output_w, C, C, C, a.out, a.out_ld, a.output_b, stream);
     }
     TileParams p;
