@@ -841,6 +841,77 @@ __device__ __forceinline__ void attend_block_direct(const uint4 *lds_k, const ui
     l_out = half_swap_sum(lsum);
 }
 
+// Again, for a block in which the two functions above ended with a sum out of range: a row's logits lie all below the -1e30 at which their
+// maximum starts, or its product with log2 e, which is rounded, is off by more than an exponential holds (from 1e10 on: rows of a pair bias or a mask of
+// -1e11 throughout were not numbers).  The true row maxima first, then the logits less these, a difference that is exact where it counts.  Not a hot
+// path: one tile at a time, nothing ahead, the pair bias (nbrow: of this lane's query, offset by 16 (lane >> 5)) element by element.
+template <bool HAS_NB>
+__device__ __forceinline__ void attend_block_far(const uint4 *lds_k, const uint4 *lds_v, const f32x4 *mask4, const bf16_t *nbrow, bf16x8 q0, bf16x8 q1,
+                                                 bf16x8 sel0, bf16x8 sel1, int NB, int S, int lane, f32x16 &o_out, float &l_out)
+{
+    const int g = lane >> 5;
+    auto logits = [&](int t) {
+        f32x16 x;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const f32x4 mv = mask4[t * 8 + a];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                x[4 * a + c] = mv[c];
+            }
+        }
+        if (HAS_NB) {
+            const uint16_t *src = reinterpret_cast<const uint16_t *>(nbrow + t * 32);
+            const int key0 = t * 32 + 16 * g;
+            uint32_t w[8];
+#pragma unroll
+            for (int v = 0; v < 8; ++v) {
+                const uint32_t a0 = key0 + 2 * v < S ? src[2 * v] : 0u, a1 = key0 + 2 * v + 1 < S ? src[2 * v + 1] : 0u;
+                w[v] = a0 | (a1 << 16);
+            }
+            x = mfma(sel0, as_bf16x8(finite_bias_words(make_uint4(w[0], w[1], w[2], w[3]))), x);
+            x = mfma(sel1, as_bf16x8(finite_bias_words(make_uint4(w[4], w[5], w[6], w[7]))), x);
+        }
+        x = mfma(as_bf16x8(lds_k[(t * 2 + 0) * 64 + lane]), q0, x);
+        return mfma(as_bf16x8(lds_k[(t * 2 + 1) * 64 + lane]), q1, x);
+    };
+    float mx = -INFINITY;
+#pragma unroll 1
+    for (int t = 0; t < NB; ++t) {
+        const f32x16 x = logits(t);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            mx = fmaxf(mx, x[v]);
+        }
+    }
+    mx = half_swap_max(mx);
+    f32x16 o = zero16();
+    float lsum = 0.f;
+    bf16x2 one2;
+    one2[0] = (bf16_t)1.0f, one2[1] = (bf16_t)1.0f;
+#pragma unroll 1
+    for (int t = 0; t < NB; ++t) {
+        f32x16 x = logits(t);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            x[v] = __builtin_amdgcn_exp2f((x[v] - mx) * LOG2E);
+        }
+        const bf16x8 p0 = pack8(x, 0), p1 = pack8(x, 8);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            bf16x2 a, c;
+            a[0] = p0[2 * v], a[1] = p0[2 * v + 1];
+            c[0] = p1[2 * v], c[1] = p1[2 * v + 1];
+            lsum = __builtin_amdgcn_fdot2_f32_bf16(a, one2, lsum, false);
+            lsum = __builtin_amdgcn_fdot2_f32_bf16(c, one2, lsum, false);
+        }
+        o = mfma(as_bf16x8(lds_v[(t * 2 + 0) * 64 + lane]), p0, o);
+        o = mfma(as_bf16x8(lds_v[(t * 2 + 1) * 64 + lane]), p1, o);
+    }
+    o_out = o;
+    l_out = half_swap_sum(lsum);
+}
+
 // Copies head h's rows of the four weight matrices into LDS in MFMA fragment order.  A unit -- a matrix's 32 rows by 32 channels, two fragments
 // -- is two wave-wide loads of half lines, put in order through 2 KB of the LDS that are the wave's own: in fragment order, 16 bytes of another
 // row in every lane, a load takes the address path 42 cycles instead of 16.  The unit's index is wave-uniform and the matrix pointer
@@ -1302,6 +1373,9 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
             const bf16_t *nbrow = HAS_NB ? p.nb + (int64_t)h * p.nb_sh + (int64_t)qrow * p.nb_sq + 16 * g : nullptr;
             attend_block_direct<HAS_NB>(lds_k, lds_v, mask4, flags, nbrow, p.nb_vec != 0, qf[i][0], qf[i][1], as_bf16x8(selw0), as_bf16x8(selw1), NB,
                                         S, lane, o, l);
+            if (__any(!(l > 1e-30f && l < 1e30f))) {
+                attend_block_far<HAS_NB>(lds_k, lds_v, mask4, nbrow, qf[i][0], qf[i][1], as_bf16x8(selw0), as_bf16x8(selw1), NB, S, lane, o, l);
+            }
         }
         if (qpos < S) {
             f32x16 gv;
@@ -1599,6 +1673,10 @@ __global__ __launch_bounds__(64 * max_waves(C, 1)) void persistent_head_kernel(F
         } else {
             attend_block<HAS_NB>(lds_k, lds_v, mask4, flags, nb_head, p.nb_sq, j * 32, p.nb_vec != 0, panel, q0, q1, sel0,
                                  sel1, NB, S, lane, o, l);
+            if (__any(!(l > 1e-30f && l < 1e30f))) {
+                const bf16_t *nbrow = HAS_NB ? nb_head + (int64_t)min(j * 32 + prow, S - 1) * p.nb_sq + 16 * g : nullptr;
+                attend_block_far<HAS_NB>(lds_k, lds_v, mask4, nbrow, q0, q1, sel0, sel1, NB, S, lane, o, l);
+            }
         }
         int lane_o = lane; // as above: the addresses of the epilogue are not worth a register during the attention loop
         asm volatile("" : "+v"(lane_o));

@@ -964,3 +964,29 @@ def test_one_row_kernels_at_ragged_lengths_without_a_mask(torch_cuda, B, S, head
             helpers.check_close(got[rows], ref_out[rows], "bf16", "out")
     finally:
         capi.set_tuning("row_pairs", None)
+
+
+@pytest.mark.parametrize("B,S,heads", [(9, 301, 4), (3, 320, 4), (2, 33, 4), (3, 385, 4), (2, 1001, 4), (2, 150, 8), (3, 289, 8), (2, 703, 8)])
+@pytest.mark.parametrize("low", [-1e11, -1e13, -2e30, -1e38])
+def test_logits_far_below_zero_in_natural_units(torch_cuda, B, S, heads, low):
+    """Where the pair bias has no copy in log2 units, rows whose logits all lie at such a value were not numbers: the running maximum starts at -1e30, and its
+    product with log2 e is off by more than an exponential holds.  A query's whole row of the pair bias, the first keys of another, and a batch row's mask."""
+    w = draw_workload(8500 + S, B, S, heads, 32, masked=0.0)
+    w.nb[:, S // 2] = low
+    w.nb[1, S - 1] = low
+    w.nb[0, 3, :S // 2] = low
+    w.nb = round_to_bf16(w.nb)
+    w.bias[B - 1] = low
+    w.bias[0, :S // 3] = low
+    w.bias = round_to_bf16(w.bias)
+    op, ten, scratch = helpers.make_op(w)
+    assert capi.set_tuning("fragments", "off") == 0
+    try:
+        names = helpers.profiled_kernels(torch_cuda, op.run)
+        torch_cuda.cuda.synchronize()
+    finally:
+        capi.set_tuning("fragments", None)
+    assert not capi.error_flag() and capi.last_path() == "fused_mfma" and not any("pair_bias" in n for n in names), names
+    ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
+    helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), ref_avg, "bf16", "gated average")
+    helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, "bf16", "out")
