@@ -95,24 +95,10 @@ __device__ __forceinline__ void make_selectors(int lane, bf16x8 &sel0, bf16x8 &s
     }
 }
 
-// Pair-bias words on their way into a selector MFMA: -inf (and any negative NaN pattern) becomes the most negative finite
-// bf16, since the MFMA multiplies every word by 0 or 1 and 0 x inf is a NaN.  As 16-bit unsigned numbers the negative
-// values sort by magnitude, so this is one packed minimum per word; what the logit then holds is absorbed like a -inf.
-__device__ __forceinline__ uint4 finite_bias_words(uint4 w)
-{
-    typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
-    union {
-        uint4 u;
-        u16x2 h[4];
-    } c;
-    c.u = w;
-    const u16x2 bound = {0xff7f, 0xff7f};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        c.h[i] = __builtin_elementwise_min(c.h[i], bound);
-    }
-    return c.u;
-}
+// Pair-bias words on their way into a selector MFMA: -inf (and any negative NaN pattern) becomes the most negative power of
+// two in bf16, since the MFMA multiplies every word by 0 or 1 and 0 x inf is a NaN; what the logit then holds is absorbed like a -inf, and finite with a mask as
+// low (finite_bias).
+__device__ __forceinline__ uint4 finite_bias_words(uint4 w) { return bias_words_at_least(w, 0xff00); }
 
 // The same selectors with fp16 ones, for the log2-unit loop, whose pair-bias fragments are fp16.
 __device__ __forceinline__ void make_selectors_f16(int lane, f16x8 &sel0, f16x8 &sel1)
@@ -155,7 +141,7 @@ __device__ __forceinline__ void stage_mask_part(const bf16_t *bias_row, float *m
             if (from_mask) {
                 mv = to_f32((bf16_t)fmaf(mv, 1e9f, -1e9f));
             }
-            mv *= scale;
+            mv = finite_bias(mv * scale);
         }
         if (k < NB * 32) {
             mask[k] = mv;
@@ -171,7 +157,7 @@ __device__ __forceinline__ void stage_mask_part(const bf16_t *bias_row, float *m
 // stage_mask_part for the two-row kernel, which adds a row's mask bias to its logits with one more MFMA (a rank-one
 // product of the per-key values with ones) instead of sixteen vector additions per tile: the value of key k is stored
 // as two bf16, v = hi + lo to 2^-17 of |v|, the k-slots 0 and 1 of that MFMA's A operand.  -inf (keys past S): hi = -inf,
-// lo = 0.  Keys from `flagged` on set no flag: those past S need no mask where the tiles of the pair bias have them at -3e38, so that rows of a ragged
+// lo = 0.  Keys from `flagged` on set no flag: those past S need no mask where the tiles of the pair bias have them at LOWEST_BIAS, so that rows of a ragged
 // length without a mask take the loop without one (the operator, us: 199 residues 38.0 -> 36.2, 255 43.5 -> 42.1, 352 80.5 -> 75.6, 383 90.9 -> 86.2; MSA
 // rows of 255, whole block, 119.6 -> 116.9).
 template <bool NEAR = false>
@@ -186,7 +172,7 @@ __device__ __forceinline__ void stage_mask_words(const bf16_t *bias_row, uint32_
             if (from_mask) {
                 mv = to_f32((bf16_t)fmaf(mv, 1e9f, -1e9f));
             }
-            mv *= scale;
+            mv = finite_bias(mv * scale);
         }
         if (k < NB * 32) {
             words[k] = mask_word(mv);
@@ -213,7 +199,7 @@ __device__ __forceinline__ float mask_bias_finish(bf16_t raw, bool in_range, flo
     if (from_mask) {
         mv = to_f32((bf16_t)fmaf(mv, 1e9f, -1e9f));
     }
-    return in_range ? mv * scale : -INFINITY;
+    return in_range ? finite_bias(mv * scale) : -INFINITY;
 }
 
 // Flash-style attention of one 32-query block against all keys of the unit.
@@ -1746,7 +1732,7 @@ __device__ __forceinline__ void panel32_store(uint4 *panel, int lane, const Pane
 // Pair bias [H, S, S] -> fp32 tiles in accumulator order, in log2 units: for head h, query block j and key tile t,
 // [h][j][t][4][64 lanes] x 16 bytes; lane (r, g) holds keys 32 t + 16 g .. + 15 of query 32 j + pi(r), four per 16-byte
 // piece -- registers 4 a .. 4 a + 3 of the logits accumulator.  Queries past S repeat row S - 1, keys past S are at
-// -3e38; -inf entries become the most negative finite value so that a row of them still has a
+// LOWEST_BIAS, and so are entries below it (-inf): a row of them still has a
 // finite maximum.
 __global__ __launch_bounds__(64) void pair_bias_tiles_kernel(const bf16_t *__restrict__ nb, int64_t nb_sh, int64_t nb_sq, int S,
                                                              int NB, int NT, int vec, f32x4 *__restrict__ out)
@@ -1768,7 +1754,7 @@ __global__ __launch_bounds__(64) void pair_bias_tiles_kernel(const bf16_t *__res
     } else {
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-            v[e] = key0 + e < S ? to_f32(src[e]) : -3.0e38f;
+            v[e] = key0 + e < S ? to_f32(src[e]) : LOWEST_BIAS;
         }
     }
     f32x4 *dst = out + ((((int64_t)h * NB + j) * NT + t) * 4) * 64 + lane;
@@ -1778,7 +1764,7 @@ __global__ __launch_bounds__(64) void pair_bias_tiles_kernel(const bf16_t *__res
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const float x = v[4 * a + c] * LOG2E;
-            o[c] = x < -3.0e38f ? -3.0e38f : x; // a comparison, not a max: a NaN stays a NaN
+            o[c] = x < LOWEST_BIAS ? LOWEST_BIAS : x; // a comparison, not a max: a NaN stays a NaN
         }
         dst[a * 64] = o;
     }

@@ -339,8 +339,8 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 if (4 * g + v < H) {
-                    const float x = real ? (float)(bf16_t)acc[v] * kutacc_dev::LOG2E : -3.0e38f;
-                    t32[(4 * g + v) * 32 + col] = x < -3.0e38f ? -3.0e38f : x; // -inf: the most negative finite value
+                    const float x = real ? (float)(bf16_t)acc[v] * kutacc_dev::LOG2E : kutacc_dev::LOWEST_BIAS;
+                    t32[(4 * g + v) * 32 + col] = x < kutacc_dev::LOWEST_BIAS ? kutacc_dev::LOWEST_BIAS : x; // finite, -inf too
                 }
             }
             __builtin_amdgcn_wave_barrier(); // other lanes' stores: keep the loads below behind them
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
                 uint4 *dst = nbf + ((((int64_t)h * frag_nb + (q >> 5)) * frag_nt + t) * 4 + (c & 3)) * 64 + qlane + 32 * (c >> 2);
                 *dst = val;
                 if (t + 1 == frag_nb && frag_nt > frag_nb) { // the phantom tile that pads the key tiles to a pair
-                    const uint32_t out = __float_as_uint(-3.0e38f);
+                    const uint32_t out = __float_as_uint(kutacc_dev::LOWEST_BIAS);
                     dst[256] = make_uint4(out, out, out, out);
                 }
             }

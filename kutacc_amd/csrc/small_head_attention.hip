@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256) void seed_tiles_kernel(const SmallHeadParams p
             f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                v[e] = key0 + 4 * a + e < p.S ? to_f32(raw[4 * a + e]) * LOG2E : -INFINITY;
+                v[e] = key0 + 4 * a + e < p.S ? finite_bias(to_f32(raw[4 * a + e]) * LOG2E) : -INFINITY;
             }
             to[(2 * u + a) * 64] = v;
         }
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
                 uint2 *to = stash + (i * NB + t) * 128;
                 to[lane] = make_uint2(q2[0], q2[1]), to[64 + lane] = make_uint2(sw[0], sw[1]);
                 const int key = 32 * t + lane;
-                const float mask = key < S ? mask_here * LOG2E : 0.f;
+                const float mask = key < S ? finite_bias(mask_here * LOG2E) : 0.f;
                 if (lane < 32) {
                     masks[t * TILE + i * 32 + lane] = mask;
                     if (mask != 0.f) {
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
             const Piece w = piece;
             piece = fetch(min(unit + waves, units - 1));
             const int i = unit & 3, key = 64 * (unit >> 2) + lane;
-            const float mask = key < S ? to_f32(w.mask) * LOG2E : 0.f;
+            const float mask = key < S ? finite_bias(to_f32(w.mask) * LOG2E) : 0.f;
             if (key < keys) {
                 const int tile_row = (key >> 5) * TILE + i * 32;
                 ks[tile_row + key_slot(key & 31)] = key < S ? w.k : zero_u4();
@@ -497,7 +497,12 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
                     if constexpr (TILES) {
                         return logits(i, t, load_tile(t), std::true_type{});
                     } else {
-                        return logits(i, t, t < full ? seeds(load_nb(t), std::false_type{}) : seeds(load_tail(), std::true_type{}), std::true_type{});
+                        Raw w = t < full ? load_nb(t) : load_tail();
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            w.r[u] = bias_words_at_least(w.r[u], 0xfec0); // -1.28e38: finite in log2 units, with a mask as low too
+                        }
+                        return logits(i, t, t < full ? seeds(w, std::false_type{}) : seeds(w, std::true_type{}), std::true_type{});
                     }
                 };
                 float mx[2] = {-INFINITY, -INFINITY};

@@ -276,7 +276,7 @@ __global__ __launch_bounds__(512, 1) void qkvg_projection_kernel(const StreamedP
                         if (p.bias_is_mask) {
                             mv = to_f32((bf16_t)fmaf(mv, 1e9f, -1e9f));
                         }
-                        mv *= LOG2E;
+                        mv = finite_bias(mv * LOG2E);
                     }
                     const uint32_t word = mask_word(mv), first_word = __builtin_amdgcn_readfirstlane(word); // lane 0: key 32 j
                     if (lane < 32) {

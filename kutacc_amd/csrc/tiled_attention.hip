@@ -191,7 +191,7 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const TileParam
         for (int i = 0; i < DB; ++i) {
             stage[v_slot[i]] = keep(vreg[i], v_real[i]); // (the element-wise form has zeroed what it must already)
         }
-        reinterpret_cast<float *>(stage + K_SLOTS + V_SLOTS)[tid & (CHUNK - 1)] = bias_keep ? to_f32(bias_raw) * LOG2E : -INFINITY;
+        reinterpret_cast<float *>(stage + K_SLOTS + V_SLOTS)[tid & (CHUNK - 1)] = bias_keep ? finite_bias(to_f32(bias_raw) * LOG2E) : -INFINITY;
     };
     // Pair bias of this lane's query for the keys of chunk c, in accumulator order: [key block][j] holds keys
     // 32 kb + 16 j + 8 g .. + 7.  Straight from global memory into registers: a load instruction touches 32 rows, a quarter
@@ -280,10 +280,12 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const TileParam
                             if constexpr (HAS_NB) {
                                 v = fmaf(to_f32(nbv[e]), LOG2E, v);
                             }
-                            x[kb][8 * j + e] = v;
-                            if constexpr (SAFE) {
+                            if constexpr (SAFE) { // finite for every key that is there (past the end the mask is -inf)
+                                const float lowest = (e < 4 ? b0[e & 3] : b1[e & 3]) + LOWEST_BIAS;
+                                v = v < lowest ? lowest : v;
                                 mx = fmaxf(mx, v);
                             }
+                            x[kb][8 * j + e] = v;
                         }
                     }
                 }

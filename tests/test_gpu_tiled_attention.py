@@ -377,3 +377,64 @@ def test_handle_based_entry_point_takes_the_route(torch_cuda):
     hop.run()
     assert not capi.error_flag() and capi.last_path() == "tiled_mfma"
     np.testing.assert_array_equal(hten["out"], ten["out"].view(torch_cuda.int16).cpu().numpy().view(np.uint16))
+
+
+LOWEST = float(np.float32(np.array(0xff7f0000, dtype=np.uint32).view(np.float32)))  # of bf16
+
+
+# the persistent kernels on single rows (fragments, tiles, neither) and on pairs, a workgroup per unit, the streamed kernels, the tiles, heads of 8
+@pytest.mark.parametrize("B,S,H,d", [(9, 301, 4, 32), (16, 384, 4, 32), (130, 96, 4, 32), (66, 200, 4, 32), (40, 200, 4, 32), (6, 64, 4, 32), (3, 385, 4, 32),
+                                     (64, 64, 8, 32), (20, 259, 8, 32), (2, 1200, 4, 32), (64, 77, 8, 8), (6, 70, 8, 8), (3, 200, 4, 16), (1, 70, 3, 40)])
+@pytest.mark.parametrize("pair_bias", [True, False])
+def test_rows_masked_with_the_types_lowest_value(torch_cuda, B, S, H, d, pair_bias):
+    """The lowest value of bf16 times log2(e) is past fp32's range: a batch row with such a mask throughout gave NaN.  It is an even average, as with a mask
+    of -1e9, and a key with such a mask among others has no weight."""
+    w = draw_workload(9100 + S, B, S, H, d, pair_bias=pair_bias, masked=0.0)
+    w.bias[B - 1] = LOWEST
+    w.bias[0, S // 3:] = LOWEST
+    op, ten, scratch = helpers.make_op(w)
+    op.run()
+    torch_cuda.cuda.synchronize()
+    assert not capi.error_flag() and capi.last_path() != "generic"
+    ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
+    helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), ref_avg, "bf16", "gated average")
+    helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, "bf16", "out")
+
+
+@pytest.mark.parametrize("B,S,H,d", [(2, 1200, 4, 32), (64, 77, 8, 8), (6, 64, 8, 8), (5, 7, 8, 8), (3, 200, 4, 16), (2, 96, 3, 24), (2, 100, 2, 64)])
+def test_pair_bias_rows_of_the_types_lowest_value(torch_cuda, B, S, H, d):
+    """The same of a query whose row of the pair bias has it throughout, on the kernels that read the bias as it lies."""
+    w = draw_workload(9200 + S, B, S, H, d, masked=0.0)
+    w.nb[:, S // 2] = LOWEST
+    w.nb[1, S - 1] = LOWEST
+    w.nb[0, 0, :S // 2] = LOWEST
+    run_and_check(w, capi.PATH_TILED)
+
+
+def test_pair_bias_rows_of_the_types_lowest_value_in_the_lanes_order(torch_cuda):
+    """The same where the bias of heads of 8 is brought into the order of the logits by a pass of its own: the bits of the kernel that reads it as it lies."""
+    torch = torch_cuda
+    B, S = 1880, 127
+    g = torch.Generator(device="cuda").manual_seed(9300)
+    bf16 = lambda *shape, scale=1.0: (torch.randn(*shape, device="cuda", generator=g) * scale).to(torch.bfloat16)  # noqa: E731
+    x = torch.nn.functional.layer_norm(torch.randn(B, S, 64, device="cuda", generator=g), (64,)).to(torch.bfloat16)
+    wq, wk, wv, wg, wo = (bf16(64, 64, scale=0.125) for _ in range(5))
+    bg, bo = torch.ones(64, device="cuda"), torch.zeros(64, device="cuda")
+    bias = torch.zeros(B, S, device="cuda", dtype=torch.bfloat16)
+    bias[B - 1] = LOWEST
+    wide = torch.zeros(8, S, 136, device="cuda", dtype=torch.bfloat16)
+    wide[..., :S] = bf16(8, S, S)
+    wide[:, S // 2, :S] = LOWEST
+    wide[1, S - 1, :S] = LOWEST
+    got = []
+    for nb, passes in ((wide[..., :S], False), (wide[..., :S].contiguous(), True)):
+        out = torch.full_like(x, 7.0)
+        scratch = {k: torch.zeros(B, S, 8, 8, device="cuda", dtype=torch.bfloat16) for k in ("q", "k", "gate", "avg")}
+        scratch["v"] = torch.zeros(8, 8, B, S, device="cuda", dtype=torch.bfloat16)
+        names = helpers.profiled_kernels(torch, capi.GatedAttention(x, wq, wk, wv, wg, bg, wo, bo, bias, nb, 8, out, scratch).run)
+        torch.cuda.synchronize()
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert ("seed_tiles_kernel" in names) == passes, names
+        assert not capi.error_flag() and bool(torch.isfinite(out).all()) and bool(torch.isfinite(scratch["avg"]).all())
+        got.append((out, scratch["avg"]))
+    assert helpers.same_bits(got[0][0], got[1][0]) and helpers.same_bits(got[0][1], got[1][1])
