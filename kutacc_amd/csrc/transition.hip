@@ -589,9 +589,11 @@ hipError_t launch(const TransitionParams &p, int64_t c_o, hipStream_t stream)
     const bool few = c_o != 64 && blocks <= cus;
     // While eight waves a CU take all rows, they are one workgroup, which brings the weights once, in four stages or in slices of twice the size.  Against
     // two or three workgroups (us): 256 -> 1024 40000 rows 51.6 49.7, 50000 57.3 53.0, 65000 65.3 60.8, 128 -> 512 9000 rows 13.1 12.3, 30000 14.3 13.3,
-    // 65000 22.2 19.7, 128 -> 256 20000 9.9 9.9, 50000 14.3 13.2.  Beyond, a second round of it costs: 80000 89.5 94.2, 27.6 30.9.  With 256 channels and up
-    // to four waves a CU no gain: 256 -> 1024 20000 34.1 34.0, 256 -> 512 22.0 22.5.
-    const bool one_round = blocks <= 8 * cus && (c_o == 128 || blocks > 4 * cus);
+    // 65000 22.2 19.7, 128 -> 256 20000 10.1 9.9, 50000 15.2 13.4.  Beyond, a second round of it costs: 80000 89.5 94.2, 27.6 30.9.  With 256 channels and up
+    // to four waves a CU no gain: 256 -> 1024 20000 34.1 34.0, 256 -> 512 22.0 22.5.  Few hidden units are one or two slices of twice the size, whose two
+    // products cannot run side by side, which up to four waves a CU do not make up for: 128 -> 64 9000 rows 6.6 7.2, 32768 7.5 8.0, 40000 9.3 9.1, 65536 10.4 9.5,
+    // 128 -> 128 9000 7.6 8.0, 24577 8.3 8.5, 33000 10.7 10.0; 256 -> 64 50000 17.6 17.9, 65536 19.3 19.4.
+    const bool one_round = blocks <= 8 * cus && (c_o == 128 ? p.c_i > 128 || blocks > 4 * cus : p.c_i > 64 && blocks > 4 * cus);
     kutacc_prof::KernelTimer t(few ? (BLOCK ? "transition_split_kernel<block>" : "transition_split_kernel")
                                    : (BLOCK ? "transition_rows_kernel<block>" : "transition_rows_kernel"),
                                flops, stream);

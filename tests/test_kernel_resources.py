@@ -97,3 +97,21 @@ def test_transition_fits_its_workgroups_into_the_lds(tmp_path, c_o, c_i, per_cu)
     assert len(launches) == 1 and launches[0][1] == "256", out
     pieces = -(-int(launches[0][2]) // 1280)
     assert per_cu * pieces <= 160 * 1024 // 1280, f"{launches[0][2]} bytes: {160 * 1024 // 1280 // pieces} workgroups a CU"
+
+
+# (on 256 CUs) one workgroup of eight waves a CU where that pays: not for few rows with few hidden units, which it slowed down by up to 8 %
+@pytest.mark.parametrize("rows,c_o,c_i,threads", [(9000, 128, 64, 256), (32768, 128, 64, 256), (32769, 128, 64, 512), (9000, 128, 128, 256), (32768, 128, 128, 256),
+                                                  (33000, 128, 128, 512), (9000, 128, 192, 512), (65536, 128, 512, 512), (65537, 128, 512, 256),
+                                                  (50000, 256, 64, 256), (32768, 256, 1024, 256), (32769, 256, 128, 512), (65537, 256, 1024, 256)])
+def test_transition_takes_one_workgroup_a_cu_where_that_pays(tmp_path, rows, c_o, c_i, threads):
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None or not os.path.exists(build.LIB_PATH):
+        pytest.skip("needs the built library and a C compiler")
+    from kutacc_amd import capi
+    source, shim = tmp_path / "launches.c", tmp_path / "launches.so"
+    source.write_text(LAUNCHES)
+    subprocess.run([cc, "-shared", "-fPIC", "-O1", str(source), "-o", str(shim)], check=True)
+    out = subprocess.run([sys.executable, "-c", CALL, str(shim), build.LIB_PATH, str(rows), str(c_o), str(c_i), str(capi.K_BF16)], capture_output=True,
+                         text=True, check=True).stdout
+    launches = re.findall(r"launch (\d+) (\d+) (\d+)", out)
+    assert "rc 0" in out and [int(n) for _, n, _ in launches] == [threads], out
