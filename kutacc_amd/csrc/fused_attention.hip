@@ -946,10 +946,13 @@ __device__ inline void stage_weight_lines(uint4 *lds_w, const FusedParams &p, in
     for (int hi = 0; hi < 2; ++hi) {
         lane_bytes[hi] = 2u * (uint32_t)(rl * C + 8 * ((lane & 7) ^ rl ^ hi));
     }
-    for (int f = wave; f < count * CK; f += nwaves) {
-        const int m = first + f / CK, k = f % CK;
-        const bf16_t *w = m == 0 ? p.w[0] : m == 1 ? p.w[1] : m == 2 ? p.w[2] : p.w[3];
-        load_to_lds(to + f * 1024u, w + (int64_t)(h * HEAD + 8 * (k & 3)) * C + (k >> 2) * 64, k & 2 ? lane_bytes[1] : lane_bytes[0]);
+    // the copies of all matrices are dealt to the waves in turn
+    for (int i = 0, k = wave; i < count; ++i, k -= CK) {
+        const bf16_t *const *at = &p.w[first + i];
+        const bf16_t *w = *at + (int64_t)h * HEAD * C;
+        for (; k < CK; k += nwaves) {
+            load_to_lds(to + (uint32_t)(i * CK + k) * 1024u, w + 8 * (k & 3) * C + (k >> 2) * 64, k & 2 ? lane_bytes[1] : lane_bytes[0]);
+        }
     }
     wait_for_loads<0>();
 }
