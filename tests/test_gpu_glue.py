@@ -1060,14 +1060,11 @@ def test_transition_block(torch_cuda, rows, c_o, c_i):
                                              capi.K_BF16, None) == capi.EINVAL
 
 
-# one row; a row past a wave's 32; the last row count of the kernel for few rows (32 per CU) and the first past it; the first and the last
-# row count of one workgroup of eight waves a CU (from 128 rows a CU with 256 channels, up to 256), few hidden units and many; whole
-# rounds of workgroups and a remainder, for each width, with b2 behind b1 in the LDS and in its place; the narrowest and the widest
-# hidden layer
+# one row; a row past a wave's 32; the last row count of the kernel for few rows (32 per CU) and the first past it; whole
+# rounds of workgroups and a remainder, for each width; the narrowest and the widest hidden layer
 @pytest.mark.parametrize("rows,c_o,c_i", [(1, 64, 64), (1, 256, 64), (33, 128, 2048), (33, 64, 2048), (31, 256, 2048), (8192, 128, 192),
-                                          (8193, 128, 192), (8192, 256, 64), (8193, 256, 64), (20011, 128, 512), (65536, 128, 64), (32768, 256, 64),
-                                          (32769, 256, 64), (40011, 256, 192), (65536, 256, 1024), (98304 + 4133, 128, 64), (98304 + 4133, 128, 192),
-                                          (65536 + 33, 256, 64), (65536 + 33, 256, 320), (131072 + 33, 64, 64), (131072 + 33, 64, 128)])
+                                          (8193, 128, 192), (8192, 256, 64), (8193, 256, 64), (98304 + 4133, 128, 64),
+                                          (65536 + 33, 256, 64), (131072 + 33, 64, 128)])
 def test_transition_block_at_the_edges_of_its_kernels(torch_cuda, rows, c_o, c_i):
     from oracle import oracle
     torch = torch_cuda
@@ -1091,6 +1088,14 @@ def test_transition_block_at_the_edges_of_its_kernels(torch_cuda, rows, c_o, c_i
     few = c_o != 64 and (rows + 31) // 32 <= torch.cuda.get_device_properties(0).multi_processor_count
     assert names == ["transition_split_kernel<block>" if few else "transition_rows_kernel<block>"], names
     helpers.check_close(num(act), want, "bf16", f"transition block {rows}x{c_o}->{c_i}")
+
+
+# one workgroup of eight waves a CU (with 256 channels from 128 rows a CU on, with 128 from 32, up to 256): first and last row counts, few hidden
+# units and many; and b2 behind b1 in the LDS and in its place
+@pytest.mark.parametrize("rows,c_o,c_i", [(20011, 128, 512), (65536, 128, 64), (32768, 256, 64), (32769, 256, 64), (32769, 256, 128), (40011, 256, 192), (65536, 256, 1024),
+                                          (98304 + 4133, 128, 192), (65536 + 33, 256, 320), (131072 + 33, 64, 64)])
+def test_transition_block_with_one_workgroup_a_cu(torch_cuda, rows, c_o, c_i):
+    test_transition_block_at_the_edges_of_its_kernels(torch_cuda, rows, c_o, c_i)
 
 
 # ---- MSA attention blocks ------------------------------------------------------------------------------------------

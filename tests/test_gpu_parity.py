@@ -990,3 +990,28 @@ def test_logits_far_below_zero_in_natural_units(torch_cuda, B, S, heads, low):
     ref_out, ref_avg = helpers.oracle_out(w, return_avg=True)
     helpers.check_close(helpers.to_numpy(scratch["avg"]).reshape(w.B, w.S, w.C), ref_avg, "bf16", "gated average")
     helpers.check_close(helpers.to_numpy(ten["out"]), ref_out, "bf16", "out")
+
+
+@pytest.mark.parametrize("B,S,heads", [(16, 130, 4), (15, 161, 4), (13, 191, 4), (19, 225, 4), (27, 353, 4), (25, 383, 4), (16, 129, 8), (13, 191, 8), (17, 223, 8), (18, 255, 8)])
+def test_keys_past_the_end_have_no_weight_without_a_mask(torch_cuda, B, S, heads):
+    """Keys past the end repeat the last row, here the one with the largest logits, and rows without a mask take a loop that knows them by the pair bias's tiles
+    alone.  Against the loop with masks, to which a mask of -1e-30 sends every row without changing a logit: the same probabilities, whose sums may differ in the
+    last of their 24 bits, and so an average by one step of bf16, 2^-7 of it at most."""
+    torch = torch_cuda
+    w = draw_workload(8700 + S, B, S, heads, 32, masked=0.0, nb_scale=3.0)
+    w.x[:, S - 1] *= 4
+    w.x = round_to_bf16(w.x)
+    assert capi.set_tuning("row_pairs", "1") == 0
+    try:
+        got = []
+        for mask in (0.0, -1e-30):
+            w.bias[:] = round_to_bf16(np.full_like(w.bias, mask))
+            op, ten, scratch = helpers.make_op(w)
+            names = helpers.profiled_kernels(torch, op.run)
+            torch.cuda.synchronize()
+            assert not capi.error_flag() and "persistent_pair_kernel" in names, names
+            got.append(helpers.to_numpy(scratch["avg"]).astype(np.float64))
+    finally:
+        capi.set_tuning("row_pairs", None)
+    assert np.isfinite(got[0]).all()
+    helpers.assert_within(got[0], got[1], 2.0 ** -7 * np.abs(got[1]), "gated average")

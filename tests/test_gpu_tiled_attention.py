@@ -219,13 +219,11 @@ def test_heads_of_eight_with_the_projections_inside(torch_cuda, B, S, form, proj
         assert float((x - y).norm() / y.norm()) <= 2.0 ** -9 and float((x - y).abs().max()) <= 2.0 ** -6 * float(y.abs().max())
 
 
-# (the last three: the fewest sets that pay for the pass, one set less, and no room for it in the gate tensor)
-@pytest.mark.parametrize("B,S,passes", [(304, 311, True), (480, 253, True), (482, 255, True), (2005, 100, True), (2003, 97, True), (1880, 127, True),
-                                        (7600, 64, True), (7599, 63, True), (300, 301, True), (296, 301, False), (64, 1001, False)])
+@pytest.mark.parametrize("B,S", [(304, 311), (480, 253), (482, 255), (2005, 100), (2003, 97), (1880, 127), (7600, 64), (7599, 63)])
 @pytest.mark.parametrize("offset", [0.0, 150.0])
-def test_heads_of_eight_with_the_bias_in_the_lanes_order(torch_cuda, B, S, passes, offset):
-    """A bias whose rows start on any address, brought into the order of the logits by a pass of its own (passes: on 256 CUs), against the same bias in
-    rows of 16 bytes, which the kernel reads as they lie: the same bits.  Masked keys, a fully masked row, entries of -inf and, with the offset, rows that are repeated."""
+def test_heads_of_eight_with_the_bias_in_the_lanes_order(torch_cuda, B, S, offset):
+    """A bias whose rows start on any address, brought into the order of the logits by a pass of its own, against the same bias in rows of 16 bytes,
+    which the kernel reads as they lie: the same bits.  Masked keys, a fully masked row, entries of -inf and, with the offset, rows that are repeated."""
     torch = torch_cuda
     g = torch.Generator(device="cuda").manual_seed(500 + S)
     bf16 = lambda *shape, scale=1.0: (torch.randn(*shape, device="cuda", generator=g) * scale).to(torch.bfloat16)  # noqa: E731
@@ -248,12 +246,43 @@ def test_heads_of_eight_with_the_bias_in_the_lanes_order(torch_cuda, B, S, passe
         out = torch.full_like(x, 7.0)
         scratch = {k: torch.zeros(B, S, 8, 8, device="cuda", dtype=torch.bfloat16) for k in ("q", "k", "gate", "avg")}
         scratch["v"] = torch.zeros(8, 8, B, S, device="cuda", dtype=torch.bfloat16)
+        capi.GatedAttention(x, wq, wk, wv, wg, bg, wo, bo, bias, nb, 8, out, scratch).run()
+        torch.cuda.synchronize()
+        assert not capi.error_flag() and capi.last_path() == "tiled_mfma"
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            # the seeds of the keys past the end lie in the gate tensor: 64-bit pairs of fp32 -inf, which no stash of queries and gates holds
+            assert S % 32 in (0, 31) or bool((scratch["gate"].view(torch.int64) == -0x007fffff00800000).any()) == (nb.stride(1) % 8 != 0)
+        assert bool((scratch["v"] == 0).all()) and bool(torch.isfinite(out).all())
+        got.append((out, scratch["avg"]))
+    assert helpers.same_bits(got[0][0], got[1][0]) and helpers.same_bits(got[0][1], got[1][1])
+
+
+# (the last three: the fewest sets that pay for the pass on 256 CUs, one set less, and no room for it in the gate tensor)
+@pytest.mark.parametrize("B,S,passes", [(304, 311, True), (480, 253, True), (482, 255, True), (2005, 100, True), (2003, 97, True), (1880, 127, True),
+                                        (7600, 64, True), (7599, 63, True), (300, 301, True), (296, 301, False), (64, 1001, False)])
+def test_which_biases_of_heads_of_eight_come_through_the_pass(torch_cuda, B, S, passes):
+    """The pass runs, by its name, where the bias's rows start on any address and sets and tiles pay for it; the bits are those of the bias in rows of 16 bytes."""
+    torch = torch_cuda
+    g = torch.Generator(device="cuda").manual_seed(600 + S)
+    bf16 = lambda *shape, scale=1.0: (torch.randn(*shape, device="cuda", generator=g) * scale).to(torch.bfloat16)  # noqa: E731
+    x = torch.nn.functional.layer_norm(torch.randn(B, S, 64, device="cuda", generator=g), (64,)).to(torch.bfloat16)
+    wq, wk, wv, wg, wo = (bf16(64, 64, scale=0.125) for _ in range(5))
+    bg, bo = torch.ones(64, device="cuda"), torch.zeros(64, device="cuda")
+    bias = torch.zeros(B, S, device="cuda", dtype=torch.bfloat16)
+    wide = torch.zeros(8, S, (S + 7) // 8 * 8 + 8, device="cuda", dtype=torch.bfloat16)
+    wide[..., :S] = bf16(8, S, S)
+    narrow = torch.zeros(8, S, S + 1 if S % 8 == 0 else S, device="cuda", dtype=torch.bfloat16)
+    narrow[..., :S] = wide[..., :S]
+    got = []
+    for nb, unaligned in ((wide[..., :S], False), (narrow[..., :S], True)):
+        out = torch.full_like(x, 7.0)
+        scratch = {k: torch.zeros(B, S, 8, 8, device="cuda", dtype=torch.bfloat16) for k in ("q", "k", "gate", "avg")}
+        scratch["v"] = torch.zeros(8, 8, B, S, device="cuda", dtype=torch.bfloat16)
         names = helpers.profiled_kernels(torch, capi.GatedAttention(x, wq, wk, wv, wg, bg, wo, bo, bias, nb, 8, out, scratch).run)
         torch.cuda.synchronize()
-        assert not capi.error_flag() and capi.last_path() == "tiled_mfma" and "small_head_attention_kernel" in names, names
+        assert not capi.error_flag() and "small_head_attention_kernel" in names, names
         if torch.cuda.get_device_properties(0).multi_processor_count == 256:
-            assert ("seed_tiles_kernel" in names) == (passes and nb.stride(1) % 8 != 0), names
-        assert bool((scratch["v"] == 0).all()) and bool(torch.isfinite(out).all())
+            assert ("seed_tiles_kernel" in names) == (passes and unaligned), names
         got.append((out, scratch["avg"]))
     assert helpers.same_bits(got[0][0], got[1][0]) and helpers.same_bits(got[0][1], got[1][1])
 
