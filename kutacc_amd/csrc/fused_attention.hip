@@ -76,7 +76,8 @@ struct FusedParams {
     int ngrp;     // persistent kernel: batch-row groups per XCD
     const uint4 *nbf; // pair bias * log2(e): fp16, in fragment-major order (pair_bias_fragments_kernel), or fp32 tiles, or nullptr
     int NT;           // key tiles the LDS arrays are laid out for: NB rounded up to an even number (the log2-unit
-                      // loop walks tile pairs; a phantom tile is all zeros behind a -inf mask)
+                      // loop walks tile pairs; the phantom tile's K and V are zeros, its mask is -inf, and in the copies
+                      // of the pair bias it holds what keys past the end hold: PAST_THE_END_F16 or LOWEST_BIAS)
     int l2mode;       // logits in log2 units (attend_block_l2); needs nbf when there is a pair bias
 };
 
@@ -960,7 +961,7 @@ __device__ inline void stage_weight_lines(uint4 *lds_w, const FusedParams &p, in
 // ------------------------------------------------------------------------------------------------
 // fused_head_kernel: one workgroup per (b, h) unit
 // LDS carve-up, in 16-byte units unless noted:
-//   [0, GW*CK*64)               staged weight fragments  [slot][kstep][lane]
+//   [0, GW*CK*64)               staged weights           [matrix][panel of 64 channels][32 rows x 8 pieces, weight_slot]
 //   [.., +NT*2*64)              K fragments              [tile][kstep][lane]
 //   [.., +NT*2*64)              V fragments              [tile][kstep][lane]
 // The mask of the batch row (floats, -inf past S) and the tile flags are needed only by the attention phase and take
@@ -1045,7 +1046,6 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
         const int pass = staged_input ? npass - 1 - pi : pi;
         if (pi > 0) {
             __syncthreads(); // previous group's fragments are no longer being read
-        } else {
         }
         // One block a wave: its rows and its gate's bias are asked for in front of the weights, one round trip for all (with 256 channels, columns of
         // 500 sequences x 100 lose 1.8 % by it).
@@ -1293,7 +1293,7 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
     __syncthreads();
 
     // ---- attention: each wave walks the key tiles for its own query blocks ----
-    uint32_t flags = 0; // bit t: key tile t needs the mask added (non-zero bias or ragged tail)
+    uint32_t flags = 0; // bit t: key tile t needs the mask added (a non-zero one; past the end only where no copy of the pair bias takes those keys out)
     uint32_t differ = 0;
     for (int part = 0; part * 64 < NT * 32; ++part) {
         flags |= (ONE_PASS ? part_flags[part] & 3u : part_flags[part]) << (2 * part);
@@ -1304,7 +1304,8 @@ __global__ __launch_bounds__(64 * max_waves(C, BPW)) void fused_head_kernel(Fuse
     // rows used to be attended three times (triangle attention of 450 residues, 5 % of them padding, whole block 218 -> 203 us, 203 without
     // padding).  With 256 channels (columns of 501 sequences x 91 95.6 -> 96.9), with one block a wave, and in persistent_head_kernel, the choice in front of the loops slows rows without such a mask
     // (77 residues 22.0 -> 22.15 us, 320 74.4 -> 77.9); there the first pass is made in vain (128 residues 22.9 -> 22.3, 320 85.0 -> 83.3).
-    // persistent_pair_kernel has no register left for either (three more spilled: the operator at 384 residues 88.1 -> 89.5).
+    // persistent_pair_kernel, which has no register for a choice in front of its loop (three more spilled: the operator at 384 residues 88.1 -> 89.5), makes
+    // that first pass in vain too, and repeats such a row with its one mask.
     constexpr uint32_t ONE_MASK = 2;
     if (ONE_PASS && l2mode && flags != 0u) { // whose loops know no mask, masks, and one mask
         flags = differ == 0u && one_mask_of(mask, S, lane) != 0.f ? ONE_MASK : 1u;
@@ -2548,7 +2549,8 @@ __global__ __launch_bounds__(2 * F, WALK && F == 128 ? 3 : 2) void output_projec
 // operands of the selector MFMAs, [h][j][t][2][64 lanes] x 16 bytes, so that a wave of the attention
 // kernels fetches the pair bias of a tile with two contiguous 1 KB loads straight into registers.
 // Lane (r, g) holds 16 consecutive keys 32t+16g.. of query row 32j+pi(r); queries past S repeat row
-// S-1 and keys past S read as zero (their mask bias is -inf).  The pair bias is shared by every batch
+// S-1, keys past S and the phantom tile are PAST_THE_END_F16: the loops without a mask know those keys by that alone, so that
+// every pass that writes such a copy (here, pair_bias_bf16_kernel; LOWEST_BIAS in tiles) must.  The pair bias is shared by every batch
 // row, so this pass moves 2*H*S*S bytes once per call, against B times that in the attention kernel.
 __global__ __launch_bounds__(64) void pair_bias_fragments_kernel(const bf16_t *__restrict__ nb, int64_t nb_sh,
                                                                  int64_t nb_sq, int S, int NB, int NT, int vec,
@@ -2638,7 +2640,7 @@ size_t head_kernel_lds(int C, int NB, int GW, int NW, int BPW)
         const size_t kv = (size_t)NT * 2 * 64 * 16, wbytes = (size_t)4 * (C / 16) * 64 * 16;
         return kv + (kv > wbytes ? kv : wbytes) + (size_t)NW * 4096;
     }
-    // weight fragments (the mask, 4 bytes per key, and 16 flag words take their place later), K and V
+    // weights (the mask, 4 bytes per key, and 16 flag words take their place later), K and V
     return (size_t)GW * (C / 16) * 64 * 16 + (size_t)NT * 2 * 64 * 16 * 2;
 }
 

@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256) void pair_bias_bf16_kernel(const bf16_t *__res
     const uint32_t nrows = (uint32_t)rows, ncol = (uint32_t)rows_j, nrow_i = (uint32_t)rows_i;
     // A wave's rows: row0 and the `count` - 1 behind it.  Without the attention's copy they are 32 rows as they come.  With it they are
     // key tile t of query q, on a grid of whole blocks of queries and whole tiles of keys: the last tile of a query has fewer
-    // rows (zeros take the place of the others in the copy), and queries past the last repeat that one, in the copy only.  A workgroup's
+    // rows (PAST_THE_END_F16 or LOWEST_BIAS takes the place of the others in the copy), and queries past the last repeat that one, in the copy only.  A workgroup's
     // waves take four queries that follow each other: their pieces of 16 bytes in the copy are neighbours, and so are their rows of z for the
     // ending node.  (Four tiles of one query, now: triangle attention of 160 residues 33.0 and 32.5 us, of 200 42.1 and 41.6, of 256 46.9 and 46.5, of 128 no
     // difference, of 112 20.0 and 20.6; MSA rows 256 x 256 100.6 and 99.2; 508 x 259 with eight heads, this kernel, 12.8 and 10.6.)

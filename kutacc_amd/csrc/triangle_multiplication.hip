@@ -197,29 +197,29 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
         const uint32_t write_at = 32u * col + 8u * (uint32_t)(chunk ^ (2 * ((col >> 2) & 1)));
         auto multiply = [&](auto kept) __attribute__((always_inline)) {
 #pragma unroll
-        for (int pb = 0; pb < 4; ++pb) { // 16 positions
-            f32x4 pa = {0.f, 0.f, 0.f, 0.f}, ga = pa;
+            for (int pb = 0; pb < 4; ++pb) { // 16 positions
+                f32x4 pa = {0.f, 0.f, 0.f, 0.f}, ga = pa;
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                const bf16x8 y = as_bf16x8(stage[row_slot(16 * pb + col, 4 * ks + chunk)]);
-                pa = product(wp[ks], y, pa);
-                ga = product(wg[ks], y, ga);
-            }
-            const float mk = decltype(kept)::value ? 1.0f : __uint_as_float((uint32_t)mask_row[16 * pb + col] << 16);
-            bf16x4 pp, ov;
+                for (int ks = 0; ks < 4; ++ks) {
+                    const bf16x8 y = as_bf16x8(stage[row_slot(16 * pb + col, 4 * ks + chunk)]);
+                    pa = product(wp[ks], y, pa);
+                    ga = product(wg[ks], y, ga);
+                }
+                const float mk = decltype(kept)::value ? 1.0f : __uint_as_float((uint32_t)mask_row[16 * pb + col] << 16);
+                bf16x4 pp, ov;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                pp[v] = (bf16_t)(pa[v] + pbias[v]);
-            }
-            asm volatile("" : "+v"(pp)); // else each value is rounded by itself
+                for (int v = 0; v < 4; ++v) {
+                    pp[v] = (bf16_t)(pa[v] + pbias[v]);
+                }
+                asm volatile("" : "+v"(pp)); // else each value is rounded by itself
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                // sigmoid(gate + bias) = 1 / (1 + 2^-(gate*log2e + bias*log2e)); the gate stays in fp32
-                const float e = __builtin_amdgcn_exp2f(fmaf(ga[v], -LOG2E, gneg[v]));
-                ov[v] = (bf16_t)((decltype(kept)::value ? to_f32(pp[v]) : to_f32(pp[v]) * mk) * __builtin_amdgcn_rcpf(1.0f + e));
+                for (int v = 0; v < 4; ++v) {
+                    // sigmoid(gate + bias) = 1 / (1 + 2^-(gate*log2e + bias*log2e)); the gate stays in fp32
+                    const float e = __builtin_amdgcn_exp2f(fmaf(ga[v], -LOG2E, gneg[v]));
+                    ov[v] = (bf16_t)((decltype(kept)::value ? to_f32(pp[v]) : to_f32(pp[v]) * mk) * __builtin_amdgcn_rcpf(1.0f + e));
+                }
+                *reinterpret_cast<bf16x4 *>(panel + write_at + 512 * pb) = ov;
             }
-            *reinterpret_cast<bf16x4 *>(panel + write_at + 512 * pb) = ov;
-        }
         };
         // Positions that are all there are not multiplied by their masks: the same bits, 20 vector instructions of 370 a step and wave (whole block, us: 256
         // residues 47.4 -> 46.5, 384 87.8 -> 86.8, 1024 685 -> 677).
