@@ -932,8 +932,9 @@ __device__ inline void stage_weight_fragments(uint4 *lds_w, uint4 *own, const Fu
 // The same in whole lines, eight rows by 64 channels a copy (in fragment order, a 16-byte piece of another row in every
 // lane, a load takes the address path 42 cycles instead of 16, and a workgroup of one unit waits for them all), straight into the LDS: no
 // registers, all copies of a wave on their way at once.  Through registers, most copies one after the other, the weights of 77 residues took 1.6 us of
-// that kernel's 7; with this and a wave's rows asked for before them the whole block takes 16.05 us, 16.8 before, 96 residues 17.5 and 16.9, 420 164 and
-// 160.5, 512 216 and 212; with 256 channels nothing to 2 %.  A matrix lies as panels of 32 rows x 64 channels (panel_slot); complete when the wave's
+// that kernel's 7; with this and a wave's rows asked for before them the whole block takes 15.8 us, 16.8 before, 96 residues 17.3 and 17.7, 420 160 and
+// 164.  A wave's copies follow each other by their scalar instructions: with the matrix chosen for each of them (45 and six branches, now 20 and one) 77 residues
+// took 16.1, and rows of 290 and 350 keys with 256 channels (16 x 350 35.5 us, now 35.0) more than through registers (35.1).  A matrix lies as panels of 32 rows x 64 channels (panel_slot); complete when the wave's
 // loads are and behind a barrier.
 __device__ inline int weight_slot(int lane, int ks) { return (ks >> 2) * 256 + (panel_slot(lane & 31, lane >> 5) ^ (2 * (ks & 3))); }
 template <int C>

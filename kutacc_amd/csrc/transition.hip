@@ -7,16 +7,16 @@
 // second without leaving the registers.  For that, row i of a W1 block in the LDS is hidden unit sigma(i) (bits 2 and 3 of i
 // swapped), which makes the eight values a lane holds per k-step consecutive hidden units.
 //
-// What bounds it: power.  With two waves a SIMD in their loops the matrix pipes work for 93 of 100 clocks, at the 1.6 to 1.7 GHz that
-// the chip holds under it; a third of a workgroup's time (of 103 000 clocks at 256 -> 1024) goes to its rows' way in and out, in
-// which the other workgroup of the CU has the pipes to itself.  Weights come straight into the LDS (global_load_lds_dwordx4, no
-// registers, no LDS write instructions) into a ring with one barrier per slice.
+// What bounds it: the clock and the rows' way in and out.  At 195072 rows, 256 -> 1024, the matrix pipes work for 58 % of the kernel's clocks (vector
+// issue 32 %, both at once 10 %), at the 1.67 GHz that the chip holds under it; between a wave's loops over the weights lie its rows' load,
+// LayerNorm, residual and store, which the other workgroup of the CU covers in part.  Weights come straight into the LDS
+// (global_load_lds_dwordx4, no registers, no LDS write instructions) into a ring with one barrier per slice.
 // The two products of a slice are a step apart: while W1 of slice j runs, W2 of slice j - 1 runs between its products, whose sums
 // depend on each other; the hidden units of slice j are rounded beside the last products of W2, and every weight fragment leaves the LDS
 // AHEAD products before its own.  With both products of one slice in a step a wave waited for the end of the first product, for its
-// rounding and for most of its fragments.  A wave alone on its SIMD gains most: 20000 rows, 256 -> 1024 39.5 -> 34.1 us; 195072 rows 199
-// -> 186.5 (1097 TFLOP/s), 400000 rows, 256 -> 512 248 -> 229, 147456 rows, 128 -> 256 33.0 -> 31.8, 64 -> 256 19.2 -> 18.3.
-// Two workgroups or three per CU rather than one of twice the waves: one computes while the other fetches its rows or
+// rounding and for most of its fragments.  A wave alone on its SIMD gains most: 20000 rows, 256 -> 1024 40.4 -> 35.0 us; 195072 rows 201
+// -> 189 (1082 TFLOP/s), 400000 rows, 256 -> 512 263 -> 246, 147456 rows, 128 -> 256 33.6 -> 32.2, 64 -> 256 20.3 -> 18.9 (whole block, two sets of rows
+// in turn).  Two workgroups or three per CU rather than one of twice the waves: one computes while the other fetches its rows or
 // stores its result (400000 rows, 256 -> 512 232 against 245 us, 147456 rows, 128 -> 512 48 and 51).  Two sets of rows a wave, for half the fragments,
 // leave no registers: 128 -> 512 70 us with 38 of them spilled.
 //   195072 rows, 256 -> 1024, block: 328 us with weights through registers and one wave per SIMD; 500000 rows, 64 -> 256: 200 us in three
@@ -588,8 +588,8 @@ hipError_t launch(const TransitionParams &p, int64_t c_o, hipStream_t stream)
     const int64_t blocks = (p.rows + 31) / 32, cus = kutacc_cu_count();
     const bool few = c_o != 64 && blocks <= cus;
     // While eight waves a CU take all rows, they are one workgroup, which brings the weights once, in four stages or in slices of twice the size.  Against
-    // two or three workgroups (us): 256 -> 1024 40000 rows 51.6 49.7, 50000 57.3 53.0, 65000 65.3 60.8, 128 -> 512 9000 rows 13.1 12.3, 30000 14.3 13.3,
-    // 65000 22.2 19.7, 128 -> 256 20000 10.1 9.9, 50000 15.2 13.4.  Beyond, a second round of it costs: 80000 89.5 94.2, 27.6 30.9.  With 256 channels and up
+    // two or three workgroups (us): 256 -> 1024 40000 rows 53.7 51.7, 50000 58.7 55.4, 65000 66.9 63.7, 128 -> 512 9000 rows 12.9 12.15, 30000 14.6 13.7,
+    // 65000 22.3 20.2, 128 -> 256 20000 10.1 9.9, 50000 15.2 13.4.  Beyond, a second round of it costs: 80000 89.5 94.2, 27.6 30.9.  With 256 channels and up
     // to four waves a CU no gain: 256 -> 1024 20000 34.1 34.0, 256 -> 512 22.0 22.5.  Few hidden units are one or two slices of twice the size, whose two
     // products cannot run side by side, which up to four waves a CU do not make up for: 128 -> 64 9000 rows 6.6 7.2, 32768 7.5 8.0, 40000 9.3 9.1, 65536 10.4 9.5,
     // 128 -> 128 9000 7.6 8.0, 24577 8.3 8.5, 33000 10.7 10.0; 256 -> 64 50000 17.6 17.9, 65536 19.3 19.4.

@@ -221,8 +221,8 @@ __global__ __launch_bounds__(64 * FRONT_WAVES, 1) void triangle_front_kernel(con
                 *reinterpret_cast<bf16x4 *>(panel + write_at + 512 * pb) = ov;
             }
         };
-        // Positions that are all there are not multiplied by their masks: the same bits, 20 vector instructions of 370 a step and wave (whole block, us: 256
-        // residues 47.4 -> 46.5, 384 87.8 -> 86.8, 1024 685 -> 677).
+        // Positions that are all there are not multiplied by their masks: the same bits, 20 vector instructions of 370 a step and wave (whole block, two
+        // activations in turn, us: 256 residues 46.9 -> 46.3, 384 92.5 -> 91.7, 1024 704 -> 700).
         if (__all(mask_row[lane] == 0x3f80)) {
             multiply(std::true_type{});
         } else {
@@ -544,7 +544,7 @@ int triangle_back(const kutacc_hip_triangle_multiplication_args_t &a, const void
     }
     kutacc_prof::KernelTimer t("triangle_back_kernel", 4.0 * (double)(a.n_res * a.n_res) * C * C, stream);
     // The workgroups that take a step more come first, one a CU: 384 residues give a CU nine steps, five and four, where equal runs of five gave
-    // most ten (whole block 94.4 -> 91.9 us; 200 residues 41.9 -> 39.3).
+    // most ten (whole block, two activations in turn, 94.7 -> 92.3 us; 200 residues 41.6 -> 38.7).
     const int64_t steps = (a.n_res * np + STEP - 1) / STEP, groups = std::min(steps, 2 * (int64_t)kutacc_cu_count());
     triangle_back_kernel<<<dim3((unsigned)groups), 256, BACK_LDS, stream>>>(
         (const bf16_t *)centre, plane, a.ln_center_gamma, a.ln_center_beta, (const bf16_t *)a.output_w, a.output_b, (const bf16_t *)a.gating_w,
