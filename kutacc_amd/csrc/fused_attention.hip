@@ -97,9 +97,24 @@ __device__ __forceinline__ void make_selectors(int lane, bf16x8 &sel0, bf16x8 &s
 }
 
 // Pair-bias words on their way into a selector MFMA: -inf (and any negative NaN pattern) becomes the most negative power of
-// two in bf16, since the MFMA multiplies every word by 0 or 1 and 0 x inf is a NaN; what the logit then holds is absorbed like a -inf, and finite with a mask as
-// low (finite_bias).
-__device__ __forceinline__ uint4 finite_bias_words(uint4 w) { return bias_words_at_least(w, 0xff00); }
+// two in bf16, since the MFMA multiplies every word by 0 or 1 and 0 x inf is a NaN.  As 16-bit unsigned numbers the negative
+// values sort by magnitude, so this is one packed minimum per word; what the logit then holds is absorbed like a -inf, and finite with a mask as low
+// (finite_bias).
+__device__ __forceinline__ uint4 finite_bias_words(uint4 w)
+{
+    typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
+    union {
+        uint4 u;
+        u16x2 h[4];
+    } c;
+    c.u = w;
+    const u16x2 bound = {0xff00, 0xff00};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        c.h[i] = __builtin_elementwise_min(c.h[i], bound);
+    }
+    return c.u;
+}
 
 // The same selectors with fp16 ones, for the log2-unit loop, whose pair-bias fragments are fp16.
 __device__ __forceinline__ void make_selectors_f16(int lane, f16x8 &sel0, f16x8 &sel1)

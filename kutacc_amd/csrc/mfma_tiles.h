@@ -57,28 +57,11 @@ __device__ __forceinline__ uint4 as_uint4(f16x8 h)
     return c.u;
 }
 
-// Eight words of a bias, none below a negative bound: as 16-bit unsigned numbers the negative values (and NaN patterns) sort by magnitude, so
-// this is one packed minimum per two.
-__device__ __forceinline__ uint4 bias_words_at_least(uint4 w, unsigned short bound)
-{
-    typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
-    union {
-        uint4 u;
-        u16x2 h[4];
-    } c;
-    c.u = w;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        c.h[i] = __builtin_elementwise_min(c.h[i], u16x2{bound, bound});
-    }
-    return c.u;
-}
-
 // A mask or pair bias in the units of the logits, finite, as is then the sum of both: the lowest values of bf16 times log2(e) are past fp32's
 // range, and a row whose logits were all -inf would have no maximum to be taken against (a batch row masked with the type's lowest value gave NaN).  One
-// minimum of unsigned numbers, as above.
+// instruction, the maximum that keeps a NaN.
 constexpr float LOWEST_BIAS = -1.5e38f;
-__device__ __forceinline__ float finite_bias(float v) { return __uint_as_float(min(__float_as_uint(v), 0xfee1b1e6u)); } // the pattern of LOWEST_BIAS
+__device__ __forceinline__ float finite_bias(float v) { return __builtin_elementwise_maximum(v, LOWEST_BIAS); }
 
 // nb * log2(e) as an fp16 bit pattern, for the fragment-major pair bias: magnitudes past fp16's range (|nb| > 45 403,
 // infinities included) act as that bound -- 2^-65504 is zero all the same, and the selector products stay finite

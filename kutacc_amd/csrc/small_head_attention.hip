@@ -330,14 +330,15 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
         struct Tile {
             f32x4 x[2][2]; // [query half][key half]
         };
-        auto seeds = [&](const Raw &w, auto tail) { // of the four rows' logits: the pair bias, -inf past the last key
+        auto seeds = [&](const Raw &w, auto tail, auto finite) { // of the four rows' logits: the pair bias (finite: as finite_bias), -inf past the last key
             Tile s;
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 const bf16x8 raw = as_bf16x8(w.r[u]);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    s.x[u][e >> 2][e & 3] = HAS_NB ? to_f32(raw[e]) * LOG2E : 0.f;
+                    const float x = HAS_NB ? to_f32(raw[e]) * LOG2E : 0.f;
+                    s.x[u][e >> 2][e & 3] = decltype(finite)::value ? finite_bias(x) : x;
                 }
             }
             if constexpr (decltype(tail)::value) {
@@ -447,7 +448,7 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
             }
             auto run = [&](int from, int to, auto masked) __attribute__((always_inline)) {
                 for (int t = from; t < to; ++t) {
-                    Tile C = seeds(raw, std::false_type{});
+                    Tile C = seeds(raw, std::false_type{}, std::false_type{});
                     raw = load_nb(t + 1);
                     rows(t, C, masked, [] {});
                 }
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
                         raw = load_tail();
                     }
                 }
-                Tile C = seeds(raw, std::true_type{});
+                Tile C = seeds(raw, std::true_type{}, std::false_type{});
                 rows(full, C, std::true_type{}, [] {});
             }
         }
@@ -500,12 +501,8 @@ __global__ __launch_bounds__(512, 3) void small_head_attention_kernel(const Smal
                     if constexpr (TILES) {
                         return logits(i, t, load_tile(t), std::true_type{});
                     } else {
-                        Raw w = t < full ? load_nb(t) : load_tail();
-#pragma unroll
-                        for (int u = 0; u < 2; ++u) {
-                            w.r[u] = bias_words_at_least(w.r[u], 0xfec0); // -1.28e38: finite in log2 units, with a mask as low too
-                        }
-                        return logits(i, t, t < full ? seeds(w, std::false_type{}) : seeds(w, std::true_type{}), std::true_type{});
+                        return logits(i, t, t < full ? seeds(load_nb(t), std::false_type{}, std::true_type{}) : seeds(load_tail(), std::true_type{}, std::true_type{}),
+                                      std::true_type{});
                     }
                 };
                 float mx[2] = {-INFINITY, -INFINITY};

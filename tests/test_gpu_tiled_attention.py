@@ -467,3 +467,18 @@ def test_pair_bias_rows_of_the_types_lowest_value_in_the_lanes_order(torch_cuda)
         assert not capi.error_flag() and bool(torch.isfinite(out).all()) and bool(torch.isfinite(scratch["avg"]).all())
         got.append((out, scratch["avg"]))
     assert helpers.same_bits(got[0][0], got[1][0]) and helpers.same_bits(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("B,S,H,d", [(9, 301, 4, 32), (66, 200, 4, 32), (40, 200, 4, 32), (6, 64, 4, 32), (3, 385, 4, 32), (20, 259, 8, 32), (2, 1200, 4, 32),
+                                     (64, 77, 8, 8), (3, 200, 4, 16)])
+@pytest.mark.parametrize("bits", [0x7fc0, 0xffc0])
+def test_a_mask_that_is_no_number_is_not_taken_for_a_low_one(torch_cuda, B, S, H, d, bits):
+    """A NaN of either sign in a batch row's mask shows in all of that row's averages, and in no other row's."""
+    w = draw_workload(9400 + S, B, S, H, d, masked=0.0)
+    op, ten, scratch = helpers.make_op(w)
+    ten["bias"].view(torch_cuda.int16)[1, S // 3] = bits - 0x10000 if bits > 0x7fff else bits
+    op.run()
+    torch_cuda.cuda.synchronize()
+    avg = scratch["avg"].float().reshape(B, S, H * d)
+    assert not capi.error_flag() and capi.last_path() != "generic"
+    assert bool(torch_cuda.isnan(avg[1]).all()) and bool(torch_cuda.isfinite(avg[[b for b in range(B) if b != 1]]).all())
